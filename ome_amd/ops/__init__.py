@@ -138,7 +138,7 @@ def ssm_conv1d(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, stat
         return ref.ssm_conv1d(x, w, bias, state, cu, slot, reset, out)
     assert x.stride(1) == 1 and out.stride(1) == 1 and w.is_contiguous() and state.is_contiguous()
     call("ome_ssm_conv1d", x.data_ptr(), x.stride(0), w.data_ptr(), ptr(bias), out.data_ptr(), out.stride(0),
-         state.data_ptr(), _i32(cu).data_ptr(), _i32(slot).data_ptr(), _i32(reset).data_ptr(), slot.shape[0], C,
+         state.data_ptr(), _i32(cu).data_ptr(), _i32(slot).data_ptr(), _i32(reset).data_ptr(), slot.shape[0], T, C,
          w.shape[1], _f32(x, w, bias, out, state), stream_ptr())
     return out
 
