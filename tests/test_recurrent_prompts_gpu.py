@@ -54,3 +54,19 @@ def test_short_conv_in_place():
     want = ops.ssm_conv1d(x, w, None, st, *sq)
     got = ops.ssm_conv1d(x, w, None, s2, *sq, out=x)
     assert torch.allclose(got.float(), want.float(), rtol=2.0 ** -7, atol=1e-5) and torch.equal(st, s2)
+
+
+@pytest.mark.parametrize("group", [64, 128, 256, 512, 1024, 2048])
+@pytest.mark.parametrize("mode", [(False, False, "silu"), (True, False, "silu"), (False, True, "silu"), (True, True, "silu"),
+                                  (True, True, "sigmoid")])
+@pytest.mark.parametrize("rows,off", [(1, 8), (37, 8), (9, 1)])
+def test_gated_norm(group, mode, rows, off):
+    torch.manual_seed(group)
+    first, exact, gate = mode
+    y = torch.randn(rows, 3 * group + off, device=DEV).to(BF)[:, off:]   # off 1: rows that 16-byte loads cannot take
+    z = torch.randn(rows, 3 * group + 16, device=DEV).to(BF)[:, 16:]
+    w = (1 + 0.2 * torch.randn(group if first else 3 * group, device=DEV)).to(BF)
+    want = ref.gated_rmsnorm(*cpu(y, z, w), group, 1e-5, first, exact, gate).float()
+    got = ops.gated_rmsnorm(y, z, w, group, 1e-5, first, exact, gate).cpu().float()
+    # up to three bf16 roundings, each of which a last-bit difference of the fp32 norm can turn by one step
+    assert torch.allclose(got, want, rtol=2.0 ** -6, atol=1e-6)
