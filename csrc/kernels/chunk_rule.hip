@@ -1,0 +1,550 @@
+// Prompt rows of the matrix-state layers with one decay per head, in chunks of 32 rows on the matrix
+// cores (gfx950): the gated delta rule of Qwen3-Next / Jet-Nemotron (DELTA) and the selective scan of
+// Mamba-2 (not DELTA).  With S [dk, dv] the state a chunk starts from, k_i / q_i its key and query
+// rows (unit-norm for DELTA, B / C for Mamba-2), g_i = exp(cum_i) the decay from the chunk's start up to and
+// with row i:
+//   DELTA   A_ij = beta_i exp(cum_i - cum_j) k_i.k_j (j < i),  T = (I + A)^-1,
+//           U = T R,  R_i = beta_i (v_i - g_i k_i S)                    Mamba-2   U_i = dt_i x_i
+//   o_i = g_i q_i S + sum_{j <= i} P_ij U_j,  P_ij = exp(cum_i - cum_j) q_i.k_j     (+ D x_i)
+//       (DELTA: P U = (P T) R, so that o and U both follow from R)
+//   S'  = g_C S + sum_i exp(cum_C - cum_i) k_i U_i^T
+//
+// Two launches.  chunk_gram_kernel, one wave per (chunk, head), parallel over all rows: the 32 x 32
+// matrices P (DELTA: P T) and T and the chunk's scalars, into a workspace.  chunk_rule_kernel walks the chunks of a
+// (sequence, head) in order: a wave owns 16 value columns and keeps its S in VGPR accumulators.
+//
+// fp32 throughout: k and q enter the matrix cores as the bf16 values that they are (their norms, 1 / |k| and
+// 1 / (|q| sqrt(dk)), scale results), S and U as three bf16 parts that sum to the fp32 value exactly, at
+// 3/16 of the fp32 MFMA's time; T R and P U, where both operands are fp32, take the fp32 MFMA.  Decay
+// exponents are summed in fp64 (differences of a long sum).  The row-by-row kernels stay for decode steps
+// (one row per sequence), dk other than 64 / 128, and unaligned views.
+#include "common.h"
+
+namespace {
+
+constexpr int RC = 32;            // rows of a chunk
+constexpr int LDM = RC + 4;       // padded row of a 32 x 32 fp32 matrix in LDS
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// workspace of one (chunk, head): P (DELTA: P T), T (DELTA), then the vectors a, b, c, d [32] and g_C
+template <bool DELTA>
+constexpr int ws_floats() { return (DELTA ? 2 : 1) * RC * RC + 4 * RC + 4; }
+
+struct RuleArgs {
+  const bf16 *q, *k, *v;          // rows of stride `stride` (v: v_stride)
+  int64_t stride, v_stride;
+  const bf16 *a, *b;              // per-head rows: a | b (DELTA), dt (Mamba-2)
+  int64_t ab_stride;
+  const float *A, *D, *dt_bias;   // A_log (DELTA) / A, D (Mamba-2)
+  float dt_min;
+  float* ws;
+  float* state;                   // [slots, H, dv, dk]
+  bf16* out;
+  int64_t out_stride;
+  const int *cu, *slot, *reset;
+  int S, H, Hk, dv;
+};
+
+// Chunk `id` of the launch -> (sequence, first row).  Sequence s owns ids cu[s] / 32 + s and up, one per
+// chunk: ceil(len / 32) <= (cu[s + 1] / 32 + s + 1) - (cu[s] / 32 + s), so ids never overlap and stay
+// below T / 32 + S.  Whole wave; false: an id that no chunk has.
+__device__ __forceinline__ bool chunk_of(int id, const int* cu, int S, int& r0, int& n) {
+  const int lane = threadIdx.x & 63;
+  int s = -1;
+  for (int b = 0; b < S; b += 64) {
+    const int i = b + lane;
+    const int c = __popcll(__ballot(i < S && cu[min(i, S)] / RC + i <= id));
+    s += c;
+    if (c < 64) break;
+  }
+  if (s < 0) return false;
+  r0 = cu[s] + (id - cu[s] / RC - s) * RC;
+  n = min(RC, cu[s + 1] - r0);
+  return n > 0;
+}
+
+__device__ __forceinline__ f32x4 mma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mma_f32(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// eight fp32 values -> three bf16 vectors that sum to them exactly (8 bits of the mantissa each)
+__device__ __forceinline__ void split3(f32x4 x0, f32x4 x1, bf16x8 (&p)[3]) {
+  float r[8];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) r[j] = x0[j], r[4 + j] = x1[j];
+#pragma unroll
+  for (int t = 0; t < 3; ++t) {
+    u32x4 w;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t lo = __float_as_uint(r[2 * j]), hi = __float_as_uint(r[2 * j + 1]);
+      w[j] = __builtin_amdgcn_perm(hi, lo, 0x07060302);   // the two upper halves
+      if (t < 2) {
+        r[2 * j] -= __uint_as_float(lo & 0xffff0000u);
+        r[2 * j + 1] -= __uint_as_float(hi & 0xffff0000u);
+      }
+    }
+    p[t] = __builtin_bit_cast(bf16x8, w);
+  }
+}
+
+// LDS written by lanes of a wave, read by others of the same wave
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+__device__ __forceinline__ float softplus_rule(float x) { return x > 20.f ? x : log1pf(__expf(x)); }
+
+// ---------------------------------------------------------------------------------------------
+// One wave per (chunk, head).  The 16-byte row pieces that a lane loads are both operands of q k^T and
+// k k^T (rows and columns of a 16 x 16 x 32 product have the same lane layout).  T by forward substitution: lane j
+// keeps column j in registers and reads the rows of A from LDS as broadcasts.
+// ---------------------------------------------------------------------------------------------
+template <int DK, bool DELTA>
+__global__ __launch_bounds__(256) void chunk_gram_kernel(RuleArgs a) {
+  constexpr int NS = DK / 32;
+  __shared__ __attribute__((aligned(16))) float sA[4][DELTA ? RC * LDM : 4];
+  __shared__ double s_cum[4][RC];
+  __shared__ float s_vec[4][3][RC];   // 1 / |k|, 1 / (|q| sqrt(dk)), beta
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
+  const int h = blockIdx.y * 4 + w;
+  int r0, n;
+  if (h >= a.H || !chunk_of(blockIdx.x, a.cu, a.S, r0, n)) return;   // whole wave; no block barrier below
+  const int hk = h / (a.H / a.Hk);
+  float* ws = a.ws + ((int64_t)blockIdx.x * a.H + h) * ws_floats<DELTA>();
+
+  bf16x8 kf[2][NS], qf[2][NS];
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb) {
+    const int64_t r = r0 + min(16 * rb + col, n - 1);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      kf[rb][s] = ld8(a.k + r * a.stride + hk * DK + 32 * s + 8 * g);
+      qf[rb][s] = ld8(a.q + r * a.stride + hk * DK + 32 * s + 8 * g);
+    }
+  }
+  // per-row scalars: lane i (and i + 32) holds row i
+  const int row = lane & 31, rv = r0 + min(row, n - 1);
+  const bool ok = row < n;
+  float ga, beta;   // log decay; beta (DELTA) or dt
+  {
+    const float av = (float)a.a[(int64_t)rv * a.ab_stride + h];
+    if constexpr (DELTA) {
+      ga = -__expf(a.A[h]) * softplus_rule(av + a.dt_bias[h]);
+      beta = 1.f / (1.f + __expf(-(float)a.b[(int64_t)rv * a.ab_stride + h]));
+    } else {
+      beta = fmaxf(softplus_rule(av + a.dt_bias[h]), a.dt_min);
+      ga = beta * a.A[h];
+    }
+  }
+  double cum = ok ? (double)ga : 0.0;
+#pragma unroll
+  for (int o = 1; o < 32; o <<= 1) {
+    const double up = __shfl_up(cum, o, 32);
+    if (row >= o) cum += up;
+  }
+  const double total = __shfl(cum, 31);   // rows past the chunk's end add nothing
+  float ik = 1.f, iq = 1.f;
+  if constexpr (DELTA) {
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+      float sk = 0.f, sq = 0.f;
+#pragma unroll
+      for (int s = 0; s < NS; ++s)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          sk += (float)kf[rb][s][j] * (float)kf[rb][s][j];
+          sq += (float)qf[rb][s][j] * (float)qf[rb][s][j];
+        }
+      sk = group4_sum(sk);
+      sq = group4_sum(sq);
+      if (g == 0) {
+        s_vec[w][0][16 * rb + col] = rsqrtf(sk + 1e-6f);
+        s_vec[w][1][16 * rb + col] = rsqrtf(sq + 1e-6f) * rsqrtf((float)DK);
+      }
+    }
+  }
+  if (lane < RC) {
+    s_cum[w][row] = cum;
+    s_vec[w][2][row] = beta;
+  }
+  wave_sync();
+  if constexpr (DELTA) {
+    ik = s_vec[w][0][row];
+    iq = s_vec[w][1][row];
+  }
+  if (lane < RC) {   // the chunk's vectors (zero past its end: such rows add nothing anywhere)
+    float* vec = ws + (DELTA ? 2 : 1) * RC * RC;
+    const float gi = __expf((float)cum), up = __expf((float)(total - cum));
+    vec[row] = ok ? beta : 0.f;
+    vec[RC + row] = ok && DELTA ? beta * gi * ik : 0.f;
+    vec[2 * RC + row] = ok ? gi * iq : 0.f;
+    vec[3 * RC + row] = ok ? up * ik : 0.f;
+    if (row == 0) vec[4 * RC] = __expf((float)total);
+  }
+  f32x4 pm[2][2];
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb) {
+      f32x4 qk = {0.f, 0.f, 0.f, 0.f}, kk = {0.f, 0.f, 0.f, 0.f};
+      if (cb <= rb) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+          qk = mma_bf16(qf[rb][s], kf[cb][s], qk);
+          if constexpr (DELTA) kk = mma_bf16(kf[rb][s], kf[cb][s], kk);
+        }
+      }
+      const int j = 16 * cb + col;
+      const double cj = s_cum[w][j];
+      const float ikj = DELTA ? s_vec[w][0][j] : 1.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 16 * rb + 4 * g + e;
+        float p = 0.f, m = 0.f;
+        if (j <= i && i < n) {
+          const float dec = __expf((float)(s_cum[w][i] - cj)) * ikj;
+          p = qk[e] * dec * (DELTA ? s_vec[w][1][i] : 1.f);
+          if constexpr (DELTA) m = j < i ? kk[e] * dec * s_vec[w][0][i] * s_vec[w][2][i] : 0.f;
+        }
+        if constexpr (DELTA) {
+          pm[rb][cb][e] = p;
+          sA[w][i * LDM + j] = m;
+        } else {
+          ws[i * RC + j] = p;
+        }
+      }
+    }
+  if constexpr (DELTA) {
+    wave_sync();
+    float t[RC];
+#pragma unroll
+    for (int i = 0; i < RC; ++i) {
+      float acc[4] = {i == row ? 1.f : 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int m = 0; m < i; m += 4) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(&sA[w][i * LDM + m]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (m + e < i) acc[e] -= x[e] * t[m + e];
+      }
+      t[i] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    }
+    if (lane < RC) {
+#pragma unroll
+      for (int i = 0; i < RC; ++i) ws[RC * RC + i * RC + row] = t[i];
+    }
+    // P T: T's columns go through LDS into the product's operand layout (k-slot of step e: row 4 g + e)
+    wave_sync();
+    if (lane < RC) {
+#pragma unroll
+      for (int i = 0; i < RC; ++i) sA[w][i * LDM + row] = t[i];
+    }
+    wave_sync();
+    f32x4 tb[2][2];   // [row block][column block]
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int cb = 0; cb <= kb; ++cb)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tb[kb][cb][e] = sA[w][(16 * kb + 4 * g + e) * LDM + 16 * cb + col];
+    wave_sync();
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+      for (int cb = 0; cb <= rb; ++cb)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sA[w][(16 * rb + 4 * g + e) * LDM + 16 * cb + col] = pm[rb][cb][e];
+    wave_sync();
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb) {
+        f32x4 d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kb = cb; kb <= rb; ++kb) {
+          const f32x4 m = *reinterpret_cast<const f32x4*>(&sA[w][(16 * rb + col) * LDM + 16 * kb + 4 * g]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) d = mma_f32(m[e], tb[kb][cb][e], d);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ws[(16 * rb + 4 * g + e) * RC + 16 * cb + col] = d[e];
+      }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
+// The chunks of one (sequence, head) in order; block = NW waves x 16 value columns.  D rows of a 16 x 16
+// product sit at 4 g + e, so with block b of S standing for key channels 32 (b / 2) + 8 (row / 4) + 4 (b % 2) +
+// row % 4, blocks 2 s and 2 s + 1 of a lane are the eight k-slots of step s of k S and q S: S never
+// leaves its registers.  S += k^T U takes k transposed out of the same LDS image (ds_read_b64_tr_b16).  The
+// next chunk's rows and matrices travel to registers while this chunk is computed and to the other LDS
+// buffer after it: one barrier per chunk.
+// ---------------------------------------------------------------------------------------------
+template <int DK>
+__device__ __forceinline__ int img(int row, int chunk) { return row * (DK / 8) + (chunk ^ (row & (DK / 8 - 1))); }
+
+__device__ __forceinline__ bf16x4 tr4(const bf16* base, int elem) {
+  const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (s16x4 __attribute__((address_space(3)))*)((__attribute__((address_space(3))) bf16*)base + elem));
+  return __builtin_bit_cast(bf16x4, v);
+}
+
+template <int DK, bool DELTA, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
+  constexpr int NS = DK / 32, NB = DK / 16, NT = 64 * NW;
+  constexpr int NKL = RC * DK / 8 / NT, NML = RC * RC / 4 / NT;   // 16-byte loads per thread: k (and q), P (and T)
+  static_assert(NKL * NT * 8 == RC * DK && NML * NT * 4 == RC * RC, "whole loads");
+  __shared__ __attribute__((aligned(16))) bf16 sK[2][RC * DK], sQ[2][RC * DK];
+  __shared__ __attribute__((aligned(16))) float sP[2][RC * LDM], sT[DELTA ? 2 : 1][DELTA ? RC * LDM : 4], sV[2][4 * RC + 4];
+  const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, g = lane >> 4;
+  const int s = blockIdx.z, h = blockIdx.x, hk = h / (a.H / a.Hk);
+  const int n0 = (blockIdx.y * NW + (tid >> 6)) * 16;   // this wave's columns
+  const bool live = n0 < a.dv;                          // dv is a multiple of 16: a wave has all of them or none
+  const int r0 = a.cu[s], r1 = a.cu[s + 1];
+  if (r1 <= r0) return;                                 // whole block
+  const int chunks = (r1 - r0 + RC - 1) / RC;
+  const int nc = (live ? n0 : 0) + col;
+
+  // byte offsets of this thread's pieces within a chunk's 32 rows, against uniform bases; a last chunk of fewer
+  // rows repeats its last one (whose scalars are zero)
+  uint32_t ko[NKL], vo[8];
+  auto offsets = [&](int n) {
+#pragma unroll
+    for (int i = 0; i < NKL; ++i) {
+      const int e = tid + NT * i;
+      ko[i] = 2 * ((uint32_t)min(e / (DK / 8), n - 1) * (uint32_t)a.stride + 8 * (e % (DK / 8)));
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      vo[e] = 2 * ((uint32_t)min(16 * (e >> 2) + 4 * g + (e & 3), n - 1) * (uint32_t)a.v_stride + (uint32_t)nc);
+  };
+  const char* kp = reinterpret_cast<const char*>(a.k + (int64_t)r0 * a.stride + hk * DK);
+  const char* qp = reinterpret_cast<const char*>(a.q + (int64_t)r0 * a.stride + hk * DK);
+  const char* vp = reinterpret_cast<const char*>(a.v + (int64_t)r0 * a.v_stride + (int64_t)h * a.dv);
+  const char* mp = reinterpret_cast<const char*>(a.ws + ((int64_t)(r0 / RC + s) * a.H + h) * ws_floats<DELTA>());
+  bf16x8 rk[NKL], rq[NKL];
+  f32x4 rp[NML], rt[NML], rvec;
+  bf16 rv[8];
+  auto fetch = [&](int c) {   // rows and matrices of chunk c
+    if (r0 + (c + 1) * RC > r1) offsets(r1 - r0 - c * RC);
+    const int64_t kc = (int64_t)c * RC * 2 * a.stride;
+#pragma unroll
+    for (int i = 0; i < NKL; ++i) {
+      rk[i] = *reinterpret_cast<const bf16x8*>(kp + kc + ko[i]);
+      rq[i] = *reinterpret_cast<const bf16x8*>(qp + kc + ko[i]);
+    }
+    const char* m = mp + (int64_t)c * a.H * (4 * ws_floats<DELTA>());
+#pragma unroll
+    for (int i = 0; i < NML; ++i) {
+      rp[i] = *reinterpret_cast<const f32x4*>(m + (uint32_t)(16 * (tid + NT * i)));
+      if constexpr (DELTA) rt[i] = *reinterpret_cast<const f32x4*>(m + (uint32_t)(4 * RC * RC + 16 * (tid + NT * i)));
+    }
+    if (tid < RC + 1) rvec = *reinterpret_cast<const f32x4*>(m + (uint32_t)((DELTA ? 8 : 4) * RC * RC + 16 * tid));
+    const char* v = vp + (int64_t)c * RC * 2 * a.v_stride;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) rv[e] = *reinterpret_cast<const bf16*>(v + vo[e]);
+  };
+  auto put = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < NKL; ++i) {
+      const int e = tid + NT * i, o = img<DK>(e / (DK / 8), e % (DK / 8)) * 8;
+      st8(&sK[b][o], rk[i]);
+      st8(&sQ[b][o], rq[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < NML; ++i) {
+      const int e = tid + NT * i, o = e / (RC / 4) * LDM + 4 * (e % (RC / 4));
+      *reinterpret_cast<f32x4*>(&sP[b][o]) = rp[i];
+      if constexpr (DELTA) *reinterpret_cast<f32x4*>(&sT[b][o]) = rt[i];
+    }
+    if (tid < RC + 1) *reinterpret_cast<f32x4*>(&sV[b][4 * tid]) = rvec;
+  };
+
+  // state: lane (col, g) holds column nc, key channels 32 s + 8 g .. + 7 in blocks 2 s, 2 s + 1
+  float* st = a.state + (((int64_t)a.slot[s] * a.H + h) * a.dv + nc) * DK + 8 * g;
+  f32x4 S[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+    S[b] = a.reset[s] != 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4*>(st + 32 * (b >> 1) + 4 * (b & 1));
+  const float Dh = DELTA ? 0.f : a.D[h];
+  uint32_t oo[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) oo[e] = 2 * ((uint32_t)(16 * (e >> 2) + 4 * g + (e & 3)) * (uint32_t)a.out_stride + (uint32_t)nc);
+  char* op = reinterpret_cast<char*>(a.out + (int64_t)r0 * a.out_stride + (int64_t)h * a.dv);
+
+  offsets(RC);
+  fetch(0);
+  put(0);
+  bf16 vc[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) vc[e] = rv[e];
+  __syncthreads();
+  const auto step = [&](int c, int b) {
+    if (c + 1 < chunks) fetch(c + 1);
+    const bf16 *K = sK[b], *Q = sQ[b];
+    // ---- k S and q S ----
+    f32x4 ks[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int t = 0; t < NS; ++t) {
+      bf16x8 part[3], qa[2], ka[2];
+      split3(S[2 * t], S[2 * t + 1], part);
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) {
+        const int at = img<DK>(16 * rb + col, 4 * t + g) * 8;
+        qa[rb] = ld8(&Q[at]);
+        if constexpr (DELTA) ka[rb] = ld8(&K[at]);
+      }
+#pragma unroll
+      for (int p = 2; p >= 0; --p)
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb) {
+          if constexpr (DELTA) ks[rb] = mma_bf16(ka[rb], part[p], ks[rb]);
+          o[rb] = mma_bf16(qa[rb], part[p], o[rb]);
+        }
+    }
+    // ---- R (DELTA) / U (Mamba-2) ----
+    f32x4 r[2], u[2];
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+      const f32x4 va = *reinterpret_cast<const f32x4*>(&sV[b][16 * rb + 4 * g]);
+      const f32x4 vb = *reinterpret_cast<const f32x4*>(&sV[b][RC + 16 * rb + 4 * g]);
+      const f32x4 vg = *reinterpret_cast<const f32x4*>(&sV[b][2 * RC + 16 * rb + 4 * g]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x = (float)vc[4 * rb + e];
+        r[rb][e] = va[e] * x;
+        if constexpr (DELTA) r[rb][e] -= vb[e] * ks[rb][e];
+        o[rb][e] = o[rb][e] * vg[e] + (DELTA ? 0.f : Dh * x);
+      }
+      u[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    const float gc = sV[b][4 * RC];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) S[nb] *= gc;
+    // ---- U = T R, o += (P T) R (Mamba-2: o += P U) ----
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      f32x4 pm[2], tm[2];
+#pragma unroll
+      for (int rb = kb; rb < 2; ++rb) {
+        pm[rb] = *reinterpret_cast<const f32x4*>(&sP[b][(16 * rb + col) * LDM + 16 * kb + 4 * g]);
+        if constexpr (DELTA) tm[rb] = *reinterpret_cast<const f32x4*>(&sT[b][(16 * rb + col) * LDM + 16 * kb + 4 * g]);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int rb = kb; rb < 2; ++rb) {
+          if constexpr (DELTA) u[rb] = mma_f32(tm[rb][e], r[kb][e], u[rb]);
+          o[rb] = mma_f32(pm[rb][e], r[kb][e], o[rb]);
+        }
+    }
+    // ---- S = g_C S + k^T U ----
+    {
+      bf16x8 part[3], ka[NB];
+      const int qr = 4 * g + (col >> 2), p4 = col & 3;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        const int ch = 4 * (nb >> 1) + p4, half = 4 * (nb & 1);
+        const bf16x4 lo = tr4(K, img<DK>(qr, ch) * 8 + half), hi = tr4(K, img<DK>(16 + qr, ch) * 8 + half);
+        ka[nb] = bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      }
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) {
+        const f32x4 vd = *reinterpret_cast<const f32x4*>(&sV[b][3 * RC + 16 * rb + 4 * g]);
+        u[rb] = (DELTA ? u[rb] : r[rb]) * vd;
+      }
+      split3(u[0], u[1], part);
+#pragma unroll
+      for (int p = 2; p >= 0; --p)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) S[nb] = mma_bf16(ka[nb], part[p], S[nb]);
+    }
+    if (live) {
+      char* oc = op + (int64_t)c * RC * 2 * a.out_stride;
+      const int n = r1 - r0 - c * RC;
+      if (n >= RC) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) *reinterpret_cast<bf16*>(oc + oo[e]) = (bf16)o[e >> 2][e & 3];
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (16 * (e >> 2) + 4 * g + (e & 3) < n) *reinterpret_cast<bf16*>(oc + oo[e]) = (bf16)o[e >> 2][e & 3];
+      }
+    }
+    if (c + 1 < chunks) {
+      put(b ^ 1);   // last read before the previous barrier
+#pragma unroll
+      for (int e = 0; e < 8; ++e) vc[e] = rv[e];
+    }
+    __syncthreads();
+  };
+  for (int c = 0; c < chunks; c += 2) {
+    step(c, 0);
+    if (c + 1 < chunks) step(c + 1, 1);
+  }
+  if (live) {
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) *reinterpret_cast<f32x4*>(st + 32 * (nb >> 1) + 4 * (nb & 1)) = S[nb];
+  }
+}
+
+template <bool DELTA>
+int launch_rule(const RuleArgs& a, int T, int dk, hipStream_t stream) {
+  const dim3 gram(T / RC + a.S, (a.H + 3) / 4);
+  const dim3 rule(a.H, (a.dv + 63) / 64, a.S);
+  if (dk == 128) {
+    chunk_gram_kernel<128, DELTA><<<gram, 256, 0, stream>>>(a);
+    chunk_rule_kernel<128, DELTA, 4><<<rule, 256, 0, stream>>>(a);
+  } else {
+    chunk_gram_kernel<64, DELTA><<<gram, 256, 0, stream>>>(a);
+    chunk_rule_kernel<64, DELTA, 4><<<rule, 256, 0, stream>>>(a);
+  }
+  OME_CHECK_LAUNCH();
+  return 0;
+}
+
+// (row strides below 2^24 elements: a chunk's byte offsets stay in 32 bits)
+bool rule_shape(int S, int H, int Hk, int dk, int dv, int64_t s0, int64_t s1, int64_t s2) {
+  return s0 >= 0 && s1 >= 0 && s2 >= 0 && s0 < 1 << 24 && s1 < 1 << 24 && s2 < 1 << 24 && S > 0 && S <= 65535 && H > 0 && Hk > 0 && H % Hk == 0 && (dk == 64 || dk == 128) && dv > 0 && dv % 16 == 0 &&
+         (dv + 63) / 64 <= 65535 && (H + 3) / 4 <= 65535;
+}
+
+bool aligned16(const void* p, int64_t elems) { return ((uintptr_t)p | (uintptr_t)(elems * 2)) % 16 == 0; }
+
+}  // namespace
+
+// fp32 words of workspace of one (chunk, head); T rows of S sequences and H heads need (T / 32 + S) * H of them
+OME_API int ome_chunk_rule_floats(int delta) { return delta ? ws_floats<true>() : ws_floats<false>(); }
+
+// Gated delta rule over all rows of every sequence; operands as ome_gdn_scan.  -3: a shape, stride or
+// alignment that the chunked kernels do not take (nothing is launched).
+OME_API int ome_gdn_chunks(const void* q, const void* k, const void* v, int64_t qkv_stride, const void* a, const void* b,
+                           int64_t ab_stride, const float* A_log, const float* dt_bias, float* state, void* out,
+                           int64_t out_stride, const int* cu, const int* slot, const int* reset, int S, int T, int Hv, int Hk,
+                           int dk, int dv, float* ws, hipStream_t stream) {
+  if (T <= 0 || !ws || !rule_shape(S, Hv, Hk, dk, dv, qkv_stride, qkv_stride, out_stride) || !aligned16(q, qkv_stride) || !aligned16(k, qkv_stride) ||
+      (uintptr_t)state % 16 || (uintptr_t)ws % 16)
+    return -3;
+  const RuleArgs r{(const bf16*)q, (const bf16*)k, (const bf16*)v, qkv_stride, qkv_stride, (const bf16*)a, (const bf16*)b,
+                   ab_stride, A_log, nullptr, dt_bias, 0.f, ws, state, (bf16*)out, out_stride, cu, slot, reset, S, Hv, Hk, dv};
+  return launch_rule<true>(r, T, dk, stream);
+}
+
+// Mamba-2's selective scan over all rows of every sequence; operands as ome_ssm_scan.
+OME_API int ome_ssm_chunks(const void* x, int64_t x_stride, const void* dt, int64_t dt_stride, const void* B, const void* Cm,
+                           int64_t bc_stride, const float* A, const float* D, const float* dt_bias, float dt_min, float* state,
+                           void* y, int64_t y_stride, const int* cu, const int* slot, const int* reset, int S, int T, int H,
+                           int P, int N, int G, float* ws, hipStream_t stream) {
+  if (T <= 0 || !ws || !rule_shape(S, H, G, N, P, bc_stride, x_stride, y_stride) || !aligned16(B, bc_stride) || !aligned16(Cm, bc_stride) ||
+      (uintptr_t)state % 16 || (uintptr_t)ws % 16)
+    return -3;
+  const RuleArgs r{(const bf16*)Cm, (const bf16*)B, (const bf16*)x, bc_stride, x_stride, (const bf16*)dt, nullptr,
+                   dt_stride, A, D, dt_bias, dt_min, ws, state, (bf16*)y, y_stride, cu, slot, reset, S, H, G, P};
+  return launch_rule<false>(r, T, N, stream);
+}

@@ -70,3 +70,77 @@ def test_gated_norm(group, mode, rows, off):
     got = ops.gated_rmsnorm(y, z, w, group, 1e-5, first, exact, gate).cpu().float()
     # up to three bf16 roundings, each of which a last-bit difference of the fp32 norm can turn by one step
     assert torch.allclose(got, want, rtol=2.0 ** -6, atol=1e-6)
+
+
+def exact_gdn(q, k, v, a, b, A_log, dtb, state, cu, slot, reset, Hv, Hk):
+    q, k, v, a, b, A_log, dtb = (t.cpu().double() for t in (q, k, v, a, b, A_log, dtb))
+    st, dv, dk = state.cpu().double(), state.shape[2], state.shape[3]
+    unit = lambda t: t / (t.square().sum(-1, keepdim=True) + 1e-6).sqrt()  # noqa: E731
+    out = torch.zeros(q.shape[0], Hv, dv, dtype=torch.float64)
+    for s, sl in enumerate(slot.tolist()):
+        r0, r1 = cu[s:s + 2].tolist()
+        S = st[sl] * (0.0 if reset[s] else 1.0)
+        for r in range(r0, r1):
+            kr = unit(k[r].view(Hk, dk)).repeat_interleave(Hv // Hk, 0)
+            qr = unit(q[r].view(Hk, dk)).repeat_interleave(Hv // Hk, 0) * dk ** -0.5
+            S = S * torch.exp(-A_log.exp() * torch.nn.functional.softplus(a[r] + dtb))[:, None, None]
+            u = (v[r].view(Hv, dv) - (S @ kr[:, :, None])[..., 0]) * b[r].sigmoid()[:, None]
+            S = S + u[:, :, None] * kr[:, None]
+            out[r] = (S @ qr[:, :, None])[..., 0]
+        if r1 > r0:
+            st[sl] = S
+    return out.flatten(1), st
+
+
+def exact_ssm(x, dt, B, C, A, D, dtb, dt_min, state, cu, slot, reset, H, P, N, G):
+    x, dt, B, C, A, D, dtb = (t.cpu().double() for t in (x, dt, B, C, A, D, dtb))
+    st = state.cpu().double()
+    out = torch.zeros(x.shape[0], H, P, dtype=torch.float64)
+    for s, sl in enumerate(slot.tolist()):
+        r0, r1 = cu[s:s + 2].tolist()
+        S = st[sl] * (0.0 if reset[s] else 1.0)
+        for r in range(r0, r1):
+            d = torch.nn.functional.softplus(dt[r] + dtb).clamp(min=dt_min)
+            b, c = (t[r].view(G, N).repeat_interleave(H // G, 0) for t in (B, C))
+            S = S * (d * A).exp()[:, None, None] + (d[:, None] * x[r].view(H, P))[:, :, None] * b[:, None]
+            out[r] = (S @ c[:, :, None])[..., 0] + D[:, None] * x[r].view(H, P)
+        if r1 > r0:
+            st[sl] = S
+    return out.flatten(1), st
+
+
+def near(out, state, want, want_state):
+    """Outputs: one rounding to bf16 (2^-9 of each value at most, so of the whole).  States: fp32 sums; a state row is a
+    sum of at most 2^8 products whose weights (decays, norms) carry a few fp32 roundings each: 2^-24 * 2^5."""
+    rel = lambda x, y: ((x.cpu().double() - y).norm() / y.norm()).item()  # noqa: E731
+    return rel(out, want) < 2.0 ** -9 and rel(state, want_state) < 2.0 ** -19
+
+
+@pytest.mark.parametrize("lens", LENS, ids=str)
+@pytest.mark.parametrize("dk,dv,Hk,Hv,off", [(128, 128, 2, 4, 8), (64, 16, 1, 5, 0), (128, 80, 3, 3, 8), (64, 128, 2, 2, 1)])
+def test_delta_rule_prompts(lens, dk, dv, Hk, Hv, off):
+    torch.manual_seed(dk + dv)
+    T, slots, kd, vd = sum(lens), 71, Hk * dk, Hv * dv
+    c = torch.randn(T, 2 * kd + vd + off, device=DEV).to(BF)[:, off:]   # off 1: the row-by-row kernel
+    ab = torch.randn(T, 2 * Hv, device=DEV).to(BF)
+    A_log, dtb = torch.linspace(-4, 2.5, Hv, device=DEV), torch.randn(Hv, device=DEV)
+    st = torch.randn(slots, Hv, dv, dk, device=DEV) * 0.2
+    sq = seqs(lens, slots)
+    args = (c[:, :kd], c[:, kd:2 * kd], c[:, 2 * kd:], ab[:, :Hv], ab[:, Hv:], A_log, dtb)
+    want = exact_gdn(*args, st, *sq, Hv, Hk)
+    assert near(ops.gdn_scan(*args, st, *sq, Hv, Hk), st, *want)
+
+
+@pytest.mark.parametrize("lens", LENS, ids=str)
+@pytest.mark.parametrize("H,P,N,G,off", [(16, 64, 128, 2, 8), (3, 16, 64, 1, 0), (5, 80, 128, 5, 8), (4, 64, 128, 2, 1)])
+def test_selective_scan_prompts(lens, H, P, N, G, off):
+    torch.manual_seed(H + N)
+    T, slots = sum(lens), 71
+    c = torch.randn(T, H * P + 2 * G * N + off, device=DEV).to(BF)[:, off:]
+    dt = torch.randn(T, H + 3, device=DEV).to(BF)[:, 3:]
+    A, D, dtb = -torch.logspace(-1, 1.2, H, device=DEV), torch.randn(H, device=DEV), torch.linspace(-6, 1, H, device=DEV)
+    st = torch.randn(slots, H, P, N, device=DEV) * 0.2
+    sq = seqs(lens, slots)
+    args = (c[:, :H * P], dt, c[:, H * P:H * P + G * N], c[:, H * P + G * N:], A, D, dtb, 0.001)
+    want = exact_ssm(*args, st, *sq, H, P, N, G)
+    assert near(ops.ssm_scan(*args, st, *sq, H, P, N, G), st, *want)
