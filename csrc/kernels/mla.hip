@@ -203,162 +203,392 @@ __global__ __launch_bounds__(256) void mla_attn_kernel(
   }
 }
 
+// One wave's share of a latent page's move to LDS: 64 lanes x 16 bytes from `off` (per lane) of the page at `base`
+// to `lds` + 16 lane.  By asm, because the compiler takes every later LDS read of the image's array for a reader of
+// the move and waits for all of it (vmcnt 0) there; the kernels below wait themselves, once, before the barrier
+// after which a tile is read.  (No register is written; the descriptor's size bounds the reads to the page.)
+__device__ __forceinline__ void page_to_lds(const bf16* base, uint32_t bytes, uint32_t off, const void* lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  const uint64_t b = (uint64_t)base;
+  const u32x4 rs = {(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, bytes, 0x00020000u};
+  const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)lds;
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+               :
+               : "s"(__builtin_amdgcn_readfirstlane(at)), "v"(off), "s"(rs)
+               : "m0", "memory");
+#endif
+}
+
 // ------------------------------------------------------------------------------------------
-// All-heads variant: one workgroup of NW waves owns 16 * NW heads of a token and one split-K
-// partition, so each latent key tile is streamed from HBM and staged in LDS ONCE for all of them
-// (the 16-head kernel above re-reads every token's latent KV H / 16 times -- 8x for DeepSeek-V3's
-// 128 heads -- and its four waves each recompute the same S^T).  Wave w owns heads 16 w .. 16 w + 15
-// and ALL DV value dims:
-//   S^T [32 keys x 16 heads] = K . Q^T   (2 x DK/32 MFMAs, Q^T resident in 72 VGPRs)
-//   O^T [DV x 16] += V^T . P^T           (DV/16 MFMAs, V^T by hardware-transposed LDS reads)
-// Key tiles arrive by LDS DMA (buffer_load ... lds) into a double-buffered image: the DMA of tile
-// n+1 is issued before tile n is computed and retired (vmcnt(0) + barrier) after it.
+// Row tiles: one workgroup of NW waves owns 32 * NW neighbouring query rows (row = token * H + head) and one
+// split-K partition, so that each latent key tile is streamed and staged in LDS ONCE for all of them: the heads
+// of one token in decode, the heads of several prompt tokens of a sequence otherwise (the 16-head
+// kernel above streams the prefix again for every token, and its four waves each compute the same S^T).  A tile
+// whose tokens belong to different block-table rows walks those rows one after the other, its other tokens masked.
+//
+// Bound by the matrix cores, with LDS reads close behind: a wave owns 32 rows and all DV value dims, so each
+// LDS operand feeds 32 columns (16 rows a wave, the layout before, read every key tile eight times per
+// 128 rows).  That takes one wave per SIMD: O^T [DV x 32] fills the 256 accumulation registers, Q^T 144 of
+// the others.
+//   S^T [32 keys x 32 rows] = K . Q^T   (DK/16 MFMAs 32x32x16, lane = key / row, 8 dims a lane half)
+//   O^T [DV x 32] += V^T . P^T          (DV/32 x 2 MFMAs; V^T by hardware-transposed LDS reads, key order of S^T)
+// Nothing else runs on the SIMD meanwhile, so the loop is pipelined by hand: S^T of tile n + 1 is multiplied while
+// the softmax of tile n runs on the vector ALU, and the LDS DMA of tile n + 2 is in flight (three images).
+// O^T is rescaled only where a row's maximum rose by more than 2^8 since its last rescale (weights stay below
+// 2^8), almost never after a row's first tile.  The denominator sums the weights as rounded to bf16.
+//
+// Measured (16-head kernel, or for decode the 16-row waves before -> now): three prompts of 3394 rows x 16 heads
+// 738 -> 128 us (118 -> 680 TFLOP/s), one of 5500 rows 4830 -> 545 us (965; a large bf16 product reaches 1530 on this
+// card); decode, 48 contexts of ~3000 keys x 128 heads 100 -> 79 us, x 16 heads 104 -> 65 us.  Error against 64 bits
+// 0.0018 -> 0.0020 of the result: bf16 weights and outputs as before, but a row's largest weight is no longer
+// exactly 1.
 // ------------------------------------------------------------------------------------------
-typedef __attribute__((address_space(3))) void mla_lds_t;
+// The products by asm: with one wave per SIMD, what covers an LDS read is the distance to its product, and the
+// compiler sinks reads to their use (or hoists them all, into scratch).  Volatile with a memory clobber, each stays
+// between the reads around it.  The waits that the compiler cannot see: `mma_new` after a VALU write of its
+// operands, `MMA_WAIT` between a last product and the first other reader of its result.
+#define MMA_WAIT "s_nop 15\n\ts_nop 3"
+__device__ __forceinline__ void mma_new(f32x16& c, bf16x8 a, bf16x8 b) {   // c = a b
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_nop 3\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b) : "memory");
+#endif
+}
+__device__ __forceinline__ void mma_add(f32x16& c, bf16x8 a, bf16x8 b) {   // c += a b, c in vector registers
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b) : "memory");
+#endif
+}
+__device__ __forceinline__ void mma_acc(f32x16& c, bf16x8 a, bf16x8 b) {   // c += a b, c in accumulation registers
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b) : "memory");
+#endif
+}
 
 template <int DK, int DV, int NW>
-__global__ __launch_bounds__(64 * NW, 1) void mla_attn_all_kernel(
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1))) void mla_attn_rows_kernel(
     const bf16* __restrict__ q, int64_t q_stride_t, const bf16* __restrict__ cache,
     const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ tok_row,
-    const int* __restrict__ kv_lens, int H, float scale_log2, int parts, bf16* __restrict__ out,
-    int64_t out_stride_t, float* __restrict__ ws_o, float* __restrict__ ws_ml) {
+    const int* __restrict__ kv_lens, int T, int H, float scale_log2, int parts, int2* __restrict__ plan,
+    bf16* __restrict__ out, int64_t out_stride_t, float* __restrict__ ws_o, float* __restrict__ ws_ml) {
   static_assert(DK == 576 && lds_chunks<DK>() == DK / 8, "LDS DMA image assumes unpadded 72-chunk rows");
-  constexpr int CH = DK / 8, NI = KT * CH / 64, NB = DV / 16;
-  constexpr int IMG = KT * CH * 8;   // bf16 elements per K-tile image
-  __shared__ __attribute__((aligned(16))) bf16 sK[2 * IMG];
-  const int t = blockIdx.x, part = blockIdx.z;
+  constexpr int CH = DK / 8, NI = KT * CH / 64, NJ = NI / NW, NV = DV / 32, NS = DK / 16;
+  static_assert(NI % NW == 0, "whole DMA instructions per wave");
+  constexpr int IMG = KT * CH * 16;   // bytes per key-tile image
+  constexpr float LAZY = 8.f;
+  constexpr int AHEAD = 4;            // LDS operands in flight: 4 x 32 cycles of matrix work cover a read
+  __shared__ __attribute__((aligned(16))) char sK[3 * IMG];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int col = lane & 15, g = lane >> 4;
-  const int head = blockIdx.y * 16 * NW + wave * 16 + col;   // this lane's head (S^T / O^T column)
-  const int L = kv_lens[t];
-  const int n_pages = (L + 15) >> 4;
-  const int pairs = (n_pages + 1) >> 1;
-  const int per_part = (pairs + parts - 1) / parts;
-  const int pair_begin = part * per_part, pair_end = min(pairs, pair_begin + per_part);
-  const int* bt = block_tables + (int64_t)tok_row[t] * bt_stride;
-
-  // K tile pair -> LDS image: instruction i writes chunks [64 i, 64 i + 64) lane-linearly, each
-  // lane fetching the source chunk the row's XOR swizzle puts there.  A page is 16 rows x 72 chunks
-  // = 18 instructions, so each instruction reads one page: its descriptor is based at that page.
-  auto dma_pair = [&](int pr, bf16* img) {
+  const int col = lane & 31, hf = lane >> 5;
+  constexpr int RT = 32 * NW, SPAN = 2, UNITS = 256;
+  // `plan`: a tile is RT heads of one token, and contexts are cut by length (decode); else RT rows of [T * H]
+  const bool decode = plan != nullptr;
+  const int R = T * H, HG = (H + RT - 1) / RT;
+  int unit = decode ? blockIdx.x : gridDim.x - 1 - blockIdx.x, part = blockIdx.y, my_parts = parts;   // (longest rows first)
+  if (decode && parts > 1) {
+    // Workgroup w of 256 takes piece w.  The span is the smallest number of key tiles that cuts all units
+    // into at most 256 pieces: one a CU (also within each XCD, to which workgroups go in turn), and none longer
+    // than it has to be, however ragged the contexts.  Every wave finds it from the lengths: lane l holds
+    // tokens 4 l .. 4 l + 3.
+    int nt4[4], most = SPAN, all = 0;
 #pragma unroll
-    for (int j = 0; j < (NI + NW - 1) / NW; ++j) {
-      const int i = wave + NW * j;
-      if (i >= NI) break;
-      const int c = 64 * i + lane, row = c / CH, xl = c - row * CH;
-      const int pg = 2 * pr + (i >= NI / 2);
-      const int page = bt[pg < n_pages ? pg : 0];
-      const auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)(cache + (int64_t)page * 16 * DK), (short)0,
-                                                        16 * DK * 2, 0x00020000);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (mla_lds_t*)(img + 64 * 8 * i), 16,
-                                               (uint32_t)(((row & 15) * CH + (xl ^ (row & 7))) * 16), 0, 0, 0);
+    for (int i = 0; i < 4; ++i) {
+      const int tk = 4 * lane + i;
+      nt4[i] = tk < T ? (kv_lens[tk] + KT - 1) / KT : 0;
+      most = max(most, nt4[i]);
+      all += nt4[i];
+    }
+    auto count = [&](int span, int i) { return 4 * lane + i < T ? min(parts, max(1, (nt4[i] + span - 1) / span)) : 0; };
+    auto pieces = [&](int span) {
+      int n = count(span, 0) + count(span, 1) + count(span, 2) + count(span, 3);
+#pragma unroll
+      for (int x = 32; x > 0; x >>= 1) n += __shfl_xor(n, x);
+      return __builtin_amdgcn_readfirstlane(n) * HG;
+    };
+#pragma unroll
+    for (int x = 32; x > 0; x >>= 1) most = max(most, __shfl_xor(most, x)), all += __shfl_xor(all, x);
+    most = __builtin_amdgcn_readfirstlane(most);
+    all = __builtin_amdgcn_readfirstlane(all) * HG;
+    // all / span <= pieces <= all / span + units; one piece a unit is at most 256 (the caller's rule)
+    int lo = max(SPAN, min(most, all / UNITS)), hi = T * HG < UNITS ? max(lo, min(most, all / (UNITS - T * HG) + 1)) : most;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (pieces(mid) <= UNITS) hi = mid;
+      else lo = mid + 1;
+    }
+    const int w = blockIdx.x, c0 = count(lo, 0), c1 = count(lo, 1), c2 = count(lo, 2), c3 = count(lo, 3);
+    int incl = c0 + c1 + c2 + c3;
+#pragma unroll
+    for (int x = 1; x < 64; x <<= 1) {
+      const int up = __shfl_up(incl, x);
+      if (lane >= x) incl += up;
+    }
+    if (w >= __builtin_amdgcn_readlane(incl, 63) * HG) return;   // whole block
+    const int at = __popcll(__ballot(incl * HG <= w));            // the lane whose tokens piece w belongs to
+    int tok = 4 * at, base = at ? __builtin_amdgcn_readlane(incl, at - 1) : 0;
+    my_parts = __builtin_amdgcn_readlane(c0, at);
+    if ((base + my_parts) * HG <= w) base += my_parts, ++tok, my_parts = __builtin_amdgcn_readlane(c1, at);
+    if ((base + my_parts) * HG <= w) base += my_parts, ++tok, my_parts = __builtin_amdgcn_readlane(c2, at);
+    if ((base + my_parts) * HG <= w) base += my_parts, ++tok, my_parts = __builtin_amdgcn_readlane(c3, at);
+    const int hg = (w - base * HG) / my_parts;
+    part = (w - base * HG) - hg * my_parts;
+    unit = tok * HG + hg;
+    if (part == 0 && tid == 0) plan[unit] = int2{w, my_parts};
+  }
+  const int row0 = decode ? unit / HG * H + unit % HG * RT : unit * RT;
+  const int row_end = decode ? (unit / HG + 1) * H : R;
+  const int row = row0 + wave * 32 + col;                           // this lane's row (S^T / O^T column)
+  const bool hv = row < row_end;
+  const int t = min(decode ? unit / HG : row / H, T - 1), head = hv ? row - t * H : 0;
+  const int my_row = tok_row[t], my_len = hv ? kv_lens[t] : 0;
+
+  // Key tile -> LDS image: instruction i writes chunks [64 i, 64 i + 64) lane-linearly, each lane fetching the source
+  // chunk that the row's XOR swizzle puts there.  A page is 16 rows x 72 chunks = 18 instructions, so each
+  // instruction reads one page: its descriptor is based at that page.
+  auto dma = [&](const int* bt, int n_pages, int tile, int img) {
+    const int p0 = 2 * tile, p1 = p0 + 1;
+    const bf16* b0 = cache + (int64_t)bt[p0 < n_pages ? p0 : 0] * 16 * DK;
+    const bf16* b1 = cache + (int64_t)bt[p1 < n_pages ? p1 : 0] * 16 * DK;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int i = wave + NW * j, c = 64 * i + lane, kr = c / CH, xl = c - kr * CH;
+      page_to_lds(i < NI / 2 ? b0 : b1, 16 * DK * 2, (uint32_t)(((kr & 15) * CH + (xl ^ (kr & 7))) * 16),
+                  sK + img * IMG + 64 * 16 * i);
     }
   };
-  if (pair_begin < pair_end) dma_pair(pair_begin, sK);
 
-  bf16x8 qf[DK / 32];
-  const bf16* qp = q + (int64_t)t * q_stride_t + (int64_t)head * DK + 8 * g;
+  bf16x8 qf[NS];
+  const bf16* qp = q + (int64_t)t * q_stride_t + (int64_t)head * DK + 8 * hf;
 #pragma unroll
-  for (int s = 0; s < DK / 32; ++s) qf[s] = ld8(qp + 32 * s);
+  for (int s = 0; s < NS; ++s) qf[s] = ld8(qp + 16 * s);
 
-  f32x4 o[NB];
+  f32x16 o[NV];
 #pragma unroll
-  for (int i = 0; i < NB; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int v = 0; v < NV; ++v)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[v][i] = 0.f;
   float m = OME_NEG_INF, lsum = 0.f;
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
 
-  // The XOR swizzle makes every LDS offset lane-dependent; split it so the compiler sees a lane
-  // base plus an immediate: (8k + c) ^ z = 8k + (c ^ z) for c, z < 8.  S^T reads chunk 4 s + g of
-  // row col (2 bases by s parity); V^T reads chunk 2 nb + pcol/2 of row 4 g + qrow (4 bases by
-  // nb mod 4).  Rows 16..31 sit 16 * CH chunks further on with the same (row & 7).
-  const int qrow = (lane & 15) >> 2, pcol = lane & 3;
-  int sofs[2], vofs[4];
+  // LDS lane bases; the XOR swizzle acts on the low three bits of a chunk index, the rest are immediates.
+  // S^T reads chunk 2 s + hf of key row col; V^T reads, for 16-lane group gr = lane / 16, rows 4 hf + qr (+ 8, 16, 24)
+  // and chunk 4 v + 2 (gr & 1) + pc / 2.
+  const int gr = lane >> 4, qr = (lane & 15) >> 2, pc = lane & 3;
+  uint32_t sofs[4], vofs[2];
 #pragma unroll
-  for (int e = 0; e < 2; ++e) sofs[e] = (col * CH + ((4 * e + g) ^ (col & 7))) * 16;
-  const int rv = 4 * g + qrow;
+  for (int e = 0; e < 4; ++e) sofs[e] = (col * CH + ((2 * e + hf) ^ (col & 7))) * 16;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) vofs[e] = (rv * CH + ((2 * e + (pcol >> 1)) ^ (rv & 7))) * 16 + (pcol & 1) * 8;
-  int buf = 0;
-  for (int pr = pair_begin; pr < pair_end; ++pr) {
-    const bf16* img = sK + buf * IMG;
-    // the other image's last readers passed the barrier that ended the previous tile
-    if (pr + 1 < pair_end) dma_pair(pr + 1, sK + (buf ^ 1) * IMG);
-    // ---- S^T [32 keys x 16 heads] ----
-    const char* ib = reinterpret_cast<const char*>(img);
-    f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+  for (int e = 0; e < 2; ++e)
+    vofs[e] = ((4 * hf + qr) * CH + ((4 * e + 2 * (gr & 1) + (pc >> 1)) ^ (4 * hf + qr))) * 16 + (pc & 1) * 8;
+  auto kfrag = [&](uint32_t img, int s) { return *reinterpret_cast<const bf16x8*>(sK + (sofs[s & 3] + img) + (s >> 2) * 128); };
+  auto score = [&](uint32_t img) {   // S^T of the tile in image `img` (byte offset)
+    f32x16 a;
+    bf16x8 k[AHEAD];   // operands on their way from LDS
 #pragma unroll
-    for (int s = 0; s < DK / 32; ++s) {
-      const int off = sofs[s & 1] + (s >> 1) * 128;   // swz(col, 4 s + g): lane base + immediate
-      const bf16x8 a0 = *reinterpret_cast<const bf16x8*>(ib + off);
-      const bf16x8 a1 = *reinterpret_cast<const bf16x8*>(ib + off + 16 * CH * 16);
-      s0 = mfma16x32(a0, qf[s], s0);
-      s1 = mfma16x32(a1, qf[s], s1);
+    for (int s = 0; s < AHEAD; ++s) k[s] = kfrag(img, s);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      if (s == 0) mma_new(a, k[0], qf[0]);
+      else mma_add(a, k[s % AHEAD], qf[s]);
+      if (s + AHEAD < NS) k[s % AHEAD] = kfrag(img, s + AHEAD);
     }
-    const int kbase = pr * KT;
-    float mx = OME_NEG_INF;
+    asm volatile(MMA_WAIT : "+v"(a));
+    return a;
+  };
+  auto vfrag = [&](uint32_t img, int v, int st) {
+    const int at = vofs[v & 1] + img + (v >> 1) * 128 + st * 16 * CH * 16;
+    const bf16x4 x = tr_read(reinterpret_cast<const bf16*>(sK), at), y = tr_read(reinterpret_cast<const bf16*>(sK), at + 8 * CH * 16);
+    return bf16x8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+  };
+
+  // the tile's tokens (at most 64: H >= 4), one a lane; the same in every wave
+  const int t0 = row0 / H, nt = (min(row0 + RT, row_end) - 1) / H - t0 + 1;
+  const int tl_row = tok_row[t0 + min(lane, nt - 1)], tl_len = kv_lens[t0 + min(lane, nt - 1)];
+  uint64_t left = nt >= 64 ? ~0ull : (1ull << nt) - 1;
+  while (left) {   // block-table rows of the tile; each pass takes at least one token off `left`
+    const int bt_row = __builtin_amdgcn_readlane(tl_row, __builtin_ctzll(left));
+    const bool same = ((left >> lane) & 1) && tl_row == bt_row;
+    left &= ~__ballot(same);
+    int Lmax = same ? tl_len : 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      s0[i] = (kbase + 4 * g + i < L) ? s0[i] * scale_log2 : OME_NEG_INF;
-      s1[i] = (kbase + 16 + 4 * g + i < L) ? s1[i] * scale_log2 : OME_NEG_INF;
-      mx = fmaxf(mx, fmaxf(s0[i], s1[i]));
-    }
-    mx = group4_max(mx);
-    const float m_new = fmaxf(m, mx);
-    const float alpha = (m_new == OME_NEG_INF) ? 1.f : __builtin_amdgcn_exp2f(m - m_new);
-    bf16x8 pb;
-    float ps = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float p0 = (m_new == OME_NEG_INF) ? 0.f : __builtin_amdgcn_exp2f(s0[i] - m_new);
-      const float p1 = (m_new == OME_NEG_INF) ? 0.f : __builtin_amdgcn_exp2f(s1[i] - m_new);
-      ps += p0 + p1;
-      pb[i] = (bf16)p0;
-      pb[4 + i] = (bf16)p1;
-    }
-    ps = group4_sum(ps);
-    lsum = lsum * alpha + ps;
-    m = m_new;
-    // ---- O^T [DV x 16 heads] += V^T . P^T (keys permuted as in pb: 4g + i, 16 + 4g + i) ----
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      const int off = vofs[nb & 3] + (nb >> 2) * 128;   // swz(4g + qrow, 2 nb + pcol/2) + 8 (pcol & 1)
-      const bf16x4 va = tr_read(img, off);
-      const bf16x4 vb = tr_read(img, off + 16 * CH * 16);
-      bf16x8 a;
-      a[0] = va[0]; a[1] = va[1]; a[2] = va[2]; a[3] = va[3];
-      a[4] = vb[0]; a[5] = vb[1]; a[6] = vb[2]; a[7] = vb[3];
-      o[nb] *= alpha;
-      o[nb] = mfma16x32(a, pb, o[nb]);
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next tile's DMA has landed
+    for (int x = 32; x > 0; x >>= 1) Lmax = max(Lmax, __shfl_xor(Lmax, x));
+    Lmax = __builtin_amdgcn_readfirstlane(Lmax);
+    const int* bt = block_tables + (int64_t)bt_row * bt_stride;
+    const int n_pages = (Lmax + 15) >> 4, tiles = (n_pages + 1) >> 1, per = (tiles + my_parts - 1) / my_parts;
+    const int begin = part * per, end = min(tiles, begin + per);
+    if (begin >= end) continue;
+    const int L = my_row == bt_row ? my_len : 0;
+
+    dma(bt, n_pages, begin, 0);
+    if (begin + 1 < end) dma(bt, n_pages, begin + 1, 1);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    buf ^= 1;
+    f32x16 sc = score(0);
+    int cur = 0;
+    for (int n = begin; n < end; ++n) {
+      const int nxt = cur == 2 ? 0 : cur + 1;
+      // image nxt + 1 was last read in the previous round, before its barrier
+      if (n + 2 < end) dma(bt, n_pages, n + 2, nxt == 2 ? 0 : nxt + 1);
+      const f32x16 sn = score(nxt * IMG);   // (after the last tile: of whatever is there, unused)
+      const int key = n * KT + 4 * hf;
+      float mx = OME_NEG_INF;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        sc[i] = key + 8 * (i >> 2) + (i & 3) < L ? sc[i] * scale_log2 : OME_NEG_INF;
+        mx = fmaxf(mx, sc[i]);
+      }
+      {
+        auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+        mx = vmax_f32(__uint_as_float(w[0]), __uint_as_float(w[1]));
+      }
+      const bool rise = mx > m + LAZY;   // (also a row's first tile: m = -inf)
+      const float mn = rise ? mx : m, ms = mn == OME_NEG_INF ? 0.f : mn;
+      float ps = 0.f;
+      bf16x8 pb[2];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        pb[i >> 3][i & 7] = (bf16)__builtin_amdgcn_exp2f(sc[i] - ms);
+        ps += (float)pb[i >> 3][i & 7];   // the weights as they are used: their rounding cancels in the quotient
+      }
+      {
+        auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(ps), __float_as_uint(ps), false, false);
+        ps = __uint_as_float(w[0]) + __uint_as_float(w[1]);
+      }
+      bf16x8 vf[AHEAD];
+#pragma unroll
+      for (int k = 0; k < AHEAD; ++k) vf[k] = vfrag(cur * IMG, k >> 1, k & 1);
+      if (__ballot(rise && m != OME_NEG_INF)) {   // (a first tile has nothing to rescale: O^T and the sum are zero)
+        const float alpha = rise && m != OME_NEG_INF ? __builtin_amdgcn_exp2f(m - mn) : 1.f;
+        lsum *= alpha;
+        // in the accumulation registers, by asm: as plain C++ all 256 products are computed every time and moved
+        // through the other registers.  (waits: the last MFMA's results; the next one's operands)
+        asm volatile(MMA_WAIT ::: "memory");
+#pragma unroll
+        for (int v = 0; v < NV; ++v)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            float x = o[v][i];
+#if defined(__HIP_DEVICE_COMPILE__)   // ("a": an accumulation register, unknown to the host pass)
+            float y;
+            asm volatile("v_accvgpr_read_b32 %1, %0\n\tv_mul_f32 %1, %1, %2\n\tv_accvgpr_write_b32 %0, %1"
+                         : "+a"(x), "=&v"(y)
+                         : "v"(alpha));
+#endif
+            o[v][i] = x;
+          }
+        asm volatile("s_nop 7" ::: "memory");
+      }
+      lsum += ps;
+      m = mn;
+      asm volatile("s_nop 3" : "+v"(pb[0]), "+v"(pb[1])::"memory");   // (written by the vector ALU just now)
+#pragma unroll
+      for (int k = 0; k < 2 * NV; ++k) {
+        mma_acc(o[k >> 1], vf[k % AHEAD], pb[k & 1]);
+        if (k + AHEAD < 2 * NV) vf[k % AHEAD] = vfrag(cur * IMG, (k + AHEAD) >> 1, k & 1);
+      }
+      sc = sn;
+      cur = nxt;
+      asm volatile(MMA_WAIT "\n\ts_waitcnt vmcnt(0)" ::: "memory");   // tile n + 2 has landed
+      __syncthreads();
+    }
   }
 
-  // ---- epilogue: O^T lane map dim = 16 nb + 4 g + i, head = col ----
+  // ---- epilogue: O^T lane map dim = 32 v + 8 (i / 4) + 4 hf + i % 4, row = col ----
   const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
-  if (parts == 1) {
-    bf16* op = out + (int64_t)t * out_stride_t + (int64_t)head * DV + 4 * g;
+  if (my_parts == 1 && NW == 4 && !decode) {
+    // through LDS (the images are done with): 32 rows x 256 dims at a time, so that rows leave in 512-byte runs
+    // instead of 8-byte pieces (prompts of 128-row tiles 3..5% faster; lower tiles and decode steps not)
+    constexpr int LD = DV / 2 + 8;   // padded row
+    static_assert(NW * 32 * LD * 2 <= (int)sizeof(sK), "the output fits the images");
+    bf16* so = reinterpret_cast<bf16*>(sK) + wave * 32 * LD;
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      bf16x4 v;
+    for (int half = 0; half < 2; ++half) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the first half's reads
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = (bf16)(o[nb][i] * inv);
-      *reinterpret_cast<bf16x4*>(op + 16 * nb) = v;
+      for (int v = 0; v < NV / 2; ++v)
+#pragma unroll
+        for (int i = 0; i < 16; i += 4) {
+          const f32x16& x = o[half * (NV / 2) + v];
+          *reinterpret_cast<bf16x4*>(so + col * LD + 32 * v + 2 * i + 4 * hf) =
+              bf16x4{(bf16)(x[i] * inv), (bf16)(x[i + 1] * inv), (bf16)(x[i + 2] * inv), (bf16)(x[i + 3] * inv)};
+        }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (a wave's own rows: no barrier)
+      for (int i = 0; i < 16; ++i) {
+        const int lr = 2 * i + hf, r = row0 + wave * 32 + lr;
+        if (r < row_end) {
+          const int tt = r / H;
+          st8(out + (int64_t)tt * out_stride_t + (int64_t)(r - tt * H) * DV + half * (DV / 2) + 8 * col, ld8(so + lr * LD + 8 * col));
+        }
+      }
     }
-  } else {
-    const int64_t ws_row = ((int64_t)t * H + head) * parts + part;
-    float* wp = ws_o + ws_row * DV + 4 * g;
+  } else if (my_parts == 1) {
+    if (!hv) return;
+    bf16* op = out + (int64_t)t * out_stride_t + (int64_t)head * DV + 4 * hf;
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-      *reinterpret_cast<f32x4*>(wp + 16 * nb) = f32x4{o[nb][0] * inv, o[nb][1] * inv, o[nb][2] * inv,
-                                                       o[nb][3] * inv};
-    if (g == 0) {
-      ws_ml[2 * ws_row] = m;
-      ws_ml[2 * ws_row + 1] = lsum;
+    for (int v = 0; v < NV; ++v)
+#pragma unroll
+      for (int i = 0; i < 16; i += 4)
+        *reinterpret_cast<bf16x4*>(op + 32 * v + 2 * i) = bf16x4{(bf16)(o[v][i] * inv), (bf16)(o[v][i + 1] * inv),
+                                                                 (bf16)(o[v][i + 2] * inv), (bf16)(o[v][i + 3] * inv)};
+  } else {   // partials in the lanes' own order: 1 KiB a store (mla_reduce_rows_kernel reads them so)
+    const int64_t slot = decode ? blockIdx.x : (int64_t)unit * parts + part;
+    float* wp = ws_o + (slot * NW + wave) * (32 * DV) + 4 * lane;
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+#pragma unroll
+      for (int i = 0; i < 16; i += 4)
+        *reinterpret_cast<f32x4*>(wp + (4 * v + i / 4) * 256) =
+            f32x4{o[v][i] * inv, o[v][i + 1] * inv, o[v][i + 2] * inv, o[v][i + 3] * inv};
+    if (hf == 0) {
+      ws_ml[2 * (slot * RT + wave * 32 + col)] = m;
+      ws_ml[2 * (slot * RT + wave * 32 + col) + 1] = lsum;
     }
   }
+}
+
+// Merge the partials of row tiles: a wave of (tile, 32 rows, 32 value dims) per quarter, lanes as the tile kernel's, 1 KiB a
+// load; partials eight at a time with their loads issued up front, as below.
+template <int DV, int NW>
+__global__ __launch_bounds__(256) void mla_reduce_rows_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
+                                                              int T, int H, int parts, const int2* __restrict__ plan,
+                                                              bf16* __restrict__ out, int64_t out_stride_t) {
+  constexpr int RT = 32 * NW;
+  const int unit = blockIdx.x / NW, wave = blockIdx.x % NW, v = blockIdx.y, qd = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int col = lane & 31, hf = lane >> 5, HG = (H + RT - 1) / RT;
+  int64_t base = (int64_t)unit * parts;
+  if (plan != nullptr) {
+    const int2 pl = plan[unit];
+    base = pl.x;
+    parts = pl.y;
+    if (parts == 1) return;   // written by its one piece
+  }
+  const int row = (plan ? unit / HG * H + unit % HG * RT : unit * RT) + wave * 32 + col;
+  if (row >= (plan ? (unit / HG + 1) * H : T * H)) return;
+  float M = OME_NEG_INF, den = 0.f;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int p0 = 0; p0 < parts; p0 += 8) {
+    float mm[8], ll[8];
+    f32x4 vv[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int64_t r = base + min(p0 + j, parts - 1);
+      mm[j] = ws_ml[2 * (r * RT + wave * 32 + col)];
+      ll[j] = p0 + j < parts ? ws_ml[2 * (r * RT + wave * 32 + col) + 1] : 0.f;
+      vv[j] = *reinterpret_cast<const f32x4*>(ws_o + (r * NW + wave) * (32 * DV) + (4 * v + qd) * 256 + 4 * lane);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (!(ll[j] > 0.f)) continue;
+      const float mn = fmaxf(M, mm[j]);
+      const float a = __builtin_amdgcn_exp2f(M - mn), w = ll[j] * __builtin_amdgcn_exp2f(mm[j] - mn);
+      acc = acc * a + w * vv[j];
+      den = den * a + w;
+      M = mn;
+    }
+  }
+  const float inv = den > 0.f ? 1.f / den : 0.f;
+  const int t = row / H;
+  *reinterpret_cast<bf16x4*>(out + (int64_t)t * out_stride_t + (int64_t)(row - t * H) * DV + 32 * v + 8 * qd + 4 * hf) =
+      bf16x4{(bf16)(acc[0] * inv), (bf16)(acc[1] * inv), (bf16)(acc[2] * inv), (bf16)(acc[3] * inv)};
 }
 
 // merge split-K partitions: one workgroup per (token, head), DV / 4 threads x 4 dims.  Partitions
@@ -413,54 +643,53 @@ __global__ __launch_bounds__(128) void mla_reduce_kernel(const float* __restrict
 template <int DK, int DV>
 static void mla_launch(const void* q, int64_t q_stride_t, const void* cache, const int* block_tables, int bt_stride,
                        const int* tok_row, const int* kv_lens, int T, int H, float scale_log2, int parts, void* out,
-                       int64_t out_stride_t, float* ws_o, float* ws_ml, hipStream_t stream,
-                       const float* sinks = nullptr, int window = -1) {
-  // all-heads kernel when the heads tile into groups of 128 (DeepSeek-V3 / Kimi-K2 at TP 1) or 64
-  // (TP 2): one latent stream per token and partition; else the 16-head kernel.  OME_MLA_ALL=0
-  // forces the 16-head kernel (A/B timing).  Batches of at most OME_MLA_ALL_MIN_T tokens (default
-  // 2) also take the 16-head kernel: the all-heads kernel's fixed cost (Q load, first DMA, fp32
-  // partials + reduce) loses at T = 1 / 2 (41.0 / 40.1 vs 35.2 / 36.0 us) and wins from T = 4
-  // (43.1 vs 61.4 us) -- profiles/r06_mla_cutover.txt.
-  static const bool all_env = !getenv("OME_MLA_ALL") || atoi(getenv("OME_MLA_ALL")) != 0;
-  static const int min_t = getenv("OME_MLA_ALL_MIN_T") ? atoi(getenv("OME_MLA_ALL_MIN_T")) : 2;
-  const bool all_ok = all_env && T > min_t;
-  bool done = false;
+                       int64_t out_stride_t, float* ws_o, float* ws_ml, hipStream_t stream, int rows = 0,
+                       int2* plan = nullptr, const float* sinks = nullptr, int window = -1) {
+  // `rows`: query rows of a workgroup of the row-tile kernel (32 / 64 / 128, the caller's choice), 0: the
+  // 16-head kernel, which alone has the sink term and the window
   if constexpr (DK == 576) {
-    if (sinks != nullptr || window > 0) {
-      // (the all-heads kernel has no sink term and no window: these take the 16-head kernel)
-    } else if (all_ok && H % 128 == 0) {
-      mla_attn_all_kernel<DK, DV, 8><<<dim3(T, H / 128, parts), 512, 0, stream>>>(
-          (const bf16*)q, q_stride_t, (const bf16*)cache, block_tables, bt_stride, tok_row, kv_lens, H, scale_log2,
-          parts, (bf16*)out, out_stride_t, ws_o, ws_ml);
-      done = true;
-    } else if (all_ok && H % 64 == 0) {
-      mla_attn_all_kernel<DK, DV, 4><<<dim3(T, H / 64, parts), 256, 0, stream>>>(
-          (const bf16*)q, q_stride_t, (const bf16*)cache, block_tables, bt_stride, tok_row, kv_lens, H, scale_log2,
-          parts, (bf16*)out, out_stride_t, ws_o, ws_ml);
-      done = true;
+    if (rows > 0) {
+      const unsigned units = (unsigned)(plan ? T * ((H + rows - 1) / rows) : ((int64_t)T * H + rows - 1) / rows);
+      const dim3 grid(plan && parts > 1 ? 256 : units, plan ? 1 : parts);
+#define MLA_ROWS(NW)                                                                                                    \
+  {                                                                                                                      \
+    mla_attn_rows_kernel<DK, DV, NW><<<grid, 64 * NW, 0, stream>>>(                                                      \
+        (const bf16*)q, q_stride_t, (const bf16*)cache, block_tables, bt_stride, tok_row, kv_lens, T, H, scale_log2,      \
+        parts, plan, (bf16*)out, out_stride_t, ws_o, ws_ml);                                                             \
+    if (parts > 1)                                                                                                       \
+      mla_reduce_rows_kernel<DV, NW><<<dim3(units * NW, DV / 32), 256, 0, stream>>>(ws_o, ws_ml, T, H, parts, plan,       \
+                                                                                    (bf16*)out, out_stride_t);            \
+  }
+      if (rows == 128) MLA_ROWS(4)
+      else if (rows == 64) MLA_ROWS(2)
+      else MLA_ROWS(1)
+#undef MLA_ROWS
+      return;
     }
   }
-  if (!done)
-    mla_attn_kernel<DK, DV><<<dim3(T, (H + 15) / 16, parts), 256, 0, stream>>>(
-        (const bf16*)q, q_stride_t, (const bf16*)cache, block_tables, bt_stride, tok_row, kv_lens, H, scale_log2,
-        parts, (bf16*)out, out_stride_t, ws_o, ws_ml, sinks, window);
+  mla_attn_kernel<DK, DV><<<dim3(T, (H + 15) / 16, parts), 256, 0, stream>>>(
+      (const bf16*)q, q_stride_t, (const bf16*)cache, block_tables, bt_stride, tok_row, kv_lens, H, scale_log2,
+      parts, (bf16*)out, out_stride_t, ws_o, ws_ml, sinks, window);
   if (parts > 1)
     mla_reduce_kernel<DV><<<dim3(T, H), DV / 4, 0, stream>>>(ws_o, ws_ml, H, parts, (bf16*)out, out_stride_t, sinks);
 }
 
 OME_API int ome_mla_attn(const void* q, int64_t q_stride_t, const void* cache, const int* block_tables,
                          int bt_stride, const int* tok_row, const int* kv_lens, int T, int H, int dk, int dv,
-                         float scale, int parts, void* out, int64_t out_stride_t, float* ws_o, float* ws_ml,
-                         hipStream_t stream) {
+                         float scale, int parts, int rows, void* plan, void* out, int64_t out_stride_t, float* ws_o,
+                         float* ws_ml, hipStream_t stream) {
   if (T <= 0) return 0;
+  if ((rows != 0 && rows != 32 && rows != 64 && rows != 128) || (int64_t)T * H > 0x7fffff00 || parts > 65535) return -2;
+  if (rows != 0 && (dk != 576 || dv != 512 || H < 4 || (uintptr_t)out % 16 || out_stride_t % 8)) return -2;
+  if (plan && (rows == 0 || (parts > 1 && (int64_t)T * ((H + rows - 1) / rows) > 256))) return -2;   // (256 pieces)
   if (H <= 0 || parts < 1 || (parts > 1 && (!ws_o || !ws_ml))) return -2;
   const float scale_log2 = scale * 1.4426950408889634f;
   if (dk == 576 && dv == 512)
     mla_launch<576, 512>(q, q_stride_t, cache, block_tables, bt_stride, tok_row, kv_lens, T, H, scale_log2, parts, out,
-                         out_stride_t, ws_o, ws_ml, stream);
+                         out_stride_t, ws_o, ws_ml, stream, rows, (int2*)plan);
   else if (dk == 288 && dv == 256)
     mla_launch<288, 256>(q, q_stride_t, cache, block_tables, bt_stride, tok_row, kv_lens, T, H, scale_log2, parts, out,
-                         out_stride_t, ws_o, ws_ml, stream);
+                         out_stride_t, ws_o, ws_ml, stream, rows, (int2*)plan);
   else
     return -3;
   OME_CHECK_LAUNCH();
@@ -475,15 +704,19 @@ OME_API int ome_mla_attn(const void* q, int64_t q_stride_t, const void* cache, c
 // the caller.
 OME_API int ome_latent_attn(const void* q, int64_t q_stride_t, const void* cache, const int* block_tables,
                             int bt_stride, const int* tok_row, const int* kv_lens, int T, int H, int dk, int dv,
-                            float scale, int parts, void* out, int64_t out_stride_t, float* ws_o, float* ws_ml,
-                            const float* sinks, int window, hipStream_t stream) {
+                            float scale, int parts, int rows, void* plan, void* out, int64_t out_stride_t, float* ws_o,
+                            float* ws_ml, const float* sinks, int window, hipStream_t stream) {
   if (T <= 0) return 0;
+  if ((rows != 0 && rows != 32 && rows != 64 && rows != 128) || (int64_t)T * H > 0x7fffff00 || parts > 65535) return -2;
+  if (rows != 0 && (sinks || window > 0)) return -2;
+  if (rows != 0 && (dk != 576 || dv != 512 || H < 4 || (uintptr_t)out % 16 || out_stride_t % 8)) return -2;
+  if (plan && (rows == 0 || (parts > 1 && (int64_t)T * ((H + rows - 1) / rows) > 256))) return -2;   // (256 pieces)
   if (H <= 0 || parts < 1 || (parts > 1 && (!ws_o || !ws_ml))) return -2;
   const float scale_log2 = scale * 1.4426950408889634f;
 #define LATENT_CASE(DK_, DV_)                                                                                       \
   if (dk == DK_ && dv == DV_) {                                                                                     \
     mla_launch<DK_, DV_>(q, q_stride_t, cache, block_tables, bt_stride, tok_row, kv_lens, T, H, scale_log2, parts,  \
-                         out, out_stride_t, ws_o, ws_ml, stream, sinks, window);                                    \
+                         out, out_stride_t, ws_o, ws_ml, stream, rows, (int2*)plan, sinks, window);                                \
     OME_CHECK_LAUNCH();                                                                                             \
     return 0;                                                                                                       \
   }

@@ -943,15 +943,18 @@ def _sinks(s: torch.Tensor | None):
     return s.data_ptr()
 
 
+_MLA_ROW_TILES = os.environ.get("OME_MLA_ALL", "1") != "0"   # 0: the 16-head kernel everywhere (A/B timing)
+
+
 class MLAWorkspace:
     """Split-K partials for :func:`mla_attn` (``ws_o`` [rows, 512] f32, ``ws_ml`` [rows, 2]; rows =
     tokens x heads x partitions, bounded by ``ROWS``).
 
-    Two kernels (``mla.hip``): the all-heads kernel (DK 576 with 64 | H: one workgroup streams a
-    token's latent KV once for 64 / 128 heads, one workgroup per CU) and the 16-head kernel (MiniCPM3
-    shapes, TP-sharded head counts).  Partitions lift the grid towards ~1 workgroup per CU (all-heads)
-    or ~1024 workgroups (16-head), and never beyond what the f32 partials' HBM round trip repays:
-    large decode batches (T x H / 128 >= 256) run unsplit."""
+    Two kernels (``mla.hip``): row tiles (:meth:`rows`: one workgroup, one to a CU, streams the latent KV once
+    for 32 / 64 / 128 query rows) and the 16-head kernel (other widths, sinks, windows).  Row tiles of prompts are
+    cut into equal partitions up to ~1 workgroup per CU; those of decode steps by the kernel itself, by their
+    lengths, into at most 256 pieces (``plan``: each tile's first partial and piece count).  The 16-head
+    kernel takes partitions up to ~1024 workgroups.  None beyond what the f32 partials' HBM round trip repays."""
 
     TARGET_WGS = 1024
     TARGET_WGS_ALL = 256
@@ -962,22 +965,40 @@ class MLAWorkspace:
     def __init__(self, device="cuda"):
         self.ws_o = torch.empty(self.ROWS * 512, dtype=torch.float32, device=device)
         self.ws_ml = torch.empty(self.ROWS * 2, dtype=torch.float32, device=device)
-
-    @staticmethod
-    def all_heads(H: int, DK: int = 576, T: int = 1 << 30) -> bool:
-        """Mirror of mla.hip's kernel choice (same env knobs): all-heads only above
-        ``OME_MLA_ALL_MIN_T`` (default 2) tokens -- T = 1 / 2 keep the 16-head kernel."""
-        return (DK == 576 and H % 64 == 0 and os.environ.get("OME_MLA_ALL", "1") != "0"
-                and T > int(os.environ.get("OME_MLA_ALL_MIN_T", "2")))
+        self.plan = torch.empty(self.TARGET_WGS_ALL, 2, dtype=torch.int32, device=device)
 
     @classmethod
-    def parts(cls, T: int, H: int, DK: int = 576) -> int:
-        if cls.all_heads(H, DK, T):
-            wgs = T * (H // (128 if H % 128 == 0 else 64))
-            p = max(1, min(cls.MAX_PARTS_ALL, cls.TARGET_WGS_ALL // max(wgs, 1)))
-        else:
-            wgs = T * -(-H // 16)
-            p = 1 if wgs >= cls.TARGET_WGS else max(1, min(cls.MAX_PARTS, cls.TARGET_WGS // max(wgs, 1)))
+    def rows(cls, T: int, H: int, DK: int = 576, seqs: int = 1 << 30, pages: int = 1 << 30) -> tuple[int, bool]:
+        """(query rows of a row tile or 0 for the 16-head kernel, whether its tiles are heads of one token) for T
+        tokens of ``seqs`` block-table rows of ``pages`` pages (a bound of every context).  Prompts (at least 4
+        tokens a sequence): rows of neighbouring tokens share a tile.  Taller tiles do more work per LDS read, lower
+        ones start sooner and fill the chip with fewer rows; the fixed cost of a row tile (12..20 us, the
+        16-head kernel 10) loses where there is little to stream.  Device times, 16-head / row tiles: prompts, 16 heads,
+        30 x 30 12 / 21 us, 25 rows at 2000 keys 48 / 32, 120 x 60 25 / 24, 3400 x 1300 750 / 129; decode, 32 heads,
+        8 x 100 keys 11 / 15, 4 x 3000 41 / 31, 48 x 3000 196 / 69; 16 heads, 4 x 3000 21 / 26, 48 x 3000
+        105 / 65; 128 heads, 1 x 500 14 / 15, 8 x 100 23 / 17, 48 x 3000 104 (the tiles before) / 76."""
+        n = T * H
+        if DK != 576 or H < 4 or not _MLA_ROW_TILES:
+            return 0, False
+        if T >= 4 * seqs:
+            if n < (1024 if pages <= 32 else 256):
+                return 0, False
+            return (128 if n >= 128 * cls.TARGET_WGS_ALL else 64 if n >= 64 * cls.TARGET_WGS_ALL else 32), False
+        if n < (384 if H < 32 else 192) or (H <= 32 and pages <= 16 and n < 1024):
+            return 0, False
+        return (128 if H > 64 and T >= 16 else 64 if H > 32 and n >= 512 else 32), True
+
+    @classmethod
+    def parts(cls, T: int, H: int, DK: int = 576, rows: int = 0, decode: bool = False) -> int:
+        """Partitions of a tile's keys; for the row tiles of a decode step the most that a tile may get."""
+        if rows and decode:
+            units = T * -(-H // rows)
+            return 1 if units > cls.TARGET_WGS_ALL else min(cls.MAX_PARTS_ALL, -(-2 * cls.TARGET_WGS_ALL // units))
+        if rows:
+            wgs = -(-T * H // rows)
+            return max(1, min(cls.MAX_PARTS_ALL, cls.TARGET_WGS_ALL // wgs, cls.ROWS // (wgs * rows)))
+        wgs = T * -(-H // 16)
+        p = 1 if wgs >= cls.TARGET_WGS else max(1, min(cls.MAX_PARTS, cls.TARGET_WGS // max(wgs, 1)))
         return max(1, min(p, cls.ROWS // max(T * H, 1)))
 
 
@@ -998,13 +1019,16 @@ def mla_attn(q, cache, block_tables, tok_row, kv_lens, scale: float, ws: MLAWork
     assert q.stride(2) == 1 and q.stride(1) == DK and cache.shape[-1] == DK
     if out is None:
         out = torch.empty(T, H, dv, dtype=q.dtype, device=q.device)
-    parts = MLAWorkspace.parts(T, H, DK)
-    if parts > 1 and ws is None:
+    rows, decode = MLAWorkspace.rows(T, H, DK, *block_tables.shape)
+    if out.data_ptr() % 16 or out.stride(0) % 8:
+        rows, decode = 0, False
+    parts = MLAWorkspace.parts(T, H, DK, rows, decode)
+    if ws is None and (parts > 1 or decode):
         ws = MLAWorkspace(q.device)
     call("ome_mla_attn", q.data_ptr(), q.stride(0), cache.data_ptr(), _i32(block_tables).data_ptr(),
          block_tables.stride(0), _i32(tok_row).data_ptr(), _i32(kv_lens).data_ptr(), T, H, DK, dv, float(scale),
-         parts, out.data_ptr(), out.stride(0), ws.ws_o.data_ptr() if parts > 1 else None,
-         ws.ws_ml.data_ptr() if parts > 1 else None, stream_ptr())
+         parts, rows, ws.plan.data_ptr() if decode else None, out.data_ptr(), out.stride(0),
+         ws.ws_o.data_ptr() if parts > 1 else None, ws.ws_ml.data_ptr() if parts > 1 else None, stream_ptr())
     return out
 
 
@@ -1894,17 +1918,19 @@ def latent_attn(q, cache, block_tables, tok_row, kv_lens, scale: float, dv: int,
     if out is None:
         out = torch.empty(T, H, dv, dtype=q.dtype, device=q.device)
     assert out.stride(2) == 1 and out.stride(1) == dv
-    parts = MLAWorkspace.parts(T, H, DK)
-    if (sinks is not None or window > 0) and DK == 576:   # (these run the 16-head kernel: partition as it does)
-        parts = MLAWorkspace.parts(T, H, 0)
+    rows, decode = MLAWorkspace.rows(T, H, DK, *block_tables.shape)
+    if sinks is not None or window > 0 or out.data_ptr() % 16 or out.stride(0) % 8:
+        rows, decode = 0, False
+    parts = MLAWorkspace.parts(T, H, DK, rows, decode)
     if window > 0:   # at least four 32-key tiles of the window per partition (fewer only move partials around)
         parts = max(1, min(parts, window // 128))
-    if parts > 1 and ws is None:
+    if ws is None and (parts > 1 or decode):
         ws = MLAWorkspace(q.device)
     call("ome_latent_attn", q.data_ptr(), q.stride(0), cache.data_ptr(), _i32(block_tables).data_ptr(),
          block_tables.stride(0), _i32(tok_row).data_ptr(), _i32(kv_lens).data_ptr(), T, H, DK, dv, float(scale),
-         parts, out.data_ptr(), out.stride(0), ws.ws_o.data_ptr() if parts > 1 else None,
-         ws.ws_ml.data_ptr() if parts > 1 else None, _sinks(sinks), int(window), stream_ptr())
+         parts, rows, ws.plan.data_ptr() if decode else None, out.data_ptr(), out.stride(0),
+         ws.ws_o.data_ptr() if parts > 1 else None, ws.ws_ml.data_ptr() if parts > 1 else None, _sinks(sinks),
+         int(window), stream_ptr())
     return out
 
 

@@ -2,9 +2,8 @@
 cached tokens each, H = 128 heads, DK = 576 / DV = 512 latent rows.  Prints one JSON line per shape
 with microseconds per call and the effective latent-KV read bandwidth (every sequence's KV once).
 
-    python scripts/mla_bench.py                 # all-heads kernel
+    python scripts/mla_bench.py                 # row tiles
     OME_MLA_ALL=0 python scripts/mla_bench.py   # 16-head kernel (A/B)
-    OME_MLA_ALL_MIN_T=0 python scripts/mla_bench.py   # all-heads even at T <= 4 (A/B of the cutover)
 """
 import json
 import os
@@ -38,9 +37,9 @@ def run(T, L, H=128, iters=50):
     us = e0.elapsed_time(e1) * 1e3 / iters
     kv = T * L * 576 * 2
     flops = 2 * T * H * L * (576 + 512)
-    return {"T": T, "L": L, "H": H, "parts": ops.MLAWorkspace.parts(T, H), "us": round(us, 1),
+    return {"T": T, "L": L, "H": H, "parts": ops.MLAWorkspace.parts(T, H, 576, *ops.MLAWorkspace.rows(T, H)), "us": round(us, 1),
             "kv_GBps": round(kv / us / 1e3, 1), "TFLOPs": round(flops / us / 1e6, 1),
-            "kernel": "all-heads" if ops.MLAWorkspace.all_heads(H, 576, T) else "16-head"}
+            "kernel": "row tiles" if ops.MLAWorkspace.rows(T, H)[0] else "16-head"}
 
 
 if __name__ == "__main__":

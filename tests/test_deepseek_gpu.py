@@ -151,3 +151,49 @@ def test_mla_prep_matches_reference(qlr, lat, rope, H, nope):
     assert (f1 - f0).abs().max().item() <= 2e-2 * max(1.0, f0.abs().max().item())
     assert (q1[:, :, lat:] - q0[:, :, lat:]).abs().max().item() <= 2e-2 * max(1.0, q0.abs().max().item())
     assert f1[0].abs().sum() > 0   # the padding row landed in the scratch row
+
+
+def _exact(q, cache, bt, rows, kl, scale):
+    """Attention in 64 bits, token by token."""
+    out = torch.zeros(q.shape[0], q.shape[1], 512, dtype=torch.float64)
+    q, cache, bt = q.cpu().double(), cache.cpu().double().view(-1, 576), bt.cpu().long()
+    for t, (r, n) in enumerate(zip(rows.tolist(), kl.tolist())):
+        at = torch.arange(n)
+        kv = cache[bt[r][at // 16] * 16 + at % 16]
+        out[t] = (q[t] @ kv.T * scale).softmax(-1) @ kv[:, :512] if n else 0
+    return out
+
+
+@pytest.mark.parametrize("rows", [0, 32, 64, 128])
+@pytest.mark.parametrize("H", [16, 20, 64, 128])
+@pytest.mark.parametrize("seqs", [[(1, 1), (33, 33), (0, 40)], [(70, 9), (5, 3), (0, 1), (31, 34)], [(700, 30)]], ids=str)
+def test_mla_row_tiles_of_prompts(monkeypatch, seqs, H, rows):
+    """(cached tokens, new tokens) per sequence: tiles that end inside a token's heads, hold several sequences, or
+    are cut into partitions; contexts around whole key tiles and pages."""
+    torch.manual_seed(H)
+    cache, bt = _setup([a + n for a, n in seqs])
+    row = torch.tensor([s for s, (_, n) in enumerate(seqs) for _ in range(n)], dtype=torch.int32)
+    kl = torch.tensor([a + j + 1 for a, n in seqs for j in range(n)], dtype=torch.int32)
+    q = torch.randn(len(row), H, 576, device=DEV).to(torch.bfloat16)
+    monkeypatch.setattr(ops.MLAWorkspace, "rows", classmethod(lambda cls, *a: (rows, False)))
+    out = ops.mla_attn(q, cache, bt, row.to(DEV), kl.to(DEV), 0.06)
+    want = _exact(q, cache, bt, row, kl, 0.06)
+    # probabilities and the output are rounded to bf16 once each: 2^-9 of the largest value they sum, and of the result
+    assert (out.cpu().double() - want).abs().max() < 2.0 ** -8 * cache.float().abs().max().item()
+
+
+@pytest.mark.parametrize("rows", [32, 64, 128])
+@pytest.mark.parametrize("H", [16, 32, 64, 128])
+@pytest.mark.parametrize("lens", [[1, 0, 32, 33], [5000, 16, 700], [200, 31, 64, 65, 1] * 13, [40] * 260, list(range(1, 257))],
+                         ids=lambda v: f"{len(v)}x{max(v)}")
+def test_mla_row_tiles_of_decode_steps(monkeypatch, lens, H, rows):
+    """Contexts cut by length into at most 256 pieces: empty and single-key ones, one long among short, as many tokens
+    as pieces, more."""
+    torch.manual_seed(len(lens))
+    cache, bt = _setup(lens)
+    q = torch.randn(len(lens), H, 576, device=DEV).to(torch.bfloat16)
+    row, kl = torch.arange(len(lens), dtype=torch.int32), torch.tensor(lens, dtype=torch.int32)
+    monkeypatch.setattr(ops.MLAWorkspace, "rows", classmethod(lambda cls, *a: (rows, True)))
+    out = ops.mla_attn(q, cache, bt, row.to(DEV), kl.to(DEV), 0.06)
+    want = _exact(q, cache, bt, row, kl, 0.06)
+    assert (out.cpu().double() - want).abs().max() < 2.0 ** -8 * cache.float().abs().max().item()
