@@ -707,6 +707,27 @@ def moe_tile_m(rows: int, E: int, N: int) -> int:
     return 64
 
 
+#: average rows per expert from which the 256-row ping-pong tiles run (:func:`_moe_pp`).  Whole layer, 64 / 128-row
+#: tiles -> these: Mixtral 64 rows 790 -> 798 us, 100 800 -> 770, 128 983 -> 775, 250 1429 -> 1018, 750 3529 ->
+#: 2042; Nemotron-3-Nano (widths 2688 / 1856) 94 780 -> 689, 140 975 -> 829; Qwen3-Next 59 953 -> 924.
+MOE_PP_ROWS = 80
+
+
+def _moe_pp(x: torch.Tensor, ids: torch.Tensor | None, div: int, w: torch.Tensor, offsets: torch.Tensor, rows: int,
+            bias: torch.Tensor | None, silu: bool) -> torch.Tensor | None:
+    """Grouped GEMM on 256-row tiles (``ome_moe_gemm_pp``; ``silu``: SiLU(gate) * up applied to the accumulators),
+    or None where the 64 / 128-row tiles run: experts with few rows, shapes the tiles do not take, ``OME_MOE_TILE``."""
+    E, N, K = w.shape
+    if rows < MOE_PP_ROWS * E or os.environ.get("OME_MOE_TILE") or K % 64 or N % (32 if silu else 4) or (silu and bias is not None) or \
+            x.stride(0) % 8 or x.stride(1) != 1 or (x.data_ptr() | w.data_ptr()) % 16 or not w.is_contiguous() or \
+            x.shape[0] * x.stride(0) >= 1 << 30 or N * K >= 1 << 30:
+        return None
+    out = torch.empty(rows, N // 2 if silu else N, dtype=x.dtype, device=x.device)
+    call("ome_moe_gemm_pp", x.data_ptr(), x.stride(0), x.shape[0], ptr(ids), div, w.data_ptr(), offsets.data_ptr(), E, N, K,
+         rows, out.data_ptr(), out.stride(0), ptr(bias), 2 if silu else 0, stream_ptr())
+    return out
+
+
 def moe_fp8_tile_m(rows: int, E: int) -> int:
     """Row tile of the fp8 grouped GEMM: 64 (64x128 tiles, 3-stage LDS ring) at every size, or
     128 (128x128, 2 stages) via ``OME_MOE_FP8_TILE=128``.  Measured (``scripts/fp8_moe_tile_bench.py``,
@@ -745,15 +766,22 @@ def fused_moe(x: torch.Tensor, topk_w: torch.Tensor, topk_ids: torch.Tensor, w13
     inv = torch.empty(n, dtype=torch.int32, device=dev)
     call("ome_moe_align", topk_ids.data_ptr(), n, E, offsets.data_ptr(), sorted_ids.data_ptr(), inv.data_ptr(),
          stream_ptr())
-    tm = moe_tile_m(n, E, I2)
-    gu = torch.empty(n, I2, dtype=x.dtype, device=dev)
-    call("ome_moe_gemm", x.data_ptr(), x.stride(0), sorted_ids.data_ptr(), k, w13.data_ptr(), offsets.data_ptr(),
-         E, I2, H, -(-n // tm) + E, gu.data_ptr(), gu.stride(0), ptr(b13), tm, stream_ptr())
-    h = act_and_mul(gu, act, limit=limit) if gated else _act_inplace(gu, act)
-    y = torch.empty(n, H, dtype=x.dtype, device=dev)
-    tm = moe_tile_m(n, E, H)
-    call("ome_moe_gemm", h.data_ptr(), h.stride(0), None, 0, w2.data_ptr(), offsets.data_ptr(), E, H, I,
-         -(-n // tm) + E, y.data_ptr(), y.stride(0), ptr(b2), tm, stream_ptr())
+    fused = gated and act == 0 and b13 is None
+    h = _moe_pp(x, sorted_ids, k, w13, offsets, n, b13, fused)
+    if h is None:
+        fused = False
+        tm = moe_tile_m(n, E, I2)
+        h = torch.empty(n, I2, dtype=x.dtype, device=dev)
+        call("ome_moe_gemm", x.data_ptr(), x.stride(0), sorted_ids.data_ptr(), k, w13.data_ptr(), offsets.data_ptr(),
+             E, I2, H, -(-n // tm) + E, h.data_ptr(), h.stride(0), ptr(b13), tm, stream_ptr())
+    if not fused:
+        h = act_and_mul(h, act, limit=limit) if gated else _act_inplace(h, act)
+    y = _moe_pp(h, None, 1, w2, offsets, n, b2, False)
+    if y is None:
+        y = torch.empty(n, H, dtype=x.dtype, device=dev)
+        tm = moe_tile_m(n, E, H)
+        call("ome_moe_gemm", h.data_ptr(), h.stride(0), None, 0, w2.data_ptr(), offsets.data_ptr(), E, H, I,
+             -(-n // tm) + E, y.data_ptr(), y.stride(0), ptr(b2), tm, stream_ptr())
     return _combine(y, topk_w, inv, T, k, H, scale, add)
 
 

@@ -56,3 +56,36 @@ def test_tiny_moe_engine_graphs():
     b = [r.output_ids for r in e.generate(prompts, sp)]
     match = sum(x == y for x, y in zip(a, b))
     assert match >= 5, (a, b)  # bf16 batch-shape differences may flip a rare near-tie
+
+
+@pytest.mark.parametrize("counts", [[1, 0, 255, 257, 0, 512, 3], [40] * 70, [0, 0, 700]], ids=lambda c: f"{len(c)}x{max(c)}")
+@pytest.mark.parametrize("H,I", [(256, 128), (192, 224), (128, 1856)])
+@pytest.mark.parametrize("kind", ["silu", "gelu", "bias", "relu2"])
+def test_moe_prompt_tiles(monkeypatch, counts, H, I, kind):
+    """256-row tiles: empty experts, tiles of one row and of all, more experts than lanes, widths that end inside a
+    tile, every epilogue."""
+    torch.manual_seed(H + I)
+    E, n = len(counts), sum(counts)
+    bf = lambda *s: torch.randn(*s, device=DEV).to(torch.bfloat16)  # noqa: E731
+    gated = kind != "relu2"
+    x, w13, w2 = bf(n, H + 8)[:, 8:], bf(E, 2 * I if gated else I, H) * 0.1, bf(E, H, I) * 0.1
+    b13, b2 = (bf(E, 2 * I), bf(E, H)) if kind == "bias" else (None, None)
+    ids = torch.cat([torch.full((c,), e, dtype=torch.int32) for e, c in enumerate(counts)])[torch.randperm(n)].to(DEV)[:, None]
+    tw = torch.rand(n, 1, device=DEV)
+    monkeypatch.setattr(ops, "MOE_PP_ROWS", 0)
+    act = {"silu": 0, "gelu": 1, "bias": 0, "relu2": 4}[kind]
+    got = ops.fused_moe(x, tw, ids.contiguous(), w13, w2, act, 1.0, b13, b2, gated).cpu().double()
+    d = lambda t: t.cpu().double()  # noqa: E731
+    want = torch.zeros(n, H, dtype=torch.float64)
+    for e in range(E):
+        r = (ids[:, 0] == e).nonzero()[:, 0].cpu()
+        h = d(x)[r] @ d(w13[e]).T + (d(b13[e]) if b13 is not None else 0)
+        if gated:
+            g = h[:, :I]
+            h = (torch.nn.functional.gelu(g, approximate="tanh") if kind == "gelu" else g * g.sigmoid()) * h[:, I:]
+        else:
+            h = h.clamp(min=0).square()
+        want[r] = (h @ d(w2[e]).T + (d(b2[e]) if b2 is not None else 0)) * d(tw)[r]
+    # bf16 roundings of the intermediate (two where the activation is a pass of its own), the expert's row and the output
+    assert ((got - want).norm() / want.norm()).item() < 2.0 ** -7
+    assert torch.isfinite(got).all()
