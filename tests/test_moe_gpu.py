@@ -89,3 +89,36 @@ def test_moe_prompt_tiles(monkeypatch, counts, H, I, kind):
     # bf16 roundings of the intermediate (two where the activation is a pass of its own), the expert's row and the output
     assert ((got - want).norm() / want.norm()).item() < 2.0 ** -7
     assert torch.isfinite(got).all()
+
+
+@pytest.mark.parametrize("E,k", [(1, 1), (64, 64), (65, 3), (200, 70), (512, 10)])
+def test_moe_route_picks_in_order(E, k):
+    """Ties go to the lower expert, zeros of both signs are ties, minus infinity comes last, NaN never (an expert
+    id comes out all the same); also with more picks than lanes."""
+    torch.manual_seed(E)
+    logits = torch.randint(-3, 4, (9, E)).float()
+    logits[1], logits[2], logits[3] = 0.0, -0.0, float("-inf")
+    logits[2, ::2] = 0.0
+    logits[4, E // 2:] = float("-inf")
+    w, ids = (t.cpu() for t in ops.moe_route(logits.to(DEV), k, True, "sigmoid"))
+    order = torch.sort(logits, dim=1, descending=True, stable=True).indices[:, :k]
+    assert torch.equal(ids.long(), order)
+    s = logits.double().sigmoid().gather(1, order)
+    assert torch.allclose(w.double(), s / (s.sum(1, keepdim=True) + 1e-20), rtol=1e-5, atol=1e-7)
+    nan = torch.full((2, E), float("nan"))
+    nan[1, E // 2] = 1.0
+    _, ids = ops.moe_route(nan.to(DEV), k, True, "sigmoid")
+    assert ids[1, 0].item() == E // 2 and ((ids >= 0) & (ids < E)).all()
+
+
+@pytest.mark.parametrize("E", [1, 64, 1023, 1024, 1025, 3000])
+@pytest.mark.parametrize("n", [1, 5000])
+def test_moe_align_offsets(E, n):
+    torch.manual_seed(E + n)
+    ids = torch.randint(0, E, (n,), dtype=torch.int32, device=DEV)
+    off, srt, inv = (torch.full((s,), -1, dtype=torch.int32, device=DEV) for s in (E + 1, n, n))
+    ops.call("ome_moe_align", ids.data_ptr(), n, E, off.data_ptr(), srt.data_ptr(), inv.data_ptr(), ops.stream_ptr())
+    count = torch.bincount(ids.cpu().long(), minlength=E)
+    assert torch.equal(off.cpu().long(), torch.cat([torch.zeros(1, dtype=torch.long), count.cumsum(0)]))
+    assert torch.equal(ids[srt.long()].cpu(), ids.cpu().sort().values)
+    assert torch.equal(srt[inv.long()].cpu(), torch.arange(n, dtype=torch.int32))
