@@ -9,9 +9,19 @@
 //       (DELTA: P U = (P T) R, so that o and U both follow from R)
 //   S'  = g_C S + sum_i exp(cum_C - cum_i) k_i U_i^T
 //
-// Two launches.  chunk_gram_kernel, one wave per (chunk, head), parallel over all rows: the 32 x 32
-// matrices P (DELTA: P T) and T and the chunk's scalars, into a workspace.  chunk_rule_kernel walks the chunks of a
-// (sequence, head) in order: a wave owns 16 value columns and keeps its S in VGPR accumulators.
+// Two launches.  chunk_gram_kernel (Mamba-2: ssm_gram_kernel), parallel over all rows: the 32 x 32 matrices
+// P T and T (Mamba-2: q k^T, which the heads of a group share) and the chunk's scalars, into a workspace.
+// chunk_rule_kernel walks the chunks of a (sequence, head) in order: a wave owns 16 value columns and keeps its
+// S in VGPR accumulators.
+//
+// What bounds it: the chain of chunks.  Two waves a SIMD (S, one chunk's rows in flight and the split
+// parts fill the registers) share its matrix and vector units at about 60 matrix (DELTA: 96) and 500 vector
+// instructions a chunk, near 3 us with the latencies between them; its memory traffic hides behind that (leaving
+// the reads out gives 1%).  Per-head P, formed in the first launch, cost 40 us there and 108 in the scan
+// (Mamba-2, below): written and read back it is 16 times the bytes of its group's q k^T.
+//   gated delta rule, 32 heads of 128 x 128, prompts of 1001 / 1435 / 1564 rows:   24 + 123 us (row by row: 1098)
+//   selective scan, 128 heads of 64 x 128, 8 groups, 1033 / 926 / 1248 / 293 rows:  11 + 116 us (row by row: 1745)
+// Largest error of the state against 64 bits: 1.1e-7 (row by row: 2.0e-7) and 1.4e-7 (6.2e-7) of its norm.
 //
 // fp32 throughout: k and q enter the matrix cores as the bf16 values that they are (their norms, 1 / |k| and
 // 1 / (|q| sqrt(dk)), scale results), S and U as three bf16 parts that sum to the fp32 value exactly, at
@@ -27,9 +37,16 @@ constexpr int LDM = RC + 4;       // padded row of a 32 x 32 fp32 matrix in LDS
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// workspace of one (chunk, head): P (DELTA: P T), T (DELTA), then the vectors a, b, c, d [32] and g_C
+// workspace of one chunk.  DELTA, per head: P T, T, then the vectors a, b, c, d [32] and g_C.  Mamba-2, per group: q k^T
+// (its heads differ in their decays only, which the scan applies: P itself would be 16 times the bytes); then
+// per head the vectors a, cum's upper and lower parts, c, d and g_C.
+constexpr int NV_DELTA = 4 * RC + 4, NV_SSM = 5 * RC + 4;
 template <bool DELTA>
-constexpr int ws_floats() { return (DELTA ? 2 : 1) * RC * RC + 4 * RC + 4; }
+constexpr int vec_floats() { return DELTA ? NV_DELTA : NV_SSM; }
+template <bool DELTA>
+__host__ __device__ constexpr int64_t ws_floats(int H, int G) {
+  return DELTA ? (int64_t)H * (2 * RC * RC + NV_DELTA) : (int64_t)G * RC * RC + (int64_t)H * NV_SSM;
+}
 
 struct RuleArgs {
   const bf16 *q, *k, *v;          // rows of stride `stride` (v: v_stride)
@@ -105,10 +122,10 @@ __device__ __forceinline__ float softplus_rule(float x) { return x > 20.f ? x : 
 // k k^T (rows and columns of a 16 x 16 x 32 product have the same lane layout).  T by forward substitution: lane j
 // keeps column j in registers and reads the rows of A from LDS as broadcasts.
 // ---------------------------------------------------------------------------------------------
-template <int DK, bool DELTA>
+template <int DK>
 __global__ __launch_bounds__(256) void chunk_gram_kernel(RuleArgs a) {
   constexpr int NS = DK / 32;
-  __shared__ __attribute__((aligned(16))) float sA[4][DELTA ? RC * LDM : 4];
+  __shared__ __attribute__((aligned(16))) float sA[4][RC * LDM];
   __shared__ double s_cum[4][RC];
   __shared__ float s_vec[4][3][RC];   // 1 / |k|, 1 / (|q| sqrt(dk)), beta
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
@@ -116,7 +133,7 @@ __global__ __launch_bounds__(256) void chunk_gram_kernel(RuleArgs a) {
   int r0, n;
   if (h >= a.H || !chunk_of(blockIdx.x, a.cu, a.S, r0, n)) return;   // whole wave; no block barrier below
   const int hk = h / (a.H / a.Hk);
-  float* ws = a.ws + ((int64_t)blockIdx.x * a.H + h) * ws_floats<DELTA>();
+  float* ws = a.ws + ((int64_t)blockIdx.x * a.H + h) * (2 * RC * RC + NV_DELTA);
 
   bf16x8 kf[2][NS], qf[2][NS];
 #pragma unroll
@@ -131,17 +148,8 @@ __global__ __launch_bounds__(256) void chunk_gram_kernel(RuleArgs a) {
   // per-row scalars: lane i (and i + 32) holds row i
   const int row = lane & 31, rv = r0 + min(row, n - 1);
   const bool ok = row < n;
-  float ga, beta;   // log decay; beta (DELTA) or dt
-  {
-    const float av = (float)a.a[(int64_t)rv * a.ab_stride + h];
-    if constexpr (DELTA) {
-      ga = -__expf(a.A[h]) * softplus_rule(av + a.dt_bias[h]);
-      beta = 1.f / (1.f + __expf(-(float)a.b[(int64_t)rv * a.ab_stride + h]));
-    } else {
-      beta = fmaxf(softplus_rule(av + a.dt_bias[h]), a.dt_min);
-      ga = beta * a.A[h];
-    }
-  }
+  const float ga = -__expf(a.A[h]) * softplus_rule((float)a.a[(int64_t)rv * a.ab_stride + h] + a.dt_bias[h]);   // log decay
+  const float beta = 1.f / (1.f + __expf(-(float)a.b[(int64_t)rv * a.ab_stride + h]));
   double cum = ok ? (double)ga : 0.0;
 #pragma unroll
   for (int o = 1; o < 32; o <<= 1) {
@@ -149,24 +157,21 @@ __global__ __launch_bounds__(256) void chunk_gram_kernel(RuleArgs a) {
     if (row >= o) cum += up;
   }
   const double total = __shfl(cum, 31);   // rows past the chunk's end add nothing
-  float ik = 1.f, iq = 1.f;
-  if constexpr (DELTA) {
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
-      float sk = 0.f, sq = 0.f;
+  for (int rb = 0; rb < 2; ++rb) {
+    float sk = 0.f, sq = 0.f;
 #pragma unroll
-      for (int s = 0; s < NS; ++s)
+    for (int s = 0; s < NS; ++s)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          sk += (float)kf[rb][s][j] * (float)kf[rb][s][j];
-          sq += (float)qf[rb][s][j] * (float)qf[rb][s][j];
-        }
-      sk = group4_sum(sk);
-      sq = group4_sum(sq);
-      if (g == 0) {
-        s_vec[w][0][16 * rb + col] = rsqrtf(sk + 1e-6f);
-        s_vec[w][1][16 * rb + col] = rsqrtf(sq + 1e-6f) * rsqrtf((float)DK);
+      for (int j = 0; j < 8; ++j) {
+        sk += (float)kf[rb][s][j] * (float)kf[rb][s][j];
+        sq += (float)qf[rb][s][j] * (float)qf[rb][s][j];
       }
+    sk = group4_sum(sk);
+    sq = group4_sum(sq);
+    if (g == 0) {
+      s_vec[w][0][16 * rb + col] = rsqrtf(sk + 1e-6f);
+      s_vec[w][1][16 * rb + col] = rsqrtf(sq + 1e-6f) * rsqrtf((float)DK);
     }
   }
   if (lane < RC) {
@@ -174,15 +179,12 @@ __global__ __launch_bounds__(256) void chunk_gram_kernel(RuleArgs a) {
     s_vec[w][2][row] = beta;
   }
   wave_sync();
-  if constexpr (DELTA) {
-    ik = s_vec[w][0][row];
-    iq = s_vec[w][1][row];
-  }
+  const float ik = s_vec[w][0][row], iq = s_vec[w][1][row];
   if (lane < RC) {   // the chunk's vectors (zero past its end: such rows add nothing anywhere)
-    float* vec = ws + (DELTA ? 2 : 1) * RC * RC;
+    float* vec = ws + 2 * RC * RC;
     const float gi = __expf((float)cum), up = __expf((float)(total - cum));
     vec[row] = ok ? beta : 0.f;
-    vec[RC + row] = ok && DELTA ? beta * gi * ik : 0.f;
+    vec[RC + row] = ok ? beta * gi * ik : 0.f;
     vec[2 * RC + row] = ok ? gi * iq : 0.f;
     vec[3 * RC + row] = ok ? up * ik : 0.f;
     if (row == 0) vec[4 * RC] = __expf((float)total);
@@ -197,84 +199,133 @@ __global__ __launch_bounds__(256) void chunk_gram_kernel(RuleArgs a) {
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
           qk = mma_bf16(qf[rb][s], kf[cb][s], qk);
-          if constexpr (DELTA) kk = mma_bf16(kf[rb][s], kf[cb][s], kk);
+          kk = mma_bf16(kf[rb][s], kf[cb][s], kk);
         }
       }
       const int j = 16 * cb + col;
       const double cj = s_cum[w][j];
-      const float ikj = DELTA ? s_vec[w][0][j] : 1.f;
+      const float ikj = s_vec[w][0][j];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int i = 16 * rb + 4 * g + e;
         float p = 0.f, m = 0.f;
         if (j <= i && i < n) {
           const float dec = __expf((float)(s_cum[w][i] - cj)) * ikj;
-          p = qk[e] * dec * (DELTA ? s_vec[w][1][i] : 1.f);
-          if constexpr (DELTA) m = j < i ? kk[e] * dec * s_vec[w][0][i] * s_vec[w][2][i] : 0.f;
+          p = qk[e] * dec * s_vec[w][1][i];
+          m = j < i ? kk[e] * dec * s_vec[w][0][i] * s_vec[w][2][i] : 0.f;
         }
-        if constexpr (DELTA) {
-          pm[rb][cb][e] = p;
-          sA[w][i * LDM + j] = m;
-        } else {
-          ws[i * RC + j] = p;
-        }
+        pm[rb][cb][e] = p;
+        sA[w][i * LDM + j] = m;
       }
     }
-  if constexpr (DELTA) {
-    wave_sync();
-    float t[RC];
+  wave_sync();
+  float t[RC];
 #pragma unroll
-    for (int i = 0; i < RC; ++i) {
-      float acc[4] = {i == row ? 1.f : 0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < RC; ++i) {
+    float acc[4] = {i == row ? 1.f : 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int m = 0; m < i; m += 4) {
-        const f32x4 x = *reinterpret_cast<const f32x4*>(&sA[w][i * LDM + m]);
+    for (int m = 0; m < i; m += 4) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(&sA[w][i * LDM + m]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (m + e < i) acc[e] -= x[e] * t[m + e];
+      for (int e = 0; e < 4; ++e)
+        if (m + e < i) acc[e] -= x[e] * t[m + e];
+    }
+    t[i] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+  }
+  if (lane < RC) {
+#pragma unroll
+    for (int i = 0; i < RC; ++i) ws[RC * RC + i * RC + row] = t[i];
+  }
+  // P T: T's columns go through LDS into the product's operand layout (k-slot of step e: row 4 g + e)
+  wave_sync();
+  if (lane < RC) {
+#pragma unroll
+    for (int i = 0; i < RC; ++i) sA[w][i * LDM + row] = t[i];
+  }
+  wave_sync();
+  f32x4 tb[2][2];   // [row block][column block]
+#pragma unroll
+  for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+    for (int cb = 0; cb <= kb; ++cb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) tb[kb][cb][e] = sA[w][(16 * kb + 4 * g + e) * LDM + 16 * cb + col];
+  wave_sync();
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+    for (int cb = 0; cb <= rb; ++cb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sA[w][(16 * rb + 4 * g + e) * LDM + 16 * cb + col] = pm[rb][cb][e];
+  wave_sync();
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb) {
+      f32x4 d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kb = cb; kb <= rb; ++kb) {
+        const f32x4 m = *reinterpret_cast<const f32x4*>(&sA[w][(16 * rb + col) * LDM + 16 * kb + 4 * g]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d = mma_f32(m[e], tb[kb][cb][e], d);
       }
-      t[i] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ws[(16 * rb + 4 * g + e) * RC + 16 * cb + col] = d[e];
     }
-    if (lane < RC) {
+}
+
+// Mamba-2: one block per (chunk, group).  Wave 0 multiplies q k^T (lower triangle), every half wave takes heads.
+template <int DK>
+__global__ __launch_bounds__(256) void ssm_gram_kernel(RuleArgs a) {
+  constexpr int NS = DK / 32;
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4, hk = blockIdx.y;
+  int r0, n;
+  if (!chunk_of(blockIdx.x, a.cu, a.S, r0, n)) return;   // the same in every wave
+  float* ws = a.ws + blockIdx.x * ws_floats<false>(a.H, a.Hk);
+  if (w == 0) {
+    bf16x8 kf[2][NS], qf[2][NS];
 #pragma unroll
-      for (int i = 0; i < RC; ++i) ws[RC * RC + i * RC + row] = t[i];
+    for (int rb = 0; rb < 2; ++rb) {
+      const int64_t r = r0 + min(16 * rb + col, n - 1);
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        kf[rb][s] = ld8(a.k + r * a.stride + hk * DK + 32 * s + 8 * g);
+        qf[rb][s] = ld8(a.q + r * a.stride + hk * DK + 32 * s + 8 * g);
+      }
     }
-    // P T: T's columns go through LDS into the product's operand layout (k-slot of step e: row 4 g + e)
-    wave_sync();
-    if (lane < RC) {
-#pragma unroll
-      for (int i = 0; i < RC; ++i) sA[w][i * LDM + row] = t[i];
-    }
-    wave_sync();
-    f32x4 tb[2][2];   // [row block][column block]
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int cb = 0; cb <= kb; ++cb)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) tb[kb][cb][e] = sA[w][(16 * kb + 4 * g + e) * LDM + 16 * cb + col];
-    wave_sync();
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
-      for (int cb = 0; cb <= rb; ++cb)
+      for (int cb = 0; cb <= rb; ++cb) {
+        f32x4 qk = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sA[w][(16 * rb + 4 * g + e) * LDM + 16 * cb + col] = pm[rb][cb][e];
-    wave_sync();
+        for (int s = 0; s < NS; ++s) qk = mma_bf16(qf[rb][s], kf[cb][s], qk);
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-      for (int cb = 0; cb < 2; ++cb) {
-        f32x4 d = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kb = cb; kb <= rb; ++kb) {
-          const f32x4 m = *reinterpret_cast<const f32x4*>(&sA[w][(16 * rb + col) * LDM + 16 * kb + 4 * g]);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) d = mma_f32(m[e], tb[kb][cb][e], d);
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) ws[(16 * rb + 4 * g + e) * RC + 16 * cb + col] = d[e];
+        for (int e = 0; e < 4; ++e) ws[hk * RC * RC + (16 * rb + 4 * g + e) * RC + 16 * cb + col] = qk[e];
       }
+  }
+  const int row = lane & 31, rv = r0 + min(row, n - 1), per = a.H / a.Hk;
+  const bool ok = row < n;
+  for (int i0 = 0; i0 < per; i0 += 8) {   // (the same trips in every lane: the prefix sums run on whole waves)
+    const int i = i0 + threadIdx.x / 32, h = hk * per + min(i, per - 1);
+    const float dt = fmaxf(softplus_rule((float)a.a[(int64_t)rv * a.ab_stride + h] + a.dt_bias[h]), a.dt_min);
+    double cum = ok ? (double)(dt * a.A[h]) : 0.0;
+#pragma unroll
+    for (int o = 1; o < 32; o <<= 1) {
+      const double up = __shfl_up(cum, o, 32);
+      if (row >= o) cum += up;
+    }
+    const double total = __shfl(cum, 31, 32);   // rows past the chunk's end add nothing
+    if (i < per) {
+      float* vec = ws + a.Hk * RC * RC + h * NV_SSM;
+      const float hi = (float)cum;
+      vec[row] = ok ? dt : 0.f;
+      vec[RC + row] = hi;
+      vec[2 * RC + row] = (float)(cum - (double)hi);
+      vec[3 * RC + row] = ok ? __expf(hi) : 0.f;
+      vec[4 * RC + row] = ok ? __expf((float)(total - cum)) : 0.f;
+      if (row == 0) vec[5 * RC] = __expf((float)total);
+    }
   }
 }
 
@@ -301,7 +352,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   constexpr int NKL = RC * DK / 8 / NT, NML = RC * RC / 4 / NT;   // 16-byte loads per thread: k (and q), P (and T)
   static_assert(NKL * NT * 8 == RC * DK && NML * NT * 4 == RC * RC, "whole loads");
   __shared__ __attribute__((aligned(16))) bf16 sK[2][RC * DK], sQ[2][RC * DK];
-  __shared__ __attribute__((aligned(16))) float sP[2][RC * LDM], sT[DELTA ? 2 : 1][DELTA ? RC * LDM : 4], sV[2][4 * RC + 4];
+  __shared__ __attribute__((aligned(16))) float sP[2][RC * LDM], sT[DELTA ? 2 : 1][DELTA ? RC * LDM : 4], sV[2][vec_floats<DELTA>()];
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, g = lane >> 4;
   const int s = blockIdx.z, h = blockIdx.x, hk = h / (a.H / a.Hk);
   const int n0 = (blockIdx.y * NW + (tid >> 6)) * 16;   // this wave's columns
@@ -327,9 +378,13 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   const char* kp = reinterpret_cast<const char*>(a.k + (int64_t)r0 * a.stride + hk * DK);
   const char* qp = reinterpret_cast<const char*>(a.q + (int64_t)r0 * a.stride + hk * DK);
   const char* vp = reinterpret_cast<const char*>(a.v + (int64_t)r0 * a.v_stride + (int64_t)h * a.dv);
-  const char* mp = reinterpret_cast<const char*>(a.ws + ((int64_t)(r0 / RC + s) * a.H + h) * ws_floats<DELTA>());
+  const int64_t ws_step = 4 * ws_floats<DELTA>(a.H, a.Hk);
+  const char* mp = reinterpret_cast<const char*>(a.ws) + (r0 / RC + s) * ws_step +
+                   4 * (DELTA ? (int64_t)h * (2 * RC * RC + NV_DELTA) : (int64_t)hk * RC * RC);
+  const uint32_t vec_at = 4 * (DELTA ? 2 * RC * RC : (a.Hk - hk) * RC * RC + h * NV_SSM);   // the vectors, from there
   bf16x8 rk[NKL], rq[NKL];
-  f32x4 rp[NML], rt[NML], rvec;
+  f32x4 rp[NML], rt[NML], rvec, rhj[NML], rlj[NML];
+  float rhi[NML], rli[NML];
   bf16 rv[8];
   auto fetch = [&](int c) {   // rows and matrices of chunk c
     if (r0 + (c + 1) * RC > r1) offsets(r1 - r0 - c * RC);
@@ -339,13 +394,21 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
       rk[i] = *reinterpret_cast<const bf16x8*>(kp + kc + ko[i]);
       rq[i] = *reinterpret_cast<const bf16x8*>(qp + kc + ko[i]);
     }
-    const char* m = mp + (int64_t)c * a.H * (4 * ws_floats<DELTA>());
+    const char* m = mp + c * ws_step;
 #pragma unroll
     for (int i = 0; i < NML; ++i) {
       rp[i] = *reinterpret_cast<const f32x4*>(m + (uint32_t)(16 * (tid + NT * i)));
-      if constexpr (DELTA) rt[i] = *reinterpret_cast<const f32x4*>(m + (uint32_t)(4 * RC * RC + 16 * (tid + NT * i)));
+      if constexpr (DELTA) {
+        rt[i] = *reinterpret_cast<const f32x4*>(m + (uint32_t)(4 * RC * RC + 16 * (tid + NT * i)));
+      } else {
+        const uint32_t e = tid + NT * i, hi = vec_at + 4 * (RC + e / (RC / 4)), hj = vec_at + 4 * (RC + 4 * (e % (RC / 4)));
+        rhi[i] = *reinterpret_cast<const float*>(m + hi);
+        rli[i] = *reinterpret_cast<const float*>(m + (hi + 4 * RC));
+        rhj[i] = *reinterpret_cast<const f32x4*>(m + hj);
+        rlj[i] = *reinterpret_cast<const f32x4*>(m + (hj + 4 * RC));
+      }
     }
-    if (tid < RC + 1) rvec = *reinterpret_cast<const f32x4*>(m + (uint32_t)((DELTA ? 8 : 4) * RC * RC + 16 * tid));
+    if (tid < vec_floats<DELTA>() / 4) rvec = *reinterpret_cast<const f32x4*>(m + (vec_at + 16 * tid));
     const char* v = vp + (int64_t)c * RC * 2 * a.v_stride;
 #pragma unroll
     for (int e = 0; e < 8; ++e) rv[e] = *reinterpret_cast<const bf16*>(v + vo[e]);
@@ -359,11 +422,18 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
     }
 #pragma unroll
     for (int i = 0; i < NML; ++i) {
-      const int e = tid + NT * i, o = e / (RC / 4) * LDM + 4 * (e % (RC / 4));
+      const int e = tid + NT * i, row = e / (RC / 4), j = 4 * (e % (RC / 4)), o = row * LDM + j;
+      if constexpr (!DELTA) {   // P_ij = q_i.k_j exp(cum_i - cum_j), j <= i; cum in two parts (long sums, short differences)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const float p = rp[i][t] * __expf((rhi[i] - rhj[i][t]) + (rli[i] - rlj[i][t]));
+          rp[i][t] = j + t <= row ? p : 0.f;
+        }
+      }
       *reinterpret_cast<f32x4*>(&sP[b][o]) = rp[i];
       if constexpr (DELTA) *reinterpret_cast<f32x4*>(&sT[b][o]) = rt[i];
     }
-    if (tid < RC + 1) *reinterpret_cast<f32x4*>(&sV[b][4 * tid]) = rvec;
+    if (tid < vec_floats<DELTA>() / 4) *reinterpret_cast<f32x4*>(&sV[b][4 * tid]) = rvec;
   };
 
   // state: lane (col, g) holds column nc, key channels 32 s + 8 g .. + 7 in blocks 2 s, 2 s + 1
@@ -414,7 +484,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
     for (int rb = 0; rb < 2; ++rb) {
       const f32x4 va = *reinterpret_cast<const f32x4*>(&sV[b][16 * rb + 4 * g]);
       const f32x4 vb = *reinterpret_cast<const f32x4*>(&sV[b][RC + 16 * rb + 4 * g]);
-      const f32x4 vg = *reinterpret_cast<const f32x4*>(&sV[b][2 * RC + 16 * rb + 4 * g]);
+      const f32x4 vg = *reinterpret_cast<const f32x4*>(&sV[b][(DELTA ? 2 : 3) * RC + 16 * rb + 4 * g]);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float x = (float)vc[4 * rb + e];
@@ -424,7 +494,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
       }
       u[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    const float gc = sV[b][4 * RC];
+    const float gc = sV[b][(DELTA ? 4 : 5) * RC];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) S[nb] *= gc;
     // ---- U = T R, o += (P T) R (Mamba-2: o += P U) ----
@@ -456,7 +526,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
       }
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb) {
-        const f32x4 vd = *reinterpret_cast<const f32x4*>(&sV[b][3 * RC + 16 * rb + 4 * g]);
+        const f32x4 vd = *reinterpret_cast<const f32x4*>(&sV[b][(DELTA ? 3 : 4) * RC + 16 * rb + 4 * g]);
         u[rb] = (DELTA ? u[rb] : r[rb]) * vd;
       }
       split3(u[0], u[1], part);
@@ -496,13 +566,15 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
 
 template <bool DELTA>
 int launch_rule(const RuleArgs& a, int T, int dk, hipStream_t stream) {
-  const dim3 gram(T / RC + a.S, (a.H + 3) / 4);
+  const dim3 gram(T / RC + a.S, DELTA ? (a.H + 3) / 4 : a.Hk);
   const dim3 rule(a.H, (a.dv + 63) / 64, a.S);
   if (dk == 128) {
-    chunk_gram_kernel<128, DELTA><<<gram, 256, 0, stream>>>(a);
+    if constexpr (DELTA) chunk_gram_kernel<128><<<gram, 256, 0, stream>>>(a);
+    else ssm_gram_kernel<128><<<gram, 256, 0, stream>>>(a);
     chunk_rule_kernel<128, DELTA, 4><<<rule, 256, 0, stream>>>(a);
   } else {
-    chunk_gram_kernel<64, DELTA><<<gram, 256, 0, stream>>>(a);
+    if constexpr (DELTA) chunk_gram_kernel<64><<<gram, 256, 0, stream>>>(a);
+    else ssm_gram_kernel<64><<<gram, 256, 0, stream>>>(a);
     chunk_rule_kernel<64, DELTA, 4><<<rule, 256, 0, stream>>>(a);
   }
   OME_CHECK_LAUNCH();
@@ -512,15 +584,17 @@ int launch_rule(const RuleArgs& a, int T, int dk, hipStream_t stream) {
 // (row strides below 2^24 elements: a chunk's byte offsets stay in 32 bits)
 bool rule_shape(int S, int H, int Hk, int dk, int dv, int64_t s0, int64_t s1, int64_t s2) {
   return s0 >= 0 && s1 >= 0 && s2 >= 0 && s0 < 1 << 24 && s1 < 1 << 24 && s2 < 1 << 24 && S > 0 && S <= 65535 && H > 0 && Hk > 0 && H % Hk == 0 && (dk == 64 || dk == 128) && dv > 0 && dv % 16 == 0 &&
-         (dv + 63) / 64 <= 65535 && (H + 3) / 4 <= 65535;
+         (dv + 63) / 64 <= 65535 && H <= 65535;
 }
 
 bool aligned16(const void* p, int64_t elems) { return ((uintptr_t)p | (uintptr_t)(elems * 2)) % 16 == 0; }
 
 }  // namespace
 
-// fp32 words of workspace of one (chunk, head); T rows of S sequences and H heads need (T / 32 + S) * H of them
-OME_API int ome_chunk_rule_floats(int delta) { return delta ? ws_floats<true>() : ws_floats<false>(); }
+// fp32 words of workspace of one chunk of H heads (Mamba-2: in G groups); T rows of S sequences have up to T / 32 + S
+OME_API int ome_chunk_rule_floats(int H, int G, int delta) {
+  return (int)(delta ? ws_floats<true>(H, G) : ws_floats<false>(H, G));
+}
 
 // Gated delta rule over all rows of every sequence; operands as ome_gdn_scan.  -3: a shape, stride or
 // alignment that the chunked kernels do not take (nothing is launched).

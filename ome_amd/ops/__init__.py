@@ -161,7 +161,7 @@ def dyn_conv1d(x: torch.Tensor, kern: torch.Tensor, state: torch.Tensor, cu, slo
     return out
 
 
-def _chunk_rule_ws(T: int, S: int, H: int, dk: int, dv: int, delta: bool, state: torch.Tensor, rows: tuple) -> torch.Tensor | None:
+def _chunk_rule_ws(T: int, S: int, H: int, G: int, dk: int, dv: int, delta: bool, state: torch.Tensor, rows: tuple) -> torch.Tensor | None:
     """Workspace of the chunked kernels (``chunk_rule.hip``) for T rows of S sequences and H heads, or None
     where the row-by-row kernels run: one row per sequence (a decode step; a chunk would be 1/32 full), key
     widths other than 64 / 128, value widths not of 16 columns, or key / query rows (the first two
@@ -169,7 +169,7 @@ def _chunk_rule_ws(T: int, S: int, H: int, dk: int, dv: int, delta: bool, state:
     if T <= S or dk not in (64, 128) or dv % 16 or state.data_ptr() % 16 or S > 65535 or H > 65535 or \
             any(r.data_ptr() % 16 or r.stride(0) % 8 for r in rows[:2]) or any(not 0 <= r.stride(0) < 1 << 24 for r in rows):
         return None
-    return torch.empty((T // 32 + S) * H * load().ome_chunk_rule_floats(int(delta)), dtype=torch.float32,
+    return torch.empty((T // 32 + S) * load().ome_chunk_rule_floats(H, G, int(delta)), dtype=torch.float32,
                        device=state.device)
 
 
@@ -183,7 +183,7 @@ def ssm_scan(x, dt, B, C, A, D, dt_bias, dt_min: float, state, cu, slot, reset, 
         return ref.ssm_scan(x, dt, B, C, A, D, dt_bias, dt_min, state, cu, slot, reset, H, P, N, G, out)
     assert B.stride(0) == C.stride(0) and B.stride(1) == 1 and x.stride(1) == 1 and dt.stride(1) == 1
     f32 = _f32(x, dt, B, C, out)
-    ws = None if f32 or H % G else _chunk_rule_ws(T, slot.shape[0], H, N, P, False, state, (B, C, x, out))
+    ws = None if f32 or H % G else _chunk_rule_ws(T, slot.shape[0], H, G, N, P, False, state, (B, C, x, out))
     if ws is not None:
         call("ome_ssm_chunks", x.data_ptr(), x.stride(0), dt.data_ptr(), dt.stride(0), B.data_ptr(), C.data_ptr(),
              B.stride(0), A.data_ptr(), D.data_ptr(), dt_bias.data_ptr(), float(dt_min), state.data_ptr(), out.data_ptr(),
@@ -214,7 +214,7 @@ def gdn_scan(q, k, v, a, b, A_log, dt_bias, state, cu, slot, reset, Hv: int, Hk:
     assert q.stride(1) == k.stride(1) == v.stride(1) == a.stride(1) == 1 and out.stride(1) == 1
     assert state.is_contiguous() and state.dtype == torch.float32
     f32 = _f32(q, k, v, a, b, out)
-    ws = None if v1 or f32 or Hk <= 0 or Hv % Hk else _chunk_rule_ws(T, slot.shape[0], Hv, dk, dv, True, state, (q, k, out))
+    ws = None if v1 or f32 or Hk <= 0 or Hv % Hk else _chunk_rule_ws(T, slot.shape[0], Hv, Hk, dk, dv, True, state, (q, k, out))
     if ws is not None:   # prompts: chunks of 32 rows on the matrix cores
         call("ome_gdn_chunks", q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), a.data_ptr(), b.data_ptr(),
              a.stride(0), A_log.data_ptr(), dt_bias.data_ptr(), state.data_ptr(), out.data_ptr(), out.stride(0),

@@ -132,7 +132,8 @@ def test_delta_rule_prompts(lens, dk, dv, Hk, Hv, off):
 
 
 @pytest.mark.parametrize("lens", LENS, ids=str)
-@pytest.mark.parametrize("H,P,N,G,off", [(16, 64, 128, 2, 8), (3, 16, 64, 1, 0), (5, 80, 128, 5, 8), (4, 64, 128, 2, 1)])
+@pytest.mark.parametrize("H,P,N,G,off", [(16, 64, 128, 2, 8), (3, 16, 64, 1, 0), (5, 80, 128, 5, 8), (4, 64, 128, 2, 1),
+                                         (20, 16, 64, 2, 8)])
 def test_selective_scan_prompts(lens, H, P, N, G, off):
     torch.manual_seed(H + N)
     T, slots = sum(lens), 71
