@@ -221,6 +221,13 @@ def gdn_scan(q, k, v, a, b, A_log, dt_bias, state, cu, slot, reset, Hv: int, Hk:
              _i32(cu).data_ptr(), _i32(slot).data_ptr(), _i32(reset).data_ptr(), slot.shape[0], T, Hv, Hk, dk, dv,
              ws.data_ptr(), stream_ptr())
         return out
+    if not v1 and not f32 and T == slot.shape[0] and dk in (64, 128, 256) and 0 < Hv <= 65535 and Hk > 0 and Hv % Hk == 0 and \
+            q.data_ptr() % 16 == 0 and k.data_ptr() % 16 == 0 and q.stride(0) % 8 == 0 and 0 < dv < 1 << 20:
+        # a decode step: the normalisation inside the scan (47.9 -> 43.9 us at 64 sequences of 32 heads)
+        call("ome_gdn_step", q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), a.data_ptr(), b.data_ptr(),
+             a.stride(0), A_log.data_ptr(), dt_bias.data_ptr(), state.data_ptr(), out.data_ptr(), out.stride(0),
+             _i32(cu).data_ptr(), _i32(slot).data_ptr(), _i32(reset).data_ptr(), T, Hv, Hk, dk, dv, stream_ptr())
+        return out
     # (key widths other than 64 / 128 / 256, and fp32 models, run the launcher's generic kernel: no workspace)
     ws = None if v1 or f32 or dk not in (64, 128, 256) else \
         torch.empty(T * (2 * Hk * dk + Hk + 2 * Hv), dtype=torch.float32, device=q.device)

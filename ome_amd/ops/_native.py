@@ -92,6 +92,7 @@ _SIGNATURES = {
                          i32, i32, i32, vp],
         "ome_gdn_scan": [vp, vp, vp, i64, vp, vp, i64, vp, vp, vp, vp, i64, vp, vp, vp, i32, i32, i32, i32, i32,
                          i32, vp, i32, vp],
+        "ome_gdn_step": [vp, vp, vp, i64, vp, vp, i64, vp, vp, vp, vp, i64, vp, vp, vp, i32, i32, i32, i32, i32, vp],
         "ome_chunk_rule_floats": [i32, i32, i32],
         "ome_gdn_chunks": [vp, vp, vp, i64, vp, vp, i64, vp, vp, vp, vp, i64, vp, vp, vp, i32, i32, i32, i32, i32, i32, vp,
                            vp],

@@ -131,6 +131,13 @@ def test_delta_rule_prompts(lens, dk, dv, Hk, Hv, off):
     assert near(ops.gdn_scan(*args, st, *sq, Hv, Hk), st, *want)
 
 
+@pytest.mark.parametrize("lens", [[1], [1] * 5, [1, 0, 2, 1], [1] * 70], ids=str)
+@pytest.mark.parametrize("dk,dv,Hk,Hv,off", [(128, 128, 2, 4, 8), (64, 16, 1, 5, 0), (256, 40, 3, 3, 8), (128, 33, 1, 2, 8),
+                                             (64, 128, 2, 2, 1)])
+def test_delta_rule_steps(lens, dk, dv, Hk, Hv, off):   # off 1: the scan behind its prep pass
+    test_delta_rule_prompts(lens, dk, dv, Hk, Hv, off)
+
+
 @pytest.mark.parametrize("lens", LENS, ids=str)
 @pytest.mark.parametrize("H,P,N,G,off", [(16, 64, 128, 2, 8), (3, 16, 64, 1, 0), (5, 80, 128, 5, 8), (4, 64, 128, 2, 1),
                                          (20, 16, 64, 2, 8)])
