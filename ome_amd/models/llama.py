@@ -360,6 +360,8 @@ class LlamaForCausalLM:
             plan = ops.gemm_sk_plan(x.shape[0], w.shape[0], w.shape[1], 2) if x.shape[0] > _GEMV_ROWS else None
             if plan is not None and x.stride(1) == 1 and x.stride(0) % 8 == 0:
                 a = ops.gemm_sk(x, w, epi=2, bn=plan[0], nwg=plan[1], bm=plan[2])
+            elif x.is_cuda and x.shape[0] <= _GEMV_ROWS and ops.gemv_ok(x, w):
+                a = ops.gemv_swiglu(x, w)
             else:
                 a = ops.act_and_mul(linear(x, w), self.act, interleaved=True)
             return self._row_parallel(a, wd)
@@ -408,12 +410,17 @@ class LlamaForCausalLM:
             if i > 0:  # the previous layer's MLP partial sums -> all-reduce + add + norm (a pipeline
                 # stage's first layer receives the previous stage's already-reduced output)
                 x = self._reduce_add_norm(x, residual, self.ln1[i], reduce=partial and i > first)
-            qkv = linear(x, self.w_qkv[i], self.b_qkv[i])
             q = torch.empty(T, tp.hq, D, dtype=self.dtype, device=x.device)
             k_cache, v_cache = kv.layer(i)
             ks, vs = kv.scales(i)
-            ops.rope_qkv_cache(qkv, meta.positions, self.cos_sin, cfg.rot_dim, q, k_cache, v_cache, meta.slots,
-                               tp.hq, tp.hkv, D, True, self.qn[i], self.kn[i], self.eps, ks, vs)
+            if T <= _GEMV_ROWS and self.qn[i] is None and \
+                    ops.gemv_qkv_ok(x, self.w_qkv[i], self.b_qkv[i], cfg.rot_dim, D, tp.hq, tp.hkv, k_cache):
+                ops.gemv_qkv(x, self.w_qkv[i], self.b_qkv[i], meta.positions, self.cos_sin, q, k_cache, v_cache,
+                             meta.slots, tp.hq, tp.hkv, D, ks, vs)
+            else:
+                qkv = linear(x, self.w_qkv[i], self.b_qkv[i])
+                ops.rope_qkv_cache(qkv, meta.positions, self.cos_sin, cfg.rot_dim, q, k_cache, v_cache, meta.slots,
+                                   tp.hq, tp.hkv, D, True, self.qn[i], self.kn[i], self.eps, ks, vs)
             attn = self.attention(q, k_cache, v_cache, meta, ks, vs)
             o = self._reduce_add_norm(self._row_parallel(attn.view(T, tp.hq * D), self.w_o[i]), residual,
                                       self.ln2[i])

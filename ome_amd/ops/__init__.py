@@ -1248,6 +1248,32 @@ def gemv_act(gu: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None)
     return out
 
 
+def gemv_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """``act_and_mul(gemv(x, w), 0, interleaved=True)`` in one launch (M <= 8 rows; ``gemv_ok`` operands, w
+    [2 I, K] from :func:`interleave_gate_up`), the same bits."""
+    assert x.is_cuda and gemv_ok(x, w) and w.shape[0] % 32 == 0, (tuple(x.shape), x.stride(), w.shape)
+    M, I = x.shape[0], w.shape[0] // 2
+    out = torch.empty(M, I, dtype=x.dtype, device=x.device)
+    call("ome_gemv_swiglu", x.data_ptr(), x.stride(0), w.data_ptr(), out.data_ptr(), I, M, I, x.shape[1], stream_ptr())
+    return out
+
+
+def gemv_qkv_ok(x: torch.Tensor, w, bias, rot_dim: int, D: int, Hq: int, Hkv: int, k_cache: torch.Tensor) -> bool:
+    """:func:`gemv_qkv` takes this projection: plain bf16 rows of a GEMV, whole heads rotated, pages of 16 tokens."""
+    return (x.is_cuda and gemv_ok(x, w, bias) and rot_dim == D and D in (64, 128, 256) and min(Hq, Hkv) > 0
+            and w.shape[0] == (Hq + 2 * Hkv) * D and k_cache.shape[2] == 16)
+
+
+def gemv_qkv(x, w, bias, positions, cos_sin, q_out, k_cache, v_cache, slots, Hq, Hkv, D, k_scale: float = 1.0,
+             v_scale: float = 1.0) -> None:
+    """:func:`gemv`, then :func:`rope_qkv_cache` (no per-head norm) of its rows, in one launch: the projection never
+    reaches memory.  Operands as :func:`gemv_qkv_ok` wants them."""
+    call("ome_gemv_qkv", x.data_ptr(), x.stride(0), w.data_ptr(), ptr(bias), _i32(positions).data_ptr(),
+         cos_sin.data_ptr(), q_out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), _i32(slots).data_ptr(),
+         x.shape[0], Hq, Hkv, D, k_cache.shape[2], x.shape[1], kv_format(k_cache), float(k_scale), float(v_scale),
+         stream_ptr())
+
+
 # ---- decode GEMM routing: ome_stream_gemm where it measured faster than hipBLASLt --------------
 # Filled during the engine's eager pre-capture pass (``decode_gemm_tuning``): every (M, N, K, bias)
 # a decode bucket issues is timed once against the library GEMM and the winner recorded; graphs

@@ -126,6 +126,8 @@ _SIGNATURES = {
         "ome_w8a16_mgemv": [vp, i64, vp, i64, vp, i32, vp, vp, i64, i32, i32, i32, i32, vp, vp, vp],
         "ome_stream_gemm": [vp, i64, vp, vp, vp, i64, i32, i32, i32, i32, i32, vp, vp, vp],
         "ome_gemv": [vp, i64, vp, vp, vp, i64, i32, i32, i32, vp],
+        "ome_gemv_swiglu": [vp, i64, vp, vp, i64, i32, i32, i32, vp],
+        "ome_gemv_qkv": [vp, i64, vp, vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, i32, f32, f32, vp],
         "ome_gemv_act": [vp, i64, vp, vp, vp, i64, i32, i32, i32, vp],
         "ome_gemm": [vp, i64, vp, i64, vp, i64, i32, i32, i32, i32, i32, vp, vp],
         "ome_gemm_set_variant": [i32],
