@@ -898,21 +898,40 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_prefill_v2_kernel(
     const typename KVStore<F>::T* __restrict__ v_cache, const int* __restrict__ block_tables, int bt_stride,
     const int* __restrict__ cu_q, const int* __restrict__ kv_lens, const int2* __restrict__ items,
     bf16* __restrict__ out, int64_t out_stride, int Hq, int Hkv, Scaler scl, int window, float v_scale,
-    const float* __restrict__ sinks, const int* __restrict__ row_hi, int chunk, float* __restrict__ part_o,
-    float* __restrict__ part_ml) {
+    const float* __restrict__ sinks, const int* __restrict__ row_hi, int chunk, int listed,
+    float* __restrict__ part_o, float* __restrict__ part_ml) {
   constexpr int D = 128, P = 16, NB = D / 16, KS = D / 32;
   typedef typename KVRaw<F>::K8 Raw8;  // 8 consecutive cache elements
   __shared__ __attribute__((aligned(16))) bf16 sK[2][SUB][32 * PF_KLD];
   __shared__ __attribute__((aligned(16))) bf16 sV[2][SUB][D * PF_VLD];
-  int s, r0_item, c_lo = 0, part = -1;
+  // head-major: consecutive blocks, which go to consecutive XCDs, take different kv heads of the same rows, so an
+  // XCD's L2 holds the K / V of Hkv / 8 heads.  Items in the grid's x and heads in its y, every L2 saw every
+  // head: 2 x 2048 rows 136 -> 97 us, 4096 rows 246 -> 166, 8000 rows 662 -> 575 (8 kv heads, bf16)
+  const int kvh = blockIdx.x % Hkv;
+  int e0 = blockIdx.x / Hkv, e1 = e0 + 1;
+  const int4* list = reinterpret_cast<const int4*>(items);
+  if (SPLIT && listed > 0) {   // a block's run of pieces, behind the pieces
+    const int4 run = list[listed + e0];
+    e0 = run.x, e1 = run.y;
+  }
+  for (int entry = e0; entry < e1; ++entry) {
+  if (SPLIT && entry > e0) __syncthreads();   // the piece before is done with the LDS images
+  int s, r0_item, c_lo = 0, c_hi = 0x7fffffff, part = -1;
   if constexpr (SPLIT) {
-    const int4 it4 = reinterpret_cast<const int4*>(items)[blockIdx.x];
+    const int4 it4 = list[entry];
     s = it4.x, r0_item = it4.y, c_lo = it4.z, part = it4.w;
+    if (listed > 0) {   // up to the item's next piece
+      if (entry + 1 < listed && part >= 0) {
+        const int4 nx = list[entry + 1];
+        if (nx.x == s && nx.y == r0_item) c_hi = nx.z;
+      }
+    } else {
+      c_hi = c_lo + chunk;
+    }
   } else {
-    const int2 it = items[blockIdx.x];
+    const int2 it = items[e0];
     s = it.x, r0_item = it.y;
   }
-  const int kvh = blockIdx.y;
   const int q0 = cu_q[s];
   const int q_len = cu_q[s + 1] - q0;
   const int kv_len = kv_lens[s];
@@ -933,7 +952,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_prefill_v2_kernel(
   kv_lo = attn_lo(prefix + r0_item, window) & ~31;
   if constexpr (SPLIT) {   // chunk starts are multiples of 64 keys: kv_lo stays 32-aligned
     kv_lo = max(kv_lo, c_lo);
-    kv_end = min(kv_end, c_lo + chunk);
+    kv_end = min(kv_end, c_hi);
   }
   // first visible key of this lane's two rows, and the key from which all rows of the wave see all
   // (keys at or beyond it need the mask only at the diagonal)
@@ -1253,7 +1272,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_prefill_v2_kernel(
     kB = kD;
     kC = kE;
   }
-  if (!active) return;
+  if (!active) continue;
   if constexpr (FAST) {   // per-lane partial row sums -> the row's total (its 4 lane groups)
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
@@ -1270,7 +1289,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_prefill_v2_kernel(
       for (int nb = 0; nb < NB; ++nb) *reinterpret_cast<f32x4*>(po + row * D + 16 * nb + 4 * g) = o[rb][nb];
       if (g == 0) *reinterpret_cast<float2*>(part_ml + (pw * 32 + row) * 2) = make_float2(m_i[rb], l_i[rb]);
     }
-    return;
+    continue;
   }
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb) {
@@ -1287,6 +1306,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_prefill_v2_kernel(
         *reinterpret_cast<bf16x4*>(orow + 16 * nb + 4 * g) = v;
       }
     }
+  }
   }
 }
 
@@ -1353,9 +1373,9 @@ static void launch_prefill(int variant, int rows, int G, dim3 grid, hipStream_t 
   if constexpr (D == 128) {
     if (variant == 2 && G == 4) {  // one head per wave over 32-row items (GQA-4: Llama-3, Qwen3, Mixtral)
 #define OME_PF2B(FAST, NW, BS)                                                                                    \
-  paged_prefill_v2_kernel<2, F, false, FAST, NW, 0, BS><<<grid, 64 * NW, 0, stream>>>(                            \
+  paged_prefill_v2_kernel<2, F, false, FAST, NW, 0, BS><<<grid.x * grid.y, 64 * NW, 0, stream>>>(                            \
       (const bf16*)q, q_stride, (const T*)k_cache, (const T*)v_cache, block_tables, bt_stride, cu_q, kv_lens,      \
-      (const int2*)items, (bf16*)out, out_stride, Hq, Hkv, scl, window, v_scale, sinks, row_hi, 0, nullptr, nullptr)
+      (const int2*)items, (bf16*)out, out_stride, Hq, Hkv, scl, window, v_scale, sinks, row_hi, 0, 0, nullptr, nullptr)
 #define OME_PF2(FAST, NW) OME_PF2B(FAST, NW, false)
       const bool bs = scl.bs_shift != 0;   // BS kernels need blocks >= 64 keys (else: generic body, mask only)
       const bool bs_fast = bs && scl.bs_shift >= 6 && prefill_fast(scl, window, row_hi);
@@ -1369,9 +1389,9 @@ static void launch_prefill(int variant, int rows, int G, dim3 grid, hipStream_t 
         static const int probe = getenv("OME_PREFILL_PROBE") ? atoi(getenv("OME_PREFILL_PROBE")) : 0;
         if (!bs && prefill_fast(scl, window, row_hi)) {
 #define OME_PF2P(PR)                                                                                              \
-  paged_prefill_v2_kernel<2, F, false, true, 4, PR><<<grid, 256, 0, stream>>>(                                    \
+  paged_prefill_v2_kernel<2, F, false, true, 4, PR><<<grid.x * grid.y, 256, 0, stream>>>(                                    \
       (const bf16*)q, q_stride, (const T*)k_cache, (const T*)v_cache, block_tables, bt_stride, cu_q, kv_lens,      \
-      (const int2*)items, (bf16*)out, out_stride, Hq, Hkv, scl, window, v_scale, sinks, row_hi, 0, nullptr, nullptr)
+      (const int2*)items, (bf16*)out, out_stride, Hq, Hkv, scl, window, v_scale, sinks, row_hi, 0, 0, nullptr, nullptr)
           bool done = false;
           if constexpr (F == KV_BF16) {   // diagnostic instantiations for the bf16 cache only
             done = probe >= 1 && probe <= 3;
@@ -1447,28 +1467,28 @@ OME_API int ome_paged_prefill(const void* q, int64_t q_stride, const void* k_cac
 // [n_comb][4]; part_o [parts][Hkv][4][32][128] and part_ml [parts][Hkv][4][32][2] fp32 workspaces.
 OME_API int ome_paged_prefill_split(const void* q, int64_t q_stride, const void* k_cache, const void* v_cache,
                                     const int* block_tables, int bt_stride, const int* cu_q, const int* kv_lens,
-                                    const int* items4, int n_items, const int* comb, int n_comb, int chunk,
-                                    void* part_o, void* part_ml, void* out, int64_t out_stride, int Hq, int Hkv,
+                                    const int* items4, int n_items, int n_blocks, const int* comb, int n_comb,
+                                    int chunk, void* part_o, void* part_ml, void* out, int64_t out_stride, int Hq, int Hkv,
                                     float scale, int window, int kv_fmt, float k_scale, float v_scale, float softcap,
                                     const float* sinks, const float* alibi, int64_t bsparse, int keep_first,
                                     hipStream_t stream) {
   if (n_items <= 0) return 0;
-  if (Hq != 4 * Hkv || chunk % 64 || kv_fmt < 0 || kv_fmt > 2) return -2;
+  if (Hq != 4 * Hkv || chunk % 64 || kv_fmt < 0 || kv_fmt > 2 || n_blocks < 0 || (n_blocks == 0 && chunk <= 0)) return -2;
   if (window > 0 && keep_first > 0) return -6;   // kept first keys: ome_paged_prefill only
   const Scaler scl = make_scaler(scale * k_scale, softcap, alibi, bsparse);
-  dim3 grid(n_items, Hkv);
+  const int grid = (n_blocks > 0 ? n_blocks : n_items) * Hkv, listed = n_blocks > 0 ? n_items : 0;
 #define OME_PFS(F, FAST)                                                                                       \
   if (FAST && scl.bs_shift >= 6)                                                                               \
     paged_prefill_v2_kernel<2, F, true, FAST, 4, 0, FAST><<<grid, 256, 0, stream>>>(                           \
         (const bf16*)q, q_stride, (const typename KVStore<F>::T*)k_cache,                                      \
         (const typename KVStore<F>::T*)v_cache, block_tables, bt_stride, cu_q, kv_lens, (const int2*)items4,   \
-        (bf16*)out, out_stride, Hq, Hkv, scl, window, v_scale, sinks, nullptr, chunk, (float*)part_o,          \
+        (bf16*)out, out_stride, Hq, Hkv, scl, window, v_scale, sinks, nullptr, chunk, listed, (float*)part_o,  \
         (float*)part_ml);                                                                                      \
   else                                                                                                         \
   paged_prefill_v2_kernel<2, F, true, FAST><<<grid, 256, 0, stream>>>(                                         \
       (const bf16*)q, q_stride, (const typename KVStore<F>::T*)k_cache, (const typename KVStore<F>::T*)v_cache, \
       block_tables, bt_stride, cu_q, kv_lens, (const int2*)items4, (bf16*)out, out_stride, Hq, Hkv, scl, window,  \
-      v_scale, sinks, nullptr, chunk, (float*)part_o, (float*)part_ml)
+      v_scale, sinks, nullptr, chunk, listed, (float*)part_o, (float*)part_ml)
   // block-sparse with blocks < 64 keys: generic body (mask only)
   const bool fast = prefill_fast(scl, window, nullptr) && (scl.bs_shift == 0 || scl.bs_shift >= 6);
   if (kv_fmt == KV_BF16) {

@@ -5,6 +5,7 @@ native library is missing on a GPU the call raises.
 from __future__ import annotations
 
 import contextlib
+import heapq
 import os
 
 import torch
@@ -1659,7 +1660,10 @@ class PrefillPlan:
     """Work decomposition of one prefill attention call, built host-side by
     :func:`prefill_plan` and uploaded with the step's other inputs.  ``items`` is the classic
     [n, 2] (seq, row0) list; ``split`` [n4, 4] (seq, row0, chunk start, part) and ``comb``
-    [nc, 4] (seq, row0, first part, parts) are the split-KV form (empty when nothing splits)."""
+    [nc, 4] (seq, row0, first part, parts) are the split-KV form (empty when nothing splits).
+    ``chunk`` > 0: one workgroup per row of ``split`` and kv head, ``chunk`` keys each.  ``chunk`` =
+    -n: n workgroups a kv head; the last n rows of ``split`` are their runs (first, past the last)
+    of pieces, a piece reaches to its item's next one (:func:`_prefill_runs`)."""
 
     __slots__ = ("items", "split", "comb", "chunk", "parts", "rows")
 
@@ -1689,6 +1693,56 @@ def prefill_rows(Hq: int, Hkv: int, D: int, page: int = 16) -> int:
 PREFILL_SPLIT_MIN_KEYS = int(os.environ.get("OME_PREFILL_SPLIT_MIN_KEYS", "2048"))
 
 
+# workgroups of the 32-row GQA-4 kernel that the chip holds at once: 2 (LDS, registers) on each of 256 CUs
+_PREFILL_SLOTS = 512
+
+
+def _prefill_runs(items: list, ends: list[int], kv_heads: int):
+    """(pieces + runs, combine items, -runs, parts) that give each of the chip's workgroups the same number of 64-key
+    stages, or None where one workgroup per item is about as good.  A workgroup walks one run of the (item,
+    stage) sequence, so only the items at a run's ends are cut (at a stage, no piece under 4).
+
+    Estimated in stages of a workgroup (2.65 us with both of a CU's at work): the classic launch takes its
+    greedy schedule in item order; the runs their share, 8 for the second launch and short runs, and
+    the cut items' partials (64 KiB each, written and read: 0.0124).  Against one workgroup per item, 8 kv heads:
+    1500 rows over 6100 keys (376 workgroups for 512 places) 282 -> 230 us with an fp8 cache, 248 -> 224 in bf16;
+    3000 over 5000: 427 -> 408; 256 over 3840: 110 -> 47 (in equal chunks: 51); 64 over 15936, fp8: 475 -> 41 (56).
+    Where the estimate is above 0.93 the partials cost what the balance gains: 1000 and 1000 over 2000, fp8, 96 -> 99."""
+    slots = _PREFILL_SLOTS // max(1, kv_heads)
+    units = [-(-e // 64) for e in ends]
+    if not slots or len(items) > 4 * slots:   # the last wave is at most a quarter of the work
+        return None
+    busy = [0] * slots
+    for u in units:
+        heapq.heapreplace(busy, busy[0] + u)
+    total, cuts = sum(units), slots + len(items)
+    if total / slots + 8 + 0.0124 * cuts * kv_heads >= 0.93 * max(busy):
+        return None
+    pieces, comb, runs, parts = [], [], [], 0
+    done, first, bound = 0, 0, total / slots   # stages dealt out; this run's first piece and end
+    for (s, r), u in zip(items, units):
+        at = [0]
+        while True:
+            take = round(bound - done)
+            if take >= u - at[-1] - 3:   # the rest of the item (all but 3 stages: those too)
+                done += u - at[-1]
+                break
+            if take >= 4:
+                done += take
+                at.append(at[-1] + take)
+            n = len(pieces) + len(at) - 1   # the run ends at this cut
+            if n > first:
+                runs.append((first, n, 0, 0))
+                first = n
+            bound += total / slots
+        if len(at) > 1:
+            comb.append((s, r, parts, len(at)))
+        pieces += [(s, r, 64 * a, parts + j if len(at) > 1 else -1) for j, a in enumerate(at)]
+        parts += len(at) if len(at) > 1 else 0
+    runs.append((first, len(pieces), 0, 0))
+    return pieces + runs, comb, -len(runs), parts
+
+
 def prefill_plan(q_lens: list[int], kv_lens: list[int], tile: int = 32, target: int | None = None,
                  kv_heads: int = 8, force: bool = False):
     """(classic items, split items, combine items, chunk, parts) for the split-KV prefill kernel.
@@ -1701,7 +1755,8 @@ def prefill_plan(q_lens: list[int], kv_lens: list[int], tile: int = 32, target: 
     Measured (profiles/r03_prefill_split_bench.txt): splitting pays when the classic grid is
     smaller than the chip (items x kv heads < 256 workgroups) AND some item has a long key range
     (> ``PREFILL_SPLIT_MIN_KEYS`` keys), e.g. 256 new rows over a 4096-token prefix 243 -> 68 us; at ~900 rows over
-    <= 480 keys the classic grid is already full and splitting costs the partial round trip."""
+    <= 480 keys the classic grid is already full and splitting costs the partial round trip.  Long
+    ranges whose classic grid leaves places of the chip empty: :func:`_prefill_runs`."""
     target = target or PREFILL_SPLIT_TARGET
     items = prefill_work_items(q_lens, kv_lens, tile)
     # the split decision and the split items use 32-row items (the split kernel's partial layout)
@@ -1712,6 +1767,10 @@ def prefill_plan(q_lens: list[int], kv_lens: list[int], tile: int = 32, target: 
         e = (kv_lens[s] - q_lens[s]) + min(r + 32, q_lens[s])
         ends.append(e)
         work += e
+    if not force and max(ends, default=0) > PREFILL_SPLIT_MIN_KEYS:
+        runs = _prefill_runs(items32, ends, kv_heads)
+        if runs is not None:
+            return items, *runs
     if not force and (len(items32) * kv_heads >= 256 or max(ends, default=0) <= PREFILL_SPLIT_MIN_KEYS):
         return items, [], [], 0, 0
     chunk = max(128, -(-(-(-work // max(1, target))) // 64) * 64)
@@ -1764,13 +1823,15 @@ def paged_prefill(q, k_cache, v_cache, block_tables, cu_q, kv_lens, items, scale
             raise ValueError(f"paged_prefill: {rows}-row items need the GQA-4 / D=128 kernel, got Hq={Hq} "
                              f"Hkv={Hkv} D={D} page={P} (build the plan with prefill_rows of this layer)")
         if (plan.parts and D == 128 and P == 16 and Hq == 4 * Hkv and row_hi is None and keep_first <= 0 and
+                (plan.chunk > 0 or (window <= 0 and blocksparse is None)) and
                 os.environ.get("OME_PREFILL_ATTN", "2") == "2"):
+            nb = max(0, -plan.chunk)
             po = torch.empty(plan.parts * Hkv * 4 * 32 * 128, dtype=torch.float32, device=q.device)
             pml = torch.empty(plan.parts * Hkv * 4 * 32 * 2, dtype=torch.float32, device=q.device)
             call("ome_paged_prefill_split", q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
                  _i32(block_tables).data_ptr(), block_tables.stride(0), _i32(cu_q).data_ptr(),
-                 _i32(kv_lens).data_ptr(), plan.split.data_ptr(), plan.split.shape[0], plan.comb.data_ptr(),
-                 plan.comb.shape[0], int(plan.chunk), po.data_ptr(), pml.data_ptr(), out.data_ptr(), out.stride(0),
+                 _i32(kv_lens).data_ptr(), plan.split.data_ptr(), plan.split.shape[0] - nb, nb, plan.comb.data_ptr(),
+                 plan.comb.shape[0], max(0, int(plan.chunk)), po.data_ptr(), pml.data_ptr(), out.data_ptr(), out.stride(0),
                  Hq, Hkv, float(scale), int(window), kv_format(k_cache), float(k_scale), float(v_scale),
                  float(softcap), _sinks(sinks), _sinks(alibi), blocksparse_pack(blocksparse), int(keep_first),
                  stream_ptr())

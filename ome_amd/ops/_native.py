@@ -118,7 +118,7 @@ _SIGNATURES = {
                              i32, vp, i32, f32, f32, f32, vp, vp, vp, i64, i32, vp],
         "ome_paged_prefill": [vp, i64, vp, vp, vp, i32, vp, vp, vp, i32, vp, i64, i32, i32, i32, i32, f32, i32,
                               i32, f32, f32, f32, vp, vp, vp, i32, i64, i32, vp],
-        "ome_paged_prefill_split": [vp, i64, vp, vp, vp, i32, vp, vp, vp, i32, vp, i32, i32, vp, vp, vp, i64, i32,
+        "ome_paged_prefill_split": [vp, i64, vp, vp, vp, i32, vp, vp, vp, i32, i32, vp, i32, i32, vp, vp, vp, i64, i32,
                                     i32, f32, i32, i32, f32, f32, f32, vp, vp, i64, i32, vp],
         "ome_varlen_attention": [vp, i64, vp, i64, vp, i64, vp, vp, vp, i32, vp, i64, i32, i32, i32, f32, i32, vp],
         "ome_skinny_gemm": [vp, i64, vp, vp, vp, i64, i32, i32, i32, i32, vp, vp, vp],

@@ -1,0 +1,74 @@
+"""Long-range prefill attention dealt out as equal runs of 64-key stages (``ops._prefill_runs``)."""
+import random
+
+import pytest
+import torch
+
+from ome_amd import ops
+from ome_amd.ops import reference as ref
+
+
+def _spans(split, nb, ends):
+    """{item: [(first key, past the last, part)]} of a plan's pieces, as the kernel reads them, and each run's stages."""
+    pieces, spans, load = split[:-nb], {}, []
+    for i, (s, r, c, part) in enumerate(pieces):
+        nxt = pieces[i + 1] if i + 1 < len(pieces) and part >= 0 else None
+        hi = nxt[2] if nxt and nxt[:2] == (s, r) else ends[s, r]
+        spans.setdefault((s, r), []).append((c, hi, part))
+        load.append(-(-(hi - c) // 64))
+    return spans, [sum(load[a:b]) for a, b, _, _ in split[-nb:]]
+
+
+@pytest.mark.parametrize("seed", range(40))
+def test_runs_cover_every_item_once(seed):
+    rng = random.Random(seed)
+    n = rng.randint(1, 6)
+    q = [rng.choice([1, 31, 32, 33, rng.randint(1, 3000)]) for _ in range(n)]
+    kv = [a + rng.choice([0, 5, rng.randint(2000, 20000)]) for a in q]
+    heads = rng.choice([1, 2, 4, 8, 16, 32])
+    items, split, comb, chunk, parts = ops.prefill_plan(q, kv, kv_heads=heads)
+    if chunk >= 0:
+        return
+    ends = {(s, r): kv[s] - q[s] + min(r + 32, q[s]) for s, r in items}
+    spans, load = _spans(split, -chunk, ends)
+    runs = split[chunk:]
+    assert -chunk * heads <= 512 and runs[0][0] == 0 and runs[-1][1] == len(split) + chunk
+    assert all(a[0] < a[1] for a in runs) and all(a[1] == b[0] for a, b in zip(runs, runs[1:]))
+    assert list(spans) == [tuple(i) for i in items]
+    for item, v in spans.items():
+        assert v[0][0] == 0 and v[-1][1] == ends[item] and all(a[1] == b[0] and a[1] % 64 == 0 for a, b in zip(v, v[1:]))
+        assert all(lo < hi for lo, hi, _ in v) and (v[0][2] < 0) == (len(v) == 1)
+    cut = [v for v in spans.values() if len(v) > 1]
+    assert [p for v in cut for *_, p in v] == list(range(parts))
+    assert [(i, v[0][2], len(v)) for i, v in spans.items() if len(v) > 1] == [((s, r), p, m) for s, r, p, m in comb]
+    assert max(load) <= sum(load) / len(load) + 8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("q_lens,kv_lens,Hq,Hkv", [([64], [2100], 32, 8), ([33, 1, 90], [4097, 2200, 90], 4, 1),
+                                                   ([700], [2749], 16, 4)])
+@pytest.mark.parametrize("cache", [torch.bfloat16, torch.float8_e4m3fn], ids=str)
+@pytest.mark.parametrize("mode", ["plain", "softcap", "window", "sinks"])
+def test_runs_match_reference(q_lens, kv_lens, Hq, Hkv, cache, mode):
+    torch.manual_seed(sum(kv_lens))
+    D, P, dev = 128, 16, "cuda"
+    t = lambda a, c: torch.tensor(a, dtype=torch.int32, device=dev).view(-1, c)  # noqa: E731
+    pages = [-(-n // P) for n in kv_lens]
+    kc = (torch.randn(sum(pages) + 1, Hkv, P, D, device=dev) * 0.5).to(cache)
+    vc = (torch.randn(sum(pages) + 1, Hkv, D, P, device=dev) * 0.5).to(cache)
+    perm = (torch.randperm(sum(pages), device=dev) + 1).int()
+    bt = torch.zeros(len(pages), max(pages), dtype=torch.int32, device=dev)
+    for i, n in enumerate(pages):
+        bt[i, :n] = perm[sum(pages[:i]):sum(pages[:i]) + n]
+    cu = torch.tensor([sum(q_lens[:i]) for i in range(len(q_lens) + 1)], dtype=torch.int32, device=dev)
+    kl = torch.tensor(kv_lens, dtype=torch.int32, device=dev)
+    q = torch.randn(sum(q_lens), Hq, D, device=dev).to(torch.bfloat16)
+    items, split, comb, chunk, parts = ops.prefill_plan(q_lens, kv_lens, kv_heads=Hkv)
+    assert chunk < 0 and parts > 0
+    plan = ops.PrefillPlan(t(items, 2), t(split, 4), t(comb, 4), chunk, parts)
+    kw = {"softcap": dict(softcap=20.0), "window": dict(window=300), "sinks": dict(sinks=torch.randn(Hq, device=dev))}.get(mode, {})
+    out = ops.paged_prefill(q, kc, vc, bt, cu, kl, plan, 0.0884, **kw)
+    want = ref.paged_prefill(q, kc, vc, bt, cu, kl, 0.0884, kw.get("window", -1), 1.0, 1.0, kw.get("softcap", 0.0),
+                             kw.get("sinks"))
+    # probabilities and output rounded to bf16 once each: 2^-9 of the largest |v| (about 2.3) apiece
+    assert (out.float() - want.float()).abs().max().item() < 2 * 2.0 ** -9 * 2.5
