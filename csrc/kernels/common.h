@@ -157,6 +157,12 @@ __device__ __forceinline__ void kv_st8(typename KVStore<F>::T* p, const float (&
 }
 
 template <int F>
+__device__ __forceinline__ void kv_st4(typename KVStore<F>::T* p, const float (&f)[4]) {
+  if constexpr (F == KV_BF16) *reinterpret_cast<bf16x4*>(p) = bf16x4{(bf16)f[0], (bf16)f[1], (bf16)f[2], (bf16)f[3]};
+  else *reinterpret_cast<uint32_t*>(p) = (uint32_t)fp8_pack2<F, true>(f[2], f[3], fp8_pack2<F, false>(f[0], f[1], 0));
+}
+
+template <int F>
 __device__ __forceinline__ void kv_st1(typename KVStore<F>::T* p, float f) {
   if constexpr (F == KV_BF16) *p = (bf16)f;
   else *p = (uint8_t)(fp8_pack2<F, false>(f, 0.f, 0) & 0xff);
