@@ -5,6 +5,7 @@ native library is missing on a GPU the call raises.
 from __future__ import annotations
 
 import contextlib
+import functools
 import heapq
 import os
 
@@ -167,8 +168,12 @@ def _chunk_rule_ws(T: int, S: int, H: int, G: int, dk: int, dv: int, delta: bool
     where the row-by-row kernels run: one row per sequence (a decode step; a chunk would be 1/32 full), key
     widths other than 64 / 128, value widths not of 16 columns, or key / query rows (the first two
     of ``rows``, the operands and the output) that 16-byte loads cannot take."""
-    if T <= S or dk not in (64, 128) or dv % 16 or state.data_ptr() % 16 or S > 65535 or H > 65535 or \
-            any(r.data_ptr() % 16 or r.stride(0) % 8 for r in rows[:2]) or any(not 0 <= r.stride(0) < 1 << 24 for r in rows):
+    if T <= S or dk not in (64, 128) or dv % 16 or S > 65535 or H > 65535:
+        return None
+    q, k, o = rows[0], rows[1], rows[-1]   # (a shared row stride for q, k and v / B and C)
+    sq, so = q.stride(0), o.stride(0)
+    if (state.data_ptr() | q.data_ptr() | k.data_ptr()) % 16 or sq % 8 or not (0 <= sq < 1 << 24 and 0 <= so < 1 << 24) or \
+            not 0 <= rows[-2].stride(0) < 1 << 24:
         return None
     return torch.empty((T // 32 + S) * load().ome_chunk_rule_floats(H, G, int(delta)), dtype=torch.float32,
                        device=state.device)
@@ -1005,28 +1010,46 @@ class MLAWorkspace:
 
     @classmethod
     def rows(cls, T: int, H: int, DK: int = 576, seqs: int = 1 << 30, pages: int = 1 << 30) -> tuple[int, bool]:
-        """(query rows of a row tile or 0 for the 16-head kernel, whether its tiles are heads of one token) for T
-        tokens of ``seqs`` block-table rows of ``pages`` pages (a bound of every context).  Prompts (at least 4
-        tokens a sequence): rows of neighbouring tokens share a tile.  Taller tiles do more work per LDS read, lower
-        ones start sooner and fill the chip with fewer rows; the fixed cost of a row tile (12..20 us, the
-        16-head kernel 10) loses where there is little to stream.  Device times, 16-head / row tiles: prompts, 16 heads,
-        30 x 30 12 / 21 us, 25 rows at 2000 keys 48 / 32, 120 x 60 25 / 24, 3400 x 1300 750 / 129; decode, 32 heads,
-        8 x 100 keys 11 / 15, 4 x 3000 41 / 31, 48 x 3000 196 / 69; 16 heads, 4 x 3000 21 / 26, 48 x 3000
-        105 / 65; 128 heads, 1 x 500 14 / 15, 8 x 100 23 / 17, 48 x 3000 104 (the tiles before) / 76."""
+        """The first two of :meth:`tiles`."""
+        return cls.tiles(T, H, DK, seqs, pages)[:2]
+
+    @classmethod
+    @functools.lru_cache(maxsize=4096)
+    def tiles(cls, T: int, H: int, DK: int = 576, seqs: int = 1 << 30, pages: int = 1 << 30) -> tuple[int, bool, int]:
+        """(query rows of a row tile or 0 for the 16-head kernel, whether its tiles are heads of one token, partitions)
+        for T tokens of ``seqs`` block-table rows of ``pages`` pages (a bound of every context).
+
+        Prompts (at least 4 tokens a sequence): rows of neighbouring tokens share a tile.  A workgroup has a CU to itself and
+        a wave for every 32 rows, so 128-row tiles use all of the matrix cores, and 32-row ones a quarter, which start
+        sooner and need no partitions to cover the chip with few rows.  Estimated in us for the contexts expected: per
+        launch wave 12 / 14 / 20 to start and drain (32 / 64 / 128 rows) and 0.06 a key; partitions 5, and 0.5 per 1000
+        rows and partition for their fp32 partials.  Device times of 32 / 64 / 128 rows (16-head kernel): 64 heads,
+        4 x 49 of 73 keys 28.5 / 17.2 / 38.5 (33.7), 174 26.4 / 22.6 / 36.2 (40.5), 100 of 3100 238 / 114 / 70 (496);
+        16 heads, 4 x 100 18.9 / 27.2 / 30.8 (35.2), 4 x 200 37.7 / 24.9 / 39.6 (50.9), 20 21.9 / 26.9 / 30.7 (12.2).
+
+        Decode (16-head kernel / row tiles): 16 heads, 32 x 400 keys 19 / 21, 32 x 3000 53 / 46, 64 x 200 29 / 22; 32 heads,
+        8 x 100 11 / 15, 12 x 1000 27 / 24, 48 x 3000 196 / 69; 64 heads, 4 x 2000 22 / 27, 12 x 100 21 / 17; 128 heads,
+        4 x 64 16 / 17, 4 x 500 23 / 20, 8 x 100 23 / 17, 48 x 3000 104 (the tiles before) / 76."""
         n = T * H
-        if DK != 576 or H < 4 or not _MLA_ROW_TILES:
-            return 0, False
-        if T >= 4 * seqs:
-            if n < (1024 if pages <= 32 else 256):
-                return 0, False
-            return (128 if n >= 128 * cls.TARGET_WGS_ALL else 64 if n >= 64 * cls.TARGET_WGS_ALL else 32), False
-        if n < (384 if H < 32 else 192) or (H <= 32 and pages <= 16 and n < 1024):
-            return 0, False
-        return (128 if H > 64 and T >= 16 else 64 if H > 32 and n >= 512 else 32), True
+        if DK == 576 and H >= 4 and _MLA_ROW_TILES:
+            if T >= 4 * seqs:
+                if n >= (512 if pages <= 32 else 256):
+                    keys, best = min(16 * pages, max(1024, 2 * T // seqs)), None
+                    for rows, start in ((32, 12), (64, 14), (128, 20)):
+                        wgs = -(-n // rows)
+                        for p in {1, cls.parts(T, H, DK, rows)}:
+                            us = -(-wgs // cls.TARGET_WGS_ALL) * (start + 0.06 * keys / p) + (p > 1) * (5 + n * p / 2000)
+                            best = min(best or (us, rows, p), (us, rows, p))
+                    return best[1], False, best[2]
+            elif n >= 1024 or (n >= 384 and (pages > 64 if H < 32 else pages > 16 or (H > 32 and n >= 640))):
+                rows = 128 if H > 64 and T >= 16 else 64 if H > 32 and n >= 512 else 32
+                return rows, True, cls.parts(T, H, DK, rows, True)
+        return 0, False, cls.parts(T, H, DK)
 
     @classmethod
     def parts(cls, T: int, H: int, DK: int = 576, rows: int = 0, decode: bool = False) -> int:
-        """Partitions of a tile's keys; for the row tiles of a decode step the most that a tile may get."""
+        """Partitions of a tile's keys; for the row tiles of a decode step the most that a tile may get, for those of
+        prompts the most that fit the chip."""
         if rows and decode:
             units = T * -(-H // rows)
             return 1 if units > cls.TARGET_WGS_ALL else min(cls.MAX_PARTS_ALL, -(-2 * cls.TARGET_WGS_ALL // units))
@@ -1055,10 +1078,9 @@ def mla_attn(q, cache, block_tables, tok_row, kv_lens, scale: float, ws: MLAWork
     assert q.stride(2) == 1 and q.stride(1) == DK and cache.shape[-1] == DK
     if out is None:
         out = torch.empty(T, H, dv, dtype=q.dtype, device=q.device)
-    rows, decode = MLAWorkspace.rows(T, H, DK, *block_tables.shape)
-    if out.data_ptr() % 16 or out.stride(0) % 8:
-        rows, decode = 0, False
-    parts = MLAWorkspace.parts(T, H, DK, rows, decode)
+    rows, decode, parts = MLAWorkspace.tiles(T, H, DK, *block_tables.shape)
+    if rows and (out.data_ptr() % 16 or out.stride(0) % 8):
+        rows, decode, parts = 0, False, MLAWorkspace.parts(T, H, DK)
     if ws is None and (parts > 1 or decode):
         ws = MLAWorkspace(q.device)
     call("ome_mla_attn", q.data_ptr(), q.stride(0), cache.data_ptr(), _i32(block_tables).data_ptr(),
@@ -2040,10 +2062,9 @@ def latent_attn(q, cache, block_tables, tok_row, kv_lens, scale: float, dv: int,
     if out is None:
         out = torch.empty(T, H, dv, dtype=q.dtype, device=q.device)
     assert out.stride(2) == 1 and out.stride(1) == dv
-    rows, decode = MLAWorkspace.rows(T, H, DK, *block_tables.shape)
-    if sinks is not None or window > 0 or out.data_ptr() % 16 or out.stride(0) % 8:
-        rows, decode = 0, False
-    parts = MLAWorkspace.parts(T, H, DK, rows, decode)
+    rows, decode, parts = MLAWorkspace.tiles(T, H, DK, *block_tables.shape)
+    if rows and (sinks is not None or window > 0 or out.data_ptr() % 16 or out.stride(0) % 8):
+        rows, decode, parts = 0, False, MLAWorkspace.parts(T, H, DK)
     if window > 0:   # at least four 32-key tiles of the window per partition (fewer only move partials around)
         parts = max(1, min(parts, window // 128))
     if ws is None and (parts > 1 or decode):

@@ -175,7 +175,7 @@ def test_mla_row_tiles_of_prompts(monkeypatch, seqs, H, rows):
     row = torch.tensor([s for s, (_, n) in enumerate(seqs) for _ in range(n)], dtype=torch.int32)
     kl = torch.tensor([a + j + 1 for a, n in seqs for j in range(n)], dtype=torch.int32)
     q = torch.randn(len(row), H, 576, device=DEV).to(torch.bfloat16)
-    monkeypatch.setattr(ops.MLAWorkspace, "rows", classmethod(lambda cls, *a: (rows, False)))
+    monkeypatch.setattr(ops.MLAWorkspace, "tiles", lambda T, H, DK, *a: (rows, False, ops.MLAWorkspace.parts(T, H, DK, rows)))
     out = ops.mla_attn(q, cache, bt, row.to(DEV), kl.to(DEV), 0.06)
     want = _exact(q, cache, bt, row, kl, 0.06)
     # probabilities and the output are rounded to bf16 once each: 2^-9 of the largest value they sum, and of the result
@@ -193,7 +193,22 @@ def test_mla_row_tiles_of_decode_steps(monkeypatch, lens, H, rows):
     cache, bt = _setup(lens)
     q = torch.randn(len(lens), H, 576, device=DEV).to(torch.bfloat16)
     row, kl = torch.arange(len(lens), dtype=torch.int32), torch.tensor(lens, dtype=torch.int32)
-    monkeypatch.setattr(ops.MLAWorkspace, "rows", classmethod(lambda cls, *a: (rows, True)))
+    monkeypatch.setattr(ops.MLAWorkspace, "tiles", lambda T, H, DK, *a: (rows, True, ops.MLAWorkspace.parts(T, H, DK, rows, True)))
     out = ops.mla_attn(q, cache, bt, row.to(DEV), kl.to(DEV), 0.06)
     want = _exact(q, cache, bt, row, kl, 0.06)
     assert (out.cpu().double() - want).abs().max() < 2.0 ** -8 * cache.float().abs().max().item()
+
+
+def test_mla_tile_rule_fits_workspace_and_chip():
+    """Tiles of prompts fill at most one launch wave when partitioned; partials fit the workspace."""
+    W = ops.MLAWorkspace
+    for H in (4, 16, 20, 64, 128):
+        for T in (1, 3, 4, 7, 30, 63, 64, 200, 700, 5000):
+            for seqs in (1, 2, 7, 64, 600):
+                for pages in (1, 2, 16, 17, 64, 65, 1024):
+                    rows, decode, parts = W.tiles(T, H, 576, seqs, pages)
+                    assert rows in (0, 32, 64, 128) and parts >= 1 and (rows or not decode)
+                    if rows and not decode and parts > 1:
+                        wgs = -(-T * H // rows)
+                        assert wgs * parts <= W.TARGET_WGS_ALL and wgs * rows * parts <= W.ROWS
+                    assert W.tiles(T, H, 288, seqs, pages)[0] == 0
