@@ -163,6 +163,11 @@ def dyn_conv1d(x: torch.Tensor, kern: torch.Tensor, state: torch.Tensor, cu, slo
     return out
 
 
+@functools.lru_cache(maxsize=256)
+def _chunk_rule_floats(H: int, G: int, delta: bool) -> int:
+    return load().ome_chunk_rule_floats(H, G, int(delta))
+
+
 def _chunk_rule_ws(T: int, S: int, H: int, G: int, dk: int, dv: int, delta: bool, state: torch.Tensor, rows: tuple) -> torch.Tensor | None:
     """Workspace of the chunked kernels (``chunk_rule.hip``) for T rows of S sequences and H heads, or None
     where the row-by-row kernels run: one row per sequence (a decode step; a chunk would be 1/32 full), key
@@ -175,8 +180,7 @@ def _chunk_rule_ws(T: int, S: int, H: int, G: int, dk: int, dv: int, delta: bool
     if (state.data_ptr() | q.data_ptr() | k.data_ptr()) % 16 or sq % 8 or not (0 <= sq < 1 << 24 and 0 <= so < 1 << 24) or \
             not 0 <= rows[-2].stride(0) < 1 << 24:
         return None
-    return torch.empty((T // 32 + S) * load().ome_chunk_rule_floats(H, G, int(delta)), dtype=torch.float32,
-                       device=state.device)
+    return torch.empty((T // 32 + S) * _chunk_rule_floats(H, G, delta), dtype=torch.float32, device=state.device)
 
 
 def ssm_scan(x, dt, B, C, A, D, dt_bias, dt_min: float, state, cu, slot, reset, H: int, P: int, N: int, G: int,
@@ -189,7 +193,7 @@ def ssm_scan(x, dt, B, C, A, D, dt_bias, dt_min: float, state, cu, slot, reset, 
         return ref.ssm_scan(x, dt, B, C, A, D, dt_bias, dt_min, state, cu, slot, reset, H, P, N, G, out)
     assert B.stride(0) == C.stride(0) and B.stride(1) == 1 and x.stride(1) == 1 and dt.stride(1) == 1
     f32 = _f32(x, dt, B, C, out)
-    ws = None if f32 or H % G else _chunk_rule_ws(T, slot.shape[0], H, G, N, P, False, state, (B, C, x, out))
+    ws = None if f32 or T <= slot.shape[0] or H % G else _chunk_rule_ws(T, slot.shape[0], H, G, N, P, False, state, (B, C, x, out))
     if ws is not None:
         call("ome_ssm_chunks", x.data_ptr(), x.stride(0), dt.data_ptr(), dt.stride(0), B.data_ptr(), C.data_ptr(),
              B.stride(0), A.data_ptr(), D.data_ptr(), dt_bias.data_ptr(), float(dt_min), state.data_ptr(), out.data_ptr(),
@@ -220,14 +224,15 @@ def gdn_scan(q, k, v, a, b, A_log, dt_bias, state, cu, slot, reset, Hv: int, Hk:
     assert q.stride(1) == k.stride(1) == v.stride(1) == a.stride(1) == 1 and out.stride(1) == 1
     assert state.is_contiguous() and state.dtype == torch.float32
     f32 = _f32(q, k, v, a, b, out)
-    ws = None if v1 or f32 or Hk <= 0 or Hv % Hk else _chunk_rule_ws(T, slot.shape[0], Hv, Hk, dk, dv, True, state, (q, k, out))
+    S = slot.shape[0]
+    ws = None if T <= S or v1 or f32 or Hk <= 0 or Hv % Hk else _chunk_rule_ws(T, S, Hv, Hk, dk, dv, True, state, (q, k, v, out))
     if ws is not None:   # prompts: chunks of 32 rows on the matrix cores
         call("ome_gdn_chunks", q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), a.data_ptr(), b.data_ptr(),
              a.stride(0), A_log.data_ptr(), dt_bias.data_ptr(), state.data_ptr(), out.data_ptr(), out.stride(0),
              _i32(cu).data_ptr(), _i32(slot).data_ptr(), _i32(reset).data_ptr(), slot.shape[0], T, Hv, Hk, dk, dv,
              ws.data_ptr(), stream_ptr())
         return out
-    if not v1 and not f32 and T == slot.shape[0] and dk in (64, 128, 256) and 0 < Hv <= 65535 and Hk > 0 and Hv % Hk == 0 and \
+    if T == S and not v1 and not f32 and dk in (64, 128, 256) and 0 < Hv <= 65535 and Hk > 0 and Hv % Hk == 0 and \
             q.data_ptr() % 16 == 0 and k.data_ptr() % 16 == 0 and q.stride(0) % 8 == 0 and 0 < dv < 1 << 20:
         # a decode step: the normalisation inside the scan (47.9 -> 43.9 us at 64 sequences of 32 heads)
         call("ome_gdn_step", q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), a.data_ptr(), b.data_ptr(),
