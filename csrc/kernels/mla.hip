@@ -204,18 +204,17 @@ __global__ __launch_bounds__(256) void mla_attn_kernel(
 }
 
 // One wave's share of a latent page's move to LDS: 64 lanes x 16 bytes from `off` (per lane) of the page at `base`
-// to `lds` + 16 lane.  By asm, because the compiler takes every later LDS read of the image's array for a reader of
+// to LDS address `lds` + 16 lane.  By asm, because the compiler takes every later LDS read of the image's array for a reader of
 // the move and waits for all of it (vmcnt 0) there; the kernels below wait themselves, once, before the barrier
 // after which a tile is read.  (No register is written; the descriptor's size bounds the reads to the page.)
-__device__ __forceinline__ void page_to_lds(const bf16* base, uint32_t bytes, uint32_t off, const void* lds) {
+__device__ __forceinline__ void page_to_lds(const bf16* base, uint32_t bytes, uint32_t off, uint32_t lds) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   const uint64_t b = (uint64_t)base;
   const u32x4 rs = {(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, bytes, 0x00020000u};
-  const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)lds;
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
                :
-               : "s"(__builtin_amdgcn_readfirstlane(at)), "v"(off), "s"(rs)
+               : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(off), "s"(rs)
                : "m0", "memory");
 #endif
 }
@@ -224,8 +223,10 @@ __device__ __forceinline__ void page_to_lds(const bf16* base, uint32_t bytes, ui
 // Row tiles: one workgroup of NW waves owns 32 * NW neighbouring query rows (row = token * H + head) and one
 // split-K partition, so that each latent key tile is streamed and staged in LDS ONCE for all of them: the heads
 // of one token in decode, the heads of several prompt tokens of a sequence otherwise (the 16-head
-// kernel above streams the prefix again for every token, and its four waves each compute the same S^T).  A tile
-// whose tokens belong to different block-table rows walks those rows one after the other, its other tokens masked.
+// kernel above streams the prefix again for every token, and its four waves each compute the same S^T).  A workgroup
+// takes the tokens of one block-table row only: the tile's own the first, one more for each sequence that begins inside
+// a tile.  The others' rows ride along with weights 0 and are not stored (0 times an infinite or NaN value of a
+// broken sequence is NaN, which must stay in that sequence).
 //
 // Bound by the matrix cores, with LDS reads close behind: a wave owns 32 rows and all DV value dims, so each
 // LDS operand feeds 32 columns (16 rows a wave, the layout before, read every key tile eight times per
@@ -265,11 +266,78 @@ __device__ __forceinline__ void mma_acc(f32x16& c, bf16x8 a, bf16x8 b) {   // c 
 #endif
 }
 
-template <int DK, int DV, int NW>
+// First token whose block-table row is e, by a 64-way search of the whole wave; -1: none.  tok_row ascends in the
+// runtime's prompts; of rows in any other order it may miss e, the same way for every caller.
+__device__ __forceinline__ int first_token(const int* __restrict__ tok_row, int T, int e) {
+  const int lane = threadIdx.x & 63;
+  int lo = 0, n = T;   // it is in [lo, lo + n]
+  while (n > 0) {
+    const int step = (n + 63) >> 6, d = lane * step;
+    const uint64_t rest = __ballot(d >= n || tok_row[lo + d] >= e);
+    const int k = rest ? __builtin_ctzll(rest) : 64;   // tokens before lane k's are below e
+    if (k == 0) break;
+    const int at = (k - 1) * step + 1;
+    n = min(k * step, n) - at;
+    lo += at;
+  }
+  lo = __builtin_amdgcn_readfirstlane(lo);
+  return lo < T && tok_row[lo] == e ? lo : -1;
+}
+
+// One query row over L keys by one wave, lane = key, then 8 value dims: to `out`, or as a partial in the row tiles' layout
+template <int DK, int DV>
+__device__ __forceinline__ void plain_row(const bf16* q, const bf16* cache, const int* bt, int L, float scale_log2, bool whole,
+                                          bf16* out, float* part_o, float* part_ml) {
+  const int lane = threadIdx.x & 63;
+  float m = OME_NEG_INF, l = 0.f, acc[8] = {};
+  for (int k0 = 0; k0 < L; k0 += 64) {
+    const int key = min(k0 + lane, L - 1);
+    const bf16* kv = cache + ((int64_t)bt[key >> 4] * 16 + (key & 15)) * DK;
+    float s = 0.f;
+#pragma unroll 1
+    for (int c = 0; c < DK; c += 8) {
+      const bf16x8 a = ld8(q + c), b = ld8(kv + c);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s += (float)a[e] * (float)b[e];
+    }
+    s = k0 + lane < L ? s * scale_log2 : OME_NEG_INF;
+    float mn = fmaxf(m, s);
+    for (int x = 32; x > 0; x >>= 1) mn = fmaxf(mn, __shfl_xor(mn, x));
+    const float alpha = m == OME_NEG_INF ? 0.f : __builtin_amdgcn_exp2f(m - mn);
+    const float p = mn == OME_NEG_INF ? 0.f : __builtin_amdgcn_exp2f(s - mn);
+    float ps = p;
+    for (int x = 32; x > 0; x >>= 1) ps += __shfl_xor(ps, x);
+    l = l * alpha + ps;
+    m = mn;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] *= alpha;
+#pragma unroll 1
+    for (int j = 0; j < min(64, L - k0); ++j) {
+      const float w = __shfl(p, j);
+      const bf16x8 v = ld8(cache + ((int64_t)bt[(k0 + j) >> 4] * 16 + ((k0 + j) & 15)) * DK + 8 * lane);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] += w * (float)v[e];
+    }
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  static_assert(DV == 512, "8 dims a lane");
+  if (whole) {
+    bf16x8 o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = (bf16)(acc[e] * inv);
+    st8(out + 8 * lane, o);
+  } else {   // dims 8 lane .. + 3 belong to the tile's lane (row, half 0), the next four to (row, half 1)
+    *reinterpret_cast<f32x4*>(part_o + lane * 256) = f32x4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
+    *reinterpret_cast<f32x4*>(part_o + lane * 256 + 128) = f32x4{acc[4] * inv, acc[5] * inv, acc[6] * inv, acc[7] * inv};
+    if (lane == 0) part_ml[0] = m, part_ml[1] = l;
+  }
+}
+
+template <int DK, int DV, int NW, bool DECODE>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1))) void mla_attn_rows_kernel(
     const bf16* __restrict__ q, int64_t q_stride_t, const bf16* __restrict__ cache,
     const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ tok_row,
-    const int* __restrict__ kv_lens, int T, int H, float scale_log2, int parts, int2* __restrict__ plan,
+    const int* __restrict__ kv_lens, int T, int H, int seqs, float scale_log2, int parts, int2* __restrict__ plan,
     bf16* __restrict__ out, int64_t out_stride_t, float* __restrict__ ws_o, float* __restrict__ ws_ml) {
   static_assert(DK == 576 && lds_chunks<DK>() == DK / 8, "LDS DMA image assumes unpadded 72-chunk rows");
   constexpr int CH = DK / 8, NI = KT * CH / 64, NJ = NI / NW, NV = DV / 32, NS = DK / 16;
@@ -278,14 +346,23 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
   constexpr float LAZY = 8.f;
   constexpr int AHEAD = 4;            // LDS operands in flight: 4 x 32 cycles of matrix work cover a read
   __shared__ __attribute__((aligned(16))) char sK[3 * IMG];
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)sK;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int col = lane & 31, hf = lane >> 5;
   constexpr int RT = 32 * NW, SPAN = 2, UNITS = 256;
-  // `plan`: a tile is RT heads of one token, and contexts are cut by length (decode); else RT rows of [T * H]
-  const bool decode = plan != nullptr;
+  // DECODE: a tile is RT heads of one token, and contexts are cut by length; else RT rows of [T * H], and the
+  // workgroups past the tiles (`own_seq`) take a sequence's first rows where it begins inside a tile
   const int R = T * H, HG = (H + RT - 1) / RT;
-  int unit = decode ? blockIdx.x : gridDim.x - 1 - blockIdx.x, part = blockIdx.y, my_parts = parts;   // (longest rows first)
-  if (decode && parts > 1) {
+  int unit = DECODE ? blockIdx.x : gridDim.x - 1 - blockIdx.x, part = blockIdx.y, my_parts = parts;   // (longest rows first)
+  int own_seq = 0, own_first = 0;
+  if constexpr (!DECODE) {
+    own_seq = max(unit - (R + RT - 1) / RT + 1, 0);
+    if (own_seq > 0) {
+      own_first = first_token(tok_row, T, own_seq);
+      if (own_first < 0) return;   // whole block
+      unit = (int)((int64_t)own_first * H / RT);
+    }
+  }
+  if (DECODE && parts > 1) {
     // Workgroup w of 256 takes piece w.  The span is the smallest number of key tiles that cuts all units
     // into at most 256 pieces: one a CU (also within each XCD, to which workgroups go in turn), and none longer
     // than it has to be, however ragged the contexts.  Every wave finds it from the lengths: lane l holds
@@ -335,79 +412,28 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
     unit = tok * HG + hg;
     if (part == 0 && tid == 0) plan[unit] = int2{w, my_parts};
   }
-  const int row0 = decode ? unit / HG * H + unit % HG * RT : unit * RT;
-  const int row_end = decode ? (unit / HG + 1) * H : R;
-  const int row = row0 + wave * 32 + col;                           // this lane's row (S^T / O^T column)
-  const bool hv = row < row_end;
-  const int t = min(decode ? unit / HG : row / H, T - 1), head = hv ? row - t * H : 0;
-  const int my_row = tok_row[t], my_len = hv ? kv_lens[t] : 0;
-
-  // Key tile -> LDS image: instruction i writes chunks [64 i, 64 i + 64) lane-linearly, each lane fetching the source
-  // chunk that the row's XOR swizzle puts there.  A page is 16 rows x 72 chunks = 18 instructions, so each
-  // instruction reads one page: its descriptor is based at that page.
-  auto dma = [&](const int* bt, int n_pages, int tile, int img) {
-    const int p0 = 2 * tile, p1 = p0 + 1;
-    const bf16* b0 = cache + (int64_t)bt[p0 < n_pages ? p0 : 0] * 16 * DK;
-    const bf16* b1 = cache + (int64_t)bt[p1 < n_pages ? p1 : 0] * 16 * DK;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int i = wave + NW * j, c = 64 * i + lane, kr = c / CH, xl = c - kr * CH;
-      page_to_lds(i < NI / 2 ? b0 : b1, 16 * DK * 2, (uint32_t)(((kr & 15) * CH + (xl ^ (kr & 7))) * 16),
-                  sK + img * IMG + 64 * 16 * i);
-    }
-  };
-
-  bf16x8 qf[NS];
-  const bf16* qp = q + (int64_t)t * q_stride_t + (int64_t)head * DK + 8 * hf;
-#pragma unroll
-  for (int s = 0; s < NS; ++s) qf[s] = ld8(qp + 16 * s);
-
-  f32x16 o[NV];
-#pragma unroll
-  for (int v = 0; v < NV; ++v)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) o[v][i] = 0.f;
-  float m = OME_NEG_INF, lsum = 0.f;
-
-  // LDS lane bases; the XOR swizzle acts on the low three bits of a chunk index, the rest are immediates.
-  // S^T reads chunk 2 s + hf of key row col; V^T reads, for 16-lane group gr = lane / 16, rows 4 hf + qr (+ 8, 16, 24)
-  // and chunk 4 v + 2 (gr & 1) + pc / 2.
-  const int gr = lane >> 4, qr = (lane & 15) >> 2, pc = lane & 3;
-  uint32_t sofs[4], vofs[2];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) sofs[e] = (col * CH + ((2 * e + hf) ^ (col & 7))) * 16;
-#pragma unroll
-  for (int e = 0; e < 2; ++e)
-    vofs[e] = ((4 * hf + qr) * CH + ((4 * e + 2 * (gr & 1) + (pc >> 1)) ^ (4 * hf + qr))) * 16 + (pc & 1) * 8;
-  auto kfrag = [&](uint32_t img, int s) { return *reinterpret_cast<const bf16x8*>(sK + (sofs[s & 3] + img) + (s >> 2) * 128); };
-  auto score = [&](uint32_t img) {   // S^T of the tile in image `img` (byte offset)
-    f32x16 a;
-    bf16x8 k[AHEAD];   // operands on their way from LDS
-#pragma unroll
-    for (int s = 0; s < AHEAD; ++s) k[s] = kfrag(img, s);
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      if (s == 0) mma_new(a, k[0], qf[0]);
-      else mma_add(a, k[s % AHEAD], qf[s]);
-      if (s + AHEAD < NS) k[s % AHEAD] = kfrag(img, s + AHEAD);
-    }
-    asm volatile(MMA_WAIT : "+v"(a));
-    return a;
-  };
-  auto vfrag = [&](uint32_t img, int v, int st) {
-    const int at = vofs[v & 1] + img + (v >> 1) * 128 + st * 16 * CH * 16;
-    const bf16x4 x = tr_read(reinterpret_cast<const bf16*>(sK), at), y = tr_read(reinterpret_cast<const bf16*>(sK), at + 8 * CH * 16);
-    return bf16x8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
-  };
-
+  const int row0 = DECODE ? unit / HG * H + unit % HG * RT : unit * RT;
+  const int row_end = DECODE ? (unit / HG + 1) * H : R;
   // the tile's tokens (at most 64: H >= 4), one a lane; the same in every wave
   const int t0 = row0 / H, nt = (min(row0 + RT, row_end) - 1) / H - t0 + 1;
   const int tl_row = tok_row[t0 + min(lane, nt - 1)], tl_len = kv_lens[t0 + min(lane, nt - 1)];
   uint64_t left = nt >= 64 ? ~0ull : (1ull << nt) - 1;
-  while (left) {   // block-table rows of the tile; each pass takes at least one token off `left`
-    const int bt_row = __builtin_amdgcn_readlane(tl_row, __builtin_ctzll(left));
-    const bool same = ((left >> lane) & 1) && tl_row == bt_row;
-    left &= ~__ballot(same);
+  if (own_seq > 0) {
+    const uint64_t theirs = left & __ballot(tl_row == own_seq);
+    if (own_first == t0 || own_first != t0 + __builtin_ctzll(theirs)) return;   // the tile's own workgroup takes them
+    left = theirs;
+  }
+  // One pass: block-table row `bt_row`, whose tokens `same` marks
+  const auto walk = [&](int bt_row, bool same, int lane) __attribute__((always_inline)) {
+    const int col = lane & 31, hf = lane >> 5;
+    const int row = row0 + wave * 32 + col;                           // this lane's row (S^T / O^T column)
+    const bool hv = row < row_end;
+    const int t = min(DECODE ? unit / HG : row / H, T - 1), head = hv ? row - t * H : 0;
+    const int my_row = tok_row[t], my_len = hv ? kv_lens[t] : 0;
+    bf16x8 qf[NS];
+    const bf16* qp = q + (int64_t)t * q_stride_t + (int64_t)head * DK + 8 * hf;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) qf[s] = ld8(qp + 16 * s);
     int Lmax = same ? tl_len : 0;
 #pragma unroll
     for (int x = 32; x > 0; x >>= 1) Lmax = max(Lmax, __shfl_xor(Lmax, x));
@@ -415,14 +441,71 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
     const int* bt = block_tables + (int64_t)bt_row * bt_stride;
     const int n_pages = (Lmax + 15) >> 4, tiles = (n_pages + 1) >> 1, per = (tiles + my_parts - 1) / my_parts;
     const int begin = part * per, end = min(tiles, begin + per);
-    if (begin >= end) continue;
-    const int L = my_row == bt_row ? my_len : 0;
+    // Key tile -> LDS image: instruction i writes chunks [64 i, 64 i + 64) lane-linearly, each lane fetching the source
+    // chunk that the row's XOR swizzle puts there.  A page is 16 rows x 72 chunks = 18 instructions, so each
+    // instruction reads one page: its descriptor is based at that page.
+    auto dma = [&](const int* bt, int n_pages, int tile, int img) {
+      const int p0 = 2 * tile, p1 = p0 + 1;
+      const bf16* b0 = cache + (int64_t)bt[p0 < n_pages ? p0 : 0] * 16 * DK;
+      const bf16* b1 = cache + (int64_t)bt[p1 < n_pages ? p1 : 0] * 16 * DK;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int i = wave + NW * j, c = 64 * i + lane, kr = c / CH, xl = c - kr * CH;
+        page_to_lds(i < NI / 2 ? b0 : b1, 16 * DK * 2, (uint32_t)(((kr & 15) * CH + (xl ^ (kr & 7))) * 16),
+                    lds0 + img * IMG + 64 * 16 * i);
+      }
+    };
 
-    dma(bt, n_pages, begin, 0);
-    if (begin + 1 < end) dma(bt, n_pages, begin + 1, 1);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    f32x16 sc = score(0);
+    f32x16 o[NV];
+
+    // LDS lane bases; the XOR swizzle acts on the low three bits of a chunk index, the rest are immediates.
+    // S^T reads chunk 2 s + hf of key row col; V^T reads, for 16-lane group gr = lane / 16, rows 4 hf + qr (+ 8, 16, 24)
+    // and chunk 4 v + 2 (gr & 1) + pc / 2.
+    const int gr = lane >> 4, qr = (lane & 15) >> 2, pc = lane & 3;
+    uint32_t sofs[4], vofs[2];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sofs[e] = (col * CH + ((2 * e + hf) ^ (col & 7))) * 16;
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      vofs[e] = ((4 * hf + qr) * CH + ((4 * e + 2 * (gr & 1) + (pc >> 1)) ^ (4 * hf + qr))) * 16 + (pc & 1) * 8;
+    auto kfrag = [&](uint32_t img, int s) { return *reinterpret_cast<const bf16x8*>(sK + (sofs[s & 3] + img) + (s >> 2) * 128); };
+    auto score = [&](uint32_t img) {   // S^T of the tile in image `img` (byte offset)
+      f32x16 a;
+      bf16x8 k[AHEAD];   // operands on their way from LDS
+#pragma unroll
+      for (int s = 0; s < AHEAD; ++s) k[s] = kfrag(img, s);
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        if (s == 0) mma_new(a, k[0], qf[0]);
+        else mma_add(a, k[s % AHEAD], qf[s]);
+        if (s + AHEAD < NS) k[s % AHEAD] = kfrag(img, s + AHEAD);
+      }
+      asm volatile(MMA_WAIT : "+v"(a));
+      return a;
+    };
+    auto vfrag = [&](uint32_t img, int v, int st) {
+      const int at = vofs[v & 1] + img + (v >> 1) * 128 + st * 16 * CH * 16;
+      const bf16x4 x = tr_read(reinterpret_cast<const bf16*>(sK), at), y = tr_read(reinterpret_cast<const bf16*>(sK), at + 8 * CH * 16);
+      return bf16x8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+    };
+
+    const bool mine = hv && my_row == bt_row;
+    const int L = mine ? my_len : 0;
+    float m = OME_NEG_INF, lsum = 0.f;
+    f32x16 sc;
+    if (begin < end) {
+      dma(bt, n_pages, begin, 0);
+      if (begin + 1 < end) dma(bt, n_pages, begin + 1, 1);
+    }
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[v][i] = 0.f;
+    if (begin < end) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      sc = score(0);
+    }
     int cur = 0;
     for (int n = begin; n < end; ++n) {
       const int nxt = cur == 2 ? 0 : cur + 1;
@@ -490,57 +573,80 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
       asm volatile(MMA_WAIT "\n\ts_waitcnt vmcnt(0)" ::: "memory");   // tile n + 2 has landed
       __syncthreads();
     }
-  }
 
-  // ---- epilogue: O^T lane map dim = 32 v + 8 (i / 4) + 4 hf + i % 4, row = col ----
-  const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
-  if (my_parts == 1 && NW == 4 && !decode) {
-    // through LDS (the images are done with): 32 rows x 256 dims at a time, so that rows leave in 512-byte runs
-    // instead of 8-byte pieces (prompts of 128-row tiles 3..5% faster; lower tiles and decode steps not)
-    constexpr int LD = DV / 2 + 8;   // padded row
-    static_assert(NW * 32 * LD * 2 <= (int)sizeof(sK), "the output fits the images");
-    bf16* so = reinterpret_cast<bf16*>(sK) + wave * 32 * LD;
+    // ---- epilogue: O^T lane map dim = 32 v + 8 (i / 4) + 4 hf + i % 4, row = col ----
+    const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+    if (my_parts == 1 && NW == 4 && !DECODE) {
+      // through LDS (the images are done with): 32 rows x 256 dims at a time, so that rows leave in 512-byte runs
+      // instead of 8-byte pieces (prompts of 128-row tiles 3..5% faster; lower tiles and decode steps not)
+      constexpr int LD = DV / 2 + 8;   // padded row
+      static_assert(NW * 32 * LD * 2 <= (int)sizeof(sK), "the output fits the images");
+      bf16* so = reinterpret_cast<bf16*>(sK) + wave * 32 * LD;
+      const uint64_t own = __ballot(mine);
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the first half's reads
+      for (int half = 0; half < 2; ++half) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the first half's reads
 #pragma unroll
-      for (int v = 0; v < NV / 2; ++v)
+        for (int v = 0; v < NV / 2; ++v)
 #pragma unroll
-        for (int i = 0; i < 16; i += 4) {
-          const f32x16& x = o[half * (NV / 2) + v];
-          *reinterpret_cast<bf16x4*>(so + col * LD + 32 * v + 2 * i + 4 * hf) =
-              bf16x4{(bf16)(x[i] * inv), (bf16)(x[i + 1] * inv), (bf16)(x[i + 2] * inv), (bf16)(x[i + 3] * inv)};
-        }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (a wave's own rows: no barrier)
-      for (int i = 0; i < 16; ++i) {
-        const int lr = 2 * i + hf, r = row0 + wave * 32 + lr;
-        if (r < row_end) {
-          const int tt = r / H;
-          st8(out + (int64_t)tt * out_stride_t + (int64_t)(r - tt * H) * DV + half * (DV / 2) + 8 * col, ld8(so + lr * LD + 8 * col));
+          for (int i = 0; i < 16; i += 4) {
+            const f32x16& x = o[half * (NV / 2) + v];
+            *reinterpret_cast<bf16x4*>(so + col * LD + 32 * v + 2 * i + 4 * hf) =
+                bf16x4{(bf16)(x[i] * inv), (bf16)(x[i + 1] * inv), (bf16)(x[i + 2] * inv), (bf16)(x[i + 3] * inv)};
+          }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (a wave's own rows: no barrier)
+#pragma unroll 4
+        for (int i = 0; i < 16; ++i) {
+          const int lr = 2 * i + hf, r = row0 + wave * 32 + lr;
+          if ((own >> lr) & 1) {
+            const int tt = r / H;
+            st8(out + (int64_t)tt * out_stride_t + (int64_t)(r - tt * H) * DV + half * (DV / 2) + 8 * col, ld8(so + lr * LD + 8 * col));
+          }
         }
       }
+    } else if (!mine) {
+      // written by its own pass
+    } else if (my_parts == 1) {
+      bf16* op = out + (int64_t)t * out_stride_t + (int64_t)head * DV + 4 * hf;
+#pragma unroll
+      for (int v = 0; v < NV; ++v)
+#pragma unroll
+        for (int i = 0; i < 16; i += 4)
+          *reinterpret_cast<bf16x4*>(op + 32 * v + 2 * i) = bf16x4{(bf16)(o[v][i] * inv), (bf16)(o[v][i + 1] * inv),
+                                                                   (bf16)(o[v][i + 2] * inv), (bf16)(o[v][i + 3] * inv)};
+    } else {   // partials in the lanes' own order: 1 KiB a store (mla_reduce_rows_kernel reads them so)
+      const int64_t slot = DECODE ? blockIdx.x : (int64_t)unit * parts + part;
+      float* wp = ws_o + (slot * NW + wave) * (32 * DV) + 4 * lane;
+#pragma unroll
+      for (int v = 0; v < NV; ++v)
+#pragma unroll
+        for (int i = 0; i < 16; i += 4)
+          *reinterpret_cast<f32x4*>(wp + (4 * v + i / 4) * 256) =
+              f32x4{o[v][i] * inv, o[v][i + 1] * inv, o[v][i + 2] * inv, o[v][i + 3] * inv};
+      if (hf == 0) {
+        ws_ml[2 * (slot * RT + wave * 32 + col)] = m;
+        ws_ml[2 * (slot * RT + wave * 32 + col) + 1] = lsum;
+      }
     }
-  } else if (my_parts == 1) {
-    if (!hv) return;
-    bf16* op = out + (int64_t)t * out_stride_t + (int64_t)head * DV + 4 * hf;
-#pragma unroll
-    for (int v = 0; v < NV; ++v)
-#pragma unroll
-      for (int i = 0; i < 16; i += 4)
-        *reinterpret_cast<bf16x4*>(op + 32 * v + 2 * i) = bf16x4{(bf16)(o[v][i] * inv), (bf16)(o[v][i + 1] * inv),
-                                                                 (bf16)(o[v][i + 2] * inv), (bf16)(o[v][i + 3] * inv)};
-  } else {   // partials in the lanes' own order: 1 KiB a store (mla_reduce_rows_kernel reads them so)
-    const int64_t slot = decode ? blockIdx.x : (int64_t)unit * parts + part;
-    float* wp = ws_o + (slot * NW + wave) * (32 * DV) + 4 * lane;
-#pragma unroll
-    for (int v = 0; v < NV; ++v)
-#pragma unroll
-      for (int i = 0; i < 16; i += 4)
-        *reinterpret_cast<f32x4*>(wp + (4 * v + i / 4) * 256) =
-            f32x4{o[v][i] * inv, o[v][i + 1] * inv, o[v][i + 2] * inv, o[v][i + 3] * inv};
-    if (hf == 0) {
-      ws_ml[2 * (slot * RT + wave * 32 + col)] = m;
-      ws_ml[2 * (slot * RT + wave * 32 + col) + 1] = lsum;
+  };
+  const int bt0 = __builtin_amdgcn_readlane(tl_row, __builtin_ctzll(left));
+  const bool same0 = ((left >> lane) & 1) && tl_row == bt0;
+  left &= ~__ballot(same0);
+  walk(bt0, same0, lane);
+  // Tokens of further block-table rows: an `own_seq` workgroup takes them, unless they are not in order.  (Those go one
+  // row at a time: a second pass here would hold its operands over the first one's epilogue, in scratch.)
+  if constexpr (!DECODE) {
+    for (; left; left &= left - 1) {
+      const int at = __builtin_ctzll(left), bt_row = __builtin_amdgcn_readlane(tl_row, at), tok = t0 + at;
+      const int first = t0 + __builtin_ctzll(__ballot(lane < nt && tl_row == bt_row));
+      if (bt_row > 0 && bt_row < seqs && first_token(tok_row, T, bt_row) == first) continue;
+      const int lo = max(row0 + wave * 32, tok * H), hi = min(min(row0 + wave * 32 + 32, row_end), (tok + 1) * H);
+      for (int row = lo; row < hi; ++row)
+        plain_row<DK, DV>(q + (int64_t)tok * q_stride_t + (int64_t)(row - tok * H) * DK, cache, block_tables + (int64_t)bt_row * bt_stride,
+                          part == 0 ? kv_lens[tok] : 0, scale_log2, my_parts == 1,
+                          out + (int64_t)tok * out_stride_t + (int64_t)(row - tok * H) * DV,
+                          ws_o + (((int64_t)unit * parts + part) * NW + wave) * (32 * DV) + 4 * ((row - row0) & 31),
+                          ws_ml + 2 * (((int64_t)unit * parts + part) * RT + row - row0));
     }
   }
 }
@@ -643,19 +749,20 @@ __global__ __launch_bounds__(128) void mla_reduce_kernel(const float* __restrict
 template <int DK, int DV>
 static void mla_launch(const void* q, int64_t q_stride_t, const void* cache, const int* block_tables, int bt_stride,
                        const int* tok_row, const int* kv_lens, int T, int H, float scale_log2, int parts, void* out,
-                       int64_t out_stride_t, float* ws_o, float* ws_ml, hipStream_t stream, int rows = 0,
+                       int64_t out_stride_t, float* ws_o, float* ws_ml, hipStream_t stream, int rows = 0, int seqs = 1,
                        int2* plan = nullptr, const float* sinks = nullptr, int window = -1) {
   // `rows`: query rows of a workgroup of the row-tile kernel (32 / 64 / 128, the caller's choice), 0: the
   // 16-head kernel, which alone has the sink term and the window
   if constexpr (DK == 576) {
     if (rows > 0) {
       const unsigned units = (unsigned)(plan ? T * ((H + rows - 1) / rows) : ((int64_t)T * H + rows - 1) / rows);
-      const dim3 grid(plan && parts > 1 ? 256 : units, plan ? 1 : parts);
+      const dim3 grid(plan && parts > 1 ? 256 : units + (plan || seqs < 2 ? 0 : seqs - 1), plan ? 1 : parts);
 #define MLA_ROWS(NW)                                                                                                    \
   {                                                                                                                      \
-    mla_attn_rows_kernel<DK, DV, NW><<<grid, 64 * NW, 0, stream>>>(                                                      \
-        (const bf16*)q, q_stride_t, (const bf16*)cache, block_tables, bt_stride, tok_row, kv_lens, T, H, scale_log2,      \
-        parts, plan, (bf16*)out, out_stride_t, ws_o, ws_ml);                                                             \
+    const auto kernel = plan ? mla_attn_rows_kernel<DK, DV, NW, true> : mla_attn_rows_kernel<DK, DV, NW, false>;          \
+    kernel<<<grid, 64 * NW, 0, stream>>>((const bf16*)q, q_stride_t, (const bf16*)cache, block_tables, bt_stride,         \
+                                         tok_row, kv_lens, T, H, seqs, scale_log2, parts, plan, (bf16*)out,               \
+                                         out_stride_t, ws_o, ws_ml);                                                     \
     if (parts > 1)                                                                                                       \
       mla_reduce_rows_kernel<DV, NW><<<dim3(units * NW, DV / 32), 256, 0, stream>>>(ws_o, ws_ml, T, H, parts, plan,       \
                                                                                     (bf16*)out, out_stride_t);            \
@@ -675,7 +782,7 @@ static void mla_launch(const void* q, int64_t q_stride_t, const void* cache, con
 }
 
 OME_API int ome_mla_attn(const void* q, int64_t q_stride_t, const void* cache, const int* block_tables,
-                         int bt_stride, const int* tok_row, const int* kv_lens, int T, int H, int dk, int dv,
+                         int bt_stride, int seqs, const int* tok_row, const int* kv_lens, int T, int H, int dk, int dv,
                          float scale, int parts, int rows, void* plan, void* out, int64_t out_stride_t, float* ws_o,
                          float* ws_ml, hipStream_t stream) {
   if (T <= 0) return 0;
@@ -686,10 +793,10 @@ OME_API int ome_mla_attn(const void* q, int64_t q_stride_t, const void* cache, c
   const float scale_log2 = scale * 1.4426950408889634f;
   if (dk == 576 && dv == 512)
     mla_launch<576, 512>(q, q_stride_t, cache, block_tables, bt_stride, tok_row, kv_lens, T, H, scale_log2, parts, out,
-                         out_stride_t, ws_o, ws_ml, stream, rows, (int2*)plan);
+                         out_stride_t, ws_o, ws_ml, stream, rows, seqs, (int2*)plan);
   else if (dk == 288 && dv == 256)
     mla_launch<288, 256>(q, q_stride_t, cache, block_tables, bt_stride, tok_row, kv_lens, T, H, scale_log2, parts, out,
-                         out_stride_t, ws_o, ws_ml, stream, rows, (int2*)plan);
+                         out_stride_t, ws_o, ws_ml, stream, rows, seqs, (int2*)plan);
   else
     return -3;
   OME_CHECK_LAUNCH();
@@ -703,7 +810,7 @@ OME_API int ome_mla_attn(const void* q, int64_t q_stride_t, const void* cache, c
 // kv_lens keys.  Zero columns add nothing to a score, and the output's zero columns are dropped by
 // the caller.
 OME_API int ome_latent_attn(const void* q, int64_t q_stride_t, const void* cache, const int* block_tables,
-                            int bt_stride, const int* tok_row, const int* kv_lens, int T, int H, int dk, int dv,
+                            int bt_stride, int seqs, const int* tok_row, const int* kv_lens, int T, int H, int dk, int dv,
                             float scale, int parts, int rows, void* plan, void* out, int64_t out_stride_t, float* ws_o,
                             float* ws_ml, const float* sinks, int window, hipStream_t stream) {
   if (T <= 0) return 0;
@@ -716,7 +823,7 @@ OME_API int ome_latent_attn(const void* q, int64_t q_stride_t, const void* cache
 #define LATENT_CASE(DK_, DV_)                                                                                       \
   if (dk == DK_ && dv == DV_) {                                                                                     \
     mla_launch<DK_, DV_>(q, q_stride_t, cache, block_tables, bt_stride, tok_row, kv_lens, T, H, scale_log2, parts,  \
-                         out, out_stride_t, ws_o, ws_ml, stream, rows, (int2*)plan, sinks, window);                                \
+                         out, out_stride_t, ws_o, ws_ml, stream, rows, seqs, (int2*)plan, sinks, window);                                \
     OME_CHECK_LAUNCH();                                                                                             \
     return 0;                                                                                                       \
   }

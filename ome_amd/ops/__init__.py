@@ -1089,8 +1089,8 @@ def mla_attn(q, cache, block_tables, tok_row, kv_lens, scale: float, ws: MLAWork
     if ws is None and (parts > 1 or decode):
         ws = MLAWorkspace(q.device)
     call("ome_mla_attn", q.data_ptr(), q.stride(0), cache.data_ptr(), _i32(block_tables).data_ptr(),
-         block_tables.stride(0), _i32(tok_row).data_ptr(), _i32(kv_lens).data_ptr(), T, H, DK, dv, float(scale),
-         parts, rows, ws.plan.data_ptr() if decode else None, out.data_ptr(), out.stride(0),
+         block_tables.stride(0), block_tables.shape[0], _i32(tok_row).data_ptr(), _i32(kv_lens).data_ptr(), T, H, DK, dv,
+         float(scale), parts, rows, ws.plan.data_ptr() if decode else None, out.data_ptr(), out.stride(0),
          ws.ws_o.data_ptr() if parts > 1 else None, ws.ws_ml.data_ptr() if parts > 1 else None, stream_ptr())
     return out
 
@@ -2075,8 +2075,8 @@ def latent_attn(q, cache, block_tables, tok_row, kv_lens, scale: float, dv: int,
     if ws is None and (parts > 1 or decode):
         ws = MLAWorkspace(q.device)
     call("ome_latent_attn", q.data_ptr(), q.stride(0), cache.data_ptr(), _i32(block_tables).data_ptr(),
-         block_tables.stride(0), _i32(tok_row).data_ptr(), _i32(kv_lens).data_ptr(), T, H, DK, dv, float(scale),
-         parts, rows, ws.plan.data_ptr() if decode else None, out.data_ptr(), out.stride(0),
+         block_tables.stride(0), block_tables.shape[0], _i32(tok_row).data_ptr(), _i32(kv_lens).data_ptr(), T, H, DK, dv,
+         float(scale), parts, rows, ws.plan.data_ptr() if decode else None, out.data_ptr(), out.stride(0),
          ws.ws_o.data_ptr() if parts > 1 else None, ws.ws_ml.data_ptr() if parts > 1 else None, _sinks(sinks),
          int(window), stream_ptr())
     return out

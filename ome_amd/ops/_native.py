@@ -68,7 +68,7 @@ _SIGNATURES = {
         "ome_conv_mix": [vp, i64, vp, vp, i64, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, vp],
         "ome_latent_prep": [vp, i64, i32, i32, i32, vp, f32, vp, vp, vp, vp, vp, i32, i32, i32, vp, i64, i64, i32, i32,
                             vp, i64, i64, i32, i32, vp],
-        "ome_latent_attn": [vp, i64, vp, vp, i32, vp, vp, i32, i32, i32, i32, f32, i32, i32, vp, vp, i64, vp, vp, vp, i32, vp],
+        "ome_latent_attn": [vp, i64, vp, vp, i32, i32, vp, vp, i32, i32, i32, i32, f32, i32, i32, vp, vp, i64, vp, vp, vp, i32, vp],
         "ome_hgrn2_scan": [vp, vp, vp, i64, vp, vp, vp, vp, vp, vp, i32, vp, vp, vp, i32, i32, i32, i32, f32, i32, vp],
         "ome_act": [vp, i64, i32, vp],
         "ome_act_any": [vp, i64, i32, i32, vp],
@@ -106,7 +106,7 @@ _SIGNATURES = {
         "ome_apply_penalties": [vp, i32, i64, i32, i32, vp, i64, vp, vp, vp, vp, vp],
         "ome_update_counts": [vp, i64, vp, vp, vp, vp, vp, i32, vp],
         "ome_moe_route": [vp, i32, i64, i32, i32, i32, i32, i32, vp, i32, i32, i32, vp, vp, vp, vp],
-        "ome_mla_attn": [vp, i64, vp, vp, i32, vp, vp, i32, i32, i32, i32, f32, i32, i32, vp, vp, i64, vp, vp, vp],
+        "ome_mla_attn": [vp, i64, vp, vp, i32, i32, vp, vp, i32, i32, i32, i32, f32, i32, i32, vp, vp, i64, vp, vp, vp],
         "ome_moe_align": [vp, i32, i32, vp, vp, vp, vp],
         "ome_moe_gemm": [vp, i64, vp, i32, vp, vp, i32, i32, i32, i32, vp, i64, vp, i32, vp],
         "ome_moe_gemm_pp": [vp, i64, i32, vp, i32, vp, vp, i32, i32, i32, i32, vp, i64, vp, i32, vp],

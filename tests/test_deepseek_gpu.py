@@ -212,3 +212,40 @@ def test_mla_tile_rule_fits_workspace_and_chip():
                         wgs = -(-T * H // rows)
                         assert wgs * parts <= W.TARGET_WGS_ALL and wgs * rows * parts <= W.ROWS
                     assert W.tiles(T, H, 288, seqs, pages)[0] == 0
+
+
+@pytest.mark.parametrize("rows", [32, 64, 128])
+@pytest.mark.parametrize("H,parts", [(16, 1), (16, 3), (64, 1)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_mla_row_tiles_keep_a_broken_sequence_apart(monkeypatch, rows, H, parts, bad):
+    """Latents of one sequence that are not finite: the others, whose rows share tiles with it, stay what they were, bit
+    for bit."""
+    torch.manual_seed(rows + H)
+    new = [5, 1, 37, 3, 20]
+    cache, bt = _setup([40 + n for n in new])
+    row = torch.tensor([s for s, n in enumerate(new) for _ in range(n)], dtype=torch.int32, device=DEV)
+    kl = torch.tensor([40 + j + 1 for n in new for j in range(n)], dtype=torch.int32, device=DEV)
+    q = torch.randn(len(row), H, 576, device=DEV).to(torch.bfloat16)
+    monkeypatch.setattr(ops.MLAWorkspace, "tiles", lambda T, H, DK, *a: (rows, False, parts))
+    want = ops.mla_attn(q, cache, bt, row, kl, 0.06)
+    for s in (1, 3):
+        cache[bt[s].long()[:2], :, ::7] = bad
+    got = ops.mla_attn(q, cache, bt, row, kl, 0.06)
+    whole = (row != 1) & (row != 3)
+    assert torch.equal(got[whole], want[whole]) and not got[~whole].isfinite().all()
+
+
+@pytest.mark.parametrize("rows", [32, 64, 128])
+@pytest.mark.parametrize("H,parts", [(16, 1), (20, 2), (64, 1)])
+def test_mla_row_tiles_take_tokens_in_any_order(monkeypatch, rows, H, parts):
+    torch.manual_seed(rows + H)
+    new = [9, 2, 0, 30, 1, 6]
+    cache, bt = _setup([30 + n for n in new])
+    row = torch.tensor([s for s, n in enumerate(new) for _ in range(n)], dtype=torch.int32)
+    kl = torch.tensor([30 + j + 1 for n in new for j in range(n)], dtype=torch.int32)
+    at = torch.randperm(len(row))
+    row, kl = row[at], kl[at]
+    q = torch.randn(len(row), H, 576, device=DEV).to(torch.bfloat16)
+    monkeypatch.setattr(ops.MLAWorkspace, "tiles", lambda T, H, DK, *a: (rows, False, parts))
+    out = ops.mla_attn(q, cache, bt, row.to(DEV), kl.to(DEV), 0.06)
+    assert (out.cpu().double() - _exact(q, cache, bt, row, kl, 0.06)).abs().max() < 2.0 ** -8 * cache.float().abs().max().item()
