@@ -23,6 +23,11 @@
 //   selective scan, 128 heads of 64 x 128, 8 groups, 1033 / 926 / 1248 / 293 rows:  11 + 116 us (row by row: 1745)
 // Largest error of the state against 64 bits: 1.1e-7 (row by row: 2.0e-7) and 1.4e-7 (6.2e-7) of its norm.
 //
+// A chunk's products multiply the entries that causality zeroes as well, and 0 times an infinity or NaN is NaN, so a key,
+// gate or value that is not finite would reach the rows before it in its chunk.  It reaches S and stays there (each
+// U_i enters every channel of S, and no decay takes an infinity or NaN away), so S tells at the end of a sequence: a
+// wave whose S is not finite walks its columns again row by row.
+//
 // fp32 throughout: k and q enter the matrix cores as the bf16 values that they are (their norms, 1 / |k| and
 // 1 / (|q| sqrt(dk)), scale results), S and U as three bf16 parts that sum to the fp32 value exactly, at
 // 3/16 of the fp32 MFMA's time; T R and P U, where both operands are fp32, take the fp32 MFMA.  Decay
@@ -439,14 +444,68 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   // state: lane (col, g) holds column nc, key channels 32 s + 8 g .. + 7 in blocks 2 s, 2 s + 1
   float* st = a.state + (((int64_t)a.slot[s] * a.H + h) * a.dv + nc) * DK + 8 * g;
   f32x4 S[NB];
+  const auto start = [&] {
 #pragma unroll
-  for (int b = 0; b < NB; ++b)
-    S[b] = a.reset[s] != 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4*>(st + 32 * (b >> 1) + 4 * (b & 1));
+    for (int b = 0; b < NB; ++b)
+      S[b] = a.reset[s] != 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4*>(st + 32 * (b >> 1) + 4 * (b & 1));
+  };
+  start();
   const float Dh = DELTA ? 0.f : a.D[h];
   uint32_t oo[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) oo[e] = 2 * ((uint32_t)(16 * (e >> 2) + 4 * g + (e & 3)) * (uint32_t)a.out_stride + (uint32_t)nc);
   char* op = reinterpret_cast<char*>(a.out + (int64_t)r0 * a.out_stride + (int64_t)h * a.dv);
+
+  // the sequence row by row, as the row-by-row kernels do it (each lane its 8 key channels of every 32)
+  const auto walk = [&](int n) {
+    for (int i = 0; i < n; ++i) {
+      const int64_t row = r0 + i;
+      bf16x8 k8[NS], q8[NS];
+#pragma unroll
+      for (int t = 0; t < NS; ++t) {
+        k8[t] = ld8(a.k + row * a.stride + hk * DK + 32 * t + 8 * g);
+        q8[t] = ld8(a.q + row * a.stride + hk * DK + 32 * t + 8 * g);
+      }
+      const float x = (float)a.v[row * a.v_stride + (int64_t)h * a.dv + nc], ga = (float)a.a[row * a.ab_stride + h] + a.dt_bias[h];
+      float decay, ik = 1.f, iq = 1.f, kq = 0.f, add;
+      if constexpr (DELTA) {
+        float nk = 0.f, nq = 0.f;
+#pragma unroll
+        for (int t = 0; t < NS; ++t)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            nk += (float)k8[t][j] * (float)k8[t][j];
+            nq += (float)q8[t][j] * (float)q8[t][j];
+            kq += (float)k8[t][j] * (float)q8[t][j];
+          }
+        ik = rsqrtf(group4_sum(nk) + 1e-6f);
+        iq = rsqrtf(group4_sum(nq) + 1e-6f) * rsqrtf((float)DK);
+        kq = group4_sum(kq) * ik * iq;
+        decay = __expf(-__expf(a.A[h]) * softplus_rule(ga));
+        float sk = 0.f;
+#pragma unroll
+        for (int t = 0; t < NS; ++t)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) sk += S[2 * t + j / 4][j % 4] * ((float)k8[t][j] * ik);
+        add = (x - decay * group4_sum(sk)) / (1.f + __expf(-(float)a.b[row * a.ab_stride + h]));
+      } else {
+        const float dt = fmaxf(softplus_rule(ga), a.dt_min);
+        decay = __expf(dt * a.A[h]);
+        add = dt * x;
+      }
+      float sq = 0.f;
+#pragma unroll
+      for (int t = 0; t < NS; ++t)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float s0 = S[2 * t + j / 4][j % 4], s1 = s0 * decay + (float)k8[t][j] * ik * add;
+          sq += DELTA ? s0 * ((float)q8[t][j] * iq) : s1 * (float)q8[t][j];
+          S[2 * t + j / 4][j % 4] = s1;
+        }
+      sq = group4_sum(sq);
+      if (live && g == 0) a.out[row * a.out_stride + (int64_t)h * a.dv + nc] = (bf16)(DELTA ? decay * sq + add * kq : sq + Dh * x);
+    }
+  };
 
   offsets(RC);
   fetch(0);
@@ -557,6 +616,15 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   for (int c = 0; c < chunks; c += 2) {
     step(c, 0);
     if (c + 1 < chunks) step(c + 1, 1);
+  }
+  float broken = 0.f;   // NaN if a value of S is not finite
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) broken += S[nb][e] * 0.f;
+  if (live && __ballot(broken != 0.f)) {
+    start();
+    walk(r1 - r0);
   }
   if (live) {
 #pragma unroll

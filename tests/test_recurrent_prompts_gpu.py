@@ -152,3 +152,51 @@ def test_selective_scan_prompts(lens, H, P, N, G, off):
     args = (c[:, :H * P], dt, c[:, H * P:H * P + G * N], c[:, H * P + G * N:], A, D, dtb, 0.001)
     want = exact_ssm(*args, st, *sq, H, P, N, G)
     assert near(ops.ssm_scan(*args, st, *sq, H, P, N, G), st, *want)
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
+@pytest.mark.parametrize("what", ["q", "k", "v", "a", "b"])
+def test_delta_rule_stays_causal(what, bad):
+    """A value that is not finite reaches its own row and the rows after it, of its heads: nothing earlier in its chunk."""
+    torch.manual_seed(5)
+    lens, Hk, Hv, dk, dv, at = [40, 90, 33], 2, 4, 64, 32, 40 + 43   # row 11 of the second sequence's second chunk
+    T, kd, sq = sum(lens), Hk * dk, (i32([0, 40, 130, 163]), i32([0, 1, 2]), i32([0, 1, 0]))
+    t = {n: torch.randn(T, w, device=DEV).to(BF) for n, w in (("c", 2 * kd + Hv * dv), ("ab", 2 * Hv))}
+    t.update(q=t["c"][:, :kd], k=t["c"][:, kd:2 * kd], v=t["c"][:, 2 * kd:], a=t["ab"][:, :Hv], b=t["ab"][:, Hv:])
+    A_log, dtb, st = torch.linspace(-3, 1, Hv, device=DEV), torch.zeros(Hv, device=DEV), torch.randn(3, Hv, dv, dk, device=DEV)
+    run = lambda s: ops.gdn_scan(t["q"], t["k"], t["v"], t["a"], t["b"], A_log, dtb, s, *sq, Hv, Hk).float().view(T, Hv, dv)  # noqa: E731
+    s0, s1 = st.clone(), st.clone()
+    clean = run(s0)
+    t[what][at, 1] = bad   # the first key head (value heads 0, 1), head 0's column 1, head 1's gates
+    heads = {"q": [0, 1], "k": [0, 1], "v": [0], "a": [1], "b": [1]}[what]
+    got = run(s1)
+    hit = torch.zeros_like(clean, dtype=torch.bool)
+    hit[at:130, heads] = True
+    # another path's sums for the rows of its chunk: one bf16 step of the largest value
+    assert (got - clean)[~hit].abs().max() <= 2.0 ** -8 * clean.abs().max()
+    assert torch.equal(s0[[0, 2]], s1[[0, 2]])
+    want_out = torch.empty(T, Hv * dv, dtype=torch.float32)
+    want_st = st.cpu()
+    ref.gdn_scan(*cpu(t["q"], t["k"], t["v"], t["a"], t["b"], A_log, dtb), want_st, *cpu(*sq), Hv, Hk, want_out)
+    assert torch.equal(s1.cpu().isfinite(), want_st.isfinite())
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
+@pytest.mark.parametrize("what", ["x", "dt", "B", "C"])
+def test_selective_scan_stays_causal(what, bad):
+    torch.manual_seed(6)
+    lens, H, P, N, G, at = [40, 90, 33], 4, 32, 64, 2, 40 + 43
+    T, sq = sum(lens), (i32([0, 40, 130, 163]), i32([0, 1, 2]), i32([0, 1, 0]))
+    t = {n: torch.randn(T, w, device=DEV).to(BF) for n, w in (("x", H * P), ("dt", H), ("bc", 2 * G * N))}
+    t.update(B=t["bc"][:, :G * N], C=t["bc"][:, G * N:])
+    A, D, dtb = -torch.logspace(-1, 1, H, device=DEV), torch.randn(H, device=DEV), torch.linspace(-4, 0, H, device=DEV)
+    st = torch.randn(3, H, P, N, device=DEV)
+    run = lambda s: ops.ssm_scan(t["x"], t["dt"], t["B"], t["C"], A, D, dtb, 0.001, s, *sq, H, P, N, G).float().view(T, H, P)  # noqa: E731
+    s0, s1 = st.clone(), st.clone()
+    clean = run(s0)
+    t[what][at, 1] = bad
+    got = run(s1)
+    hit = torch.zeros_like(clean, dtype=torch.bool)
+    hit[at:130, {"x": [0], "dt": [1], "B": [0, 1], "C": [0, 1]}[what]] = True
+    assert (got - clean)[~hit].abs().max() <= 2.0 ** -8 * clean.abs().max()
+    assert torch.equal(s0[[0, 2]], s1[[0, 2]])
