@@ -203,18 +203,18 @@ __global__ __launch_bounds__(256) void mla_attn_kernel(
   }
 }
 
-// One wave's share of a latent page's move to LDS: 64 lanes x 16 bytes from `off` (per lane) of the page at `base`
+// One wave's share of a latent page's move to LDS: 64 lanes x 16 bytes from `off` (per lane) + `add` of the page at `base`
 // to LDS address `lds` + 16 lane.  By asm, because the compiler takes every later LDS read of the image's array for a reader of
 // the move and waits for all of it (vmcnt 0) there; the kernels below wait themselves, once, before the barrier
 // after which a tile is read.  (No register is written; the descriptor's size bounds the reads to the page.)
-__device__ __forceinline__ void page_to_lds(const bf16* base, uint32_t bytes, uint32_t off, uint32_t lds) {
+__device__ __forceinline__ void page_to_lds(const bf16* base, uint32_t bytes, uint32_t off, uint32_t add, uint32_t lds) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   const uint64_t b = (uint64_t)base;
   const u32x4 rs = {(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, bytes, 0x00020000u};
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                :
-               : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(off), "s"(rs)
+               : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(off), "s"(rs), "s"(add)
                : "m0", "memory");
 #endif
 }
@@ -237,13 +237,16 @@ __device__ __forceinline__ void page_to_lds(const bf16* base, uint32_t bytes, ui
 // Nothing else runs on the SIMD meanwhile, so the loop is pipelined by hand: S^T of tile n + 1 is multiplied while
 // the softmax of tile n runs on the vector ALU, and the LDS DMA of tile n + 2 is in flight (three images).
 // O^T is rescaled only where a row's maximum rose by more than 2^8 since its last rescale (weights stay below
-// 2^8), almost never after a row's first tile.  The denominator sums the weights as rounded to bf16.
+// 2^8), almost never after a row's first tile.  A row's largest weight is then not exactly 1, as in the 16-head
+// kernel, so its rounding to bf16 counts: the keys with a weight that stands out are multiplied a second time with what
+// rounding took (16 keys of all rows at once; w^2 over 16, or of decode steps 6, times the mean of the squares of the
+// largest weight of each tile so far, or any that may come to a row's largest where there are fewer tiles than that).
+// The denominator sums the weights as they are used.  Error against 64 bits over the shapes of DeepSeek's heads
+// 0.0017..0.0018 of the result (16-head kernel 0.0017..0.0019; without the second product 0.0019..0.0021, 127 instead
+// of 146 us below).
 //
 // Measured (16-head kernel, or for decode the 16-row waves before -> now): three prompts of 3394 rows x 16 heads
-// 738 -> 128 us (118 -> 680 TFLOP/s), one of 5500 rows 4830 -> 545 us (965; a large bf16 product reaches 1530 on this
-// card); decode, 48 contexts of ~3000 keys x 128 heads 100 -> 79 us, x 16 heads 104 -> 65 us.  Error against 64 bits
-// 0.0018 -> 0.0020 of the result: bf16 weights and outputs as before, but a row's largest weight is no longer
-// exactly 1.
+// 738 -> 146 us (118 -> 598 TFLOP/s); decode, 48 contexts of ~3000 keys x 128 heads 100 -> 86 us.
 // ------------------------------------------------------------------------------------------
 // The products by asm: with one wave per SIMD, what covers an LDS read is the distance to its product, and the
 // compiler sinks reads to their use (or hoists them all, into scratch).  Volatile with a memory clobber, each stays
@@ -444,14 +447,22 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
     // Key tile -> LDS image: instruction i writes chunks [64 i, 64 i + 64) lane-linearly, each lane fetching the source
     // chunk that the row's XOR swizzle puts there.  A page is 16 rows x 72 chunks = 18 instructions, so each
     // instruction reads one page: its descriptor is based at that page.
+    // Nine instructions are 8 rows, after which the pattern repeats.
+    static_assert(9 * 64 == 8 * CH && NI == 36, "9 offsets a lane");
+    uint32_t dofs[9];
+#pragma unroll
+    for (int j = 0; j < 9; ++j) {
+      const int c = 64 * ((wave + NW * j) % (NI / 2)) + lane, kr = c / CH;
+      dofs[j] = (kr * CH + ((c - kr * CH) ^ (kr & 7))) * 16;
+    }
     auto dma = [&](const int* bt, int n_pages, int tile, int img) {
       const int p0 = 2 * tile, p1 = p0 + 1;
       const bf16* b0 = cache + (int64_t)bt[p0 < n_pages ? p0 : 0] * 16 * DK;
       const bf16* b1 = cache + (int64_t)bt[p1 < n_pages ? p1 : 0] * 16 * DK;
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
-        const int i = wave + NW * j, c = 64 * i + lane, kr = c / CH, xl = c - kr * CH;
-        page_to_lds(i < NI / 2 ? b0 : b1, 16 * DK * 2, (uint32_t)(((kr & 15) * CH + (xl ^ (kr & 7))) * 16),
+        const int i = wave + NW * j;
+        page_to_lds(j < NJ / 2 || (NW == 4 && i < NI / 2) ? b0 : b1, 16 * DK * 2, dofs[j % 9], NW == 1 && j / 9 % 2 ? 8 * CH * 16 : 0,
                     lds0 + img * IMG + 64 * 16 * i);
       }
     };
@@ -492,6 +503,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
     const bool mine = hv && my_row == bt_row;
     const int L = mine ? my_len : 0;
     float m = OME_NEG_INF, lsum = 0.f;
+    // the squares of the largest weight of each tile, summed: what a weight's error is measured against
+    float peaks = 0.f, walked = 0.f;
+    const float large = min((end - begin) * my_parts, DECODE ? 6 : 16);
     f32x16 sc;
     if (begin < end) {
       dma(bt, n_pages, begin, 0);
@@ -513,24 +527,31 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
       if (n + 2 < end) dma(bt, n_pages, n + 2, nxt == 2 ? 0 : nxt + 1);
       const f32x16 sn = score(nxt * IMG);   // (after the last tile: of whatever is there, unused)
       const int key = n * KT + 4 * hf;
-      float mx = OME_NEG_INF;
+      float ma = OME_NEG_INF, mb = OME_NEG_INF;   // of the lane's keys of the first and second 16
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         sc[i] = key + 8 * (i >> 2) + (i & 3) < L ? sc[i] * scale_log2 : OME_NEG_INF;
-        mx = fmaxf(mx, sc[i]);
+        if (i < 8) ma = fmaxf(ma, sc[i]);
+        else mb = fmaxf(mb, sc[i]);
       }
+      float mx = fmaxf(ma, mb);
       {
         auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
         mx = vmax_f32(__uint_as_float(w[0]), __uint_as_float(w[1]));
       }
       const bool rise = mx > m + LAZY;   // (also a row's first tile: m = -inf)
       const float mn = rise ? mx : m, ms = mn == OME_NEG_INF ? 0.f : mn;
-      float ps = 0.f;
+      // keys of this half or that among which a row has a weight that stands out: used in two parts
+      const float wa = __builtin_amdgcn_exp2f(ma - ms), wb = __builtin_amdgcn_exp2f(mb - ms), wt = __builtin_amdgcn_exp2f(mx - ms);
+      const float far = large * peaks;
+      const uint64_t two[2] = {__ballot(!rise && wa * wa * walked > far), __ballot(!rise && wb * wb * walked > far)};
+      float ps = 0.f;   // of the weights as they are used: their rounding cancels in the quotient
       bf16x8 pb[2];
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        pb[i >> 3][i & 7] = (bf16)__builtin_amdgcn_exp2f(sc[i] - ms);
-        ps += (float)pb[i >> 3][i & 7];   // the weights as they are used: their rounding cancels in the quotient
+        sc[i] = __builtin_amdgcn_exp2f(sc[i] - ms);
+        pb[i >> 3][i & 7] = (bf16)sc[i];
+        ps += (float)pb[i >> 3][i & 7];
       }
       {
         auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(ps), __float_as_uint(ps), false, false);
@@ -542,6 +563,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
       if (__ballot(rise && m != OME_NEG_INF)) {   // (a first tile has nothing to rescale: O^T and the sum are zero)
         const float alpha = rise && m != OME_NEG_INF ? __builtin_amdgcn_exp2f(m - mn) : 1.f;
         lsum *= alpha;
+        peaks *= alpha * alpha;
         // in the accumulation registers, by asm: as plain C++ all 256 products are computed every time and moved
         // through the other registers.  (waits: the last MFMA's results; the next one's operands)
         asm volatile(MMA_WAIT ::: "memory");
@@ -561,6 +583,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
         asm volatile("s_nop 7" ::: "memory");
       }
       lsum += ps;
+      peaks += wt * wt;
+      walked += 1.f;
       m = mn;
       asm volatile("s_nop 3" : "+v"(pb[0]), "+v"(pb[1])::"memory");   // (written by the vector ALU just now)
 #pragma unroll
@@ -568,6 +592,27 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
         mma_acc(o[k >> 1], vf[k % AHEAD], pb[k & 1]);
         if (k + AHEAD < 2 * NV) vf[k % AHEAD] = vfrag(cur * IMG, (k + AHEAD) >> 1, k & 1);
       }
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        if (two[j]) {   // what rounding took from the weights of these 16 keys
+#pragma unroll
+          for (int v = 0; v < AHEAD; ++v) vf[v] = vfrag(cur * IMG, v, j);
+          bf16x8 pr;
+          float rs = 0.f;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            pr[i] = (bf16)(sc[8 * j + i] - (float)pb[j][i]);
+            rs += (float)pr[i];
+          }
+          auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(rs), __float_as_uint(rs), false, false);
+          lsum += __uint_as_float(w[0]) + __uint_as_float(w[1]);
+          asm volatile("s_nop 3" : "+v"(pr)::"memory");
+#pragma unroll
+          for (int v = 0; v < NV; ++v) {
+            mma_acc(o[v], vf[v % AHEAD], pr);
+            if (v + AHEAD < NV) vf[v % AHEAD] = vfrag(cur * IMG, v + AHEAD, j);
+          }
+        }
       sc = sn;
       cur = nxt;
       asm volatile(MMA_WAIT "\n\ts_waitcnt vmcnt(0)" ::: "memory");   // tile n + 2 has landed
