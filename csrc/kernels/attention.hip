@@ -873,8 +873,9 @@ __global__ __launch_bounds__(512) void paged_prefill_kernel(
 // ------------------------------------------------------------------------------------------
 constexpr int PF_KLD = 128 + 8, PF_VLD = 32 + 8;
 
-// SPLIT: the item's key range is cut into chunks of `chunk` keys run by separate workgroups
-// (items4 = {seq, row0, chunk start, part}; part < 0 = the only chunk, written as final output).
+// SPLIT 1: the item's key range is cut into chunks of `chunk` keys run by separate workgroups
+// (items4 = {seq, row0, chunk start, part}; part < 0 = the only chunk, written as final output; `listed` > 0: that many
+// pieces, each up to the item's next one).  SPLIT 2: a workgroup walks a run of such pieces.
 // A short prefill (a few hundred keys per row) otherwise leaves most CUs idle and every
 // workgroup latency-bound on its serial chain of K/V tile loads; partial (O, m, l) per part go
 // to fp32 workspaces and prefill_combine_kernel merges them.
@@ -892,7 +893,7 @@ constexpr int PF_KLD = 128 + 8, PF_VLD = 32 + 8;
 // 2 = no K/V global loads, 3 = identity pages (no block-table loads before the K/V loads).
 // BS (FAST only): block-sparse layer -- skip the key stages no head of the kv group sees and mask
 // this head's invisible keys (a separate instantiation: the dense kernels keep their registers).
-template <int SUB, int F, bool SPLIT, bool FAST = false, int NW = 4, int PROBE = 0, bool BS = false>
+template <int SUB, int F, int SPLIT, bool FAST = false, int NW = 4, int PROBE = 0, bool BS = false>
 __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_prefill_v2_kernel(
     const bf16* __restrict__ q, int64_t q_stride, const typename KVStore<F>::T* __restrict__ k_cache,
     const typename KVStore<F>::T* __restrict__ v_cache, const int* __restrict__ block_tables, int bt_stride,
@@ -910,14 +911,14 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_prefill_v2_kernel(
   const int kvh = blockIdx.x % Hkv;
   int e0 = blockIdx.x / Hkv, e1 = e0 + 1;
   const int4* list = reinterpret_cast<const int4*>(items);
-  if (SPLIT && listed > 0) {   // a block's run of pieces, behind the pieces
+  if constexpr (SPLIT == 2) {   // a block's run of pieces, behind the pieces
     const int4 run = list[listed + e0];
     e0 = run.x, e1 = run.y;
   }
   for (int entry = e0; entry < e1; ++entry) {
-  if (SPLIT && entry > e0) __syncthreads();   // the piece before is done with the LDS images
+  if (SPLIT == 2 && entry > e0) __syncthreads();   // the piece before is done with the LDS images
   int s, r0_item, c_lo = 0, c_hi = 0x7fffffff, part = -1;
-  if constexpr (SPLIT) {
+  if constexpr (SPLIT > 0) {
     const int4 it4 = list[entry];
     s = it4.x, r0_item = it4.y, c_lo = it4.z, part = it4.w;
     if (listed > 0) {   // up to the item's next piece
@@ -938,7 +939,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_prefill_v2_kernel(
   const int prefix = kv_len - q_len;
   const int G = Hq / Hkv;
   static_assert(NW == 4 || NW == 8, "NW");
-  static_assert(!SPLIT || NW == 4, "split partials are laid out for 4 waves");
+  static_assert(SPLIT == 0 || NW == 4, "split partials are laid out for 4 waves");
   constexpr int PT = 2 * 4 / NW;   // K (and V) chunks of 8 elements per thread per 32-key subtile
   const int rows_per_item = 32 * (NW / G);
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -950,7 +951,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_prefill_v2_kernel(
   int kv_end = row_hi ? kv_len : min(kv_len, prefix + item_hi);
   int kv_lo = 0;
   kv_lo = attn_lo(prefix + r0_item, window) & ~31;
-  if constexpr (SPLIT) {   // chunk starts are multiples of 64 keys: kv_lo stays 32-aligned
+  if constexpr (SPLIT > 0) {   // chunk starts are multiples of 64 keys: kv_lo stays 32-aligned
     kv_lo = max(kv_lo, c_lo);
     kv_end = min(kv_end, c_hi);
   }
@@ -1279,7 +1280,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_prefill_v2_kernel(
       l_i[rb] = group4_sum(l_i[rb]);
     }
   }
-  if (SPLIT && part >= 0) {   // unnormalised partial: O^T rows of this wave + (m, l) per row
+  if (SPLIT > 0 && part >= 0) {   // unnormalised partial: O^T rows of this wave + (m, l) per row
     const int64_t pw = ((int64_t)part * Hkv + kvh) * 4 + wave;
     float* po = part_o + pw * 32 * D;
 #pragma unroll
@@ -1373,7 +1374,7 @@ static void launch_prefill(int variant, int rows, int G, dim3 grid, hipStream_t 
   if constexpr (D == 128) {
     if (variant == 2 && G == 4) {  // one head per wave over 32-row items (GQA-4: Llama-3, Qwen3, Mixtral)
 #define OME_PF2B(FAST, NW, BS)                                                                                    \
-  paged_prefill_v2_kernel<2, F, false, FAST, NW, 0, BS><<<grid.x * grid.y, 64 * NW, 0, stream>>>(                            \
+  paged_prefill_v2_kernel<2, F, 0, FAST, NW, 0, BS><<<grid.x * grid.y, 64 * NW, 0, stream>>>(                            \
       (const bf16*)q, q_stride, (const T*)k_cache, (const T*)v_cache, block_tables, bt_stride, cu_q, kv_lens,      \
       (const int2*)items, (bf16*)out, out_stride, Hq, Hkv, scl, window, v_scale, sinks, row_hi, 0, 0, nullptr, nullptr)
 #define OME_PF2(FAST, NW) OME_PF2B(FAST, NW, false)
@@ -1389,7 +1390,7 @@ static void launch_prefill(int variant, int rows, int G, dim3 grid, hipStream_t 
         static const int probe = getenv("OME_PREFILL_PROBE") ? atoi(getenv("OME_PREFILL_PROBE")) : 0;
         if (!bs && prefill_fast(scl, window, row_hi)) {
 #define OME_PF2P(PR)                                                                                              \
-  paged_prefill_v2_kernel<2, F, false, true, 4, PR><<<grid.x * grid.y, 256, 0, stream>>>(                                    \
+  paged_prefill_v2_kernel<2, F, 0, true, 4, PR><<<grid.x * grid.y, 256, 0, stream>>>(                                    \
       (const bf16*)q, q_stride, (const T*)k_cache, (const T*)v_cache, block_tables, bt_stride, cu_q, kv_lens,      \
       (const int2*)items, (bf16*)out, out_stride, Hq, Hkv, scl, window, v_scale, sinks, row_hi, 0, 0, nullptr, nullptr)
           bool done = false;
@@ -1476,31 +1477,31 @@ OME_API int ome_paged_prefill_split(const void* q, int64_t q_stride, const void*
   if (Hq != 4 * Hkv || chunk % 64 || kv_fmt < 0 || kv_fmt > 2 || n_blocks < 0 || (n_blocks == 0 && chunk <= 0)) return -2;
   if (window > 0 && keep_first > 0) return -6;   // kept first keys: ome_paged_prefill only
   const Scaler scl = make_scaler(scale * k_scale, softcap, alibi, bsparse);
-  const int grid = (n_blocks > 0 ? n_blocks : n_items) * Hkv, listed = n_blocks > 0 ? n_items : 0;
-#define OME_PFS(F, FAST)                                                                                       \
-  if (FAST && scl.bs_shift >= 6)                                                                               \
-    paged_prefill_v2_kernel<2, F, true, FAST, 4, 0, FAST><<<grid, 256, 0, stream>>>(                           \
-        (const bf16*)q, q_stride, (const typename KVStore<F>::T*)k_cache,                                      \
-        (const typename KVStore<F>::T*)v_cache, block_tables, bt_stride, cu_q, kv_lens, (const int2*)items4,   \
-        (bf16*)out, out_stride, Hq, Hkv, scl, window, v_scale, sinks, nullptr, chunk, listed, (float*)part_o,  \
-        (float*)part_ml);                                                                                      \
-  else                                                                                                         \
-  paged_prefill_v2_kernel<2, F, true, FAST><<<grid, 256, 0, stream>>>(                                         \
-      (const bf16*)q, q_stride, (const typename KVStore<F>::T*)k_cache, (const typename KVStore<F>::T*)v_cache, \
-      block_tables, bt_stride, cu_q, kv_lens, (const int2*)items4, (bf16*)out, out_stride, Hq, Hkv, scl, window,  \
-      v_scale, sinks, nullptr, chunk, listed, (float*)part_o, (float*)part_ml)
   // block-sparse with blocks < 64 keys: generic body (mask only)
   const bool fast = prefill_fast(scl, window, nullptr) && (scl.bs_shift == 0 || scl.bs_shift >= 6);
+  // the generic body has no registers for a run's loop (424 bytes of scratch, 182 -> 329 us at 512 rows over 8192 keys
+  // in a window of 4096): a workgroup a piece
+  const bool runs = n_blocks > 0 && fast;
+  const int grid = (runs ? n_blocks : n_items) * Hkv, listed = n_blocks > 0 ? n_items : 0;
+#define OME_PFS(F, SPLIT, FAST, BS)                                                                               \
+  paged_prefill_v2_kernel<2, F, SPLIT, FAST, 4, 0, BS><<<grid, 256, 0, stream>>>(                                 \
+      (const bf16*)q, q_stride, (const typename KVStore<F>::T*)k_cache, (const typename KVStore<F>::T*)v_cache,    \
+      block_tables, bt_stride, cu_q, kv_lens, (const int2*)items4, (bf16*)out, out_stride, Hq, Hkv, scl, window,   \
+      v_scale, sinks, nullptr, chunk, listed, (float*)part_o, (float*)part_ml)
+#define OME_PFS_F(F)                                                                                              \
+  if (!fast) OME_PFS(F, 1, false, false);                                                                         \
+  else if (scl.bs_shift >= 6 && runs) OME_PFS(F, 2, true, true);                                                  \
+  else if (scl.bs_shift >= 6) OME_PFS(F, 1, true, true);                                                          \
+  else if (runs) OME_PFS(F, 2, true, false);                                                                      \
+  else OME_PFS(F, 1, true, false)
   if (kv_fmt == KV_BF16) {
-    if (fast) OME_PFS(KV_BF16, true);
-    else OME_PFS(KV_BF16, false);
+    OME_PFS_F(KV_BF16);
   } else if (kv_fmt == KV_E4M3) {
-    if (fast) OME_PFS(KV_E4M3, true);
-    else OME_PFS(KV_E4M3, false);
+    OME_PFS_F(KV_E4M3);
   } else {
-    if (fast) OME_PFS(KV_E5M2, true);
-    else OME_PFS(KV_E5M2, false);
+    OME_PFS_F(KV_E5M2);
   }
+#undef OME_PFS_F
 #undef OME_PFS
   OME_CHECK_LAUNCH();
   if (n_comb > 0) {

@@ -312,6 +312,12 @@ class LlamaForCausalLM:
         return n
 
     # ------------------------------------------------------------------ forward
+    @property
+    def plain_attention(self) -> bool:
+        """Every layer's prompts run the plain causal kernel (no window, no soft-capping, no attention of a subclass)."""
+        return (self.window in (-1, 0) and not self.softcap and type(self).attention is LlamaForCausalLM.attention
+                and not any(hasattr(self, a) for a in ("windows", "swa_window", "prefill_item_rows")))
+
     def attention(self, q: torch.Tensor, k_cache, v_cache, meta: AttnMeta, ks: float = 1.0,
                   vs: float = 1.0) -> torch.Tensor:
         """``ks`` / ``vs``: the layer's fp8 KV dequantisation scales (1 for a bf16 cache)."""

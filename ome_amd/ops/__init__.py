@@ -1690,12 +1690,13 @@ class PrefillPlan:
     [nc, 4] (seq, row0, first part, parts) are the split-KV form (empty when nothing splits).
     ``chunk`` > 0: one workgroup per row of ``split`` and kv head, ``chunk`` keys each.  ``chunk`` =
     -n: n workgroups a kv head; the last n rows of ``split`` are their runs (first, past the last)
-    of pieces, a piece reaches to its item's next one (:func:`_prefill_runs`)."""
+    of pieces, a piece reaches to its item's next one (:func:`_prefill_runs`).  ``other``: beside such runs, the plan
+    (``prefill_plan(runs=False)``) of the layers that are not :func:`_plain_prefill`."""
 
-    __slots__ = ("items", "split", "comb", "chunk", "parts", "rows")
+    __slots__ = ("items", "split", "comb", "chunk", "parts", "rows", "other")
 
-    def __init__(self, items, split, comb, chunk: int, parts: int, rows: int = 32):
-        self.items, self.split, self.comb, self.chunk, self.parts = items, split, comb, chunk, parts
+    def __init__(self, items, split, comb, chunk: int, parts: int, rows: int = 32, other: PrefillPlan | None = None):
+        self.items, self.split, self.comb, self.chunk, self.parts, self.other = items, split, comb, chunk, parts, other
         self.rows = rows   # query rows per classic item (64: the 8-wave GQA-4 kernel)
 
     @property
@@ -1770,8 +1771,18 @@ def _prefill_runs(items: list, ends: list[int], kv_heads: int):
     return pieces + runs, comb, -len(runs), parts
 
 
+def _plain_prefill(window: int, softcap: float, alibi, blocksparse) -> bool:
+    """The layers that runs of equal stages are for: causal or block-sparse with blocks of whole stages, the kernel's
+    fast body (the general one has no registers for a run's loop, and of a window's range most stages are empty).
+    32 / 8 heads, equal chunks or one workgroup an item -> the run's pieces, a workgroup each: window 8192, 512 rows over 8192
+    182 -> 490 us (items alone; the pieces are for few items: 64 over 15936 85 -> 78, 256 over 4096 86 -> 95).
+    Block-sparse (64 x 16 local, every 8th), equal chunks or items -> runs: 64 over 15936 76 -> 69, 512 over 8192 131 -> 99,
+    1500 over 7600 144 -> 144."""
+    return window in (-1, 0) and softcap <= 0 and alibi is None and (blocksparse is None or blocksparse[0] >= 64)
+
+
 def prefill_plan(q_lens: list[int], kv_lens: list[int], tile: int = 32, target: int | None = None,
-                 kv_heads: int = 8, force: bool = False):
+                 kv_heads: int = 8, force: bool = False, runs: bool = True):
     """(classic items, split items, combine items, chunk, parts) for the split-KV prefill kernel.
 
     A short prefill leaves most CUs idle and each workgroup latency-bound on its serial chain of
@@ -1783,7 +1794,8 @@ def prefill_plan(q_lens: list[int], kv_lens: list[int], tile: int = 32, target: 
     smaller than the chip (items x kv heads < 256 workgroups) AND some item has a long key range
     (> ``PREFILL_SPLIT_MIN_KEYS`` keys), e.g. 256 new rows over a 4096-token prefix 243 -> 68 us; at ~900 rows over
     <= 480 keys the classic grid is already full and splitting costs the partial round trip.  Long
-    ranges whose classic grid leaves places of the chip empty: :func:`_prefill_runs`."""
+    ranges whose classic grid leaves places of the chip empty: :func:`_prefill_runs` (``runs`` False: not
+    those, for layers that are not :func:`_plain_prefill`)."""
     target = target or PREFILL_SPLIT_TARGET
     items = prefill_work_items(q_lens, kv_lens, tile)
     # the split decision and the split items use 32-row items (the split kernel's partial layout)
@@ -1794,10 +1806,10 @@ def prefill_plan(q_lens: list[int], kv_lens: list[int], tile: int = 32, target: 
         e = (kv_lens[s] - q_lens[s]) + min(r + 32, q_lens[s])
         ends.append(e)
         work += e
-    if not force and max(ends, default=0) > PREFILL_SPLIT_MIN_KEYS:
-        runs = _prefill_runs(items32, ends, kv_heads)
-        if runs is not None:
-            return items, *runs
+    if runs and not force and max(ends, default=0) > PREFILL_SPLIT_MIN_KEYS:
+        equal = _prefill_runs(items32, ends, kv_heads)
+        if equal is not None:
+            return items, *equal
     if not force and (len(items32) * kv_heads >= 256 or max(ends, default=0) <= PREFILL_SPLIT_MIN_KEYS):
         return items, [], [], 0, 0
     chunk = max(128, -(-(-(-work // max(1, target))) // 64) * 64)
@@ -1845,12 +1857,19 @@ def paged_prefill(q, k_cache, v_cache, block_tables, cu_q, kv_lens, items, scale
     rows = 32
     if isinstance(items, PrefillPlan):
         plan, items = items, items.items
+        whole = PrefillPlan(items, None, None, 0, 0, plan.rows)
+        if plan.chunk < 0 and not _plain_prefill(window, softcap, alibi, blocksparse):
+            # (a plan without the other form: its items, or its pieces where the items are too few to fill the chip)
+            plan = plan.other or (plan if items.shape[0] * Hkv < 128 else whole)
+        if 0 < window <= (512 if items.shape[0] * Hkv < 128 else 1024):
+            # narrow windows, whole items -> cut: 300 keys, 64 rows over 15936 48 -> 83 us, 512 over 8192 49 -> 94; 1024,
+            # 64 rows 83 -> 82, 16 over 8000 82 -> 59, 512 over 8192 84 -> 108; 4096, 64 rows 246 -> 78, 512 248 -> 169
+            plan = whole
         rows = plan.rows
         if rows != 32 and not (rows == 64 and D == 128 and P == 16 and Hq == 4 * Hkv):
             raise ValueError(f"paged_prefill: {rows}-row items need the GQA-4 / D=128 kernel, got Hq={Hq} "
                              f"Hkv={Hkv} D={D} page={P} (build the plan with prefill_rows of this layer)")
         if (plan.parts and D == 128 and P == 16 and Hq == 4 * Hkv and row_hi is None and keep_first <= 0 and
-                (plan.chunk > 0 or (window <= 0 and blocksparse is None)) and
                 os.environ.get("OME_PREFILL_ATTN", "2") == "2"):
             nb = max(0, -plan.chunk)
             po = torch.empty(plan.parts * Hkv * 4 * 32 * 128, dtype=torch.float32, device=q.device)

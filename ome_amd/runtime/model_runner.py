@@ -772,8 +772,11 @@ class ModelRunner:
             rows = self.model.prefill_item_rows(P)
         items, split, comb, chunk, parts = ops.prefill_plan(q_lens, kv_lens, tile=rows, kv_heads=tp_.hkv) if q_lens \
             else ([], [], [], 0, 0)
+        # equal runs are for plain causal layers; the others' plan rides along where there are any
+        _, split2, comb2, chunk2, parts2 = ops.prefill_plan(q_lens, kv_lens, tile=rows, kv_heads=tp_.hkv, runs=False) \
+            if chunk < 0 and not getattr(self.model, "plain_attention", False) else ([], [], [], 0, 0)
         T, S, n_it, nd, B = len(ids), len(q_lens), len(items), len(dec_lens), len(chunks)
-        n_sp, n_cb = len(split), len(comb)
+        n_sp, n_cb, n_s2, n_c2 = len(split), len(comb), len(split2), len(comb2)
         cu = np.zeros(S + 1, dtype=np.int32)
         cu[1:] = np.cumsum(q_lens)
         dec_order = np.argsort(-np.asarray(dec_lens, np.int64), kind="stable").astype(np.int32) if nd else \
@@ -796,7 +799,9 @@ class ModelRunner:
                                  np.asarray(dec_lens, np.int32), np.asarray(dec_req, np.int32), dec_order,
                                  np.asarray(items, np.int32).reshape(-1) if n_it else np.zeros(0, np.int32),
                                  np.asarray(split, np.int32).reshape(-1) if n_sp else np.zeros(0, np.int32),
-                                 np.asarray(comb, np.int32).reshape(-1) if n_cb else np.zeros(0, np.int32)])
+                                 np.asarray(comb, np.int32).reshape(-1) if n_cb else np.zeros(0, np.int32),
+                                 np.asarray(split2, np.int32).reshape(-1) if n_s2 else np.zeros(0, np.int32),
+                                 np.asarray(comb2, np.int32).reshape(-1) if n_c2 else np.zeros(0, np.int32)])
         self._probe_mark(mode)
         dev = self.staging.to_device(packed)
         o = 0
@@ -816,8 +821,10 @@ class ModelRunner:
         t_dlen, t_dreq, t_dord = take(nd), take(nd), take(nd)
         t_items = take(2 * n_it).view(n_it, 2)
         if n_sp:   # split-KV prefill attention (ops.prefill_plan)
-            t_items = ops.PrefillPlan(t_items, take(4 * n_sp).view(n_sp, 4), take(4 * n_cb).view(n_cb, 4), chunk,
-                                      parts, rows)
+            t_items = ops.PrefillPlan(t_items, take(4 * n_sp).view(n_sp, 4), take(4 * n_cb).view(n_cb, 4), chunk, parts, rows)
+            if chunk < 0:
+                t_items.other = ops.PrefillPlan(t_items.items, take(4 * n_s2).view(n_s2, 4), take(4 * n_c2).view(n_c2, 4),
+                                                chunk2, parts2, rows)
         elif rows != 32 and n_it:   # 64-row classic items (the 8-wave kernel)
             t_items = ops.PrefillPlan(t_items, t_items[:0], t_items[:0], 0, 0, rows)
         if any_pending:

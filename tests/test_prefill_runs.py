@@ -72,3 +72,72 @@ def test_runs_match_reference(q_lens, kv_lens, Hq, Hkv, cache, mode):
                              kw.get("sinks"))
     # probabilities and output rounded to bf16 once each: 2^-9 of the largest |v| (about 2.3) apiece
     assert (out.float() - want.float()).abs().max().item() < 2 * 2.0 ** -9 * 2.5
+
+
+@pytest.mark.parametrize("q,kv", [([64], [15936]), ([256], [4096]), ([33, 64], [9000, 3000]), ([512], [8192]), ([1500], [7600])])
+def test_plan_of_other_layers_is_in_equal_chunks(q, kv):
+    """Layers with a window, soft-capping or ALiBi: chunks where the items are too few, none where they fill the chip."""
+    assert ops.prefill_plan(q, kv)[3] < 0
+    items, split, comb, chunk, parts = ops.prefill_plan(q, kv, runs=False)
+    if len(items) * 8 >= 256:
+        assert chunk == parts == 0 and not split
+    else:
+        assert chunk >= 128 and chunk % 64 == 0 and len(split) >= 32 and parts > 0
+
+
+@pytest.mark.parametrize("model,change,other", [("tiny-llama", {}, False), ("tiny-llama", {"sliding_window": 512}, True),
+                                                ("tiny-gemma2", {}, True)])
+def test_runner_sends_the_other_plan(monkeypatch, model, change, other):
+    """... along with the runs, for a model that has such layers."""
+    import dataclasses
+
+    from ome_amd.models.config import preset
+    from ome_amd.runtime.model_runner import ModelRunner
+    from ome_amd.runtime.request import Request, SamplingParams
+    from ome_amd.runtime.scheduler import ScheduledChunk, StepBatch
+
+    cfg = dataclasses.replace(preset(model), max_position_embeddings=4096, **change)
+    runner = ModelRunner(cfg, device="cpu", dtype=torch.float32, max_running=2, max_context=4096, max_total_tokens=8192, cuda_graph=False)
+    seen = []
+    forward = runner.model.forward
+    monkeypatch.setattr(runner.model, "forward", lambda ids, meta, *a: (seen.append(meta.items), forward(ids, meta, *a))[1])
+    r = Request([3] * 3064, SamplingParams(ignore_eos=True))
+    r.pages, r.req_slot, r.num_cached = list(range(1, 193)), runner.slots.alloc(), 3000
+    runner.slots.set_pages(r.req_slot, 0, r.pages)
+    runner.slots.flush()
+    runner.launch(StepBatch("prefill", [ScheduledChunk(r, 3000, 64, True)]))
+    plan = seen[0]
+    assert plan.chunk < 0 and len(plan.split) + plan.chunk > 2
+    assert (plan.other.chunk >= 128 and len(plan.other.split) == plan.other.parts > 2) if other else not plan.other.parts
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kw,other,chunked", [(dict(window=900), True, True), (dict(softcap=20.0), True, True), (dict(window=-1024), True, True),
+                                              ({}, True, False), (dict(window=900), False, False), (dict(window=300), True, None)], ids=str)
+def test_other_layers_run_their_plan(monkeypatch, kw, other, chunked):
+    """A window over a long range with few rows is split into chunks, as is all that the kernel's fast body does not
+    take; the runs serve a caller that has no other plan."""
+    torch.manual_seed(3)
+    Hq, Hkv, D, P, n, q_len, dev = 8, 2, 128, 16, 3000, 40, "cuda"
+    t = lambda a, c: torch.tensor(a, dtype=torch.int32, device=dev).view(-1, c)  # noqa: E731
+    pages = -(-n // P)
+    kc, vc = torch.randn(pages + 1, Hkv, P, D, device=dev).bfloat16(), torch.randn(pages + 1, Hkv, D, P, device=dev).bfloat16()
+    bt = (torch.randperm(pages, device=dev) + 1).int().view(1, -1)
+    cu, kl = torch.tensor([0, q_len], dtype=torch.int32, device=dev), torch.tensor([n], dtype=torch.int32, device=dev)
+    q = torch.randn(q_len, Hq, D, device=dev).bfloat16()
+    items, split, comb, chunk, parts = ops.prefill_plan([q_len], [n], kv_heads=Hkv)
+    _, split2, comb2, chunk2, parts2 = ops.prefill_plan([q_len], [n], kv_heads=Hkv, runs=False)
+    plan = ops.PrefillPlan(t(items, 2), t(split, 4), t(comb, 4), chunk, parts,
+                           other=ops.PrefillPlan(t(items, 2), t(split2, 4), t(comb2, 4), chunk2, parts2) if other else None)
+    calls = []
+    call = ops.call
+    monkeypatch.setattr(ops, "call", lambda name, *a: (calls.append((name, a)), call(name, *a))[1])
+    out = ops.paged_prefill(q, kc, vc, bt, cu, kl, plan, 0.0884, **kw)
+    (name, a), = [c for c in calls if c[0].startswith("ome_paged_prefill")]
+    if chunked is None:   # a narrow window: its items as they are
+        assert name == "ome_paged_prefill"
+    else:
+        assert name == "ome_paged_prefill_split" and (a[10] == 0) == chunked and (a[13] == (chunk2 if chunked else 0))
+    want = ref.paged_prefill(q, kc, vc, bt, cu, kl, 0.0884, kw.get("window", -1), 1.0, 1.0, kw.get("softcap", 0.0), None)
+    # probabilities and output rounded to bf16 once each: 2^-9 of the largest |v| (about 4.5) apiece
+    assert (out.float() - want.float()).abs().max().item() < 2 * 2.0 ** -9 * 5
