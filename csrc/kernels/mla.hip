@@ -6,8 +6,10 @@
 // 288 = 256 + 32 for MiniCPM3 (template instances below).  With W_UK folded into the query
 // (q_lat = [q_nope . W_UK | q_pe], 576 wide) and W_UV applied after the attention, MLA is
 // multi-QUERY attention over that latent: scores use all 576 dims, values are the first 512.
-// The same kernel serves decode, prefill and chunked prefill: a work item is one query token
-// x 16 heads (every head of a token shares the causal limit) x one split-K partition.
+// Three kernels serve decode, prefill and chunked prefill: row tiles (mla_attn_rows_kernel, DK = 576: prompts, and
+// decode steps of some 24 rows or 6 with many heads), 128 heads a workgroup (mla_attn_all_kernel: many decode rows of
+// so many heads), and here 16 heads a workgroup (few rows, other widths, sinks, windows): a work item is one query
+// token x 16 heads (every head of a token shares the causal limit) x one split-K partition.
 //
 // Workgroup = 4 waves: all four compute S^T for the same 16 heads x 32 keys (the K tile is
 // staged once in LDS and read by all), and each wave owns 128 of the 512 value dims.
@@ -396,6 +398,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
       if (pieces(mid) <= UNITS) hi = mid;
       else lo = mid + 1;
     }
+    // pieces that save fewer key tiles than their partials' way to memory and back costs: none (64 heads, 128 rows of ~100
+    // keys 34 -> 28 us)
+    if (most - lo <= 2 + R / 2048) lo = most;
     const int w = blockIdx.x, c0 = count(lo, 0), c1 = count(lo, 1), c2 = count(lo, 2), c3 = count(lo, 3);
     int incl = c0 + c1 + c2 + c3;
 #pragma unroll
@@ -742,6 +747,162 @@ __global__ __launch_bounds__(256) void mla_reduce_rows_kernel(const float* __res
       bf16x4{(bf16)(acc[0] * inv), (bf16)(acc[1] * inv), (bf16)(acc[2] * inv), (bf16)(acc[3] * inv)};
 }
 
+// ------------------------------------------------------------------------------------------
+// Many decode rows of 128 heads: one workgroup of 8 waves owns a token's heads and one partition of its keys.  A wave owns
+// 16 heads and all DV value dims, so two waves share a SIMD: less matrix work an LDS read than the row tiles above,
+// but a piece's start, drain and tile reads overlap with another wave's work, which counts where contexts are short and
+// pieces many.  Row tiles -> these: 64 / 128 / 256 rows of ~400 keys 50 -> 44, 64 -> 56, 73 -> 69 us; 48 rows of ~3000
+// 86 -> 94.
+// Key tiles arrive by LDS DMA into a double-buffered image: the DMA of tile n + 1 is issued before tile n is
+// computed and retired (vmcnt(0) + barrier) after it.
+// ------------------------------------------------------------------------------------------
+typedef __attribute__((address_space(3))) void mla_lds_t;
+
+template <int DK, int DV, int NW>
+__global__ __launch_bounds__(64 * NW, 1) void mla_attn_all_kernel(
+    const bf16* __restrict__ q, int64_t q_stride_t, const bf16* __restrict__ cache,
+    const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ tok_row,
+    const int* __restrict__ kv_lens, int H, float scale_log2, int parts, bf16* __restrict__ out,
+    int64_t out_stride_t, float* __restrict__ ws_o, float* __restrict__ ws_ml) {
+  static_assert(DK == 576 && lds_chunks<DK>() == DK / 8, "LDS DMA image assumes unpadded 72-chunk rows");
+  constexpr int CH = DK / 8, NI = KT * CH / 64, NB = DV / 16;
+  constexpr int IMG = KT * CH * 8;   // bf16 elements per K-tile image
+  __shared__ __attribute__((aligned(16))) bf16 sK[2 * IMG];
+  const int t = blockIdx.x, part = blockIdx.z;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int col = lane & 15, g = lane >> 4;
+  const int head = blockIdx.y * 16 * NW + wave * 16 + col;   // this lane's head (S^T / O^T column)
+  const int L = kv_lens[t];
+  const int n_pages = (L + 15) >> 4;
+  const int pairs = (n_pages + 1) >> 1;
+  const int per_part = (pairs + parts - 1) / parts;
+  const int pair_begin = part * per_part, pair_end = min(pairs, pair_begin + per_part);
+  const int* bt = block_tables + (int64_t)tok_row[t] * bt_stride;
+
+  // K tile pair -> LDS image: instruction i writes chunks [64 i, 64 i + 64) lane-linearly, each
+  // lane fetching the source chunk the row's XOR swizzle puts there.  A page is 16 rows x 72 chunks
+  // = 18 instructions, so each instruction reads one page: its descriptor is based at that page.
+  auto dma_pair = [&](int pr, bf16* img) {
+#pragma unroll
+    for (int j = 0; j < (NI + NW - 1) / NW; ++j) {
+      const int i = wave + NW * j;
+      if (i >= NI) break;
+      const int c = 64 * i + lane, row = c / CH, xl = c - row * CH;
+      const int pg = 2 * pr + (i >= NI / 2);
+      const int page = bt[pg < n_pages ? pg : 0];
+      const auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)(cache + (int64_t)page * 16 * DK), (short)0,
+                                                        16 * DK * 2, 0x00020000);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (mla_lds_t*)(img + 64 * 8 * i), 16,
+                                               (uint32_t)(((row & 15) * CH + (xl ^ (row & 7))) * 16), 0, 0, 0);
+    }
+  };
+  if (pair_begin < pair_end) dma_pair(pair_begin, sK);
+
+  bf16x8 qf[DK / 32];
+  const bf16* qp = q + (int64_t)t * q_stride_t + (int64_t)head * DK + 8 * g;
+#pragma unroll
+  for (int s = 0; s < DK / 32; ++s) qf[s] = ld8(qp + 32 * s);
+
+  f32x4 o[NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = OME_NEG_INF, lsum = 0.f;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+
+  // The XOR swizzle makes every LDS offset lane-dependent; split it so the compiler sees a lane
+  // base plus an immediate: (8k + c) ^ z = 8k + (c ^ z) for c, z < 8.  S^T reads chunk 4 s + g of
+  // row col (2 bases by s parity); V^T reads chunk 2 nb + pcol/2 of row 4 g + qrow (4 bases by
+  // nb mod 4).  Rows 16..31 sit 16 * CH chunks further on with the same (row & 7).
+  const int qrow = (lane & 15) >> 2, pcol = lane & 3;
+  int sofs[2], vofs[4];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) sofs[e] = (col * CH + ((4 * e + g) ^ (col & 7))) * 16;
+  const int rv = 4 * g + qrow;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) vofs[e] = (rv * CH + ((2 * e + (pcol >> 1)) ^ (rv & 7))) * 16 + (pcol & 1) * 8;
+  int buf = 0;
+  for (int pr = pair_begin; pr < pair_end; ++pr) {
+    const bf16* img = sK + buf * IMG;
+    // the other image's last readers passed the barrier that ended the previous tile
+    if (pr + 1 < pair_end) dma_pair(pr + 1, sK + (buf ^ 1) * IMG);
+    // ---- S^T [32 keys x 16 heads] ----
+    const char* ib = reinterpret_cast<const char*>(img);
+    f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < DK / 32; ++s) {
+      const int off = sofs[s & 1] + (s >> 1) * 128;   // swz(col, 4 s + g): lane base + immediate
+      const bf16x8 a0 = *reinterpret_cast<const bf16x8*>(ib + off);
+      const bf16x8 a1 = *reinterpret_cast<const bf16x8*>(ib + off + 16 * CH * 16);
+      s0 = mfma16x32(a0, qf[s], s0);
+      s1 = mfma16x32(a1, qf[s], s1);
+    }
+    const int kbase = pr * KT;
+    float mx = OME_NEG_INF;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      s0[i] = (kbase + 4 * g + i < L) ? s0[i] * scale_log2 : OME_NEG_INF;
+      s1[i] = (kbase + 16 + 4 * g + i < L) ? s1[i] * scale_log2 : OME_NEG_INF;
+      mx = fmaxf(mx, fmaxf(s0[i], s1[i]));
+    }
+    mx = group4_max(mx);
+    const float m_new = fmaxf(m, mx);
+    const float alpha = (m_new == OME_NEG_INF) ? 1.f : __builtin_amdgcn_exp2f(m - m_new);
+    bf16x8 pb;
+    float ps = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float p0 = (m_new == OME_NEG_INF) ? 0.f : __builtin_amdgcn_exp2f(s0[i] - m_new);
+      const float p1 = (m_new == OME_NEG_INF) ? 0.f : __builtin_amdgcn_exp2f(s1[i] - m_new);
+      ps += p0 + p1;
+      pb[i] = (bf16)p0;
+      pb[4 + i] = (bf16)p1;
+    }
+    ps = group4_sum(ps);
+    lsum = lsum * alpha + ps;
+    m = m_new;
+    // ---- O^T [DV x 16 heads] += V^T . P^T (keys permuted as in pb: 4g + i, 16 + 4g + i) ----
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      const int off = vofs[nb & 3] + (nb >> 2) * 128;   // swz(4g + qrow, 2 nb + pcol/2) + 8 (pcol & 1)
+      const bf16x4 va = tr_read(img, off);
+      const bf16x4 vb = tr_read(img, off + 16 * CH * 16);
+      bf16x8 a;
+      a[0] = va[0]; a[1] = va[1]; a[2] = va[2]; a[3] = va[3];
+      a[4] = vb[0]; a[5] = vb[1]; a[6] = vb[2]; a[7] = vb[3];
+      o[nb] *= alpha;
+      o[nb] = mfma16x32(a, pb, o[nb]);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next tile's DMA has landed
+    __syncthreads();
+    buf ^= 1;
+  }
+
+  // ---- epilogue: O^T lane map dim = 16 nb + 4 g + i, head = col ----
+  const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+  if (parts == 1) {
+    bf16* op = out + (int64_t)t * out_stride_t + (int64_t)head * DV + 4 * g;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      bf16x4 v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = (bf16)(o[nb][i] * inv);
+      *reinterpret_cast<bf16x4*>(op + 16 * nb) = v;
+    }
+  } else {
+    const int64_t ws_row = ((int64_t)t * H + head) * parts + part;
+    float* wp = ws_o + ws_row * DV + 4 * g;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+      *reinterpret_cast<f32x4*>(wp + 16 * nb) = f32x4{o[nb][0] * inv, o[nb][1] * inv, o[nb][2] * inv,
+                                                       o[nb][3] * inv};
+    if (g == 0) {
+      ws_ml[2 * ws_row] = m;
+      ws_ml[2 * ws_row + 1] = lsum;
+    }
+  }
+}
+
 // merge split-K partitions: one workgroup per (token, head), DV / 4 threads x 4 dims.  Partitions
 // are consumed 8 at a time with all their loads issued up front (online max rescaling), so up to
 // 64 partitions cost ~8 memory latencies rather than one each.
@@ -789,15 +950,16 @@ __global__ __launch_bounds__(128) void mla_reduce_kernel(const float* __restrict
 
 // q [T, H, DK] (token stride q_stride_t), cache [pages, 16, DK], out [T, H, DV] with
 // (DK, DV) = (576, 512) or (288, 256).  tok_row[t] = block-table row of token t; kv_lens[t] =
-// keys visible to token t (causal).  parts > 1 needs ws_o [T*H*parts*DV] f32 and ws_ml
-// [T*H*parts*2] f32.
+// keys visible to token t (causal).  parts > 1 needs ws_o [R*DV] f32 and ws_ml [R*2] f32, R = T*H*parts; of row
+// tiles (`rows`) whole tiles: R = ceil(T*H / rows)*rows*parts for prompts, and for decode (`plan`, int2 [256], written
+// by the kernel) 256*rows, one tile a piece.
 template <int DK, int DV>
 static void mla_launch(const void* q, int64_t q_stride_t, const void* cache, const int* block_tables, int bt_stride,
                        const int* tok_row, const int* kv_lens, int T, int H, float scale_log2, int parts, void* out,
                        int64_t out_stride_t, float* ws_o, float* ws_ml, hipStream_t stream, int rows = 0, int seqs = 1,
                        int2* plan = nullptr, const float* sinks = nullptr, int window = -1) {
   // `rows`: query rows of a workgroup of the row-tile kernel (32 / 64 / 128, the caller's choice), 0: the
-  // 16-head kernel, which alone has the sink term and the window
+  // 16-head kernel, which alone has the sink term and the window, or many rows of 128 heads
   if constexpr (DK == 576) {
     if (rows > 0) {
       const unsigned units = (unsigned)(plan ? T * ((H + rows - 1) / rows) : ((int64_t)T * H + rows - 1) / rows);
@@ -819,9 +981,19 @@ static void mla_launch(const void* q, int64_t q_stride_t, const void* cache, con
       return;
     }
   }
-  mla_attn_kernel<DK, DV><<<dim3(T, (H + 15) / 16, parts), 256, 0, stream>>>(
-      (const bf16*)q, q_stride_t, (const bf16*)cache, block_tables, bt_stride, tok_row, kv_lens, H, scale_log2,
-      parts, (bf16*)out, out_stride_t, ws_o, ws_ml, sinks, window);
+  bool done = false;
+  if constexpr (DK == 576) {
+    if (H % 128 == 0 && T >= 64 && sinks == nullptr && window <= 0) {   // (MLAWorkspace.parts cuts for it)
+      mla_attn_all_kernel<DK, DV, 8><<<dim3(T, H / 128, parts), 512, 0, stream>>>(
+          (const bf16*)q, q_stride_t, (const bf16*)cache, block_tables, bt_stride, tok_row, kv_lens, H, scale_log2,
+          parts, (bf16*)out, out_stride_t, ws_o, ws_ml);
+      done = true;
+    }
+  }
+  if (!done)
+    mla_attn_kernel<DK, DV><<<dim3(T, (H + 15) / 16, parts), 256, 0, stream>>>(
+        (const bf16*)q, q_stride_t, (const bf16*)cache, block_tables, bt_stride, tok_row, kv_lens, H, scale_log2,
+        parts, (bf16*)out, out_stride_t, ws_o, ws_ml, sinks, window);
   if (parts > 1)
     mla_reduce_kernel<DV><<<dim3(T, H), DV / 4, 0, stream>>>(ws_o, ws_ml, H, parts, (bf16*)out, out_stride_t, sinks);
 }
@@ -850,9 +1022,9 @@ OME_API int ome_mla_attn(const void* q, int64_t q_stride_t, const void* cache, c
 
 // Latent attention over rows of any latent / rotary width, padded to the kernel's tiling: a cache
 // row is [latent (dv_pad wide: the values, zero beyond the latent) | rotary key (dk - dv_pad wide,
-// zero beyond it)], dv_pad a multiple of 64 up to 256 or 512, dk - dv_pad 32 or 64.  The 16-head kernel
-// serves every step kind; sinks optional; window > 0: a token sees only the last `window` of its
-// kv_lens keys.  Zero columns add nothing to a score, and the output's zero columns are dropped by
+// zero beyond it)], dv_pad a multiple of 64 up to 256 or 512, dk - dv_pad 32 or 64.  Kernels as for
+// ome_mla_attn; sinks optional, window > 0: a token sees only the last `window` of its kv_lens keys (both by the
+// 16-head kernel).  Zero columns add nothing to a score, and the output's zero columns are dropped by
 // the caller.
 OME_API int ome_latent_attn(const void* q, int64_t q_stride_t, const void* cache, const int* block_tables,
                             int bt_stride, int seqs, const int* tok_row, const int* kv_lens, int T, int H, int dk, int dv,

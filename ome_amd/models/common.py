@@ -35,6 +35,8 @@ class AttnMeta:
     order: torch.Tensor | None = None      # decode: sequences longest-first (workgroup dispatch order)
     num_prefill: int = 0                   # mixed: rows before this index are prefill rows
     dec_block_tables: torch.Tensor | None = None
+    max_kv: int | None = None              # longest ``kv_lens`` / ``seq_lens`` where the host knows them (a captured
+    max_dec: int | None = None             # decode graph does not)
     extra: dict = field(default_factory=dict)
 
     @property

@@ -297,20 +297,20 @@ class DeepseekForCausalLM(LlamaForCausalLM):
 
     # ------------------------------------------------------------------ forward
     def _token_rows(self, meta: AttnMeta, T: int):
-        """(tok_row, kv_lens) per query token, plus the block table they index."""
+        """Segments (first row, end row, block table, block-table row and visible keys per token, longest context or None)."""
         if self._arange is None or self._arange.numel() < T:
             self._arange = torch.arange(max(T, 4096), dtype=torch.int32, device=self.device)
         kv_lens = (meta.positions + 1).to(torch.int32)
         if meta.is_decode:
-            return [(0, T, meta.block_tables, self._arange[:T], meta.seq_lens)]
+            return [(0, T, meta.block_tables, self._arange[:T], meta.seq_lens, meta.max_dec)]
         n = meta.num_prefill if meta.mode == "mixed" else T
         seg = []
         if n:
             cu = meta.cu_q
             rows = torch.searchsorted(cu[1:].contiguous(), self._arange[:n].to(cu.dtype), right=True).to(torch.int32)
-            seg.append((0, n, meta.block_tables, rows, kv_lens[:n]))
+            seg.append((0, n, meta.block_tables, rows, kv_lens[:n], meta.max_kv))
         if n < T:
-            seg.append((n, T, meta.dec_block_tables, self._arange[: T - n], meta.seq_lens))
+            seg.append((n, T, meta.dec_block_tables, self._arange[: T - n], meta.seq_lens, meta.max_dec))
         return seg
 
     def attention_block(self, i: int, x: torch.Tensor, meta: AttnMeta, kv: PagedKVCache) -> torch.Tensor:
@@ -346,8 +346,8 @@ class DeepseekForCausalLM(LlamaForCausalLM):
             if ws is None:
                 ws = self._ws[sid] = ops.MLAWorkspace(x.device)
         cache3 = cache.view(cache.shape[0], -1, lat + self.rope)
-        for s, e, bt, rows, lens in self._token_rows(meta, T):
-            ops.mla_attn(q_full[s:e], cache3, bt, rows, lens, self.scale, ws, out=o_lat[s:e], dv=lat)
+        for s, e, bt, rows, lens, longest in self._token_rows(meta, T):
+            ops.mla_attn(q_full[s:e], cache3, bt, rows, lens, self.scale, ws, out=o_lat[s:e], dv=lat, max_len=longest)
         o = torch.empty(T, Hl * self.vd, dtype=x.dtype, device=x.device)
         torch.bmm(o_lat.transpose(0, 1), self.w_uv[i], out=o.view(T, Hl, self.vd).transpose(0, 1))   # token-major
         return pstate.tp_all_reduce(linear(o, self.w_o[i]))

@@ -586,9 +586,9 @@ class LatentAttention(_Block):
             o_lat = torch.empty(T, H, self.DV, dtype=h.dtype, device=h.device)
             rows3 = k_cache.view(k_cache.shape[0], k_cache.shape[2], D)
             ws = _latent_workspace(h)
-            for s, e, bt, rows, lens in latent_rows(ctx.meta, T):
+            for s, e, bt, rows, lens, longest in latent_rows(ctx.meta, T):
                 ops.latent_attn(q_full[s:e], rows3, bt, rows, lens, self.scale, self.DV, ws, out=o_lat[s:e],
-                                sinks=self.sink, window=self.window)
+                                sinks=self.sink, window=self.window, max_len=longest)
         else:
             G = self.HEAD_GROUP
             if H <= G:
@@ -611,24 +611,24 @@ _LATENT_WS: dict = {}
 
 def latent_rows(meta: AttnMeta, T: int) -> list:
     """The step's rows as the latent attention kernel takes them: segments (first row, end row,
-    block table, block-table row per token, visible keys per token) -- one for the prompt chunks,
-    one for the single decode rows of a mixed step."""
+    block table, block-table row per token, visible keys per token, longest context or None) -- one for
+    the prompt chunks, one for the single decode rows of a mixed step."""
     dev = meta.positions.device
     ar = _ARANGE.get(dev)
     if ar is None or ar.numel() < T:
         ar = _ARANGE[dev] = torch.arange(max(T, 4096), dtype=torch.int32, device=dev)
         _ARANGE_KEEP.append(ar)    # (captured decode graphs keep reading the one they were recorded with)
     if meta.is_decode:
-        return [(0, T, meta.block_tables, ar[:T], meta.seq_lens)]
+        return [(0, T, meta.block_tables, ar[:T], meta.seq_lens, meta.max_dec)]
     kv_lens = (meta.positions + 1).to(torch.int32)
     n = meta.num_prefill if meta.mode == "mixed" else T
     seg = []
     if n:
         cu = meta.cu_q
         rows = torch.searchsorted(cu[1:].contiguous(), ar[:n].to(cu.dtype), right=True).to(torch.int32)
-        seg.append((0, n, meta.block_tables, rows, kv_lens[:n]))
+        seg.append((0, n, meta.block_tables, rows, kv_lens[:n], meta.max_kv))
     if n < T:
-        seg.append((n, T, meta.dec_block_tables, ar[:T - n], meta.seq_lens))
+        seg.append((n, T, meta.dec_block_tables, ar[:T - n], meta.seq_lens, meta.max_dec))
     return seg
 
 
@@ -795,7 +795,7 @@ def attention_rows(meta: AttnMeta, T: int) -> list:
     """The step's rows for kernels that take one (block-table row, position) per query row:
     segments (first row, end row, block table, block-table row per token, position per token) --
     one for the prompt chunks, one for the single decode rows of a mixed step."""
-    return [(s, e, bt, rows, lens - 1) for s, e, bt, rows, lens in latent_rows(meta, T)]
+    return [(s, e, bt, rows, lens - 1) for s, e, bt, rows, lens, _ in latent_rows(meta, T)]
 
 
 def mask_window(size: int | None, chunked: bool) -> int:

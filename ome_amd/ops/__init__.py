@@ -996,10 +996,11 @@ class MLAWorkspace:
     """Split-K partials for :func:`mla_attn` (``ws_o`` [rows, 512] f32, ``ws_ml`` [rows, 2]; rows =
     tokens x heads x partitions, bounded by ``ROWS``).
 
-    Two kernels (``mla.hip``): row tiles (:meth:`rows`: one workgroup, one to a CU, streams the latent KV once
-    for 32 / 64 / 128 query rows) and the 16-head kernel (other widths, sinks, windows).  Row tiles of prompts are
-    cut into equal partitions up to ~1 workgroup per CU; those of decode steps by the kernel itself, by their
-    lengths, into at most 256 pieces (``plan``: each tile's first partial and piece count).  The 16-head
+    Kernels (``mla.hip``): row tiles (:meth:`tiles`: one workgroup, one to a CU, streams the latent KV once
+    for 32 / 64 / 128 query rows), 128 heads a workgroup for many decode rows, and the 16-head kernel (few rows, other
+    widths, sinks, windows).  Row tiles of prompts are cut into equal partitions up to ~1 workgroup per CU; those of decode
+    steps by the kernel itself, by their lengths, into at most 256 pieces (``plan``: each tile's first partial and
+    piece count; 256 x 128 rows are ``ROWS``).  The 16-head
     kernel takes partitions up to ~1024 workgroups.  None beyond what the f32 partials' HBM round trip repays."""
 
     TARGET_WGS = 1024
@@ -1020,34 +1021,42 @@ class MLAWorkspace:
 
     @classmethod
     @functools.lru_cache(maxsize=4096)
-    def tiles(cls, T: int, H: int, DK: int = 576, seqs: int = 1 << 30, pages: int = 1 << 30) -> tuple[int, bool, int]:
-        """(query rows of a row tile or 0 for the 16-head kernel, whether its tiles are heads of one token, partitions)
-        for T tokens of ``seqs`` block-table rows of ``pages`` pages (a bound of every context).
+    def tiles(cls, T: int, H: int, DK: int = 576, seqs: int = 1 << 30, pages: int = 1 << 30,
+              longest: bool = False) -> tuple[int, bool, int]:
+        """(query rows of a row tile or 0 for the other kernels, whether its tiles are heads of one token, partitions)
+        for T tokens of ``seqs`` block-table rows of ``pages`` pages: a bound of every context, or (``longest``)
+        the longest one.  A table is as wide as the longest context that its engine takes, so what it bounds it
+        tells little about.
 
         Prompts (at least 4 tokens a sequence): rows of neighbouring tokens share a tile.  A workgroup has a CU to itself and
         a wave for every 32 rows, so 128-row tiles use all of the matrix cores, and 32-row ones a quarter, which start
-        sooner and need no partitions to cover the chip with few rows.  Estimated in us for the contexts expected: per
-        launch wave 12 / 14 / 20 to start and drain (32 / 64 / 128 rows) and 0.06 a key; partitions 5, and 0.5 per 1000
-        rows and partition for their fp32 partials.  Device times of 32 / 64 / 128 rows (16-head kernel): 64 heads,
-        4 x 49 of 73 keys 28.5 / 17.2 / 38.5 (33.7), 174 26.4 / 22.6 / 36.2 (40.5), 100 of 3100 238 / 114 / 70 (496);
-        16 heads, 4 x 100 18.9 / 27.2 / 30.8 (35.2), 4 x 200 37.7 / 24.9 / 39.6 (50.9), 20 21.9 / 26.9 / 30.7 (12.2).
+        sooner and need no partitions to cover the chip with few rows.  Estimated in us for the longest context: per
+        launch wave 9 / 12 / 15 to start and drain (32 / 64 / 128 rows) and 0.06 a key; partitions 6, and 0.67 per 1000
+        rows and partition for their fp32 partials.  Device times of 32 / 64 / 128 rows (before them): 64 heads,
+        4 x 49 of 73 keys 26 / 20 / 22 (20), 100 of 3100 202 / 122 / 79 (145); 16 heads, 4 x 100 18 / 20 / 25 (36),
+        4 x 200 36 / 28 / 31 (51), 20 10 / 13 / 16 (13), 20 of 3020 27 / 29 / 31 (50).  Fewer than 320 rows: 8 x 16 heads of
+        308 keys 15 / 16 / 18 (12).
 
-        Decode (16-head kernel / row tiles): 16 heads, 32 x 400 keys 19 / 21, 32 x 3000 53 / 46, 64 x 200 29 / 22; 32 heads,
-        8 x 100 11 / 15, 12 x 1000 27 / 24, 48 x 3000 196 / 69; 64 heads, 4 x 2000 22 / 27, 12 x 100 21 / 17; 128 heads,
-        4 x 64 16 / 17, 4 x 500 23 / 20, 8 x 100 23 / 17, 48 x 3000 104 (the tiles before) / 76."""
-        n = T * H
+        Decode, whose contexts a captured graph does not know (before the row tiles / them, at about 100, 400, 1000 and
+        3000 keys): 8 heads, 32 rows 12 19 35 74 / 15 18 24 40, 48 rows 14 24 40 92 / 16 20 29 54; 16 heads, 16 rows 11 14 22
+        42 / 15 17 21 32, 24 rows 14 20 36 72 / 16 19 25 41; 32 heads, 12 rows 14 21 32 62 / 16 18 23 30, 16 rows 15 23 37
+        72 / 16 19 24 32; 64 heads, 4 rows 12 14 16 23 / 16 16 18 25, 6 rows 15 22 33 65 / 16 18 23 31 of 32 rows, 12 rows 21 30
+        44 87 / 19 22 27 36 of 64 rows, 48 rows 22 31 45 95 / 25 29 39 68; 128 heads, 16 rows 29 33 38 52 / 22 27 35 54 of
+        64 rows, 32 rows 32 38 47 75 / 33 38 47 69 of 128 rows; from 64 rows on, ``mla_attn_all_kernel`` in ``mla.hip``."""
+        n, wide = T * H, T * -(-H // 16) * 16
         if DK == 576 and H >= 4 and _MLA_ROW_TILES:
             if T >= 4 * seqs:
-                if n >= (512 if pages <= 32 else 256):
-                    keys, best = min(16 * pages, max(1024, 2 * T // seqs)), None
-                    for rows, start in ((32, 12), (64, 14), (128, 20)):
-                        wgs = -(-n // rows)
-                        for p in {1, cls.parts(T, H, DK, rows)}:
-                            us = -(-wgs // cls.TARGET_WGS_ALL) * (start + 0.06 * keys / p) + (p > 1) * (5 + n * p / 2000)
+                if n >= 320:
+                    keys, best = 16 * pages if longest else min(16 * pages, max(1024, 2 * T // seqs)), None
+                    for rows, start in ((32, 9), (64, 12), (128, 15)):
+                        wgs = -(-n // rows) + seqs - 1   # (one more where a sequence begins inside a tile)
+                        most = min(cls.parts(T, H, DK, rows), max(1, cls.TARGET_WGS_ALL // wgs))
+                        for p in {1, max(1, most // 4), max(1, most // 2), most}:
+                            us = -(-wgs // cls.TARGET_WGS_ALL) * (start + 0.06 * keys / p) + (p > 1) * (6 + n * p / 1500)
                             best = min(best or (us, rows, p), (us, rows, p))
                     return best[1], False, best[2]
-            elif n >= 1024 or (n >= 384 and (pages > 64 if H < 32 else pages > 16 or (H > 32 and n >= 640))):
-                rows = 128 if H > 64 and T >= 16 else 64 if H > 32 and n >= 512 else 32
+            elif wide >= (768 if H <= 8 or pages <= 16 and H % 64 else 512 if 16 < H <= 32 else 384) and not (H % 128 == 0 and T >= 64):
+                rows = 32 if n < 704 or 0 < H % 64 <= 32 else 128 if H % 128 == 0 and T >= 24 else 64
                 return rows, True, cls.parts(T, H, DK, rows, True)
         return 0, False, cls.parts(T, H, DK)
 
@@ -1057,21 +1066,32 @@ class MLAWorkspace:
         prompts the most that fit the chip."""
         if rows and decode:
             units = T * -(-H // rows)
-            return 1 if units > cls.TARGET_WGS_ALL else min(cls.MAX_PARTS_ALL, -(-2 * cls.TARGET_WGS_ALL // units))
+            return 1 if units >= cls.TARGET_WGS_ALL else min(cls.MAX_PARTS_ALL, -(-2 * cls.TARGET_WGS_ALL // units))
         if rows:
             wgs = -(-T * H // rows)
             return max(1, min(cls.MAX_PARTS_ALL, cls.TARGET_WGS_ALL // wgs, cls.ROWS // (wgs * rows)))
-        wgs = T * -(-H // 16)
-        p = 1 if wgs >= cls.TARGET_WGS else max(1, min(cls.MAX_PARTS, cls.TARGET_WGS // max(wgs, 1)))
+        if DK == 576 and H % 128 == 0 and T >= 64:   # 128 heads a workgroup
+            p = max(1, min(cls.MAX_PARTS_ALL, cls.TARGET_WGS_ALL // (T * H // 128)))
+        else:
+            wgs = T * -(-H // 16)
+            p = 1 if wgs >= cls.TARGET_WGS else max(1, min(cls.MAX_PARTS, cls.TARGET_WGS // max(wgs, 1)))
         return max(1, min(p, cls.ROWS // max(T * H, 1)))
 
 
+def _latent_tiles(T: int, H: int, DK: int, table: torch.Tensor, max_len: int | None) -> tuple[int, bool, int]:
+    seqs, pages = table.shape
+    if max_len is None:
+        return MLAWorkspace.tiles(T, H, DK, seqs, pages)
+    return MLAWorkspace.tiles(T, H, DK, seqs, min(pages, -(-max_len // 16)), True)
+
+
 def mla_attn(q, cache, block_tables, tok_row, kv_lens, scale: float, ws: MLAWorkspace | None = None,
-             out: torch.Tensor | None = None, dv: int = 512) -> torch.Tensor:
+             out: torch.Tensor | None = None, dv: int = 512, max_len: int | None = None) -> torch.Tensor:
     """Absorbed multi-head latent attention (MLA) over the paged latent cache: q [T, H, DK]
     (latent-projected nope part | roped pe part), cache [pages, 16, DK] -> out [T, H, dv] (values
     = the first dv latent dims); (DK, dv) = (576, 512) DeepSeek / Kimi-K2 or (288, 256) MiniCPM3.
-    Token t sees keys [0, kv_lens[t]) of block-table row tok_row[t]."""
+    Token t sees keys [0, kv_lens[t]) of block-table row tok_row[t].  ``max_len``: the largest of kv_lens where the
+    caller knows it (it chooses the tiles; a wide table says little about the contexts)."""
     if not _gpu(q):
         r = ref.mla_attn(q, cache, block_tables, tok_row, kv_lens, scale, dv)
         if out is not None:
@@ -1083,7 +1103,7 @@ def mla_attn(q, cache, block_tables, tok_row, kv_lens, scale: float, ws: MLAWork
     assert q.stride(2) == 1 and q.stride(1) == DK and cache.shape[-1] == DK
     if out is None:
         out = torch.empty(T, H, dv, dtype=q.dtype, device=q.device)
-    rows, decode, parts = MLAWorkspace.tiles(T, H, DK, *block_tables.shape)
+    rows, decode, parts = _latent_tiles(T, H, DK, block_tables, max_len)
     if rows and (out.data_ptr() % 16 or out.stride(0) % 8):
         rows, decode, parts = 0, False, MLAWorkspace.parts(T, H, DK)
     if ws is None and (parts > 1 or decode):
@@ -2066,13 +2086,14 @@ def latent_shape(lat: int, rope: int) -> tuple[int, int] | None:
 
 
 def latent_attn(q, cache, block_tables, tok_row, kv_lens, scale: float, dv: int, ws: MLAWorkspace | None = None,
-                out: torch.Tensor | None = None, sinks: torch.Tensor | None = None, window: int = -1) -> torch.Tensor:
+                out: torch.Tensor | None = None, sinks: torch.Tensor | None = None, window: int = -1,
+                max_len: int | None = None) -> torch.Tensor:
     """Absorbed latent attention over a paged cache of key rows that carry their own values: q [T,
     H, DK], cache [pages, 16, DK] -> out [T, H, dv] (values = the first ``dv`` columns of a row);
     (DK, dv) one of :data:`LATENT_SHAPES`.  Token t sees keys [0, kv_lens[t]) of block-table row
     tok_row[t] (prompt chunks, decode rows and mixed batches alike).  ``sinks``: fp32 [H] logits
     that join each head's softmax denominator (no key, no value, unscaled).  ``window`` > 0: only
-    the last ``window`` of those keys, [kv_lens[t] - window, kv_lens[t])."""
+    the last ``window`` of those keys, [kv_lens[t] - window, kv_lens[t]).  ``max_len``: as for :func:`mla_attn`."""
     if not _gpu(q):
         r = ref.mla_attn(q, cache, block_tables, tok_row, kv_lens, scale, dv, sinks, window)
         if out is not None:
@@ -2086,9 +2107,9 @@ def latent_attn(q, cache, block_tables, tok_row, kv_lens, scale: float, dv: int,
     if out is None:
         out = torch.empty(T, H, dv, dtype=q.dtype, device=q.device)
     assert out.stride(2) == 1 and out.stride(1) == dv
-    rows, decode, parts = MLAWorkspace.tiles(T, H, DK, *block_tables.shape)
-    if rows and (sinks is not None or window > 0 or out.data_ptr() % 16 or out.stride(0) % 8):
-        rows, decode, parts = 0, False, MLAWorkspace.parts(T, H, DK)
+    rows, decode, parts = _latent_tiles(T, H, DK, block_tables, max_len)
+    if sinks is not None or window > 0 or (rows and (out.data_ptr() % 16 or out.stride(0) % 8)):
+        rows, decode, parts = 0, False, MLAWorkspace.parts(T, H, DK if sinks is None and window <= 0 else 0)   # (0: the 16-head kernel)
     if window > 0:   # at least four 32-key tiles of the window per partition (fewer only move partials around)
         parts = max(1, min(parts, window // 128))
     if ws is None and (parts > 1 or decode):

@@ -836,13 +836,14 @@ class ModelRunner:
         if S and nd:
             meta = AttnMeta("mixed", t_pos, t_slots, self.slots.table.index_select(0, t_req), seq_lens=t_dlen,
                             cu_q=t_cu, kv_lens=t_kv, items=t_items, decode_ws=ws, order=t_dord,
-                            num_prefill=int(cu[-1]), dec_block_tables=self.slots.table.index_select(0, t_dreq))
+                            num_prefill=int(cu[-1]), dec_block_tables=self.slots.table.index_select(0, t_dreq),
+                            max_kv=max(kv_lens), max_dec=max(dec_lens))
         elif S:
             meta = AttnMeta("prefill", t_pos, t_slots, self.slots.table.index_select(0, t_req), cu_q=t_cu,
-                            kv_lens=t_kv, items=t_items)
+                            kv_lens=t_kv, items=t_items, max_kv=max(kv_lens))
         else:
             meta = AttnMeta("decode", t_pos, t_slots, self.slots.table.index_select(0, t_dreq), seq_lens=t_dlen,
-                            decode_ws=ws, order=t_dord)
+                            decode_ws=ws, order=t_dord, max_dec=max(dec_lens))
         self._init_penalty_rows(chunks)
         if self.stateful:  # sequences in row order: prefill chunks, then single-token rows
             lens = [chunks[i].length for i in pre + dec]

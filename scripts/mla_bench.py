@@ -37,9 +37,10 @@ def run(T, L, H=128, iters=50):
     us = e0.elapsed_time(e1) * 1e3 / iters
     kv = T * L * 576 * 2
     flops = 2 * T * H * L * (576 + 512)
-    return {"T": T, "L": L, "H": H, "parts": ops.MLAWorkspace.parts(T, H, 576, *ops.MLAWorkspace.rows(T, H)), "us": round(us, 1),
+    tile, _, parts = ops.MLAWorkspace.tiles(T, H, 576, *bt.shape)
+    return {"T": T, "L": L, "H": H, "parts": parts, "us": round(us, 1),
             "kv_GBps": round(kv / us / 1e3, 1), "TFLOPs": round(flops / us / 1e6, 1),
-            "kernel": "row tiles" if ops.MLAWorkspace.rows(T, H)[0] else "16-head"}
+            "kernel": f"{tile}-row tiles" if tile else "16 / 128 heads"}
 
 
 if __name__ == "__main__":
