@@ -32,7 +32,7 @@
 // 1 / (|q| sqrt(dk)), scale results), S and U as three bf16 parts that sum to the fp32 value exactly, at
 // 3/16 of the fp32 MFMA's time; T R and P U, where both operands are fp32, take the fp32 MFMA.  Decay
 // exponents are summed in fp64 (differences of a long sum).  The row-by-row kernels stay for decode steps
-// (one row per sequence), dk other than 64 / 128, and unaligned views.
+// (one row per sequence), few rows in all, dk other than 64 / 128, and unaligned views.
 #include "common.h"
 
 namespace {
@@ -68,9 +68,16 @@ struct RuleArgs {
   int S, H, Hk, dv;
 };
 
+// Sequences of at most FEW rows (the decode rows beside a prompt) are walked row by row instead: no chunk in the workspace,
+// no products 1/32 full.  The walk is bound by its vector instructions, near 1 us a row and four waves a CU.  Chunks -> walk, in us,
+// delta rule of 32 heads of 128 x 128 (selective scan of 128 of 64 x 128): 200 sequences of 1 row with a prompt of 40
+// 224 -> 193 (365 -> 327), of 2000 259 -> 224 (416 -> 346); 64 of 2 rows 81 -> 70 (131 -> 118), of 3 81 -> 81
+// (126 -> 130), of 4 81 -> 93 (127 -> 144); one of 3 rows 16 -> 11 (12 -> 10).
+constexpr int FEW = 3;
+
 // Chunk `id` of the launch -> (sequence, first row).  Sequence s owns ids cu[s] / 32 + s and up, one per
 // chunk: ceil(len / 32) <= (cu[s + 1] / 32 + s + 1) - (cu[s] / 32 + s), so ids never overlap and stay
-// below T / 32 + S.  Whole wave; false: an id that no chunk has.
+// below T / 32 + S.  Whole wave; false: an id that no chunk has, or of a sequence that is walked.
 __device__ __forceinline__ bool chunk_of(int id, const int* cu, int S, int& r0, int& n) {
   const int lane = threadIdx.x & 63;
   int s = -1;
@@ -83,7 +90,7 @@ __device__ __forceinline__ bool chunk_of(int id, const int* cu, int S, int& r0, 
   if (s < 0) return false;
   r0 = cu[s] + (id - cu[s] / RC - s) * RC;
   n = min(RC, cu[s + 1] - r0);
-  return n > 0;
+  return n > 0 && cu[s + 1] - cu[s] > FEW;
 }
 
 __device__ __forceinline__ f32x4 mma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
@@ -507,13 +514,16 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
     }
   };
 
-  offsets(RC);
-  fetch(0);
-  put(0);
+  const bool few = r1 - r0 <= FEW;                      // whole block
   bf16 vc[8];
+  if (!few) {
+    offsets(RC);
+    fetch(0);
+    put(0);
 #pragma unroll
-  for (int e = 0; e < 8; ++e) vc[e] = rv[e];
-  __syncthreads();
+    for (int e = 0; e < 8; ++e) vc[e] = rv[e];
+    __syncthreads();
+  }
   const auto step = [&](int c, int b) {
     if (c + 1 < chunks) fetch(c + 1);
     const bf16 *K = sK[b], *Q = sQ[b];
@@ -613,7 +623,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
     }
     __syncthreads();
   };
-  for (int c = 0; c < chunks; c += 2) {
+  for (int c = 0; !few && c < chunks; c += 2) {
     step(c, 0);
     if (c + 1 < chunks) step(c + 1, 1);
   }
@@ -622,8 +632,8 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
     for (int e = 0; e < 4; ++e) broken += S[nb][e] * 0.f;
-  if (live && __ballot(broken != 0.f)) {
-    start();
+  if (live && (few || __ballot(broken != 0.f))) {
+    if (!few) start();
     walk(r1 - r0);
   }
   if (live) {

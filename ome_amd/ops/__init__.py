@@ -170,10 +170,16 @@ def _chunk_rule_floats(H: int, G: int, delta: bool) -> int:
 
 def _chunk_rule_ws(T: int, S: int, H: int, G: int, dk: int, dv: int, delta: bool, state: torch.Tensor, rows: tuple) -> torch.Tensor | None:
     """Workspace of the chunked kernels (``chunk_rule.hip``) for T rows of S sequences and H heads, or None
-    where the row-by-row kernels run: one row per sequence (a decode step; a chunk would be 1/32 full), key
+    where the row-by-row kernels run: one row per sequence (a decode step; a chunk would be 1/32 full), few rows in all, key
     widths other than 64 / 128, value widths not of 16 columns, or key / query rows (the first two
-    of ``rows``, the operands and the output) that 16-byte loads cannot take."""
-    if T <= S or dk not in (64, 128) or dv % 16 or S > 65535 or H > 65535:
+    of ``rows``, the operands and the output) that 16-byte loads cannot take.
+
+    Few rows: the two launches of the chunks and their serial chain take 16 us (delta rule, 32 heads of 128 x 128) and 12
+    (selective scan, 128 of 64 x 128) for one sequence of up to 32 rows.  Row by row, 2 / 8 / 20 / 40 rows 8 / 11 / 15 / 24
+    (chunks 20), 8 sequences of 2 / 4 / 8 14 / 16 / 20 (chunks 22; 16 of 2 walked in the chunked kernel); the scan's 2 / 4 / 6
+    rows 9 / 10.5 / 12.  Of more rows the host does not know how they lie: 64 x 2..8 delta rule 55..84 (chunks
+    70..82), 64 x 1 and a prompt of 32 76 (66), 200 x 1 and one of 300 522 (197)."""
+    if T <= max(S, 32 if delta else 4) or dk not in (64, 128) or dv % 16 or S > 65535 or H > 65535:
         return None
     q, k, o = rows[0], rows[1], rows[-1]   # (a shared row stride for q, k and v / B and C)
     sq, so = q.stride(0), o.stride(0)
@@ -193,7 +199,7 @@ def ssm_scan(x, dt, B, C, A, D, dt_bias, dt_min: float, state, cu, slot, reset, 
         return ref.ssm_scan(x, dt, B, C, A, D, dt_bias, dt_min, state, cu, slot, reset, H, P, N, G, out)
     assert B.stride(0) == C.stride(0) and B.stride(1) == 1 and x.stride(1) == 1 and dt.stride(1) == 1
     f32 = _f32(x, dt, B, C, out)
-    ws = None if f32 or T <= slot.shape[0] or H % G else _chunk_rule_ws(T, slot.shape[0], H, G, N, P, False, state, (B, C, x, out))
+    ws = None if f32 or H % G else _chunk_rule_ws(T, slot.shape[0], H, G, N, P, False, state, (B, C, x, out))
     if ws is not None:
         call("ome_ssm_chunks", x.data_ptr(), x.stride(0), dt.data_ptr(), dt.stride(0), B.data_ptr(), C.data_ptr(),
              B.stride(0), A.data_ptr(), D.data_ptr(), dt_bias.data_ptr(), float(dt_min), state.data_ptr(), out.data_ptr(),
@@ -213,7 +219,7 @@ def gdn_scan(q, k, v, a, b, A_log, dt_bias, state, cu, slot, reset, Hv: int, Hk:
     and v [T, Hv*dv] are row-strided views of one buffer, a / b [T, Hv] views of another, A_log /
     dt_bias fp32 [Hv], state fp32 [slots, Hv, dv, dk] (S transposed: columns contiguous).  q / k
     are L2-normalised in the kernel.  Prompts run in chunks of 32 rows (:func:`_chunk_rule_ws`); one row
-    per sequence, other widths: prep pass + DPP-row scan; ``v1`` selects the one-lane-per-column
+    per sequence, few rows, other widths: prep pass + DPP-row scan; ``v1`` selects the one-lane-per-column
     kernel."""
     T = q.shape[0]
     dv, dk = state.shape[2], state.shape[3]
@@ -225,7 +231,7 @@ def gdn_scan(q, k, v, a, b, A_log, dt_bias, state, cu, slot, reset, Hv: int, Hk:
     assert state.is_contiguous() and state.dtype == torch.float32
     f32 = _f32(q, k, v, a, b, out)
     S = slot.shape[0]
-    ws = None if T <= S or v1 or f32 or Hk <= 0 or Hv % Hk else _chunk_rule_ws(T, S, Hv, Hk, dk, dv, True, state, (q, k, v, out))
+    ws = None if v1 or f32 or Hk <= 0 or Hv % Hk else _chunk_rule_ws(T, S, Hv, Hk, dk, dv, True, state, (q, k, v, out))
     if ws is not None:   # prompts: chunks of 32 rows on the matrix cores
         call("ome_gdn_chunks", q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), a.data_ptr(), b.data_ptr(),
              a.stride(0), A_log.data_ptr(), dt_bias.data_ptr(), state.data_ptr(), out.data_ptr(), out.stride(0),

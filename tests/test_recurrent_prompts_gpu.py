@@ -200,3 +200,34 @@ def test_selective_scan_stays_causal(what, bad):
     hit[at:130, {"x": [0], "dt": [1], "B": [0, 1], "C": [0, 1]}[what]] = True
     assert (got - clean)[~hit].abs().max() <= 2.0 ** -8 * clean.abs().max()
     assert torch.equal(s0[[0, 2]], s1[[0, 2]])
+
+
+@pytest.mark.parametrize("delta", [True, False])
+@pytest.mark.parametrize("lens", [[1] * 3 + [40] + [1] * 60, [3, 4, 0, 2, 33, 1, 5, 32], [2] * 33], ids=str)
+def test_decode_rows_beside_prompts_take_no_chunks(lens, delta, monkeypatch):
+    """Sequences of up to three rows are walked row by row: their chunks of the workspace stay untouched."""
+    kept = []
+
+    def poisoned(*a):
+        kept.append(make(*a).fill_(-7.0))
+        return kept[0]
+
+    make = ops._chunk_rule_ws
+    monkeypatch.setattr(ops, "_chunk_rule_ws", poisoned)
+    (test_delta_rule_prompts(lens, 128, 80, 3, 3, 8) if delta else test_selective_scan_prompts(lens, 16, 64, 128, 2, 8))
+    ws, r0 = kept[0].view(sum(lens) // 32 + len(lens), -1), 0
+    for s, n in enumerate(lens):
+        if n:
+            assert bool((ws[r0 // 32 + s] == -7.0).all()) == (n <= 3), (s, n)
+        r0 += n
+
+
+def test_few_rows_take_the_row_by_row_kernels():
+    def ws(T, S, delta):
+        c = torch.empty(T, 512, dtype=BF, device=DEV)
+        st = torch.empty(S, 2, 64, 128, device=DEV)
+        return ops._chunk_rule_ws(T, S, 2, 2, 128, 64, delta, st, (c[:, :256], c[:, 256:], c, c))
+
+    for delta, few in ((True, 32), (False, 4)):
+        assert ws(few, 1, delta) is None and ws(few, 2, delta) is None and ws(40, 40, delta) is None
+        assert ws(few + 1, 1, delta) is not None and ws(41, 40, delta) is not None
