@@ -389,21 +389,24 @@ __global__ __launch_bounds__(256) void gated_rmsnorm_wave_kernel(const T* __rest
 }
 
 // Any tap count 1 <= K <= 32, and an output that is the input (each thread reads a row before it writes
-// it): one thread per channel walks its sequence, runtime loops.
-template <typename T>
+// it): one thread per channel walks its sequence.  KK > 0: that many taps, known at compile time, so that the window and
+// the taps stay in registers (bf16; sums in the order of ssm_conv1d_kernel).  In place, runtime loops -> KK = 4:
+// 4000 rows of 8192 channels in 3 sequences 827 -> 451 us, one of 500 rows of 4352 218 -> 101, 64 decode rows 11 either way.
+template <typename T, int KK = 0>
 __global__ __launch_bounds__(256) void ssm_conv1d_any_kernel(const T* __restrict__ x, int64_t x_stride,
                                                              const T* __restrict__ w, const T* __restrict__ bias,
                                                              T* __restrict__ out, int64_t out_stride,
                                                              T* __restrict__ state, const int* __restrict__ cu,
                                                              const int* __restrict__ slot, const int* __restrict__ reset,
-                                                             int C, int K) {
+                                                             int C, int taps) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   const int s = blockIdx.y;
   if (c >= C) return;
   const int r0 = cu[s], r1 = cu[s + 1];
   if (r1 <= r0) return;
+  const int K = KK > 0 ? KK : taps;
   T* st = state + ((int64_t)slot[s] * C + c) * (K - 1);
-  float win[31], wt[32];
+  float win[KK > 0 ? KK : 31], wt[KK > 0 ? KK : 32];
   const bool fresh = reset[s] != 0;
   for (int j = 0; j < K - 1; ++j) win[j] = fresh ? 0.f : (float)st[j];
   for (int j = 0; j < K; ++j) wt[j] = (float)w[(int64_t)c * K + j];
@@ -414,7 +417,7 @@ __global__ __launch_bounds__(256) void ssm_conv1d_any_kernel(const T* __restrict
     for (int j = 0; j < K - 1; ++j) acc += wt[j] * win[j];
     for (int j = 0; j + 1 < K - 1; ++j) win[j] = win[j + 1];
     if (K > 1) win[K - 2] = v;
-    out[(int64_t)r * out_stride + c] = (T)(acc / (1.f + expf(-acc)));
+    out[(int64_t)r * out_stride + c] = (T)(KK > 0 ? silu_f(acc) : acc / (1.f + expf(-acc)));
   }
   for (int j = 0; j < K - 1; ++j) st[j] = (T)win[j];
 }
@@ -484,7 +487,7 @@ OME_API int ome_ssm_conv1d(const void* x, int64_t x_stride, const void* w, const
     return 0;
   }
   // 16-byte pieces where every row and the taps allow them, single channels otherwise; an output that
-  // overlaps the input, and more than 6 taps: the kernel that walks each sequence in order
+  // overlaps the input (or lies between its rows), and more than 6 taps: the kernel that walks each sequence in order
   const bf16 *xb = (const bf16*)x, *ob = (const bf16*)out;
   const bool apart = T > 0 && (xb + (int64_t)(T - 1) * x_stride + C <= ob || ob + (int64_t)(T - 1) * out_stride + C <= xb);
   const bool vec8 = C % 8 == 0 && x_stride % 8 == 0 && out_stride % 8 == 0 &&
@@ -494,14 +497,17 @@ OME_API int ome_ssm_conv1d(const void* x, int64_t x_stride, const void* w, const
   const dim3 tiles(((by_seq ? 0 : T / CT) + S + 3) / 4, (lanes + 63) / 64);
 #define CONV_CASE(KK)                                                                                                  \
   case KK:                                                                                                              \
-    if (vec8)                                                                                                           \
+    if (!apart || tiles.y > 65535)                                                                                      \
+      ssm_conv1d_any_kernel<bf16, KK><<<grid, 256, 0, stream>>>((const bf16*)x, x_stride, (const bf16*)w, (const bf16*)bias, \
+                                                                (bf16*)out, out_stride, (bf16*)state, cu, slot, reset, C, K); \
+    else if (vec8)                                                                                                      \
       ssm_conv1d_kernel<KK, 8><<<tiles, 256, 0, stream>>>((const bf16*)x, x_stride, (const bf16*)w, (const bf16*)bias,  \
                                                           (bf16*)out, out_stride, (bf16*)state, cu, slot, reset, S, C, by_seq); \
     else                                                                                                                \
       ssm_conv1d_kernel<KK, 1><<<tiles, 256, 0, stream>>>((const bf16*)x, x_stride, (const bf16*)w, (const bf16*)bias,  \
                                                           (bf16*)out, out_stride, (bf16*)state, cu, slot, reset, S, C, by_seq); \
     break;
-  switch (apart && tiles.y <= 65535 ? K : 0) {
+  switch (K) {
     CONV_CASE(2)
     CONV_CASE(3)
     CONV_CASE(4)

@@ -45,15 +45,17 @@ def test_short_conv(lens, K, C, off):
     assert torch.equal(st.cpu(), sr)
 
 
-def test_short_conv_in_place():
-    """The output may be the input."""
+@pytest.mark.parametrize("K", [2, 3, 4, 5, 6, 7])
+def test_short_conv_in_place(K):
+    """The output may be the input: the same sums in the same order (7 taps: another exponential, one bf16 rounding)."""
     torch.manual_seed(1)
-    sq, C = seqs([40, 1, 19], 4), 256
-    x, w, st = torch.randn(60, C, device=DEV).to(BF), torch.randn(C, 4, device=DEV).to(BF), torch.randn(4, C, 3, device=DEV).to(BF)
+    sq, C = seqs([40, 1, 19], 4), 264
+    x, w, st = torch.randn(60, C, device=DEV).to(BF), torch.randn(C, K, device=DEV).to(BF), torch.randn(4, C, K - 1, device=DEV).to(BF)
     s2 = st.clone()
     want = ops.ssm_conv1d(x, w, None, st, *sq)
     got = ops.ssm_conv1d(x, w, None, s2, *sq, out=x)
     assert torch.allclose(got.float(), want.float(), rtol=2.0 ** -7, atol=1e-5) and torch.equal(st, s2)
+    assert K > 6 or torch.equal(got, want)
 
 
 @pytest.mark.parametrize("group", [64, 128, 256, 512, 1024, 2048])
