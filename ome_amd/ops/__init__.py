@@ -171,8 +171,9 @@ def _chunk_rule_floats(H: int, G: int, delta: bool) -> int:
 def _chunk_rule_ws(T: int, S: int, H: int, G: int, dk: int, dv: int, delta: bool, state: torch.Tensor, rows: tuple) -> torch.Tensor | None:
     """Workspace of the chunked kernels (``chunk_rule.hip``) for T rows of S sequences and H heads, or None
     where the row-by-row kernels run: one row per sequence (a decode step; a chunk would be 1/32 full), few rows in all, key
-    widths other than 64 / 128, value widths not of 16 columns, or key / query rows (the first two
-    of ``rows``, the operands and the output) that 16-byte loads cannot take.
+    widths other than 64 / 128, value widths not of 16 columns, key / query rows (the first two
+    of ``rows``, the operands and the output) that 16-byte loads cannot take, or an output in the place of the values
+    (a sequence whose state is no longer finite is read a second time).
 
     Few rows: the two launches of the chunks and their serial chain take 16 us (delta rule, 32 heads of 128 x 128) and 12
     (selective scan, 128 of 64 x 128) for one sequence of up to 32 rows.  Row by row, 2 / 8 / 20 / 40 rows 8 / 11 / 15 / 24
@@ -184,7 +185,7 @@ def _chunk_rule_ws(T: int, S: int, H: int, G: int, dk: int, dv: int, delta: bool
     q, k, o = rows[0], rows[1], rows[-1]   # (a shared row stride for q, k and v / B and C)
     sq, so = q.stride(0), o.stride(0)
     if (state.data_ptr() | q.data_ptr() | k.data_ptr()) % 16 or sq % 8 or not (0 <= sq < 1 << 24 and 0 <= so < 1 << 24) or \
-            not 0 <= rows[-2].stride(0) < 1 << 24:
+            not 0 <= rows[-2].stride(0) < 1 << 24 or o.data_ptr() == rows[-2].data_ptr():
         return None
     return torch.empty((T // 32 + S) * _chunk_rule_floats(H, G, delta), dtype=torch.float32, device=state.device)
 

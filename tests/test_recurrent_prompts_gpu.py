@@ -205,6 +205,30 @@ def test_selective_scan_stays_causal(what, bad):
 
 
 @pytest.mark.parametrize("delta", [True, False])
+def test_scans_in_place_of_their_values(delta):
+    """... as elsewhere, with a value that is not finite in the second of three sequences."""
+    torch.manual_seed(7)
+    H, dk, dv, lens, at = 4, 64, 32, [40, 90, 33], 40 + 43
+    T, sq = sum(lens), (i32([0, 40, 130, 163]), i32([0, 1, 2]), i32([0, 1, 0]))
+    c, ab = torch.randn(T, 2 * H * dk + H * dv, device=DEV).to(BF), torch.randn(T, 2 * H, device=DEV).to(BF)
+    c[at, 2 * H * dk + 1] = float("nan")
+    A, D, dtb, st = torch.linspace(-2, -0.1, H, device=DEV), torch.ones(H, device=DEV), torch.zeros(H, device=DEV), torch.randn(3, H, dv, dk, device=DEV)
+
+    def run(s, out):
+        q, k, v = c[:, :H * dk], c[:, H * dk:2 * H * dk], c[:, 2 * H * dk:]
+        if delta:
+            return ops.gdn_scan(q, k, v, ab[:, :H], ab[:, H:], A, dtb, s, *sq, H, H, out=out)
+        return ops.ssm_scan(v, ab[:, :H], k, q, A, D, dtb, 0.001, s, *sq, H, dv, dk, H, out=out)
+
+    s0, s1 = st.clone(), st.clone()
+    want = run(s0, None).float()
+    got = run(s1, c[:, 2 * H * dk:]).float()
+    # another path's sums: one bf16 step of the largest value; states in fp32, of the same order
+    assert torch.equal(got.isfinite(), want.isfinite()) and (got - want).nan_to_num(0.0).abs().max() <= 2.0 ** -8 * want.nan_to_num(0.0).abs().max()
+    assert torch.equal(s0.isfinite(), s1.isfinite()) and (s0 - s1).nan_to_num(0.0).abs().max() <= 1e-5 * st.abs().max()
+
+
+@pytest.mark.parametrize("delta", [True, False])
 @pytest.mark.parametrize("lens", [[1] * 3 + [40] + [1] * 60, [3, 4, 0, 2, 33, 1, 5, 32], [2] * 33], ids=str)
 def test_decode_rows_beside_prompts_take_no_chunks(lens, delta, monkeypatch):
     """Sequences of up to three rows are walked row by row: their chunks of the workspace stay untouched."""
@@ -228,7 +252,7 @@ def test_few_rows_take_the_row_by_row_kernels():
     def ws(T, S, delta):
         c = torch.empty(T, 512, dtype=BF, device=DEV)
         st = torch.empty(S, 2, 64, 128, device=DEV)
-        return ops._chunk_rule_ws(T, S, 2, 2, 128, 64, delta, st, (c[:, :256], c[:, 256:], c, c))
+        return ops._chunk_rule_ws(T, S, 2, 2, 128, 64, delta, st, (c[:, :256], c[:, 256:], c, torch.empty_like(c)))
 
     for delta, few in ((True, 32), (False, 4)):
         assert ws(few, 1, delta) is None and ws(few, 2, delta) is None and ws(40, 40, delta) is None
