@@ -200,7 +200,10 @@ OME_API int ome_rope_qkv_cache(const void* qkv, int64_t qkv_stride, const int* p
   const float ki = 1.f / k_scale, vi = 1.f / v_scale;
   // blocks per token: enough 4-wave blocks that each covers at most one 4-head group per wave
   const int per_block = 4 * (512 / D);
-  // (decode batches only: 5.4 vs 6.3 us at T = 256; no gain once T fills the chip)
+  // Blocks over heads (decode batches: 4.1 us against 5.3 with one block a token at T = 256, 5.1 / 6.2 at 384, 5.9 / 6.7 at 500;
+  // no gain once T fills the chip, 6.7 / 6.7 at 512) or whole pages of V (prompts; one block a token): 3.3 / 3.7 us at T = 128,
+  // 4.1 / 4.0 at 256, 5.9 / 5.1 at 500, 6.7 / 4.6 at 512, 10.3 / 6.4 at 1024, 31 / 18 at 4096; fp8 3.1 / 3.8, 3.6 / 3.9,
+  // 4.9 / 4.8, 5.7 / 4.6, 8.1 / 6.0, 23 / 18.  Below 512 a step is as likely decode rows, which share no page.
   int ny = g_rope_split > 0 ? g_rope_split : (T < 512 ? (Hq + Hkv + per_block - 1) / per_block : 1);
   ny = ny < 1 ? 1 : (ny > 8 ? 8 : ny);
   const dim3 grid(T, ny);
