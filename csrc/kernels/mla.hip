@@ -248,7 +248,7 @@ __device__ __forceinline__ void page_to_lds(const bf16* base, uint32_t bytes, ui
 // of 146 us below).
 //
 // Measured (16-head kernel, or for decode the 16-row waves before -> now): three prompts of 3394 rows x 16 heads
-// 738 -> 146 us (118 -> 598 TFLOP/s); decode, 48 contexts of ~3000 keys x 128 heads 100 -> 86 us.
+// 738 -> 146 us (118 -> 598 TFLOP/s); decode, 48 contexts of ~3000 keys x 128 heads 100 -> 88 us.
 // ------------------------------------------------------------------------------------------
 // The products by asm: with one wave per SIMD, what covers an LDS read is the distance to its product, and the
 // compiler sinks reads to their use (or hoists them all, into scratch).  Volatile with a memory clobber, each stays
