@@ -1022,11 +1022,6 @@ class MLAWorkspace:
         self.plan = torch.empty(self.TARGET_WGS_ALL, 2, dtype=torch.int32, device=device)
 
     @classmethod
-    def rows(cls, T: int, H: int, DK: int = 576, seqs: int = 1 << 30, pages: int = 1 << 30) -> tuple[int, bool]:
-        """The first two of :meth:`tiles`."""
-        return cls.tiles(T, H, DK, seqs, pages)[:2]
-
-    @classmethod
     @functools.lru_cache(maxsize=4096)
     def tiles(cls, T: int, H: int, DK: int = 576, seqs: int = 1 << 30, pages: int = 1 << 30,
               longest: bool = False) -> tuple[int, bool, int]:
