@@ -14,14 +14,16 @@
 // chunk_rule_kernel walks the chunks of a (sequence, head) in order: a wave owns 16 value columns and keeps its
 // S in VGPR accumulators.
 //
-// What bounds it: the chain of chunks.  Two waves a SIMD (S, one chunk's rows in flight and the split
-// parts fill the registers) share its matrix and vector units at about 60 matrix (DELTA: 96) and 500 vector
-// instructions a chunk, near 3 us with the latencies between them; its memory traffic hides behind that (leaving
-// the reads out gives 1%).  Per-head P, formed in the first launch, cost 40 us there and 108 in the scan
-// (Mamba-2, below): written and read back it is 16 times the bytes of its group's q k^T.
-//   gated delta rule, 32 heads of 128 x 128, prompts of 1001 / 1435 / 1564 rows:   24 + 123 us (row by row: 1098)
-//   selective scan, 128 heads of 64 x 128, 8 groups, 1033 / 926 / 1248 / 293 rows:  11 + 116 us (row by row: 1745)
-// Largest error of the state against 64 bits: 1.1e-7 (row by row: 2.0e-7) and 1.4e-7 (6.2e-7) of its norm.
+// What bounds it: the instructions of a wave that has its SIMD almost for itself, 96 matrix (Mamba-2: 60) and some 250 (310) vector
+// ones a chunk.  A product takes 16 cycles alone, but about 9 of them stay its own where vector instructions of 4 cycles fill
+// the rest, so a chunk is 2000 cycles of issue and as much again of LDS latency, address arithmetic and dependencies.  Hence the
+// next chunk moves to LDS by DMA, without a register or a store on the way; values and outputs move in pieces of four columns
+// (q S is formed transposed for that); T and P T are products of three bf16 parts each, at half the fp32 product's time.
+// Memory traffic hides behind that.  Two fp16 parts instead of three bf16 ones would take a quarter less time, but the state came out
+// 2.3 times further from 64 bits: an fp16 value below 2^-14 has no lower part.
+//   gated delta rule, 32 heads of 128 x 128, prompts of 1001 / 1435 / 1564 rows:   22 + 97 us (before: 24 + 123; row by row: 1098)
+//   selective scan, 128 heads of 64 x 128, 8 groups, 1033 / 926 / 1248 / 293 rows:  10 + 93 us (before: 11 + 116; row by row: 1745)
+// Largest error of the state against 64 bits: 1.2e-7 (row by row: 2.0e-7) and 1.2e-7 (6.2e-7) of its norm.
 //
 // A chunk's products multiply the entries that causality zeroes as well, and 0 times an infinity or NaN is NaN, so a key,
 // gate or value that is not finite would reach the rows before it in its chunk.  It reaches S and stays there (each
@@ -30,9 +32,10 @@
 //
 // fp32 throughout: k and q enter the matrix cores as the bf16 values that they are (their norms, 1 / |k| and
 // 1 / (|q| sqrt(dk)), scale results), S and U as three bf16 parts that sum to the fp32 value exactly, at
-// 3/16 of the fp32 MFMA's time; T R and P U, where both operands are fp32, take the fp32 MFMA.  Decay
-// exponents are summed in fp64 (differences of a long sum).  The row-by-row kernels stay for decode steps
-// (one row per sequence), few rows in all, dk other than 64 / 128, and unaligned views.
+// 3/16 of the fp32 MFMA's time; T R and P U, where both operands are fp32, take the six products of their parts down to
+// 2^-16 of the first (what is left out is below 2^-24, an fp32 rounding).  Decay exponents are summed in fp64 (differences of
+// a long sum).  The row-by-row kernels stay for decode steps (one row per sequence), few rows in all, dk other than 64 / 128, and
+// unaligned views of q and k.
 #include "common.h"
 
 namespace {
@@ -40,18 +43,23 @@ namespace {
 constexpr int RC = 32;            // rows of a chunk
 constexpr int LDM = RC + 4;       // padded row of a 32 x 32 fp32 matrix in LDS
 typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// workspace of one chunk.  DELTA, per head: P T, T, then the vectors a, b, c, d [32] and g_C.  Mamba-2, per group: q k^T
-// (its heads differ in their decays only, which the scan applies: P itself would be 16 times the bytes); then
-// per head the vectors a, cum's upper and lower parts, c, d and g_C.
-constexpr int NV_DELTA = 4 * RC + 4, NV_SSM = 5 * RC + 4;
+// Workspace of one chunk, in bytes: (Mamba-2) of every group q k^T in fp32, which its heads share (they differ in their decays only,
+// which the scan applies: P itself would be 16 times the bytes); of every head (DELTA) the images of T and P T, each in three
+// bf16 parts, as LDS holds them, and its vectors, 32 floats each: DELTA a, b, c, d of the scan, then g_C;  Mamba-2 a, cum's upper and
+// lower parts, c, d, then g_C.
+constexpr int MAT = RC * RC * 2;      // a part of a 32 x 32 matrix
+constexpr int VECS = 1024;            // the vectors, in whole LDS moves
 template <bool DELTA>
-constexpr int vec_floats() { return DELTA ? NV_DELTA : NV_SSM; }
+constexpr int vec_floats() { return (DELTA ? 4 : 5) * RC + 4; }
 template <bool DELTA>
-__host__ __device__ constexpr int64_t ws_floats(int H, int G) {
-  return DELTA ? (int64_t)H * (2 * RC * RC + NV_DELTA) : (int64_t)G * RC * RC + (int64_t)H * NV_SSM;
-}
+__host__ __device__ constexpr int64_t group_bytes() { return DELTA ? 0 : 4 * RC * RC; }
+template <bool DELTA>
+__host__ __device__ constexpr int64_t head_bytes() { return (DELTA ? 6 * MAT : 0) + VECS; }
+template <bool DELTA>
+__host__ __device__ constexpr int64_t ws_bytes(int H, int G) { return G * group_bytes<DELTA>() + H * head_bytes<DELTA>(); }
 
 struct RuleArgs {
   const bf16 *q, *k, *v;          // rows of stride `stride` (v: v_stride)
@@ -60,7 +68,7 @@ struct RuleArgs {
   int64_t ab_stride;
   const float *A, *D, *dt_bias;   // A_log (DELTA) / A, D (Mamba-2)
   float dt_min;
-  float* ws;
+  char* ws;
   float* state;                   // [slots, H, dv, dk]
   bf16* out;
   int64_t out_stride;
@@ -100,25 +108,37 @@ __device__ __forceinline__ f32x4 mma_f32(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// eight fp32 values -> three bf16 vectors that sum to them exactly (8 bits of the mantissa each)
+// Eight fp32 values -> three bf16 vectors that sum to them exactly.  What a rounding took by v_dot2_f32_bf16, the value minus the
+// half of a packed pair: seven instructions a pair (eleven by masks, shifts and subtractions).
 __device__ __forceinline__ void split3(f32x4 x0, f32x4 x1, bf16x8 (&p)[3]) {
-  float r[8];
+  uint32_t lo = 0x0000bf80u, hi = 0xbf800000u;   // (-1, 0) and (0, -1); out of sight, or they become inline constants, of which
+  asm("" : "+s"(lo), "+s"(hi));                  // the instruction takes another pair of halves
+  const bf16x2 first = __builtin_bit_cast(bf16x2, lo), second = __builtin_bit_cast(bf16x2, hi);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) r[j] = x0[j], r[4 + j] = x1[j];
+  for (int j = 0; j < 4; ++j) {
+    float a = j < 2 ? x0[2 * j] : x1[2 * j - 4], b = j < 2 ? x0[2 * j + 1] : x1[2 * j - 3];
 #pragma unroll
-  for (int t = 0; t < 3; ++t) {
-    u32x4 w;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t lo = __float_as_uint(r[2 * j]), hi = __float_as_uint(r[2 * j + 1]);
-      w[j] = __builtin_amdgcn_perm(hi, lo, 0x07060302);   // the two upper halves
+    for (int t = 0; t < 3; ++t) {
+      const bf16x2 h = {(bf16)a, (bf16)b};
+      p[t][2 * j] = h[0];
+      p[t][2 * j + 1] = h[1];
       if (t < 2) {
-        r[2 * j] -= __uint_as_float(lo & 0xffff0000u);
-        r[2 * j + 1] -= __uint_as_float(hi & 0xffff0000u);
+        a = __builtin_amdgcn_fdot2_f32_bf16(h, first, a, false);
+        b = __builtin_amdgcn_fdot2_f32_bf16(h, second, b, false);
       }
     }
-    p[t] = __builtin_bit_cast(bf16x8, w);
   }
+}
+
+// c + a b of operands in three parts: the six products down to 2^-16 of the first
+template <bool SWAP = false>
+__device__ __forceinline__ void mma_parts(const bf16x8 (&a)[2][3], const bf16x8 (&b)[3], f32x4 (&c)[2]) {
+#pragma unroll
+  for (int sum = 2; sum >= 0; --sum)
+#pragma unroll
+    for (int i = 0; i <= sum; ++i)
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) c[rb] = SWAP ? mma_bf16(b[sum - i], a[rb][i], c[rb]) : mma_bf16(a[rb][i], b[sum - i], c[rb]);
 }
 
 // LDS written by lanes of a wave, read by others of the same wave
@@ -129,10 +149,26 @@ __device__ __forceinline__ void wave_sync() {
 
 __device__ __forceinline__ float softplus_rule(float x) { return x > 20.f ? x : log1pf(__expf(x)); }
 
+// 16-byte piece `chunk` of row `row` in an image of k or q rows; byte offset of columns 4 g .. + 3 and 16 + 4 g .. + 3 (the
+// k-slots of a lane of group g) of row `row` in a part of a 32 x 32 matrix; piece of eight columns in an image of values.
+// Swizzled, so that the pieces of 16 rows (k and q: and four pieces of four rows, as a transposed read takes them) lie in all banks.
+template <int DK>
+__device__ __forceinline__ int img(int row, int chunk) {
+  return row * (DK / 8) + (chunk ^ (DK == 128 ? (row & 3) << 2 | ((row >> 2) & 3) : ((row >> 1) & 1) << 2 | ((row >> 2) & 3)));
+}
+__device__ __forceinline__ int mat_img(int row, int g) { return row * (RC * 2) + ((g ^ ((row >> 2) & 3)) << 4); }
+__device__ __forceinline__ int val_img(int row, int piece) { return row * 8 + (piece ^ (((row >> 1) & 3) << 1)); }
+
+__device__ __forceinline__ bf16x4 tr4(const bf16* base, int elem) {
+  const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (s16x4 __attribute__((address_space(3)))*)((__attribute__((address_space(3))) bf16*)base + elem));
+  return __builtin_bit_cast(bf16x4, v);
+}
+
 // ---------------------------------------------------------------------------------------------
 // One wave per (chunk, head).  The 16-byte row pieces that a lane loads are both operands of q k^T and
-// k k^T (rows and columns of a 16 x 16 x 32 product have the same lane layout).  T by forward substitution: lane j
-// keeps column j in registers and reads the rows of A from LDS as broadcasts.
+// k k^T (rows and columns of a 16 x 16 x 32 product have the same lane layout).  T's diagonal blocks by forward substitution:
+// lane j keeps column j in registers and reads the rows of A from LDS as broadcasts.
 // ---------------------------------------------------------------------------------------------
 template <int DK>
 __global__ __launch_bounds__(256) void chunk_gram_kernel(RuleArgs a) {
@@ -145,7 +181,7 @@ __global__ __launch_bounds__(256) void chunk_gram_kernel(RuleArgs a) {
   int r0, n;
   if (h >= a.H || !chunk_of(blockIdx.x, a.cu, a.S, r0, n)) return;   // whole wave; no block barrier below
   const int hk = h / (a.H / a.Hk);
-  float* ws = a.ws + ((int64_t)blockIdx.x * a.H + h) * (2 * RC * RC + NV_DELTA);
+  char* ws = a.ws + blockIdx.x * ws_bytes<true>(a.H, a.Hk) + h * head_bytes<true>();
 
   bf16x8 kf[2][NS], qf[2][NS];
 #pragma unroll
@@ -193,7 +229,7 @@ __global__ __launch_bounds__(256) void chunk_gram_kernel(RuleArgs a) {
   wave_sync();
   const float ik = s_vec[w][0][row], iq = s_vec[w][1][row];
   if (lane < RC) {   // the chunk's vectors (zero past its end: such rows add nothing anywhere)
-    float* vec = ws + 2 * RC * RC;
+    float* vec = reinterpret_cast<float*>(ws + 6 * MAT);
     const float gi = __expf((float)cum), up = __expf((float)(total - cum));
     vec[row] = ok ? beta : 0.f;
     vec[RC + row] = ok ? beta * gi * ik : 0.f;
@@ -231,37 +267,55 @@ __global__ __launch_bounds__(256) void chunk_gram_kernel(RuleArgs a) {
       }
     }
   wave_sync();
-  float t[RC];
+  // T in blocks of 16: T11 and T22 by substitution, in place of A11 and A22; T21 = -T22 (A21 T11)
+  const int d16 = row & 16;
+  float t[16];
 #pragma unroll
-  for (int i = 0; i < RC; ++i) {
-    float acc[4] = {i == row ? 1.f : 0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < 16; ++i) {
+    float acc[4] = {i == col ? 1.f : 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int m = 0; m < i; m += 4) {
-      const f32x4 x = *reinterpret_cast<const f32x4*>(&sA[w][i * LDM + m]);
+      const f32x4 x = *reinterpret_cast<const f32x4*>(&sA[w][(d16 + i) * LDM + d16 + m]);
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         if (m + e < i) acc[e] -= x[e] * t[m + e];
     }
     t[i] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
   }
-  if (lane < RC) {
-#pragma unroll
-    for (int i = 0; i < RC; ++i) ws[RC * RC + i * RC + row] = t[i];
-  }
-  // P T: T's columns go through LDS into the product's operand layout (k-slot of step e: row 4 g + e)
   wave_sync();
-  if (lane < RC) {
 #pragma unroll
-    for (int i = 0; i < RC; ++i) sA[w][i * LDM + row] = t[i];
-  }
+  for (int i = 0; i < 16; ++i) sA[w][(d16 + i) * LDM + d16 + col] = t[i];   // (both half waves the same)
   wave_sync();
-  f32x4 tb[2][2];   // [row block][column block]
+  // operands of 16 x 16 x 4 products: the k-slot of step e is row (column) 4 g + e
+  f32x4 tb[2][2];   // T [row block][column block], as a right operand
 #pragma unroll
-  for (int kb = 0; kb < 2; ++kb)
+  for (int d = 0; d < 2; ++d)
 #pragma unroll
-    for (int cb = 0; cb <= kb; ++cb)
+    for (int e = 0; e < 4; ++e) tb[d][d][e] = sA[w][(16 * d + 4 * g + e) * LDM + 16 * d + col];
+  const f32x4 a21 = *reinterpret_cast<const f32x4*>(&sA[w][(16 + col) * LDM + 4 * g]), t22 = *reinterpret_cast<const f32x4*>(&sA[w][(16 + col) * LDM + 16 + 4 * g]);
+  f32x4 at = {0.f, 0.f, 0.f, 0.f};
+  tb[1][0] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) tb[kb][cb][e] = sA[w][(16 * kb + 4 * g + e) * LDM + 16 * cb + col];
+  for (int e = 0; e < 4; ++e) at = mma_f32(-a21[e], tb[0][0][e], at);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) tb[1][0] = mma_f32(t22[e], at[e], tb[1][0]);
+  wave_sync();
+#pragma unroll
+  for (int e = 0; e < 4; ++e) sA[w][(16 + 4 * g + e) * LDM + col] = tb[1][0][e];
+  wave_sync();
+  // a 32 x 32 matrix out of LDS, in three bf16 parts, to its images
+  const auto parts = [&](char* to) {
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+      const f32x4 lo = *reinterpret_cast<const f32x4*>(&sA[w][(16 * rb + col) * LDM + 4 * g]);
+      const f32x4 hi = *reinterpret_cast<const f32x4*>(&sA[w][(16 * rb + col) * LDM + 16 + 4 * g]);
+      bf16x8 p[3];
+      split3(lo, hi, p);
+#pragma unroll
+      for (int x = 0; x < 3; ++x) *reinterpret_cast<bf16x8*>(to + x * MAT + mat_img(16 * rb + col, g)) = p[x];
+    }
+  };
+  parts(ws);
   wave_sync();
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb)
@@ -270,20 +324,28 @@ __global__ __launch_bounds__(256) void chunk_gram_kernel(RuleArgs a) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) sA[w][(16 * rb + 4 * g + e) * LDM + 16 * cb + col] = pm[rb][cb][e];
   wave_sync();
+  f32x4 pt[2][2];
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
     for (int cb = 0; cb < 2; ++cb) {
-      f32x4 d = {0.f, 0.f, 0.f, 0.f};
+      pt[rb][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kb = cb; kb <= rb; ++kb) {
         const f32x4 m = *reinterpret_cast<const f32x4*>(&sA[w][(16 * rb + col) * LDM + 16 * kb + 4 * g]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) d = mma_f32(m[e], tb[kb][cb][e], d);
+        for (int e = 0; e < 4; ++e) pt[rb][cb] = mma_f32(m[e], tb[kb][cb][e], pt[rb][cb]);
       }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) ws[(16 * rb + 4 * g + e) * RC + 16 * cb + col] = d[e];
     }
+  wave_sync();
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sA[w][(16 * rb + 4 * g + e) * LDM + 16 * cb + col] = pt[rb][cb][e];
+  wave_sync();
+  parts(ws + 3 * MAT);
 }
 
 // Mamba-2: one block per (chunk, group).  Wave 0 multiplies q k^T (lower triangle), every half wave takes heads.
@@ -293,7 +355,7 @@ __global__ __launch_bounds__(256) void ssm_gram_kernel(RuleArgs a) {
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4, hk = blockIdx.y;
   int r0, n;
   if (!chunk_of(blockIdx.x, a.cu, a.S, r0, n)) return;   // the same in every wave
-  float* ws = a.ws + blockIdx.x * ws_floats<false>(a.H, a.Hk);
+  char* ws = a.ws + blockIdx.x * ws_bytes<false>(a.H, a.Hk);
   if (w == 0) {
     bf16x8 kf[2][NS], qf[2][NS];
 #pragma unroll
@@ -305,6 +367,7 @@ __global__ __launch_bounds__(256) void ssm_gram_kernel(RuleArgs a) {
         qf[rb][s] = ld8(a.q + r * a.stride + hk * DK + 32 * s + 8 * g);
       }
     }
+    float* gram = reinterpret_cast<float*>(ws + hk * group_bytes<false>());
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
@@ -313,7 +376,7 @@ __global__ __launch_bounds__(256) void ssm_gram_kernel(RuleArgs a) {
 #pragma unroll
         for (int s = 0; s < NS; ++s) qk = mma_bf16(qf[rb][s], kf[cb][s], qk);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) ws[hk * RC * RC + (16 * rb + 4 * g + e) * RC + 16 * cb + col] = qk[e];
+        for (int e = 0; e < 4; ++e) gram[(16 * rb + 4 * g + e) * RC + 16 * cb + col] = qk[e];
       }
   }
   const int row = lane & 31, rv = r0 + min(row, n - 1), per = a.H / a.Hk;
@@ -329,7 +392,7 @@ __global__ __launch_bounds__(256) void ssm_gram_kernel(RuleArgs a) {
     }
     const double total = __shfl(cum, 31, 32);   // rows past the chunk's end add nothing
     if (i < per) {
-      float* vec = ws + a.Hk * RC * RC + h * NV_SSM;
+      float* vec = reinterpret_cast<float*>(ws + a.Hk * group_bytes<false>() + h * head_bytes<false>());
       const float hi = (float)cum;
       vec[row] = ok ? dt : 0.f;
       vec[RC + row] = hi;
@@ -341,111 +404,129 @@ __global__ __launch_bounds__(256) void ssm_gram_kernel(RuleArgs a) {
   }
 }
 
+// The sequence whose workgroups (`per` of them) come z-th: the longest first, and of the sequences that begin a second round over the CUs
+// the shortest first, so that a CU's two workgroups are as long as another's (four prompts of 293 to 1248 rows, 128 heads: 106 -> 93 us).
+// Whole wave.  (More than a wave of sequences: as they come.)
+__device__ __forceinline__ int in_turn(int z, int per, const int* cu, int S) {
+  if (S == 1 || S > 64) return z;
+  const int lane = threadIdx.x & 63, len = lane < S ? cu[lane + 1] - cu[lane] : -1, round = max(256 / per, 1), k = z / round;
+  int rank = 0;
+  for (int j = 0; j < S; ++j) {
+    const int other = __builtin_amdgcn_readlane(len, j);
+    rank += other > len || (other == len && j < lane);
+  }
+  const int want = k & 1 ? min(S, (k + 1) * round) - 1 - (z - k * round) : z;
+  return __builtin_ctzll(__ballot(lane < S && rank == want));
+}
+
 // ---------------------------------------------------------------------------------------------
 // The chunks of one (sequence, head) in order; block = NW waves x 16 value columns.  D rows of a 16 x 16
 // product sit at 4 g + e, so with block b of S standing for key channels 32 (b / 2) + 8 (row / 4) + 4 (b % 2) +
 // row % 4, blocks 2 s and 2 s + 1 of a lane are the eight k-slots of step s of k S and q S: S never
 // leaves its registers.  S += k^T U takes k transposed out of the same LDS image (ds_read_b64_tr_b16).  The
-// next chunk's rows and matrices travel to registers while this chunk is computed and to the other LDS
-// buffer after it: one barrier per chunk.
+// next chunk moves to the other LDS buffer while this one is computed: one barrier per chunk.
+// VEC: values in 16-byte pieces by DMA, outputs in 8-byte ones; not: element by element (views that are not aligned for that).
 // ---------------------------------------------------------------------------------------------
-template <int DK>
-__device__ __forceinline__ int img(int row, int chunk) { return row * (DK / 8) + (chunk ^ (row & (DK / 8 - 1))); }
-
-__device__ __forceinline__ bf16x4 tr4(const bf16* base, int elem) {
-  const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      (s16x4 __attribute__((address_space(3)))*)((__attribute__((address_space(3))) bf16*)base + elem));
-  return __builtin_bit_cast(bf16x4, v);
-}
-
-template <int DK, bool DELTA, int NW>
+template <int DK, bool DELTA, int NW, bool VEC>
 __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
-  constexpr int NS = DK / 32, NB = DK / 16, NT = 64 * NW;
-  constexpr int NKL = RC * DK / 8 / NT, NML = RC * RC / 4 / NT;   // 16-byte loads per thread: k (and q), P (and T)
-  static_assert(NKL * NT * 8 == RC * DK && NML * NT * 4 == RC * RC, "whole loads");
-  __shared__ __attribute__((aligned(16))) bf16 sK[2][RC * DK], sQ[2][RC * DK];
-  __shared__ __attribute__((aligned(16))) float sP[2][RC * LDM], sT[DELTA ? 2 : 1][DELTA ? RC * LDM : 4], sV[2][vec_floats<DELTA>()];
-  const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, g = lane >> 4;
-  const int s = blockIdx.z, h = blockIdx.x, hk = h / (a.H / a.Hk);
-  const int n0 = (blockIdx.y * NW + (tid >> 6)) * 16;   // this wave's columns
-  const bool live = n0 < a.dv;                          // dv is a multiple of 16: a wave has all of them or none
+  constexpr int NS = DK / 32, NB = DK / 16, NT = 64 * NW, COLS = 16 * NW;
+  constexpr int NML = RC * RC / 4 / NT;                  // 16-byte loads of q k^T per thread (Mamba-2)
+  static_assert(NML * NT * 4 == RC * RC && RC * COLS == 8 * NT, "whole loads");
+  // a chunk in LDS: k and q rows, T and P T (Mamba-2: P) in three parts each, the vectors, the values
+  constexpr int ROWS = RC * DK * 2, M_AT = 2 * ROWS, V_AT = M_AT + (DELTA ? 6 : 3) * MAT, X_AT = V_AT + VECS, IMG = X_AT + RC * COLS * 2;
+  __shared__ __attribute__((aligned(1024))) char lds[2 * IMG];
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)lds;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4;
+  const int s = in_turn(blockIdx.z, gridDim.x * gridDim.y, a.cu, a.S), h = blockIdx.x, hk = h / (a.H / a.Hk);
+  const int c0 = blockIdx.y * COLS, n0 = c0 + wave * 16;   // the block's and this wave's columns
+  const bool live = n0 < a.dv;                             // dv is a multiple of 16: a wave has all of them or none
   const int r0 = a.cu[s], r1 = a.cu[s + 1];
-  if (r1 <= r0) return;                                 // whole block
+  if (r1 <= r0) return;                                    // whole block
   const int chunks = (r1 - r0 + RC - 1) / RC;
   const int nc = (live ? n0 : 0) + col;
 
-  // byte offsets of this thread's pieces within a chunk's 32 rows, against uniform bases; a last chunk of fewer
-  // rows repeats its last one (whose scalars are zero)
-  uint32_t ko[NKL], vo[8];
-  auto offsets = [&](int n) {
+  // values: thread -> row tid / 8, eight columns (beyond dv: the first eight); a last chunk of fewer rows repeats its last
+  // one (whose scalars are zero)
+  static_assert(COLS == 64, "eight pieces a row");
+  const int xr = tid / 8, xp8 = 8 * (val_img(xr, tid % 8) - 8 * xr), xc = c0 + xp8 < a.dv ? xp8 : 0;
+  uint32_t xo;
+  const char* xp = reinterpret_cast<const char*>(a.v + (int64_t)r0 * a.v_stride + (int64_t)h * a.dv + c0);
+  // rows of k and q: a lane's 16-byte piece of each move of 1024 bytes, against uniform bases
+  constexpr int NR = ROWS / 1024 / NW, NH = (int)head_bytes<DELTA>() / 1024;
+  static_assert(NR * NW * 1024 == ROWS && (NH - 1) % NW == 0, "whole moves");
+  uint32_t ko[NR];
+  const auto offsets = [&](int n) {
+    xo = 2 * ((uint32_t)min(xr, n - 1) * (uint32_t)a.v_stride + (uint32_t)xc);
 #pragma unroll
-    for (int i = 0; i < NKL; ++i) {
-      const int e = tid + NT * i;
-      ko[i] = 2 * ((uint32_t)min(e / (DK / 8), n - 1) * (uint32_t)a.stride + 8 * (e % (DK / 8)));
+    for (int i = 0; i < NR; ++i) {
+      const int e = 64 * (wave + NW * i) + lane, row = e / (DK / 8);
+      ko[i] = 2 * ((uint32_t)min(row, n - 1) * (uint32_t)a.stride + 8 * (uint32_t)(img<DK>(row, e % (DK / 8)) - row * (DK / 8)));
     }
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-      vo[e] = 2 * ((uint32_t)min(16 * (e >> 2) + 4 * g + (e & 3), n - 1) * (uint32_t)a.v_stride + (uint32_t)nc);
   };
-  const char* kp = reinterpret_cast<const char*>(a.k + (int64_t)r0 * a.stride + hk * DK);
+  const int64_t x_step = (int64_t)RC * 2 * a.v_stride, k_step = (int64_t)RC * 2 * a.stride, ws_step = ws_bytes<DELTA>(a.H, a.Hk), o_step = (int64_t)RC * 2 * a.out_stride;
+  const char* kp = reinterpret_cast<const char*>(a.k + (int64_t)r0 * a.stride + hk * DK);   // these walk with the chunks fetched
   const char* qp = reinterpret_cast<const char*>(a.q + (int64_t)r0 * a.stride + hk * DK);
-  const char* vp = reinterpret_cast<const char*>(a.v + (int64_t)r0 * a.v_stride + (int64_t)h * a.dv);
-  const int64_t ws_step = 4 * ws_floats<DELTA>(a.H, a.Hk);
-  const char* mp = reinterpret_cast<const char*>(a.ws) + (r0 / RC + s) * ws_step +
-                   4 * (DELTA ? (int64_t)h * (2 * RC * RC + NV_DELTA) : (int64_t)hk * RC * RC);
-  const uint32_t vec_at = 4 * (DELTA ? 2 * RC * RC : (a.Hk - hk) * RC * RC + h * NV_SSM);   // the vectors, from there
-  bf16x8 rk[NKL], rq[NKL];
-  f32x4 rp[NML], rt[NML], rvec, rhj[NML], rlj[NML];
+  const char* gp = a.ws + (r0 / RC + s) * ws_step + hk * group_bytes<DELTA>();
+  const char* hp = a.ws + (r0 / RC + s) * ws_step + a.Hk * group_bytes<DELTA>() + h * head_bytes<DELTA>();
+  f32x4 rp[NML], rhj[NML], rlj[NML];
   float rhi[NML], rli[NML];
-  bf16 rv[8];
-  auto fetch = [&](int c) {   // rows and matrices of chunk c
-    if (r0 + (c + 1) * RC > r1) offsets(r1 - r0 - c * RC);
-    const int64_t kc = (int64_t)c * RC * 2 * a.stride;
+  bf16x8 rx;
+  // The next chunk to LDS buffer b in three steps, for the vector memory unit to take one while another is computed.  `more`: there
+// is one; without, nothing is moved and what goes to registers is the last one again (no branch, which would part the stages).
+  const auto fetch = [&](int n, bool more, int b) {
+    if (more && n < RC) offsets(n);
+    const uint32_t to = lds0 + b * IMG, kb = (RC - 1) * 2 * (uint32_t)a.stride + 2 * DK;
+    if constexpr (VEC) {
+      buffer_to_lds(xp, more ? (uint32_t)(RC - 1) * 2 * (uint32_t)a.v_stride + 2 * COLS : 0, xo, 0, to + X_AT + 1024 * wave);
+    } else {
 #pragma unroll
-    for (int i = 0; i < NKL; ++i) {
-      rk[i] = *reinterpret_cast<const bf16x8*>(kp + kc + ko[i]);
-      rq[i] = *reinterpret_cast<const bf16x8*>(qp + kc + ko[i]);
+      for (int e = 0; e < 8; ++e) rx[e] = *reinterpret_cast<const bf16*>(xp + xo + 2 * e);
     }
-    const char* m = mp + c * ws_step;
 #pragma unroll
-    for (int i = 0; i < NML; ++i) {
-      rp[i] = *reinterpret_cast<const f32x4*>(m + (uint32_t)(16 * (tid + NT * i)));
-      if constexpr (DELTA) {
-        rt[i] = *reinterpret_cast<const f32x4*>(m + (uint32_t)(4 * RC * RC + 16 * (tid + NT * i)));
-      } else {
-        const uint32_t e = tid + NT * i, hi = vec_at + 4 * (RC + e / (RC / 4)), hj = vec_at + 4 * (RC + 4 * (e % (RC / 4)));
-        rhi[i] = *reinterpret_cast<const float*>(m + hi);
-        rli[i] = *reinterpret_cast<const float*>(m + (hi + 4 * RC));
-        rhj[i] = *reinterpret_cast<const f32x4*>(m + hj);
-        rlj[i] = *reinterpret_cast<const f32x4*>(m + (hj + 4 * RC));
+    for (int i = 0; i < NR; ++i) {
+      buffer_to_lds(kp, more ? kb : 0, ko[i], 0, to + 1024 * (wave + NW * i));
+      buffer_to_lds(qp, more ? kb : 0, ko[i], 0, to + ROWS + 1024 * (wave + NW * i));
+    }
+#pragma unroll
+    for (int i = 0; i < (NH - 1) / NW; ++i)
+      buffer_to_lds(hp, more ? (NH - 1) * 1024 : 0, 16 * lane, 1024 * (wave + NW * i), to + M_AT + 1024 * (wave + NW * i));
+    buffer_to_lds4(hp + (NH - 1) * 1024, more ? 4 * vec_floats<DELTA>() : 0, 4 * tid, to + V_AT + 256 * wave);
+    static_assert(NT * 4 == VECS, "a float a thread");
+    if constexpr (!DELTA) {   // q k^T and its decays go through registers
+#pragma unroll
+      for (int i = 0; i < NML; ++i) {
+        rp[i] = *reinterpret_cast<const f32x4*>(gp + (uint32_t)(16 * (tid + NT * i)));
+        const uint32_t e = tid + NT * i, hi = 4 * (RC + e / (RC / 4)), hj = 4 * (RC + 4 * (e % (RC / 4)));
+        rhi[i] = *reinterpret_cast<const float*>(hp + hi);
+        rli[i] = *reinterpret_cast<const float*>(hp + (hi + 4 * RC));
+        rhj[i] = *reinterpret_cast<const f32x4*>(hp + hj);
+        rlj[i] = *reinterpret_cast<const f32x4*>(hp + (hj + 4 * RC));
       }
     }
-    if (tid < vec_floats<DELTA>() / 4) rvec = *reinterpret_cast<const f32x4*>(m + (vec_at + 16 * tid));
-    const char* v = vp + (int64_t)c * RC * 2 * a.v_stride;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) rv[e] = *reinterpret_cast<const bf16*>(v + vo[e]);
   };
-  auto put = [&](int b) {
+  const auto advance = [&](bool more) {
+    xp += more ? x_step : 0;
+    kp += more ? k_step : 0;
+    qp += more ? k_step : 0;
+    gp += more ? ws_step : 0;
+    hp += more ? ws_step : 0;
+  };
+  const auto put = [&](int b) {   // P_ij = q_i.k_j exp(cum_i - cum_j), j <= i; cum in two parts (long sums, short differences)
+    if constexpr (!VEC) *reinterpret_cast<bf16x8*>(lds + b * IMG + X_AT + 16 * tid) = rx;
+    if constexpr (!DELTA) {
 #pragma unroll
-    for (int i = 0; i < NKL; ++i) {
-      const int e = tid + NT * i, o = img<DK>(e / (DK / 8), e % (DK / 8)) * 8;
-      st8(&sK[b][o], rk[i]);
-      st8(&sQ[b][o], rq[i]);
-    }
+      for (int i = 0; i < NML; ++i) {
+        const int e = tid + NT * i, row = e / (RC / 4), j = 4 * (e % (RC / 4));
+        f32x4 x;
 #pragma unroll
-    for (int i = 0; i < NML; ++i) {
-      const int e = tid + NT * i, row = e / (RC / 4), j = 4 * (e % (RC / 4)), o = row * LDM + j;
-      if constexpr (!DELTA) {   // P_ij = q_i.k_j exp(cum_i - cum_j), j <= i; cum in two parts (long sums, short differences)
+        for (int t = 0; t < 4; ++t) x[t] = j + t <= row ? rp[i][t] * __expf((rhi[i] - rhj[i][t]) + (rli[i] - rlj[i][t])) : 0.f;
+        bf16x8 p[3];
+        split3(x, f32x4{0.f, 0.f, 0.f, 0.f}, p);
+        const int at = b * IMG + M_AT + mat_img(row, (j & 15) >> 2) + 8 * (j >> 4);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const float p = rp[i][t] * __expf((rhi[i] - rhj[i][t]) + (rli[i] - rlj[i][t]));
-          rp[i][t] = j + t <= row ? p : 0.f;
-        }
+        for (int m = 0; m < 3; ++m) *reinterpret_cast<bf16x4*>(lds + at + m * MAT) = bf16x4{p[m][0], p[m][1], p[m][2], p[m][3]};
       }
-      *reinterpret_cast<f32x4*>(&sP[b][o]) = rp[i];
-      if constexpr (DELTA) *reinterpret_cast<f32x4*>(&sT[b][o]) = rt[i];
     }
-    if (tid < vec_floats<DELTA>() / 4) *reinterpret_cast<f32x4*>(&sV[b][4 * tid]) = rvec;
   };
 
   // state: lane (col, g) holds column nc, key channels 32 s + 8 g .. + 7 in blocks 2 s, 2 s + 1
@@ -458,10 +539,10 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   };
   start();
   const float Dh = DELTA ? 0.f : a.D[h];
-  uint32_t oo[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) oo[e] = 2 * ((uint32_t)(16 * (e >> 2) + 4 * g + (e & 3)) * (uint32_t)a.out_stride + (uint32_t)nc);
-  char* op = reinterpret_cast<char*>(a.out + (int64_t)r0 * a.out_stride + (int64_t)h * a.dv);
+  // outputs: lane (col, g) holds rows col and 16 + col, columns n0 + 4 g .. + 3
+  char* op = reinterpret_cast<char*>(a.out + (int64_t)r0 * a.out_stride + (int64_t)h * a.dv + c0);
+  const uint32_t ol = 2 * (16 * wave + 4 * g);
+  const uint32_t oo[2] = {2 * (uint32_t)col * (uint32_t)a.out_stride, 2 * (uint32_t)(16 + col) * (uint32_t)a.out_stride};
 
   // the sequence row by row, as the row-by-row kernels do it (each lane its 8 key channels of every 32)
   const auto walk = [&](int n) {
@@ -515,77 +596,97 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   };
 
   const bool few = r1 - r0 <= FEW;                      // whole block
-  bf16 vc[8];
   if (!few) {
-    offsets(RC);
-    fetch(0);
+    offsets(min(RC, r1 - r0));
+    fetch(RC, true, 0);
+    advance(chunks > 1);
     put(0);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) vc[e] = rv[e];
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
   }
+  // One chunk.  With one or two waves a SIMD nothing else covers an LDS read: each is issued a stage before its use, and the
+  // scheduling barriers keep the compiler from sinking it there.
   const auto step = [&](int c, int b) {
-    if (c + 1 < chunks) fetch(c + 1);
-    const bf16 *K = sK[b], *Q = sQ[b];
-    // ---- k S and q S ----
+    const bool more = c + 1 < chunks;
+    const char* L = lds + b * IMG;
+    const bf16 *K = reinterpret_cast<const bf16*>(L), *Q = reinterpret_cast<const bf16*>(L + ROWS), *X = reinterpret_cast<const bf16*>(L + X_AT);
+    const float* V = reinterpret_cast<const float*>(L + V_AT);
+    const auto vec = [&](int i, int rb) { return *reinterpret_cast<const f32x4*>(V + i * RC + 16 * rb + 4 * g); };
+    const auto mat = [&](int m, int rb) { return *reinterpret_cast<const bf16x8*>(L + M_AT + m * MAT + mat_img(16 * rb + col, g)); };
+    const auto rows = [&](const bf16* R, int rb, int t) { return ld8(R + img<DK>(16 * rb + col, 4 * t + g) * 8); };
+    // ---- first operands; the next chunk's moves ----
+    bf16x4 x[2], y[2];
+    f32x4 va[2], vb[2], vd[2];
+    bf16x8 kf[2][NS], qf[2][NS];
+    const float gc = V[(DELTA ? 4 : 5) * RC];
+#pragma unroll
+    for (int t = 0; t < NS; ++t)
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) (DELTA ? kf : qf)[rb][t] = rows(DELTA ? K : Q, rb, t);
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+      x[rb] = tr4(X, 8 * val_img(16 * rb + 4 * g + (col >> 2), 2 * wave + ((col >> 1) & 1)) + 4 * (col & 1));
+      va[rb] = vec(0, rb);
+      if constexpr (DELTA) vb[rb] = vec(1, rb);
+    }
+    __builtin_amdgcn_sched_barrier(0x0f);
+    fetch(r1 - r0 - (c + 1) * RC, more, b ^ 1);   // (that buffer was read last before the previous barrier)
+    advance(c + 2 < chunks);
+    if constexpr (DELTA) {
+#pragma unroll
+      for (int t = 0; t < NS; ++t)
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb) qf[rb][t] = rows(Q, rb, t);
+    }
+    __builtin_amdgcn_sched_barrier(0x0f);
+    // ---- S in three parts; k S ----
     f32x4 ks[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    bf16x8 part[NS][3];
 #pragma unroll
-    for (int t = 0; t < NS; ++t) {
-      bf16x8 part[3], qa[2], ka[2];
-      split3(S[2 * t], S[2 * t + 1], part);
+    for (int t = 0; t < NS; ++t) {   // (S is scaled first: what a rounding leaves is computed in the place of its value)
+      const f32x4 s0 = S[2 * t], s1 = S[2 * t + 1];
+      S[2 * t] *= gc;
+      S[2 * t + 1] *= gc;
+      split3(s0, s1, part[t]);
+      if constexpr (DELTA) {
 #pragma unroll
-      for (int rb = 0; rb < 2; ++rb) {
-        const int at = img<DK>(16 * rb + col, 4 * t + g) * 8;
-        qa[rb] = ld8(&Q[at]);
-        if constexpr (DELTA) ka[rb] = ld8(&K[at]);
+        for (int p = 2; p >= 0; --p)
+#pragma unroll
+          for (int rb = 0; rb < 2; ++rb) ks[rb] = mma_bf16(kf[rb][t], part[t][p], ks[rb]);
       }
+    }
+    __builtin_amdgcn_sched_barrier(0x0f);
+    // ---- q S (transposed); R (DELTA) / U (Mamba-2) ----
+    bf16x8 tm[2][3], pm[2][3];
+    float vo[2];
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+#pragma unroll
+      for (int p = 0; p < 3; ++p) tm[rb][p] = mat(p, rb);
+      vo[rb] = V[(DELTA ? 2 : 3) * RC + 16 * rb + col];
+      vd[rb] = vec(DELTA ? 3 : 4, rb);
+    }
+    __builtin_amdgcn_sched_barrier(0x0f);
+#pragma unroll
+    for (int t = 0; t < NS; ++t)
 #pragma unroll
       for (int p = 2; p >= 0; --p)
 #pragma unroll
-        for (int rb = 0; rb < 2; ++rb) {
-          if constexpr (DELTA) ks[rb] = mma_bf16(ka[rb], part[p], ks[rb]);
-          o[rb] = mma_bf16(qa[rb], part[p], o[rb]);
-        }
-    }
-    // ---- R (DELTA) / U (Mamba-2) ----
-    f32x4 r[2], u[2];
+        for (int rb = 0; rb < 2; ++rb) o[rb] = mma_bf16(part[t][p], qf[rb][t], o[rb]);
+    f32x4 r[2], u[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
-      const f32x4 va = *reinterpret_cast<const f32x4*>(&sV[b][16 * rb + 4 * g]);
-      const f32x4 vb = *reinterpret_cast<const f32x4*>(&sV[b][RC + 16 * rb + 4 * g]);
-      const f32x4 vg = *reinterpret_cast<const f32x4*>(&sV[b][(DELTA ? 2 : 3) * RC + 16 * rb + 4 * g]);
+    for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float x = (float)vc[4 * rb + e];
-        r[rb][e] = va[e] * x;
-        if constexpr (DELTA) r[rb][e] -= vb[e] * ks[rb][e];
-        o[rb][e] = o[rb][e] * vg[e] + (DELTA ? 0.f : Dh * x);
+        r[rb][e] = va[rb][e] * (float)x[rb][e];
+        if constexpr (DELTA) r[rb][e] -= vb[rb][e] * ks[rb][e];
       }
-      u[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    const float gc = sV[b][(DELTA ? 4 : 5) * RC];
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) S[nb] *= gc;
+    bf16x8 rs[3];
+    split3(r[0], r[1], rs);
+    __builtin_amdgcn_sched_barrier(0x0f);
     // ---- U = T R, o += (P T) R (Mamba-2: o += P U) ----
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      f32x4 pm[2], tm[2];
-#pragma unroll
-      for (int rb = kb; rb < 2; ++rb) {
-        pm[rb] = *reinterpret_cast<const f32x4*>(&sP[b][(16 * rb + col) * LDM + 16 * kb + 4 * g]);
-        if constexpr (DELTA) tm[rb] = *reinterpret_cast<const f32x4*>(&sT[b][(16 * rb + col) * LDM + 16 * kb + 4 * g]);
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int rb = kb; rb < 2; ++rb) {
-          if constexpr (DELTA) u[rb] = mma_f32(tm[rb][e], r[kb][e], u[rb]);
-          o[rb] = mma_f32(pm[rb][e], r[kb][e], o[rb]);
-        }
-    }
-    // ---- S = g_C S + k^T U ----
+    bf16x8 ka[NB];
     {
-      bf16x8 part[3], ka[NB];
       const int qr = 4 * g + (col >> 2), p4 = col & 3;
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
@@ -593,34 +694,53 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
         const bf16x4 lo = tr4(K, img<DK>(qr, ch) * 8 + half), hi = tr4(K, img<DK>(16 + qr, ch) * 8 + half);
         ka[nb] = bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
       }
-#pragma unroll
-      for (int rb = 0; rb < 2; ++rb) {
-        const f32x4 vd = *reinterpret_cast<const f32x4*>(&sV[b][(DELTA ? 3 : 4) * RC + 16 * rb + 4 * g]);
-        u[rb] = (DELTA ? u[rb] : r[rb]) * vd;
-      }
-      split3(u[0], u[1], part);
-#pragma unroll
-      for (int p = 2; p >= 0; --p)
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) S[nb] = mma_bf16(ka[nb], part[p], S[nb]);
     }
-    if (live) {
-      char* oc = op + (int64_t)c * RC * 2 * a.out_stride;
-      const int n = r1 - r0 - c * RC;
-      if (n >= RC) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) *reinterpret_cast<bf16*>(oc + oo[e]) = (bf16)o[e >> 2][e & 3];
+    for (int rb = 0; rb < 2; ++rb) {
+      if constexpr (DELTA) {
+#pragma unroll
+        for (int p = 0; p < 3; ++p) pm[rb][p] = mat(3 + p, rb);
       } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          if (16 * (e >> 2) + 4 * g + (e & 3) < n) *reinterpret_cast<bf16*>(oc + oo[e]) = (bf16)o[e >> 2][e & 3];
+        y[rb] = *reinterpret_cast<const bf16x4*>(X + 8 * val_img(16 * rb + col, 2 * wave + (g >> 1)) + 4 * (g & 1));
       }
     }
-    if (c + 1 < chunks) {
-      put(b ^ 1);   // last read before the previous barrier
+    __builtin_amdgcn_sched_barrier(0x0f);
+    if constexpr (DELTA) mma_parts(tm, rs, u);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) vc[e] = rv[e];
+    for (int rb = 0; rb < 2; ++rb) o[rb] *= vo[rb];
+    mma_parts<true>(DELTA ? pm : tm, rs, o);
+    // ---- S = g_C S + k^T U ----
+    bf16x8 us[3];
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) u[rb] = (DELTA ? u[rb] : r[rb]) * vd[rb];
+    split3(u[0], u[1], us);
+#pragma unroll
+    for (int p = 2; p >= 0; --p)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) S[nb] = mma_bf16(ka[nb], us[p], S[nb]);
+    // ---- the outputs ----
+    if constexpr (!DELTA) {
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) o[rb][t] += Dh * (float)y[rb][t];
     }
+    put(b ^ 1);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next chunk has landed (before the stores below, which nobody waits for)
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+      const bool in = live && 16 * rb + col < r1 - r0 - c * RC;
+      const bf16x4 v = {(bf16)o[rb][0], (bf16)o[rb][1], (bf16)o[rb][2], (bf16)o[rb][3]};
+      if constexpr (VEC) {   // (rows past the end: an offset past the descriptor's, so not stored)
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), __builtin_amdgcn_make_buffer_rsrc(op, 0, 0x7fffffff, 0x00020000),
+                                              in ? oo[rb] + ol : 0x80000000u, 0, 0);
+      } else if (in) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) *reinterpret_cast<bf16*>(op + oo[rb] + ol + 2 * e) = v[e];
+      }
+    }
+    op += o_step;
     __syncthreads();
   };
   for (int c = 0; !few && c < chunks; c += 2) {
@@ -642,18 +762,23 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   }
 }
 
+bool aligned16(const void* p, int64_t elems) { return ((uintptr_t)p | (uintptr_t)(elems * 2)) % 16 == 0; }
+
 template <bool DELTA>
 int launch_rule(const RuleArgs& a, int T, int dk, hipStream_t stream) {
   const dim3 gram(T / RC + a.S, DELTA ? (a.H + 3) / 4 : a.Hk);
   const dim3 rule(a.H, (a.dv + 63) / 64, a.S);
+  const bool vec = aligned16(a.v, a.v_stride) && ((uintptr_t)a.out | (uintptr_t)(2 * a.out_stride)) % 8 == 0;   // (dv is a multiple of 16)
   if (dk == 128) {
     if constexpr (DELTA) chunk_gram_kernel<128><<<gram, 256, 0, stream>>>(a);
     else ssm_gram_kernel<128><<<gram, 256, 0, stream>>>(a);
-    chunk_rule_kernel<128, DELTA, 4><<<rule, 256, 0, stream>>>(a);
+    if (vec) chunk_rule_kernel<128, DELTA, 4, true><<<rule, 256, 0, stream>>>(a);
+    else chunk_rule_kernel<128, DELTA, 4, false><<<rule, 256, 0, stream>>>(a);
   } else {
     if constexpr (DELTA) chunk_gram_kernel<64><<<gram, 256, 0, stream>>>(a);
     else ssm_gram_kernel<64><<<gram, 256, 0, stream>>>(a);
-    chunk_rule_kernel<64, DELTA, 4><<<rule, 256, 0, stream>>>(a);
+    if (vec) chunk_rule_kernel<64, DELTA, 4, true><<<rule, 256, 0, stream>>>(a);
+    else chunk_rule_kernel<64, DELTA, 4, false><<<rule, 256, 0, stream>>>(a);
   }
   OME_CHECK_LAUNCH();
   return 0;
@@ -665,13 +790,11 @@ bool rule_shape(int S, int H, int Hk, int dk, int dv, int64_t s0, int64_t s1, in
          (dv + 63) / 64 <= 65535 && H <= 65535;
 }
 
-bool aligned16(const void* p, int64_t elems) { return ((uintptr_t)p | (uintptr_t)(elems * 2)) % 16 == 0; }
-
 }  // namespace
 
 // fp32 words of workspace of one chunk of H heads (Mamba-2: in G groups); T rows of S sequences have up to T / 32 + S
 OME_API int ome_chunk_rule_floats(int H, int G, int delta) {
-  return (int)(delta ? ws_floats<true>(H, G) : ws_floats<false>(H, G));
+  return (int)((delta ? ws_bytes<true>(H, G) : ws_bytes<false>(H, G)) / 4);
 }
 
 // Gated delta rule over all rows of every sequence; operands as ome_gdn_scan.  -3: a shape, stride or
@@ -684,7 +807,7 @@ OME_API int ome_gdn_chunks(const void* q, const void* k, const void* v, int64_t 
       (uintptr_t)state % 16 || (uintptr_t)ws % 16)
     return -3;
   const RuleArgs r{(const bf16*)q, (const bf16*)k, (const bf16*)v, qkv_stride, qkv_stride, (const bf16*)a, (const bf16*)b,
-                   ab_stride, A_log, nullptr, dt_bias, 0.f, ws, state, (bf16*)out, out_stride, cu, slot, reset, S, Hv, Hk, dv};
+                   ab_stride, A_log, nullptr, dt_bias, 0.f, (char*)ws, state, (bf16*)out, out_stride, cu, slot, reset, S, Hv, Hk, dv};
   return launch_rule<true>(r, T, dk, stream);
 }
 
@@ -697,6 +820,6 @@ OME_API int ome_ssm_chunks(const void* x, int64_t x_stride, const void* dt, int6
       (uintptr_t)state % 16 || (uintptr_t)ws % 16)
     return -3;
   const RuleArgs r{(const bf16*)Cm, (const bf16*)B, (const bf16*)x, bc_stride, x_stride, (const bf16*)dt, nullptr,
-                   dt_stride, A, D, dt_bias, dt_min, ws, state, (bf16*)y, y_stride, cu, slot, reset, S, H, G, P};
+                   dt_stride, A, D, dt_bias, dt_min, (char*)ws, state, (bf16*)y, y_stride, cu, slot, reset, S, H, G, P};
   return launch_rule<false>(r, T, N, stream);
 }

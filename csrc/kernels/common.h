@@ -168,6 +168,35 @@ __device__ __forceinline__ void kv_st1(typename KVStore<F>::T* p, float f) {
   else *p = (uint8_t)(fp8_pack2<F, false>(f, 0.f, 0) & 0xff);
 }
 
+// A wave's move to LDS: 64 lanes x 16 bytes from `off` (per lane) + `add` of the `bytes` at `base` to LDS address `lds` + 16 lane.
+// By asm, because the compiler takes every later LDS read of the target array for a reader of the move and waits for all
+// of it (vmcnt 0) there; the kernels wait themselves, once, before the barrier after which a tile is read.  (No register
+// is written; the descriptor's size bounds the reads, and what lies past it arrives as zeros.)
+__device__ __forceinline__ void buffer_to_lds(const void* base, uint32_t bytes, uint32_t off, uint32_t add, uint32_t lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  const uint64_t b = (uint64_t)base;
+  const u32x4 rs = {(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, bytes, 0x00020000u};
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :
+               : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(off), "s"(rs), "s"(add)
+               : "m0", "memory");
+#endif
+}
+
+// ... and of 64 lanes x 4 bytes
+__device__ __forceinline__ void buffer_to_lds4(const void* base, uint32_t bytes, uint32_t off, uint32_t lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  const uint64_t b = (uint64_t)base;
+  const u32x4 rs = {(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, bytes, 0x00020000u};
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
+               :
+               : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(off), "s"(rs)
+               : "m0", "memory");
+#endif
+}
+
 // XCD-aware remap of a linear workgroup id (bijective for any nwg; T1 of the guide).
 // Blocks b and b+8 share an XCD under round-robin dispatch, so give each XCD group a
 // contiguous chunk of the logical id space.

@@ -205,22 +205,6 @@ __global__ __launch_bounds__(256) void mla_attn_kernel(
   }
 }
 
-// One wave's share of a latent page's move to LDS: 64 lanes x 16 bytes from `off` (per lane) + `add` of the page at `base`
-// to LDS address `lds` + 16 lane.  By asm, because the compiler takes every later LDS read of the image's array for a reader of
-// the move and waits for all of it (vmcnt 0) there; the kernels below wait themselves, once, before the barrier
-// after which a tile is read.  (No register is written; the descriptor's size bounds the reads to the page.)
-__device__ __forceinline__ void page_to_lds(const bf16* base, uint32_t bytes, uint32_t off, uint32_t add, uint32_t lds) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-  const uint64_t b = (uint64_t)base;
-  const u32x4 rs = {(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, bytes, 0x00020000u};
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :
-               : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(off), "s"(rs), "s"(add)
-               : "m0", "memory");
-#endif
-}
-
 // ------------------------------------------------------------------------------------------
 // Row tiles: one workgroup of NW waves owns 32 * NW neighbouring query rows (row = token * H + head) and one
 // split-K partition, so that each latent key tile is streamed and staged in LDS ONCE for all of them: the heads
@@ -467,7 +451,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
         const int i = wave + NW * j;
-        page_to_lds(j < NJ / 2 || (NW == 4 && i < NI / 2) ? b0 : b1, 16 * DK * 2, dofs[j % 9], NW == 1 && j / 9 % 2 ? 8 * CH * 16 : 0,
+        buffer_to_lds(j < NJ / 2 || (NW == 4 && i < NI / 2) ? b0 : b1, 16 * DK * 2, dofs[j % 9], NW == 1 && j / 9 % 2 ? 8 * CH * 16 : 0,
                     lds0 + img * IMG + 64 * 16 * i);
       }
     };

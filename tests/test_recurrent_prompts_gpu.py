@@ -133,6 +133,30 @@ def test_delta_rule_prompts(lens, dk, dv, Hk, Hv, off):
     assert near(ops.gdn_scan(*args, st, *sq, Hv, Hk), st, *want)
 
 
+@pytest.mark.parametrize("delta", [True, False])
+@pytest.mark.parametrize("dv,shift,gap", [(128, 1, 0), (16, 8, 4), (80, 0, 2), (48, 0, 1), (64, 8, 0)])
+def test_chunked_scans_of_values_and_outputs_of_any_alignment(dv, shift, gap, delta):
+    """Keys and queries that the chunks take, values ``shift`` columns and outputs ``gap`` columns further in their rows: pieces of
+    16 and 8 bytes where both are aligned for them, single values elsewhere; columns that fill no block of 64."""
+    torch.manual_seed(dv + shift)
+    lens, H, dk = [40, 0, 7, 65], 2, 128
+    T, kd, sq = sum(lens), H * dk, seqs(lens, 71)
+    c, ab = torch.randn(T, 2 * kd + H * dv + 16, device=DEV).to(BF), torch.randn(T, 2 * H, device=DEV).to(BF)
+    q, k, v = c[:, :kd], c[:, kd:2 * kd], c[:, 2 * kd + shift:2 * kd + shift + H * dv]
+    out = torch.full((T, H * dv + 2 * gap), 7.0, device=DEV).to(BF)
+    o, st, bias = out[:, gap:gap + H * dv], torch.randn(71, H, dv, dk, device=DEV) * 0.2, torch.randn(H, device=DEV)
+    if delta:
+        args = (q, k, v, ab[:, :H], ab[:, H:], torch.linspace(-3, 2, H, device=DEV), bias)
+        want = exact_gdn(*args, st, *sq, H, H)
+        ops.gdn_scan(*args, st, *sq, H, H, out=o)
+    else:
+        args = (v, ab[:, :H], k, q, -torch.logspace(-1, 1, H, device=DEV), torch.randn(H, device=DEV), bias, 0.001)
+        want = exact_ssm(*args, st, *sq, H, dv, dk, H)
+        ops.ssm_scan(*args, st, *sq, H, dv, dk, H, out=o)
+    assert near(o, st, *want)
+    assert bool((out[:, :gap] == 7).all()) and bool((out[:, gap + H * dv:] == 7).all())
+
+
 @pytest.mark.parametrize("lens", [[1], [1] * 5, [1, 0, 2, 1], [1] * 70], ids=str)
 @pytest.mark.parametrize("dk,dv,Hk,Hv,off", [(128, 128, 2, 4, 8), (64, 16, 1, 5, 0), (256, 40, 3, 3, 8), (128, 33, 1, 2, 8),
                                              (64, 128, 2, 2, 1)])
