@@ -7,9 +7,9 @@
 //                     device (graph-capturable: no host sync on the per-expert counts).
 //   ome_moe_gemm    : grouped GEMM  out[p, :] = A[row(p), :] @ W[e(p)]^T  over the sorted
 //                     assignments p; A rows are gathered through sorted_ids / k (gate_up) or
-//                     read in sorted order (down).  64x64 MFMA tiles, tiles of an expert never
-//                     straddle experts; each workgroup finds its (expert, m-tile) by scanning
-//                     the offsets, so the grid is a static upper bound.
+//                     read in sorted order (down).  Tiles never straddle experts; each workgroup finds its
+//                     (expert, m-tile) by scanning the offsets, so the grid is a static upper bound.
+//   ome_moe_gemm_stream : the same for experts with few rows, on tiles listed by ome_moe_align_tiles
 //   ome_moe_combine : out[t] = sum_j w[t, j] * Y[inv[t*k + j]]   (fp32 accumulate)
 #include "common.h"
 
@@ -230,7 +230,8 @@ OME_API int ome_moe_route(const void* logits, int is_bf16, int64_t stride, int n
 // ------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__ topk_ids, int n, int E,
                                                          int* __restrict__ offsets, int* __restrict__ sorted_ids,
-                                                         int* __restrict__ inv) {
+                                                         int* __restrict__ inv, int4* __restrict__ tiles, int bm, int e_tiles,
+                                                         int max_tiles) {
   extern __shared__ int sh[];  // [E] counts then [E] cursors
   int* cnt = sh;
   int* cur = sh + E;
@@ -241,28 +242,49 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
   __syncthreads();
   // exclusive prefix sums: a thread's run of experts, its wave, the waves before (one thread summing 512 experts
   // through LDS took 15 of the kernel's 20 us)
-  __shared__ int s_wave[16];
+  __shared__ int s_wave[16], s_tiles[16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, per = (E + 1023) / 1024, e0 = threadIdx.x * per;
-  int own = 0;
+  int own = 0, own_t = 0;
   for (int i = 0; i < per; ++i)
-    if (e0 + i < E) own += cnt[e0 + i];
-  int incl = own;
+    if (e0 + i < E) {
+      own += cnt[e0 + i];
+      own_t += e0 + i < e_tiles ? (cnt[e0 + i] + bm - 1) / bm : 0;
+    }
+  int incl = own, incl_t = own_t;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
-    const int up = __shfl_up(incl, d);
-    if (lane >= d) incl += up;
+    const int up = __shfl_up(incl, d), up_t = __shfl_up(incl_t, d);
+    if (lane >= d) {
+      incl += up;
+      incl_t += up_t;
+    }
   }
-  if (lane == 63) s_wave[wave] = incl;
+  if (lane == 63) {
+    s_wave[wave] = incl;
+    s_tiles[wave] = incl_t;
+  }
   __syncthreads();
-  int acc = incl - own;
-  for (int w = 0; w < wave; ++w) acc += s_wave[w];
+  int acc = incl - own, t = incl_t - own_t;
+  for (int w = 0; w < wave; ++w) {
+    acc += s_wave[w];
+    t += s_tiles[w];
+  }
   for (int i = 0; i < per; ++i)
     if (e0 + i < E) {
       offsets[e0 + i] = acc;
       cur[e0 + i] = acc;
-      acc += cnt[e0 + i];
+      const int end = acc + cnt[e0 + i];
+      if (e0 + i < e_tiles)
+        for (int m = acc; m < end; m += bm, ++t)
+          if (t < max_tiles) tiles[t] = int4{e0 + i, m, end, 0};
+      acc = end;
     }
   if (threadIdx.x == 1023) offsets[E] = acc;   // (its run is the last, or empty: the total)
+  if (tiles != nullptr) {   // the rest have no expert
+    int all = 0;
+    for (int w = 0; w < 16; ++w) all += s_tiles[w];
+    for (int i = all + threadIdx.x; i < max_tiles; i += blockDim.x) tiles[i] = int4{-1, 0, 0, 0};
+  }
   __syncthreads();
   // stable within an expert is not required (the combine uses the inverse map)
   for (int i = threadIdx.x; i < n; i += blockDim.x) {
@@ -277,7 +299,19 @@ OME_API int ome_moe_align(const int* topk_ids, int n, int E, int* offsets, int* 
   if (n <= 0) {
     return hipMemsetAsync(offsets, 0, (E + 1) * sizeof(int), stream);
   }
-  moe_align_kernel<<<1, 1024, 2 * E * sizeof(int), stream>>>(topk_ids, n, E, offsets, sorted_ids, inv);
+  moe_align_kernel<<<1, 1024, 2 * E * sizeof(int), stream>>>(topk_ids, n, E, offsets, sorted_ids, inv, nullptr, 1, 0, 0);
+  OME_CHECK_LAUNCH();
+  return 0;
+}
+
+// ... and the tiles of `bm` rows of one expert each, of experts below `e_tiles`, (expert, first row, the expert's end, 0), 16-byte aligned: a workgroup of the
+// kernels below reads its own instead of searching the offsets (512 experts: eight rounds of a wave's prefix sum, 2 us a
+// workgroup).  max_tiles >= min(n, E) + n / bm bounds their number; entries past it have expert -1.
+OME_API int ome_moe_align_tiles(const int* topk_ids, int n, int E, int* offsets, int* sorted_ids, int* inv, int* tiles, int bm,
+                                int e_tiles, int max_tiles, hipStream_t stream) {
+  if (n <= 0 || bm <= 0 || max_tiles < (n < E ? n : E) + n / bm || (uintptr_t)tiles % 16) return -2;
+  moe_align_kernel<<<1, 1024, 2 * E * sizeof(int), stream>>>(topk_ids, n, E, offsets, sorted_ids, inv, (int4*)tiles, bm, e_tiles,
+                                                               max_tiles);
   OME_CHECK_LAUNCH();
   return 0;
 }
@@ -384,11 +418,9 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(const bf16* __restrict__ 
 }
 
 // ------------------------------------------------------------------------------------------
-// grouped GEMM v2: the same 64x64 tile / 2x2-wave layout, but a BK = 64 or 128 k-step staged
-// through DOUBLE-buffered LDS: the next step's global loads are issued before this step's MFMAs
-// and written to the other buffer after them, so one barrier per k-step (v1: two per 32) and
-// BK/32 x 16 B of W + A in flight per thread.  Decode-time MoE GEMMs are weight-streaming
-// (tens of rows per expert), so this is a bandwidth kernel: the win is bytes in flight.
+// grouped GEMM v2: 128 x 128 tiles, 2x2 waves, a BK k-step staged through DOUBLE-buffered LDS: the next step's global
+// loads are issued before this step's MFMAs and written to the other buffer after them, so one barrier per k-step.  Some 60 rows
+// per expert and more (fewer: moe_stream_kernel; 80 and more, and shapes that its tiles take: gemm_pp.hip).
 // ------------------------------------------------------------------------------------------
 template <int BM, int BN, int BK>
 __global__ __launch_bounds__(256) void moe_gemm_v2_kernel(const bf16* __restrict__ A, int64_t lda,
@@ -512,36 +544,162 @@ __global__ __launch_bounds__(256) void moe_gemm_v2_kernel(const bf16* __restrict
       }
 }
 
-static int moe_gemm_variant() {
-  const char* s = getenv("OME_MOE_GEMM");  // 1 = v1 (64x64, BK 32, single buffer); default v2
-  return s ? atoi(s) : 2;
+
+// ------------------------------------------------------------------------------------------
+// bf16 experts with few rows each: out[p, :] = A[row(p)] . W[e(p)]^T (+ bias) over 64-row tiles, one workgroup per tile and 64 weight
+// rows.  Bound by the weights' way from memory: three (few workgroups: four) stages of 64 k move to LDS by DMA, counted, so that
+// two stay out across the barrier; the weights are asked for before the rows' numbers are known; a workgroup reads its
+// tile instead of searching it.  A wave without rows of its own only moves.
+// 128 weight rows a workgroup: half as many and twice as long, 3 to 5% slower with 2048 or fewer k and 1 to 3% faster with 2688.
+// Whole layer, us (register-staged 64 x 64 tiles with the search -> this): 512 experts top 10 of 2048 x 512, 1 / 48 / 1000 rows 110 ->
+// 67, 430 -> 330 (5.9 TB/s), 780 -> 645; 8 experts top 2 of 4096 x 14336, 1 / 8 / 136 rows 281 -> 182, 465 -> 398 (6.4 TB/s), 673 ->
+// 569; 128 experts top 6 of 2688 x 1856, 7 / 70 / 600 rows 145 -> 139, 335 -> 308, 491 -> 490.
+// ------------------------------------------------------------------------------------------
+typedef __attribute__((address_space(3))) void moe_lds_t;
+typedef __attribute__((address_space(1))) void moe_glb_t;
+
+// 16-byte piece `chunk` of a 128-byte row in LDS: 16 rows' pieces in all banks
+__device__ __forceinline__ int mswz(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
+
+template <int BM, int BN, int NST, int WM>
+__global__ __launch_bounds__(256) void moe_stream_kernel(const bf16* __restrict__ A, int64_t lda, const int* __restrict__ sorted_ids,
+                                                         int gather_div, const bf16* __restrict__ W, const int4* __restrict__ tiles,
+                                                         int N, int K, bf16* __restrict__ out, int64_t ldo,
+                                                         const bf16* __restrict__ bias) {
+  constexpr int AB = BM * 128, STG = AB + BN * 128;             // a stage: 64 k of BM rows and of BN weight rows
+  constexpr int WN = 4 / WM, MJ = BM / 16 / WM, NI = BN / 16 / WN;   // waves, 16 x 16 blocks of a wave
+  constexpr int AI = BM / 32, WI = BN / 32;                     // moves of 8 rows of a wave
+  __shared__ __attribute__((aligned(16))) char smem[NST * STG];
+  const int4 tile = tiles[blockIdx.y];
+  const int e = tile.x, m0 = tile.y, m_end = tile.z, n0 = blockIdx.x * BN, nt = K / 64;
+  if (e < 0) return;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  int srow[AI];
+#pragma unroll
+  for (int j = 0; j < AI; ++j) {
+    const int p = min(m0 + (wave * AI + j) * 8 + (lane >> 3), m_end - 1);
+    srow[j] = gather_div > 0 ? sorted_ids[p] : p;
+  }
+  const bf16* We = W + (int64_t)e * N * K;
+  const bf16 *asrc[AI], *wsrc[WI];
+#pragma unroll
+  for (int j = 0; j < WI; ++j) {
+    const int r = (wave * WI + j) * 8 + (lane >> 3);
+    wsrc[j] = We + (int64_t)min(n0 + r, N - 1) * K + mswz(r, lane & 7) * 8;
+  }
+  const auto stage_w = [&](int buf, int kt) {
+#pragma unroll
+    for (int j = 0; j < WI; ++j)
+      __builtin_amdgcn_global_load_lds((moe_glb_t*)(wsrc[j] + kt * 64), (moe_lds_t*)(smem + buf * STG + AB + (wave * WI + j) * 1024), 16, 0, 0);
+  };
+  const auto stage_a = [&](int buf, int kt) {
+#pragma unroll
+    for (int j = 0; j < AI; ++j)
+      __builtin_amdgcn_global_load_lds((moe_glb_t*)(asrc[j] + kt * 64), (moe_lds_t*)(smem + buf * STG + (wave * AI + j) * 1024), 16, 0, 0);
+  };
+  // the weights do not wait for the rows' numbers
+#pragma unroll
+  for (int b = 0; b < NST - 1; ++b) stage_w(b, min(b, nt - 1));
+#pragma unroll
+  for (int j = 0; j < AI; ++j) {
+    const int r = (wave * AI + j) * 8 + (lane >> 3);
+    asrc[j] = A + (int64_t)(gather_div > 0 ? srow[j] / gather_div : srow[j]) * lda + mswz(r, lane & 7) * 8;
+  }
+#pragma unroll
+  for (int b = 0; b < NST - 1; ++b) stage_a(b, min(b, nt - 1));
+  const int wm = wave / WN, wn = wave % WN, fr = lane & 15, fc = lane >> 4;
+  const bool works = __builtin_amdgcn_readfirstlane(m0 + wm * MJ * 16 < m_end);   // a wave without rows only moves
+  f32x4 acc[NI][MJ];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < MJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AI * (NST - 2)) : "memory");   // block 0 (all weights are ahead of its rows)
+  int cur = 0;
+  for (int t = 0; t < nt; ++t) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AI + WI) * (NST - 2)) : "memory");   // block t; the next ones (maybe clamped copies) stay out
+    __builtin_amdgcn_s_barrier();   // every wave's block t landed; every wave done reading block t - 1
+    // (branch-free: clamped to the last block past the end, so that the counted wait stays exact)
+    stage_w(cur == 0 ? NST - 1 : cur - 1, min(t + NST - 1, nt - 1));
+    stage_a(cur == 0 ? NST - 1 : cur - 1, min(t + NST - 1, nt - 1));
+    const char *la = smem + cur * STG, *lw = la + AB;
+    if (works) {
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        bf16x8 xa[MJ];
+#pragma unroll
+        for (int j = 0; j < MJ; ++j) {
+          const int r = (wm * MJ + j) * 16 + fr;
+          xa[j] = *reinterpret_cast<const bf16x8*>(la + r * 128 + mswz(r, 4 * kk + fc) * 16);
+        }
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          const int r = (wn * NI + i) * 16 + fr;
+          const bf16x8 wf = *reinterpret_cast<const bf16x8*>(lw + r * 128 + mswz(r, 4 * kk + fc) * 16);
+#pragma unroll
+          for (int j = 0; j < MJ; ++j) acc[i][j] = mfma16(wf, xa[j], acc[i][j]);
+        }
+      }
+    }
+    cur = cur == NST - 1 ? 0 : cur + 1;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // clamped tail moves retire before exit
+#pragma unroll
+  for (int j = 0; j < MJ; ++j) {
+    const int p = m0 + (wm * MJ + j) * 16 + fr;
+    if (p >= m_end) continue;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int n = n0 + (wn * NI + i) * 16 + 4 * fc;
+      f32x4 v = acc[i][j];
+      if (bias != nullptr)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] += (float)bias[(int64_t)e * N + min(n + r, N - 1)];
+      if (N % 4 == 0 && ldo % 4 == 0) {
+        if (n < N) *reinterpret_cast<bf16x4*>(out + (int64_t)p * ldo + n) = bf16x4{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (n + r < N) out[(int64_t)p * ldo + n + r] = (bf16)v[r];
+      }
+    }
+  }
+}
+
+// tiles: of 64 rows (ome_moe_align_tiles); A, W 16-byte aligned, lda % 8 == 0, K % 64 == 0
+OME_API int ome_moe_gemm_stream(const void* A, int64_t lda, const int* sorted_ids, int gather_div, const void* W, const int* tiles,
+                                int N, int K, int max_tiles, void* out, int64_t ldo, const void* bias, hipStream_t stream) {
+  if (max_tiles <= 0) return 0;
+  if (N <= 0 || K <= 0 || K % 64 || lda % 8 || ((uintptr_t)A | (uintptr_t)W | (uintptr_t)tiles) % 16 || (uintptr_t)out % 8) return -2;
+  if (max_tiles > 65535) return -3;
+  const dim3 grid((N + 63) / 64, max_tiles);
+  // up to two workgroups a CU: one stage more out (8 experts, 1 row: 201 -> 182 us; more of them: 398 -> 413 at 8 rows, three fit a CU)
+#define ST(NST) moe_stream_kernel<64, 64, NST, 2><<<grid, 256, 0, stream>>>((const bf16*)A, lda, sorted_ids, gather_div, (const bf16*)W, \
+    (const int4*)tiles, N, K, (bf16*)out, ldo, (const bf16*)bias)
+  if ((int64_t)grid.x * max_tiles <= 512) ST(4);
+  else ST(3);
+#undef ST
+  OME_CHECK_LAUNCH();
+  return 0;
 }
 
 // bias: optional per-expert bias [E, N] added in the epilogue.  tile_m 128: the 128x128 prefill
-// tile (max_m_tiles must then count 128-row tiles); otherwise the 64x64 decode tile.
+// tile (max_m_tiles must then count 128-row tiles); otherwise the 64x64 one (any K % 32).
 OME_API int ome_moe_gemm(const void* A, int64_t lda, const int* sorted_ids, int gather_div, const void* W,
                          const int* offsets, int E, int N, int K, int max_m_tiles, void* out, int64_t ldo,
                          const void* bias, int tile_m, hipStream_t stream) {
   if (max_m_tiles <= 0) return 0;
   if (K % GBK != 0 || lda % 8 != 0) return -2;
   if (max_m_tiles > 65535) return -3;
-  const int v = moe_gemm_variant();
-  if (tile_m == 128 && v != 1) {
+  if (tile_m == 128) {
     dim3 grid((N + 127) / 128, max_m_tiles);
     moe_gemm_v2_kernel<128, 128, 32><<<grid, 256, 0, stream>>>((const bf16*)A, lda, sorted_ids, gather_div,
                                                                (const bf16*)W, offsets, E, N, K, (bf16*)out, ldo,
                                                                (const bf16*)bias);
   } else {
-    if (tile_m == 128) return -4;  // the v1 kernel only has the 64-row tile
     dim3 grid((N + GBN - 1) / GBN, max_m_tiles);
-    if (v != 1 && K % 64 == 0) {
-      moe_gemm_v2_kernel<64, 64, 64><<<grid, 256, 0, stream>>>((const bf16*)A, lda, sorted_ids, gather_div,
-                                                               (const bf16*)W, offsets, E, N, K, (bf16*)out, ldo,
-                                                               (const bf16*)bias);
-    } else {
-      moe_gemm_kernel<<<grid, 256, 0, stream>>>((const bf16*)A, lda, sorted_ids, gather_div, (const bf16*)W, offsets,
-                                                E, N, K, (bf16*)out, ldo, (const bf16*)bias);
-    }
+    moe_gemm_kernel<<<grid, 256, 0, stream>>>((const bf16*)A, lda, sorted_ids, gather_div, (const bf16*)W, offsets, E, N, K,
+                                              (bf16*)out, ldo, (const bf16*)bias);
   }
   OME_CHECK_LAUNCH();
   return 0;
@@ -602,12 +760,8 @@ OME_API int ome_moe_combine(const void* Y, const float* w, const int* inv, int n
 // Operands go global -> LDS by global_load_lds (per-lane gathered source rows, lane-linear
 // destination, XOR-swizzled chunks), double buffered.
 // ------------------------------------------------------------------------------------------
-typedef __attribute__((address_space(3))) void moe_lds_t;
-typedef __attribute__((address_space(1))) void moe_glb_t;
 typedef int mi32x8 __attribute__((ext_vector_type(8)));
 typedef int mi32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ int mswz(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
 
 __device__ __forceinline__ mi32x8 mfrag32(const char* lds, int row, int c) {
   const mi32x4 lo = *reinterpret_cast<const mi32x4*>(lds + row * 128 + mswz(row, 2 * c) * 16);
@@ -624,44 +778,18 @@ template <int BMF, int BNF, int NST = 2>
 __global__ __launch_bounds__(256) void moe_gemm_fp8_kernel(const uint8_t* __restrict__ A, int64_t lda,
                                                            const float* __restrict__ sa, const int* __restrict__ sorted_ids,
                                                            int gather_div, const uint8_t* __restrict__ W,
-                                                           const float* __restrict__ sw, const int* __restrict__ offsets,
-                                                           int E, int N, int K, bf16* __restrict__ out, int64_t ldo) {
+                                                           const float* __restrict__ sw, const int4* __restrict__ tiles,
+                                                           int N, int K, bf16* __restrict__ out, int64_t ldo) {
   constexpr int ABYTES = BMF * 128, WBYTES = BNF * 128;
   static_assert(NST == 2 || NST == 3, "NST");
   // NST == 3 stages also carry the K block's A-row scales (4 x 256 B, one 4-byte DMA per wave):
   // an ordinary VGPR load beside the DMA makes hipcc wait vmcnt(0) and drain the ring
   constexpr int SCB = NST == 3 ? 1024 : 0, STG = ABYTES + WBYTES + SCB;
-  __shared__ __attribute__((aligned(16))) char smem[NST * STG + 16];
-  int* s_tile = reinterpret_cast<int*>(smem + NST * STG);
+  __shared__ __attribute__((aligned(16))) char smem[NST * STG];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  if (tid == 0) s_tile[0] = -1;
-  __syncthreads();
-  if (wave == 0) {   // (expert, first row) of this m-tile: prefix sum of per-expert tile counts
-    int base = 0;
-    const int y = blockIdx.y;
-    for (int e0 = 0; e0 < E; e0 += 64) {
-      const int e = e0 + lane;
-      const int nt = e < E ? (offsets[e + 1] - offsets[e] + BMF - 1) / BMF : 0;
-      int incl = nt;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int v = __shfl_up(incl, d);
-        if (lane >= d) incl += v;
-      }
-      const int t = y - base;
-      if (t >= incl - nt && t < incl) {
-        s_tile[0] = e;
-        s_tile[1] = offsets[e] + (t - (incl - nt)) * BMF;
-        s_tile[2] = offsets[e + 1];
-      }
-      base += __shfl(incl, 63);
-      if (y < base) break;
-    }
-  }
-  __syncthreads();
-  const int e = s_tile[0];
+  const int4 tile = tiles[blockIdx.y];
+  const int e = tile.x, m0 = tile.y, m_end = tile.z;
   if (e < 0) return;
-  const int m0 = s_tile[1], m_end = s_tile[2];
   const int n0 = blockIdx.x * BNF;
   const int KB = K / 128, nt = KB;
   const uint8_t* We = W + (int64_t)e * N * K;
@@ -818,12 +946,12 @@ __global__ __launch_bounds__(256) void moe_gemm_fp8_kernel(const uint8_t* __rest
 // bm = 64: 64 x 128 tiles (decode: a few rows per expert, more workgroups per weight byte);
 // bm = 128: 128 x 128 tiles, 64 x 64 per wave (prefill: twice the MFMAs per staged K block and the
 // expert's weights read once per 128 gathered rows; 64 KB of LDS, 2 workgroups per CU).
-// max_m_tiles: static upper bound of bm-row tiles (n_assign / bm + E).
+// tiles: of bm rows (ome_moe_align_tiles), max_m_tiles of them.
 OME_API int ome_moe_gemm_fp8_tile(const void* A, int64_t lda, const float* sa, const int* sorted_ids, int gather_div,
-                                  const void* W, const float* sw, const int* offsets, int E, int N, int K,
+                                  const void* W, const float* sw, const int* tiles, int N, int K,
                                   int max_m_tiles, int bm, void* out, int64_t ldo, hipStream_t stream) {
   if (max_m_tiles <= 0) return 0;
-  if (N % 128 || K % 128 || lda % 16 || ((uintptr_t)A | (uintptr_t)W) % 16) return -2;
+  if (N % 128 || K % 128 || lda % 16 || ((uintptr_t)A | (uintptr_t)W | (uintptr_t)tiles) % 16) return -2;
   if (max_m_tiles > 65535) return -3;
   // LDS stages (OME_MOE_FP8_NST): 3 for the 64-row tile (2 workgroups / CU, 2-5 % faster at
   // prefill sizes), 2 for the 128-row tile (3 stages = 96 KB would leave one workgroup per CU);
@@ -832,7 +960,7 @@ OME_API int ome_moe_gemm_fp8_tile(const void* A, int64_t lda, const float* sa, c
   const int nst = nst_env ? nst_env : (bm == 64 ? 3 : 2);
 #define MOE_FP8(BM, NS)                                                                                          \
   moe_gemm_fp8_kernel<BM, 128, NS><<<dim3(N / 128, max_m_tiles), 256, 0, stream>>>(                               \
-      (const uint8_t*)A, lda, sa, sorted_ids, gather_div, (const uint8_t*)W, sw, offsets, E, N, K, (bf16*)out, ldo)
+      (const uint8_t*)A, lda, sa, sorted_ids, gather_div, (const uint8_t*)W, sw, (const int4*)tiles, N, K, (bf16*)out, ldo)
   if (bm == 128) {
     if (nst == 3) MOE_FP8(128, 3); else MOE_FP8(128, 2);
   } else if (bm == 64) {
@@ -843,11 +971,4 @@ OME_API int ome_moe_gemm_fp8_tile(const void* A, int64_t lda, const float* sa, c
 #undef MOE_FP8
   OME_CHECK_LAUNCH();
   return 0;
-}
-
-OME_API int ome_moe_gemm_fp8(const void* A, int64_t lda, const float* sa, const int* sorted_ids, int gather_div,
-                             const void* W, const float* sw, const int* offsets, int E, int N, int K,
-                             int max_m_tiles, void* out, int64_t ldo, hipStream_t stream) {
-  return ome_moe_gemm_fp8_tile(A, lda, sa, sorted_ids, gather_div, W, sw, offsets, E, N, K, max_m_tiles, 64, out, ldo,
-                               stream);
 }

@@ -718,16 +718,15 @@ def moe_route(logits: torch.Tensor, k: int, renorm: bool = True, scoring: str = 
 
 
 def moe_tile_m(rows: int, E: int, N: int) -> int:
-    """Row tile of the grouped GEMM (static in the shapes, so graph-safe): 128x128 when experts
-    get many rows (prefill: MFMA-bound), or in the decode regime when the wide-N GEMM still gives
-    >= 1024 workgroups of 128 (more W bytes per barrier); else the 64x64 weight-streaming tile.
-    Measured on gfx950: ``scripts/moe_gemm_bench.py`` (profiles/r01_moe_gemm_bench.txt).
-    ``OME_MOE_TILE`` overrides."""
+    """Row tile of the grouped GEMM (static in the shapes, so graph-safe): 128 x 128 when experts get many rows (prefill:
+    MFMA-bound), or some 60 with >= 1024 workgroups of 128; else the 64-row tiles that stream the weights.  Whole layer, 64-row /
+    128-row tiles: Mixtral 55 rows an expert 689 / 713 us, 65 770 / 722; Qwen3-Next 49 802 / 887, 59 855 / 928;
+    Nemotron-3-Nano 61 661 / 645.  ``OME_MOE_TILE`` overrides."""
     env = os.environ.get("OME_MOE_TILE")
     if env:
         return int(env)
     avg = rows / max(1, E)
-    if avg >= 128 or (avg >= 48 and -(-N // 128) * E >= 1024):
+    if avg >= 128 or (avg >= 60 and -(-N // 128) * E >= 1024):
         return 128
     return 64
 
@@ -738,7 +737,27 @@ def moe_tile_m(rows: int, E: int, N: int) -> int:
 MOE_PP_ROWS = 80
 
 
-def _moe_pp(x: torch.Tensor, ids: torch.Tensor | None, div: int, w: torch.Tensor, offsets: torch.Tensor, rows: int,
+class _Sorted:
+    """Assignments sorted by expert (``ome_moe_align``) in one buffer: pointers to the experts' offsets [E + 1], the sorted
+    assignments [n], their inverse (also as a tensor) and, with ``bm``, the tiles of ``bm`` rows of the experts below
+    ``e_tiles`` (at most ``max_tiles``: an expert with rows has one more than its whole tiles)."""
+
+    def __init__(self, ids: torch.Tensor, E: int, bm: int = 0, e_tiles: int | None = None):
+        n = ids.numel()
+        self.max_tiles = min(n, E) + n // bm if bm else 0
+        m = self.meta = torch.empty(4 * self.max_tiles + E + 1 + 2 * n, dtype=torch.int32, device=ids.device)
+        self.inv = m[m.numel() - n:]
+        self.tiles = m.data_ptr()
+        self.offsets = self.tiles + 16 * self.max_tiles
+        self.ids = self.offsets + 4 * (E + 1)
+        if bm and n:
+            call("ome_moe_align_tiles", ids.data_ptr(), n, E, self.offsets, self.ids, self.ids + 4 * n, self.tiles, bm,
+                 E if e_tiles is None else e_tiles, self.max_tiles, stream_ptr())
+        else:
+            call("ome_moe_align", ids.data_ptr(), n, E, self.offsets, self.ids, self.ids + 4 * n, stream_ptr())
+
+
+def _moe_pp(x: torch.Tensor, ids: int | None, div: int, w: torch.Tensor, offsets: int, rows: int,
             bias: torch.Tensor | None, silu: bool) -> torch.Tensor | None:
     """Grouped GEMM on 256-row tiles (``ome_moe_gemm_pp``; ``silu``: SiLU(gate) * up applied to the accumulators),
     or None where the 64 / 128-row tiles run: experts with few rows, shapes the tiles do not take, ``OME_MOE_TILE``."""
@@ -748,7 +767,7 @@ def _moe_pp(x: torch.Tensor, ids: torch.Tensor | None, div: int, w: torch.Tensor
             x.shape[0] * x.stride(0) >= 1 << 30 or N * K >= 1 << 30:
         return None
     out = torch.empty(rows, N // 2 if silu else N, dtype=x.dtype, device=x.device)
-    call("ome_moe_gemm_pp", x.data_ptr(), x.stride(0), x.shape[0], ptr(ids), div, w.data_ptr(), offsets.data_ptr(), E, N, K,
+    call("ome_moe_gemm_pp", x.data_ptr(), x.stride(0), x.shape[0], ids, div, w.data_ptr(), offsets, E, N, K,
          rows, out.data_ptr(), out.stride(0), ptr(bias), 2 if silu else 0, stream_ptr())
     return out
 
@@ -786,28 +805,34 @@ def fused_moe(x: torch.Tensor, topk_w: torch.Tensor, topk_ids: torch.Tensor, w13
     k = topk_ids.shape[1]
     n = T * k
     dev = x.device
-    offsets = torch.empty(E + 1, dtype=torch.int32, device=dev)
-    sorted_ids = torch.empty(n, dtype=torch.int32, device=dev)
-    inv = torch.empty(n, dtype=torch.int32, device=dev)
-    call("ome_moe_align", topk_ids.data_ptr(), n, E, offsets.data_ptr(), sorted_ids.data_ptr(), inv.data_ptr(),
-         stream_ptr())
+    s = _Sorted(topk_ids, E, 64)
     fused = gated and act == 0 and b13 is None
-    h = _moe_pp(x, sorted_ids, k, w13, offsets, n, b13, fused)
+    h = _moe_pp(x, s.ids, k, w13, s.offsets, n, b13, fused)
     if h is None:
         fused = False
-        tm = moe_tile_m(n, E, I2)
-        h = torch.empty(n, I2, dtype=x.dtype, device=dev)
-        call("ome_moe_gemm", x.data_ptr(), x.stride(0), sorted_ids.data_ptr(), k, w13.data_ptr(), offsets.data_ptr(),
-             E, I2, H, -(-n // tm) + E, h.data_ptr(), h.stride(0), ptr(b13), tm, stream_ptr())
+        h = _moe_gemm(x, s, s.ids, k, w13, n, b13)
     if not fused:
         h = act_and_mul(h, act, limit=limit) if gated else _act_inplace(h, act)
-    y = _moe_pp(h, None, 1, w2, offsets, n, b2, False)
+    y = _moe_pp(h, None, 1, w2, s.offsets, n, b2, False)
     if y is None:
-        y = torch.empty(n, H, dtype=x.dtype, device=dev)
-        tm = moe_tile_m(n, E, H)
-        call("ome_moe_gemm", h.data_ptr(), h.stride(0), None, 0, w2.data_ptr(), offsets.data_ptr(), E, H, I,
-             -(-n // tm) + E, y.data_ptr(), y.stride(0), ptr(b2), tm, stream_ptr())
-    return _combine(y, topk_w, inv, T, k, H, scale, add)
+        y = _moe_gemm(h, s, None, 0, w2, n, b2)
+    return _combine(y, topk_w, s.inv, T, k, H, scale, add)
+
+
+def _moe_gemm(x: torch.Tensor, s: _Sorted, ids: int | None, div: int, w: torch.Tensor, rows: int, bias: torch.Tensor | None,
+              E: int | None = None) -> torch.Tensor:
+    """Grouped GEMM of the first E experts on 64- or 128-row tiles (:func:`moe_tile_m`)."""
+    N, K = w.shape[1:]
+    E = E or w.shape[0]
+    out = torch.empty(rows, N, dtype=x.dtype, device=x.device)
+    tm = moe_tile_m(rows, E, N)
+    if tm == 64 and K % 64 == 0 and x.stride(0) % 8 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0:
+        call("ome_moe_gemm_stream", x.data_ptr(), x.stride(0), ids, div, w.data_ptr(), s.tiles, N, K, s.max_tiles,
+             out.data_ptr(), out.stride(0), ptr(bias), stream_ptr())
+    else:
+        call("ome_moe_gemm", x.data_ptr(), x.stride(0), ids, div, w.data_ptr(), s.offsets, E, N, K, -(-rows // tm) + E,
+             out.data_ptr(), out.stride(0), ptr(bias), tm, stream_ptr())
+    return out
 
 
 def _combine(y, topk_w, inv, T, k, H, scale, add):
@@ -833,24 +858,18 @@ def fused_moe_fp8(x: torch.Tensor, topk_w: torch.Tensor, topk_ids: torch.Tensor,
     k = topk_ids.shape[1]
     n = T * k
     dev = x.device
-    offsets = torch.empty(E + 1, dtype=torch.int32, device=dev)
-    sorted_ids = torch.empty(n, dtype=torch.int32, device=dev)
-    inv = torch.empty(n, dtype=torch.int32, device=dev)
-    call("ome_moe_align", topk_ids.data_ptr(), n, E, offsets.data_ptr(), sorted_ids.data_ptr(), inv.data_ptr(),
-         stream_ptr())
-    qx, sx = fp8_quant(x, 128)
     tm = moe_fp8_tile_m(n, E)
-    tiles = -(-n // tm) + E
+    s = _Sorted(topk_ids, E, tm)
+    qx, sx = fp8_quant(x, 128)
     gu = torch.empty(n, I2, dtype=x.dtype, device=dev)
-    call("ome_moe_gemm_fp8_tile", qx.data_ptr(), qx.stride(0), sx.data_ptr(), sorted_ids.data_ptr(), k,
-         w13.q.data_ptr(), w13.scale.data_ptr(), offsets.data_ptr(), E, I2, H, tiles, tm, gu.data_ptr(), gu.stride(0),
-         stream_ptr())
+    call("ome_moe_gemm_fp8_tile", qx.data_ptr(), qx.stride(0), sx.data_ptr(), s.ids, k, w13.q.data_ptr(),
+         w13.scale.data_ptr(), s.tiles, I2, H, s.max_tiles, tm, gu.data_ptr(), gu.stride(0), stream_ptr())
     h = act_and_mul(gu, act)
     qh, sh = fp8_quant(h, 128)
     y = torch.empty(n, H, dtype=x.dtype, device=dev)
     call("ome_moe_gemm_fp8_tile", qh.data_ptr(), qh.stride(0), sh.data_ptr(), None, 0, w2.q.data_ptr(),
-         w2.scale.data_ptr(), offsets.data_ptr(), E, H, I, tiles, tm, y.data_ptr(), y.stride(0), stream_ptr())
-    return _combine(y, topk_w, inv, T, k, H, scale, add)
+         w2.scale.data_ptr(), s.tiles, H, I, s.max_tiles, tm, y.data_ptr(), y.stride(0), stream_ptr())
+    return _combine(y, topk_w, s.inv, T, k, H, scale, add)
 
 
 def moe_experts_sorted(rows: torch.Tensor, ids: torch.Tensor, w13, w2, act: int, n_experts: int):
@@ -860,39 +879,23 @@ def moe_experts_sorted(rows: torch.Tensor, ids: torch.Tensor, w13, w2, act: int,
     bf16 experts or Fp8Experts; nothing leaves the device (graph-capturable)."""
     n, H = rows.shape
     dev = rows.device
-    E1 = n_experts + 1
-    offsets = torch.empty(E1 + 1, dtype=torch.int32, device=dev)
-    sorted_ids = torch.empty(n, dtype=torch.int32, device=dev)
-    inv = torch.empty(n, dtype=torch.int32, device=dev)
-    call("ome_moe_align", ids.data_ptr(), n, E1, offsets.data_ptr(), sorted_ids.data_ptr(), inv.data_ptr(),
-         stream_ptr())
-    y = torch.empty(n, H, dtype=rows.dtype, device=dev)
-    if hasattr(w13, "scale") and hasattr(w13, "q"):
+    fp8 = hasattr(w13, "scale") and hasattr(w13, "q")
+    tm = moe_fp8_tile_m(n, n_experts) if fp8 else 64
+    s = _Sorted(ids, n_experts + 1, tm, n_experts)
+    if fp8:
         I2 = w13.q.shape[1]
-        tm = moe_fp8_tile_m(n, n_experts)
-        tiles = -(-n // tm) + n_experts
         qx, sx = fp8_quant(rows, 128)
         gu = torch.empty(n, I2, dtype=rows.dtype, device=dev)
-        call("ome_moe_gemm_fp8_tile", qx.data_ptr(), qx.stride(0), sx.data_ptr(), sorted_ids.data_ptr(), 1,
-             w13.q.data_ptr(), w13.scale.data_ptr(), offsets.data_ptr(), n_experts, I2, H, tiles, tm, gu.data_ptr(),
-             gu.stride(0), stream_ptr())
+        call("ome_moe_gemm_fp8_tile", qx.data_ptr(), qx.stride(0), sx.data_ptr(), s.ids, 1, w13.q.data_ptr(),
+             w13.scale.data_ptr(), s.tiles, I2, H, s.max_tiles, tm, gu.data_ptr(), gu.stride(0), stream_ptr())
         h = act_and_mul(gu, act)
         qh, sh = fp8_quant(h, 128)
+        y = torch.empty(n, H, dtype=rows.dtype, device=dev)
         call("ome_moe_gemm_fp8_tile", qh.data_ptr(), qh.stride(0), sh.data_ptr(), None, 0, w2.q.data_ptr(),
-             w2.scale.data_ptr(), offsets.data_ptr(), n_experts, H, I2 // 2, tiles, tm, y.data_ptr(), y.stride(0),
-             stream_ptr())
-        return y, inv
-    I2 = w13.shape[1]
-    tm = moe_tile_m(n, n_experts, I2)
-    gu = torch.empty(n, I2, dtype=rows.dtype, device=dev)
-    call("ome_moe_gemm", rows.data_ptr(), rows.stride(0), sorted_ids.data_ptr(), 1, w13.data_ptr(),
-         offsets.data_ptr(), n_experts, I2, H, -(-n // tm) + n_experts, gu.data_ptr(), gu.stride(0), None, tm,
-         stream_ptr())
-    h = act_and_mul(gu, act)
-    tm = moe_tile_m(n, n_experts, H)
-    call("ome_moe_gemm", h.data_ptr(), h.stride(0), None, 0, w2.data_ptr(), offsets.data_ptr(), n_experts, H,
-         I2 // 2, -(-n // tm) + n_experts, y.data_ptr(), y.stride(0), None, tm, stream_ptr())
-    return y, inv
+             w2.scale.data_ptr(), s.tiles, H, I2 // 2, s.max_tiles, tm, y.data_ptr(), y.stride(0), stream_ptr())
+        return y, s.inv
+    h = act_and_mul(_moe_gemm(rows, s, s.ids, 1, w13, n, None, n_experts), act)
+    return _moe_gemm(h, s, None, 0, w2, n, None, n_experts), s.inv
 
 
 class DecodeWorkspace:

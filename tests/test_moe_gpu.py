@@ -122,3 +122,36 @@ def test_moe_align_offsets(E, n):
     assert torch.equal(off.cpu().long(), torch.cat([torch.zeros(1, dtype=torch.long), count.cumsum(0)]))
     assert torch.equal(ids[srt.long()].cpu(), ids.cpu().sort().values)
     assert torch.equal(srt[inv.long()].cpu(), torch.arange(n, dtype=torch.int32))
+
+
+@pytest.mark.parametrize("E,e_tiles", [(1, 1), (64, 64), (300, 299), (1025, 1025)])
+@pytest.mark.parametrize("n,bm", [(1, 64), (65, 64), (5000, 64), (5000, 128)])
+def test_moe_align_tiles(E, e_tiles, n, bm):
+    torch.manual_seed(E + n)
+    ids = (torch.randint(0, E, (n,)) * torch.randint(0, 2, (n,))).to(torch.int32).to(DEV)   # half of them the first expert's
+    s = ops._Sorted(ids, E, bm, e_tiles)
+    off = torch.cat([torch.zeros(1, dtype=torch.long), torch.bincount(ids.cpu().long(), minlength=E).cumsum(0)]).tolist()
+    want = [[e, m, off[e + 1], 0] for e in range(e_tiles) for m in range(off[e], off[e + 1], bm)]
+    tiles = s.meta[:4 * s.max_tiles].view(-1, 4).tolist()
+    assert tiles[:len(want)] == want and all(t[0] == -1 for t in tiles[len(want):]) and len(want) <= len(tiles)
+
+
+@pytest.mark.parametrize("counts", [[1], [64, 0, 65], [0, 63, 128, 1, 0], [3] * 40, [0] * 30 + [130] * 12], ids=str)
+@pytest.mark.parametrize("N,K", [(64, 64), (100, 128), (37, 192), (320, 320), (3000, 64)])
+@pytest.mark.parametrize("gather", [True, False])
+def test_streamed_experts_at_tile_edges(counts, N, K, gather):
+    """Rows, weight rows and stages that fill no tile, experts without rows, few workgroups (four stages) and many (three)."""
+    torch.manual_seed(N + K)
+    E, n = len(counts), sum(counts)
+    order = torch.randperm(n)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[order].to(torch.int32).to(DEV)
+    x = torch.randn(n, K + 8, device=DEV).to(torch.bfloat16)[:, 8:] if gather else torch.randn(n, K, device=DEV).to(torch.bfloat16)
+    w, b = (torch.randn(E, N, K, device=DEV) * K ** -0.5).to(torch.bfloat16), torch.randn(E, N, device=DEV).to(torch.bfloat16)
+    s = ops._Sorted(ids, E, 64)
+    assert ops.moe_tile_m(n, E, N) == 64
+    got = ops._moe_gemm(x, s, s.ids if gather else None, 1 if gather else 0, w, n, b).cpu()
+    rows = s.meta[-2 * n:-n].long().cpu() if gather else torch.arange(n)
+    e = ids.cpu().long().sort().values
+    want = torch.einsum("nk,nok->no", x.cpu().double()[rows], w.cpu().double()[e]) + b.cpu().double()[e]
+    # fp32 sums of K products, one rounding to bf16: 2^-8 of each value (half a step), and 2^-24 K of the products' size
+    assert torch.allclose(got.double(), want, rtol=2.0 ** -8, atol=2.0 ** -24 * K * 8)
