@@ -197,6 +197,18 @@ __device__ __forceinline__ void buffer_to_lds4(const void* base, uint32_t bytes,
 #endif
 }
 
+// Eight consecutive sums of a projection whose K was cut into `splits` pieces, `stride` floats apart, in their order (gemm_rows.hip)
+__device__ __forceinline__ void sum_parts8(const float* __restrict__ p, int64_t stride, int splits, float (&f)[8]) {
+  f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
+#pragma unroll 7
+  for (int s = 1; s < splits; ++s) {
+    a += *reinterpret_cast<const f32x4*>(p + s * stride);
+    b += *reinterpret_cast<const f32x4*>(p + s * stride + 4);
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) f[j] = a[j], f[4 + j] = b[j];
+}
+
 // XCD-aware remap of a linear workgroup id (bijective for any nwg; T1 of the guide).
 // Blocks b and b+8 share an XCD under round-robin dispatch, so give each XCD group a
 // contiguous chunk of the logical id space.

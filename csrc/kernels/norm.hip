@@ -97,6 +97,47 @@ __global__ __launch_bounds__(NT) void fused_add_rmsnorm_kernel(bf16* __restrict_
   }
 }
 
+// The same where x is still in pieces (gemm_rows.hip): residual <- sum of the pieces + residual ; out <- rmsnorm(residual) * w
+template <int NT, int CHUNKS>
+__global__ __launch_bounds__(NT) void add_rmsnorm_parts_kernel(const float* __restrict__ part, int splits, bf16* __restrict__ res,
+                                                               int64_t res_stride, const bf16* __restrict__ w,
+                                                               bf16* __restrict__ out, int64_t out_stride, int rows, int H, float eps) {
+  __shared__ float red[NT / 64];
+  const int row = blockIdx.x, nvec = H >> 3;
+  bf16* rr = res + row * res_stride;
+  bf16* orow = out + row * out_stride;
+  bf16x8 v[CHUNKS], wv[CHUNKS];
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int i = threadIdx.x + c * NT;
+    if (i < nvec) {
+      const bf16x8 b = ld8(rr + i * 8);
+      wv[c] = ld8(w + i * 8);
+      float f[8];
+      sum_parts8(part + (int64_t)row * H + i * 8, (int64_t)rows * H, splits, f);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        v[c][j] = (bf16)(f[j] + (float)b[j]);   // the residual stream is stored in bf16
+        ss += (float)v[c][j] * (float)v[c][j];
+      }
+      st8(rr + i * 8, v[c]);
+    }
+  }
+  ss = block_sum<NT>(ss, red);
+  const float rs = rsqrtf(ss / (float)H + eps);
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int i = threadIdx.x + c * NT;
+    if (i < nvec) {
+      bf16x8 o;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[j] = (bf16)((float)v[c][j] * rs * (float)wv[c][j]);
+      st8(orow + i * 8, o);
+    }
+  }
+}
+
 // LayerNorm with bias (Starcoder2, GPT-NeoX): out = (x - mean) * rstd * w + b; with ``res`` set the
 // residual add is fused in front (res <- x + res, normalise res, write x), like fused_add_rmsnorm.
 template <int NT, int CHUNKS, bool ADD>
@@ -209,6 +250,15 @@ OME_API int ome_fused_add_rmsnorm(void* x, int64_t x_stride, void* res, int64_t 
     DISPATCH_CHUNKS(H, 256, (fused_add_rmsnorm_kernel<256, CH><<<rows, 256, 0, stream>>>(
                                 (bf16*)x, x_stride, (bf16*)res, res_stride, (const bf16*)w, H, eps)));
   }
+  OME_CHECK_LAUNCH();
+  return 0;
+}
+
+OME_API int ome_add_rmsnorm_parts(const float* part, int splits, void* res, int64_t res_stride, const void* w, void* out, int64_t out_stride,
+                                  int rows, int H, float eps, hipStream_t stream) {
+  if (H % 8 != 0 || rows <= 0 || splits < 1) return rows == 0 ? 0 : -2;
+  DISPATCH_CHUNKS(H, 512, (add_rmsnorm_parts_kernel<512, CH><<<rows, 512, 0, stream>>>(
+                              part, splits, (bf16*)res, res_stride, (const bf16*)w, (bf16*)out, out_stride, rows, H, eps)));
   OME_CHECK_LAUNCH();
   return 0;
 }

@@ -357,20 +357,22 @@ class LlamaForCausalLM:
     def mlp(self, i: int, x: torch.Tensor) -> torch.Tensor:
         return pstate.tp_all_reduce(self._mlp_partial(i, x))
 
-    def _mlp_partial(self, i: int, x: torch.Tensor) -> torch.Tensor:
+    def _mlp_partial(self, i: int, x: torch.Tensor, parts: bool = False) -> torch.Tensor:
         """gate_up -> SiLU*mul -> down: this rank's partial sums (before the TP all-reduce),
-        written straight into the all-reduce's staging buffer when there is one."""
+        written straight into the all-reduce's staging buffer when there is one.  ``parts`` as :meth:`_row_parallel`."""
         wd = self.w_d[i]
         if self.gu_il:
             w = self.w_gu[i]
             plan = ops.gemm_sk_plan(x.shape[0], w.shape[0], w.shape[1], 2) if x.shape[0] > _GEMV_ROWS else None
-            if plan is not None and x.stride(1) == 1 and x.stride(0) % 8 == 0:
+            if _GEMV_ROWS < x.shape[0] <= 256 and ops.gemm_rows_plan(x, w):
+                a = ops.gemm_rows(x, w, epi=2)
+            elif plan is not None and x.stride(1) == 1 and x.stride(0) % 8 == 0:
                 a = ops.gemm_sk(x, w, epi=2, bn=plan[0], nwg=plan[1], bm=plan[2])
             elif x.is_cuda and x.shape[0] <= _GEMV_ROWS and ops.gemv_ok(x, w):
                 a = ops.gemv_swiglu(x, w)
             else:
                 a = ops.act_and_mul(linear(x, w), self.act, interleaved=True)
-            return self._row_parallel(a, wd)
+            return self._row_parallel(a, wd, parts=parts)
         gu = linear(x, self.w_gu[i])
         if _GEMV_ACT and self.act == 0 and gu.is_cuda and type(wd) is torch.Tensor and gu.dim() == 2 and \
                 gu.shape[0] <= _GEMV_ROWS and gu.dtype == wd.dtype == torch.bfloat16 and gu.stride(1) == 1 and \
@@ -380,9 +382,14 @@ class LlamaForCausalLM:
                 if self.tp.tp > 1 else None
             return ops.gemv_act(gu, wd, out=st)
         a = ops.act_and_mul(gu, self.act)
-        return self._row_parallel(a, wd)
+        return self._row_parallel(a, wd, parts=parts)
 
-    def _row_parallel(self, a: torch.Tensor, w, bias=None) -> torch.Tensor:
+    def _row_parallel(self, a: torch.Tensor, w, bias=None, parts: bool = False) -> torch.Tensor:
+        """``parts``: the caller hands the result to :meth:`_reduce_add_norm`, so it may come in pieces (fp32 [pieces, T, H])."""
+        if parts and self.tp.tp == 1 and bias is None and type(w) is torch.Tensor and _GEMV_ROWS < a.shape[0] <= 256:
+            splits = ops.gemm_rows_parts_plan(a, w)
+            if splits:
+                return ops.gemm_rows_parts(a, w, splits)
         if self.tp.tp > 1:
             st = pstate.tp_ar_staging((a.shape[0], self.cfg.hidden_size), self.dtype, a.device)
             if st is not None:
@@ -394,6 +401,8 @@ class LlamaForCausalLM:
         """residual += allreduce(part); return rmsnorm(residual) * w -- one fused xGMI kernel at
         decode sizes under TP, all-reduce + fused_add_rmsnorm otherwise (``reduce=False``: the
         input is already reduced)."""
+        if part.dim() == 3:
+            return ops.add_rmsnorm_parts(part, residual, w, self.eps)
         if self.tp.tp > 1 and reduce:
             y = pstate.tp_all_reduce_add_rmsnorm(part, residual, w, self.eps)
             if y is not None:
@@ -412,6 +421,7 @@ class LlamaForCausalLM:
         first = self.layers[0] if self.layers else 0
         # subclasses that override mlp() (MoE) return already-reduced outputs
         partial = type(self).mlp is LlamaForCausalLM.mlp
+        parts = st.pp_size == 1   # every projection of the residual stream is followed by a norm here
         for i in self.layers:
             if i > 0:  # the previous layer's MLP partial sums -> all-reduce + add + norm (a pipeline
                 # stage's first layer receives the previous stage's already-reduced output)
@@ -428,9 +438,9 @@ class LlamaForCausalLM:
                 ops.rope_qkv_cache(qkv, meta.positions, self.cos_sin, cfg.rot_dim, q, k_cache, v_cache, meta.slots,
                                    tp.hq, tp.hkv, D, True, self.qn[i], self.kn[i], self.eps, ks, vs)
             attn = self.attention(q, k_cache, v_cache, meta, ks, vs)
-            o = self._reduce_add_norm(self._row_parallel(attn.view(T, tp.hq * D), self.w_o[i]), residual,
-                                      self.ln2[i])
-            x = self._mlp_partial(i, o) if partial else self.mlp(i, o)
+            o = self._reduce_add_norm(self._row_parallel(attn.view(T, tp.hq * D), self.w_o[i], parts=parts),
+                                      residual, self.ln2[i])
+            x = self._mlp_partial(i, o, parts) if partial else self.mlp(i, o)
         if self.layers and (st.pp_size == 1 or st.is_last_pp):
             return self._reduce_add_norm(x, residual, self.norm, reduce=partial)   # final norm
         if self.layers and partial:

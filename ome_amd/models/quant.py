@@ -175,7 +175,7 @@ def _sk_operands_ok(x, w, bias, out) -> bool:
 
 def linear(x: torch.Tensor, w, bias: torch.Tensor | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
     """Dispatch: bf16 weight at a row count where the stream-K MFMA kernel was measured faster
-    (``ops.gemm_sk_plan``) -> ``ops.gemm_sk``; single-row decode -> the GEMV stream kernel
+    (``ops.gemm_sk_plan``) -> ``ops.gemm_sk``; up to 256 rows of a wide weight -> ``ops.gemm_rows``; single-row decode -> the GEMV stream kernel
     (``ops.gemv``, ``OME_GEMV_ROWS``); the weight-streaming MFMA GEMM for decode shapes where it
     was measured faster (``ops.decode_gemm_plan``, opt-in); other plain tensors -> hipBLASLt;
     Fp8Weight -> W8A16 (fp8 weight, bf16 activation) at the decode rows where ``ops.w8a16_plan``
@@ -183,6 +183,8 @@ def linear(x: torch.Tensor, w, bias: torch.Tensor | None = None, out: torch.Tens
     staging buffer)."""
     if (x.dim() == 2 and x.is_cuda and x.shape[0] > _GEMV_ROWS and type(w) is torch.Tensor
             and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16):
+        if x.shape[0] <= 256 and ops.gemm_rows_plan(x, w, bias, out):
+            return ops.gemm_rows(x, w, bias, out)
         plan = ops.gemm_sk_plan(x.shape[0], w.shape[0], w.shape[1], 0)
         if plan is not None and _sk_operands_ok(x, w, bias, out):
             return ops.gemm_sk(x, w, bias, out=out, bn=plan[0], nwg=plan[1], bm=plan[2])

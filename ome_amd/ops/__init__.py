@@ -1577,6 +1577,78 @@ def gemm_sk(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, 
     return out
 
 
+# ---- projections of 5 to 256 decode rows (csrc/kernels/gemm_rows.hip) ---------------------------
+def gemm_rows_ok(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, out: torch.Tensor | None = None) -> bool:
+    """Operands that ``ome_gemm_rows`` (and the kernels that add its pieces) take."""
+    return (x.is_cuda and x.dim() == 2 and w.dim() == 2 and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.stride(1) == 1
+            and w.stride(1) == 1 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.shape[1] <= x.stride(0) < 1 << 22
+            and w.shape[1] <= w.stride(0) < 1 << 23 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and 0 < x.shape[0] <= 256
+            and w.shape[0] % 128 == 0 and w.shape[0] > 0 and w.shape[1] % 64 == 0 and w.shape[1] >= 64
+            and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous()))
+            and (out is None or (out.dim() == 2 and out.dtype == torch.bfloat16 and out.stride(1) == 1 and out.stride(0) % 4 == 0
+                                 and out.stride(0) >= out.shape[1] and out.data_ptr() % 8 == 0)))
+
+
+def gemm_rows_plan(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, out: torch.Tensor | None = None) -> bool:
+    """:func:`gemm_rows` takes this product and fills the chip with it: its workgroups of 128 columns come in whole waves over the 256
+    CUs, three quarters full at the least (288 of them, 36864 x 7168: 106 us against the library's 100), and beyond 128 rows, where
+    the matrix cores count too, in one (57344 x 8192 at 160 rows: 228 us against 190; at 128 174 against 178)."""
+    if not gemm_rows_ok(x, w, bias, out):
+        return False
+    tiles = w.shape[0] // 128
+    waves = -(-tiles // 256)
+    return tiles >= 192 * waves and (x.shape[0] <= 128 or waves == 1)
+
+
+def gemm_rows(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, out: torch.Tensor | None = None,
+              epi: int = 0) -> torch.Tensor:
+    """out = x @ w.T (+ bias) of at most 256 rows (:func:`gemm_rows_ok` operands); ``epi=2`` as :func:`gemm_sk`."""
+    M, K = x.shape
+    N = w.shape[0]
+    if out is None:
+        out = torch.empty(M, N // 2 if epi == 2 else N, dtype=x.dtype, device=x.device)
+    call("ome_gemm_rows", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), ptr(bias), out.data_ptr(), out.stride(0), M, N, K, epi, 1,
+         None, stream_ptr())
+    return out
+
+
+def gemm_rows_splits(M: int, N: int, K: int) -> int:
+    """Pieces of K for :func:`gemm_rows_parts`: as many as bring about 256 workgroups, of four steps of 64 at the least, 8 at the most.
+    Beyond 128 rows of ten steps, as more of them cost more to add than they save (4096 x 4096, 256 rows with the norm: 6 pieces
+    26.6 us, 8 29.6; at 64 rows 16.6 and 16.5)."""
+    return min(256 // (N // 128), K // (256 if M <= 128 else 640), 8)
+
+
+def gemm_rows_parts_plan(x: torch.Tensor, w: torch.Tensor) -> int:
+    """Pieces of :func:`gemm_rows_parts` where it, with :func:`add_rmsnorm_parts`, is faster than a projection and
+    :func:`fused_add_rmsnorm`; else 0."""
+    if not gemm_rows_ok(x, w):
+        return 0
+    M, K = x.shape
+    splits = gemm_rows_splits(M, w.shape[0], K)
+    return splits if splits > 1 else 0
+
+
+def gemm_rows_parts(x: torch.Tensor, w: torch.Tensor, splits: int) -> torch.Tensor:
+    """x @ w.T over ``splits`` pieces of K, not added: fp32 [splits, M, N], for :func:`add_rmsnorm_parts`, which adds them as it
+    reads (no pass of its own)."""
+    M, K = x.shape
+    N = w.shape[0]
+    part = torch.empty(splits, M, N, dtype=torch.float32, device=x.device)
+    call("ome_gemm_rows", x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), None, None, 0, M, N, K, 3, splits, part.data_ptr(),
+         stream_ptr())
+    return part
+
+
+def add_rmsnorm_parts(part: torch.Tensor, res: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
+    """:func:`fused_add_rmsnorm` of a projection in pieces: res <- sum of them + res; returns rmsnorm(res) * w."""
+    S, M, H = part.shape
+    out = torch.empty(M, H, dtype=res.dtype, device=res.device)
+    call("ome_add_rmsnorm_parts", part.data_ptr(), S, res.data_ptr(), res.stride(0), w.data_ptr(), out.data_ptr(), out.stride(0), M, H,
+         float(eps), stream_ptr())
+    return out
+
+
 def gemm_xl_ok(M: int, N: int, K: int, bn: int = 256, nwg: int = 256) -> bool:
     """Shapes / decompositions accepted by ``ome_gemm_xl`` with the shared stream-K workspace."""
     return bn in (128, 256) and M > 0 and N % bn == 0 and K % 32 == 0 and K > 0 and nwg % 8 == 0 and \
