@@ -24,11 +24,14 @@ def _f32(t: torch.Tensor, *same) -> int:
     """1 when ``t`` (and every tensor of ``same`` that is not None) is float32, 0 when they are all
     bfloat16 -- the element-type switch of the kernels that serve fp32 models too; anything else
     (or a mix) raises."""
+    dt = t.dtype
+    if dt is torch.bfloat16 or dt is torch.float32:
+        for x in same:
+            if x is not None and x.dtype is not dt:
+                break
+        else:
+            return int(dt is torch.float32)
     ts = [t] + [x for x in same if x is not None]
-    if all(x.dtype == torch.float32 for x in ts):
-        return 1
-    if all(x.dtype == torch.bfloat16 for x in ts):
-        return 0
     raise TypeError(f"operands must be all bfloat16 or all float32, got {[str(x.dtype) for x in ts]}")
 
 
