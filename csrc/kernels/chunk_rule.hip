@@ -12,7 +12,9 @@
 // Two launches.  chunk_gram_kernel (Mamba-2: ssm_gram_kernel), parallel over all rows: the 32 x 32 matrices
 // P T and T (Mamba-2: q k^T, which the heads of a group share) and the chunk's scalars, into a workspace.
 // chunk_rule_kernel walks the chunks of a (sequence, head) in order: a wave owns 16 value columns and keeps its
-// S in VGPR accumulators.
+// S in VGPR accumulators.  Long prompts of few heads are cut into segments that are walked side by side, in two launches of it
+// (ops._chunk_rule_seg; S at a segment's end is linear in S at its start): 8000 rows of 8 heads of 128 x 128 450 -> 150 us,
+// 32 heads of 64 x 128 410 -> 110.  The state's error against 64 bits, eight prompts of 1000 to 8000 rows: 1.10e-7 both ways (8.55e-8).
 //
 // What bounds it: the instructions of a wave that has its SIMD almost for itself, 96 matrix (Mamba-2: 60) and some 250 (310) vector
 // ones a chunk.  A product takes 16 cycles alone, but about 9 of them stay its own where vector instructions of 4 cycles fill
@@ -74,7 +76,29 @@ struct RuleArgs {
   int64_t out_stride;
   const int *cu, *slot, *reset;
   int S, H, Hk, dv;
+  int seg;                        // chunks of a segment (0: sequences in one piece)
+  float* segs;                    // seg_floats of every (segment, head)
 };
+
+// Floats that a segment leaves of a head: its state [dv, dk]; then DELTA its transition [dk, dk], Mamba-2 its decay (a sequence's first
+// segment: what the sequence started from).
+__host__ __device__ constexpr int64_t seg_floats(int dv, int dk) { return (int64_t)dv * dk + (int64_t)(dv > dk ? dv : dk) * dk + 4; }
+
+// Segment `id` of `R` rows -> (sequence, number in it); ids as those of chunks below.  Whole wave.
+__device__ __forceinline__ bool segment_of(int id, int R, const int* cu, int S, int& s, int& j) {
+  const int lane = threadIdx.x & 63;
+  s = -1;
+  for (int b = 0; b < S; b += 64) {
+    const int i = b + lane;
+    const int c = __popcll(__ballot(i < S && cu[min(i, S)] / R + i <= id));
+    s += c;
+    if (c < 64) break;
+  }
+  s = __builtin_amdgcn_readfirstlane(s);
+  if (s < 0) return false;
+  j = id - cu[s] / R - s;
+  return cu[s] + (int64_t)j * R < cu[s + 1];
+}
 
 // Sequences of at most FEW rows (the decode rows beside a prompt) are walked row by row instead: no chunk in the workspace,
 // no products 1/32 full.  The walk is bound by its vector instructions, near 1 us a row and four waves a CU.  Chunks -> walk, in us,
@@ -426,8 +450,13 @@ __device__ __forceinline__ int in_turn(int z, int per, const int* cu, int S) {
 // leaves its registers.  S += k^T U takes k transposed out of the same LDS image (ds_read_b64_tr_b16).  The
 // next chunk moves to the other LDS buffer while this one is computed: one barrier per chunk.
 // VEC: values in 16-byte pieces by DMA, outputs in 8-byte ones; not: element by element (views that are not aligned for that).
+//
+// SEG: few sequences of few heads leave most of the chip idle for their length, so they run in segments side by side.
+//   1  a segment's own state: S from zero (a sequence's first segment: from where the sequence starts), without outputs, and for DELTA its
+//      transition M, the state of the identity's columns without values (workgroups beyond the values' in y).  The last segment has none.
+//   2  the segment itself, from S = M_i S + S_i over the segments before it (Mamba-2: M is the product of the decays).
 // ---------------------------------------------------------------------------------------------
-template <int DK, bool DELTA, int NW, bool VEC>
+template <int DK, bool DELTA, int NW, bool VEC, int SEG = 0>
 __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   constexpr int NS = DK / 32, NB = DK / 16, NT = 64 * NW, COLS = 16 * NW;
   constexpr int NML = RC * RC / 4 / NT;                  // 16-byte loads of q k^T per thread (Mamba-2)
@@ -437,11 +466,19 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   __shared__ __attribute__((aligned(1024))) char lds[2 * IMG];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)lds;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4;
-  const int s = in_turn(blockIdx.z, gridDim.x * gridDim.y, a.cu, a.S), h = blockIdx.x, hk = h / (a.H / a.Hk);
-  const int c0 = blockIdx.y * COLS, n0 = c0 + wave * 16;   // the block's and this wave's columns
-  const bool live = n0 < a.dv;                             // dv is a multiple of 16: a wave has all of them or none
-  const int r0 = a.cu[s], r1 = a.cu[s + 1];
+  int s, j = 0;
+  if constexpr (SEG == 0) s = in_turn(blockIdx.z, gridDim.x * gridDim.y, a.cu, a.S);
+  else if (!segment_of(blockIdx.z, a.seg * RC, a.cu, a.S, s, j)) return;
+  const int h = blockIdx.x, hk = h / (a.H / a.Hk);
+  const int q0 = a.cu[s], r0 = q0 + j * a.seg * RC, r1 = SEG ? min(a.cu[s + 1], r0 + a.seg * RC) : a.cu[s + 1];
   if (r1 <= r0) return;                                    // whole block
+  const bool last = SEG == 0 || r1 == a.cu[s + 1];
+  const bool ident = SEG == 1 && DELTA && blockIdx.y >= (a.dv + COLS - 1) / COLS;   // columns of the transition
+  if (SEG == 1 && (last || (ident && j == 0))) return;
+  const int c0 = (ident ? blockIdx.y - (a.dv + COLS - 1) / COLS : blockIdx.y) * COLS, n0 = c0 + wave * 16;   // the block's and this wave's columns
+  const bool live = ident || n0 < a.dv;                    // dv is a multiple of 16: a wave has all of them or none
+  float* const sg = SEG ? a.segs + ((int64_t)blockIdx.z * a.H + h) * seg_floats(a.dv, DK) : nullptr;   // this segment's
+  const int64_t sg_step = (int64_t)a.H * seg_floats(a.dv, DK);
   const int chunks = (r1 - r0 + RC - 1) / RC;
   const int nc = (live ? n0 : 0) + col;
 
@@ -466,8 +503,8 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   const int64_t x_step = (int64_t)RC * 2 * a.v_stride, k_step = (int64_t)RC * 2 * a.stride, ws_step = ws_bytes<DELTA>(a.H, a.Hk), o_step = (int64_t)RC * 2 * a.out_stride;
   const char* kp = reinterpret_cast<const char*>(a.k + (int64_t)r0 * a.stride + hk * DK);   // these walk with the chunks fetched
   const char* qp = reinterpret_cast<const char*>(a.q + (int64_t)r0 * a.stride + hk * DK);
-  const char* gp = a.ws + (r0 / RC + s) * ws_step + hk * group_bytes<DELTA>();
-  const char* hp = a.ws + (r0 / RC + s) * ws_step + a.Hk * group_bytes<DELTA>() + h * head_bytes<DELTA>();
+  const char* gp = a.ws + (q0 / RC + s + j * a.seg) * ws_step + hk * group_bytes<DELTA>();
+  const char* hp = a.ws + (q0 / RC + s + j * a.seg) * ws_step + a.Hk * group_bytes<DELTA>() + h * head_bytes<DELTA>();
   f32x4 rp[NML], rhj[NML], rlj[NML];
   float rhi[NML], rli[NML];
   bf16x8 rx;
@@ -477,7 +514,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
     if (more && n < RC) offsets(n);
     const uint32_t to = lds0 + b * IMG, kb = (RC - 1) * 2 * (uint32_t)a.stride + 2 * DK;
     if constexpr (VEC) {
-      buffer_to_lds(xp, more ? (uint32_t)(RC - 1) * 2 * (uint32_t)a.v_stride + 2 * COLS : 0, xo, 0, to + X_AT + 1024 * wave);
+      buffer_to_lds(xp, more && !ident ? (uint32_t)(RC - 1) * 2 * (uint32_t)a.v_stride + 2 * COLS : 0, xo, 0, to + X_AT + 1024 * wave);
     } else {
 #pragma unroll
       for (int e = 0; e < 8; ++e) rx[e] = *reinterpret_cast<const bf16*>(xp + xo + 2 * e);
@@ -485,14 +522,14 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
       buffer_to_lds(kp, more ? kb : 0, ko[i], 0, to + 1024 * (wave + NW * i));
-      buffer_to_lds(qp, more ? kb : 0, ko[i], 0, to + ROWS + 1024 * (wave + NW * i));
+      if constexpr (SEG != 1) buffer_to_lds(qp, more ? kb : 0, ko[i], 0, to + ROWS + 1024 * (wave + NW * i));
     }
 #pragma unroll
     for (int i = 0; i < (NH - 1) / NW; ++i)
       buffer_to_lds(hp, more ? (NH - 1) * 1024 : 0, 16 * lane, 1024 * (wave + NW * i), to + M_AT + 1024 * (wave + NW * i));
     buffer_to_lds4(hp + (NH - 1) * 1024, more ? 4 * vec_floats<DELTA>() : 0, 4 * tid, to + V_AT + 256 * wave);
     static_assert(NT * 4 == VECS, "a float a thread");
-    if constexpr (!DELTA) {   // q k^T and its decays go through registers
+    if constexpr (!DELTA && SEG != 1) {   // q k^T and its decays go through registers
 #pragma unroll
       for (int i = 0; i < NML; ++i) {
         rp[i] = *reinterpret_cast<const f32x4*>(gp + (uint32_t)(16 * (tid + NT * i)));
@@ -513,7 +550,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   };
   const auto put = [&](int b) {   // P_ij = q_i.k_j exp(cum_i - cum_j), j <= i; cum in two parts (long sums, short differences)
     if constexpr (!VEC) *reinterpret_cast<bf16x8*>(lds + b * IMG + X_AT + 16 * tid) = rx;
-    if constexpr (!DELTA) {
+    if constexpr (!DELTA && SEG != 1) {
 #pragma unroll
       for (int i = 0; i < NML; ++i) {
         const int e = tid + NT * i, row = e / (RC / 4), j = 4 * (e % (RC / 4));
@@ -532,12 +569,27 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   // state: lane (col, g) holds column nc, key channels 32 s + 8 g .. + 7 in blocks 2 s, 2 s + 1
   float* st = a.state + (((int64_t)a.slot[s] * a.H + h) * a.dv + nc) * DK + 8 * g;
   f32x4 S[NB];
-  const auto start = [&] {
+  const auto load = [&](const float* from) {
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
-      S[b] = a.reset[s] != 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4*>(st + 32 * (b >> 1) + 4 * (b & 1));
+    for (int b = 0; b < NB; ++b) S[b] = *reinterpret_cast<const f32x4*>(from + 32 * (b >> 1) + 4 * (b & 1));
   };
-  start();
+  const auto store = [&](float* to) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) *reinterpret_cast<f32x4*>(to + 32 * (b >> 1) + 4 * (b & 1)) = S[b];
+  };
+  const auto finite = [&] {   // of the whole wave's S
+    float broken = 0.f;       // NaN if a value of S is not finite
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) broken += S[nb][e] * 0.f;
+    return __ballot(broken != 0.f) == 0;
+  };
+  const auto zero = [&] {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) S[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  const int64_t mine = (int64_t)nc * DK + 8 * g, copy = (int64_t)a.dv * DK;   // places in a segment's floats
   const float Dh = DELTA ? 0.f : a.D[h];
   // outputs: lane (col, g) holds rows col and 16 + col, columns n0 + 4 g .. + 3
   char* op = reinterpret_cast<char*>(a.out + (int64_t)r0 * a.out_stride + (int64_t)h * a.dv + c0);
@@ -545,9 +597,8 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   const uint32_t oo[2] = {2 * (uint32_t)col * (uint32_t)a.out_stride, 2 * (uint32_t)(16 + col) * (uint32_t)a.out_stride};
 
   // the sequence row by row, as the row-by-row kernels do it (each lane its 8 key channels of every 32)
-  const auto walk = [&](int n) {
-    for (int i = 0; i < n; ++i) {
-      const int64_t row = r0 + i;
+  const auto walk = [&](int from, int to, bool write) {
+    for (int64_t row = from; row < to; ++row) {
       bf16x8 k8[NS], q8[NS];
 #pragma unroll
       for (int t = 0; t < NS; ++t) {
@@ -591,11 +642,81 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
           S[2 * t + j / 4][j % 4] = s1;
         }
       sq = group4_sum(sq);
-      if (live && g == 0) a.out[row * a.out_stride + (int64_t)h * a.dv + nc] = (bf16)(DELTA ? decay * sq + add * kq : sq + Dh * x);
+      if (write && live && g == 0) a.out[row * a.out_stride + (int64_t)h * a.dv + nc] = (bf16)(DELTA ? decay * sq + add * kq : sq + Dh * x);
     }
   };
 
-  const bool few = r1 - r0 <= FEW;                      // whole block
+  // what the sequence starts from
+  const auto origin = [&] {
+    if (SEG == 2 && !(last && j == 0)) load(sg - j * sg_step + copy + mine);   // (its last segment may have written `state` by now)
+    else if (a.reset[s] != 0) zero();
+    else load(st);
+  };
+  // what the rows r0 and up start from
+  const auto start = [&] {
+    if (SEG == 2 && j > 0) {
+      const float* f = sg - j * sg_step;
+      load(f + mine);
+#pragma unroll 1
+      for (int i = 1; i < j; ++i) {
+        f += sg_step;
+        if constexpr (DELTA) {   // S = M S + S_i, M through LDS (16-byte pieces swizzled by the rows that a product takes together)
+          if (i > 1) __syncthreads();
+          constexpr int PR = DK / 4;   // pieces of a row
+#pragma unroll
+          for (int x = 0; x < DK * DK / 256 / NW; ++x) {
+            const int e = 64 * (wave + NW * x) + lane, row = e / PR;
+            buffer_to_lds(f + copy, 4 * DK * DK, 4 * row * DK + 16 * ((e % PR) ^ ((row & 3) | ((row >> 3) & 3) << 2)), 0, lds0 + 1024 * (wave + NW * x));
+          }
+          f32x4 n[NB];
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) n[nb] = *reinterpret_cast<const f32x4*>(f + mine + 32 * (nb >> 1) + 4 * (nb & 1));
+          bf16x8 part[NS][3];
+#pragma unroll
+          for (int t = 0; t < NS; ++t) split3(S[2 * t], S[2 * t + 1], part[t]);
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          __syncthreads();
+          const float* m = reinterpret_cast<const float*>(lds) + (8 * (col >> 2) + (col & 3)) * DK;
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) {
+            const float* r = m + (32 * (nb >> 1) + 4 * (nb & 1)) * DK;
+            bf16x8 x[NS][3];
+#pragma unroll
+            for (int t = 0; t < NS; ++t)
+              split3(*reinterpret_cast<const f32x4*>(r + 4 * ((8 * t + 2 * g) ^ col)), *reinterpret_cast<const f32x4*>(r + 4 * ((8 * t + 2 * g + 1) ^ col)), x[t]);
+            f32x4 ms = {0.f, 0.f, 0.f, 0.f};   // the smallest terms first
+#pragma unroll
+            for (int sum = 2; sum >= 0; --sum)
+#pragma unroll
+              for (int t = 0; t < NS; ++t)
+#pragma unroll
+                for (int y = 0; y <= sum; ++y) ms = mma_bf16(x[t][y], part[t][sum - y], ms);
+            S[nb] = ms + n[nb];
+          }
+        } else {
+          const float d = f[copy];
+#pragma unroll
+          for (int b = 0; b < NB; ++b) S[b] = S[b] * d + *reinterpret_cast<const f32x4*>(f + mine + 32 * (b >> 1) + 4 * (b & 1));
+        }
+      }
+      if (DELTA && j > 1) __syncthreads();
+      if (live && !finite()) {   // row by row, as the sequence in one piece has it
+        origin();
+        walk(q0, r0, false);
+      }
+    } else if (SEG == 1 && j > 0) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[b][e] = ident && 32 * (b >> 1) + 8 * g + 4 * (b & 1) + e == nc ? 1.f : 0.f;
+    } else {
+      origin();
+      if (SEG == 1 && live) store(sg + copy + mine);
+    }
+  };
+  start();
+
+  const bool few = r1 - r0 <= FEW && j == 0;            // whole block
   if (!few) {
     offsets(min(RC, r1 - r0));
     fetch(RC, true, 0);
@@ -604,6 +725,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
   }
+  float decay = 1.f;   // of the chunks so far (SEG 1, Mamba-2)
   // One chunk.  With one or two waves a SIMD nothing else covers an LDS read: each is issued a stage before its use, and the
   // scheduling barriers keep the compiler from sinking it there.
   const auto step = [&](int c, int b) {
@@ -622,7 +744,9 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
 #pragma unroll
     for (int t = 0; t < NS; ++t)
 #pragma unroll
-      for (int rb = 0; rb < 2; ++rb) (DELTA ? kf : qf)[rb][t] = rows(DELTA ? K : Q, rb, t);
+      for (int rb = 0; rb < 2; ++rb)
+        if constexpr (DELTA) kf[rb][t] = rows(K, rb, t);
+        else if constexpr (SEG != 1) qf[rb][t] = rows(Q, rb, t);
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
       x[rb] = tr4(X, 8 * val_img(16 * rb + 4 * g + (col >> 2), 2 * wave + ((col >> 1) & 1)) + 4 * (col & 1));
@@ -632,7 +756,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
     __builtin_amdgcn_sched_barrier(0x0f);
     fetch(r1 - r0 - (c + 1) * RC, more, b ^ 1);   // (that buffer was read last before the previous barrier)
     advance(c + 2 < chunks);
-    if constexpr (DELTA) {
+    if constexpr (DELTA && SEG != 1) {
 #pragma unroll
       for (int t = 0; t < NS; ++t)
 #pragma unroll
@@ -647,7 +771,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
       const f32x4 s0 = S[2 * t], s1 = S[2 * t + 1];
       S[2 * t] *= gc;
       S[2 * t + 1] *= gc;
-      split3(s0, s1, part[t]);
+      if constexpr (DELTA || SEG != 1) split3(s0, s1, part[t]);
       if constexpr (DELTA) {
 #pragma unroll
         for (int p = 2; p >= 0; --p)
@@ -662,17 +786,20 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
 #pragma unroll
-      for (int p = 0; p < 3; ++p) tm[rb][p] = mat(p, rb);
+      for (int p = 0; p < 3; ++p)
+        if constexpr (DELTA || SEG != 1) tm[rb][p] = mat(p, rb);
       vo[rb] = V[(DELTA ? 2 : 3) * RC + 16 * rb + col];
       vd[rb] = vec(DELTA ? 3 : 4, rb);
     }
     __builtin_amdgcn_sched_barrier(0x0f);
+    if constexpr (SEG != 1) {
 #pragma unroll
-    for (int t = 0; t < NS; ++t)
+      for (int t = 0; t < NS; ++t)
 #pragma unroll
-      for (int p = 2; p >= 0; --p)
+        for (int p = 2; p >= 0; --p)
 #pragma unroll
-        for (int rb = 0; rb < 2; ++rb) o[rb] = mma_bf16(part[t][p], qf[rb][t], o[rb]);
+          for (int rb = 0; rb < 2; ++rb) o[rb] = mma_bf16(part[t][p], qf[rb][t], o[rb]);
+    }
     f32x4 r[2], u[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb)
@@ -682,7 +809,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
         if constexpr (DELTA) r[rb][e] -= vb[rb][e] * ks[rb][e];
       }
     bf16x8 rs[3];
-    split3(r[0], r[1], rs);
+    if constexpr (DELTA || SEG != 1) split3(r[0], r[1], rs);
     __builtin_amdgcn_sched_barrier(0x0f);
     // ---- U = T R, o += (P T) R (Mamba-2: o += P U) ----
     bf16x8 ka[NB];
@@ -696,7 +823,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
       }
     }
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
+    for (int rb = 0; SEG != 1 && rb < 2; ++rb) {
       if constexpr (DELTA) {
 #pragma unroll
         for (int p = 0; p < 3; ++p) pm[rb][p] = mat(3 + p, rb);
@@ -706,9 +833,11 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
     }
     __builtin_amdgcn_sched_barrier(0x0f);
     if constexpr (DELTA) mma_parts(tm, rs, u);
+    if constexpr (SEG != 1) {
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) o[rb] *= vo[rb];
-    mma_parts<true>(DELTA ? pm : tm, rs, o);
+      for (int rb = 0; rb < 2; ++rb) o[rb] *= vo[rb];
+      mma_parts<true>(DELTA ? pm : tm, rs, o);
+    }
     // ---- S = g_C S + k^T U ----
     bf16x8 us[3];
 #pragma unroll
@@ -718,6 +847,13 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
     for (int p = 2; p >= 0; --p)
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) S[nb] = mma_bf16(ka[nb], us[p], S[nb]);
+    if constexpr (SEG == 1) {
+      if constexpr (!DELTA) decay *= gc;
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next chunk has landed
+      __syncthreads();
+      return;
+    }
     // ---- the outputs ----
     if constexpr (!DELTA) {
 #pragma unroll
@@ -747,37 +883,53 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
     step(c, 0);
     if (c + 1 < chunks) step(c + 1, 1);
   }
-  float broken = 0.f;   // NaN if a value of S is not finite
+  if constexpr (SEG == 1) {
+    if (ident) {   // M by rows: lane (col, g) holds column nc
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb)
+      for (int b = 0; b < NB; ++b)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) broken += S[nb][e] * 0.f;
-  if (live && (few || __ballot(broken != 0.f))) {
-    if (!few) start();
-    walk(r1 - r0);
+        for (int e = 0; e < 4; ++e) sg[copy + (32 * (b >> 1) + 8 * g + 4 * (b & 1) + e) * DK + nc] = S[b][e];
+    } else if (live) {
+      store(sg + mine);
+      if (!DELTA && j > 0 && tid == 0 && blockIdx.y == 0) sg[copy] = decay;
+    }
+    return;
   }
-  if (live) {
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) *reinterpret_cast<f32x4*>(st + 32 * (nb >> 1) + 4 * (nb & 1)) = S[nb];
+  if (live && (few || !finite())) {
+    if (!few) {
+      origin();
+      walk(q0, r0, false);
+    }
+    walk(r0, r1, true);
   }
+  if (live && last) store(st);
 }
 
 bool aligned16(const void* p, int64_t elems) { return ((uintptr_t)p | (uintptr_t)(elems * 2)) % 16 == 0; }
 
 template <bool DELTA>
-int launch_rule(const RuleArgs& a, int T, int dk, hipStream_t stream) {
-  const dim3 gram(T / RC + a.S, DELTA ? (a.H + 3) / 4 : a.Hk);
-  const dim3 rule(a.H, (a.dv + 63) / 64, a.S);
+int launch_rule(RuleArgs a, int T, int dk, hipStream_t stream) {
   const bool vec = aligned16(a.v, a.v_stride) && ((uintptr_t)a.out | (uintptr_t)(2 * a.out_stride)) % 8 == 0;   // (dv is a multiple of 16)
+  if (!vec) a.seg = 0;
+  a.segs = reinterpret_cast<float*>(a.ws + (int64_t)(T / RC + a.S) * ws_bytes<DELTA>(a.H, a.Hk));
+  const int cols = (a.dv + 63) / 64, ids = a.seg ? T / (RC * a.seg) + a.S : a.S;
+  if (ids > 65535) return -3;
+  const dim3 gram(T / RC + a.S, DELTA ? (a.H + 3) / 4 : a.Hk), rule(a.H, cols, ids), own(a.H, cols + (DELTA ? dk / 64 : 0), ids);
   if (dk == 128) {
     if constexpr (DELTA) chunk_gram_kernel<128><<<gram, 256, 0, stream>>>(a);
     else ssm_gram_kernel<128><<<gram, 256, 0, stream>>>(a);
-    if (vec) chunk_rule_kernel<128, DELTA, 4, true><<<rule, 256, 0, stream>>>(a);
+    if (vec && a.seg) {
+      chunk_rule_kernel<128, DELTA, 4, true, 1><<<own, 256, 0, stream>>>(a);
+      chunk_rule_kernel<128, DELTA, 4, true, 2><<<rule, 256, 0, stream>>>(a);
+    } else if (vec) chunk_rule_kernel<128, DELTA, 4, true><<<rule, 256, 0, stream>>>(a);
     else chunk_rule_kernel<128, DELTA, 4, false><<<rule, 256, 0, stream>>>(a);
   } else {
     if constexpr (DELTA) chunk_gram_kernel<64><<<gram, 256, 0, stream>>>(a);
     else ssm_gram_kernel<64><<<gram, 256, 0, stream>>>(a);
-    if (vec) chunk_rule_kernel<64, DELTA, 4, true><<<rule, 256, 0, stream>>>(a);
+    if (vec && a.seg) {
+      chunk_rule_kernel<64, DELTA, 4, true, 1><<<own, 256, 0, stream>>>(a);
+      chunk_rule_kernel<64, DELTA, 4, true, 2><<<rule, 256, 0, stream>>>(a);
+    } else if (vec) chunk_rule_kernel<64, DELTA, 4, true><<<rule, 256, 0, stream>>>(a);
     else chunk_rule_kernel<64, DELTA, 4, false><<<rule, 256, 0, stream>>>(a);
   }
   OME_CHECK_LAUNCH();
@@ -797,17 +949,20 @@ OME_API int ome_chunk_rule_floats(int H, int G, int delta) {
   return (int)((delta ? ws_bytes<true>(H, G) : ws_bytes<false>(H, G)) / 4);
 }
 
-// Gated delta rule over all rows of every sequence; operands as ome_gdn_scan.  -3: a shape, stride or
+// ... and of a head of a segment, of which there are up to T / (32 seg) + S; they come behind the chunks'
+OME_API int ome_chunk_rule_seg_floats(int dk, int dv) { return (int)seg_floats(dv, dk); }
+
+// Gated delta rule over all rows of every sequence, in segments of `seg` chunks (0: in one piece); operands as ome_gdn_scan.  -3: a shape, stride or
 // alignment that the chunked kernels do not take (nothing is launched).
 OME_API int ome_gdn_chunks(const void* q, const void* k, const void* v, int64_t qkv_stride, const void* a, const void* b,
                            int64_t ab_stride, const float* A_log, const float* dt_bias, float* state, void* out,
                            int64_t out_stride, const int* cu, const int* slot, const int* reset, int S, int T, int Hv, int Hk,
-                           int dk, int dv, float* ws, hipStream_t stream) {
-  if (T <= 0 || !ws || !rule_shape(S, Hv, Hk, dk, dv, qkv_stride, qkv_stride, out_stride) || !aligned16(q, qkv_stride) || !aligned16(k, qkv_stride) ||
+                           int dk, int dv, int seg, float* ws, hipStream_t stream) {
+  if (T <= 0 || seg < 0 || !ws || !rule_shape(S, Hv, Hk, dk, dv, qkv_stride, qkv_stride, out_stride) || !aligned16(q, qkv_stride) || !aligned16(k, qkv_stride) ||
       (uintptr_t)state % 16 || (uintptr_t)ws % 16)
     return -3;
   const RuleArgs r{(const bf16*)q, (const bf16*)k, (const bf16*)v, qkv_stride, qkv_stride, (const bf16*)a, (const bf16*)b,
-                   ab_stride, A_log, nullptr, dt_bias, 0.f, (char*)ws, state, (bf16*)out, out_stride, cu, slot, reset, S, Hv, Hk, dv};
+                   ab_stride, A_log, nullptr, dt_bias, 0.f, (char*)ws, state, (bf16*)out, out_stride, cu, slot, reset, S, Hv, Hk, dv, seg, nullptr};
   return launch_rule<true>(r, T, dk, stream);
 }
 
@@ -815,11 +970,11 @@ OME_API int ome_gdn_chunks(const void* q, const void* k, const void* v, int64_t 
 OME_API int ome_ssm_chunks(const void* x, int64_t x_stride, const void* dt, int64_t dt_stride, const void* B, const void* Cm,
                            int64_t bc_stride, const float* A, const float* D, const float* dt_bias, float dt_min, float* state,
                            void* y, int64_t y_stride, const int* cu, const int* slot, const int* reset, int S, int T, int H,
-                           int P, int N, int G, float* ws, hipStream_t stream) {
-  if (T <= 0 || !ws || !rule_shape(S, H, G, N, P, bc_stride, x_stride, y_stride) || !aligned16(B, bc_stride) || !aligned16(Cm, bc_stride) ||
+                           int P, int N, int G, int seg, float* ws, hipStream_t stream) {
+  if (T <= 0 || seg < 0 || !ws || !rule_shape(S, H, G, N, P, bc_stride, x_stride, y_stride) || !aligned16(B, bc_stride) || !aligned16(Cm, bc_stride) ||
       (uintptr_t)state % 16 || (uintptr_t)ws % 16)
     return -3;
   const RuleArgs r{(const bf16*)Cm, (const bf16*)B, (const bf16*)x, bc_stride, x_stride, (const bf16*)dt, nullptr,
-                   dt_stride, A, D, dt_bias, dt_min, (char*)ws, state, (bf16*)y, y_stride, cu, slot, reset, S, H, G, P};
+                   dt_stride, A, D, dt_bias, dt_min, (char*)ws, state, (bf16*)y, y_stride, cu, slot, reset, S, H, G, P, seg, nullptr};
   return launch_rule<false>(r, T, N, stream);
 }

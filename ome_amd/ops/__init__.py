@@ -171,6 +171,28 @@ def _chunk_rule_floats(H: int, G: int, delta: bool) -> int:
     return load().ome_chunk_rule_floats(H, G, int(delta))
 
 
+@functools.lru_cache(maxsize=256)
+def _chunk_rule_seg_floats(dk: int, dv: int) -> int:
+    return load().ome_chunk_rule_seg_floats(dk, dv)
+
+
+def _chunk_rule_seg(T: int, S: int, H: int, dv: int, delta: bool) -> int:
+    """Chunks of a segment, or 0 where sequences run in one piece.  A chunk is 1.7 us of a serial chain and the chip holds 512 workgroups:
+    where the sequences have far fewer, segments of them run side by side.  For that every segment but the last is walked once
+    more for its own state and (delta rule) transition, at 0.4 (1.4) of its cost, and a segment's start takes a step of
+    1 (2.5) us over each one before it; hence lengths near sqrt(chunks), longer where those fill the chip.  Whole layers in us, one
+    piece -> segments, sequences x rows in all (average chunks a sequence):
+    delta rule, 8 heads 1 x 1000 87 -> 76, 1 x 4000 259 -> 127, 1 x 8000 489 -> 190, 2 x 4000 220 -> 120, 4 x 4000 113 -> 99; 32 heads
+    1 x 1000 96 -> 91, 1 x 4000 299 -> 218, 2 x 4000 (128 workgroups) 243 -> 245; 1 x 300 46 -> 50;
+    selective scan, 32 heads 1 x 1000 81 -> 55, 1 x 8000 435 -> 136, 4 x 4000 116 -> 92, 8 x 8000 (256) 130 -> 145; 128 heads
+    1 x 1000 95 -> 84, 1 x 8000 638 -> 440, 2 x 4000 (256) 220 -> 225; 1 x 300 42 -> 44."""
+    wgs, chunks = H * -(-dv // 64) * S, -(-T // (32 * S))
+    if chunks < 24 or wgs > (64 if delta else 192):
+        return 0
+    pieces = chunks / max(8, 1.3 * chunks ** 0.5, chunks * wgs / (256 if delta else 512))
+    return -(-chunks // max(2, round(pieces)))
+
+
 def _chunk_rule_ws(T: int, S: int, H: int, G: int, dk: int, dv: int, delta: bool, state: torch.Tensor, rows: tuple) -> torch.Tensor | None:
     """Workspace of the chunked kernels (``chunk_rule.hip``) for T rows of S sequences and H heads, or None
     where the row-by-row kernels run: one row per sequence (a decode step; a chunk would be 1/32 full), few rows in all, key
@@ -190,7 +212,11 @@ def _chunk_rule_ws(T: int, S: int, H: int, G: int, dk: int, dv: int, delta: bool
     if (state.data_ptr() | q.data_ptr() | k.data_ptr()) % 16 or sq % 8 or not (0 <= sq < 1 << 24 and 0 <= so < 1 << 24) or \
             not 0 <= rows[-2].stride(0) < 1 << 24 or o.data_ptr() == rows[-2].data_ptr():
         return None
-    return torch.empty((T // 32 + S) * _chunk_rule_floats(H, G, delta), dtype=torch.float32, device=state.device)
+    floats = (T // 32 + S) * _chunk_rule_floats(H, G, delta)
+    seg = _chunk_rule_seg(T, S, H, dv, delta)
+    if seg:
+        floats += (T // (32 * seg) + S) * H * _chunk_rule_seg_floats(dk, dv)
+    return torch.empty(floats, dtype=torch.float32, device=state.device)
 
 
 def ssm_scan(x, dt, B, C, A, D, dt_bias, dt_min: float, state, cu, slot, reset, H: int, P: int, N: int, G: int,
@@ -208,7 +234,7 @@ def ssm_scan(x, dt, B, C, A, D, dt_bias, dt_min: float, state, cu, slot, reset, 
         call("ome_ssm_chunks", x.data_ptr(), x.stride(0), dt.data_ptr(), dt.stride(0), B.data_ptr(), C.data_ptr(),
              B.stride(0), A.data_ptr(), D.data_ptr(), dt_bias.data_ptr(), float(dt_min), state.data_ptr(), out.data_ptr(),
              out.stride(0), _i32(cu).data_ptr(), _i32(slot).data_ptr(), _i32(reset).data_ptr(), slot.shape[0], T, H, P, N,
-             G, ws.data_ptr(), stream_ptr())
+             G, _chunk_rule_seg(T, slot.shape[0], H, P, False), ws.data_ptr(), stream_ptr())
         return out
     call("ome_ssm_scan", x.data_ptr(), x.stride(0), dt.data_ptr(), dt.stride(0), B.data_ptr(), C.data_ptr(),
          B.stride(0), A.data_ptr(), D.data_ptr(), dt_bias.data_ptr(), float(dt_min), state.data_ptr(),
@@ -239,8 +265,8 @@ def gdn_scan(q, k, v, a, b, A_log, dt_bias, state, cu, slot, reset, Hv: int, Hk:
     if ws is not None:   # prompts: chunks of 32 rows on the matrix cores
         call("ome_gdn_chunks", q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), a.data_ptr(), b.data_ptr(),
              a.stride(0), A_log.data_ptr(), dt_bias.data_ptr(), state.data_ptr(), out.data_ptr(), out.stride(0),
-             _i32(cu).data_ptr(), _i32(slot).data_ptr(), _i32(reset).data_ptr(), slot.shape[0], T, Hv, Hk, dk, dv,
-             ws.data_ptr(), stream_ptr())
+             _i32(cu).data_ptr(), _i32(slot).data_ptr(), _i32(reset).data_ptr(), S, T, Hv, Hk, dk, dv,
+             _chunk_rule_seg(T, S, Hv, dv, True), ws.data_ptr(), stream_ptr())
         return out
     if T == S and not v1 and not f32 and dk in (64, 128, 256) and 0 < Hv <= 65535 and Hk > 0 and Hv % Hk == 0 and \
             q.data_ptr() % 16 == 0 and k.data_ptr() % 16 == 0 and q.stride(0) % 8 == 0 and 0 < dv < 1 << 20:

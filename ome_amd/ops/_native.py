@@ -94,10 +94,11 @@ _SIGNATURES = {
                          i32, vp, i32, vp],
         "ome_gdn_step": [vp, vp, vp, i64, vp, vp, i64, vp, vp, vp, vp, i64, vp, vp, vp, i32, i32, i32, i32, i32, vp],
         "ome_chunk_rule_floats": [i32, i32, i32],
-        "ome_gdn_chunks": [vp, vp, vp, i64, vp, vp, i64, vp, vp, vp, vp, i64, vp, vp, vp, i32, i32, i32, i32, i32, i32, vp,
-                           vp],
+        "ome_gdn_chunks": [vp, vp, vp, i64, vp, vp, i64, vp, vp, vp, vp, i64, vp, vp, vp, i32, i32, i32, i32, i32, i32, i32,
+                           vp, vp],
+        "ome_chunk_rule_seg_floats": [i32, i32],
         "ome_ssm_chunks": [vp, i64, vp, i64, vp, vp, i64, vp, vp, vp, f32, vp, vp, i64, vp, vp, vp, i32, i32, i32, i32,
-                           i32, i32, vp, vp],
+                           i32, i32, i32, vp, vp],
         "ome_gated_rmsnorm": [vp, i64, vp, i64, vp, vp, i64, i32, i32, i32, f32, i32, i32, vp],
         "ome_layernorm": [vp, i64, vp, i64, vp, vp, vp, i64, i32, i32, f32, vp],
         "ome_embedding": [vp, vp, vp, i32, i32, i32, i32, vp],

@@ -281,3 +281,78 @@ def test_few_rows_take_the_row_by_row_kernels():
     for delta, few in ((True, 32), (False, 4)):
         assert ws(few, 1, delta) is None and ws(few, 2, delta) is None and ws(40, 40, delta) is None
         assert ws(few + 1, 1, delta) is not None and ws(41, 40, delta) is not None
+
+
+# segments of one chunk and more, whole and not, beside sequences of one segment, a few rows and none
+@pytest.mark.parametrize("seg", [1, 2, 3])
+@pytest.mark.parametrize("lens", [[97], [3, 0, 64, 65], [32, 160, 1, 96], [33, 2, 129]], ids=str)
+@pytest.mark.parametrize("delta", [True, False])
+def test_scans_in_segments(lens, seg, delta, monkeypatch):
+    monkeypatch.setattr(ops, "_chunk_rule_seg", lambda *a: seg)
+    if delta:
+        for dims in ((128, 128, 2, 4, 8), (64, 16, 1, 5, 0), (128, 80, 3, 3, 8), (64, 128, 2, 2, 8)):
+            test_delta_rule_prompts(lens, *dims)
+    else:
+        for dims in ((16, 64, 128, 2, 8), (3, 16, 64, 1, 0), (5, 80, 128, 5, 8), (2, 144, 64, 2, 8)):
+            test_selective_scan_prompts(lens, *dims)
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
+@pytest.mark.parametrize("what", ["q", "k", "v", "a", "b"])
+def test_delta_rule_in_segments_stays_causal(what, bad, monkeypatch):
+    monkeypatch.setattr(ops, "_chunk_rule_seg", lambda *a: 1)
+    test_delta_rule_stays_causal(what, bad)
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
+@pytest.mark.parametrize("what", ["B", "C", "x", "dt"])
+def test_selective_scan_in_segments_stays_causal(what, bad, monkeypatch):
+    monkeypatch.setattr(ops, "_chunk_rule_seg", lambda *a: 1)
+    test_selective_scan_stays_causal(what, bad)
+
+
+@pytest.mark.parametrize("what", ["k", "v", "a", "b", "state"])
+def test_not_finite_in_segments_as_in_one_piece(what, monkeypatch):
+    """What follows a value that is not finite, over several segments: the same infinities and NaN."""
+    torch.manual_seed(3)
+    T, dk, dv, H = 200, 64, 32, 2
+    c, ab = torch.randn(T, H * (2 * dk + dv), device=DEV).to(BF), torch.randn(T, 2 * H, device=DEV).to(BF)
+    q, k, v, a, b = c[:, :H * dk], c[:, H * dk:2 * H * dk], c[:, 2 * H * dk:], ab[:, :H], ab[:, H:]
+    st = torch.randn(1, H, dv, dk, device=DEV)
+    (st[0, 0, 5] if what == "state" else {"k": k, "v": v, "a": a, "b": b}[what][70])[1] = float("inf")
+    got = []
+    for seg in (0, 1, 2):
+        monkeypatch.setattr(ops, "_chunk_rule_seg", lambda *x, seg=seg: seg)
+        s = st.clone()
+        o = ops.gdn_scan(q, k, v, a, b, torch.zeros(H, device=DEV), torch.zeros(H, device=DEV), s, i32([0, T]), i32([0]), i32([0]), H, H)
+        got.append((o.float(), s))
+    for o, s in got[1:]:
+        for x, y in ((o, got[0][0]), (s, got[0][1])):
+            assert torch.equal(x.isnan(), y.isnan()) and torch.equal(x.isinf(), y.isinf())
+            assert torch.allclose(x[y.isfinite()], y[y.isfinite()], rtol=2.0 ** -7, atol=1e-4)
+
+
+@pytest.mark.parametrize("delta", [True, False])
+def test_segments_are_as_exact_as_one_piece(delta, monkeypatch):
+    """A long prompt of few heads, which the rule cuts, against 64 bits."""
+    torch.manual_seed(11)
+    T, H, dk, dv, errors = 1700, 2, 128, 64, []
+    rule = ops._chunk_rule_seg
+    assert rule(T, 1, H, dv, delta) > 0
+    c, ab = torch.randn(T, 2 * H * dk + H * dv, device=DEV).to(BF), torch.randn(T, 2 * H, device=DEV).to(BF)
+    q, k, v = c[:, :H * dk], c[:, H * dk:2 * H * dk], c[:, 2 * H * dk:]
+    slow, sq = torch.linspace(-9, -6, H, device=DEV), (i32([0, T]), i32([0]), i32([0]))   # decays that a state outlives
+    st, zero = torch.randn(1, H, dv, dk, device=DEV) * 0.2, torch.zeros(H, device=DEV)
+    if delta:
+        args, tail, scan, exact = (q, k, v, ab[:, :H], ab[:, H:], slow, zero), (H, H), ops.gdn_scan, exact_gdn
+    else:
+        args, tail, scan, exact = (v, ab[:, :H], k, q, -slow.exp(), zero, zero, 0.001), (H, dv, dk, H), ops.ssm_scan, exact_ssm
+    want, want_state = exact(*args, st, *sq, *tail)
+    for f in (lambda *a: 0, rule):
+        monkeypatch.setattr(ops, "_chunk_rule_seg", f)
+        s = st.clone()
+        o = scan(*args, s, *sq, *tail)
+        assert near(o, s, want, want_state)
+        errors.append(((s.cpu().double() - want_state).norm() / want_state.norm()).item())
+    print("state, one piece and segments:", errors)
+    assert errors[1] <= 1.25 * errors[0]   # (another order of the same sums)
