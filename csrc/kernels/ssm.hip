@@ -29,18 +29,26 @@ namespace {
 typedef float f32v4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float softplus_f(float x) { return x > 20.f ? x : log1pf(__expf(x)); }
-__device__ __forceinline__ float silu_f(float x) { return x / (1.f + __expf(-x)); }
+// x / (1 + e^-x): a quarter of both (so that the reciprocal of no finite denominator is subnormal), the reciprocal and the quotient
+// with a Newton step each: eight instructions for the compiler's division's eleven, and the same bf16 for every bf16 x
+__device__ __forceinline__ float silu_f(float x) {
+  const float n = 0.25f * x, d = __builtin_fmaf(__expf(-x), 0.25f, 0.25f), r0 = __builtin_amdgcn_rcpf(d);
+  const float r = __builtin_fmaf(__builtin_fmaf(-d, r0, 1.f), r0, r0), q = n * r;
+  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, n), r, q), d, n);   // (infinities and NaN)
+}
 
 // Causal depthwise conv + SiLU, K <= 6 taps.  Not recurrent, so rows are parallel: a wave owns 64 * V
 // neighbouring channels (V = 8: 16-byte row pieces) of a tile of CT rows and slides a register window over
-// them, CT / 2 rows of loads in flight.  Tiles belong to sequences: sequence s owns tile ids cu[s] / CT + s and
+// them, CR rows computed while the next CR are on their way.  Tiles belong to sequences: sequence s owns tile ids cu[s] / CT + s and
 // up (never overlapping, below T / CT + S).  Only a sequence's first tile touches the state (K - 1 <= CT): it
 // reads the old tail before its rows and writes the new one, from the sequence's last rows or, where it is
 // shorter than K - 1, from the old tail shifted; no other tile races with it.  `by_seq` (decode steps, no more
 // rows than sequences): wave id = sequence, all its rows, without the search.  `out` must not overlap `x`.
-// Memory-bound: 4000 rows x 8192 channels 521 -> 32 us (one thread per channel walked its sequence before:
-// 96 waves of dependent 2-byte loads), 64 decode rows 6.0 -> 6.1 us.
-constexpr int CT = 16;
+// Memory-bound where rows are many, a wave's chain where they are few, so tiles are short (they read K - 1 rows again, from L2):
+// 16 rows in two halves without a load ahead -> with one -> 8 rows in halves of 4 and the quotient of silu_f, us: 4000 x 8192 31 -> 34 ->
+// 27.6 (4.8 TB/s), 3500 x 10240 35 -> 38 -> 29, 8000 x 2560 24.5 -> 28 -> 21, 1000 x 8192 17.9 -> 16.6 -> 10.2, 300 x 10240 11.7 -> 9.8 ->
+// 7.8; 32 rows a tile 33, 43, 31, 17, 15.
+constexpr int CT = 8, CR = 4;
 
 template <int K, int V>
 __global__ __launch_bounds__(256) void ssm_conv1d_kernel(const bf16* __restrict__ x, int64_t x_stride,
@@ -118,12 +126,14 @@ __global__ __launch_bounds__(256) void ssm_conv1d_kernel(const bf16* __restrict_
       for (int u = 0; u < V; ++u) win[t][u] = (float)v[u];
     }
   }
-  for (int r = a; r < e; r += CT / 2) {
-    vec xs[CT / 2];
+  vec xs[2][CR];   // rows on their way while the ones before them are computed
+  const auto fetch = [&](vec (&to)[CR], int r) {
 #pragma unroll
-    for (int i = 0; i < CT / 2; ++i) xs[i] = *reinterpret_cast<const vec*>(x + (int64_t)min(r + i, e - 1) * x_stride + c);
+    for (int i = 0; i < CR; ++i) to[i] = *reinterpret_cast<const vec*>(x + (int64_t)min(r + i, e - 1) * x_stride + c);
+  };
+  const auto rows = [&](const vec (&xs)[CR], int r) {
 #pragma unroll
-    for (int i = 0; i < CT / 2; ++i) {
+    for (int i = 0; i < CR; ++i) {
       if (r + i >= e) break;
       vec o;
 #pragma unroll
@@ -139,6 +149,14 @@ __global__ __launch_bounds__(256) void ssm_conv1d_kernel(const bf16* __restrict_
       }
       *reinterpret_cast<vec*>(out + (int64_t)(r + i) * out_stride + c) = o;
     }
+  };
+  fetch(xs[0], a);
+  for (int r = a; r < e; r += 2 * CR) {
+    if (r + CR < e) fetch(xs[1], r + CR);
+    rows(xs[0], r);
+    if (r + CR >= e) break;
+    if (r + 2 * CR < e) fetch(xs[0], r + 2 * CR);
+    rows(xs[1], r + CR);
   }
 }
 
@@ -294,7 +312,7 @@ __global__ __launch_bounds__(256) void gated_rmsnorm_kernel(const T* __restrict_
 // bf16 groups of 8 L N channels (L = 8 .. 64 lanes, N passes), every mode: a lane holds N 16-byte pieces of y and
 // z, so each is read once, and a group's sum of squares stays within its L lanes (no LDS, no barrier; the block-wide
 // kernel above read y twice, in 2-byte pieces, behind two barriers).  Memory-bound: 4000 x 4096 in groups of 128
-// 104 -> 21 us, 3500 x 8192 in groups of 1024 116 -> 45 us.
+// 104 -> 21 us, 3500 x 8192 in groups of 1024 116 -> 29 (42 with the gate computed once for the sum and once for the output).
 template <int L, int N>
 __global__ __launch_bounds__(256) void gated_rmsnorm_vec_kernel(const bf16* __restrict__ y, int64_t y_stride,
                                                                 const bf16* __restrict__ z, int64_t z_stride,
@@ -314,13 +332,13 @@ __global__ __launch_bounds__(256) void gated_rmsnorm_vec_kernel(const bf16* __re
     yv[p] = ld8(y + row * y_stride + i);
     zv[p] = ld8(z + row * z_stride + i);
   }
-  float ss = 0.f;
+  float ss = 0.f, v[N][8];   // what is normalised
 #pragma unroll
   for (int p = 0; p < N; ++p)
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const float v = norm_first ? (float)yv[p][e] : (float)yv[p][e] * silu_f((float)zv[p][e]);
-      ss += v * v;
+      v[p][e] = norm_first ? (float)yv[p][e] : (float)yv[p][e] * silu_f((float)zv[p][e]);
+      ss += v[p][e] * v[p][e];
     }
 #pragma unroll
   for (int o = L / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
@@ -332,14 +350,12 @@ __global__ __launch_bounds__(256) void gated_rmsnorm_vec_kernel(const bf16* __re
     bf16x8 o;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const float yy = (float)yv[p][e], zz = (float)zv[p][e], ww = (float)wv[e];
-      if (exact) {
-        const float zs = sig ? 1.f / (1.f + __expf(-zz)) : silu_f(zz);
-        o[e] = (bf16)(norm_first ? yy * rs * ww * zs : yy * zs * rs * ww);
-      } else if (norm_first) {
-        o[e] = (bf16)((float)(bf16)((float)(bf16)(yy * rs) * ww) * silu_f(zz));
+      const float vv = v[p][e], zz = (float)zv[p][e], ww = (float)wv[e];
+      if (norm_first) {
+        if (exact) o[e] = (bf16)(vv * rs * ww * (sig ? 1.f / (1.f + __expf(-zz)) : silu_f(zz)));
+        else o[e] = (bf16)((float)(bf16)((float)(bf16)(vv * rs) * ww) * silu_f(zz));
       } else {
-        o[e] = (bf16)((float)(bf16)(yy * silu_f(zz) * rs) * ww);
+        o[e] = (bf16)(exact ? vv * rs * ww : (float)(bf16)(vv * rs) * ww);
       }
     }
     st8(out + row * out_stride + g0 + i, o);

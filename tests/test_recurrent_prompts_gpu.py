@@ -356,3 +356,15 @@ def test_segments_are_as_exact_as_one_piece(delta, monkeypatch):
         errors.append(((s.cpu().double() - want_state).norm() / want_state.norm()).item())
     print("state, one piece and segments:", errors)
     assert errors[1] <= 1.25 * errors[0]   # (another order of the same sums)
+
+
+def test_silu_of_every_value():
+    """The convolution's SiLU for all bf16 inputs, infinities and NaN among them: the value in 64 bits, rounded (one tap of 1, each
+    row a sequence).  Where e^-x is past fp32 (x < -88.72) it is 0."""
+    x = torch.arange(1 << 16, dtype=torch.int32).to(torch.int16).view(BF).view(256, 256).to(DEV)
+    w = torch.zeros(256, 4, dtype=BF, device=DEV)
+    w[:, 3] = 1
+    y = ops.ssm_conv1d(x, w, None, torch.zeros(256, 256, 3, dtype=BF, device=DEV), i32(list(range(257))), i32(list(range(256))), i32([1] * 256))
+    want = (x.double() / (1 + (-x.double()).exp())).to(BF)
+    want[(x < -88.72) & x.isfinite()] = 0
+    assert bool(((y == want) | (y.isnan() & want.isnan())).all())
