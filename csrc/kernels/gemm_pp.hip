@@ -289,7 +289,13 @@ __global__ __launch_bounds__(PP_NT, 1) void gemm_pp_kernel(const bf16* __restric
 // image interleaves 16 gate rows with their 16 up rows (gate rows [0, N / 2), up rows [N / 2, N) of
 // the expert), so SiLU(gate) * up is formed in the accumulators: no [rows, N] intermediate, no second pass.
 // Bound by the matrix cores: 6000 rows of 8 experts, 28672 x 4096 and 4096 x 14336, took 3.5 ms (590 TFLOP/s: 128-row
-// tiles staged through registers, one barrier per 32 of K) and take 2.0 ms (1035).
+// tiles staged through registers, one barrier per 32 of K) and took 2.02 ms (1046) with every tile multiplied whole.  The rows go to
+// the waves in 16s (row 64 j + 16 wi + i of a tile is wave wi's, block j), so that the four 64-row quarters of a tile are
+// equal work on every SIMD, and a tile multiplies only the quarters that have rows; the absent rows lie past the descriptor and are
+// not fetched either.  Whole layers, before -> after, us: 8 experts of 4096 x 14336 with 750 rows each 2018 -> 1960 (the down
+// projection's two waves of tiles stay two), 250 989 -> 933, 85 765 -> 708; 128 experts of 2688 x 1856, 141 rows 837 -> 796, 94 754 -> 700.
+// Tried and slower: weights read once with the non-temporal policy (708 -> 746, 1960 -> 2084); equal: panels that
+// start at different places in K.
 // ------------------------------------------------------------------------------------------
 struct PpGroups {
   const int *ids, *offsets;   // ids: null = sorted order
@@ -348,7 +354,7 @@ __global__ __launch_bounds__(PP_NT, 1) void moe_pp_kernel(const bf16* __restrict
       const int blk = wi * 4 + (p & 3);
       prow[p] = (blk & 8) * 16 + (blk & 7) * 8 + (p >> 2) * 64;
     } else {
-      prow[p] = wi * 64 + p * 8;
+      prow[p] = (p >> 2) * 128 + wi * 32 + (p & 3) * 8;   // (the first phase reads rows 0 .. 127)
     }
     const int row = prow[p] + (lane >> 3);
     const int chunk = pp_swz(row, lane & 7);
@@ -362,9 +368,9 @@ __global__ __launch_bounds__(PP_NT, 1) void moe_pp_kernel(const bf16* __restrict
       }
     } else {
       const int rr = min(m0 + row, m_end - 1);
-      src = (int64_t)(grp.ids != nullptr ? grp.ids[rr] / grp.div : rr) * ldx;
+      src = m0 + row < m_end ? (int64_t)(grp.ids != nullptr ? grp.ids[rr] / grp.div : rr) * ldx : (int64_t)1 << 30;
     }
-    vo[p] = (uint32_t)(src * 2 + chunk * 16);
+    vo[p] = (uint32_t)(src * 2 + chunk * 16);   // (absent rows: past the descriptor, zeros that nothing fetches)
   }
   auto dma = [&](int t, int buf, int p0, int np) {
     char* base = smem + buf * PP_BUF + img_off;
@@ -384,23 +390,62 @@ __global__ __launch_bounds__(PP_NT, 1) void moe_pp_kernel(const bf16* __restrict
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) wf[i][kk] = pp_frag(img, g * 128 + (i0 + i) * 16 + fr, kk * 4 + fc);
   };
-  auto rd_x = [&](bf16x8 (&xf)[2][2], const char* img, int j0) {
+  // NJ: how many 64-row quarters of the tile have rows.  A quarter without any is neither read nor multiplied; barriers, moves and
+  // waits stay those of gemm_pp_kernel
+  const auto run = [&](auto nj_tag) {
+    constexpr int NJ = decltype(nj_tag)::value, JA = NJ < 2 ? NJ : 2, JB = NJ - JA;
+    const auto rd_x = [&](bf16x8 (&xf)[2][2], const char* img, int j0, auto n_tag) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < decltype(n_tag)::value; ++j)
 #pragma unroll
-      for (int kk = 0; kk < 2; ++kk) xf[j][kk] = pp_frag(img, wi * 64 + (j0 + j) * 16 + fr, kk * 4 + fc);
-  };
-  auto mma = [&](const bf16x8 (&xf)[2][2], int i0, int j0) {
-    __builtin_amdgcn_s_setprio(1);
+        for (int kk = 0; kk < 2; ++kk) xf[j][kk] = pp_frag(img, (j0 + j) * 64 + wi * 16 + fr, kk * 4 + fc);
+    };
+    const auto mma = [&](const bf16x8 (&xf)[2][2], int i0, int j0, auto n_tag) {
+      if constexpr (decltype(n_tag)::value > 0) {
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
+        for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+          for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i0 + i][j0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i][kk], xf[j][kk], acc[i0 + i][j0 + j],
-                                                                       0, 0, 0);
-    __builtin_amdgcn_s_setprio(0);
+            for (int j = 0; j < decltype(n_tag)::value; ++j)
+              acc[i0 + i][j0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i][kk], xf[j][kk], acc[i0 + i][j0 + j], 0, 0, 0);
+        __builtin_amdgcn_s_setprio(0);
+      }
+    };
+    const std::integral_constant<int, JA> ja{};
+    const std::integral_constant<int, JB> jb{};
+#pragma unroll 1
+    for (int t = 0; t < kt; ++t) {
+      const char* img_w = smem + (t & 1) * PP_BUF;
+      const char* img_x = img_w + PP_IMG;
+      const bool nxt = t >= 1 && t + 1 < kt;
+      if (t + 1 < kt)
+        asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      rd_w(img_w, 0);
+      rd_x(xa, img_x, 0, ja);
+      if (nxt) dma(t + 1, (t + 1) & 1, 2, 2);
+      pp_bar_lgkm();
+      mma(xa, 0, 0, ja);
+      pp_bar();
+      rd_x(xb, img_x, 2, jb);
+      if (nxt) dma(t + 1, (t + 1) & 1, 4, 2);
+      pp_bar_lgkm();
+      mma(xb, 0, 2, jb);
+      pp_bar();
+      rd_w(img_w, 4);
+      if (nxt) dma(t + 1, (t + 1) & 1, 6, 2);
+      pp_bar_lgkm();
+      mma(xb, 4, 2, jb);
+      pp_bar();
+      asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+      if (t + 2 < kt) dma(t + 2, t & 1, 0, 2);
+      pp_bar_lgkm();
+      mma(xa, 4, 0, ja);
+      pp_bar();
+    }
   };
 
   // prologue, schedule and waits of gemm_pp_kernel
@@ -409,41 +454,19 @@ __global__ __launch_bounds__(PP_NT, 1) void moe_pp_kernel(const bf16* __restrict
   asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
   pp_bar();
   if (g == 1) pp_bar();
-#pragma unroll 1
-  for (int t = 0; t < kt; ++t) {
-    const char* img_w = smem + (t & 1) * PP_BUF;
-    const char* img_x = img_w + PP_IMG;
-    const bool nxt = t >= 1 && t + 1 < kt;
-    if (t + 1 < kt)
-      asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
-    else
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    rd_w(img_w, 0);
-    rd_x(xa, img_x, 0);
-    if (nxt) dma(t + 1, (t + 1) & 1, 2, 2);
-    pp_bar_lgkm();
-    mma(xa, 0, 0);
-    pp_bar();
-    rd_x(xb, img_x, 2);
-    if (nxt) dma(t + 1, (t + 1) & 1, 4, 2);
-    pp_bar_lgkm();
-    mma(xb, 0, 2);
-    pp_bar();
-    rd_w(img_w, 4);
-    if (nxt) dma(t + 1, (t + 1) & 1, 6, 2);
-    pp_bar_lgkm();
-    mma(xb, 4, 2);
-    pp_bar();
-    asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-    if (t + 2 < kt) dma(t + 2, t & 1, 0, 2);
-    pp_bar_lgkm();
-    mma(xa, 4, 0);
-    pp_bar();
-  }
+  const int rows = __builtin_amdgcn_readfirstlane(m_end - m0);
+  if (rows > 192)
+    run(std::integral_constant<int, 4>{});
+  else if (rows > 128)
+    run(std::integral_constant<int, 3>{});
+  else if (rows > 64)
+    run(std::integral_constant<int, 2>{});
+  else
+    run(std::integral_constant<int, 1>{});
 
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const int m = m0 + wi * 64 + j * 16 + fr;
+    const int m = m0 + j * 64 + wi * 16 + fr;
     if (m < m_end) {
       if constexpr (EPI == PP_SILU) {
 #pragma unroll

@@ -420,7 +420,7 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(const bf16* __restrict__ 
 // ------------------------------------------------------------------------------------------
 // grouped GEMM v2: 128 x 128 tiles, 2x2 waves, a BK k-step staged through DOUBLE-buffered LDS: the next step's global
 // loads are issued before this step's MFMAs and written to the other buffer after them, so one barrier per k-step.  Some 60 rows
-// per expert and more (fewer: moe_stream_kernel; 80 and more, and shapes that its tiles take: gemm_pp.hip).
+// per expert and more (fewer: moe_stream_kernel; 46 and more, and shapes that its tiles take: gemm_pp.hip).
 // ------------------------------------------------------------------------------------------
 template <int BM, int BN, int BK>
 __global__ __launch_bounds__(256) void moe_gemm_v2_kernel(const bf16* __restrict__ A, int64_t lda,

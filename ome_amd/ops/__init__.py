@@ -747,9 +747,9 @@ def moe_route(logits: torch.Tensor, k: int, renorm: bool = True, scoring: str = 
 
 
 def moe_tile_m(rows: int, E: int, N: int) -> int:
-    """Row tile of the grouped GEMM (static in the shapes, so graph-safe): 128 x 128 when experts get many rows (prefill:
-    MFMA-bound), or some 60 with >= 1024 workgroups of 128; else the 64-row tiles that stream the weights.  Whole layer, 64-row /
-    128-row tiles: Mixtral 55 rows an expert 689 / 713 us, 65 770 / 722; Qwen3-Next 49 802 / 887, 59 855 / 928;
+    """Row tile of the grouped GEMM where the 256-row tiles do not run (:func:`_moe_pp`; static in the shapes, so graph-safe): 128 x
+    128 when experts get many rows (prefill: MFMA-bound), or some 60 with >= 1024 workgroups of 128; else the 64-row tiles that
+    stream the weights.  Whole layer, 64-row / 128-row tiles: Mixtral 55 rows an expert 689 / 713 us, 65 770 / 722; Qwen3-Next 49 802 / 887, 59 855 / 928;
     Nemotron-3-Nano 61 661 / 645.  ``OME_MOE_TILE`` overrides."""
     env = os.environ.get("OME_MOE_TILE")
     if env:
@@ -760,10 +760,11 @@ def moe_tile_m(rows: int, E: int, N: int) -> int:
     return 64
 
 
-#: average rows per expert from which the 256-row ping-pong tiles run (:func:`_moe_pp`).  Whole layer, 64 / 128-row
-#: tiles -> these: Mixtral 64 rows 790 -> 798 us, 100 800 -> 770, 128 983 -> 775, 250 1429 -> 1018, 750 3529 ->
-#: 2042; Nemotron-3-Nano (widths 2688 / 1856) 94 780 -> 689, 140 975 -> 829; Qwen3-Next 59 953 -> 924.
-MOE_PP_ROWS = 80
+#: average rows per expert from which the 256-row ping-pong tiles run (:func:`_moe_pp`): where experts begin to need a second
+#: 64-row tile.  Whole layer, 64 / 128-row tiles -> these, us: Mixtral 40 rows 603 -> 642, 45 615 -> 671, 48 702 -> 695, 55 760 -> 696, 75
+#: 756 -> 709, 125 1093 -> 744; Nemotron-3-Nano (widths 2688 / 1856) 42 578 -> 588, 47 602 -> 597, 61 684 -> 628; Qwen3-Next (512
+#: experts) 20 661 -> 659, 39 754 -> 730, 59 860 -> 785.
+MOE_PP_ROWS = 46
 
 
 class _Sorted:

@@ -91,6 +91,14 @@ def test_moe_prompt_tiles(monkeypatch, counts, H, I, kind):
     assert torch.isfinite(got).all()
 
 
+@pytest.mark.parametrize("rows", [1, 64, 65, 128, 129, 192, 193, 256])
+def test_moe_prompt_tile_quarters(monkeypatch, rows):
+    """256-row tiles multiply the 64-row quarters that have rows: both sides of each quarter's edge, in an expert's only tile and
+    in its second one, with one K step and with several."""
+    for H, I in ((64, 64), (192, 224)):
+        test_moe_prompt_tiles(monkeypatch, [rows, 256 + rows, 0, 3], H, I, "silu")
+
+
 @pytest.mark.parametrize("E,k", [(1, 1), (64, 64), (65, 3), (200, 70), (512, 10)])
 def test_moe_route_picks_in_order(E, k):
     """Ties go to the lower expert, zeros of both signs are ties, minus infinity comes last, NaN never (an expert
