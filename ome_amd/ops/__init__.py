@@ -1562,19 +1562,31 @@ def _sk_table() -> dict:
 
 def gemm_sk_plan(M: int, N: int, K: int, epi: int = 0) -> tuple[int, int, int] | None:
     """(bn, nwg, bm) when the stream-K kernel was measured faster than hipBLASLt (gate_up: than
-    hipBLASLt + act_and_mul) for this weight shape at the nearest measured row count, else None.
-    Table: ``ome_amd/_tuned/gemm_sk_gfx950.json`` written by ``scripts/gemm_sk_bench.py --table``
+    hipBLASLt + act_and_mul) for this weight shape at the nearest measured row count, else None.  The kernel's time
+    goes by its row tiles, so a row count of as many tiles speaks first (beyond 128 rows up to twice as far, and there only
+    where the kernel won by a tenth), and one of fewer only with its time taken times the tiles, the library's times the rows: 28672 x
+    4096 with 300 rows, two tiles, by the 256 rows' measurement 118 us, the library with its activation 82; 6144 x 4096 with
+    300 37 and 29; 4096 x 14336 with 264 by the 384 rows' plan 60 instead of 68.  Table: ``ome_amd/_tuned/gemm_sk_gfx950.json`` written by ``scripts/gemm_sk_bench.py --table``
     (cold weights, interleaved same-box timings)."""
     if _SK_MODE == "0":
         return None
     rows = _sk_table().get(f"{N},{K},{epi}")
     if not rows:
         return None
-    m_near, e = min(rows, key=lambda r: abs(r[0] - M) / max(r[0], M))
-    if max(m_near, M) > 1.34 * min(m_near, M):   # nothing measured close to this M
+
+    def tiles(m, e):
+        return -(-m // int(e.get("bm", 256)))
+
+    def near(r, far):
+        return max(r[0], M) <= far * min(r[0], M)
+
+    close = [r for r in rows if near(r, 1.34 if M <= 128 else 2) and tiles(*r) == tiles(M, r[1])] or [r for r in rows if near(r, 1.34)]
+    if not close:   # nothing measured close to this M
         return None
+    m, e = min(close, key=lambda r: abs(r[0] - M) / max(r[0], M))
     bm = int(e.get("bm", 256))
-    if e["us"] >= 0.97 * e["lib_us"] or not gemm_sk_ok(M, N, K, e["bn"], e["nwg"], bm):
+    us, lib_us = e["us"] * max(1.0, tiles(M, e) / tiles(m, e)), e["lib_us"] * (max(1.0, M / m) if tiles(M, e) > tiles(m, e) else 1.0)
+    if us >= (0.97 if near((m, e), 1.34) else 0.9) * lib_us or not gemm_sk_ok(M, N, K, e["bn"], e["nwg"], bm):
         return None
     return e["bn"], e["nwg"], bm
 
