@@ -357,23 +357,24 @@ class LlamaForCausalLM:
     def mlp(self, i: int, x: torch.Tensor) -> torch.Tensor:
         return pstate.tp_all_reduce(self._mlp_partial(i, x))
 
-    def _mlp_partial(self, i: int, x: torch.Tensor, parts: bool = False) -> torch.Tensor:
+    def _mlp_partial(self, i: int, x: torch.Tensor, parts: bool = False, steady: bool = False) -> torch.Tensor:
         """gate_up -> SiLU*mul -> down: this rank's partial sums (before the TP all-reduce),
-        written straight into the all-reduce's staging buffer when there is one.  ``parts`` as :meth:`_row_parallel`."""
+        written straight into the all-reduce's staging buffer when there is one.  ``parts`` as :meth:`_row_parallel`, ``steady`` as
+        :func:`linear`."""
         wd = self.w_d[i]
         if self.gu_il:
             w = self.w_gu[i]
-            plan = ops.gemm_sk_plan(x.shape[0], w.shape[0], w.shape[1], 2) if x.shape[0] > _GEMV_ROWS else None
-            if _GEMV_ROWS < x.shape[0] <= 256 and ops.gemm_rows_plan(x, w):
+            plan = ops.gemm_sk_plan(x.shape[0], w.shape[0], w.shape[1], 2, steady) if x.shape[0] > _GEMV_ROWS else None
+            if not steady and x.shape[0] > _GEMV_ROWS and ops.gemm_rows_plan(x, w):
                 a = ops.gemm_rows(x, w, epi=2)
             elif plan is not None and x.stride(1) == 1 and x.stride(0) % 8 == 0:
                 a = ops.gemm_sk(x, w, epi=2, bn=plan[0], nwg=plan[1], bm=plan[2])
             elif x.is_cuda and x.shape[0] <= _GEMV_ROWS and ops.gemv_ok(x, w):
                 a = ops.gemv_swiglu(x, w)
             else:
-                a = ops.act_and_mul(linear(x, w), self.act, interleaved=True)
-            return self._row_parallel(a, wd, parts=parts)
-        gu = linear(x, self.w_gu[i])
+                a = ops.act_and_mul(linear(x, w, steady=steady), self.act, interleaved=True)
+            return self._row_parallel(a, wd, parts=parts, steady=steady)
+        gu = linear(x, self.w_gu[i], steady=steady)
         if _GEMV_ACT and self.act == 0 and gu.is_cuda and type(wd) is torch.Tensor and gu.dim() == 2 and \
                 gu.shape[0] <= _GEMV_ROWS and gu.dtype == wd.dtype == torch.bfloat16 and gu.stride(1) == 1 and \
                 gu.stride(0) % 8 == 0 and gu.data_ptr() % 16 == 0 and wd.data_ptr() % 16 == 0:
@@ -382,19 +383,20 @@ class LlamaForCausalLM:
                 if self.tp.tp > 1 else None
             return ops.gemv_act(gu, wd, out=st)
         a = ops.act_and_mul(gu, self.act)
-        return self._row_parallel(a, wd, parts=parts)
+        return self._row_parallel(a, wd, parts=parts, steady=steady)
 
-    def _row_parallel(self, a: torch.Tensor, w, bias=None, parts: bool = False) -> torch.Tensor:
-        """``parts``: the caller hands the result to :meth:`_reduce_add_norm`, so it may come in pieces (fp32 [pieces, T, H])."""
-        if parts and self.tp.tp == 1 and bias is None and type(w) is torch.Tensor and _GEMV_ROWS < a.shape[0] <= 256:
+    def _row_parallel(self, a: torch.Tensor, w, bias=None, parts: bool = False, steady: bool = False) -> torch.Tensor:
+        """``parts``: the caller hands the result to :meth:`_reduce_add_norm`, so it may come in pieces (fp32 [pieces, T, H]).
+        ``steady`` as :func:`linear`."""
+        if parts and self.tp.tp == 1 and bias is None and type(w) is torch.Tensor and a.shape[0] > _GEMV_ROWS:
             splits = ops.gemm_rows_parts_plan(a, w)
             if splits:
                 return ops.gemm_rows_parts(a, w, splits)
         if self.tp.tp > 1:
             st = pstate.tp_ar_staging((a.shape[0], self.cfg.hidden_size), self.dtype, a.device)
             if st is not None:
-                return linear(a, w, bias, out=st)
-        return linear(a, w, bias)
+                return linear(a, w, bias, out=st, steady=steady)
+        return linear(a, w, bias, steady=steady)
 
     def _reduce_add_norm(self, part: torch.Tensor, residual: torch.Tensor, w: torch.Tensor,
                          reduce: bool = True) -> torch.Tensor:
@@ -421,7 +423,11 @@ class LlamaForCausalLM:
         first = self.layers[0] if self.layers else 0
         # subclasses that override mlp() (MoE) return already-reduced outputs
         partial = type(self).mlp is LlamaForCausalLM.mlp
-        parts = st.pp_size == 1   # every projection of the residual stream is followed by a norm here
+        # Steps that put prompts into an 8-bit cache keep one order of sums: another one moves some of the new keys and values
+        # by a step of the cache's type, and prompts that attend to few others showed it as 2.3 to 3.2% of their logits (an 8B
+        # model; such prompts in a bf16 cache 2.0 to 2.4%, decode steps with either 2.0%).
+        steady = bool(self.layers) and not meta.is_decode and kv.layer(first)[0].element_size() == 1
+        parts = st.pp_size == 1 and not steady   # every projection of the residual stream is followed by a norm here
         for i in self.layers:
             if i > 0:  # the previous layer's MLP partial sums -> all-reduce + add + norm (a pipeline
                 # stage's first layer receives the previous stage's already-reduced output)
@@ -434,13 +440,13 @@ class LlamaForCausalLM:
                 ops.gemv_qkv(x, self.w_qkv[i], self.b_qkv[i], meta.positions, self.cos_sin, q, k_cache, v_cache,
                              meta.slots, tp.hq, tp.hkv, D, ks, vs)
             else:
-                qkv = linear(x, self.w_qkv[i], self.b_qkv[i])
+                qkv = linear(x, self.w_qkv[i], self.b_qkv[i], steady=steady)
                 ops.rope_qkv_cache(qkv, meta.positions, self.cos_sin, cfg.rot_dim, q, k_cache, v_cache, meta.slots,
                                    tp.hq, tp.hkv, D, True, self.qn[i], self.kn[i], self.eps, ks, vs)
             attn = self.attention(q, k_cache, v_cache, meta, ks, vs)
-            o = self._reduce_add_norm(self._row_parallel(attn.view(T, tp.hq * D), self.w_o[i], parts=parts),
+            o = self._reduce_add_norm(self._row_parallel(attn.view(T, tp.hq * D), self.w_o[i], parts=parts, steady=steady),
                                       residual, self.ln2[i])
-            x = self._mlp_partial(i, o, parts) if partial else self.mlp(i, o)
+            x = self._mlp_partial(i, o, parts, steady) if partial else self.mlp(i, o)
         if self.layers and (st.pp_size == 1 or st.is_last_pp):
             return self._reduce_add_norm(x, residual, self.norm, reduce=partial)   # final norm
         if self.layers and partial:

@@ -173,19 +173,20 @@ def _sk_operands_ok(x, w, bias, out) -> bool:
             and (out is None or (out.stride(1) == 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0)))
 
 
-def linear(x: torch.Tensor, w, bias: torch.Tensor | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
+def linear(x: torch.Tensor, w, bias: torch.Tensor | None = None, out: torch.Tensor | None = None,
+           steady: bool = False) -> torch.Tensor:
     """Dispatch: bf16 weight at a row count where the stream-K MFMA kernel was measured faster
     (``ops.gemm_sk_plan``) -> ``ops.gemm_sk``; up to 256 rows of a wide weight -> ``ops.gemm_rows``; single-row decode -> the GEMV stream kernel
     (``ops.gemv``, ``OME_GEMV_ROWS``); the weight-streaming MFMA GEMM for decode shapes where it
     was measured faster (``ops.decode_gemm_plan``, opt-in); other plain tensors -> hipBLASLt;
     Fp8Weight -> W8A16 (fp8 weight, bf16 activation) at the decode rows where ``ops.w8a16_plan``
     measured it faster, else the W8A8 MFMA path.  ``out``: write the result there (e.g. the TP all-reduce's IPC
-    staging buffer)."""
+    staging buffer).  ``steady``: one order of sums at every row count's plan (no ``ops.gemm_rows``, the nearest measured plan)."""
     if (x.dim() == 2 and x.is_cuda and x.shape[0] > _GEMV_ROWS and type(w) is torch.Tensor
             and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16):
-        if x.shape[0] <= 256 and ops.gemm_rows_plan(x, w, bias, out):
+        if not steady and ops.gemm_rows_plan(x, w, bias, out):
             return ops.gemm_rows(x, w, bias, out)
-        plan = ops.gemm_sk_plan(x.shape[0], w.shape[0], w.shape[1], 0)
+        plan = ops.gemm_sk_plan(x.shape[0], w.shape[0], w.shape[1], 0, steady)
         if plan is not None and _sk_operands_ok(x, w, bias, out):
             return ops.gemm_sk(x, w, bias, out=out, bn=plan[0], nwg=plan[1], bm=plan[2])
     if out is not None:
@@ -195,7 +196,7 @@ def linear(x: torch.Tensor, w, bias: torch.Tensor | None = None, out: torch.Tens
             if bias is None:
                 return torch.matmul(x, w.t(), out=out)
             return torch.addmm(bias, x, w.t(), out=out)
-        out.copy_(linear(x, w, bias))
+        out.copy_(linear(x, w, bias, steady=steady))
         return out
     if isinstance(w, Fp8Weight):
         if x.dim() == 2 and x.dtype == torch.bfloat16:
@@ -208,7 +209,7 @@ def linear(x: torch.Tensor, w, bias: torch.Tensor | None = None, out: torch.Tens
                 if sp is not None and ops.w8a16_ok(x, w.q, w.scale, w.block):
                     return ops.w8a16_gemm(x, w.q, w.scale, w.block, bias, splits=sp)
             if copy:
-                return linear(x, w.bf16, bias)
+                return linear(x, w.bf16, bias, steady=steady)
         return ops.fp8_linear(x, w.q, w.scale, w.block, bias)
     if x.dim() == 2 and x.shape[0] <= 256 and x.is_cuda and x.dtype == torch.bfloat16:
         if x.shape[0] <= _GEMV_ROWS and ops.gemv_ok(x, w, bias):

@@ -1560,13 +1560,13 @@ def _sk_table() -> dict:
     return _SK_TABLE
 
 
-def gemm_sk_plan(M: int, N: int, K: int, epi: int = 0) -> tuple[int, int, int] | None:
+def gemm_sk_plan(M: int, N: int, K: int, epi: int = 0, nearest: bool = False) -> tuple[int, int, int] | None:
     """(bn, nwg, bm) when the stream-K kernel was measured faster than hipBLASLt (gate_up: than
     hipBLASLt + act_and_mul) for this weight shape at the nearest measured row count, else None.  The kernel's time
     goes by its row tiles, so a row count of as many tiles speaks first (beyond 128 rows up to twice as far, and there only
     where the kernel won by a tenth), and one of fewer only with its time taken times the tiles, the library's times the rows: 28672 x
     4096 with 300 rows, two tiles, by the 256 rows' measurement 118 us, the library with its activation 82; 6144 x 4096 with
-    300 37 and 29; 4096 x 14336 with 264 by the 384 rows' plan 60 instead of 68.  Table: ``ome_amd/_tuned/gemm_sk_gfx950.json`` written by ``scripts/gemm_sk_bench.py --table``
+    300 37 and 29; 4096 x 14336 with 264 by the 384 rows' plan 60 instead of 68.  ``nearest``: the nearest row count alone, as it was measured.  Table: ``ome_amd/_tuned/gemm_sk_gfx950.json`` written by ``scripts/gemm_sk_bench.py --table``
     (cold weights, interleaved same-box timings)."""
     if _SK_MODE == "0":
         return None
@@ -1580,12 +1580,15 @@ def gemm_sk_plan(M: int, N: int, K: int, epi: int = 0) -> tuple[int, int, int] |
     def near(r, far):
         return max(r[0], M) <= far * min(r[0], M)
 
-    close = [r for r in rows if near(r, 1.34 if M <= 128 else 2) and tiles(*r) == tiles(M, r[1])] or [r for r in rows if near(r, 1.34)]
+    close = [] if nearest else [r for r in rows if near(r, 1.34 if M <= 128 else 2) and tiles(*r) == tiles(M, r[1])]
+    close = close or [r for r in rows if near(r, 1.34)]
     if not close:   # nothing measured close to this M
         return None
     m, e = min(close, key=lambda r: abs(r[0] - M) / max(r[0], M))
     bm = int(e.get("bm", 256))
-    us, lib_us = e["us"] * max(1.0, tiles(M, e) / tiles(m, e)), e["lib_us"] * (max(1.0, M / m) if tiles(M, e) > tiles(m, e) else 1.0)
+    us, lib_us = e["us"], e["lib_us"]
+    if not nearest and tiles(M, e) > tiles(m, e):
+        us, lib_us = us * tiles(M, e) / tiles(m, e), lib_us * M / m
     if us >= (0.97 if near((m, e), 1.34) else 0.9) * lib_us or not gemm_sk_ok(M, N, K, e["bn"], e["nwg"], bm):
         return None
     return e["bn"], e["nwg"], bm
