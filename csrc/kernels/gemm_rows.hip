@@ -1,4 +1,4 @@
-// Projections of 5 to 256 decode rows, bf16:  X[M][K] . W[N][K]^T  (= F.linear(x, w)), M <= 256.
+// Projections of up to 256 rows (decode steps, short prompts), bf16:  X[M][K] . W[N][K]^T  (= F.linear(x, w)).
 //
 // What bounds it: the weights, which a launch of 200 workgroups and more reads at 5.5 to 6 TB/s however little of them each has in
 // flight, and the rows, which every workgroup reads again from L2.  The two add up: 28672 x 4096 alone takes 39 us, 256 rows

@@ -1622,7 +1622,7 @@ def gemm_sk(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, 
     return out
 
 
-# ---- projections of 5 to 256 decode rows (csrc/kernels/gemm_rows.hip) ---------------------------
+# ---- projections of up to 256 decode rows (csrc/kernels/gemm_rows.hip) ---------------------------
 def gemm_rows_ok(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, out: torch.Tensor | None = None) -> bool:
     """Operands that ``ome_gemm_rows`` (and the kernels that add its pieces) take."""
     return (x.is_cuda and x.dim() == 2 and w.dim() == 2 and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.stride(1) == 1
@@ -1666,8 +1666,10 @@ def gemm_rows_splits(M: int, N: int, K: int) -> int:
 
 def gemm_rows_parts_plan(x: torch.Tensor, w: torch.Tensor) -> int:
     """Pieces of :func:`gemm_rows_parts` where it, with :func:`add_rmsnorm_parts`, is faster than a projection and
-    :func:`fused_add_rmsnorm`; else 0."""
-    if not gemm_rows_ok(x, w):
+    :func:`fused_add_rmsnorm`; else 0.  A single row needs a long K for that (GEMV -> pieces, with their norms, us: 4096 x 4096
+    9.7 -> 11.1, 2048 x 8192 10.2 -> 11.4, 8192 x 8192 31.2 -> 32.5, 2560 x 9728 14.6 -> 13.9, 4096 x 14336 24.5 -> 22.8, 8192 x
+    28672 83 -> 74; four rows 12.6 -> 11.3, 14.9 -> 11.5, 34.6 -> 33.0, 18.5 -> 14.2, 28.4 -> 22.8, 90 -> 74)."""
+    if not gemm_rows_ok(x, w) or (x.shape[0] == 1 and x.shape[1] <= 9216):
         return 0
     M, K = x.shape
     splits = gemm_rows_splits(M, w.shape[0], K)
