@@ -13,8 +13,8 @@
 // P T and T (Mamba-2: q k^T, which the heads of a group share) and the chunk's scalars, into a workspace.
 // chunk_rule_kernel walks the chunks of a (sequence, head) in order: a wave owns 16 value columns and keeps its
 // S in VGPR accumulators.  Long prompts of few heads are cut into segments that are walked side by side, in two launches of it
-// (ops._chunk_rule_seg; S at a segment's end is linear in S at its start): 8000 rows of 8 heads of 128 x 128 450 -> 150 us,
-// 32 heads of 64 x 128 410 -> 110.  The state's error against 64 bits, eight prompts of 1000 to 8000 rows: 1.10e-7 both ways (8.55e-8).
+// (ops._chunk_rule_seg; S at a segment's end is linear in S at its start): whole layers of one prompt of 8000 rows, 8 heads of 128 x 128
+// 489 -> 195 us, 32 heads of 64 x 128 435 -> 158.  The state's error against 64 bits, eight prompts of 1000 to 8000 rows: 1.10e-7 both ways (8.55e-8).
 //
 // What bounds it: the instructions of a wave that has its SIMD almost for itself, 96 matrix (Mamba-2: 60) and some 250 (310) vector
 // ones a chunk.  A product takes 16 cycles alone, but about 9 of them stay its own where vector instructions of 4 cycles fill
