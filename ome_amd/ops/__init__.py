@@ -1041,7 +1041,7 @@ class MLAWorkspace:
     widths, sinks, windows).  Row tiles of prompts are cut into equal partitions up to ~1 workgroup per CU; those of decode
     steps by the kernel itself, by their lengths, into at most 256 pieces (``plan``: each tile's first partial and
     piece count; 256 x 128 rows are ``ROWS``).  The 16-head
-    kernel takes partitions up to ~1024 workgroups.  None beyond what the f32 partials' HBM round trip repays."""
+    kernel takes partitions up to ~1024 workgroups, at most 16 unless that leaves CUs without one.  None beyond what the f32 partials' HBM round trip repays."""
 
     TARGET_WGS = 1024
     TARGET_WGS_ALL = 256
@@ -1093,10 +1093,10 @@ class MLAWorkspace:
             elif wide >= (768 if H <= 8 or pages <= 16 and H % 64 else 512 if 16 < H <= 32 else 384) and not (H % 128 == 0 and T >= 64):
                 rows = 32 if n < 704 or 0 < H % 64 <= 32 else 128 if H % 128 == 0 and T >= 24 else 64
                 return rows, True, cls.parts(T, H, DK, rows, True)
-        return 0, False, cls.parts(T, H, DK)
+        return 0, False, cls.parts(T, H, DK, pages=pages)
 
     @classmethod
-    def parts(cls, T: int, H: int, DK: int = 576, rows: int = 0, decode: bool = False) -> int:
+    def parts(cls, T: int, H: int, DK: int = 576, rows: int = 0, decode: bool = False, pages: int = 1 << 30) -> int:
         """Partitions of a tile's keys; for the row tiles of a decode step the most that a tile may get, for those of
         prompts the most that fit the chip."""
         if rows and decode:
@@ -1109,7 +1109,11 @@ class MLAWorkspace:
             p = max(1, min(cls.MAX_PARTS_ALL, cls.TARGET_WGS_ALL // (T * H // 128)))
         else:
             wgs = T * -(-H // 16)
-            p = 1 if wgs >= cls.TARGET_WGS else max(1, min(cls.MAX_PARTS, cls.TARGET_WGS // max(wgs, 1)))
+            # (few workgroups and contexts that may pass 2048 keys: one to a CU, which only long contexts use.  16 -> these, us, at 8000 keys 1
+            # token of 16 heads 44 -> 32, 1 of 128 or 8 of 16 58 -> 41, 3 of 32 58 -> 39; at 3000 23 -> 21, 26 -> 25, 25 -> 25; at 300
+            # 11.7 -> 12.0.  With two to a CU 52 at 8000, and 64 for 8 of 32, which 16 take 57)
+            most = cls.MAX_PARTS if wgs >= cls.MAX_PARTS or pages <= 128 else min(cls.MAX_PARTS_ALL, cls.TARGET_WGS_ALL // max(wgs, 1))
+            p = 1 if wgs >= cls.TARGET_WGS else max(1, min(most, cls.TARGET_WGS // max(wgs, 1)))
         return max(1, min(p, cls.ROWS // max(T * H, 1)))
 
 

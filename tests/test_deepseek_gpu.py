@@ -272,3 +272,19 @@ def test_mla_row_tiles_are_as_exact_as_the_16_head_kernel(monkeypatch, rows, H, 
         out = ops.mla_attn(q, cache, bt, row.to(DEV), kl.to(DEV), 2 * 192 ** -0.5).cpu().double()
         err.append(((out - want).norm() / want.norm()).item())
     assert err[1] < 1.02 * err[0], err
+
+
+@pytest.mark.parametrize("T,H", [(1, 16), (3, 32), (7, 40), (15, 16)])
+def test_mla_partitions_by_length(T, H):
+    """Few decode rows: partitions of up to four key tiles and more, empty ones, contexts at the edges of both.  bf16 weights and outputs:
+    two roundings of 2^-9."""
+    torch.manual_seed(T)
+    every = [1, 31, 32, 33, 127, 511, 512, 513, 1537, 2047, 2048, 2049, 3000, 5000, 8193]
+    for at in range(0, len(every), T):
+        ctx = (every[at:] + every)[:T]
+        cache, bt = _setup(ctx)
+        row, kl = torch.arange(T, dtype=torch.int32), torch.tensor(ctx, dtype=torch.int32)
+        q = torch.randn(T, H, 576, device=DEV).to(torch.bfloat16)
+        want = _exact(q, cache, bt, row, kl, 192 ** -0.5)
+        out = ops.mla_attn(q, cache, bt, row.to(DEV), kl.to(DEV), 192 ** -0.5).cpu().double()
+        assert ((out - want).flatten(1).norm(dim=1) <= 2.0 ** -8 * want.flatten(1).norm(dim=1)).all(), ctx
