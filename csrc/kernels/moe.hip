@@ -12,6 +12,7 @@
 //   ome_moe_gemm_stream : the same for experts with few rows, on tiles listed by ome_moe_align_tiles
 //   ome_moe_combine : out[t] = sum_j w[t, j] * Y[inv[t*k + j]]   (fp32 accumulate)
 #include "common.h"
+#include "lds_stages.h"
 
 #include <cstdlib>
 
@@ -547,9 +548,8 @@ __global__ __launch_bounds__(256) void moe_gemm_v2_kernel(const bf16* __restrict
 
 // ------------------------------------------------------------------------------------------
 // bf16 experts with few rows each: out[p, :] = A[row(p)] . W[e(p)]^T (+ bias) over 64-row tiles, one workgroup per tile and 64 weight
-// rows.  Bound by the weights' way from memory: three (few workgroups: four) stages of 64 k move to LDS by DMA, counted, so that
-// two stay out across the barrier; the weights are asked for before the rows' numbers are known; a workgroup reads its
-// tile instead of searching it.  A wave without rows of its own only moves.
+// rows.  Bound by the weights' way from memory: three (few workgroups: four) stages of 64 k move to LDS by DMA (lds_stages.h: one stage
+// before the wait, two or three behind it); a workgroup reads its tile instead of searching it.  A wave without rows of its own only moves.
 // 128 weight rows a workgroup: half as many and twice as long, 3 to 5% slower with 2048 or fewer k and 1 to 3% faster with 2688.
 // Whole layer, us (register-staged 64 x 64 tiles with the search -> this): 512 experts top 10 of 2048 x 512, 1 / 48 / 1000 rows 110 ->
 // 67, 430 -> 330 (5.9 TB/s), 780 -> 645; 8 experts top 2 of 4096 x 14336, 1 / 8 / 136 rows 281 -> 182, 465 -> 398 (6.4 TB/s), 673 ->
@@ -580,6 +580,8 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16* __restrict_
     const int p = min(m0 + (wave * AI + j) * 8 + (lane >> 3), m_end - 1);
     srow[j] = gather_div > 0 ? sorted_ids[p] : p;
   }
+#pragma unroll
+  for (int j = 0; j < AI; ++j) asm volatile("" ::"v"(srow[j]) : "memory");   // the rows' numbers come before any move: the compiler's wait for them is for all that is out
   const bf16* We = W + (int64_t)e * N * K;
   const bf16 *asrc[AI], *wsrc[WI];
 #pragma unroll
@@ -587,26 +589,19 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16* __restrict_
     const int r = (wave * WI + j) * 8 + (lane >> 3);
     wsrc[j] = We + (int64_t)min(n0 + r, N - 1) * K + mswz(r, lane & 7) * 8;
   }
-  const auto stage_w = [&](int buf, int kt) {
-#pragma unroll
-    for (int j = 0; j < WI; ++j)
-      __builtin_amdgcn_global_load_lds((moe_glb_t*)(wsrc[j] + kt * 64), (moe_lds_t*)(smem + buf * STG + AB + (wave * WI + j) * 1024), 16, 0, 0);
-  };
-  const auto stage_a = [&](int buf, int kt) {
-#pragma unroll
-    for (int j = 0; j < AI; ++j)
-      __builtin_amdgcn_global_load_lds((moe_glb_t*)(asrc[j] + kt * 64), (moe_lds_t*)(smem + buf * STG + (wave * AI + j) * 1024), 16, 0, 0);
-  };
-  // the weights do not wait for the rows' numbers
-#pragma unroll
-  for (int b = 0; b < NST - 1; ++b) stage_w(b, min(b, nt - 1));
 #pragma unroll
   for (int j = 0; j < AI; ++j) {
     const int r = (wave * AI + j) * 8 + (lane >> 3);
     asrc[j] = A + (int64_t)(gather_div > 0 ? srow[j] / gather_div : srow[j]) * lda + mswz(r, lane & 7) * 8;
   }
+  const auto stage = [&](int buf, int kt) {
 #pragma unroll
-  for (int b = 0; b < NST - 1; ++b) stage_a(b, min(b, nt - 1));
+    for (int j = 0; j < WI; ++j)
+      __builtin_amdgcn_global_load_lds((moe_glb_t*)(wsrc[j] + kt * 64), (moe_lds_t*)(smem + buf * STG + AB + (wave * WI + j) * 1024), 16, 0, 0);
+#pragma unroll
+    for (int j = 0; j < AI; ++j)
+      __builtin_amdgcn_global_load_lds((moe_glb_t*)(asrc[j] + kt * 64), (moe_lds_t*)(smem + buf * STG + (wave * AI + j) * 1024), 16, 0, 0);
+  };
   const int wm = wave / WN, wn = wave % WN, fr = lane & 15, fc = lane >> 4;
   const bool works = __builtin_amdgcn_readfirstlane(m0 + wm * MJ * 16 < m_end);   // a wave without rows only moves
   f32x4 acc[NI][MJ];
@@ -614,14 +609,11 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16* __restrict_
   for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < MJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AI * (NST - 2)) : "memory");   // block 0 (all weights are ahead of its rows)
-  int cur = 0;
-  for (int t = 0; t < nt; ++t) {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AI + WI) * (NST - 2)) : "memory");   // block t; the next ones (maybe clamped copies) stay out
-    __builtin_amdgcn_s_barrier();   // every wave's block t landed; every wave done reading block t - 1
-    // (branch-free: clamped to the last block past the end, so that the counted wait stays exact)
-    stage_w(cur == 0 ? NST - 1 : cur - 1, min(t + NST - 1, nt - 1));
-    stage_a(cur == 0 ? NST - 1 : cur - 1, min(t + NST - 1, nt - 1));
+  const auto landed = [](auto out) {
+    // every wave's block landed; every wave done reading the one before
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(decltype(out)::value) : "memory");
+  };
+  const auto multiply = [&](int cur) {
     const char *la = smem + cur * STG, *lw = la + AB;
     if (works) {
 #pragma unroll
@@ -641,9 +633,9 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16* __restrict_
         }
       }
     }
-    cur = cur == NST - 1 ? 0 : cur + 1;
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // clamped tail moves retire before exit
+  };
+  lds_stages<NST, AI + WI>(nt, stage, landed, multiply);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the copies of the last block past the end
 #pragma unroll
   for (int j = 0; j < MJ; ++j) {
     const int p = m0 + (wm * MJ + j) * 16 + fr;

@@ -163,3 +163,24 @@ def test_streamed_experts_at_tile_edges(counts, N, K, gather):
     want = torch.einsum("nk,nok->no", x.cpu().double()[rows], w.cpu().double()[e]) + b.cpu().double()[e]
     # fp32 sums of K products, one rounding to bf16: 2^-8 of each value (half a step), and 2^-24 K of the products' size
     assert torch.allclose(got.double(), want, rtol=2.0 ** -8, atol=2.0 ** -24 * K * 8)
+
+
+@pytest.mark.parametrize("counts,N,K", [([1, 0, 2, 1], 1024, 512), ([1, 1], 4096, 14336), ([1] * 6, 2688, 1856), ([0, 64, 3], 64, 128)], ids=str)
+@pytest.mark.parametrize("gather", [True, False])
+def test_streamed_experts_out_of_memory(counts, N, K, gather):
+    """Few workgroups, four stages: rows and weights that no cache holds, so that each block is late and has to be waited for."""
+    torch.manual_seed(N)
+    E, n = len(counts), sum(counts)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).to(torch.int32).to(DEV)
+    x, b = torch.randn(n, K, device=DEV).to(torch.bfloat16), torch.randn(E, N, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(E, N, K, device=DEV) * K ** -0.5).to(torch.bfloat16)
+    s = ops._Sorted(ids, E, 64)
+    assert ops.moe_tile_m(n, E, N) == 64 and -(-N // 64) * s.max_tiles <= 512
+    rows = s.meta[-2 * n:-n].long() if gather else torch.arange(n, device=DEV)
+    want = torch.cat([x[rows[ids == e]].double() @ w[e].double().t() + b[e].double() for e in range(E)])
+    others = torch.empty(1 << 28, dtype=torch.float32, device=DEV)   # four times the last-level cache
+    for i in range(4):
+        others.fill_(i)
+        got = ops._moe_gemm(x, s, s.ids if gather else None, 1 if gather else 0, w, n, b)
+        # as above: 2^-8 of each value and 2^-24 K of the products' size
+        assert torch.allclose(got.double(), want, rtol=2.0 ** -8, atol=2.0 ** -24 * K * 8)
