@@ -337,13 +337,23 @@ class LlamaForCausalLM:
         return ops.paged_prefill(q, k_cache, v_cache, meta.block_tables, meta.cu_q, meta.kv_lens, meta.items,
                                  self.scale, self.window, k_scale=ks, v_scale=vs, softcap=cap)
 
-    def gemm_probe(self, i: int, x: torch.Tensor, a: torch.Tensor) -> None:
-        """Layer i's projection GEMMs exactly as the forward routes them (QKV, O, gate_up with its
-        SiLU epilogue, down), without the TP all-reduce: the row-count cost probe of
-        ``runtime/step_cost.py``.  ``x`` [M, hidden], ``a`` [M, O-projection input width]."""
-        linear(x, self.w_qkv[i], self.b_qkv[i])
-        self._row_parallel(a, self.w_o[i])
-        self._mlp_partial(i, x)
+    def _sums(self, prompts: bool, kv: PagedKVCache) -> tuple[bool, bool]:
+        """(``parts``, ``steady``) of a step's projections (:meth:`_row_parallel`), of which some rows are prompts or none.
+        Steps that put prompts into an 8-bit cache keep one order of sums: another one moves some of the new keys and values
+        by a step of the cache's type, and prompts that attend to few others showed it as 2.3 to 3.2% of their logits (an 8B
+        model; such prompts in a bf16 cache 2.0 to 2.4%, decode steps with either 2.0%)."""
+        steady = prompts and bool(self.layers) and kv.layer(self.layers[0])[0].element_size() == 1
+        return pstate.get().pp_size == 1 and not steady, steady   # pieces: every projection of the residual stream is followed by a norm here
+
+    def gemm_probe(self, i: int, x: torch.Tensor, a: torch.Tensor, res: torch.Tensor, kv: PagedKVCache) -> None:
+        """Layer i's projection GEMMs exactly as the forward of a mixed step routes them (QKV, O, gate_up with its
+        SiLU epilogue, down) with the norms that may add their pieces, without the TP all-reduce: the row-count cost probe of
+        ``runtime/step_cost.py``.  ``x`` [M, hidden], ``a`` [M, O-projection input width], ``res`` [M, hidden] written over."""
+        parts, steady = self._sums(True, kv)
+        linear(x, self.w_qkv[i], self.b_qkv[i], steady=steady)
+        o = self._row_parallel(a, self.w_o[i], parts=parts, steady=steady)
+        self._reduce_add_norm(o, res, self.ln2[i], reduce=False)
+        self._reduce_add_norm(self._mlp_partial(i, x, parts, steady), res, self.ln1[i], reduce=False)
 
     def gemm_probe_widths(self) -> tuple[int, int] | None:
         """(hidden, O-projection input width) when this model's layers run exactly the dense
@@ -423,11 +433,7 @@ class LlamaForCausalLM:
         first = self.layers[0] if self.layers else 0
         # subclasses that override mlp() (MoE) return already-reduced outputs
         partial = type(self).mlp is LlamaForCausalLM.mlp
-        # Steps that put prompts into an 8-bit cache keep one order of sums: another one moves some of the new keys and values
-        # by a step of the cache's type, and prompts that attend to few others showed it as 2.3 to 3.2% of their logits (an 8B
-        # model; such prompts in a bf16 cache 2.0 to 2.4%, decode steps with either 2.0%).
-        steady = bool(self.layers) and not meta.is_decode and kv.layer(first)[0].element_size() == 1
-        parts = st.pp_size == 1 and not steady   # every projection of the residual stream is followed by a norm here
+        parts, steady = self._sums(not meta.is_decode, kv)
         for i in self.layers:
             if i > 0:  # the previous layer's MLP partial sums -> all-reduce + add + norm (a pipeline
                 # stage's first layer receives the previous stage's already-reduced output)

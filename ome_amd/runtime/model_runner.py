@@ -293,7 +293,7 @@ class ModelRunner:
     # ------------------------------------------------------------------ step-cost table
     def measure_step_cost(self, max_rows: int, grid: int = 16, reps: int = 3):
         """GEMM time of one decoder layer at M = grid, 2 grid, ... max_rows rows, routed exactly as
-        the forward routes it (``model.gemm_probe``), alternating two layers so the weights come
+        the forward of a mixed step routes it (``model.gemm_probe``), alternating two layers so the weights come
         from HBM as in a layer stack.  Returns a :class:`~ome_amd.runtime.step_cost.StepCost`, or
         None when the model has no probe or this is not a GPU run."""
         m = self.model
@@ -314,18 +314,19 @@ class ModelRunner:
         h, wo = widths
         x = torch.randn(max_rows, h, device=self.device, dtype=self.dtype) * 0.5
         a = torch.randn(max_rows, wo, device=self.device, dtype=self.dtype) * 0.5
+        res = torch.zeros_like(x)
         rows, us = [], []
         s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
         t0 = time.perf_counter()
         with torch.no_grad():
             for M in range(grid, max_rows + 1, grid):
                 for i in layers:   # warm-up: routing plans, hipBLASLt heuristics
-                    probe(i, x[:M], a[:M])
+                    probe(i, x[:M], a[:M], res[:M], self.kv)
                 best = float("inf")
                 for _ in range(reps):
                     s.record()
                     for i in layers:
-                        probe(i, x[:M], a[:M])
+                        probe(i, x[:M], a[:M], res[:M], self.kv)
                     e.record()
                     e.synchronize()
                     best = min(best, s.elapsed_time(e) * 1000.0 / len(layers))

@@ -8,8 +8,8 @@ projections, cold weights: ``profiles/r06_m_staircase.txt``).  A scheduler that 
 is pending, up to ``chunked_prefill_size``" lands on the expensive side of a step about half the
 time.
 
-:class:`StepCost` holds t(M) -- the measured GEMM time of one decoder layer at M rows, on a
-16-row grid -- and picks the prefill chunk p for a step with D decode rows and ``avail`` prompt
+:class:`StepCost` holds t(M) -- the measured GEMM time of one decoder layer at M rows (with its two
+norms, which may add a projection's pieces), on a 16-row grid -- and picks the prefill chunk p for a step with D decode rows and ``avail`` prompt
 tokens ready so that the marginal cost per prompt token, (t(D + p) - t(D)) / p, is lowest among
 the chunks that leave at most ``slack`` tokens behind (so prefill keeps pace with arrivals and
 the leftover is bounded), the leftover priced at what a full-size chunk costs per token.  When everything pending is a small remainder whose best marginal cost
