@@ -168,9 +168,12 @@ _GEMV_ROWS = int(os.environ.get("OME_GEMV_ROWS", "4"))
 
 
 def _sk_operands_ok(x, w, bias, out) -> bool:
-    return (x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.is_contiguous()
-            and w.data_ptr() % 16 == 0 and (bias is None or bias.dtype == torch.bfloat16)
-            and (out is None or (out.stride(1) == 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0)))
+    return (x.shape[1] == w.shape[1] and x.device == w.device
+            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.is_contiguous()
+            and w.data_ptr() % 16 == 0
+            and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.shape == w.shape[:1] and bias.device == x.device))
+            and (out is None or (out.shape == (x.shape[0], w.shape[0]) and out.dtype == x.dtype and out.device == x.device
+                                 and out.stride(1) == 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0)))
 
 
 def linear(x: torch.Tensor, w, bias: torch.Tensor | None = None, out: torch.Tensor | None = None,
@@ -183,7 +186,8 @@ def linear(x: torch.Tensor, w, bias: torch.Tensor | None = None, out: torch.Tens
     measured it faster, else the W8A8 MFMA path.  ``out``: write the result there (e.g. the TP all-reduce's IPC
     staging buffer).  ``steady``: one order of sums at every row count's plan (no ``ops.gemm_rows``, the nearest measured plan)."""
     if (x.dim() == 2 and x.is_cuda and x.shape[0] > _GEMV_ROWS and type(w) is torch.Tensor
-            and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16):
+            and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (bias is not None and bias.requires_grad)))):
         if not steady and ops.gemm_rows_plan(x, w, bias, out):
             return ops.gemm_rows(x, w, bias, out)
         plan = ops.gemm_sk_plan(x.shape[0], w.shape[0], w.shape[1], 0, steady)

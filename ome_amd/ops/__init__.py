@@ -1628,14 +1628,17 @@ def gemm_sk(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, 
 
 # ---- projections of up to 256 decode rows (csrc/kernels/gemm_rows.hip) ---------------------------
 def gemm_rows_ok(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, out: torch.Tensor | None = None) -> bool:
-    """Operands that ``ome_gemm_rows`` (and the kernels that add its pieces) take."""
+    """Operands of one product that ``ome_gemm_rows`` (and the kernels that add its pieces) take; what is no product (widths, a bias or
+    an output of other sizes, other devices) is left to the library, which broadcasts, resizes or refuses it."""
     return (x.is_cuda and x.dim() == 2 and w.dim() == 2 and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.stride(1) == 1
+            and x.shape[1] == w.shape[1] and w.device == x.device
             and w.stride(1) == 1 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.shape[1] <= x.stride(0) < 1 << 22
             and w.shape[1] <= w.stride(0) < 1 << 23 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and 0 < x.shape[0] <= 256
             and w.shape[0] % 128 == 0 and w.shape[0] > 0 and w.shape[1] % 64 == 0 and w.shape[1] >= 64
-            and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous()))
-            and (out is None or (out.dim() == 2 and out.dtype == torch.bfloat16 and out.stride(1) == 1 and out.stride(0) % 4 == 0
-                                 and out.stride(0) >= out.shape[1] and out.data_ptr() % 8 == 0)))
+            and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.shape == w.shape[:1] and bias.device == x.device))
+            and (out is None or (out.shape == (x.shape[0], w.shape[0]) and out.dtype == torch.bfloat16 and out.stride(1) == 1
+                                 and out.stride(0) % 4 == 0 and out.stride(0) >= out.shape[1] and out.data_ptr() % 8 == 0
+                                 and out.device == x.device)))
 
 
 def gemm_rows_plan(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, out: torch.Tensor | None = None) -> bool:

@@ -1,8 +1,10 @@
-"""The rule that chooses between the stream-K kernel and the library from a table of measured row counts."""
+"""The rules that choose a projection's kernel: between stream-K and the library from a table of measured row counts, and by operands."""
 
 import pytest
+import torch
 
 from ome_amd import ops
+from ome_amd.models import quant
 
 
 @pytest.mark.parametrize("M,us,lib_us,want", [
@@ -30,3 +32,35 @@ def test_every_plan_fits_its_kernel():
         for M in range(1, 2600, 7):
             plan = ops.gemm_sk_plan(M, N, K, epi)
             assert plan is None or ops.gemm_sk_ok(M, N, K, *plan)
+
+
+class _OnGpu:
+    """A tensor that says it is on a GPU."""
+    is_cuda = True
+
+    def __init__(self, *shape, dtype=torch.bfloat16, device="cpu"):
+        self._t = torch.empty(*shape, dtype=dtype, device=device)
+
+    def __getattr__(self, name):
+        return getattr(self._t, name)
+
+
+@pytest.mark.parametrize("bias,out,M,K,fits", [
+    (None, None, 9, 128, True), ((256,), (9, 256), 9, 128, True),
+    (None, None, 9, 64, False),        # fewer columns than the weight
+    ((1,), None, 9, 128, False), ((128,), None, 9, 128, False), ((9, 256), None, 9, 128, False), ((256, 1), None, 9, 128, False),
+    (None, (8, 256), 9, 128, False), (None, (9, 128), 9, 128, False), (None, (9, 512), 9, 128, False),
+])
+def test_what_is_no_product_is_the_librarys(bias, out, M, K, fits):
+    """The kernels take sizes from x and w: a bias or an output of other sizes, and other widths, are refused, resized or broadcast
+    by the library as before."""
+    x, w = _OnGpu(M, K), _OnGpu(256, 128)
+    b, o = (None if s is None else _OnGpu(*s) for s in (bias, out))
+    assert ops.gemm_rows_ok(x, w, b, o) == fits
+    assert quant._sk_operands_ok(x, w, b, o) == fits
+
+
+def test_operands_of_other_devices_are_the_librarys():
+    x, w, b, o = _OnGpu(9, 128), _OnGpu(256, 128), _OnGpu(256), _OnGpu(9, 256)
+    for bad in ((x, w, _OnGpu(256, device="meta"), o), (x, w, b, _OnGpu(9, 256, dtype=torch.float32))):
+        assert not ops.gemm_rows_ok(*bad) and not quant._sk_operands_ok(*bad)

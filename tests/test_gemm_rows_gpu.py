@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from ome_amd import ops
+from ome_amd.models.quant import linear
 from ome_amd.ops import reference as ref
 
 pytestmark = pytest.mark.gpu
@@ -95,3 +96,19 @@ def test_replayed_in_a_graph():
         torch.cuda.synchronize()
         assert torch.equal(got, want)
         torch.randn(1 << 20, device=D)
+
+
+def test_linear_refuses_and_broadcasts_as_the_library():
+    """Widths, biases and outputs of other sizes, operands of other devices and gradients, at a size that the kernel takes."""
+    g = torch.Generator(device=D).manual_seed(1)
+    x, w, b = (torch.empty(*s, device=D, dtype=torch.bfloat16).normal_(generator=g) for s in ((9, 128), (24576, 128), (24576,)))
+    assert ops.gemm_rows_plan(x, w, b)
+    for args in ((x[:, :64].contiguous(), w), (x, w, b[:128].contiguous()), (x, w, b.cpu()), (x, w.cpu())):
+        with pytest.raises(RuntimeError):
+            linear(*args)
+    want = torch.nn.functional.linear(x, w, b[:1])
+    assert torch.equal(linear(x, w, b[:1]), want)
+    y, wanted = (t.clone().requires_grad_() for t in (x, x))
+    linear(y, w, b).float().square().sum().backward()
+    torch.nn.functional.linear(wanted, w, b).float().square().sum().backward()
+    assert torch.equal(y.grad, wanted.grad)
