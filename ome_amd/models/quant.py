@@ -82,7 +82,7 @@ def fp8_bf16_copy_bytes() -> int:
 class Fp8Experts:
     """MoE expert weights kept in FP8 (``quantization: fp8``, 128x128 block scales): q [E, N, K]
     float8_e4m3fn, scale [E, N/128, K/128] float32.  Consumed by ``ops.fused_moe`` through the
-    block-scaled grouped GEMM (csrc/kernels/moe.hip ``ome_moe_gemm_fp8``)."""
+    block-scaled grouped GEMM (csrc/kernels/moe.hip ``ome_moe_gemm_fp8_tile``)."""
     q: torch.Tensor
     scale: torch.Tensor
     block: int = 128

@@ -1,4 +1,4 @@
-"""FP8 block-scaled grouped MoE GEMM (csrc/kernels/moe.hip ome_moe_gemm_fp8) through
+"""FP8 block-scaled grouped MoE GEMM (csrc/kernels/moe.hip ome_moe_gemm_fp8_tile) through
 ops.fused_moe with Fp8Experts, against the fp32 emulation of the same quantisation
 (ops.reference.fused_moe_fp8) and against the bf16 MoE within fp8 tolerance."""
 import pytest
