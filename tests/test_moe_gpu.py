@@ -26,9 +26,8 @@ def test_moe_route(T, E, k, dtype):
 
 @pytest.mark.parametrize("T,E,k,H,I", [(1, 8, 2, 256, 128), (64, 8, 2, 512, 256), (200, 16, 4, 256, 96),
                                        (7, 64, 6, 1024, 64), (513, 8, 2, 4096, 1024)])
-@pytest.mark.parametrize("kernel,tile", [("1", "64"), ("2", "64"), ("2", "128")])  # v1 / v2 64x64 / v2 128x128
-def test_fused_moe(T, E, k, H, I, kernel, tile, monkeypatch):
-    monkeypatch.setenv("OME_MOE_GEMM", kernel)
+@pytest.mark.parametrize("tile", ["64", "128"])
+def test_fused_moe(T, E, k, H, I, tile, monkeypatch):
     monkeypatch.setenv("OME_MOE_TILE", tile)
     x = torch.randn(T, H, device=DEV, dtype=torch.bfloat16)
     w13 = torch.randn(E, 2 * I, H, device=DEV, dtype=torch.bfloat16) * 0.05
@@ -184,3 +183,26 @@ def test_streamed_experts_out_of_memory(counts, N, K, gather):
         got = ops._moe_gemm(x, s, s.ids if gather else None, 1 if gather else 0, w, n, b)
         # as above: 2^-8 of each value and 2^-24 K of the products' size
         assert torch.allclose(got.double(), want, rtol=2.0 ** -8, atol=2.0 ** -24 * K * 8)
+
+
+@pytest.mark.parametrize("counts", [[1], [64, 0, 65], [0, 63, 128, 1, 0]], ids=str)
+@pytest.mark.parametrize("N,K,shift", [(100, 96, 0), (37, 32, 4), (320, 224, 8), (100, 128, 4), (64, 192, 1)])
+@pytest.mark.parametrize("gather", [True, False])
+def test_experts_of_any_width_and_start(monkeypatch, counts, N, K, shift, gather):
+    """64-row tiles where K is no multiple of 64 (the kernel that searches its tile itself), and where it is but rows start on no
+    16-byte boundary (streamed, from a copy)."""
+    torch.manual_seed(N + K)
+    E, n = len(counts), sum(counts)
+    order = torch.randperm(n)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[order].to(torch.int32).to(DEV)
+    x = torch.randn(n, K + 8, device=DEV).to(torch.bfloat16)[:, shift:shift + K]
+    w, b = (torch.randn(E, N, K, device=DEV) * K ** -0.5).to(torch.bfloat16), torch.randn(E, N, device=DEV).to(torch.bfloat16)
+    s, ran, call = ops._Sorted(ids, E, 64), [], ops.call
+    monkeypatch.setattr(ops, "call", lambda fn, *a: (ran.append(fn), call(fn, *a)))
+    got = ops._moe_gemm(x, s, s.ids if gather else None, 1 if gather else 0, w, n, b).cpu()
+    assert ran == ["ome_moe_gemm" if K % 64 else "ome_moe_gemm_stream"]
+    rows = s.meta[-2 * n:-n].long().cpu() if gather else torch.arange(n)
+    e = ids.cpu().long().sort().values
+    want = torch.einsum("nk,nok->no", x.cpu().double()[rows], w.cpu().double()[e]) + b.cpu().double()[e]
+    # fp32 sums of K products, one rounding to bf16: 2^-8 of each value (half a step), and 2^-24 K of the products' size
+    assert torch.allclose(got.double(), want, rtol=2.0 ** -8, atol=2.0 ** -24 * K * 8)
