@@ -375,7 +375,7 @@ class LlamaForCausalLM:
         if self.gu_il:
             w = self.w_gu[i]
             plan = ops.gemm_sk_plan(x.shape[0], w.shape[0], w.shape[1], 2, steady) if x.shape[0] > _GEMV_ROWS else None
-            if not steady and ops.gemm_rows_plan(x, w):   # (one row 28672 x 4096 36 us, gemv_swiglu 41; 57344 x 8192 139, 169; 49152 x 3072 50, 51.5)
+            if not steady and ops.gemm_rows_plan(x, w, epi=2):   # (one row 28672 x 4096 36 us, gemv_swiglu 41; 57344 x 8192 139, 169; 49152 x 3072 50, 51.5)
                 a = ops.gemm_rows(x, w, epi=2)
             elif plan is not None and x.stride(1) == 1 and x.stride(0) % 8 == 0:
                 a = ops.gemm_sk(x, w, epi=2, bn=plan[0], nwg=plan[1], bm=plan[2])

@@ -1655,15 +1655,26 @@ def gemm_rows_ok(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = N
                                  and out.device == x.device)))
 
 
-def gemm_rows_plan(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, out: torch.Tensor | None = None) -> bool:
+def gemm_rows_plan(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, out: torch.Tensor | None = None,
+                   epi: int = 0) -> bool:
     """:func:`gemm_rows` takes this product and fills the chip with it: its workgroups of 128 columns come in whole waves over the 256
     CUs, three quarters full at the least (288 of them, 36864 x 7168: 106 us against the library's 100), and beyond 128 rows, where
-    the matrix cores count too, in one (57344 x 8192 at 160 rows: 228 us against 190; at 128 174 against 178)."""
+    the matrix cores count too, in one (57344 x 8192 at 160 rows: 228 us against 190; at 128 174 against 178).
+    Weight rows of a multiple of 4 KB lie in few of the memory's channels, which costs the library up to a third and this kernel nothing
+    (it starts at different places in K).  Without that the library is ahead sooner (with its activation pass, ``epi`` 2, it is not).  This kernel's
+    time over its: one wave, 129 to 192 rows 1.01 to 1.12 for K of 3072 and 5120 (0.70 to 1.05 for 2048, 4096, 6144 and 8192), 200 to 256
+    0.88 to 1.05; two to five waves of those K, 64 rows 0.89 to 1.02, 80 to 128 0.91 to 1.16, of K up to 1024 up to 1.07;
+    six and more, 48 rows 0.86 to 1.03, 64 to 128 0.95 to 1.14.  K of 16384 in two waves, 128 rows 1.13 to 1.19, 100 0.89."""
     if not gemm_rows_ok(x, w, bias, out):
         return False
+    M, K = x.shape
     tiles = w.shape[0] // 128
     waves = -(-tiles // 256)
-    return tiles >= 192 * waves and (x.shape[0] <= 128 or waves == 1)
+    if tiles < 192 * waves or (waves > 1 and M > (128 if K < 16384 else 112)):
+        return False
+    if epi or K % 2048 == 0:
+        return True
+    return not 128 < M < 200 if waves == 1 else K <= 1024 or M < (80 if waves < 6 else 49)
 
 
 def gemm_rows(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, out: torch.Tensor | None = None,

@@ -74,3 +74,18 @@ def test_operands_of_other_devices_are_the_librarys():
     x, w, b, o = _OnGpu(9, 128), _OnGpu(256, 128), _OnGpu(256), _OnGpu(9, 256)
     for bad in ((x, w, _OnGpu(256, device="meta"), o), (x, w, b, _OnGpu(9, 256, dtype=torch.float32))):
         assert not ops.gemm_rows_ok(*bad) and not quant._sk_operands_ok(*bad)
+
+
+# (library or library and activation, this kernel, us)
+@pytest.mark.parametrize("N,K,M,epi,want", [
+    (27392, 5120, 128, 0, True), (27392, 5120, 160, 0, False), (27392, 5120, 200, 0, True),   # 70 and 79 at 160
+    (27392, 5120, 160, 2, True), (28672, 4096, 160, 0, True),
+    (49152, 3072, 65, 0, True), (49152, 3072, 80, 0, False), (49152, 3072, 128, 2, True),     # 65 and 70
+    (57344, 8192, 128, 0, True), (57344, 8192, 129, 0, False),
+    (131072, 1024, 128, 0, True), (128256, 4096, 128, 0, True),
+    (256000, 2304, 48, 0, True), (256000, 2304, 64, 0, False),                                # 219 and 235; 245 and 283 at 128
+    (53248, 16384, 112, 2, True), (53248, 16384, 128, 2, False),                              # 351 and 396
+    (36864, 7168, 9, 0, False),
+])
+def test_row_kernel_where_it_was_measured_faster(N, K, M, epi, want):
+    assert ops.gemm_rows_plan(_OnGpu(M, K, device="meta"), _OnGpu(N, K, device="meta"), epi=epi) == want
