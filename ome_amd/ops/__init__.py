@@ -1698,13 +1698,26 @@ def gemm_rows_splits(M: int, N: int, K: int) -> int:
 
 def gemm_rows_parts_plan(x: torch.Tensor, w: torch.Tensor) -> int:
     """Pieces of :func:`gemm_rows_parts` where it, with :func:`add_rmsnorm_parts`, is faster than a projection and
-    :func:`fused_add_rmsnorm`; else 0.  A single row needs a long K for that (GEMV -> pieces, with their norms, us: 4096 x 4096
+    :func:`fused_add_rmsnorm`; else 0.  The GEMV takes few rows of small weights in less time than two launches with fp32 between them:
+    a single row needs a long K for the pieces (GEMV -> pieces, with their norms, us: 4096 x 4096
     9.7 -> 11.1, 2048 x 8192 10.2 -> 11.4, 8192 x 8192 31.2 -> 32.5, 2560 x 9728 14.6 -> 13.9, 4096 x 14336 24.5 -> 22.8, 8192 x
-    28672 83 -> 74; four rows 12.6 -> 11.3, 14.9 -> 11.5, 34.6 -> 33.0, 18.5 -> 14.2, 28.4 -> 22.8, 90 -> 74)."""
-    if not gemm_rows_ok(x, w) or (x.shape[0] == 1 and x.shape[1] <= 9216):
+    28672 83 -> 74), two rows 40 MB (2048 x 8192 11.2 -> 11.9, 3584 x 3584 9.8 -> 10.4, 3072 x 8192 equal, 5120 x 5120 0.96), three 8 MB or K of 4096
+    (2048 x 2048 7.2 -> 7.4, 1024 x 4096 0.96, 5120 x 1024 0.96), four 8 MB or K of 2048
+    (1536 x 1536 6.9 -> 7.7, 2048 x 512 5.9 -> 6.4, 1024 x 2048 0.96).  From some 112 rows
+    small weights are too few steps for as many pieces as fill the chip (library -> pieces at 256 rows: 1024 x 3072 12.3 -> 20.0, 2048 x
+    2048 14.6 -> 19.9, 3072 x 3072 20.9 -> 25.8, 3584 x 3584 23.8 -> 25.7, 4096 x 4096 26.3 -> 27.5; 5120 x 5120 0.59, 1536 x 8960 0.90; at 160
+    3072 x 3072 19.4 -> 21.6, 3584 x 3584 0.84, 2048 x 6144 0.94; at 128 1536 x 1536 10.8 -> 12.7, 5632 x 2048 18.8 -> 20.5, 2048 x 2048 1.02,
+    1024 x 2048 0.96)."""
+    if not gemm_rows_ok(x, w):
         return 0
     M, K = x.shape
-    splits = gemm_rows_splits(M, w.shape[0], K)
+    N = w.shape[0]
+    if M <= 4:
+        if not (K > 9216, N * K >= 20 << 20, N * K > 4 << 20 or K >= 4096, N * K > 4 << 20 or K >= 2048)[M - 1]:
+            return 0
+    elif M > 112 and 1024 < K <= 2048 or M > 128 and K < 8192 and N * K < (12 << 20 if M <= 160 else (16 << 20) + 1):
+        return 0
+    splits = gemm_rows_splits(M, N, K)
     return splits if splits > 1 else 0
 
 

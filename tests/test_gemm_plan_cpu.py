@@ -89,3 +89,13 @@ def test_operands_of_other_devices_are_the_librarys():
 ])
 def test_row_kernel_where_it_was_measured_faster(N, K, M, epi, want):
     assert ops.gemm_rows_plan(_OnGpu(M, K, device="meta"), _OnGpu(N, K, device="meta"), epi=epi) == want
+
+
+@pytest.mark.parametrize("N,K,rows", [
+    (4096, 14336, {1, 2, 3, 4, 5, 64, 128, 160, 256}), (4096, 4096, {3, 4, 5, 64, 128, 160}), (5120, 5120, {2, 3, 4, 5, 64, 128, 160, 256}),
+    (1536, 8960, {3, 4, 5, 64, 128, 160, 256}), (3584, 3584, {3, 4, 5, 64, 128, 160}), (3072, 3072, {3, 4, 5, 64, 128}), (1024, 4096, {3, 4, 5, 64, 128}),
+    (2048, 2048, {4, 5, 64}), (5120, 1024, {3, 4, 5, 64, 128}), (2048, 512, {5, 64, 128}), (8192, 256, set()),
+])
+def test_pieces_where_they_were_measured_faster(N, K, rows):
+    w = _OnGpu(N, K, device="meta")
+    assert {M for M in (1, 2, 3, 4, 5, 64, 128, 160, 256) if ops.gemm_rows_parts_plan(_OnGpu(M, K, device="meta"), w)} == rows
