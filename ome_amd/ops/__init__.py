@@ -1112,10 +1112,11 @@ class MLAWorkspace:
             p = max(1, min(cls.MAX_PARTS_ALL, cls.TARGET_WGS_ALL // (T * H // 128)))
         else:
             wgs = T * -(-H // 16)
-            # (few workgroups and contexts that may pass 2048 keys: one to a CU, which only long contexts use.  16 -> these, us, at 8000 keys 1
-            # token of 16 heads 44 -> 32, 1 of 128 or 8 of 16 58 -> 41, 3 of 32 58 -> 39; at 3000 23 -> 21, 26 -> 25, 25 -> 25; at 300
-            # 11.7 -> 12.0.  With two to a CU 52 at 8000, and 64 for 8 of 32, which 16 take 57)
-            most = cls.MAX_PARTS if wgs >= cls.MAX_PARTS or pages <= 128 else min(cls.MAX_PARTS_ALL, cls.TARGET_WGS_ALL // max(wgs, 1))
+            # (at most 12 workgroups and contexts that may pass 2048 keys: one to a CU, which only long contexts use.  16 -> these, us, at 8000 keys 1
+            # token of 16 heads 44 -> 32, 1 of 128 or 8 of 16 58 -> 41, 3 of 64 59 -> 50; at 4000 27 -> 23, 35 -> 29, 35 -> 33; at 300 to 2500, where
+            # the merge still asks for the length, up to 0.5 us more.  15 workgroups: 17 partitions 1.02 up to 4000 keys, 0.98 at 8000.  With two to
+            # a CU 52 at 8000, and 64 for 8 of 32, which 16 take 57)
+            most = cls.MAX_PARTS if wgs > 12 or pages <= 128 else min(cls.MAX_PARTS_ALL, cls.TARGET_WGS_ALL // max(wgs, 1))
             p = 1 if wgs >= cls.TARGET_WGS else max(1, min(most, cls.TARGET_WGS // max(wgs, 1)))
         return max(1, min(p, cls.ROWS // max(T * H, 1)))
 

@@ -288,3 +288,25 @@ def test_mla_partitions_by_length(T, H):
         want = _exact(q, cache, bt, row, kl, 192 ** -0.5)
         out = ops.mla_attn(q, cache, bt, row.to(DEV), kl.to(DEV), 192 ** -0.5).cpu().double()
         assert ((out - want).flatten(1).norm(dim=1) <= 2.0 ** -8 * want.flatten(1).norm(dim=1)).all(), ctx
+
+
+@pytest.mark.parametrize("T,H", [(1, 16), (3, 32), (12, 16)])
+def test_mla_reads_no_partition_that_is_not_written(T, H):
+    """A workspace that holds NaN, contexts of fewer partitions than the table's width allows, and the tokens' own lengths.  Tolerance as above."""
+    torch.manual_seed(T)
+    for every in ([0, 1, 300, 511], [513, 2048, 2049, 2500], [3000, 4097, 8000, 0]):
+        ctx = (every * T)[:T]
+        cache, bt = _setup(ctx + [8192])
+        row, kl = torch.arange(T, dtype=torch.int32), torch.tensor(ctx, dtype=torch.int32)
+        q = torch.randn(T, H, 576, device=DEV).to(torch.bfloat16)
+        ws = ops.MLAWorkspace(DEV)
+        ws.ws_o.fill_(float("nan"))
+        ws.ws_ml.fill_(float("nan"))
+        assert ops.MLAWorkspace.tiles(T, H, 576, *bt.shape)[2] > 16
+        out = ops.mla_attn(q, cache, bt, row.to(DEV), kl.to(DEV), 192 ** -0.5, ws).cpu().double()
+        for t, n in enumerate(ctx):
+            if n == 0:
+                assert bool((out[t] == 0).all())
+                continue
+            want = _exact(q[t:t + 1], cache, bt[t:t + 1], row[:1], kl[t:t + 1], 192 ** -0.5)
+            assert ((out[t:t + 1] - want).flatten(1).norm(dim=1) <= 2.0 ** -8 * want.flatten(1).norm(dim=1)).all(), (ctx, t)
