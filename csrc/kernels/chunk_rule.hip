@@ -78,7 +78,36 @@ struct RuleArgs {
   int S, H, Hk, dv;
   int seg;                        // chunks of a segment (0: sequences in one piece)
   float* segs;                    // seg_floats of every (segment, head)
+  int4* turn;                     // the sequences in the order of their workgroups (set_turns), or null: as they come
 };
+
+constexpr int TURNS = 64;         // of at most so many
+
+// A sequence: its number, rows, place in the state, whether it starts afresh.
+struct Seq {
+  int s, q0, q1, slot;
+  bool fresh;
+};
+
+__device__ __forceinline__ Seq seq_of(const RuleArgs& a, int s) { return {s, a.cu[s], a.cu[s + 1], a.slot[s], a.reset[s] != 0}; }
+
+// The order of the sequences' workgroups: the longest first, and of the sequences that begin a second round over the CUs
+// the shortest first, so that a CU's two workgroups are as long as another's (four prompts of 293 to 1248 rows, 128 heads: 106 -> 93 us).
+// Set beside the chunks' matrices, by the last workgroup, which rarely has a chunk; a workgroup of the scan then reads a sequence whole.
+// (Searched by each workgroup of the scan it took as long as a short sequence.  10 prompts of 33 rows beside 50 of 1, delta rule of 32 heads
+// and selective scan of 128: 74 and 113 us so, 54 and 75 now and without an order; 48 prompts of 30 to 289 rows 204 and 293 -> 190 and 279.)
+__device__ __forceinline__ void set_turns(const RuleArgs& a) {
+  if (a.turn == nullptr || blockIdx.x != gridDim.x - 1 || blockIdx.y != 0 || threadIdx.x >= 64) return;
+  const int lane = threadIdx.x, len = lane < a.S ? a.cu[lane + 1] - a.cu[lane] : -1;
+  const Seq own = seq_of(a, min(lane, a.S - 1));
+  int rank = 0;
+  for (int j = 0; j < a.S; ++j) {
+    const int other = __builtin_amdgcn_readlane(len, j);
+    rank += other > len || (other == len && j < lane);
+  }
+  const int round = max(256 / (a.H * ((a.dv + 63) / 64)), 1), k = rank / round;
+  if (lane < a.S) a.turn[k & 1 ? min(a.S, (k + 1) * round) - 1 - (rank - k * round) : rank] = int4{own.s | (own.fresh ? 1 << 31 : 0), own.q0, own.q1, own.slot};
+}
 
 // Floats that a segment leaves of a head: its state [dv, dk]; then DELTA its transition [dk, dk], Mamba-2 its decay (a sequence's first
 // segment: what the sequence started from).
@@ -203,6 +232,7 @@ __global__ __launch_bounds__(256) void chunk_gram_kernel(RuleArgs a) {
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
   const int h = blockIdx.y * 4 + w;
   int r0, n;
+  set_turns(a);
   if (h >= a.H || !chunk_of(blockIdx.x, a.cu, a.S, r0, n)) return;   // whole wave; no block barrier below
   const int hk = h / (a.H / a.Hk);
   char* ws = a.ws + blockIdx.x * ws_bytes<true>(a.H, a.Hk) + h * head_bytes<true>();
@@ -378,6 +408,7 @@ __global__ __launch_bounds__(256) void ssm_gram_kernel(RuleArgs a) {
   constexpr int NS = DK / 32;
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4, hk = blockIdx.y;
   int r0, n;
+  set_turns(a);
   if (!chunk_of(blockIdx.x, a.cu, a.S, r0, n)) return;   // the same in every wave
   char* ws = a.ws + blockIdx.x * ws_bytes<false>(a.H, a.Hk);
   if (w == 0) {
@@ -428,21 +459,6 @@ __global__ __launch_bounds__(256) void ssm_gram_kernel(RuleArgs a) {
   }
 }
 
-// The sequence whose workgroups (`per` of them) come z-th: the longest first, and of the sequences that begin a second round over the CUs
-// the shortest first, so that a CU's two workgroups are as long as another's (four prompts of 293 to 1248 rows, 128 heads: 106 -> 93 us).
-// Whole wave.  (More than a wave of sequences: as they come.)
-__device__ __forceinline__ int in_turn(int z, int per, const int* cu, int S) {
-  if (S == 1 || S > 64) return z;
-  const int lane = threadIdx.x & 63, len = lane < S ? cu[lane + 1] - cu[lane] : -1, round = max(256 / per, 1), k = z / round;
-  int rank = 0;
-  for (int j = 0; j < S; ++j) {
-    const int other = __builtin_amdgcn_readlane(len, j);
-    rank += other > len || (other == len && j < lane);
-  }
-  const int want = k & 1 ? min(S, (k + 1) * round) - 1 - (z - k * round) : z;
-  return __builtin_ctzll(__ballot(lane < S && rank == want));
-}
-
 // ---------------------------------------------------------------------------------------------
 // The chunks of one (sequence, head) in order; block = NW waves x 16 value columns.  D rows of a 16 x 16
 // product sit at 4 g + e, so with block b of S standing for key channels 32 (b / 2) + 8 (row / 4) + 4 (b % 2) +
@@ -466,13 +482,24 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   __shared__ __attribute__((aligned(1024))) char lds[2 * IMG];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)lds;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g = lane >> 4;
-  int s, j = 0;
-  if constexpr (SEG == 0) s = in_turn(blockIdx.z, gridDim.x * gridDim.y, a.cu, a.S);
-  else if (!segment_of(blockIdx.z, a.seg * RC, a.cu, a.S, s, j)) return;
-  const int h = blockIdx.x, hk = h / (a.H / a.Hk);
-  const int q0 = a.cu[s], r0 = q0 + j * a.seg * RC, r1 = SEG ? min(a.cu[s + 1], r0 + a.seg * RC) : a.cu[s + 1];
+  int j = 0;
+  Seq seq;
+  if constexpr (SEG == 0) {
+    if (a.turn != nullptr) {
+      const int4 t = a.turn[blockIdx.z];
+      seq = {t.x & 0x7fffffff, t.y, t.z, t.w, t.x < 0};
+    } else {
+      seq = seq_of(a, blockIdx.z);
+    }
+  } else {
+    int id;
+    if (!segment_of(blockIdx.z, a.seg * RC, a.cu, a.S, id, j)) return;
+    seq = seq_of(a, id);
+  }
+  const int s = seq.s, h = blockIdx.x, hk = h / (a.H / a.Hk);
+  const int q0 = seq.q0, r0 = q0 + j * a.seg * RC, r1 = SEG ? min(seq.q1, r0 + a.seg * RC) : seq.q1;
   if (r1 <= r0) return;                                    // whole block
-  const bool last = SEG == 0 || r1 == a.cu[s + 1];
+  const bool last = SEG == 0 || r1 == seq.q1;
   const bool ident = SEG == 1 && DELTA && blockIdx.y >= (a.dv + COLS - 1) / COLS;   // columns of the transition
   if (SEG == 1 && (last || (ident && j == 0))) return;
   const int c0 = (ident ? blockIdx.y - (a.dv + COLS - 1) / COLS : blockIdx.y) * COLS, n0 = c0 + wave * 16;   // the block's and this wave's columns
@@ -567,7 +594,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   };
 
   // state: lane (col, g) holds column nc, key channels 32 s + 8 g .. + 7 in blocks 2 s, 2 s + 1
-  float* st = a.state + (((int64_t)a.slot[s] * a.H + h) * a.dv + nc) * DK + 8 * g;
+  float* st = a.state + (((int64_t)seq.slot * a.H + h) * a.dv + nc) * DK + 8 * g;
   f32x4 S[NB];
   const auto load = [&](const float* from) {
 #pragma unroll
@@ -649,7 +676,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   // what the sequence starts from
   const auto origin = [&] {
     if (SEG == 2 && !(last && j == 0)) load(sg - j * sg_step + copy + mine);   // (its last segment may have written `state` by now)
-    else if (a.reset[s] != 0) zero();
+    else if (seq.fresh) zero();
     else load(st);
   };
   // what the rows r0 and up start from
@@ -911,7 +938,9 @@ template <bool DELTA>
 int launch_rule(RuleArgs a, int T, int dk, hipStream_t stream) {
   const bool vec = aligned16(a.v, a.v_stride) && ((uintptr_t)a.out | (uintptr_t)(2 * a.out_stride)) % 8 == 0;   // (dv is a multiple of 16)
   if (!vec) a.seg = 0;
-  a.segs = reinterpret_cast<float*>(a.ws + (int64_t)(T / RC + a.S) * ws_bytes<DELTA>(a.H, a.Hk));
+  char* end = a.ws + (int64_t)(T / RC + a.S) * ws_bytes<DELTA>(a.H, a.Hk);
+  a.turn = a.S > 1 && a.S <= TURNS && !a.seg ? reinterpret_cast<int4*>(end) : nullptr;
+  a.segs = reinterpret_cast<float*>(end);
   const int cols = (a.dv + 63) / 64, ids = a.seg ? T / (RC * a.seg) + a.S : a.S;
   if (ids > 65535) return -3;
   const dim3 gram(T / RC + a.S, DELTA ? (a.H + 3) / 4 : a.Hk), rule(a.H, cols, ids), own(a.H, cols + (DELTA ? dk / 64 : 0), ids);
@@ -949,7 +978,7 @@ OME_API int ome_chunk_rule_floats(int H, int G, int delta) {
   return (int)((delta ? ws_bytes<true>(H, G) : ws_bytes<false>(H, G)) / 4);
 }
 
-// ... and of a head of a segment, of which there are up to T / (32 seg) + S; they come behind the chunks'
+// ... and of a head of a segment, of which there are up to T / (32 seg) + S; they come behind the chunks' (without segments: 256 words, the order)
 OME_API int ome_chunk_rule_seg_floats(int dk, int dv) { return (int)seg_floats(dv, dk); }
 
 // Gated delta rule over all rows of every sequence, in segments of `seg` chunks (0: in one piece); operands as ome_gdn_scan.  -3: a shape, stride or
@@ -962,7 +991,7 @@ OME_API int ome_gdn_chunks(const void* q, const void* k, const void* v, int64_t 
       (uintptr_t)state % 16 || (uintptr_t)ws % 16)
     return -3;
   const RuleArgs r{(const bf16*)q, (const bf16*)k, (const bf16*)v, qkv_stride, qkv_stride, (const bf16*)a, (const bf16*)b,
-                   ab_stride, A_log, nullptr, dt_bias, 0.f, (char*)ws, state, (bf16*)out, out_stride, cu, slot, reset, S, Hv, Hk, dv, seg, nullptr};
+                   ab_stride, A_log, nullptr, dt_bias, 0.f, (char*)ws, state, (bf16*)out, out_stride, cu, slot, reset, S, Hv, Hk, dv, seg, nullptr, nullptr};
   return launch_rule<true>(r, T, dk, stream);
 }
 
@@ -975,6 +1004,6 @@ OME_API int ome_ssm_chunks(const void* x, int64_t x_stride, const void* dt, int6
       (uintptr_t)state % 16 || (uintptr_t)ws % 16)
     return -3;
   const RuleArgs r{(const bf16*)Cm, (const bf16*)B, (const bf16*)x, bc_stride, x_stride, (const bf16*)dt, nullptr,
-                   dt_stride, A, D, dt_bias, dt_min, (char*)ws, state, (bf16*)y, y_stride, cu, slot, reset, S, H, G, P, seg, nullptr};
+                   dt_stride, A, D, dt_bias, dt_min, (char*)ws, state, (bf16*)y, y_stride, cu, slot, reset, S, H, G, P, seg, nullptr, nullptr};
   return launch_rule<false>(r, T, N, stream);
 }

@@ -216,7 +216,7 @@ def _chunk_rule_ws(T: int, S: int, H: int, G: int, dk: int, dv: int, delta: bool
     seg = _chunk_rule_seg(T, S, H, dv, delta)
     if seg:
         floats += (T // (32 * seg) + S) * H * _chunk_rule_seg_floats(dk, dv)
-    return torch.empty(floats, dtype=torch.float32, device=state.device)
+    return torch.empty(floats + 256, dtype=torch.float32, device=state.device)[:floats]   # (the sequences' order lies behind)
 
 
 def ssm_scan(x, dt, B, C, A, D, dt_bias, dt_min: float, state, cu, slot, reset, H: int, P: int, N: int, G: int,

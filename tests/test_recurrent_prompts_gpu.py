@@ -368,3 +368,17 @@ def test_silu_of_every_value():
     want = (x.double() / (1 + (-x.double()).exp())).to(BF)
     want[(x < -88.72) & x.isfinite()] = 0
     assert bool(((y == want) | (y.isnan() & want.isnan())).all())
+
+
+@pytest.mark.parametrize("S", [2, 63, 64, 65])
+@pytest.mark.parametrize("delta", [True, False])
+def test_sequences_in_turn(S, delta):
+    """Ragged sequences, equal ones and empty ones among them, on both sides of the number that is ordered by length, in a part of a round over
+    the chip (few heads) and in many."""
+    lens = [(0, 33, 1, 70, 3, 4, 33, 128)[(5 * i + i // 8) % 8] for i in range(S)]
+    if delta:
+        for dims in ((64, 16, 1, 5, 0), (64, 16, 2, 48, 0)):
+            test_delta_rule_prompts(lens, *dims)
+    else:
+        for dims in ((3, 16, 64, 1, 0), (48, 16, 64, 2, 0)):
+            test_selective_scan_prompts(lens, *dims)
