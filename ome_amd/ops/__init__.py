@@ -1572,11 +1572,12 @@ def gemm_sk_plan(M: int, N: int, K: int, epi: int = 0, nearest: bool = False) ->
     """(bn, nwg, bm) when the stream-K kernel was measured faster than hipBLASLt (gate_up: than
     hipBLASLt + act_and_mul) for this weight shape at the nearest measured row count, else None.  The kernel's time
     goes by its row tiles, so a row count of as many tiles speaks first (beyond 128 rows up to twice as far, and there only
-    where the kernel won by a tenth), and one of fewer only with its time taken times the tiles, the library's half way there (it has
-    tiles too): 28672 x 4096 with 300 rows, two tiles, by the 256 rows' measurement 118 us, the library with its activation 82; 6144 x 4096 with
-    300 37 and 29; 4096 x 14336 with 264 by the 384 rows' plan 60 instead of 68, with 1100 by the 1024 rows' 142, the library 158.  Where all
-    tiles are few beside the workgroups (two fifths at the most), which share them, a further one costs little: there the nearest row
-    count decides if the kernel won by a fifth (4096 x 4096 with 160 rows 21 us, the library 27; 4096 x 14336 with 520 96 and 112).
+    where the kernel won by a tenth), and one of fewer only with its time taken times the tiles, the library's times the rows: 28672 x
+    4096 with 300 rows, two tiles, by the 256 rows' measurement 118 us, the library with its activation 82; 6144 x 4096 with
+    300 37 and 29; 4096 x 14336 with 264 by the 384 rows' plan 60 instead of 68 (with 1043 by the 1024 rows' 143 and the library 147,
+    but steps of an 8B model are 2 to 3% shorter with the library).  Where all tiles are few beside the workgroups (two fifths at the
+    most), which share them, a further one costs little: there the nearest row count decides if the kernel won by a fifth (4096 x 4096
+    with 160 rows 21 us, the library 27; 4096 x 14336 with 520 96 and 112).
     ``nearest``: the nearest row count alone, as it was measured.  Table: ``ome_amd/_tuned/gemm_sk_gfx950.json`` written by ``scripts/gemm_sk_bench.py --table``
     (cold weights, interleaved same-box timings)."""
     if _SK_MODE == "0":
@@ -1601,8 +1602,7 @@ def gemm_sk_plan(M: int, N: int, K: int, epi: int = 0, nearest: bool = False) ->
     m, e = nearest_of(as_many or measured)
     us, lib_us = e["us"], e["lib_us"]
     if not nearest and tiles(M, e) > tiles(m, e):
-        more = tiles(M, e) / tiles(m, e)
-        us, lib_us = us * more, lib_us * (1 + more) / 2
+        us, lib_us = us * tiles(M, e) / tiles(m, e), lib_us * M / m
     if us >= (0.97 if near((m, e), 1.34) else 0.9) * lib_us:
         if nearest or not measured:
             return None

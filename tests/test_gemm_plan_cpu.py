@@ -37,7 +37,7 @@ def test_every_plan_fits_its_kernel():
 @pytest.mark.parametrize("M,N,K,want", [
     (160, 4096, 4096, (128, 192, 128)),     # 21 us, the library 27: few tiles for the workgroups, so the second row tile costs little
     (520, 4096, 14336, (128, 256, 256)),    # 96 and 112
-    (1100, 4096, 14336, (128, 256, 256)),   # 142 and 158: the library has a fifth row tile too
+    (1100, 4096, 14336, None),              # 143 and 154 alone, but whole steps with the library are 2 to 3% shorter
     (300, 6144, 4096, None), (300, 10240, 8192, None), (520, 8192, 28672, None),   # 38 and 29, 94 and 82, 371 and 273
 ])
 def test_plans_by_what_was_measured_between_the_table_s_rows(M, N, K, want):
