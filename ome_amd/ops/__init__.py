@@ -1664,8 +1664,8 @@ def gemm_rows_plan(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None =
     Weight rows of a multiple of 4 KB lie in few of the memory's channels, which costs the library up to a third and this kernel nothing
     (it starts at different places in K).  Without that the library is ahead sooner (with its activation pass, ``epi`` 2, it is not).  This kernel's
     time over its: one wave, 129 to 192 rows 1.01 to 1.12 for K of 3072 and 5120 (0.70 to 1.05 for 2048, 4096, 6144 and 8192), 200 to 256
-    0.88 to 1.05; two to five waves of those K, 64 rows 0.89 to 1.02, 80 to 128 0.91 to 1.16, of K up to 1024 up to 1.07;
-    six and more, 48 rows 0.86 to 1.03, 64 to 128 0.95 to 1.14.  K of 16384 in two waves, 128 rows 1.13 to 1.19, 100 0.89."""
+    0.88 to 1.05; two to five waves of those K, 64 rows 0.87 to 1.02, 80 to 128 0.91 to 1.16, of K up to 1024 up to 1.07;
+    six and more, 48 rows 0.96 to 1.03, 64 to 128 0.95 to 1.14.  K of 16384 in two waves, 128 rows 1.13 to 1.19, 100 0.89."""
     if not gemm_rows_ok(x, w, bias, out):
         return False
     M, K = x.shape
