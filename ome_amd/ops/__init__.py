@@ -1148,7 +1148,7 @@ def mla_attn(q, cache, block_tables, tok_row, kv_lens, scale: float, ws: MLAWork
         out = torch.empty(T, H, dv, dtype=q.dtype, device=q.device)
     rows, decode, parts = _latent_tiles(T, H, DK, block_tables, max_len)
     if rows and (out.data_ptr() % 16 or out.stride(0) % 8):
-        rows, decode, parts = 0, False, MLAWorkspace.parts(T, H, DK)
+        rows, decode, parts = 0, False, MLAWorkspace.parts(T, H, DK, pages=block_tables.shape[1])
     if ws is None and (parts > 1 or decode):
         ws = MLAWorkspace(q.device)
     call("ome_mla_attn", q.data_ptr(), q.stride(0), cache.data_ptr(), _i32(block_tables).data_ptr(),
@@ -2279,7 +2279,7 @@ def latent_attn(q, cache, block_tables, tok_row, kv_lens, scale: float, dv: int,
     assert out.stride(2) == 1 and out.stride(1) == dv
     rows, decode, parts = _latent_tiles(T, H, DK, block_tables, max_len)
     if sinks is not None or window > 0 or (rows and (out.data_ptr() % 16 or out.stride(0) % 8)):
-        rows, decode, parts = 0, False, MLAWorkspace.parts(T, H, DK if sinks is None and window <= 0 else 0)   # (0: the 16-head kernel)
+        rows, decode, parts = 0, False, MLAWorkspace.parts(T, H, DK if sinks is None and window <= 0 else 0, pages=block_tables.shape[1])   # (0: the 16-head kernel)
     if window > 0:   # at least four 32-key tiles of the window per partition (fewer only move partials around)
         parts = max(1, min(parts, window // 128))
     if ws is None and (parts > 1 or decode):

@@ -310,3 +310,24 @@ def test_mla_reads_no_partition_that_is_not_written(T, H):
                 continue
             want = _exact(q[t:t + 1], cache, bt[t:t + 1], row[:1], kl[t:t + 1], 192 ** -0.5)
             assert ((out[t:t + 1] - want).flatten(1).norm(dim=1) <= 2.0 ** -8 * want.flatten(1).norm(dim=1)).all(), (ctx, t)
+
+
+@pytest.mark.parametrize("pages,most", [(20, 16), (128, 16), (129, 64)])
+@pytest.mark.parametrize("window", [0, 4096])
+def test_latent_partitions_with_sinks_go_by_the_tables_width(monkeypatch, pages, most, window):
+    """Sinks and windows, which take the 16-head kernel: no more partitions than a table of that width is worth.  Tolerance as above."""
+    torch.manual_seed(pages)
+    n = 16 * pages - 5
+    cache, bt = _setup([16 * (pages - 1)])
+    assert bt.shape[1] == pages
+    q, sinks = torch.randn(1, 16, 576, device=DEV).to(torch.bfloat16), torch.randn(16, device=DEV)
+    row, kl = torch.zeros(1, dtype=torch.int32, device=DEV), torch.tensor([n], dtype=torch.int32, device=DEV)
+    parts, call = [], ops.call
+    monkeypatch.setattr(ops, "call", lambda fn, *a: (parts.append(a[13]), call(fn, *a)))
+    out = ops.latent_attn(q, cache, bt, row, kl, 192 ** -0.5, 512, sinks=sinks, window=window).cpu().double()
+    assert parts == [min(most, window // 128 if window else most)]
+    at = torch.arange(max(0, n - window) if window else 0, n)
+    kv = cache.cpu().double().view(-1, 576)[bt[0].cpu().long()[at // 16] * 16 + at % 16]
+    s = torch.cat([q[0].cpu().double() @ kv.T * 192 ** -0.5, sinks.cpu().double()[:, None]], 1).softmax(-1)[:, :-1]
+    want = s @ kv[:, :512]
+    assert (out[0] - want).norm() <= 2.0 ** -8 * want.norm()
