@@ -185,7 +185,8 @@ def _chunk_rule_seg(T: int, S: int, H: int, dv: int, delta: bool) -> int:
     delta rule, 8 heads 1 x 1000 87 -> 76, 1 x 4000 259 -> 127, 1 x 8000 489 -> 190, 2 x 4000 220 -> 120, 4 x 4000 113 -> 99; 32 heads
     1 x 1000 96 -> 91, 1 x 4000 299 -> 218, 2 x 4000 (128 workgroups) 243 -> 245; 1 x 300 46 -> 50;
     selective scan, 32 heads 1 x 1000 81 -> 55, 1 x 8000 435 -> 136, 4 x 4000 116 -> 92, 8 x 8000 (256) 130 -> 145; 128 heads
-    1 x 1000 95 -> 84, 1 x 8000 638 -> 440, 2 x 4000 (256) 220 -> 225; 1 x 300 42 -> 44."""
+    1 x 1000 95 -> 84, 1 x 8000 638 -> 440, 2 x 4000 (256) 220 -> 225; 1 x 300 42 -> 44.
+    Lengths are on the device, so decode rows beside a prompt count as sequences like it, and such a step stays in one piece."""
     wgs, chunks = H * -(-dv // 64) * S, -(-T // (32 * S))
     if chunks < 24 or wgs > (64 if delta else 192):
         return 0
