@@ -225,19 +225,24 @@ __global__ __launch_bounds__(256) void mla_attn_kernel(
 // the others.
 //   S^T [32 keys x 32 rows] = K . Q^T   (DK/16 MFMAs 32x32x16, lane = key / row, 8 dims a lane half)
 //   O^T [DV x 32] += V^T . P^T          (DV/32 x 2 MFMAs; V^T by hardware-transposed LDS reads, key order of S^T)
-// Nothing else runs on the SIMD meanwhile, so the loop is pipelined by hand: S^T of tile n + 1 is multiplied while
-// the softmax of tile n runs on the vector ALU, and the LDS DMA of tile n + 2 is in flight (three images).
+// Nothing else runs on the SIMD meanwhile, so the loop is pipelined by hand.  A product takes 32 cycles of the matrix cores and 4 of issue, so up
+// to six vector instructions beside it cost next to nothing: the softmax of tile n stands between the products of S^T of tile n + 1 (the
+// exponentials of its last 16 keys between those of O^T), and the nine moves of tile n + 3 one by one beside the last products of O^T (four
+// images; nine in a row hold a wave up for some 450 cycles).  A branch beside each product, taken or not, costs 40 cycles, so the loop
+// has none there.  Of 128 rows, 256 workgroups of 100 tiles that share their keys, a tile took 2.65 us with moves and softmax ahead of the products and
+// takes 2.42; its products alone take 1.65, the rate at which the card runs out of power (1380 TFLOP/s): the rest is LDS reads at 128 bytes a
+// cycle, which the products need all of, and waiting for the wave whose weights stand out most often.
 // O^T is rescaled only where a row's maximum rose by more than 2^8 since its last rescale (weights stay below
 // 2^8), almost never after a row's first tile.  A row's largest weight is then not exactly 1, as in the 16-head
 // kernel, so its rounding to bf16 counts: the keys with a weight that stands out are multiplied a second time with what
 // rounding took (16 keys of all rows at once; w^2 over 16, or of decode steps 6, times the mean of the squares of the
 // largest weight of each tile so far, or any that may come to a row's largest where there are fewer tiles than that).
 // The denominator sums the weights as they are used.  Error against 64 bits over the shapes of DeepSeek's heads
-// 0.0017..0.0018 of the result (16-head kernel 0.0017..0.0019; without the second product 0.0019..0.0021, 127 instead
-// of 146 us below).
+// 0.0017..0.0018 of the result (16-head kernel 0.0017..0.0019; without the second product 0.0019..0.0021, in 0.87 of the
+// time).
 //
 // Measured (16-head kernel, or for decode the 16-row waves before -> now): three prompts of 3394 rows x 16 heads
-// 738 -> 146 us (118 -> 598 TFLOP/s); decode, 48 contexts of ~3000 keys x 128 heads 100 -> 88 us.
+// 738 -> 135 us (118 -> 645 TFLOP/s); decode, 48 contexts of ~3000 keys x 128 heads 100 -> 86 us.
 // ------------------------------------------------------------------------------------------
 // The products by asm: with one wave per SIMD, what covers an LDS read is the distance to its product, and the
 // compiler sinks reads to their use (or hoists them all, into scratch).  Volatile with a memory clobber, each stays
@@ -254,11 +259,28 @@ __device__ __forceinline__ void mma_add(f32x16& c, bf16x8 a, bf16x8 b) {   // c 
   asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b) : "memory");
 #endif
 }
+__device__ __forceinline__ void mma_last(f32x16& d, bf16x8 a, bf16x8 b, const f32x16& c) {   // d = c + a b, which others may read
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %3\n\t" MMA_WAIT : "=&v"(d) : "v"(a), "v"(b), "v"(c) : "memory");
+#endif
+}
 __device__ __forceinline__ void mma_acc(f32x16& c, bf16x8 a, bf16x8 b) {   // c += a b, c in accumulation registers
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b) : "memory");
 #endif
 }
+
+__device__ __forceinline__ void mma_acc2(f32x16& c, bf16x8 a, bf16x8 b, bf16x8 b2, uint32_t both) {   // c += a b (+ a b2)
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0\n\ts_cmp_eq_u32 %4, 0\n\ts_cbranch_scc1 .Lone%=\n\t"
+               "v_mfma_f32_32x32x16_bf16 %0, %1, %3, %0\n.Lone%=:"
+               : "+a"(c) : "v"(a), "v"(b), "v"(b2), "s"(both) : "memory", "scc");
+#endif
+}
+
+// Chunk x of key row r lies at x ^ row_swz(r): the same chunk of 16 rows, and four chunks of four, in all of the 64 banks (rows are 9 times
+// half of them wide)
+__device__ __forceinline__ int row_swz(int r) { return (r >> 1 & 1) << 2 | (r >> 2 & 1) << 1 | (r >> 3 & 1); }
 
 // First token whose block-table row is e, by a 64-way search of the whole wave; -1: none.  tok_row ascends in the
 // runtime's prompts; of rows in any other order it may miss e, the same way for every caller.
@@ -339,7 +361,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
   constexpr int IMG = KT * CH * 16;   // bytes per key-tile image
   constexpr float LAZY = 8.f;
   constexpr int AHEAD = 4;            // LDS operands in flight: 4 x 32 cycles of matrix work cover a read
-  __shared__ __attribute__((aligned(16))) char sK[3 * IMG];
+  __shared__ __attribute__((aligned(16))) char sK[4 * IMG];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)sK;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   constexpr int RT = 32 * NW, SPAN = 2, UNITS = 256;
@@ -441,24 +463,44 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
     // Key tile -> LDS image: instruction i writes chunks [64 i, 64 i + 64) lane-linearly, each lane fetching the source
     // chunk that the row's XOR swizzle puts there.  A page is 16 rows x 72 chunks = 18 instructions, so each
     // instruction reads one page: its descriptor is based at that page.
-    // Nine instructions are 8 rows, after which the pattern repeats.
+    // Nine instructions are 8 rows; those of the next 8 differ in the chunk's lowest bit (row_swz).
     static_assert(9 * 64 == 8 * CH && NI == 36, "9 offsets a lane");
-    uint32_t dofs[9];
+    uint32_t dofs2[5] = {};   // two in a register (below 2^15)
 #pragma unroll
     for (int j = 0; j < 9; ++j) {
       const int c = 64 * ((wave + NW * j) % (NI / 2)) + lane, kr = c / CH;
-      dofs[j] = (kr * CH + ((c - kr * CH) ^ (kr & 7))) * 16;
+      dofs2[j >> 1] |= (uint32_t)((kr * CH + ((c - kr * CH) ^ row_swz(kr))) * 16) << 16 * (j & 1);
     }
-    auto dma = [&](const int* bt, int n_pages, int tile, int img) {
-      const int p0 = 2 * tile, p1 = p0 + 1;
-      const bf16* b0 = cache + (int64_t)bt[p0 < n_pages ? p0 : 0] * 16 * DK;
-      const bf16* b1 = cache + (int64_t)bt[p1 < n_pages ? p1 : 0] * 16 * DK;
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        const int i = wave + NW * j;
-        buffer_to_lds(j < NJ / 2 || (NW == 4 && i < NI / 2) ? b0 : b1, 16 * DK * 2, dofs[j % 9], NW == 1 && j / 9 % 2 ? 8 * CH * 16 : 0,
-                    lds0 + img * IMG + 64 * 16 * i);
-      }
+    // The pages of 32 tiles from `pg0` on, one a lane: a scalar load on its way would turn every wait for an LDS operand
+    // into one for all of them.
+    int pages = 0, pg0 = 0;
+    auto look = [&](int tile) {
+      const int p = 2 * tile + lane;
+#if defined(__HIP_DEVICE_COMPILE__)   // (waited for here: the compiler would wait before every use, and for the moves as well)
+      asm volatile("global_load_dword %0, %1, off\n\ts_waitcnt vmcnt(0)" : "=&v"(pages) : "v"(bt + (p < n_pages ? p : 0)) : "memory");
+#endif
+      pg0 = tile;
+    };
+    const bf16 *b0 = cache, *b1 = cache;   // pages of the tile on its way, its image, its descriptors' size
+    uint32_t to = 0, bytes = 0;
+    auto aim = [&](int tile, int img) {    // (of a tile past the last nothing is read, zeros are written)
+      if (tile < end && tile - pg0 == 32) look(tile);
+      const int at = 2 * (tile - pg0);
+      b0 = cache + (int64_t)__builtin_amdgcn_readlane(pages, at & 63) * 16 * DK;
+      b1 = cache + (int64_t)__builtin_amdgcn_readlane(pages, (at + 1) & 63) * 16 * DK;
+      to = lds0 + img * IMG;
+      bytes = tile < end ? 16 * DK * 2 : 0;
+      asm volatile("" : "+v"(dofs2[0]), "+v"(dofs2[1]), "+v"(dofs2[2]), "+v"(dofs2[3]), "+v"(dofs2[4]));   // (or the loop would hold them unpacked)
+    };
+    auto landed = [&](bool more) {   // the tile before the one that was moved last (`more`: if one was)
+      if (NW > 1 || more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NJ) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    };
+    auto dma = [&](int j) __attribute__((always_inline)) {
+      const int i = wave + NW * j;
+      const uint32_t two = dofs2[j % 9 >> 1], at = j % 9 & 1 ? two >> 16 : two & 0xffff;
+      buffer_to_lds(j < NJ / 2 || (NW == 4 && i < NI / 2) ? b0 : b1, bytes, NW == 1 && j / 9 % 2 ? at ^ 16 : at, NW == 1 && j / 9 % 2 ? 8 * CH * 16 : 0,
+                    to + 64 * 16 * i);
     };
 
     f32x16 o[NV];
@@ -467,14 +509,16 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
     // S^T reads chunk 2 s + hf of key row col; V^T reads, for 16-lane group gr = lane / 16, rows 4 hf + qr (+ 8, 16, 24)
     // and chunk 4 v + 2 (gr & 1) + pc / 2.
     const int gr = lane >> 4, qr = (lane & 15) >> 2, pc = lane & 3;
-    uint32_t sofs[4], vofs[2];
+    uint32_t sofs[4], vofs[2], vofs8[2];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) sofs[e] = (col * CH + ((2 * e + hf) ^ (col & 7))) * 16;
+    for (int e = 0; e < 4; ++e) sofs[e] = (col * CH + ((2 * e + hf) ^ row_swz(col))) * 16;
 #pragma unroll
-    for (int e = 0; e < 2; ++e)
-      vofs[e] = ((4 * hf + qr) * CH + ((4 * e + 2 * (gr & 1) + (pc >> 1)) ^ (4 * hf + qr))) * 16 + (pc & 1) * 8;
+    for (int e = 0; e < 2; ++e) {
+      vofs[e] = ((4 * hf + qr) * CH + ((4 * e + 2 * (gr & 1) + (pc >> 1)) ^ row_swz(4 * hf + qr))) * 16 + (pc & 1) * 8;
+      vofs8[e] = (vofs[e] ^ 16) + 8 * CH * 16;   // of the row 8 further on
+    }
     auto kfrag = [&](uint32_t img, int s) { return *reinterpret_cast<const bf16x8*>(sK + (sofs[s & 3] + img) + (s >> 2) * 128); };
-    auto score = [&](uint32_t img) {   // S^T of the tile in image `img` (byte offset)
+    auto score = [&](uint32_t img, f32x16& to, auto&& beside) __attribute__((always_inline)) {   // S^T of the tile in image `img` (byte offset)
       f32x16 a;
       bf16x8 k[AHEAD];   // operands on their way from LDS
 #pragma unroll
@@ -482,15 +526,16 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
         if (s == 0) mma_new(a, k[0], qf[0]);
-        else mma_add(a, k[s % AHEAD], qf[s]);
+        else if (s + 1 < NS) mma_add(a, k[s % AHEAD], qf[s]);
+        else mma_last(to, k[s % AHEAD], qf[s], a);
         if (s + AHEAD < NS) k[s % AHEAD] = kfrag(img, s + AHEAD);
+        beside(s);
+        __builtin_amdgcn_sched_barrier(0);   // what stands beside a product stays there
       }
-      asm volatile(MMA_WAIT : "+v"(a));
-      return a;
     };
     auto vfrag = [&](uint32_t img, int v, int st) {
-      const int at = vofs[v & 1] + img + (v >> 1) * 128 + st * 16 * CH * 16;
-      const bf16x4 x = tr_read(reinterpret_cast<const bf16*>(sK), at), y = tr_read(reinterpret_cast<const bf16*>(sK), at + 8 * CH * 16);
+      const int add = (v >> 1) * 128 + st * 16 * CH * 16;
+      const bf16x4 x = tr_read(reinterpret_cast<const bf16*>(sK), vofs[v & 1] + img + add), y = tr_read(reinterpret_cast<const bf16*>(sK), vofs8[v & 1] + img + add);
       return bf16x8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
     };
 
@@ -502,8 +547,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
     const float large = min((end - begin) * my_parts, DECODE ? 6 : 16);
     f32x16 sc;
     if (begin < end) {
-      dma(bt, n_pages, begin, 0);
-      if (begin + 1 < end) dma(bt, n_pages, begin + 1, 1);
+      look(begin);
+      aim(begin, 0);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) dma(j);
     }
 #pragma unroll
     for (int v = 0; v < NV; ++v)
@@ -512,48 +559,103 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
     if (begin < end) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
-      sc = score(0);
+      if constexpr (NW == 1) {
+#pragma unroll 1
+        for (int t = 1; t < 3 && begin + t < end; ++t) {
+          aim(begin + t, t);
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) dma(j);
+        }
+        score(0, sc, [](int) {});
+      } else {
+        score(0, sc, [&](int s) __attribute__((always_inline)) {   // the next two tiles' moves beside it
+          if (s % (NS / 2) == 0) aim(begin + 1 + s / (NS / 2), 1 + s / (NS / 2));
+          if (NW == 2) dma(s % NJ);
+          else if (s % 2 == 0) dma(s / 2 % NJ);
+        });
+      }
+      landed(begin + 2 < end);
+      __syncthreads();
     }
+    int Lmin = L;   // the wave's shortest row: tiles below it have no key to mask
+#pragma unroll
+    for (int x = 32; x > 0; x >>= 1) Lmin = min(Lmin, __shfl_xor(Lmin, x));
+    Lmin = __builtin_amdgcn_readfirstlane(Lmin);
     int cur = 0;
     for (int n = begin; n < end; ++n) {
-      const int nxt = cur == 2 ? 0 : cur + 1;
-      // image nxt + 1 was last read in the previous round, before its barrier
-      if (n + 2 < end) dma(bt, n_pages, n + 2, nxt == 2 ? 0 : nxt + 1);
-      const f32x16 sn = score(nxt * IMG);   // (after the last tile: of whatever is there, unused)
-      const int key = n * KT + 4 * hf;
-      float ma = OME_NEG_INF, mb = OME_NEG_INF;   // of the lane's keys of the first and second 16
+      const int nxt = (cur + 1) & 3;
+      aim(n + 3, (cur + 3) & 3);   // (that image was last read in the previous round, before its barrier)
+      if (NW == 1 && n + 3 < end)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        sc[i] = key + 8 * (i >> 2) + (i & 3) < L ? sc[i] * scale_log2 : OME_NEG_INF;
-        if (i < 8) ma = fmaxf(ma, sc[i]);
-        else mb = fmaxf(mb, sc[i]);
+        for (int j = 0; j < NJ; ++j) dma(j);
+      if ((n + 1) * KT > Lmin) {
+        const int key = n * KT + 4 * hf;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sc[i] = key + 8 * (i >> 2) + (i & 3) < L ? sc[i] : OME_NEG_INF;
       }
-      float mx = fmaxf(ma, mb);
-      {
-        auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-        mx = vmax_f32(__uint_as_float(w[0]), __uint_as_float(w[1]));
-      }
-      const bool rise = mx > m + LAZY;   // (also a row's first tile: m = -inf)
-      const float mn = rise ? mx : m, ms = mn == OME_NEG_INF ? 0.f : mn;
-      // keys of this half or that among which a row has a weight that stands out: used in two parts
-      const float wa = __builtin_amdgcn_exp2f(ma - ms), wb = __builtin_amdgcn_exp2f(mb - ms), wt = __builtin_amdgcn_exp2f(mx - ms);
-      const float far = large * peaks;
-      const uint64_t two[2] = {__ballot(!rise && wa * wa * walked > far), __ballot(!rise && wb * wb * walked > far)};
-      float ps = 0.f;   // of the weights as they are used: their rounding cancels in the quotient
+      // The softmax, in pieces that stand beside the products of the next tile's scores: up to six vector instructions beside each cost
+      // next to nothing.
+      float ma = OME_NEG_INF, mb = OME_NEG_INF;   // of the lane's keys of the first and second 16, unscaled
+      float mx, mn, ms, wt, ps = 0.f;             // ps: of the weights as they are used: their rounding cancels in the quotient
+      bool rise;
+      uint64_t two[2];
+      float p[16];
       bf16x8 pb[2];
+      const auto piece = [&](int s) __attribute__((always_inline)) {
+        if (s < 8) {
+          if (s < 4) ma = fmaxf(ma, fmaxf(sc[2 * s], sc[2 * s + 1]));
+          else mb = fmaxf(mb, fmaxf(sc[2 * s], sc[2 * s + 1]));
+        } else if (s == 8) {
+          mx = fmaxf(ma, mb);
+          auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+          mx = vmax_f32(__uint_as_float(w[0]), __uint_as_float(w[1])) * scale_log2;
+        } else if (s == 9) {
+          rise = mx > m + LAZY;   // (also a row's first tile: m = -inf)
+          mn = rise ? mx : m;
+          ms = mn == OME_NEG_INF ? 0.f : mn;
+        } else if (s == 10) {
+          // keys of this half or that among which a row has a weight that stands out: used in two parts
+          const float wa = __builtin_amdgcn_exp2f(ma * scale_log2 - ms), wb = __builtin_amdgcn_exp2f(mb * scale_log2 - ms);
+          const float far = large * peaks;
+          two[0] = __ballot(!rise && wa * wa * walked > far);
+          two[1] = __ballot(!rise && wb * wb * walked > far);
+        } else if (s == 11) {
+          wt = __builtin_amdgcn_exp2f(mx - ms);
+        }
+      };
+      const auto weights = [&](int i, int part) __attribute__((always_inline)) {   // of keys i and i + 1, in four pieces
+        if (part == 0) {
+          if (i < 8) p[i] = sc[i] * scale_log2 - ms, p[i + 1] = sc[i + 1] * scale_log2 - ms;
+          p[i] = __builtin_amdgcn_exp2f(p[i]);
+        } else if (part == 1) {
+          p[i + 1] = __builtin_amdgcn_exp2f(p[i + 1]);
+        } else if (part == 2) {
+          const bf16x2 h = {(bf16)p[i], (bf16)p[i + 1]};
+          pb[i >> 3][i & 7] = h[0];
+          pb[i >> 3][(i & 7) + 1] = h[1];
+        } else {
+          ps += (float)pb[i >> 3][i & 7] + (float)pb[i >> 3][(i & 7) + 1];
+        }
+      };
+      if (n + 1 < end) {
+        score(nxt * IMG, sc, [&](int s) __attribute__((always_inline)) {
+          piece(s);
+          if (s >= 12 && (s - 12) % 6 < 4) weights((s - 12) / 6 * 2, (s - 12) % 6);   // (the first half's)
+          if (s >= 12 && s < 20) p[s - 4] = sc[s - 4] * scale_log2 - ms;   // (the second half's follow beside O's products)
+        });
+      } else {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        sc[i] = __builtin_amdgcn_exp2f(sc[i] - ms);
-        pb[i >> 3][i & 7] = (bf16)sc[i];
-        ps += (float)pb[i >> 3][i & 7];
-      }
-      {
-        auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(ps), __float_as_uint(ps), false, false);
-        ps = __uint_as_float(w[0]) + __uint_as_float(w[1]);
+        for (int s = 0; s < 12; ++s) piece(s);
+#pragma unroll
+        for (int i = 0; i < 8; i += 2)
+#pragma unroll
+          for (int part = 0; part < 4; ++part) weights(i, part);
+#pragma unroll
+        for (int i = 8; i < 16; ++i) p[i] = sc[i] * scale_log2 - ms;
       }
       bf16x8 vf[AHEAD];
 #pragma unroll
-      for (int k = 0; k < AHEAD; ++k) vf[k] = vfrag(cur * IMG, k >> 1, k & 1);
+      for (int k = 0; k < AHEAD; ++k) vf[k] = vfrag(cur * IMG, k, 0);
       if (__ballot(rise && m != OME_NEG_INF)) {   // (a first tile has nothing to rescale: O^T and the sum are zero)
         const float alpha = rise && m != OME_NEG_INF ? __builtin_amdgcn_exp2f(m - mn) : 1.f;
         lsum *= alpha;
@@ -576,15 +678,22 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
           }
         asm volatile("s_nop 7" ::: "memory");
       }
-      lsum += ps;
       peaks += wt * wt;
       walked += 1.f;
       m = mn;
-      asm volatile("s_nop 3" : "+v"(pb[0]), "+v"(pb[1])::"memory");   // (written by the vector ALU just now)
+      asm volatile("s_nop 3" : "+v"(pb[0])::"memory");   // (written by the vector ALU just now)
 #pragma unroll
       for (int k = 0; k < 2 * NV; ++k) {
-        mma_acc(o[k >> 1], vf[k % AHEAD], pb[k & 1]);
-        if (k + AHEAD < 2 * NV) vf[k % AHEAD] = vfrag(cur * IMG, (k + AHEAD) >> 1, k & 1);
+        if (k == NV) asm volatile("s_nop 3" : "+v"(pb[1])::"memory");
+        mma_acc(o[k % NV], vf[k % AHEAD], pb[k / NV]);
+        if (k + AHEAD < 2 * NV) vf[k % AHEAD] = vfrag(cur * IMG, (k + AHEAD) % NV, (k + AHEAD) / NV);
+        if (k < NV) weights(8 + k / 4 * 2, k % 4);   // the second half's, beside the first half's products
+        if ((NW == 2 && k >= 14) || (NW == 4 && k >= 14 && k % 2 == 0)) dma(NW == 2 ? k - 14 : (k - 14) / 2);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      {
+        auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(ps), __float_as_uint(ps), false, false);
+        lsum += __uint_as_float(w[0]) + __uint_as_float(w[1]);
       }
 #pragma unroll
       for (int j = 0; j < 2; ++j)
@@ -595,7 +704,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
           float rs = 0.f;
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
-            pr[i] = (bf16)(sc[8 * j + i] - (float)pb[j][i]);
+            pr[i] = (bf16)(p[8 * j + i] - (float)pb[j][i]);
             rs += (float)pr[i];
           }
           auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(rs), __float_as_uint(rs), false, false);
@@ -607,11 +716,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
             if (v + AHEAD < NV) vf[v % AHEAD] = vfrag(cur * IMG, v + AHEAD, j);
           }
         }
-      sc = sn;
       cur = nxt;
-      asm volatile(MMA_WAIT "\n\ts_waitcnt vmcnt(0)" ::: "memory");   // tile n + 2 has landed
+      landed(n + 3 < end);   // (tile n + 2)
       __syncthreads();
     }
+    asm volatile(MMA_WAIT "\n\ts_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
 
     // ---- epilogue: O^T lane map dim = 32 v + 8 (i / 4) + 4 hf + i % 4, row = col ----
     const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
@@ -956,6 +1066,7 @@ static void mla_launch(const void* q, int64_t q_stride_t, const void* cache, con
                        int2* plan = nullptr, const float* sinks = nullptr, int window = -1) {
   // `rows`: query rows of a workgroup of the row-tile kernel (32 / 64 / 128, the caller's choice), 0: the
   // 16-head kernel, which alone has the sink term and the window, or many rows of 128 heads
+  if (rows > 0 && !(scale_log2 > 0.f)) rows = 0, parts = 1;   // (row tiles look for the largest score before they scale it)
   if constexpr (DK == 576) {
     if (rows > 0) {
       const unsigned units = (unsigned)(plan ? T * ((H + rows - 1) / rows) : ((int64_t)T * H + rows - 1) / rows);

@@ -183,6 +183,25 @@ def test_mla_row_tiles_of_prompts(monkeypatch, seqs, H, rows):
 
 
 @pytest.mark.parametrize("rows", [32, 64, 128])
+@pytest.mark.parametrize("decode", [False, True])
+@pytest.mark.parametrize("scale", [0.06, -0.06, 0.0])
+def test_mla_row_tiles_of_long_contexts(monkeypatch, rows, decode, scale):
+    """Pieces of 31 to 66 key tiles: the pages are looked up 32 tiles at a time and moves run three ahead of the products.
+    Scales that the row tiles leave to the 16-head kernel."""
+    torch.manual_seed(rows)
+    new = [1] * 5 if decode else [2, 5, 3]
+    ctx = [980, 1024, 1056, 1057, 2100][:len(new)]
+    cache, bt = _setup([a + n for a, n in zip(ctx, new)])
+    row = torch.tensor([s for s, n in enumerate(new) for _ in range(n)], dtype=torch.int32)
+    kl = torch.tensor([a + j + 1 for a, n in zip(ctx, new) for j in range(n)], dtype=torch.int32)
+    q = torch.randn(len(row), 16, 576, device=DEV).to(torch.bfloat16)
+    monkeypatch.setattr(ops.MLAWorkspace, "tiles", lambda T, H, DK, *a: (rows, decode, 1))
+    out = ops.mla_attn(q, cache, bt, row.to(DEV), kl.to(DEV), scale)
+    want = _exact(q, cache, bt, row, kl, scale)
+    assert (out.cpu().double() - want).abs().max() < 2.0 ** -8 * cache.float().abs().max().item()
+
+
+@pytest.mark.parametrize("rows", [32, 64, 128])
 @pytest.mark.parametrize("H", [16, 32, 64, 128])
 @pytest.mark.parametrize("lens", [[1, 0, 32, 33], [5000, 16, 700], [200, 31, 64, 65, 1] * 13, [40] * 260, list(range(1, 257))],
                          ids=lambda v: f"{len(v)}x{max(v)}")
