@@ -4,7 +4,8 @@
 // rows (unit-norm for DELTA, B / C for Mamba-2), g_i = exp(cum_i) the decay from the chunk's start up to and
 // with row i:
 //   DELTA   A_ij = beta_i exp(cum_i - cum_j) k_i.k_j (j < i),  T = (I + A)^-1,
-//           U = T R,  R_i = beta_i (v_i - g_i k_i S)                    Mamba-2   U_i = dt_i x_i
+//           U = T R,  R_i = beta_i (v_i - g_i k_i S)                    Mamba-2   U_i = dt_i x_i (P's columns and the last
+//                                                                            factors below take dt_i: x_i stays as it is)
 //   o_i = g_i q_i S + sum_{j <= i} P_ij U_j,  P_ij = exp(cum_i - cum_j) q_i.k_j     (+ D x_i)
 //       (DELTA: P U = (P T) R, so that o and U both follow from R)
 //   S'  = g_C S + sum_i exp(cum_C - cum_i) k_i U_i^T
@@ -16,7 +17,7 @@
 // (ops._chunk_rule_seg; S at a segment's end is linear in S at its start): whole layers of one prompt of 8000 rows, 8 heads of 128 x 128
 // 489 -> 195 us, 32 heads of 64 x 128 435 -> 158.  The state's error against 64 bits, eight prompts of 1000 to 8000 rows: 1.10e-7 both ways (8.55e-8).
 //
-// What bounds it: the instructions of a wave that has its SIMD almost for itself, 96 matrix (Mamba-2: 60) and some 250 (310) vector
+// What bounds it: the instructions of a wave that has its SIMD almost for itself, 96 matrix (Mamba-2: 54) and some 250 (270) vector
 // ones a chunk.  A product takes 16 cycles alone, but about 9 of them stay its own where vector instructions of 4 cycles fill
 // the rest, so a chunk is 2000 cycles of issue and as much again of LDS latency, address arithmetic and dependencies.  Hence the
 // next chunk moves to LDS by DMA, without a register or a store on the way; values and outputs move in pieces of four columns
@@ -24,7 +25,7 @@
 // Memory traffic hides behind that.  Two fp16 parts instead of three bf16 ones would take a quarter less time, but the state came out
 // 2.3 times further from 64 bits: an fp16 value below 2^-14 has no lower part.
 //   gated delta rule, 32 heads of 128 x 128, prompts of 1001 / 1435 / 1564 rows:   22 + 97 us (before: 24 + 123; row by row: 1098)
-//   selective scan, 128 heads of 64 x 128, 8 groups, 1033 / 926 / 1248 / 293 rows:  10 + 93 us (before: 11 + 116; row by row: 1745)
+//   selective scan, 128 heads of 64 x 128, 8 groups, 1033 / 926 / 1248 / 293 rows:  10 + 74 us (values scaled by dt in three parts: 80; before: 116; row by row: 1745)
 // Largest error of the state against 64 bits: 1.2e-7 (row by row: 2.0e-7) and 1.2e-7 (6.2e-7) of its norm.
 //
 // A chunk's products multiply the entries that causality zeroes as well, and 0 times an infinity or NaN is NaN, so a key,
@@ -34,7 +35,7 @@
 //
 // fp32 throughout: k and q enter the matrix cores as the bf16 values that they are (their norms, 1 / |k| and
 // 1 / (|q| sqrt(dk)), scale results), S and U as three bf16 parts that sum to the fp32 value exactly, at
-// 3/16 of the fp32 MFMA's time; T R and P U, where both operands are fp32, take the six products of their parts down to
+// 3/16 of the fp32 MFMA's time; T R and P T R, where both operands are fp32, take the six products of their parts down to
 // 2^-16 of the first (what is left out is below 2^-24, an fp32 rounding).  Decay exponents are summed in fp64 (differences of
 // a long sum).  The row-by-row kernels stay for decode steps (one row per sequence), few rows in all, dk other than 64 / 128, and
 // unaligned views of q and k.
@@ -50,7 +51,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // Workspace of one chunk, in bytes: (Mamba-2) of every group q k^T in fp32, which its heads share (they differ in their decays only,
 // which the scan applies: P itself would be 16 times the bytes); of every head (DELTA) the images of T and P T, each in three
-// bf16 parts, as LDS holds them, and its vectors, 32 floats each: DELTA a, b, c, d of the scan, then g_C;  Mamba-2 a, cum's upper and
+// bf16 parts, as LDS holds them, and its vectors, 32 floats each: DELTA a, b, c, d of the scan, then g_C;  Mamba-2 dt, cum's upper and
 // lower parts, c, d, then g_C.
 constexpr int MAT = RC * RC * 2;      // a part of a 32 x 32 matrix
 constexpr int VECS = 1024;            // the vectors, in whole LDS moves
@@ -180,6 +181,20 @@ __device__ __forceinline__ void split3(f32x4 x0, f32x4 x1, bf16x8 (&p)[3]) {
         b = __builtin_amdgcn_fdot2_f32_bf16(h, second, b, false);
       }
     }
+  }
+}
+
+// Four, by cutting the lower bits off: half as many instructions again, but a dot product waits for the products around it (20 cycles each way).
+// For a wave that has little else to do beside its products (Mamba-2's P: 85.4 -> 83.8 us of the prompts above; S and U so: 86 to 87).
+__device__ __forceinline__ void cut3(f32x4 x, bf16x4 (&p)[3]) {
+#pragma unroll
+  for (int t = 0; t < 3; ++t) {
+    uint32_t u[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) u[e] = __float_as_uint(x[e]);
+    p[t] = __builtin_bit_cast(bf16x4, u32x2{__builtin_amdgcn_perm(u[1], u[0], 0x07060302u), __builtin_amdgcn_perm(u[3], u[2], 0x07060302u)});
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] -= __uint_as_float(u[e] & 0xffff0000u);
   }
 }
 
@@ -453,7 +468,7 @@ __global__ __launch_bounds__(256) void ssm_gram_kernel(RuleArgs a) {
       vec[RC + row] = hi;
       vec[2 * RC + row] = (float)(cum - (double)hi);
       vec[3 * RC + row] = ok ? __expf(hi) : 0.f;
-      vec[4 * RC + row] = ok ? __expf((float)(total - cum)) : 0.f;
+      vec[4 * RC + row] = ok ? dt * __expf((float)(total - cum)) : 0.f;
       if (row == 0) vec[5 * RC] = __expf((float)total);
     }
   }
@@ -532,7 +547,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   const char* qp = reinterpret_cast<const char*>(a.q + (int64_t)r0 * a.stride + hk * DK);
   const char* gp = a.ws + (q0 / RC + s + j * a.seg) * ws_step + hk * group_bytes<DELTA>();
   const char* hp = a.ws + (q0 / RC + s + j * a.seg) * ws_step + a.Hk * group_bytes<DELTA>() + h * head_bytes<DELTA>();
-  f32x4 rp[NML], rhj[NML], rlj[NML];
+  f32x4 rp[NML], rhj[NML], rlj[NML], rdj[NML];
   float rhi[NML], rli[NML];
   bf16x8 rx;
   // The next chunk to LDS buffer b in three steps, for the vector memory unit to take one while another is computed.  `more`: there
@@ -565,6 +580,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
         rli[i] = *reinterpret_cast<const float*>(hp + (hi + 4 * RC));
         rhj[i] = *reinterpret_cast<const f32x4*>(hp + hj);
         rlj[i] = *reinterpret_cast<const f32x4*>(hp + (hj + 4 * RC));
+        rdj[i] = *reinterpret_cast<const f32x4*>(hp + (hj - 4 * RC));
       }
     }
   };
@@ -575,7 +591,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
     gp += more ? ws_step : 0;
     hp += more ? ws_step : 0;
   };
-  const auto put = [&](int b) {   // P_ij = q_i.k_j exp(cum_i - cum_j), j <= i; cum in two parts (long sums, short differences)
+  const auto put = [&](int b) {   // P_ij dt_j = q_i.k_j exp(cum_i - cum_j) dt_j, j <= i; cum in two parts (long sums, short differences)
     if constexpr (!VEC) *reinterpret_cast<bf16x8*>(lds + b * IMG + X_AT + 16 * tid) = rx;
     if constexpr (!DELTA && SEG != 1) {
 #pragma unroll
@@ -583,12 +599,12 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
         const int e = tid + NT * i, row = e / (RC / 4), j = 4 * (e % (RC / 4));
         f32x4 x;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) x[t] = j + t <= row ? rp[i][t] * __expf((rhi[i] - rhj[i][t]) + (rli[i] - rlj[i][t])) : 0.f;
-        bf16x8 p[3];
-        split3(x, f32x4{0.f, 0.f, 0.f, 0.f}, p);
+        for (int t = 0; t < 4; ++t) x[t] = j + t <= row ? rp[i][t] * __expf((rhi[i] - rhj[i][t]) + (rli[i] - rlj[i][t])) * rdj[i][t] : 0.f;
+        bf16x4 p[3];
+        cut3(x, p);
         const int at = b * IMG + M_AT + mat_img(row, (j & 15) >> 2) + 8 * (j >> 4);
 #pragma unroll
-        for (int m = 0; m < 3; ++m) *reinterpret_cast<bf16x4*>(lds + at + m * MAT) = bf16x4{p[m][0], p[m][1], p[m][2], p[m][3]};
+        for (int m = 0; m < 3; ++m) *reinterpret_cast<bf16x4*>(lds + at + m * MAT) = p[m];
       }
     }
   };
@@ -777,8 +793,10 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
       x[rb] = tr4(X, 8 * val_img(16 * rb + 4 * g + (col >> 2), 2 * wave + ((col >> 1) & 1)) + 4 * (col & 1));
-      va[rb] = vec(0, rb);
-      if constexpr (DELTA) vb[rb] = vec(1, rb);
+      if constexpr (DELTA) {
+        va[rb] = vec(0, rb);
+        vb[rb] = vec(1, rb);
+      }
     }
     __builtin_amdgcn_sched_barrier(0x0f);
     fetch(r1 - r0 - (c + 1) * RC, more, b ^ 1);   // (that buffer was read last before the previous barrier)
@@ -832,13 +850,12 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
     for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        r[rb][e] = va[rb][e] * (float)x[rb][e];
-        if constexpr (DELTA) r[rb][e] -= vb[rb][e] * ks[rb][e];
+        r[rb][e] = DELTA ? va[rb][e] * (float)x[rb][e] - vb[rb][e] * ks[rb][e] : (float)x[rb][e];
       }
     bf16x8 rs[3];
-    if constexpr (DELTA || SEG != 1) split3(r[0], r[1], rs);
+    if constexpr (DELTA) split3(r[0], r[1], rs);
     __builtin_amdgcn_sched_barrier(0x0f);
-    // ---- U = T R, o += (P T) R (Mamba-2: o += P U) ----
+    // ---- U = T R, o += (P T) R (Mamba-2: o += P dt x) ----
     bf16x8 ka[NB];
     {
       const int qr = 4 * g + (col >> 2), p4 = col & 3;
@@ -863,7 +880,15 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
     if constexpr (SEG != 1) {
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb) o[rb] *= vo[rb];
-      mma_parts<true>(DELTA ? pm : tm, rs, o);
+      if constexpr (DELTA) {
+        mma_parts<true>(pm, rs, o);
+      } else {   // the values as they are
+        const bf16x8 xv = {x[0][0], x[0][1], x[0][2], x[0][3], x[1][0], x[1][1], x[1][2], x[1][3]};
+#pragma unroll
+        for (int p = 2; p >= 0; --p)
+#pragma unroll
+          for (int rb = 0; rb < 2; ++rb) o[rb] = mma_bf16(xv, tm[rb][p], o[rb]);
+      }
     }
     // ---- S = g_C S + k^T U ----
     bf16x8 us[3];
