@@ -10,6 +10,7 @@ Two in-tree shared objects are produced (they travel to GPU boxes with the repo 
   safetensors header parser, multi-threaded pread -> pinned-host -> HBM loader,
   paged-KV block allocator, radix prefix cache.
 * ``ome_amd/_lib/libome_comm.so`` — xGMI peer-to-peer collectives (``csrc/comm``).
+* ``ome_amd/_lib/libome_call.so`` — a Python module that calls the launchers (``csrc/host``; ctypes does without it).
 
 Usage: ``python -m ome_amd.build [--force] [--jobs N]``.
 """
@@ -21,6 +22,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 ROOT = Path(__file__).resolve().parent.parent
@@ -95,12 +97,12 @@ def _check_loadable(lib: Path) -> None:
 
 def build(force: bool = False, jobs: int | None = None, verbose: bool = True,
           only: tuple[str, ...] | None = None) -> list[Path]:
-    """Build the native libraries (``only``: a subset of ome_kernels / omeio / ome_comm)."""
+    """Build the native libraries (``only``: a subset of ome_kernels / omeio / ome_comm / ome_call)."""
     jobs = jobs or min(8, os.cpu_count() or 4)
     hipcc = _hipcc()
     built = []
     kdir = CSRC / "kernels"
-    want = set(only or ("ome_kernels", "omeio", "ome_comm"))
+    want = set(only or ("ome_kernels", "omeio", "ome_comm", "ome_call"))
     if "ome_kernels" in want:
         built.append(_build_lib("ome_kernels", sorted(kdir.glob("*.hip")), sorted(kdir.glob("*.h")), hipcc,
                                 HIP_FLAGS, [], force, jobs))
@@ -115,6 +117,10 @@ def build(force: bool = False, jobs: int | None = None, verbose: bool = True,
     if comm_src and "ome_comm" in want:
         built.append(_build_lib("ome_comm", comm_src, sorted(cdir.glob("*.h")) + [kdir / "common.h"], hipcc,
                                 HIP_FLAGS + [f"-I{kdir}"], [], force, jobs))
+    include = Path(sysconfig.get_paths()["include"])
+    if "ome_call" in want and (include / "Python.h").exists():
+        built.append(_build_lib("ome_call", sorted((CSRC / "host").glob("*.cpp")), [], shutil.which("g++") or "c++",
+                                [*CXX_FLAGS, f"-I{include}"], [], force, jobs))
     if verbose:
         for b in built:
             print(f"[ome_amd.build] {b.relative_to(ROOT)}  ({b.stat().st_size // 1024} KiB)")

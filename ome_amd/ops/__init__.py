@@ -138,7 +138,7 @@ def ssm_conv1d(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, stat
     """Mamba causal depthwise conv1d + SiLU over varlen sequences (rows ``cu[s]:cu[s+1]``), continuing
     from and updating ``state`` [slots, C, K-1]; ``reset[s]`` = 1 starts sequence ``s`` from zeros."""
     T, C = x.shape
-    out = torch.empty(T, C, dtype=x.dtype, device=x.device) if out is None else out
+    out = x.new_empty(T, C) if out is None else out
     if not _gpu(x):
         return ref.ssm_conv1d(x, w, bias, state, cu, slot, reset, out)
     assert x.stride(1) == 1 and out.stride(1) == 1 and w.is_contiguous() and state.is_contiguous()
@@ -217,7 +217,7 @@ def _chunk_rule_ws(T: int, S: int, H: int, G: int, dk: int, dv: int, delta: bool
     seg = _chunk_rule_seg(T, S, H, dv, delta)
     if seg:
         floats += (T // (32 * seg) + S) * H * _chunk_rule_seg_floats(dk, dv)
-    return torch.empty(floats + 256, dtype=torch.float32, device=state.device)[:floats]   # (the sequences' order lies behind)
+    return state.new_empty(floats + 256, dtype=torch.float32)[:floats]   # (the sequences' order lies behind)
 
 
 def ssm_scan(x, dt, B, C, A, D, dt_bias, dt_min: float, state, cu, slot, reset, H: int, P: int, N: int, G: int,
@@ -225,7 +225,7 @@ def ssm_scan(x, dt, B, C, A, D, dt_bias, dt_min: float, state, cu, slot, reset, 
     """Mamba-2 selective scan, recurrent over each sequence's rows: x [T, H*P], dt [T, H], B/C
     [T, G*N] (row-strided views are fine), A/D/dt_bias fp32 [H], state fp32 [slots, H, P, N]."""
     T = x.shape[0]
-    out = torch.empty(T, H * P, dtype=x.dtype, device=x.device) if out is None else out
+    out = x.new_empty(T, H * P) if out is None else out
     if not _gpu(x):
         return ref.ssm_scan(x, dt, B, C, A, D, dt_bias, dt_min, state, cu, slot, reset, H, P, N, G, out)
     assert B.stride(0) == C.stride(0) and B.stride(1) == 1 and x.stride(1) == 1 and dt.stride(1) == 1
@@ -254,7 +254,7 @@ def gdn_scan(q, k, v, a, b, A_log, dt_bias, state, cu, slot, reset, Hv: int, Hk:
     kernel."""
     T = q.shape[0]
     dv, dk = state.shape[2], state.shape[3]
-    out = torch.empty(T, Hv * dv, dtype=v.dtype, device=v.device) if out is None else out
+    out = v.new_empty(T, Hv * dv) if out is None else out
     if not _gpu(q):
         return ref.gdn_scan(q, k, v, a, b, A_log, dt_bias, state, cu, slot, reset, Hv, Hk, out)
     assert q.stride(0) == k.stride(0) == v.stride(0) and a.stride(0) == b.stride(0)
@@ -297,7 +297,7 @@ def gated_rmsnorm(y: torch.Tensor, z: torch.Tensor, w: torch.Tensor, group: int,
     if not _gpu(y):
         return ref.gated_rmsnorm(y, z, w, group, eps, norm_first, exact, gate)
     T, I = y.shape
-    out = torch.empty(T, I, dtype=y.dtype, device=y.device)
+    out = y.new_empty(T, I)
     call("ome_gated_rmsnorm", y.data_ptr(), y.stride(0), z.data_ptr(), z.stride(0), w.data_ptr(), out.data_ptr(),
          out.stride(0), T, I, group, float(eps), int(norm_first) | (2 if exact else 0) | (4 if gate == "sigmoid" else 0),
          _f32(y, z, w), stream_ptr())
@@ -354,7 +354,7 @@ def act_and_mul(x: torch.Tensor, act: int = 0, out: torch.Tensor | None = None,
     I = x.shape[-1] // 2
     rows = x.numel() // x.shape[-1]
     assert x.is_contiguous()
-    out = torch.empty(*x.shape[:-1], I, dtype=x.dtype, device=x.device) if out is None else out
+    out = x.new_empty(*x.shape[:-1], I) if out is None else out
     code = act | (16 if interleaved else 0) | (32 if _f32(x, out) else 0)
     if row_gate is not None:
         assert row_gate.dtype == torch.float32 and row_gate.dim() == 1 and row_gate.shape[0] == rows
@@ -737,8 +737,8 @@ def moe_route(logits: torch.Tensor, k: int, renorm: bool = True, scoring: str = 
             return out_w, out_ids
         return w, ids
     T, E = logits.shape
-    out_w = torch.empty(T, k, dtype=torch.float32, device=logits.device) if out_w is None else out_w
-    out_ids = torch.empty(T, k, dtype=torch.int32, device=logits.device) if out_ids is None else out_ids
+    out_w = logits.new_empty(T, k, dtype=torch.float32) if out_w is None else out_w
+    out_ids = logits.new_empty(T, k, dtype=torch.int32) if out_ids is None else out_ids
     for b in (bias, logit_bias):
         assert b is None or (b.dtype == torch.float32 and b.is_contiguous() and b.numel() == E)
     call("ome_moe_route", logits.data_ptr(), int(logits.dtype == torch.bfloat16), logits.stride(0), T, E, k,
@@ -776,7 +776,7 @@ class _Sorted:
     def __init__(self, ids: torch.Tensor, E: int, bm: int = 0, e_tiles: int | None = None):
         n = ids.numel()
         self.max_tiles = min(n, E) + n // bm if bm else 0
-        m = self.meta = torch.empty(4 * self.max_tiles + E + 1 + 2 * n, dtype=torch.int32, device=ids.device)
+        m = self.meta = ids.new_empty(4 * self.max_tiles + E + 1 + 2 * n, dtype=torch.int32)
         self.inv = m[m.numel() - n:]
         self.tiles = m.data_ptr()
         self.offsets = self.tiles + 16 * self.max_tiles
@@ -797,7 +797,7 @@ def _moe_pp(x: torch.Tensor, ids: int | None, div: int, w: torch.Tensor, offsets
             x.stride(0) % 8 or x.stride(1) != 1 or (x.data_ptr() | w.data_ptr()) % 16 or not w.is_contiguous() or \
             x.shape[0] * x.stride(0) >= 1 << 30 or N * K >= 1 << 30:
         return None
-    out = torch.empty(rows, N // 2 if silu else N, dtype=x.dtype, device=x.device)
+    out = x.new_empty(rows, N // 2 if silu else N)
     call("ome_moe_gemm_pp", x.data_ptr(), x.stride(0), x.shape[0], ids, div, w.data_ptr(), offsets, E, N, K,
          rows, out.data_ptr(), out.stride(0), ptr(bias), 2 if silu else 0, stream_ptr())
     return out
@@ -855,7 +855,7 @@ def _moe_gemm(x: torch.Tensor, s: _Sorted, ids: int | None, div: int, w: torch.T
     """Grouped GEMM of the first E experts on 64- or 128-row tiles (:func:`moe_tile_m`)."""
     N, K = w.shape[1:]
     E = E or w.shape[0]
-    out = torch.empty(rows, N, dtype=x.dtype, device=x.device)
+    out = x.new_empty(rows, N)
     tm = moe_tile_m(rows, E, N)
     if tm == 64 and K % 64 == 0 and x.stride(0) % 8 == 0 and w.data_ptr() % 16 == 0:
         # (rows that start on no 16-byte boundary: a copy of them for the streamed tiles.  Whole layers, us, tiles that search -> this: 128 experts with 70
@@ -872,7 +872,7 @@ def _moe_gemm(x: torch.Tensor, s: _Sorted, ids: int | None, div: int, w: torch.T
 def _combine(y, topk_w, inv, T, k, H, scale, add):
     if add is not None:
         assert add.shape == (T, H) and add.is_contiguous() and add.dtype == y.dtype
-    out = add if add is not None else torch.empty(T, H, dtype=y.dtype, device=y.device)
+    out = add if add is not None else y.new_empty(T, H)
     call("ome_moe_combine_add", y.data_ptr(), topk_w.data_ptr(), inv.data_ptr(), T, k, H, out.data_ptr(), ptr(add),
          float(scale), stream_ptr())
     return out
@@ -1146,7 +1146,7 @@ def mla_attn(q, cache, block_tables, tok_row, kv_lens, scale: float, ws: MLAWork
     assert (DK, dv) in ((576, 512), (288, 256)), (DK, dv)
     assert q.stride(2) == 1 and q.stride(1) == DK and cache.shape[-1] == DK
     if out is None:
-        out = torch.empty(T, H, dv, dtype=q.dtype, device=q.device)
+        out = q.new_empty(T, H, dv)
     rows, decode, parts = _latent_tiles(T, H, DK, block_tables, max_len)
     if rows and (out.data_ptr() % 16 or out.stride(0) % 8):
         rows, decode, parts = 0, False, MLAWorkspace.parts(T, H, DK, pages=block_tables.shape[1])
@@ -2276,7 +2276,7 @@ def latent_attn(q, cache, block_tables, tok_row, kv_lens, scale: float, dv: int,
     assert q.dtype == torch.bfloat16 and cache.dtype == torch.bfloat16 and cache.is_contiguous()
     assert q.stride(2) == 1 and q.stride(1) == DK and cache.shape[-1] == DK and cache.shape[-2] == 16
     if out is None:
-        out = torch.empty(T, H, dv, dtype=q.dtype, device=q.device)
+        out = q.new_empty(T, H, dv)
     assert out.stride(2) == 1 and out.stride(1) == dv
     rows, decode, parts = _latent_tiles(T, H, DK, block_tables, max_len)
     if sinks is not None or window > 0 or (rows and (out.data_ptr() % 16 or out.stride(0) % 8)):

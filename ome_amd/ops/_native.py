@@ -15,6 +15,8 @@ import os
 import threading
 from pathlib import Path
 
+import torch
+
 # OME_LIB_DIR: load the native libraries from another in-tree directory (compiler-flag A/B runs,
 # scripts/build_variant.py); default ome_amd/_lib
 # (a library missing there comes from the default directory)
@@ -206,6 +208,8 @@ def load(name: str = "ome_kernels") -> C.CDLL:
             f = getattr(lib, fn)
             f.argtypes = argt
             f.restype = C.c_int
+            if name == "ome_kernels" and _caller is not None and all(a in _KINDS for a in argt):
+                _caller.bind(fn, C.cast(f, vp).value, "".join(_KINDS[a] for a in argt))
         _libs[name] = lib
         return lib
 
@@ -218,17 +222,41 @@ def available(name: str = "ome_kernels") -> bool:
         return False
 
 
-def call(fn: str, *args, lib: str = "ome_kernels") -> None:
-    rc = getattr(load(lib), fn)(*args)
+def _fail(fn: str, rc: int) -> None:
+    raise NativeError(f"{fn} failed with code {rc}")
+
+
+def _slow_call(fn: str, *args) -> None:
+    rc = getattr(load("ome_kernels"), fn)(*args)
     if rc != 0:
-        raise NativeError(f"{fn} failed with code {rc}")
+        _fail(fn, rc)
+
+
+def _load_caller():
+    """The module that calls launchers without ctypes (``csrc/host/ome_call.cpp``), or None where it was not built."""
+    path = lib_path("ome_call")
+    if not path.exists():
+        return None
+    import importlib.machinery
+    import importlib.util
+
+    loader = importlib.machinery.ExtensionFileLoader("ome_call", str(path))
+    spec = importlib.util.spec_from_file_location("ome_call", str(path), loader=loader)
+    module = importlib.util.module_from_spec(spec)
+    loader.exec_module(module)
+    return module
+
+
+_KINDS = {vp: "p", i32: "i", i64: "l", u64: "l", f32: "f"}
+_caller = _load_caller()
+if _caller is not None:   # (names and arguments that it does not know come back to ctypes, the first call of all, which loads the library, too)
+    _caller.hooks(_slow_call, _fail)
+call = _slow_call if _caller is None else _caller.call
 
 
 def stream_ptr(device=None) -> int:
     """Handle of the current stream (of ``device``: the current one).  Asked of torch's C++ side: a ``torch.cuda.Stream`` made
     to read its handle took 2.9 us a launch, as long as the launch; this 0.4."""
-    import torch
-
     if device is not None:
         return torch.cuda.current_stream(device).cuda_stream
     return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
