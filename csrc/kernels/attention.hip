@@ -22,6 +22,7 @@
 // registers just before the MFMA; the host folds k_scale into the softmax scale and the
 // kernels multiply the normalised output by v_scale.
 #include "common.h"
+#include "prefill_pair.h"
 
 #include <cstdlib>
 
@@ -880,8 +881,8 @@ constexpr int PF_KLD = 128 + 8, PF_VLD = 32 + 8;
 // workgroup latency-bound on its serial chain of K/V tile loads; partial (O, m, l) per part go
 // to fp32 workspaces and prefill_combine_kernel merges them.
 //
-// FAST: plain causal attention (no soft-capping, ALiBi, window or row_hi) -- the Llama / Qwen /
-// Mixtral prefill.  The generic per-score code (soft-cap select, ALiBi term, window and row_hi
+// FAST: plain causal attention (no soft-capping, ALiBi, window or row_hi) -- block-sparse layers, fp8 caches of few items and
+// items of 64 rows; the Llama / Qwen / Mixtral prefill otherwise is prefill_pair.hip's.  The generic per-score code (soft-cap select, ALiBi term, window and row_hi
 // bounds, each a per-element branch) made the loop VALU-issue bound at ~3.3 us per 64-key step
 // (8x the MFMA time, profiles/r03_prefill_attn_fast.txt).  The fast body keeps raw scores, masks
 // only diagonal stages (key <= qpos also bounds kv_len), folds the scale into the exp2 FMA,
@@ -889,11 +890,9 @@ constexpr int PF_KLD = 128 + 8, PF_VLD = 32 + 8;
 // rescales O / l lazily (only when some row's max grew by more than 2^8).
 // NW = waves per workgroup: 4 (one 32-row block per head of the kv group) or 8 (two row blocks:
 // 64-row items, every K/V stage staged once for twice the query rows, one chunk per thread).
-// PROBE (timing diagnostics, wrong results by design; OME_PREFILL_PROBE): 1 = no V image stores,
-// 2 = no K/V global loads, 3 = identity pages (no block-table loads before the K/V loads).
 // BS (FAST only): block-sparse layer -- skip the key stages no head of the kv group sees and mask
 // this head's invisible keys (a separate instantiation: the dense kernels keep their registers).
-template <int SUB, int F, int SPLIT, bool FAST = false, int NW = 4, int PROBE = 0, bool BS = false>
+template <int SUB, int F, int SPLIT, bool FAST = false, int NW = 4, bool BS = false>
 __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_prefill_v2_kernel(
     const bf16* __restrict__ q, int64_t q_stride, const typename KVStore<F>::T* __restrict__ k_cache,
     const typename KVStore<F>::T* __restrict__ v_cache, const int* __restrict__ block_tables, int bt_stride,
@@ -986,19 +985,12 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_prefill_v2_kernel(
   // stage the loop was latency-bound at ~3.9 us per 64-key step (profiles/r03_prefill_*).
   Raw8 rkA[SUB][PT], rvA[SUB][PT], rkB[SUB][PT], rvB[SUB][PT];
   auto load_tile = [&](Raw8 (&rk)[SUB][PT], Raw8 (&rv)[SUB][PT], int kb0) {
-    if constexpr (PROBE == 2) {
-#pragma unroll
-      for (int u = 0; u < SUB; ++u)
-#pragma unroll
-        for (int i = 0; i < PT; ++i) asm volatile("" : "+v"(rk[u][i]), "+v"(rv[u][i]));
-      return;
-    }
 #pragma unroll
     for (int u = 0; u < SUB; ++u) {
       const int kb = kb0 + 32 * u;
       const int pi = kb / P;
-      const int pA = PROBE == 3 ? pi : (kb < kv_len) ? bt[pi] : bt[0];  // out-of-range subtiles: any valid page (masked)
-      const int pB = PROBE == 3 ? pi + 1 : (kb + P < kv_len) ? bt[pi + 1] : pA;
+      const int pA = (kb < kv_len) ? bt[pi] : bt[0];  // out-of-range subtiles: any valid page (masked)
+      const int pB = (kb + P < kv_len) ? bt[pi + 1] : pA;
 #pragma unroll
       for (int i = 0; i < PT; ++i) {
         const int c = tid + 64 * NW * i;
@@ -1019,10 +1011,6 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_prefill_v2_kernel(
         const int c = tid + 64 * NW * i;
         const int key = c >> 4, dc = c & 15;
         *reinterpret_cast<bf16x8*>(&sK[buf][u][key * PF_KLD + dc * 8]) = k8_bf16<F>(rk[u][i]);
-        if constexpr (PROBE == 1) {
-          asm volatile("" ::"v"(rv[u][i]));
-          continue;
-        }
         const int page = c >> 8, dim = (c & 255) >> 1, half = c & 1;
         bf16* vrow = &sV[buf][u][dim * PF_VLD];
         const bf16x8 vv = k8_bf16<F>(rv[u][i]);
@@ -1319,12 +1307,13 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const int4* __rest
                                                               const float* __restrict__ part_o,
                                                               const float* __restrict__ part_ml,
                                                               bf16* __restrict__ out, int64_t out_stride, int Hkv,
-                                                              float v_scale, const float* __restrict__ sinks) {
+                                                              float v_scale, const float* __restrict__ sinks, bool pair) {
   constexpr int D = 128;
   const int4 c = comb[blockIdx.x >> 2];
   const int s = c.x, p0 = c.z, np = c.w;
   const int head = blockIdx.y, kvh = head >> 2, w = head & 3;
-  const int r = 8 * (blockIdx.x & 3) + (threadIdx.x >> 5), quad = threadIdx.x & 31;
+  // (pair: prefill_pair.hip's order, 16 bytes of every row, then the next 16; read in runs of 128 bytes: 47 items of some 250 tiles 15.1 us, 16.2 in runs of 32)
+  const int r = 8 * (blockIdx.x & 3) + (pair ? threadIdx.x & 7 : threadIdx.x >> 5), quad = pair ? threadIdx.x >> 3 : threadIdx.x & 31;
   const int q0 = cu_q[s], q_len = cu_q[s + 1] - q0;
   const int row = c.y + r;
   if (row >= q_len) return;
@@ -1336,11 +1325,12 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const int4* __rest
   const float Mu = M == OME_NEG_INF ? 0.f : M;
   float L = sinks ? fast_exp2(sink - Mu) : 0.f;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  const int at = pair ? (quad >> 1) * 256 + (quad & 1) * 128 + r * 4 : r * D + 4 * quad;
 #pragma unroll 4
   for (int p = 0; p < np; ++p) {
     const int64_t pw = pw_of(p);
     const float2 ml = *reinterpret_cast<const float2*>(part_ml + (pw * 32 + r) * 2);
-    const f32x4 ov = *reinterpret_cast<const f32x4*>(part_o + (pw * 32 + r) * D + 4 * quad);
+    const f32x4 ov = *reinterpret_cast<const f32x4*>(part_o + pw * 32 * D + at);
     const float wt = fast_exp2(ml.x - Mu);
     L += wt * ml.y;
     acc += wt * ov;
@@ -1360,7 +1350,7 @@ static bool prefill_fast(const Scaler& scl, int window, const int* row_hi) {
     const char* e = getenv("OME_PREFILL_FAST");
     return e && atoi(e) == 0;
   }();
-  return !off && scl.cap_inv == 0.f && scl.alibi == nullptr && row_hi == nullptr &&
+  return !off && scl.mul > 0.f && scl.cap_inv == 0.f && scl.alibi == nullptr && row_hi == nullptr &&
          (window == -1 || window == 0);
 }
 
@@ -1374,7 +1364,7 @@ static void launch_prefill(int variant, int rows, int G, dim3 grid, hipStream_t 
   if constexpr (D == 128) {
     if (variant == 2 && G == 4) {  // one head per wave over 32-row items (GQA-4: Llama-3, Qwen3, Mixtral)
 #define OME_PF2B(FAST, NW, BS)                                                                                    \
-  paged_prefill_v2_kernel<2, F, 0, FAST, NW, 0, BS><<<grid.x * grid.y, 64 * NW, 0, stream>>>(                            \
+  paged_prefill_v2_kernel<2, F, 0, FAST, NW, BS><<<grid.x * grid.y, 64 * NW, 0, stream>>>(                            \
       (const bf16*)q, q_stride, (const T*)k_cache, (const T*)v_cache, block_tables, bt_stride, cu_q, kv_lens,      \
       (const int2*)items, (bf16*)out, out_stride, Hq, Hkv, scl, window, v_scale, sinks, row_hi, 0, 0, nullptr, nullptr)
 #define OME_PF2(FAST, NW) OME_PF2B(FAST, NW, false)
@@ -1387,21 +1377,15 @@ static void launch_prefill(int variant, int rows, int G, dim3 grid, hipStream_t 
       } else if (bs_fast) {
         OME_PF2B(true, 4, true);
       } else {
-        static const int probe = getenv("OME_PREFILL_PROBE") ? atoi(getenv("OME_PREFILL_PROBE")) : 0;
-        if (!bs && prefill_fast(scl, window, row_hi)) {
-#define OME_PF2P(PR)                                                                                              \
-  paged_prefill_v2_kernel<2, F, 0, true, 4, PR><<<grid.x * grid.y, 256, 0, stream>>>(                                    \
-      (const bf16*)q, q_stride, (const T*)k_cache, (const T*)v_cache, block_tables, bt_stride, cu_q, kv_lens,      \
-      (const int2*)items, (bf16*)out, out_stride, Hq, Hkv, scl, window, v_scale, sinks, row_hi, 0, 0, nullptr, nullptr)
-          bool done = false;
-          if constexpr (F == KV_BF16) {   // diagnostic instantiations for the bf16 cache only
-            done = probe >= 1 && probe <= 3;
-            if (probe == 1) OME_PF2P(1);
-            else if (probe == 2) OME_PF2P(2);
-            else if (probe == 3) OME_PF2P(3);
-          }
-          if (!done) OME_PF2(true, 4);
-#undef OME_PF2P
+        const bool fast = !bs && prefill_fast(scl, window, row_hi);
+        // An fp8 cache's tiles are converted by two waves there and by four here: of up to one round of workgroups, which are as long as their
+        // longest, 80 of 300 keys 15.7 against 14.4 us, 376 of 1500 51.9 against 51.0, 512 of 256 18.0 against 17.2 (500 rows over 900 keys: 38.6
+        // against 39.8); 528 of some 2000 80 against 89.
+        if (F != KV_BF16 && fast && (int64_t)grid.x * grid.y <= 512) {
+          if constexpr (F != KV_BF16) OME_PF2(true, 4);
+        } else if (fast) {
+          ome_prefill_pair({(const bf16*)q, q_stride, k_cache, v_cache, block_tables, bt_stride, cu_q, kv_lens, items, 0, 0, nullptr, nullptr, (bf16*)out,
+                            out_stride, Hkv, scl.mul, v_scale, sinks}, F, 0, grid.x * grid.y, stream);
         } else {
           OME_PF2(false, 4);
         }
@@ -1483,18 +1467,21 @@ OME_API int ome_paged_prefill_split(const void* q, int64_t q_stride, const void*
   // in a window of 4096): a workgroup a piece
   const bool runs = n_blocks > 0 && fast;
   const int grid = (runs ? n_blocks : n_items) * Hkv, listed = n_blocks > 0 ? n_items : 0;
+  const bool pair = fast && scl.bs_shift == 0;
+  if (pair)
+    ome_prefill_pair({(const bf16*)q, q_stride, k_cache, v_cache, block_tables, bt_stride, cu_q, kv_lens, items4, listed, chunk, (float*)part_o,
+                      (float*)part_ml, (bf16*)out, out_stride, Hkv, scl.mul, v_scale, sinks}, kv_fmt, runs ? 2 : 1, grid, stream);
 #define OME_PFS(F, SPLIT, FAST, BS)                                                                               \
-  paged_prefill_v2_kernel<2, F, SPLIT, FAST, 4, 0, BS><<<grid, 256, 0, stream>>>(                                 \
+  paged_prefill_v2_kernel<2, F, SPLIT, FAST, 4, BS><<<grid, 256, 0, stream>>>(                                 \
       (const bf16*)q, q_stride, (const typename KVStore<F>::T*)k_cache, (const typename KVStore<F>::T*)v_cache,    \
       block_tables, bt_stride, cu_q, kv_lens, (const int2*)items4, (bf16*)out, out_stride, Hq, Hkv, scl, window,   \
       v_scale, sinks, nullptr, chunk, listed, (float*)part_o, (float*)part_ml)
 #define OME_PFS_F(F)                                                                                              \
   if (!fast) OME_PFS(F, 1, false, false);                                                                         \
-  else if (scl.bs_shift >= 6 && runs) OME_PFS(F, 2, true, true);                                                  \
-  else if (scl.bs_shift >= 6) OME_PFS(F, 1, true, true);                                                          \
-  else if (runs) OME_PFS(F, 2, true, false);                                                                      \
-  else OME_PFS(F, 1, true, false)
-  if (kv_fmt == KV_BF16) {
+  else if (runs) OME_PFS(F, 2, true, true);                                                                       \
+  else OME_PFS(F, 1, true, true)
+  if (pair) {
+  } else if (kv_fmt == KV_BF16) {
     OME_PFS_F(KV_BF16);
   } else if (kv_fmt == KV_E4M3) {
     OME_PFS_F(KV_E4M3);
@@ -1507,7 +1494,7 @@ OME_API int ome_paged_prefill_split(const void* q, int64_t q_stride, const void*
   if (n_comb > 0) {
     prefill_combine_kernel<<<dim3(4 * n_comb, Hq), 256, 0, stream>>>((const int4*)comb, cu_q, (const float*)part_o,
                                                                   (const float*)part_ml, (bf16*)out, out_stride, Hkv,
-                                                                  v_scale, sinks);
+                                                                  v_scale, sinks, pair);
     OME_CHECK_LAUNCH();
   }
   return 0;
