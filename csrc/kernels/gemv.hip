@@ -42,8 +42,9 @@ __device__ __forceinline__ bf16x8 ldx8(const bf16* p, int K) {
 //   SWIGLU: W is gate / up interleaved in 16-row blocks; a wave takes R / 2 gate rows and their up rows.
 //   QKV:    a wave takes R / 2 dims d of a head and their partners d + D / 2, rotates them and writes q or the cache.
 // Both round the projection to bf16 first, as its own store did: the results are the same bits.
-// A decode step of one request (Llama-3-8B, 700 tokens of context): 3.69 -> 3.57 ms with both.
-enum { PLAIN = 0, SWIGLU = 1, QKV = 2 };
+//   ADD:    out += the projection, the residual stream's sum ahead of a norm that is folded into the next product (gemm_rows.hip).
+// A decode step of one request (Llama-3-8B, 700 tokens of context): 3.69 -> 3.57 ms with the first two.
+enum { PLAIN = 0, SWIGLU = 1, QKV = 2, ADD = 3 };
 struct GemvQkv {
   const int *positions, *slots;
   const float* cos_sin;
@@ -53,10 +54,10 @@ struct GemvQkv {
   float k_inv, v_inv;
 };
 
-// weight row r of the R rows of a wave that begins at row (PLAIN) or output pair n0 / 2
+// weight row r of the R rows of a wave that begins at row (PLAIN, ADD) or output pair n0 / 2
 template <int R, int EPI>
 __device__ __forceinline__ int weight_row(int n0, int r, int N, int D) {
-  if constexpr (EPI == PLAIN) return min(n0 + r, N - 1);   // clamp: rows past N are computed, not stored
+  if constexpr (EPI == PLAIN || EPI == ADD) return min(n0 + r, N - 1);   // clamp: rows past N are computed, not stored
   const int p = n0 / 2 + r % (R / 2), up = r / (R / 2);
   if constexpr (EPI == SWIGLU) return 32 * (p >> 4) + (p & 15) + 16 * up;
   const int half = D >> 1;
@@ -88,6 +89,8 @@ __global__ __launch_bounds__(256) void gemv_kernel(const bf16* __restrict__ X, i
       sn = cs[half];
     }
   }
+  float before = 0.f;   // ADD: of this lane's element
+  if constexpr (EPI == ADD) before = (float)out[(int64_t)em * ldo + min(n0 + er, N - 1)];
   float acc[M][R];
 #pragma unroll
   for (int m = 0; m < M; ++m)
@@ -136,6 +139,13 @@ __global__ __launch_bounds__(256) void gemv_kernel(const bf16* __restrict__ X, i
       for (int r = 0; r < R; ++r)
         if (lane == m * R + r && n0 + r < N)
           out[(int64_t)m * ldo + n0 + r] = (bf16)(acc[m][r] + (bias ? (float)bias[n0 + r] : 0.f));
+  } else if constexpr (EPI == ADD) {
+    float x = 0.f;
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+      for (int r = 0; r < R; ++r) x = lane == m * R + r ? acc[m][r] : x;
+    if (lane < M * R && n0 + er < N) out[(int64_t)em * ldo + n0 + er] = (bf16)(before + (float)(bf16)x);
   } else if constexpr (EPI == SWIGLU) {
 #pragma unroll
     for (int m = 0; m < M; ++m)
@@ -208,6 +218,13 @@ OME_API int ome_gemv(const void* X, int64_t ldx, const void* W, const void* bias
   if (M <= 0 || N <= 0) return 0;
   if (M > 8 || K % 8 || ldx % 8 || K <= 0) return -2;
   return gemv_launch<false>(X, ldx, W, bias, out, ldo, M, N, K, stream);
+}
+
+// out [M, N] += X . W^T, the product and the sum each rounded to bf16
+OME_API int ome_gemv_add(const void* X, int64_t ldx, const void* W, void* out, int64_t ldo, int M, int N, int K, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return 0;
+  if (M > 8 || K % 8 || ldx % 8 || K <= 0) return -2;
+  return gemv_launch<false, ADD>(X, ldx, W, nullptr, out, ldo, M, N, K, stream);
 }
 
 OME_API int ome_gemv_act(const void* X, int64_t ldx, const void* W, const void* bias, void* out, int64_t ldo, int M,

@@ -450,8 +450,14 @@ class LlamaForCausalLM:
                 ops.rope_qkv_cache(qkv, meta.positions, self.cos_sin, cfg.rot_dim, q, k_cache, v_cache, meta.slots,
                                    tp.hq, tp.hkv, D, True, self.qn[i], self.kn[i], self.eps, ks, vs)
             attn = self.attention(q, k_cache, v_cache, meta, ks, vs)
-            o = self._reduce_add_norm(self._row_parallel(attn.view(T, tp.hq * D), self.w_o[i], parts=parts, steady=steady),
-                                      residual, self.ln2[i])
+            a = attn.view(T, tp.hq * D)
+            if T <= _GEMV_ROWS and self.gu_il and partial and parts and tp.tp == 1 and \
+                    ops.gemm_rows_norm_ok(a, self.w_o[i], residual, self.ln2[i], self.w_gu[i]):
+                # a row or two: the norm between as part of the product after it
+                ops.gemv_add(a, self.w_o[i], residual)
+                x = self._row_parallel(ops.gemm_rows_norm(residual, self.ln2[i], self.eps, self.w_gu[i]), self.w_d[i], parts=parts)
+                continue
+            o = self._reduce_add_norm(self._row_parallel(a, self.w_o[i], parts=parts, steady=steady), residual, self.ln2[i])
             x = self._mlp_partial(i, o, parts, steady) if partial else self.mlp(i, o)
         if self.layers and (st.pp_size == 1 or st.is_last_pp):
             return self._reduce_add_norm(x, residual, self.norm, reduce=partial)   # final norm

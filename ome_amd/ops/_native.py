@@ -132,9 +132,11 @@ _SIGNATURES = {
         "ome_gemv": [vp, i64, vp, vp, vp, i64, i32, i32, i32, vp],
         "ome_gemv_swiglu": [vp, i64, vp, vp, i64, i32, i32, i32, vp],
         "ome_gemv_qkv": [vp, i64, vp, vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, i32, f32, f32, vp],
+        "ome_gemv_add": [vp, i64, vp, vp, i64, i32, i32, i32, vp],
         "ome_gemv_act": [vp, i64, vp, vp, vp, i64, i32, i32, i32, vp],
         "ome_gemm": [vp, i64, vp, i64, vp, i64, i32, i32, i32, i32, i32, vp, vp],
         "ome_gemm_set_variant": [i32],
+        "ome_gemm_rows_norm": [vp, i64, vp, f32, vp, i64, vp, i64, i32, i32, i32, vp],
         "ome_gemm_rows": [vp, i64, vp, i64, vp, vp, i64, i32, i32, i32, i32, i32, vp, vp],
         "ome_add_rmsnorm_parts": [vp, i32, vp, i64, vp, vp, i64, i32, i32, f32, vp],
         "ome_gemm_sk": [vp, i64, vp, i64, vp, vp, i64, i32, i32, i32, i32, i32, i32, i32, vp, vp, vp],
