@@ -556,6 +556,17 @@ def fp8_quant(x: torch.Tensor, group: int = 0):
     return q, s
 
 
+def _act_fp8_quant(gu: torch.Tensor, act: int):
+    """:func:`fp8_quant` in groups of 128 of :func:`act_and_mul` of ``gu`` [M, 2 K] (contiguous): one launch for SwiGLU, the same bits."""
+    M, K = gu.shape[0], gu.shape[1] // 2
+    if act != 0 or K % 128:
+        return fp8_quant(act_and_mul(gu, act), 128)
+    q = gu.new_empty(M, K, dtype=torch.float8_e4m3fn)
+    s = gu.new_empty(M, K // 128, dtype=torch.float32)
+    call("ome_fp8_quant_swiglu", gu.data_ptr(), gu.stride(0), M, K, q.data_ptr(), s.data_ptr(), stream_ptr())
+    return q, s
+
+
 def fp8_gemm(qa, sa, qw, sw, block: int = 0, bias=None, out: torch.Tensor | None = None) -> torch.Tensor:
     """out[M, N] bf16 = dequant(qa) . dequant(qw)^T (+ bias); qw [N, K] e4m3 with per-channel (block=0,
     sw [N]) or 128x128 block scales (block=128, sw [N/128, K/128])."""
@@ -898,8 +909,7 @@ def fused_moe_fp8(x: torch.Tensor, topk_w: torch.Tensor, topk_ids: torch.Tensor,
     gu = torch.empty(n, I2, dtype=x.dtype, device=dev)
     call("ome_moe_gemm_fp8_tile", qx.data_ptr(), qx.stride(0), sx.data_ptr(), s.ids, k, w13.q.data_ptr(),
          w13.scale.data_ptr(), s.tiles, I2, H, s.max_tiles, tm, gu.data_ptr(), gu.stride(0), stream_ptr())
-    h = act_and_mul(gu, act)
-    qh, sh = fp8_quant(h, 128)
+    qh, sh = _act_fp8_quant(gu, act)
     y = torch.empty(n, H, dtype=x.dtype, device=dev)
     call("ome_moe_gemm_fp8_tile", qh.data_ptr(), qh.stride(0), sh.data_ptr(), None, 0, w2.q.data_ptr(),
          w2.scale.data_ptr(), s.tiles, H, I, s.max_tiles, tm, y.data_ptr(), y.stride(0), stream_ptr())
@@ -922,8 +932,7 @@ def moe_experts_sorted(rows: torch.Tensor, ids: torch.Tensor, w13, w2, act: int,
         gu = torch.empty(n, I2, dtype=rows.dtype, device=dev)
         call("ome_moe_gemm_fp8_tile", qx.data_ptr(), qx.stride(0), sx.data_ptr(), s.ids, 1, w13.q.data_ptr(),
              w13.scale.data_ptr(), s.tiles, I2, H, s.max_tiles, tm, gu.data_ptr(), gu.stride(0), stream_ptr())
-        h = act_and_mul(gu, act)
-        qh, sh = fp8_quant(h, 128)
+        qh, sh = _act_fp8_quant(gu, act)
         y = torch.empty(n, H, dtype=rows.dtype, device=dev)
         call("ome_moe_gemm_fp8_tile", qh.data_ptr(), qh.stride(0), sh.data_ptr(), None, 0, w2.q.data_ptr(),
              w2.scale.data_ptr(), s.tiles, H, I2 // 2, s.max_tiles, tm, y.data_ptr(), y.stride(0), stream_ptr())

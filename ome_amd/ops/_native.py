@@ -149,6 +149,7 @@ _SIGNATURES = {
                             vp],
         "ome_fp8_gemm_mx": [vp, i64, vp, vp, i64, vp, i32, i32, i32, i32, vp, i64, vp, vp],
         "ome_fp8_quant": [vp, i64, i32, i32, vp, vp, i32, vp],
+        "ome_fp8_quant_swiglu": [vp, i64, i32, i32, vp, vp, vp],
         "ome_fp8_gemm": [vp, i64, vp, vp, vp, i32, i32, i32, i32, vp, i64, vp, vp],
         "ome_sample": [vp, i32, i64, i32, i32, vp, vp, vp, vp, vp, u64, vp, vp, vp],
     },
