@@ -12,6 +12,8 @@
 //   ome_moe_gemm_stream : the same for experts with few rows, on tiles listed by ome_moe_align_tiles
 //   ome_moe_combine : out[t] = sum_j w[t, j] * Y[inv[t*k + j]]   (fp32 accumulate)
 #include "common.h"
+
+#include <type_traits>
 #include "lds_stages.h"
 
 #include <cstdlib>
@@ -702,36 +704,54 @@ OME_API int ome_moe_gemm(const void* A, int64_t lda, const int* sorted_ids, int 
 // ------------------------------------------------------------------------------------------
 // add (optional, may alias out): out = add + scale * sum -- an always-on shared expert's output
 // folded into the combine instead of a separate elementwise add
+// A thread has eight columns of a token.  The experts' rows come up to eight at a time, added in their order: one after the other, each behind its
+// place and weight, a row took a round trip to memory, and a workgroup took all of a token's
+// columns.  us, 8 rows a token of 7168: 700 tokens 27.8 -> 18.0 (90 MB at 5.0 TB/s), 8 tokens 18.6 -> 4.8; 10 rows of 2048, 48 tokens 7.3 -> 4.8.
 __global__ __launch_bounds__(256) void moe_combine_kernel(const bf16* __restrict__ Y, const float* __restrict__ w,
                                                           const int* __restrict__ inv, int k, int H,
                                                           bf16* out, const bf16* add, float scale) {
-  const int t = blockIdx.x;
-  for (int c = threadIdx.x; c < H / 8; c += blockDim.x) {
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int j = 0; j < k; ++j) {
-      const float wj = w[(int64_t)t * k + j];
-      const bf16x8 y = ld8(Y + (int64_t)inv[(int64_t)t * k + j] * H + c * 8);
+  const int64_t t = blockIdx.x;
+  const int c = blockIdx.y * 256 + threadIdx.x;
+  if (c >= H / 8) return;
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  bf16x8 a = {};
+  if (add != nullptr) a = ld8(add + t * H + c * 8);
+  int j = 0;
+  const auto take = [&](auto count) {
+    constexpr int N = decltype(count)::value;
+    bf16x8 y[N];
+    float wj[N];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) acc[q] += wj * (float)y[q];
+    for (int i = 0; i < N; ++i) {
+      wj[i] = w[t * k + j + i];
+      y[i] = ld8(Y + (int64_t)inv[t * k + j + i] * H + c * 8);
     }
-    bf16x8 o;
-    if (add != nullptr) {
-      const bf16x8 a = ld8(add + (int64_t)t * H + c * 8);
 #pragma unroll
-      for (int q = 0; q < 8; ++q) o[q] = (bf16)((float)a[q] + acc[q] * scale);
-    } else {
+    for (int i = 0; i < N; ++i)
 #pragma unroll
-      for (int q = 0; q < 8; ++q) o[q] = (bf16)(acc[q] * scale);
-    }
-    st8(out + (int64_t)t * H + c * 8, o);
+      for (int q = 0; q < 8; ++q) acc[q] += wj[i] * (float)y[i][q];
+    j += N;
+  };
+  while (k - j >= 8) take(std::integral_constant<int, 8>{});
+  if (k - j >= 4) take(std::integral_constant<int, 4>{});
+  if (k - j >= 2) take(std::integral_constant<int, 2>{});
+  if (k - j >= 1) take(std::integral_constant<int, 1>{});
+  bf16x8 o;
+  if (add != nullptr) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) o[q] = (bf16)((float)a[q] + acc[q] * scale);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) o[q] = (bf16)(acc[q] * scale);
   }
+  st8(out + t * H + c * 8, o);
 }
 
 OME_API int ome_moe_combine_add(const void* Y, const float* w, const int* inv, int n_tok, int k, int H, void* out,
                                 const void* add, float scale, hipStream_t stream) {
   if (n_tok <= 0) return 0;
   if (H % 8) return -2;
-  moe_combine_kernel<<<n_tok, 256, 0, stream>>>((const bf16*)Y, w, inv, k, H, (bf16*)out, (const bf16*)add, scale);
+  moe_combine_kernel<<<dim3(n_tok, (H / 8 + 255) / 256), 256, 0, stream>>>((const bf16*)Y, w, inv, k, H, (bf16*)out, (const bf16*)add, scale);
   OME_CHECK_LAUNCH();
   return 0;
 }
