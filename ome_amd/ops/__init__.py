@@ -1956,7 +1956,7 @@ def _prefill_runs(items: list, ends: list[int], kv_heads: int):
     stages, or None where one workgroup per item is about as good.  A workgroup walks one run of the (item,
     stage) sequence, so only the items at a run's ends are cut (at a stage, no piece under 4).
 
-    Estimated in stages of a workgroup (2.65 us with both of a CU's at work): the classic launch takes its
+    Estimated in stages of a workgroup (2.65 us with both of a CU's at work; prefill_pair.hip's take 2.1 to 2.2, and its partials as much less): the classic launch takes its
     greedy schedule in item order; the runs their share, 8 for the second launch and short runs, and
     the cut items' partials (64 KiB each, written and read: 0.0124).  Against one workgroup per item, 8 kv heads:
     1500 rows over 6100 keys (376 workgroups for 512 places) 282 -> 230 us with an fp8 cache, 248 -> 224 in bf16;
