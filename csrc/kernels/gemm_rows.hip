@@ -39,7 +39,8 @@ __device__ __forceinline__ void gr_to_lds_nt(__amdgpu_buffer_rsrc_t rs, char* ld
 // NORM: X holds one or two rows of the residual stream, and out is the product of their RMSNorm (weights `ln`).  Every workgroup forms the norm itself,
 // in LDS, while its first weights are on their way: no rows move with the weights.  One row, 28672 x 4096: 4.6 + 38.1 us -> 39.1 (scaled between LDS
 // and the products instead 39.4, its loads ahead of the weights' 39.3, two more stages 39.6).
-constexpr int LN_ROWS = 2, LN_K = 8192;   // at most
+// The squares are added in the order of fused_add_rmsnorm_kernel of 8 waves, which these rows take elsewhere: the norm is the same bits.
+constexpr int LN_ROWS = 2, LN_K = 8192, LN_WAVES = 8;   // rows and K at most
 template <int WM, int WN, int FR, int NST, int EPI, bool NORM = false>
 __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_rows_kernel(
     const bf16* __restrict__ X, int64_t ldx, const bf16* __restrict__ W, int64_t ldw, const bf16* __restrict__ bias,
@@ -90,7 +91,7 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_rows_kernel(
     for (int f = 0; f < FR; ++f) acc[i][f] = f32x4{0.f, 0.f, 0.f, 0.f};
   bf16x8 wa[NI], wb[NI], xa[FR], xb[FR];
   __shared__ __attribute__((aligned(16))) bf16 rows[NORM ? LN_ROWS * LN_K : 8];   // NORM: the normalised rows (lanes of other rows read the last)
-  __shared__ float sums[NORM ? LN_ROWS * NW : 1];
+  __shared__ float sums[NORM ? LN_ROWS * LN_WAVES : 1];
   const char* xrow = reinterpret_cast<const char*>(rows) + min(fr, M - 1) * (LN_K * 2) + 16 * fc;
   int kr = tile % n;   // K tile of the buffer that is read
   const auto read = [&](bf16x8 (&w)[NI], bf16x8 (&x)[FR], int b, int kk) {
@@ -134,22 +135,27 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_rows_kernel(
   }
   if constexpr (NORM) {
 #pragma unroll
-    for (int m = 0; m < LN_ROWS; ++m) {
-      float ss = 0.f;
+    for (int m = 0; m < LN_ROWS; ++m)
 #pragma unroll
-      for (int c = 0; c < CH; ++c)
-        if (8 * (tid + 64 * NW * c) < 64 * steps)
+      for (int p = 0; p < LN_WAVES / NW; ++p) {   // (wave + NW p of those eight)
+        float ss = 0.f;
 #pragma unroll
-          for (int j = 0; j < 8; ++j) ss += (float)raw[m][c][j] * (float)raw[m][c][j];
-      ss = wave_sum(ss);
-      if (lane == 0) sums[m * NW + wave] = ss;
-    }
+        for (int c = p; c < CH; c += LN_WAVES / NW)
+          if (8 * (tid + 64 * NW * c) < 64 * steps)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              const float f = (float)raw[m][c][j];
+              ss += f * f;
+            }
+        ss = wave_sum(ss);
+        if (lane == 0) sums[m * LN_WAVES + wave + NW * p] = ss;
+      }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
     for (int m = 0; m < LN_ROWS; ++m) {
       float ss = 0.f;
 #pragma unroll
-      for (int x = 0; x < NW; ++x) ss += sums[m * NW + x];
+      for (int x = 0; x < LN_WAVES; ++x) ss += sums[m * LN_WAVES + x];
       const float rms = rsqrtf(ss / (float)(64 * steps) + eps);
 #pragma unroll
       for (int c = 0; c < CH; ++c) {

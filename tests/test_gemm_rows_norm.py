@@ -1,8 +1,14 @@
 """One or two rows through a norm and the product after it in one launch (``ops.gemv_add``, ``ops.gemm_rows_norm``)."""
+import dataclasses
+
 import pytest
 import torch
 
 from ome_amd import ops
+from ome_amd.models.config import preset
+from ome_amd.runtime.model_runner import ModelRunner
+from ome_amd.runtime.request import Request, SamplingParams
+from ome_amd.runtime.scheduler import ScheduledChunk, StepBatch
 
 pytestmark = pytest.mark.gpu
 
@@ -25,6 +31,7 @@ def test_matches_norm_and_product(M, K, N):
     ops.gemv_add(a, wo, res)
     assert torch.equal(res, before)
     out = ops.gemm_rows_norm(res, ln, eps, w)
+    assert torch.equal(out, ops.gemm_rows(part, w, epi=2))   # (the norm's sums in the same order, the products too)
     r = res.double()
     x = (r * torch.rsqrt((r * r).mean(-1, keepdim=True) + eps) * ln.double()).to(torch.bfloat16).double()
     g, u = (x @ w.double().t()).view(M, N // 32, 2, 16).unbind(2)
@@ -51,3 +58,31 @@ def test_takes_what_it_is_for():
     f32 = args()
     f32[2] = f32[2].float()
     assert not ops.gemm_rows_norm_ok(*f32)
+
+
+@pytest.mark.parametrize("rows", [1, 2])
+@pytest.mark.parametrize("mode", ["decode", "prefill"])
+def test_a_model_takes_it(rows, mode, monkeypatch):
+    """Two layers of an 8B model: steps of one and two rows give the same bits with the norm as a launch of its own."""
+    cfg = dataclasses.replace(preset("llama-3-8b"), num_layers=2, vocab_size=1024)
+    r = ModelRunner(cfg, device="cuda", max_running=4, max_context=1024, max_total_tokens=4096, cuda_graph=False, keep_logits=True)
+    took, norm = [], ops.gemm_rows_norm
+    monkeypatch.setattr(ops, "gemm_rows_norm", lambda *a: (took.append(a[0].shape[0]), norm(*a))[1])
+    reqs = []
+    for i in range(rows if mode == "decode" else 1):
+        reqs.append(Request([5 + i, 7, 9], SamplingParams(ignore_eos=True)))
+        reqs[i].pages, reqs[i].req_slot = [1 + i], r.slots.alloc()
+        r.slots.set_pages(reqs[i].req_slot, 0, reqs[i].pages)
+    r.slots.flush()
+    before = 0
+    if mode == "decode":
+        before = 2
+        r.launch(StepBatch("prefill", [ScheduledChunk(q, 0, 2, True, want=[1]) for q in reqs]))
+        for q in reqs:
+            q.num_cached = 2
+    took.clear()
+    step = lambda: r.launch(StepBatch(mode, [ScheduledChunk(q, before, 1 if mode == "decode" else rows, True, want=[0]) for q in reqs])).logits.clone()  # noqa: E731
+    folded = step()
+    assert took == 2 * [rows]
+    monkeypatch.setattr(ops, "gemm_rows_norm_ok", lambda *a: False)
+    assert torch.equal(folded, step()) and took == 2 * [rows]
