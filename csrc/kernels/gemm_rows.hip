@@ -135,24 +135,32 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void gemm_rows_kernel(
   }
   if constexpr (NORM) {
 #pragma unroll
-    for (int m = 0; m < LN_ROWS; ++m)
+    for (int m = 0; m < LN_ROWS; ++m) {
+      if (m >= M) break;
+      float ss[LN_WAVES / NW];   // (of waves wave + NW p of those eight)
 #pragma unroll
-      for (int p = 0; p < LN_WAVES / NW; ++p) {   // (wave + NW p of those eight)
-        float ss = 0.f;
+      for (int p = 0; p < LN_WAVES / NW; ++p) {
+        ss[p] = 0.f;
 #pragma unroll
         for (int c = p; c < CH; c += LN_WAVES / NW)
-          if (8 * (tid + 64 * NW * c) < 64 * steps)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-              const float f = (float)raw[m][c][j];
-              ss += f * f;
-            }
-        ss = wave_sum(ss);
-        if (lane == 0) sums[m * LN_WAVES + wave + NW * p] = ss;
+          for (int j = 0; j < 8; ++j) {
+            const float f = (float)raw[m][c][j], next = ss[p] + f * f;
+            ss[p] = 8 * (tid + 64 * NW * c) < 64 * steps ? next : ss[p];
+          }
       }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+        for (int p = 0; p < LN_WAVES / NW; ++p) ss[p] += __shfl_xor(ss[p], o);
+#pragma unroll
+      for (int p = 0; p < LN_WAVES / NW; ++p)
+        if (lane == 0) sums[m * LN_WAVES + wave + NW * p] = ss[p];
+    }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
     for (int m = 0; m < LN_ROWS; ++m) {
+      if (m >= M) break;
       float ss = 0.f;
 #pragma unroll
       for (int x = 0; x < LN_WAVES; ++x) ss += sums[m * LN_WAVES + x];
