@@ -10,7 +10,8 @@ Two in-tree shared objects are produced (they travel to GPU boxes with the repo 
   safetensors header parser, multi-threaded pread -> pinned-host -> HBM loader,
   paged-KV block allocator, radix prefix cache.
 * ``ome_amd/_lib/libome_comm.so`` — xGMI peer-to-peer collectives (``csrc/comm``).
-* ``ome_amd/_lib/libome_call.so`` — a Python module that calls the launchers (``csrc/host``; ctypes does without it).
+* ``ome_amd/_lib/libome_call.<ABI of the Python>.so`` — a Python module that calls the launchers (``csrc/host``), for x86-64 where
+  Python's headers and a C++ compiler are; ctypes does without it.
 
 Usage: ``python -m ome_amd.build [--force] [--jobs N]``.
 """
@@ -19,6 +20,7 @@ from __future__ import annotations
 import argparse
 import concurrent.futures as cf
 import os
+import platform
 import shutil
 import subprocess
 import sys
@@ -118,8 +120,9 @@ def build(force: bool = False, jobs: int | None = None, verbose: bool = True,
         built.append(_build_lib("ome_comm", comm_src, sorted(cdir.glob("*.h")) + [kdir / "common.h"], hipcc,
                                 HIP_FLAGS + [f"-I{kdir}"], [], force, jobs))
     include = Path(sysconfig.get_paths()["include"])
-    if "ome_call" in want and (include / "Python.h").exists():
-        built.append(_build_lib("ome_call", sorted((CSRC / "host").glob("*.cpp")), [], shutil.which("g++") or "c++",
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if "ome_call" in want and platform.machine() == "x86_64" and (include / "Python.h").exists() and cxx:
+        built.append(_build_lib(f"ome_call.{sysconfig.get_config_var('SOABI')}", sorted((CSRC / "host").glob("*.cpp")), [], cxx,
                                 [*CXX_FLAGS, f"-I{include}"], [], force, jobs))
     if verbose:
         for b in built:

@@ -12,7 +12,9 @@ scheduler are tested without a GPU).
 from __future__ import annotations
 
 import ctypes as C
+import logging
 import os
+import sysconfig
 import threading
 from pathlib import Path
 
@@ -23,6 +25,8 @@ import torch
 # (a library missing there comes from the default directory)
 _LIB_DIR = Path(__file__).resolve().parent.parent / "_lib"
 _LIB_OVERRIDE = Path(os.environ["OME_LIB_DIR"]).resolve() if os.environ.get("OME_LIB_DIR") else None
+CALLER = f"ome_call.{sysconfig.get_config_var('SOABI')}"
+_log = logging.getLogger(__name__)
 _lock = threading.Lock()
 _libs: dict[str, C.CDLL] = {}
 
@@ -205,6 +209,11 @@ def load(name: str = "ome_kernels") -> C.CDLL:
                 from ome_amd import build as _b
 
                 _b.build(verbose=False, only=(name,))   # (only the library asked for)
+                if name == "ome_kernels":   # (and what calls it without ctypes, from the next process on)
+                    try:
+                        _b.build(verbose=False, only=("ome_call",))
+                    except (RuntimeError, OSError) as e:
+                        _log.warning("launchers are called by ctypes: %s", e)
             if not path.exists():
                 raise NativeError(f"{path} missing — run `python -m ome_amd.build` (hipcc, gfx950)")
         lib = C.CDLL(str(path), mode=C.RTLD_GLOBAL)
@@ -237,8 +246,9 @@ def _slow_call(fn: str, *args) -> None:
 
 
 def _load_caller():
-    """The module that calls launchers without ctypes (``csrc/host/ome_call.cpp``), or None where it was not built."""
-    path = lib_path("ome_call")
+    """The module that calls launchers without ctypes (``csrc/host/ome_call.cpp``), or None where it was not built or does not load: it
+    is of one Python's ABI, which its name says."""
+    path = lib_path(CALLER)
     if not path.exists():
         return None
     import importlib.machinery
@@ -246,8 +256,12 @@ def _load_caller():
 
     loader = importlib.machinery.ExtensionFileLoader("ome_call", str(path))
     spec = importlib.util.spec_from_file_location("ome_call", str(path), loader=loader)
-    module = importlib.util.module_from_spec(spec)
-    loader.exec_module(module)
+    try:
+        module = importlib.util.module_from_spec(spec)
+        loader.exec_module(module)
+    except (ImportError, OSError) as e:
+        _log.warning("launchers are called by ctypes: %s does not load (%s)", path.name, e)
+        return None
     return module
 
 
