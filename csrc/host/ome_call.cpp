@@ -2,8 +2,8 @@
 // of its own: a launcher of 21 arguments takes 4.5 us that way and 0.8 so.
 //
 // bind(name, address, kinds): `kinds` has a letter an argument: p a pointer (or None), i a 32-bit, l a 64-bit integer, f a float.  call(name, *args) calls it
-// and raises by `fail(name, code)` if it returns anything but 0; a name that is not bound, or arguments of any other number or type, go to `other(name, *args)`,
-// which calls by ctypes.
+// and raises by `fail(name, code)` if it returns anything but 0; a name that is not bound, arguments of any other number or type and keywords go to
+// `other(name, *args, ...)`, which calls by ctypes.
 //
 // One prototype serves every launcher: by the System V calling convention of x86-64 integers and pointers fill six registers and then eight
 // bytes each of the stack, floats the low halves of eight vector registers, both in their own order, and a callee does not
@@ -48,8 +48,8 @@ int invoke(const Launcher& l, const uint64_t* a, const float* x, int integers) {
                                          OME_A6(s, 7), OME_A6(s, 8), s[54], s[55], s[56], s[57]);
 }
 
-PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  PyObject* const capsule = nargs > 0 ? PyDict_GetItem(g_bound, args[0]) : nullptr;   // (borrowed)
+PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObject* names) {
+  PyObject* const capsule = nargs > 0 && !names ? PyDict_GetItem(g_bound, args[0]) : nullptr;   // (borrowed)
   const Launcher* const bound = capsule ? static_cast<const Launcher*>(PyCapsule_GetPointer(capsule, nullptr)) : nullptr;
   if (bound && bound->n == nargs - 1) {
     const Launcher l = *bound;
@@ -86,7 +86,7 @@ PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     }
     PyErr_Clear();
   }
-  return PyObject_Vectorcall(g_other, args, (size_t)nargs, nullptr);
+  return PyObject_Vectorcall(g_other, args, (size_t)nargs, names);
 }
 
 PyObject* bind(PyObject*, PyObject* args) {
@@ -126,7 +126,7 @@ PyObject* hooks(PyObject*, PyObject* args) {
   Py_RETURN_NONE;
 }
 
-PyMethodDef methods[] = {{"call", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(call)), METH_FASTCALL, "call(name, *args)"},
+PyMethodDef methods[] = {{"call", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(call)), METH_FASTCALL | METH_KEYWORDS, "call(name, *args, lib)"},
                          {"bind", bind, METH_VARARGS, "bind(name, address, kinds)"},
                          {"hooks", hooks, METH_VARARGS, "hooks(other, fail)"},
                          {nullptr, nullptr, 0, nullptr}};

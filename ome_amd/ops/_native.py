@@ -239,8 +239,8 @@ def _fail(fn: str, rc: int) -> None:
     raise NativeError(f"{fn} failed with code {rc}")
 
 
-def _slow_call(fn: str, *args) -> None:
-    rc = getattr(load("ome_kernels"), fn)(*args)
+def _slow_call(fn: str, *args, lib: str = "ome_kernels") -> None:
+    rc = getattr(load(lib), fn)(*args)
     if rc != 0:
         _fail(fn, rc)
 

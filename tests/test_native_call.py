@@ -41,6 +41,20 @@ def test_other_arguments_go_to_ctypes(monkeypatch, args):
     assert got == [] and seen == [("t", *args), ("nothing of that name",)]
 
 
+def test_a_launcher_of_another_library():
+    """``lib`` names it, as it does where ctypes makes every call."""
+    with pytest.raises(N.NativeError, match="nowhere"):
+        N.call("t", 1, lib="nowhere")
+    f, got = _bind("ome_ep_handle", "i")
+    seen = []
+    N._caller.hooks(lambda *a, **kw: seen.append((a, kw)), N._fail)
+    try:
+        N.call("ome_ep_handle", 1, lib="ome_comm")
+    finally:
+        N._caller.hooks(N._slow_call, N._fail)
+    assert got == [] and seen == [(("ome_ep_handle", 1), {"lib": "ome_comm"})]
+
+
 def test_a_code_raises():
     f, got = _bind("t", "l", rc=-3)
     with pytest.raises(N.NativeError, match="t failed with code -3"):
