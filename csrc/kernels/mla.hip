@@ -247,7 +247,8 @@ __global__ __launch_bounds__(256) void mla_attn_kernel(
 // The products by asm: with one wave per SIMD, what covers an LDS read is the distance to its product, and the
 // compiler sinks reads to their use (or hoists them all, into scratch).  Volatile with a memory clobber, each stays
 // between the reads around it.  The waits that the compiler cannot see: `mma_new` after a VALU write of its
-// operands, `MMA_WAIT` between a last product and the first other reader of its result.
+// operands, `MMA_WAIT` between a last product and the first other reader of its result (without that as an operand: the
+// compiler may copy an operand ahead of the wait).
 #define MMA_WAIT "s_nop 15\n\ts_nop 3"
 __device__ __forceinline__ void mma_new(f32x16& c, bf16x8 a, bf16x8 b) {   // c = a b
 #if defined(__HIP_DEVICE_COMPILE__)

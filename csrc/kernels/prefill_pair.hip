@@ -74,6 +74,12 @@ __device__ __forceinline__ void two_to_lds(const void* base, uint32_t bytes, uin
 #endif
 }
 
+__device__ __forceinline__ void mma_acc_last(f32x16& c, bf16x8 a, bf16x8 b) {   // c += a b, the last of all
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0\n\t" MMA_WAIT : "+a"(c) : "v"(a), "v"(b) : "memory");
+#endif
+}
+
 // Keeps what computes x on this side of the next product: the compiler would sink it past them all to its use.
 template <typename T>
 __device__ __forceinline__ void here(T& x) {
@@ -257,7 +263,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     const float mul = a.mul;
 
     auto rescale = [&]() __attribute__((always_inline)) {   // O^T by what the maximum rose a tile ago
-      asm volatile(MMA_WAIT ::: "memory");
+      asm volatile(MMA_WAIT ::: "memory");   // (without O^T as an operand: the compiler would copy it ahead of the wait, two slots behind a product)
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
@@ -351,7 +357,10 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
 #pragma unroll
-        for (int rb = 0; rb < 2; ++rb) mma_acc(o[rb][i & 3], v[i & 3], p[rb][i >> 2]);
+        for (int rb = 0; rb < 2; ++rb) {
+          if (i == 7 && rb == 1) mma_acc_last(o[rb][3], v[3], p[rb][1]);   // (others read O^T from here on)
+          else mma_acc(o[rb][i & 3], v[i & 3], p[rb][i >> 2]);
+        }
         if (i < 4) v[i] = vfrag(img, i + 4);
       }
     };
@@ -591,7 +600,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       step(u, sA, sB, pA, pB, std::integral_constant<int, LAST>{});
       weighted(pB, vn);
     }
-    asm volatile(MMA_WAIT "\n\ts_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");   // (the images are done with)
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");   // (the images are done with)
 
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
