@@ -1356,22 +1356,25 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const int4* __rest
   auto pw_of = [&](int p) -> int64_t { return ((int64_t)(p0 + p) * Hkv + kvh) * 4 + w; };
   const int at = pair ? (quad >> 1) * 256 + (quad & 1) * 128 + r * 4 : r * D + 4 * quad;
   // Parts that are read at a time; the first, which are all of most items, with their outputs at once (47 items of some 250 tiles 15.1 -> 12.9 us, 8
-  // items of 120 10.2 -> 8.1; eight at a time 13.3 and 9.2)
+  // items of 120 10.2 -> 8.1; eight at a time 13.3 and 9.2), those after the second four while the four before them are added (two items of 32
+  // parts 9.8 -> 9.0 us, the 8 items, of 8 parts, 8.1 -> 8.4; the second four so, too: 8.7 and 8.5)
   constexpr int AHEAD = 4;
-  float2 ml[AHEAD];
-  f32x4 ov[AHEAD];
-  const auto fetch = [&](int p) {
+  struct Batch {
+    float2 ml[AHEAD];
+    f32x4 o[AHEAD];
+  } now, next;
+  const auto fetch = [&](Batch& x, int p) {
 #pragma unroll
     for (int i = 0; i < AHEAD; ++i) {
       const int64_t pw = pw_of(min(p + i, np - 1));
-      ml[i] = *reinterpret_cast<const float2*>(part_ml + (pw * 32 + r) * 2);
-      ov[i] = *reinterpret_cast<const f32x4*>(part_o + pw * 32 * D + at);
+      x.ml[i] = *reinterpret_cast<const float2*>(part_ml + (pw * 32 + r) * 2);
+      x.o[i] = *reinterpret_cast<const f32x4*>(part_o + pw * 32 * D + at);
     }
   };
-  fetch(0);
+  fetch(now, 0);
   float M = sink;
 #pragma unroll
-  for (int i = 0; i < AHEAD; ++i) M = fmaxf(M, ml[i].x);
+  for (int i = 0; i < AHEAD; ++i) M = fmaxf(M, now.ml[i].x);
   for (int p = AHEAD; p < np; p += 2 * AHEAD) {
     float x[2 * AHEAD];
 #pragma unroll
@@ -1382,15 +1385,21 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const int4* __rest
   const float Mu = M == OME_NEG_INF ? 0.f : M;
   float L = sinks ? fast_exp2(sink - Mu) : 0.f;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int p = 0; p < np; p += AHEAD) {
-    if (p > 0) fetch(p);
+  const auto add = [&](const Batch& x, int p) {
 #pragma unroll
     for (int i = 0; i < AHEAD; ++i)
       if (p + i < np) {
-        const float wt = fast_exp2(ml[i].x - Mu);
-        L += wt * ml[i].y;
-        acc += wt * ov[i];
+        const float wt = fast_exp2(x.ml[i].x - Mu);
+        L += wt * x.ml[i].y;
+        acc += wt * x.o[i];
       }
+  };
+  add(now, 0);
+  if (np > AHEAD) fetch(now, AHEAD);
+  for (int p = AHEAD; p < np; p += AHEAD) {
+    if (p + AHEAD < np) fetch(next, p + AHEAD);
+    add(now, p);
+    now = next;
   }
   const float inv = L > 0.f ? v_scale / L : 0.f;
   bf16x4 v;

@@ -9,10 +9,10 @@ pytestmark = pytest.mark.gpu
 
 # one and two tiles of 32 keys; rows and keys around a tile's edge, pairs of steps and one left over; more than the 32 tiles whose pages a
 # wave looks up at a time; a workgroup an item, runs of pieces and (forced) equal pieces; more than 512 workgroups (fp8's rule), of more keys
-# and of one page, one row and one key too
+# and of one page, one row and one key too; items of 11, 18 and 32 pieces, which are merged four at a time
 SHAPES = [([1, 2, 32, 33], [1, 34, 32, 64], False), ([5, 31, 64, 97], [37, 95, 128, 1025], False), ([5, 31, 64, 97], [37, 95, 128, 1025], True),
           ([64], [2100], False), ([40, 3], [160, 2085], True), ([33] * 70, [33 + 31 * (i % 5) for i in range(70)], False),
-          ([1, 2, 17, 33] * 28, [1, 34, 17, 65] * 28, False)]
+          ([1, 2, 17, 33] * 28, [1, 34, 17, 65] * 28, False), ([40], [3000], False), ([100], [5000], False), ([64], [9000], False)]
 P, D, HKV, DEV = 16, 128, 4, "cuda"
 
 
@@ -32,7 +32,7 @@ def _inputs(shape, cache, sinks):
     wide = torch.randn(sum(q_lens), 6 * HKV, D, device=DEV).to(torch.bfloat16)
     q = wide[:, :4 * HKV]   # rows apart, as in a fused projection
     items, split, comb, chunk, parts = ops.prefill_plan(q_lens, kv_lens, kv_heads=HKV, force=force)
-    assert (parts > 0) == (force or max(kv_lens) > 2048) and (shape < 5 or len(items) * HKV > 512)
+    assert (parts > 0) == (force or max(kv_lens) > 2048) and (len(q_lens) < 9 or len(items) * HKV > 512)
     plan = ops.PrefillPlan(t(items, 2), t(split, 4), t(comb, 4), chunk, parts)
     return q, kc, vc, bt, cu, kl, plan, torch.randn(4 * HKV, device=DEV) if sinks else None
 
