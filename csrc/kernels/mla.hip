@@ -478,10 +478,17 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
     auto look = [&](int tile) {
       const int p = 2 * tile + lane;
 #if defined(__HIP_DEVICE_COMPILE__)   // (waited for here: the compiler would wait before every use, and for the moves as well)
-      asm volatile("global_load_dword %0, %1, off\n\ts_waitcnt vmcnt(0)" : "=&v"(pages) : "v"(bt + (p < n_pages ? p : 0)) : "memory");
+      asm volatile("global_load_dword %0, %1, off\n\ts_waitcnt vmcnt(0)" : "=&v"(pages) : "v"(begin < end ? bt + (p < n_pages ? p : 0) : tok_row) : "memory");
 #endif
       pg0 = tile;
     };
+    // (The queries have come by then too.  The compiler, which does not know the moves, would otherwise wait for a query ahead of every product of S^T,
+    // in the loop too, and so for all but a few of the moves that come after it.)
+    look(begin);
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+    for (int s = 0; s < NS; ++s) asm volatile("" : "+v"(qf[s]));
+#endif
     const bf16 *b0 = cache, *b1 = cache;   // pages of the tile on its way, its image, its descriptors' size
     uint32_t to = 0, bytes = 0;
     auto aim = [&](int tile, int img) {    // (of a tile past the last nothing is read, zeros are written)
@@ -547,32 +554,38 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
     float peaks = 0.f, walked = 0.f;
     const float large = min((end - begin) * my_parts, DECODE ? 6 : 16);
     f32x16 sc;
+    // The first two tiles together, the third beside the first one's products: the second was asked for beside them as well, and pieces of two
+    // and three tiles, which saw its whole latency, took as much longer as the pipeline saved (us, three images -> that -> this: 16 rows of 128
+    // heads over 640 keys 30.4 -> 30.5 -> 30.2, six prompts of 59 rows 36.9 -> 37.5 -> 36.4; 32 x 8000 keys of 16 heads 84.8 -> 85.9 -> 84.0).
     if (begin < end) {
-      look(begin);
       aim(begin, 0);
 #pragma unroll
       for (int j = 0; j < NJ; ++j) dma(j);
+      if (NW > 1 || begin + 1 < end) {
+        aim(begin + 1, 1);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) dma(j);
+      }
     }
 #pragma unroll
     for (int v = 0; v < NV; ++v)
 #pragma unroll
       for (int i = 0; i < 16; ++i) o[v][i] = 0.f;
     if (begin < end) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      landed(begin + 1 < end);
       __syncthreads();
       if constexpr (NW == 1) {
-#pragma unroll 1
-        for (int t = 1; t < 3 && begin + t < end; ++t) {
-          aim(begin + t, t);
+        if (begin + 2 < end) {
+          aim(begin + 2, 2);
 #pragma unroll
           for (int j = 0; j < NJ; ++j) dma(j);
         }
         score(0, sc, [](int) {});
       } else {
-        score(0, sc, [&](int s) __attribute__((always_inline)) {   // the next two tiles' moves beside it
-          if (s % (NS / 2) == 0) aim(begin + 1 + s / (NS / 2), 1 + s / (NS / 2));
-          if (NW == 2) dma(s % NJ);
-          else if (s % 2 == 0) dma(s / 2 % NJ);
+        static_assert(NW == 1 || NS % NJ == 0, "a move every so many products");
+        score(0, sc, [&](int s) __attribute__((always_inline)) {
+          if (s == 0) aim(begin + 2, 2);
+          if (s % (NS / NJ) == 0) dma(s / (NS / NJ));
         });
       }
       landed(begin + 2 < end);
