@@ -21,6 +21,7 @@
 // LDS rows are 1152 B (72 x 16-B chunks); chunk x of key row r lives at x ^ (r & 7), which
 // spreads both the row reads and the transposed reads over the banks.
 #include "common.h"
+#include "mma32.h"
 
 #include <cstdlib>
 
@@ -244,20 +245,11 @@ __global__ __launch_bounds__(256) void mla_attn_kernel(
 // Measured (16-head kernel, or for decode the 16-row waves before -> now): three prompts of 3394 rows x 16 heads
 // 738 -> 135 us (118 -> 645 TFLOP/s); decode, 48 contexts of ~3000 keys x 128 heads 100 -> 86 us.
 // ------------------------------------------------------------------------------------------
-// The products by asm: with one wave per SIMD, what covers an LDS read is the distance to its product, and the
-// compiler sinks reads to their use (or hoists them all, into scratch).  Volatile with a memory clobber, each stays
-// between the reads around it.  The waits that the compiler cannot see: `mma_new` after a VALU write of its
-// operands, `MMA_WAIT` between a last product and the first other reader of its result (without that as an operand: the
-// compiler may copy an operand ahead of the wait).
-#define MMA_WAIT "s_nop 15\n\ts_nop 3"
+// The products (mma32.h): with one wave per SIMD, what covers an LDS read is the distance to its product.  `mma_new` comes after a
+// VALU write of its operands.
 __device__ __forceinline__ void mma_new(f32x16& c, bf16x8 a, bf16x8 b) {   // c = a b
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile("s_nop 3\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b) : "memory");
-#endif
-}
-__device__ __forceinline__ void mma_add(f32x16& c, bf16x8 a, bf16x8 b) {   // c += a b, c in vector registers
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b) : "memory");
 #endif
 }
 __device__ __forceinline__ void mma_last(f32x16& d, bf16x8 a, bf16x8 b, const f32x16& c) {   // d = c + a b, which others may read
@@ -265,20 +257,6 @@ __device__ __forceinline__ void mma_last(f32x16& d, bf16x8 a, bf16x8 b, const f3
   asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %3\n\t" MMA_WAIT : "=&v"(d) : "v"(a), "v"(b), "v"(c) : "memory");
 #endif
 }
-__device__ __forceinline__ void mma_acc(f32x16& c, bf16x8 a, bf16x8 b) {   // c += a b, c in accumulation registers
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b) : "memory");
-#endif
-}
-
-__device__ __forceinline__ void mma_acc2(f32x16& c, bf16x8 a, bf16x8 b, bf16x8 b2, uint32_t both) {   // c += a b (+ a b2)
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0\n\ts_cmp_eq_u32 %4, 0\n\ts_cbranch_scc1 .Lone%=\n\t"
-               "v_mfma_f32_32x32x16_bf16 %0, %1, %3, %0\n.Lone%=:"
-               : "+a"(c) : "v"(a), "v"(b), "v"(b2), "s"(both) : "memory", "scc");
-#endif
-}
-
 // Chunk x of key row r lies at x ^ row_swz(r): the same chunk of 16 rows, and four chunks of four, in all of the 64 banks (rows are 9 times
 // half of them wide)
 __device__ __forceinline__ int row_swz(int r) { return (r >> 1 & 1) << 2 | (r >> 2 & 1) << 1 | (r >> 3 & 1); }

@@ -16,29 +16,18 @@
 // 605 -> 511 (575 -> 520), 2 x 2048 rows 94 -> 81 (94 -> 84), 4 x 500 over 900 keys 40 -> 35.5, 32 x 64 rows 13.8 -> 12.4, 8 x 256 and 300 rows
 // the same.  What it does not gain: moves of 64 rows' tiles would be shared by twice the waves, but items of 32 rows fill the chip better.
 #include "common.h"
+#include "mma32.h"
 #include "prefill_pair.h"
 
 #include <type_traits>
 
 namespace {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-#define MMA_WAIT "s_nop 15\n\ts_nop 3"
 __device__ __forceinline__ void mma_new(f32x16& c, bf16x8 a, bf16x8 b) {   // c = a b
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b) : "memory");
-#endif
-}
-__device__ __forceinline__ void mma_add(f32x16& c, bf16x8 a, bf16x8 b) {   // c += a b
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b) : "memory");
-#endif
-}
-__device__ __forceinline__ void mma_acc(f32x16& c, bf16x8 a, bf16x8 b) {   // c += a b, c in accumulation registers
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b) : "memory");
 #endif
 }
 // The last products of two chains, which others read afterwards, and what fills the wait for them: two products of O^T and four exponentials.
