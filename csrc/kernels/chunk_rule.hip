@@ -24,8 +24,10 @@
 // (q S is formed transposed for that); T and P T are products of three bf16 parts each, at half the fp32 product's time.
 // Memory traffic hides behind that.  Two fp16 parts instead of three bf16 ones would take a quarter less time, but the state came out
 // 2.3 times further from 64 bits: an fp16 value below 2^-14 has no lower part.
-//   gated delta rule, 32 heads of 128 x 128, prompts of 1001 / 1435 / 1564 rows:   22 + 97 us (before: 24 + 123; row by row: 1098)
-//   selective scan, 128 heads of 64 x 128, 8 groups, 1033 / 926 / 1248 / 293 rows:  10 + 74 us (values scaled by dt in three parts: 80; before: 116; row by row: 1745)
+// (chunks' matrices + scan, calls that are waited for one by one; many in a row, where the clock falls, the scans take 100 and 93):
+//   gated delta rule, 32 heads of 128 x 128, prompts of 1001 / 1435 / 1564 rows:   22 + 95 us (before: 24 + 123; row by row: 1098)
+//   selective scan, 128 heads of 64 x 128, 8 groups, 1033 / 926 / 1248 / 293 rows:  10 + 85 us (values scaled by dt in three parts: 10 + 93; before: 11 + 116;
+//   row by row: 1745)
 // Largest error of the state against 64 bits: 1.2e-7 (row by row: 2.0e-7) and 1.2e-7 (6.2e-7) of its norm.
 //
 // A chunk's products multiply the entries that causality zeroes as well, and 0 times an infinity or NaN is NaN, so a key,
@@ -185,7 +187,7 @@ __device__ __forceinline__ void split3(f32x4 x0, f32x4 x1, bf16x8 (&p)[3]) {
 }
 
 // Four, by cutting the lower bits off: half as many instructions again, but a dot product waits for the products around it (20 cycles each way).
-// For a wave that has little else to do beside its products (Mamba-2's P: 85.4 -> 83.8 us of the prompts above; S and U so: 86 to 87).
+// For a wave that has little else to do beside its products (Mamba-2's P: 2% of the scan; S and U so: 1 to 2% more).
 __device__ __forceinline__ void cut3(f32x4 x, bf16x4 (&p)[3]) {
 #pragma unroll
   for (int t = 0; t < 3; ++t) {

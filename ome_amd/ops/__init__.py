@@ -1703,7 +1703,10 @@ def gemm_rows(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None
 def gemm_rows_norm_ok(a: torch.Tensor, wo: torch.Tensor, res: torch.Tensor, ln: torch.Tensor, w: torch.Tensor) -> bool:
     """:func:`gemv_add` of ``a``, ``wo`` into ``res`` and :func:`gemm_rows_norm` of that, ``ln`` and ``w`` take the operands and are faster than
     projection, norm and product: where the projection is a GEMV (one or two rows of most weights; more rows come in pieces, which the
-    norm adds) and the product :func:`gemm_rows`.  A layer of 4096 x 4096 and 28672 x 4096, one row: 7.3 + 4.6 + 38.1 us -> 7.2 + 39.1."""
+    norm adds) and the product :func:`gemm_rows`.  us, weights cold, three launches -> these two, one row (two rows): 4096 x 4096 and 28672 x 4096 48.1 -> 46.2
+    (50.1 -> 48.4), 4096 x 4096 and 24576 x 4096 43.4 -> 41.7 (44.6 -> 43.3), 2048 x 2048 and 24576 x 2048 25.9 -> 24.0 (26.2 -> 24.7), 4096 x 2048 and 49152 x
+    4096 77.8 -> 75.1 (78.9 -> 76.3), 8192 x 1024 and 24576 x 8192 73.0 -> 70.5 (73.9 -> 72.0), 1024 x 2048 and 65536 x 1024 29.5 -> 28.7 (30.0 -> 29.7);
+    8192 x 8192 and 57344 x 8192 178 -> 175, 5120 x 8192 and 51200 x 5120 111 -> 108 (two rows of these come in pieces)."""
     return (res.shape[0] <= 2 and gemv_ok(a, wo, None, res) and not gemm_rows_parts_plan(a, wo) and not gemm_rows_plan(a, wo)
             and gemm_rows_plan(res, w, epi=2) and res.shape[1] <= 8192 and ln.is_contiguous() and ln.dtype == res.dtype and ln.data_ptr() % 16 == 0)
 
@@ -1956,12 +1959,13 @@ def _prefill_runs(items: list, ends: list[int], kv_heads: int):
     stages, or None where one workgroup per item is about as good.  A workgroup walks one run of the (item,
     stage) sequence, so only the items at a run's ends are cut (at a stage, no piece under 4).
 
-    Estimated in stages of a workgroup (2.65 us with both of a CU's at work; prefill_pair.hip's take 2.1 to 2.2, and its partials as much less): the classic launch takes its
+    Estimated in stages of a workgroup (2.1 to 2.2 us with both of a CU's at work): the classic launch takes its
     greedy schedule in item order; the runs their share, 8 for the second launch and short runs, and
-    the cut items' partials (64 KiB each, written and read: 0.0124).  Against one workgroup per item, 8 kv heads:
-    1500 rows over 6100 keys (376 workgroups for 512 places) 282 -> 230 us with an fp8 cache, 248 -> 224 in bf16;
-    3000 over 5000: 427 -> 408; 256 over 3840: 110 -> 47 (in equal chunks: 51); 64 over 15936, fp8: 475 -> 41 (56).
-    Where the estimate is above 0.93 the partials cost what the balance gains: 1000 and 1000 over 2000, fp8, 96 -> 99."""
+    the cut items' partials (64 KiB each, written and read: 0.0124).  One workgroup an item -> runs, us, bf16 (fp8 cache), 8 kv heads, with the
+    estimates' quotient: 64 rows over 15936 keys (0.09) 388 -> 39 (458 -> 41), 256 over 3840 (0.37) 97 -> 40 (108 -> 45), 1500 over 7600 (0.83)
+    194 -> 176 (259 -> 192), 1500 over 6100 (0.84) 176 -> 148 (207 -> 157), 1200 over 3000 (0.87) 81 -> 67 (94 -> 74).  Not taken, though a little
+    ahead: 1024 over 3000 with 512 over 2200 (0.99) 82 -> 77 (95 -> 84).  Beyond, the partials cost what the balance gains: 2000 over 4000
+    (1.07) 114 -> 119 (128 -> 126), 3000 over 5000 (1.12) 180 -> 187 (198 -> 196), 1000 and 1000 over 2000 (1.41) 68 -> 80 (72 -> 79)."""
     slots = _PREFILL_SLOTS // max(1, kv_heads)
     units = [-(-e // 64) for e in ends]
     if not slots or len(items) > 4 * slots:   # the last wave is at most a quarter of the work
