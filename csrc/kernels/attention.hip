@@ -315,7 +315,7 @@ __device__ __forceinline__ int decode_part_span(int part_size, int seq_len, int 
 // The parts of a head, added in their order.  A launch of this size is latency and little else, so what it needs comes in two round trips:
 // the length, then all parts' maxima, sums (a thread a part) and outputs (AHEAD at a time).  One part after the other, each with
 // its own wait -> this: one request of 30000 tokens (118 parts, 32 heads) 37.4 -> 9.8 us, two of 9000 20.1 -> 6.2, eight of 700 5.2 -> 4.6, which
-// is what any launch takes here.
+// is what any launch takes here.  L takes the products of a sum and its factor unrounded (fma), as one part after the other had it.
 template <int D>
 __global__ __launch_bounds__(D) void paged_decode_reduce_kernel(const int* __restrict__ seq_lens,
                                                                  const float* __restrict__ part_o,
@@ -324,7 +324,9 @@ __global__ __launch_bounds__(D) void paged_decode_reduce_kernel(const int* __res
                                                                  int part_size, int max_parts,
                                                                  const float* __restrict__ sinks = nullptr) {
   constexpr int AHEAD = 16;
-  __shared__ float s_max[D / 64], s_w[D];
+  static_assert(D % 64 == 0, "whole waves");
+  __shared__ float s_max[D / 64];
+  __shared__ float2 s_w[D];   // sum and factor of a part
   const int b = blockIdx.y, head = blockIdx.x, d = threadIdx.x;
   const int seq_len = seq_lens[b];
   const int psz = decode_part_span(part_size, seq_len, max_parts);
@@ -334,7 +336,7 @@ __global__ __launch_bounds__(D) void paged_decode_reduce_kernel(const int* __res
   const float* po = part_o + base * D + d;
   const float2* ml = reinterpret_cast<const float2*>(part_ml) + base;
   float2 own = ml[min(d, nparts - 1)];
-  const float sink = sinks != nullptr ? sinks[head] * 1.4426950408889634f : 0.f;
+  const float sink = sinks != nullptr ? sinks[head] : 0.f;
   float o[AHEAD];
 #pragma unroll
   for (int i = 0; i < AHEAD; ++i) o[i] = po[(int64_t)min(i, nparts - 1) * D];
@@ -352,7 +354,7 @@ __global__ __launch_bounds__(D) void paged_decode_reduce_kernel(const int* __res
       __syncthreads();
       own = ml[min(p0 + d, nparts - 1)];
     }
-    s_w[d] = p0 + d < nparts ? own.y * fast_exp2(own.x - Mu) : 0.f;
+    s_w[d] = make_float2(own.y, fast_exp2(own.x - Mu));
     __syncthreads();
     const int n = min(D, nparts - p0);
     for (int i0 = 0; i0 < n; i0 += AHEAD) {
@@ -363,13 +365,13 @@ __global__ __launch_bounds__(D) void paged_decode_reduce_kernel(const int* __res
 #pragma unroll
       for (int i = 0; i < AHEAD; ++i)
         if (i0 + i < n) {
-          const float w = s_w[i0 + i];
-          L += w;
-          acc += w * o[i];
+          const float2 w = s_w[i0 + i];
+          L = __builtin_fmaf(w.x, w.y, L);
+          acc = __builtin_fmaf(w.x * w.y, o[i], acc);
         }
     }
   }
-  if (sinks != nullptr) L += fast_exp2(sink - Mu);
+  if (sinks != nullptr) L += fast_exp2(__builtin_fmaf(sink, 1.4426950408889634f, -Mu));
   out[(int64_t)b * out_stride + (int64_t)head * D + d] = (bf16)(L > 0.f ? acc / L : 0.f);
 }
 

@@ -60,3 +60,42 @@ def test_every_part_counts(D, lens, dynamic):
     ws.part_ml.fill_(float("nan"))
     out = ops.paged_decode(torch.zeros(B, Hq, D, dtype=torch.bfloat16, device=dev), kc, vc, bt, torch.tensor(lens, dtype=torch.int32, device=dev), 0.1, ws)
     assert bool(((out.double().cpu() - want).abs() <= 2.0 ** -8 * want + 1e-6).all())
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("dynamic", [False, True], ids=["spans", "own length"])
+@pytest.mark.parametrize("sinks", [False, True], ids=["", "sinks"])
+def test_order_of_the_sum(D, dynamic, sinks):
+    """Bit by bit: L = fma(l, 2^(m - M), L) and O = fma(l 2^(m - M), o, O) over a head's parts, one after the other, then the sink.  (Formed in 64 bits
+    and rounded, which is the fma but for a double rounding of 2^-29 of the cases.  L as a sum of rounded products moved some outputs by a step of bf16.)"""
+    torch.manual_seed(D + sinks)
+    dev, P, Hq, Hkv, B = "cuda", 16, 8, 2, 64
+    lens = [int(x) for x in torch.randint(129, 2500, (B,))]
+    pages = -(-max(lens) // P)
+    kc = torch.randn(pages, Hkv, P, D, device=dev).to(torch.bfloat16)
+    vc = torch.randn(pages, Hkv, D, P, device=dev).to(torch.bfloat16)
+    bt = torch.stack([torch.randperm(pages, dtype=torch.int32, device=dev) for _ in lens])
+    s = torch.randn(Hq, device=dev) if sinks else None
+    ws = ops.DecodeWorkspace(B, Hq, D, max(lens), 0 if dynamic else 128, dev, parts=12 if dynamic else None)
+    out = ops.paged_decode(torch.randn(B, Hq, D, device=dev).to(torch.bfloat16), kc, vc, bt, torch.tensor(lens, dtype=torch.int32, device=dev),
+                           D ** -0.5, ws, sinks=s).cpu()
+    o = ws.part_o.view(B, Hq, ws.max_parts, D).cpu()
+    ml = ws.part_ml.view(B, Hq, ws.max_parts, 2)
+
+    def fma(a, b, c):
+        return (a.double() * b.double() + c.double()).float()
+
+    for b, n in enumerate(lens):
+        span = max(128, -(-(-(-n // ws.max_parts)) // 128) * 128) if dynamic else 128
+        parts = -(-n // span)
+        m, l = ml[b, :, :parts, 0], ml[b, :, :parts, 1].cpu()
+        M = m.max(1, keepdim=True).values
+        e, M = torch.exp2(m - M).cpu(), M[:, 0].cpu()
+        L, acc = torch.zeros(Hq), torch.zeros(Hq, D)
+        for p in range(parts):
+            L = fma(l[:, p], e[:, p], L)
+            acc = fma((l[:, p] * e[:, p])[:, None], o[b, :, p], acc)
+        if sinks:
+            L = L + torch.exp2(fma(s.cpu(), torch.tensor(1.4426950408889634), -M).to(dev)).cpu()
+        if parts > 1:
+            assert torch.equal(out[b], (acc / L[:, None]).to(torch.bfloat16)), (b, n)
