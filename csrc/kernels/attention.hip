@@ -314,7 +314,7 @@ __device__ __forceinline__ int decode_part_span(int part_size, int seq_len, int 
 
 // The parts of a head, added in their order.  A launch of this size is latency and little else, so what it needs comes in two round trips:
 // the length, then all parts' maxima, sums (a thread a part) and outputs (AHEAD at a time).  One part after the other, each with
-// its own wait -> this: one request of 30000 tokens (118 parts, 32 heads) 37.4 -> 9.8 us, two of 9000 20.1 -> 6.2, eight of 700 5.2 -> 4.6, which
+// its own wait -> this: one request of 30000 tokens (118 parts, 32 heads) 37.4 -> 9.9 us, two of 9000 20.1 -> 6.2, eight of 700 5.2 -> 4.6, which
 // is what any launch takes here.  L takes the products of a sum and its factor unrounded (fma), as one part after the other had it.
 template <int D>
 __global__ __launch_bounds__(D) void paged_decode_reduce_kernel(const int* __restrict__ seq_lens,

@@ -18,7 +18,8 @@
 //     segment writes its fp32 accumulators to a slab in FRAGMENT order (thread-private, 1 KiB
 //     contiguous per wave instruction) and takes a ticket; the tile's last arriver acquires the
 //     slabs and adds them into its own registers element-wise (the slab layout is its own
-//     accumulator layout, so no shuffle) and runs the epilogue.  Nothing ever waits on another
+//     accumulator layout, so no shuffle) and runs the epilogue.  (Its own piece first: of three pieces
+//     and more the order of the sum, and the last bits with it, are another from run to run.)  Nothing ever waits on another
 //     workgroup (no co-residency assumption).  Hand-off = MI355X_MICROARCH.md "Valid forms"
 //     producer / consumer protocol: every storing wave vmcnt(0) -> barrier -> lane-0 agent
 //     release -> vmcnt(0) -> relaxed agent ticket; last arriver: agent acquire -> vmcnt(0) ->
