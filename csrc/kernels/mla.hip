@@ -261,6 +261,31 @@ __device__ __forceinline__ void mma_last(f32x16& d, bf16x8 a, bf16x8 b, const f3
 // half of them wide)
 __device__ __forceinline__ int row_swz(int r) { return (r >> 1 & 1) << 2 | (r >> 2 & 1) << 1 | (r >> 3 & 1); }
 
+// Sums of the lanes up to and with each (a row's lanes shifted, then the rows' last lanes broadcast), without LDS: a step of a __shfl is a round trip
+__device__ __forceinline__ int wave_scan(int x) {
+#define MLA_STEP(CTRL, ROWS) x += __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, true)
+  MLA_STEP(0x111, 0xf);   // row_shr 1, 2, 4, 8
+  MLA_STEP(0x112, 0xf);
+  MLA_STEP(0x114, 0xf);
+  MLA_STEP(0x118, 0xf);
+  MLA_STEP(0x142, 0xa);   // row_bcast 15, 31
+  MLA_STEP(0x143, 0xc);
+#undef MLA_STEP
+  return x;
+}
+__device__ __forceinline__ int wave_total(int x) { return __builtin_amdgcn_readlane(wave_scan(x), 63); }
+__device__ __forceinline__ int wave_most(int x) {   // the largest
+#define MLA_STEP(CTRL, ROWS) x = max(x, __builtin_amdgcn_update_dpp(x, x, CTRL, ROWS, 0xf, false))
+  MLA_STEP(0x111, 0xf);
+  MLA_STEP(0x112, 0xf);
+  MLA_STEP(0x114, 0xf);
+  MLA_STEP(0x118, 0xf);
+  MLA_STEP(0x142, 0xa);
+  MLA_STEP(0x143, 0xc);
+#undef MLA_STEP
+  return __builtin_amdgcn_readlane(x, 63);
+}
+
 // First token whose block-table row is e, by a 64-way search of the whole wave; -1: none.  tok_row ascends in the
 // runtime's prompts; of rows in any other order it may miss e, the same way for every caller.
 __device__ __forceinline__ int first_token(const int* __restrict__ tok_row, int T, int e) {
@@ -370,17 +395,13 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
       most = max(most, nt4[i]);
       all += nt4[i];
     }
-    auto count = [&](int span, int i) { return 4 * lane + i < T ? min(parts, max(1, (nt4[i] + span - 1) / span)) : 0; };
-    auto pieces = [&](int span) {
-      int n = count(span, 0) + count(span, 1) + count(span, 2) + count(span, 3);
-#pragma unroll
-      for (int x = 32; x > 0; x >>= 1) n += __shfl_xor(n, x);
-      return __builtin_amdgcn_readfirstlane(n) * HG;
+    auto count = [&](int span, int i) {   // (a quotient of tiles is off by one at most)
+      const int n = nt4[i] + span - 1, about = (int)((float)n * __builtin_amdgcn_rcpf((float)span)), rest = n - about * span;
+      return 4 * lane + i < T ? min(parts, max(1, about + (rest >= span) - (rest < 0))) : 0;
     };
-#pragma unroll
-    for (int x = 32; x > 0; x >>= 1) most = max(most, __shfl_xor(most, x)), all += __shfl_xor(all, x);
-    most = __builtin_amdgcn_readfirstlane(most);
-    all = __builtin_amdgcn_readfirstlane(all) * HG;
+    auto pieces = [&](int span) { return wave_total(count(span, 0) + count(span, 1) + count(span, 2) + count(span, 3)) * HG; };
+    most = wave_most(most);
+    all = wave_total(all) * HG;
     // all / span <= pieces <= all / span + units; one piece a unit is at most 256 (the caller's rule)
     int lo = max(SPAN, min(most, all / UNITS)), hi = T * HG < UNITS ? max(lo, min(most, all / (UNITS - T * HG) + 1)) : most;
     while (lo < hi) {
@@ -392,12 +413,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
     // keys 34 -> 28 us)
     if (most - lo <= 2 + R / 2048) lo = most;
     const int w = blockIdx.x, c0 = count(lo, 0), c1 = count(lo, 1), c2 = count(lo, 2), c3 = count(lo, 3);
-    int incl = c0 + c1 + c2 + c3;
-#pragma unroll
-    for (int x = 1; x < 64; x <<= 1) {
-      const int up = __shfl_up(incl, x);
-      if (lane >= x) incl += up;
-    }
+    const int incl = wave_scan(c0 + c1 + c2 + c3);
     if (w >= __builtin_amdgcn_readlane(incl, 63) * HG) return;   // whole block
     const int at = __popcll(__ballot(incl * HG <= w));            // the lane whose tokens piece w belongs to
     int tok = 4 * at, base = at ? __builtin_amdgcn_readlane(incl, at - 1) : 0;
@@ -428,14 +444,40 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
     const bool hv = row < row_end;
     const int t = min(DECODE ? unit / HG : row / H, T - 1), head = hv ? row - t * H : 0;
     const int my_row = tok_row[t], my_len = hv ? kv_lens[t] : 0;
+    // LDS lane bases; the XOR swizzle acts on the low three bits of a chunk index, the rest are immediates.
+    // S^T reads chunk 2 s + hf of key row col; V^T reads, for 16-lane group gr = lane / 16, rows 4 hf + qr (+ 8, 16, 24)
+    // and chunk 4 v + 2 (gr & 1) + pc / 2.
+    const int gr = lane >> 4, qr = (lane & 15) >> 2, pc = lane & 3;
+    uint32_t sofs[4], vofs[2], vofs8[2];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sofs[e] = (col * CH + ((2 * e + hf) ^ row_swz(col))) * 16;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      vofs[e] = ((4 * hf + qr) * CH + ((4 * e + 2 * (gr & 1) + (pc >> 1)) ^ row_swz(4 * hf + qr))) * 16 + (pc & 1) * 8;
+      vofs8[e] = (vofs[e] ^ 16) + 8 * CH * 16;   // of the row 8 further on
+    }
+    auto kfrag = [&](uint32_t img, int s) { return *reinterpret_cast<const bf16x8*>(sK + (sofs[s & 3] + img) + (s >> 2) * 128); };
+    // The queries: a wave's 32 rows are one image, so they come as a tile of keys does, 1 KB a move, and out of LDS into registers.  (Straight into
+    // registers a lane holds 16 bytes of its row at a time, 32 rows of two lanes: 128 rows 5.7 us on every CU at once, now 4.2; fewer rows are no slower so.)
     bf16x8 qf[NS];
-    const bf16* qp = q + (int64_t)t * q_stride_t + (int64_t)head * DK + 8 * hf;
+    const bool moved = NW == 4 && (((uintptr_t)q | (uintptr_t)(2 * q_stride_t)) & 15) == 0 && (uint64_t)q_stride_t < 1 << 26;   // (9 tokens a wave: 32-bit offsets)
+    if (moved) {
+      const int tw = __builtin_amdgcn_readfirstlane(t);
+      const uint32_t at = 2 * ((uint32_t)(t - tw) * (uint32_t)q_stride_t + (uint32_t)head * DK);
 #pragma unroll
-    for (int s = 0; s < NS; ++s) qf[s] = ld8(qp + 16 * s);
-    int Lmax = same ? tl_len : 0;
+      for (int b = 0; b < 9; ++b) {
+        const int c = 64 * b + lane, r8 = c / CH, x = (c - r8 * CH) ^ row_swz(r8);
 #pragma unroll
-    for (int x = 32; x > 0; x >>= 1) Lmax = max(Lmax, __shfl_xor(Lmax, x));
-    Lmax = __builtin_amdgcn_readfirstlane(Lmax);
+        for (int a = 0; a < 4; ++a)
+          buffer_to_lds(q + (int64_t)tw * q_stride_t, 0x7fffffffu, (uint32_t)__builtin_amdgcn_ds_bpermute(4 * (8 * a + r8), (int)at) + 16 * (x ^ (a & 1)), 0,
+                        lds0 + wave * IMG + 1024 * (9 * a + b));
+      }
+    } else {
+      const bf16* qp = q + (int64_t)t * q_stride_t + (int64_t)head * DK + 8 * hf;
+#pragma unroll
+      for (int s = 0; s < NS; ++s) qf[s] = ld8(qp + 16 * s);
+    }
+    const int Lmax = wave_most(same ? tl_len : 0);
     const int* bt = block_tables + (int64_t)bt_row * bt_stride;
     const int n_pages = (Lmax + 15) >> 4, tiles = (n_pages + 1) >> 1, per = (tiles + my_parts - 1) / my_parts;
     const int begin = part * per, end = min(tiles, begin + per);
@@ -463,10 +505,18 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
     // (The queries have come by then too.  The compiler, which does not know the moves, would otherwise wait for a query ahead of every product of S^T,
     // in the loop too, and so for all but a few of the moves that come after it.)
     look(begin);
+    if (moved) {
+#pragma unroll
+      for (int s = 0; s < NS; ++s) qf[s] = kfrag(wave * IMG, s);
+    }
 #if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
     for (int s = 0; s < NS; ++s) asm volatile("" : "+v"(qf[s]));
 #endif
+    if constexpr (NW == 4) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __syncthreads();   // (the images are the keys' from here on)
+    }
     const bf16 *b0 = cache, *b1 = cache;   // pages of the tile on its way, its image, its descriptors' size
     uint32_t to = 0, bytes = 0;
     auto aim = [&](int tile, int img) {    // (of a tile past the last nothing is read, zeros are written)
@@ -491,19 +541,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
 
     f32x16 o[NV];
 
-    // LDS lane bases; the XOR swizzle acts on the low three bits of a chunk index, the rest are immediates.
-    // S^T reads chunk 2 s + hf of key row col; V^T reads, for 16-lane group gr = lane / 16, rows 4 hf + qr (+ 8, 16, 24)
-    // and chunk 4 v + 2 (gr & 1) + pc / 2.
-    const int gr = lane >> 4, qr = (lane & 15) >> 2, pc = lane & 3;
-    uint32_t sofs[4], vofs[2], vofs8[2];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) sofs[e] = (col * CH + ((2 * e + hf) ^ row_swz(col))) * 16;
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      vofs[e] = ((4 * hf + qr) * CH + ((4 * e + 2 * (gr & 1) + (pc >> 1)) ^ row_swz(4 * hf + qr))) * 16 + (pc & 1) * 8;
-      vofs8[e] = (vofs[e] ^ 16) + 8 * CH * 16;   // of the row 8 further on
-    }
-    auto kfrag = [&](uint32_t img, int s) { return *reinterpret_cast<const bf16x8*>(sK + (sofs[s & 3] + img) + (s >> 2) * 128); };
     auto score = [&](uint32_t img, f32x16& to, auto&& beside) __attribute__((always_inline)) {   // S^T of the tile in image `img` (byte offset)
       f32x16 a;
       bf16x8 k[AHEAD];   // operands on their way from LDS
@@ -569,10 +606,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
       landed(begin + 2 < end);
       __syncthreads();
     }
-    int Lmin = L;   // the wave's shortest row: tiles below it have no key to mask
-#pragma unroll
-    for (int x = 32; x > 0; x >>= 1) Lmin = min(Lmin, __shfl_xor(Lmin, x));
-    Lmin = __builtin_amdgcn_readfirstlane(Lmin);
+    const int Lmin = -wave_most(-L);   // the wave's shortest row: tiles below it have no key to mask
     int cur = 0;
     for (int n = begin; n < end; ++n) {
       const int nxt = (cur + 1) & 3;
@@ -724,6 +758,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
       static_assert(NW * 32 * LD * 2 <= (int)sizeof(sK), "the output fits the images");
       bf16* so = reinterpret_cast<bf16*>(sK) + wave * 32 * LD;
       const uint64_t own = __ballot(mine);
+      const int64_t place = (int64_t)t * out_stride_t + (int64_t)head * DV;
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the first half's reads
@@ -738,11 +773,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (a wave's own rows: no barrier)
 #pragma unroll 4
         for (int i = 0; i < 16; ++i) {
-          const int lr = 2 * i + hf, r = row0 + wave * 32 + lr;
-          if ((own >> lr) & 1) {
-            const int tt = r / H;
-            st8(out + (int64_t)tt * out_stride_t + (int64_t)(r - tt * H) * DV + half * (DV / 2) + 8 * col, ld8(so + lr * LD + 8 * col));
-          }
+          // the row's place from the lane that holds it: divided out again for each row, the output took 5.1 us of a tile's life instead of 3.7
+          const int lr = 2 * i + hf;
+          const uint32_t lo = __builtin_amdgcn_ds_bpermute(4 * lr, (int)(uint32_t)place), hi = __builtin_amdgcn_ds_bpermute(4 * lr, (int)(uint32_t)(place >> 32));
+          const bf16x8 x = ld8(so + lr * LD + 8 * col);
+          if ((own >> lr) & 1) st8(out + (int64_t)((uint64_t)hi << 32 | lo) + half * (DV / 2) + 8 * col, x);
         }
       }
     } else if (!mine) {

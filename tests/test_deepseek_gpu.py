@@ -218,6 +218,25 @@ def test_mla_row_tiles_of_decode_steps(monkeypatch, lens, H, rows):
     assert (out.cpu().double() - want).abs().max() < 2.0 ** -8 * cache.float().abs().max().item()
 
 
+@pytest.mark.parametrize("decode", [False, True])
+@pytest.mark.parametrize("H", [20, 128])
+@pytest.mark.parametrize("first,pad", [(0, 64), (8, 8), (1, 0), (0, 4)], ids=str)
+def test_mla_row_tiles_take_queries_of_any_stride(monkeypatch, decode, H, first, pad):
+    """Rows that start on 16 bytes come by way of LDS, others straight into registers: the same bits; outputs of a wider row too."""
+    torch.manual_seed(H + first)
+    new = [1] * 9 if decode else [11, 3, 20]
+    cache, bt = _setup([40 + n for n in new])
+    row = torch.tensor([s for s, n in enumerate(new) for _ in range(n)], dtype=torch.int32, device=DEV)
+    kl = torch.tensor([40 + j + 1 for n in new for j in range(n)], dtype=torch.int32, device=DEV)
+    T = len(row)
+    wide = torch.randn(T * (H * 576 + pad) + 16, device=DEV).to(torch.bfloat16)
+    q = wide[first:first + T * (H * 576 + pad)].view(T, H * 576 + pad)[:, :H * 576].unflatten(1, (H, 576))
+    out = torch.empty(T, H * 512 + 24, dtype=torch.bfloat16, device=DEV)[:, :H * 512].unflatten(1, (H, 512))
+    monkeypatch.setattr(ops.MLAWorkspace, "tiles", lambda T, H, DK, *a: (128, decode, 2 if decode else 1))
+    want = ops.mla_attn(q.contiguous(), cache, bt, row, kl, 0.06)
+    assert torch.equal(ops.mla_attn(q, cache, bt, row, kl, 0.06, out=out), want)
+
+
 def test_mla_tile_rule_fits_workspace_and_chip():
     """Tiles of prompts fill at most one launch wave when partitioned; partials fit the workspace."""
     W = ops.MLAWorkspace
