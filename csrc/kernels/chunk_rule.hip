@@ -19,13 +19,16 @@
 //
 // What bounds it: the instructions of a wave that has its SIMD almost for itself, 96 matrix (Mamba-2: 54) and some 250 (270) vector
 // ones a chunk.  A product takes 16 cycles alone, but about 9 of them stay its own where vector instructions of 4 cycles fill
-// the rest, so a chunk is 2000 cycles of issue and as much again of LDS latency, address arithmetic and dependencies.  Hence the
-// next chunk moves to LDS by DMA, without a register or a store on the way; values and outputs move in pieces of four columns
+// the rest, so a chunk is 2000 cycles of issue and some 1400 of LDS latency and dependencies.  Hence the
+// next chunk moves to LDS by DMA, without a register or a store on the way, and where a workgroup has its CU to itself by two waves of their own: a
+// move holds its wave up for some 50 cycles, and the nine of a wave that also computes took a quarter of its time (scan of a delta rule, 192
+// workgroups 91 -> 73 us, 64 61 -> 49; selective scan, 256 54 -> 43, 128 40 -> 32; moves by one or by four such waves 73 and 77 for the first).  With two
+// workgroups a CU each covers the other's moves, and such waves only take slots from them (448 workgroups 36.7 -> 37.8, 512 76 -> 81): none there.  Values and outputs move in pieces of four columns
 // (q S is formed transposed for that); T and P T are products of three bf16 parts each, at half the fp32 product's time.
 // Memory traffic hides behind that.  Two fp16 parts instead of three bf16 ones would take a quarter less time, but the state came out
 // 2.3 times further from 64 bits: an fp16 value below 2^-14 has no lower part.
-// (chunks' matrices + scan, calls that are waited for one by one; many in a row, where the clock falls, the scans take 100 and 93):
-//   gated delta rule, 32 heads of 128 x 128, prompts of 1001 / 1435 / 1564 rows:   22 + 95 us (before: 24 + 123; row by row: 1098)
+// (chunks' matrices + scan, calls that are waited for one by one):
+//   gated delta rule, 32 heads of 128 x 128, prompts of 1001 / 1435 / 1564 rows:   22 + 75 us (before: 24 + 123; row by row: 1098)
 //   selective scan, 128 heads of 64 x 128, 8 groups, 1033 / 926 / 1248 / 293 rows:  10 + 85 us (values scaled by dt in three parts: 10 + 93; before: 11 + 116;
 //   row by row: 1745)
 // Largest error of the state against 64 bits: 1.2e-7 (row by row: 2.0e-7) and 1.2e-7 (6.2e-7) of its norm.
@@ -481,7 +484,8 @@ __global__ __launch_bounds__(256) void ssm_gram_kernel(RuleArgs a) {
 // product sit at 4 g + e, so with block b of S standing for key channels 32 (b / 2) + 8 (row / 4) + 4 (b % 2) +
 // row % 4, blocks 2 s and 2 s + 1 of a lane are the eight k-slots of step s of k S and q S: S never
 // leaves its registers.  S += k^T U takes k transposed out of the same LDS image (ds_read_b64_tr_b16).  The
-// next chunk moves to the other LDS buffer while this one is computed: one barrier per chunk.
+// next chunk moves to the other LDS buffer while this one is computed: one barrier per chunk.  MW > 0: by MW further waves, which do
+// nothing else and meet the others at each of their barriers; 0: by the waves that compute.
 // VEC: values in 16-byte pieces by DMA, outputs in 8-byte ones; not: element by element (views that are not aligned for that).
 //
 // SEG: few sequences of few heads leave most of the chip idle for their length, so they run in segments side by side.
@@ -489,8 +493,8 @@ __global__ __launch_bounds__(256) void ssm_gram_kernel(RuleArgs a) {
 //      transition M, the state of the identity's columns without values (workgroups beyond the values' in y).  The last segment has none.
 //   2  the segment itself, from S = M_i S + S_i over the segments before it (Mamba-2: M is the product of the decays).
 // ---------------------------------------------------------------------------------------------
-template <int DK, bool DELTA, int NW, bool VEC, int SEG = 0>
-__global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
+template <int DK, bool DELTA, int NW, bool VEC, int SEG, int MW>
+__global__ __launch_bounds__(64 * (NW + MW), 2) void chunk_rule_kernel(RuleArgs a) {
   constexpr int NS = DK / 32, NB = DK / 16, NT = 64 * NW, COLS = 16 * NW;
   constexpr int NML = RC * RC / 4 / NT;                  // 16-byte loads of q k^T per thread (Mamba-2)
   static_assert(NML * NT * 4 == RC * RC && RC * COLS == 8 * NT, "whole loads");
@@ -526,85 +530,117 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   const int chunks = (r1 - r0 + RC - 1) / RC;
   const int nc = (live ? n0 : 0) + col;
 
-  // values: thread -> row tid / 8, eight columns (beyond dv: the first eight); a last chunk of fewer rows repeats its last
-  // one (whose scalars are zero)
-  static_assert(COLS == 64, "eight pieces a row");
-  const int xr = tid / 8, xp8 = 8 * (val_img(xr, tid % 8) - 8 * xr), xc = c0 + xp8 < a.dv ? xp8 : 0;
-  uint32_t xo;
-  const char* xp = reinterpret_cast<const char*>(a.v + (int64_t)r0 * a.v_stride + (int64_t)h * a.dv + c0);
+  const bool few = r1 - r0 <= FEW && j == 0;            // whole block
+  // The moves of a chunk to LDS are cut into NW shares; a wave that moves has K of them: w0, w0 + MW, ...
+  constexpr int K = MW ? NW / MW : 1, KS = MW ? MW : NW;
+  static_assert(K * KS == NW && COLS == 64 && NT * 4 == VECS, "whole shares; eight pieces a row of values; a float a thread");
+  const int w0 = MW ? wave - NW : wave;
+  // values: a lane's row and eight columns (beyond dv: the first eight); a last chunk of fewer rows repeats its last one (whose scalars are zero)
   // rows of k and q: a lane's 16-byte piece of each move of 1024 bytes, against uniform bases
   constexpr int NR = ROWS / 1024 / NW, NH = (int)head_bytes<DELTA>() / 1024;
   static_assert(NR * NW * 1024 == ROWS && (NH - 1) % NW == 0, "whole moves");
-  uint32_t ko[NR];
-  const auto offsets = [&](int n) {
-    xo = 2 * ((uint32_t)min(xr, n - 1) * (uint32_t)a.v_stride + (uint32_t)xc);
+  uint32_t xo[K], ko[K][NR];
+  const auto offsets = [&](int n) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < NR; ++i) {
-      const int e = 64 * (wave + NW * i) + lane, row = e / (DK / 8);
-      ko[i] = 2 * ((uint32_t)min(row, n - 1) * (uint32_t)a.stride + 8 * (uint32_t)(img<DK>(row, e % (DK / 8)) - row * (DK / 8)));
-    }
-  };
-  const int64_t x_step = (int64_t)RC * 2 * a.v_stride, k_step = (int64_t)RC * 2 * a.stride, ws_step = ws_bytes<DELTA>(a.H, a.Hk), o_step = (int64_t)RC * 2 * a.out_stride;
-  const char* kp = reinterpret_cast<const char*>(a.k + (int64_t)r0 * a.stride + hk * DK);   // these walk with the chunks fetched
-  const char* qp = reinterpret_cast<const char*>(a.q + (int64_t)r0 * a.stride + hk * DK);
-  const char* gp = a.ws + (q0 / RC + s + j * a.seg) * ws_step + hk * group_bytes<DELTA>();
-  const char* hp = a.ws + (q0 / RC + s + j * a.seg) * ws_step + a.Hk * group_bytes<DELTA>() + h * head_bytes<DELTA>();
-  f32x4 rp[NML], rhj[NML], rlj[NML], rdj[NML];
-  float rhi[NML], rli[NML];
-  bf16x8 rx;
-  // The next chunk to LDS buffer b in three steps, for the vector memory unit to take one while another is computed.  `more`: there
-// is one; without, nothing is moved and what goes to registers is the last one again (no branch, which would part the stages).
-  const auto fetch = [&](int n, bool more, int b) {
-    if (more && n < RC) offsets(n);
-    const uint32_t to = lds0 + b * IMG, kb = (RC - 1) * 2 * (uint32_t)a.stride + 2 * DK;
-    if constexpr (VEC) {
-      buffer_to_lds(xp, more && !ident ? (uint32_t)(RC - 1) * 2 * (uint32_t)a.v_stride + 2 * COLS : 0, xo, 0, to + X_AT + 1024 * wave);
-    } else {
+    for (int k = 0; k < K; ++k) {
+      const int vt = 64 * (w0 + KS * k) + lane, xr = vt / 8, xp8 = 8 * (val_img(xr, vt % 8) - 8 * xr), xc = c0 + xp8 < a.dv ? xp8 : 0;
+      xo[k] = 2 * ((uint32_t)min(xr, n - 1) * (uint32_t)a.v_stride + (uint32_t)xc);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) rx[e] = *reinterpret_cast<const bf16*>(xp + xo + 2 * e);
-    }
-#pragma unroll
-    for (int i = 0; i < NR; ++i) {
-      buffer_to_lds(kp, more ? kb : 0, ko[i], 0, to + 1024 * (wave + NW * i));
-      if constexpr (SEG != 1) buffer_to_lds(qp, more ? kb : 0, ko[i], 0, to + ROWS + 1024 * (wave + NW * i));
-    }
-#pragma unroll
-    for (int i = 0; i < (NH - 1) / NW; ++i)
-      buffer_to_lds(hp, more ? (NH - 1) * 1024 : 0, 16 * lane, 1024 * (wave + NW * i), to + M_AT + 1024 * (wave + NW * i));
-    buffer_to_lds4(hp + (NH - 1) * 1024, more ? 4 * vec_floats<DELTA>() : 0, 4 * tid, to + V_AT + 256 * wave);
-    static_assert(NT * 4 == VECS, "a float a thread");
-    if constexpr (!DELTA && SEG != 1) {   // q k^T and its decays go through registers
-#pragma unroll
-      for (int i = 0; i < NML; ++i) {
-        rp[i] = *reinterpret_cast<const f32x4*>(gp + (uint32_t)(16 * (tid + NT * i)));
-        const uint32_t e = tid + NT * i, hi = 4 * (RC + e / (RC / 4)), hj = 4 * (RC + 4 * (e % (RC / 4)));
-        rhi[i] = *reinterpret_cast<const float*>(hp + hi);
-        rli[i] = *reinterpret_cast<const float*>(hp + (hi + 4 * RC));
-        rhj[i] = *reinterpret_cast<const f32x4*>(hp + hj);
-        rlj[i] = *reinterpret_cast<const f32x4*>(hp + (hj + 4 * RC));
-        rdj[i] = *reinterpret_cast<const f32x4*>(hp + (hj - 4 * RC));
+      for (int i = 0; i < NR; ++i) {
+        const int e = 64 * (w0 + KS * k + NW * i) + lane, row = e / (DK / 8);
+        ko[k][i] = 2 * ((uint32_t)min(row, n - 1) * (uint32_t)a.stride + 8 * (uint32_t)(img<DK>(row, e % (DK / 8)) - row * (DK / 8)));
       }
     }
   };
-  const auto advance = [&](bool more) {
+  const int64_t x_step = (int64_t)RC * 2 * a.v_stride, k_step = (int64_t)RC * 2 * a.stride, ws_step = ws_bytes<DELTA>(a.H, a.Hk);
+  const char* xp = reinterpret_cast<const char*>(a.v + (int64_t)r0 * a.v_stride + (int64_t)h * a.dv + c0);   // these walk with the chunks moved
+  const char* kp = reinterpret_cast<const char*>(a.k + (int64_t)r0 * a.stride + hk * DK);
+  const char* qp = reinterpret_cast<const char*>(a.q + (int64_t)r0 * a.stride + hk * DK);
+  const char* gp = a.ws + (q0 / RC + s + j * a.seg) * ws_step + hk * group_bytes<DELTA>();
+  const char* hp = a.ws + (q0 / RC + s + j * a.seg) * ws_step + a.Hk * group_bytes<DELTA>() + h * head_bytes<DELTA>();
+  // A chunk of n rows to LDS buffer b.  `more`: there is one; without, nothing is moved (no branch, which would part a step's stages).
+  const auto move = [&](int n, bool more, int b) __attribute__((always_inline)) {
+    if (more && n < RC) offsets(n);
+    const uint32_t to = lds0 + b * IMG, kb = (RC - 1) * 2 * (uint32_t)a.stride + 2 * DK;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int w = w0 + KS * k;
+      if constexpr (VEC) buffer_to_lds(xp, more && !ident ? (uint32_t)(RC - 1) * 2 * (uint32_t)a.v_stride + 2 * COLS : 0, xo[k], 0, to + X_AT + 1024 * w);
+#pragma unroll
+      for (int i = 0; i < NR; ++i) {
+        buffer_to_lds(kp, more ? kb : 0, ko[k][i], 0, to + 1024 * (w + NW * i));
+        if constexpr (SEG != 1) buffer_to_lds(qp, more ? kb : 0, ko[k][i], 0, to + ROWS + 1024 * (w + NW * i));
+      }
+#pragma unroll
+      for (int i = 0; i < (NH - 1) / NW; ++i) buffer_to_lds(hp, more ? (NH - 1) * 1024 : 0, 16 * lane, 1024 * (w + NW * i), to + M_AT + 1024 * (w + NW * i));
+      buffer_to_lds4(hp + (NH - 1) * 1024, more ? 4 * vec_floats<DELTA>() : 0, 4 * (64 * w + lane), to + V_AT + 256 * w);
+    }
+  };
+  const auto advance = [&](bool more) __attribute__((always_inline)) {
     xp += more ? x_step : 0;
     kp += more ? k_step : 0;
     qp += more ? k_step : 0;
     gp += more ? ws_step : 0;
     hp += more ? ws_step : 0;
   };
-  const auto put = [&](int b) {   // P_ij dt_j = q_i.k_j exp(cum_i - cum_j) dt_j, j <= i; cum in two parts (long sums, short differences)
+  if (MW && wave >= NW) {
+    if (few) return;
+    if constexpr (SEG == 2 && DELTA) {   // the barriers of `start`
+      for (int i = 1; i < j; ++i) {
+        if (i > 1) __syncthreads();
+        __syncthreads();
+      }
+      if (j > 1) __syncthreads();
+    }
+    offsets(RC);
+    for (int c = 0; c < chunks; ++c) {   // (the buffer was read last before the previous barrier)
+      move(r1 - r0 - c * RC, true, c & 1);
+      advance(true);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+    }
+    __syncthreads();
+    return;
+  }
+
+  // What goes through registers comes a chunk ahead of the products: q k^T and its decays (Mamba-2), values by element.  Without a next chunk
+  // it is the last one again (no branch, which would part the stages).
+  f32x4 rp[NML], rhj, rlj, rdj;
+  float rhi[NML], rli[NML];
+  bf16x8 rx;
+  const auto ahead = [&](int c) __attribute__((always_inline)) {   // of chunk c
+    if constexpr (!VEC) {
+      const int xr = min(tid / 8, r1 - r0 - c * RC - 1), xp8 = 8 * (val_img(tid / 8, tid % 8) - 8 * (tid / 8));
+      const bf16* x = a.v + (int64_t)(r0 + c * RC + xr) * a.v_stride + (int64_t)h * a.dv + c0 + (c0 + xp8 < a.dv ? xp8 : 0);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) rx[e] = x[e];
+    }
+    if constexpr (!DELTA && SEG != 1) {
+      const uint32_t hj = 4 * (RC + 4 * (tid % (RC / 4)));
+      rhj = *reinterpret_cast<const f32x4*>(hp + hj);
+      rlj = *reinterpret_cast<const f32x4*>(hp + (hj + 4 * RC));
+      rdj = *reinterpret_cast<const f32x4*>(hp + (hj - 4 * RC));
+#pragma unroll
+      for (int i = 0; i < NML; ++i) {
+        const uint32_t e = tid + NT * i, hi = 4 * (RC + e / (RC / 4));
+        rp[i] = *reinterpret_cast<const f32x4*>(gp + 16 * e);
+        rhi[i] = *reinterpret_cast<const float*>(hp + hi);
+        rli[i] = *reinterpret_cast<const float*>(hp + (hi + 4 * RC));
+      }
+    }
+  };
+  const auto put = [&](int b) __attribute__((always_inline)) {   // P_ij dt_j = q_i.k_j exp(cum_i - cum_j) dt_j, j <= i; cum in two parts (long sums, short differences)
     if constexpr (!VEC) *reinterpret_cast<bf16x8*>(lds + b * IMG + X_AT + 16 * tid) = rx;
     if constexpr (!DELTA && SEG != 1) {
 #pragma unroll
       for (int i = 0; i < NML; ++i) {
-        const int e = tid + NT * i, row = e / (RC / 4), j = 4 * (e % (RC / 4));
+        const int e = tid + NT * i, row = e / (RC / 4), jj = 4 * (e % (RC / 4));
         f32x4 x;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) x[t] = j + t <= row ? rp[i][t] * __expf((rhi[i] - rhj[i][t]) + (rli[i] - rlj[i][t])) * rdj[i][t] : 0.f;
+        for (int t = 0; t < 4; ++t) x[t] = jj + t <= row ? rp[i][t] * __expf((rhi[i] - rhj[t]) + (rli[i] - rlj[t])) * rdj[t] : 0.f;
         bf16x4 p[3];
         cut3(x, p);
-        const int at = b * IMG + M_AT + mat_img(row, (j & 15) >> 2) + 8 * (j >> 4);
+        const int at = b * IMG + M_AT + mat_img(row, (jj & 15) >> 2) + 8 * (jj >> 4);
 #pragma unroll
         for (int m = 0; m < 3; ++m) *reinterpret_cast<bf16x4*>(lds + at + m * MAT) = p[m];
       }
@@ -634,6 +670,7 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
 #pragma unroll
     for (int b = 0; b < NB; ++b) S[b] = f32x4{0.f, 0.f, 0.f, 0.f};
   };
+  const int64_t o_step = (int64_t)RC * 2 * a.out_stride;
   const int64_t mine = (int64_t)nc * DK + 8 * g, copy = (int64_t)a.dv * DK;   // places in a segment's floats
   const float Dh = DELTA ? 0.f : a.D[h];
   // outputs: lane (col, g) holds rows col and 16 + col, columns n0 + 4 g .. + 3
@@ -761,27 +798,28 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
   };
   start();
 
-  const bool few = r1 - r0 <= FEW && j == 0;            // whole block
   if (!few) {
-    offsets(min(RC, r1 - r0));
-    fetch(RC, true, 0);
+    if constexpr (MW == 0) {
+      offsets(min(RC, r1 - r0));
+      move(RC, true, 0);
+    }
+    ahead(0);
     advance(chunks > 1);
     put(0);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if constexpr (MW == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
   }
   float decay = 1.f;   // of the chunks so far (SEG 1, Mamba-2)
   // One chunk.  With one or two waves a SIMD nothing else covers an LDS read: each is issued a stage before its use, and the
   // scheduling barriers keep the compiler from sinking it there.
   const auto step = [&](int c, int b) {
-    const bool more = c + 1 < chunks;
     const char* L = lds + b * IMG;
     const bf16 *K = reinterpret_cast<const bf16*>(L), *Q = reinterpret_cast<const bf16*>(L + ROWS), *X = reinterpret_cast<const bf16*>(L + X_AT);
     const float* V = reinterpret_cast<const float*>(L + V_AT);
     const auto vec = [&](int i, int rb) { return *reinterpret_cast<const f32x4*>(V + i * RC + 16 * rb + 4 * g); };
     const auto mat = [&](int m, int rb) { return *reinterpret_cast<const bf16x8*>(L + M_AT + m * MAT + mat_img(16 * rb + col, g)); };
     const auto rows = [&](const bf16* R, int rb, int t) { return ld8(R + img<DK>(16 * rb + col, 4 * t + g) * 8); };
-    // ---- first operands; the next chunk's moves ----
+    // ---- first operands ----
     bf16x4 x[2], y[2];
     f32x4 va[2], vb[2], vd[2];
     bf16x8 kf[2][NS], qf[2][NS];
@@ -800,8 +838,8 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
         vb[rb] = vec(1, rb);
       }
     }
-    __builtin_amdgcn_sched_barrier(0x0f);
-    fetch(r1 - r0 - (c + 1) * RC, more, b ^ 1);   // (that buffer was read last before the previous barrier)
+    if constexpr (MW == 0) move(r1 - r0 - (c + 1) * RC, c + 1 < chunks, b ^ 1);   // (that buffer was read last before the previous barrier)
+    ahead(min(c + 1, chunks - 1));
     advance(c + 2 < chunks);
     if constexpr (DELTA && SEG != 1) {
 #pragma unroll
@@ -903,8 +941,10 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
       for (int nb = 0; nb < NB; ++nb) S[nb] = mma_bf16(ka[nb], us[p], S[nb]);
     if constexpr (SEG == 1) {
       if constexpr (!DELTA) decay *= gc;
-      __builtin_amdgcn_sched_barrier(0);
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next chunk has landed
+      if constexpr (MW == 0) {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next chunk has landed
+      }
       __syncthreads();
       return;
     }
@@ -916,8 +956,10 @@ __global__ __launch_bounds__(64 * NW, 2) void chunk_rule_kernel(RuleArgs a) {
         for (int t = 0; t < 4; ++t) o[rb][t] += Dh * (float)y[rb][t];
     }
     put(b ^ 1);
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next chunk has landed (before the stores below, which nobody waits for)
+    if constexpr (MW == 0) {
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next chunk has landed (before the stores below, which nobody waits for)
+    }
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
       const bool in = live && 16 * rb + col < r1 - r0 - c * RC;
@@ -970,24 +1012,23 @@ int launch_rule(RuleArgs a, int T, int dk, hipStream_t stream) {
   a.segs = reinterpret_cast<float*>(end);
   const int cols = (a.dv + 63) / 64, ids = a.seg ? T / (RC * a.seg) + a.S : a.S;
   if (ids > 65535) return -3;
+  const bool alone = (int64_t)a.H * cols * ids <= 256;   // one workgroup a CU at most: waves that move (chunk_rule_kernel)
   const dim3 gram(T / RC + a.S, DELTA ? (a.H + 3) / 4 : a.Hk), rule(a.H, cols, ids), own(a.H, cols + (DELTA ? dk / 64 : 0), ids);
-  if (dk == 128) {
-    if constexpr (DELTA) chunk_gram_kernel<128><<<gram, 256, 0, stream>>>(a);
-    else ssm_gram_kernel<128><<<gram, 256, 0, stream>>>(a);
-    if (vec && a.seg) {
-      chunk_rule_kernel<128, DELTA, 4, true, 1><<<own, 256, 0, stream>>>(a);
-      chunk_rule_kernel<128, DELTA, 4, true, 2><<<rule, 256, 0, stream>>>(a);
-    } else if (vec) chunk_rule_kernel<128, DELTA, 4, true><<<rule, 256, 0, stream>>>(a);
-    else chunk_rule_kernel<128, DELTA, 4, false><<<rule, 256, 0, stream>>>(a);
-  } else {
-    if constexpr (DELTA) chunk_gram_kernel<64><<<gram, 256, 0, stream>>>(a);
-    else ssm_gram_kernel<64><<<gram, 256, 0, stream>>>(a);
-    if (vec && a.seg) {
-      chunk_rule_kernel<64, DELTA, 4, true, 1><<<own, 256, 0, stream>>>(a);
-      chunk_rule_kernel<64, DELTA, 4, true, 2><<<rule, 256, 0, stream>>>(a);
-    } else if (vec) chunk_rule_kernel<64, DELTA, 4, true><<<rule, 256, 0, stream>>>(a);
-    else chunk_rule_kernel<64, DELTA, 4, false><<<rule, 256, 0, stream>>>(a);
+#define CHUNKS(DK)                                                                                                      \
+  {                                                                                                                     \
+    if constexpr (DELTA) chunk_gram_kernel<DK><<<gram, 256, 0, stream>>>(a);                                            \
+    else ssm_gram_kernel<DK><<<gram, 256, 0, stream>>>(a);                                                              \
+    if (vec && a.seg) {                                                                                                 \
+      chunk_rule_kernel<DK, DELTA, 4, true, 1, 4><<<own, 64 * 8, 0, stream>>>(a);                                       \
+      if (alone) chunk_rule_kernel<DK, DELTA, 4, true, 2, 2><<<rule, 64 * 6, 0, stream>>>(a);                           \
+      else chunk_rule_kernel<DK, DELTA, 4, true, 2, 0><<<rule, 256, 0, stream>>>(a);                                    \
+    } else if (!vec) chunk_rule_kernel<DK, DELTA, 4, false, 0, 0><<<rule, 256, 0, stream>>>(a);                         \
+    else if (alone) chunk_rule_kernel<DK, DELTA, 4, true, 0, 2><<<rule, 64 * 6, 0, stream>>>(a);                        \
+    else chunk_rule_kernel<DK, DELTA, 4, true, 0, 0><<<rule, 256, 0, stream>>>(a);                                      \
   }
+  if (dk == 128) CHUNKS(128)
+  else CHUNKS(64)
+#undef CHUNKS
   OME_CHECK_LAUNCH();
   return 0;
 }

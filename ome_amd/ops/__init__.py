@@ -177,7 +177,7 @@ def _chunk_rule_seg_floats(dk: int, dv: int) -> int:
 
 
 def _chunk_rule_seg(T: int, S: int, H: int, dv: int, delta: bool) -> int:
-    """Chunks of a segment, or 0 where sequences run in one piece.  A chunk is 1.7 us of a serial chain and the chip holds 512 workgroups:
+    """Chunks of a segment, or 0 where sequences run in one piece.  A chunk is 1.1 to 1.7 us of a serial chain and the chip holds 512 workgroups:
     where the sequences have far fewer, segments of them run side by side.  For that every segment but the last is walked once
     more for its own state and (delta rule) transition, at 0.4 (1.4) of its cost, and a segment's start takes a step of
     1 (2.5) us over each one before it; hence lengths near sqrt(chunks), longer where those fill the chip.  Whole layers in us, one
@@ -186,12 +186,18 @@ def _chunk_rule_seg(T: int, S: int, H: int, dv: int, delta: bool) -> int:
     1 x 1000 96 -> 91, 1 x 4000 299 -> 218, 2 x 4000 (128 workgroups) 243 -> 245; 1 x 300 46 -> 50;
     selective scan, 32 heads 1 x 1000 81 -> 55, 1 x 8000 435 -> 136, 4 x 4000 116 -> 92, 8 x 8000 (256) 130 -> 145; 128 heads
     1 x 1000 95 -> 84, 1 x 8000 638 -> 440, 2 x 4000 (256) 220 -> 225; 1 x 300 42 -> 44.
+    Segments of up to twice that length where they make the workgroups at most 256: alone on a CU each takes a fifth less time a chunk, as waves
+    of its own move its data (``chunk_rule.hip``).  Scans alone in us, such lengths -> these: delta rule, 8 heads 2 x 8000 144 -> 135, 4 x 8000
+    111 -> 101; 32 heads 1 x 1000 as before (256); selective scan, 32 heads 1 x 8000 90 -> 75, 2 x 3000 53 -> 42, 64 heads 1 x 1500 45 -> 38, 1 x 4000
+    77 -> 70, 128 heads 1 x 800 43 -> 38, 1 x 7000 214 -> 223; at more than twice the length 64 heads 2 x 6000 98 -> 115.
     Lengths are on the device, so decode rows beside a prompt count as sequences like it, and such a step stays in one piece."""
-    wgs, chunks = H * -(-dv // 64) * S, -(-T // (32 * S))
+    one = H * -(-dv // 64)
+    wgs, chunks = one * S, -(-T // (32 * S))
     if chunks < 24 or wgs > (64 if delta else 192):
         return 0
     pieces = chunks / max(8, 1.3 * chunks ** 0.5, chunks * wgs / (256 if delta else 512))
-    return -(-chunks // max(2, round(pieces)))
+    seg = -(-chunks // max(2, round(pieces)))
+    return next((n for n in range(seg, 2 * seg + 1) if (T // (32 * n) + S) * one <= 256), seg)
 
 
 def _chunk_rule_ws(T: int, S: int, H: int, G: int, dk: int, dv: int, delta: bool, state: torch.Tensor, rows: tuple) -> torch.Tensor | None:

@@ -297,6 +297,33 @@ def test_scans_in_segments(lens, seg, delta, monkeypatch):
             test_selective_scan_prompts(lens, *dims)
 
 
+@pytest.mark.parametrize("seg", [0, 1, 2])
+@pytest.mark.parametrize("dk", [64, 128])
+@pytest.mark.parametrize("delta", [True, False])
+def test_many_workgroups_as_few(delta, dk, seg, monkeypatch):
+    """Chunks moved by waves of their own (up to 256 workgroups) or by those that compute (more): the same bits."""
+    monkeypatch.setattr(ops, "_chunk_rule_seg", lambda *a: seg)
+    torch.manual_seed(dk + seg)
+    lens, H, dv = [31, 3, 97, 0, 64, 1, 33], 96, 64
+    T, sq = sum(lens), seqs(lens, 8)
+    q, k, v = (torch.randn(T, H * d, device=DEV).to(BF) for d in (dk, dk, dv))
+    ab, st = torch.randn(2, T, H, device=DEV).to(BF), torch.randn(8, H, dv, dk, device=DEV)
+    A, zero = torch.linspace(-3, 0, H, device=DEV), torch.zeros(H, device=DEV)
+
+    def scan(n):
+        s = st[:, :n].clone()
+        if delta:
+            o = ops.gdn_scan(q[:, :n * dk], k[:, :n * dk], v.as_strided((T, n * dv), (H * dk, 1)), ab[0, :, :n], ab[1, :, :n], A[:n], zero[:n], s, *sq, n, n)
+        else:
+            o = ops.ssm_scan(v[:, :n * dv], ab[0, :, :n], k[:, :n * dk], q[:, :n * dk], -A[:n].exp(), zero[:n], zero[:n], 0.001, s, *sq, n, dv, dk, n)
+        return o, s
+
+    if delta:   # (values share the row stride of q and k)
+        v = torch.randn(T, H * dk, device=DEV).to(BF)
+    (o, s), (few, s2) = scan(H), scan(2)
+    assert torch.equal(o[:, :2 * dv], few) and torch.equal(s[:, :2], s2)
+
+
 @pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
 @pytest.mark.parametrize("what", ["q", "k", "v", "a", "b"])
 def test_delta_rule_in_segments_stays_causal(what, bad, monkeypatch):
