@@ -176,6 +176,7 @@ def _chunk_rule_seg_floats(dk: int, dv: int) -> int:
     return load().ome_chunk_rule_seg_floats(dk, dv)
 
 
+@functools.lru_cache(maxsize=4096)
 def _chunk_rule_seg(T: int, S: int, H: int, dv: int, delta: bool) -> int:
     """Chunks of a segment, or 0 where sequences run in one piece.  A chunk is 1.1 to 1.7 us of a serial chain and the chip holds 512 workgroups:
     where the sequences have far fewer, segments of them run side by side.  For that every segment but the last is walked once
@@ -214,10 +215,10 @@ def _chunk_rule_ws(T: int, S: int, H: int, G: int, dk: int, dv: int, delta: bool
     70..82), 64 x 1 and a prompt of 32 76 (66), 200 x 1 and one of 300 522 (197)."""
     if T <= max(S, 32 if delta else 4) or dk not in (64, 128) or dv % 16 or S > 65535 or H > 65535:
         return None
-    q, k, o = rows[0], rows[1], rows[-1]   # (a shared row stride for q, k and v / B and C)
+    q, k, v, o = rows[0], rows[1], rows[-2], rows[-1]   # (a shared row stride for q, k and v / B and C)
     sq, so = q.stride(0), o.stride(0)
     if (state.data_ptr() | q.data_ptr() | k.data_ptr()) % 16 or sq % 8 or not (0 <= sq < 1 << 24 and 0 <= so < 1 << 24) or \
-            not 0 <= rows[-2].stride(0) < 1 << 24 or o.data_ptr() == rows[-2].data_ptr():
+            not 0 <= v.stride(0) < 1 << 24 or o.data_ptr() == v.data_ptr():
         return None
     floats = (T // 32 + S) * _chunk_rule_floats(H, G, delta)
     seg = _chunk_rule_seg(T, S, H, dv, delta)
@@ -263,23 +264,23 @@ def gdn_scan(q, k, v, a, b, A_log, dt_bias, state, cu, slot, reset, Hv: int, Hk:
     out = v.new_empty(T, Hv * dv) if out is None else out
     if not _gpu(q):
         return ref.gdn_scan(q, k, v, a, b, A_log, dt_bias, state, cu, slot, reset, Hv, Hk, out)
-    assert q.stride(0) == k.stride(0) == v.stride(0) and a.stride(0) == b.stride(0)
-    assert q.stride(1) == k.stride(1) == v.stride(1) == a.stride(1) == 1 and out.stride(1) == 1
+    sq, sa, so = q.stride(), a.stride(), out.stride()
+    assert sq == k.stride() == v.stride() and sq[1] == 1 and sa[0] == b.stride(0) and sa[1] == 1 and so[1] == 1
     assert state.is_contiguous() and state.dtype == torch.float32
     f32 = _f32(q, k, v, a, b, out)
     S = slot.shape[0]
     ws = None if v1 or f32 or Hk <= 0 or Hv % Hk else _chunk_rule_ws(T, S, Hv, Hk, dk, dv, True, state, (q, k, v, out))
     if ws is not None:   # prompts: chunks of 32 rows on the matrix cores
-        call("ome_gdn_chunks", q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), a.data_ptr(), b.data_ptr(),
-             a.stride(0), A_log.data_ptr(), dt_bias.data_ptr(), state.data_ptr(), out.data_ptr(), out.stride(0),
+        call("ome_gdn_chunks", q.data_ptr(), k.data_ptr(), v.data_ptr(), sq[0], a.data_ptr(), b.data_ptr(),
+             sa[0], A_log.data_ptr(), dt_bias.data_ptr(), state.data_ptr(), out.data_ptr(), so[0],
              _i32(cu).data_ptr(), _i32(slot).data_ptr(), _i32(reset).data_ptr(), S, T, Hv, Hk, dk, dv,
              _chunk_rule_seg(T, S, Hv, dv, True), ws.data_ptr(), stream_ptr())
         return out
     if T == S and not v1 and not f32 and dk in (64, 128, 256) and 0 < Hv <= 65535 and Hk > 0 and Hv % Hk == 0 and \
-            q.data_ptr() % 16 == 0 and k.data_ptr() % 16 == 0 and q.stride(0) % 8 == 0 and 0 < dv < 1 << 20:
+            q.data_ptr() % 16 == 0 and k.data_ptr() % 16 == 0 and sq[0] % 8 == 0 and 0 < dv < 1 << 20:
         # a decode step: the normalisation inside the scan (47.9 -> 43.9 us at 64 sequences of 32 heads)
-        call("ome_gdn_step", q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), a.data_ptr(), b.data_ptr(),
-             a.stride(0), A_log.data_ptr(), dt_bias.data_ptr(), state.data_ptr(), out.data_ptr(), out.stride(0),
+        call("ome_gdn_step", q.data_ptr(), k.data_ptr(), v.data_ptr(), sq[0], a.data_ptr(), b.data_ptr(),
+             sa[0], A_log.data_ptr(), dt_bias.data_ptr(), state.data_ptr(), out.data_ptr(), so[0],
              _i32(cu).data_ptr(), _i32(slot).data_ptr(), _i32(reset).data_ptr(), T, Hv, Hk, dk, dv, stream_ptr())
         return out
     # (key widths other than 64 / 128 / 256, and fp32 models, run the launcher's generic kernel: no workspace)
