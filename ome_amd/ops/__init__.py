@@ -1955,6 +1955,8 @@ def prefill_rows(Hq: int, Hkv: int, D: int, page: int = 16) -> int:
 # 2000 keys (27 vs 34 us, 85 vs 93 us).  r06 tried 256: +0.5 % in-process (16.30k -> 16.39k,
 # within box noise) but -7 % over HTTP (15.05k -> 14.01k, profiles/r06_step_cost_ab.txt), so 2048 stays
 PREFILL_SPLIT_MIN_KEYS = int(os.environ.get("OME_PREFILL_SPLIT_MIN_KEYS", "2048"))
+# ... and more than 17 stages of 64 keys before runs of equal stages are looked at, which are a little ahead down to 10 (40 rows over 740 keys 24 -> 17 us)
+PREFILL_RUNS_MIN_KEYS = 1088
 
 
 # workgroups of the 32-row GQA-4 kernel that the chip holds at once: 2 (LDS, registers) on each of 256 CUs
@@ -1966,13 +1968,16 @@ def _prefill_runs(items: list, ends: list[int], kv_heads: int):
     stages, or None where one workgroup per item is about as good.  A workgroup walks one run of the (item,
     stage) sequence, so only the items at a run's ends are cut (at a stage, no piece under 4).
 
-    Estimated in stages of a workgroup (2.1 to 2.2 us with both of a CU's at work): the classic launch takes its
-    greedy schedule in item order; the runs their share, 8 for the second launch and short runs, and
-    the cut items' partials (64 KiB each, written and read: 0.0124).  One workgroup an item -> runs, us, bf16 (fp8 cache), 8 kv heads, with the
-    estimates' quotient: 64 rows over 15936 keys (0.09) 388 -> 39 (458 -> 41), 256 over 3840 (0.37) 97 -> 40 (108 -> 45), 1500 over 7600 (0.83)
-    194 -> 176 (259 -> 192), 1500 over 6100 (0.84) 176 -> 148 (207 -> 157), 1200 over 3000 (0.87) 81 -> 67 (94 -> 74).  Not taken, though a little
-    ahead: 1024 over 3000 with 512 over 2200 (0.99) 82 -> 77 (95 -> 84).  Beyond, the partials cost what the balance gains: 2000 over 4000
-    (1.07) 114 -> 119 (128 -> 126), 3000 over 5000 (1.12) 180 -> 187 (198 -> 196), 1000 and 1000 over 2000 (1.41) 68 -> 80 (72 -> 79)."""
+    Estimated in stages of a workgroup (1.7 us, 2.1 to 2.2 with both of a CU's at work): the classic launch takes its
+    greedy schedule in item order; the runs their share, of 4 at the least, 4 (where there is work for every place: 8) for the second launch and short runs,
+    and the cut items' partials (64 KiB each, written and read: 0.0124; no piece is under 4).  One workgroup an item -> runs, us,
+    bf16 (fp8 cache), 8 kv heads, with the estimates' quotient: 64 rows over 15936 keys (0.09) 388 -> 39 (458 -> 41), 256 over 3840 (0.37) 97 -> 40
+    (108 -> 45), 1500 over 7600 (0.83) 194 -> 176 (259 -> 192), 1500 over 6100 (0.84) 176 -> 148 (207 -> 157), 1200 over 3000 (0.87) 81 -> 67 (94 -> 74);
+    twice 28 over 1900 (0.32) 52 -> 23 (56 -> 24), 40 over 1540 (0.36) 43 -> 20 (47 -> 21), 139 over 1540 (0.47) 44 -> 27 (47 -> 29), four of 30 over 1430
+    (0.49) 41 -> 24 (45 -> 26), 300 over 1300 (0.65) 38 -> 30 (41 -> 32).  Not taken, though a little ahead: 1000 over 2000 (0.94) 56 -> 52 (61 -> 57), 1024
+    over 3000 with 512 over 2200 (0.99) 82 -> 77 (95 -> 84), 600 over 1200 (1.08) 36 -> 33 (38 -> 36), four of 200 over 1700 (1.05) 48 -> 46 (52 -> 49).
+    Beyond, the partials cost what the balance gains: 2000 over 4000 (1.07) 114 -> 119 (128 -> 126), 3000 over 5000 (1.12) 180 -> 187 (198 -> 196), 1900 alone (1.16)
+    55 -> 68 (63 -> 71), 1000 and 1000 over 2000 (1.41) 68 -> 80 (72 -> 79)."""
     slots = _PREFILL_SLOTS // max(1, kv_heads)
     units = [-(-e // 64) for e in ends]
     if not slots or len(items) > 4 * slots:   # the last wave is at most a quarter of the work
@@ -1980,8 +1985,10 @@ def _prefill_runs(items: list, ends: list[int], kv_heads: int):
     busy = [0] * slots
     for u in units:
         heapq.heapreplace(busy, busy[0] + u)
-    total, cuts = sum(units), slots + len(items)
-    if total / slots + 8 + 0.0124 * cuts * kv_heads >= 0.93 * max(busy):
+    total = sum(units)
+    few = total < 4 * slots   # fewer runs than places
+    cuts = (total // 4 if few else slots) + len(items)
+    if max(total / slots, 4) + (4 if few else 8) + 0.0124 * cuts * kv_heads >= 0.93 * max(busy):
         return None
     pieces, comb, runs, parts = [], [], [], 0
     done, first, bound = 0, 0, total / slots   # stages dealt out; this run's first piece and end
@@ -2043,7 +2050,7 @@ def prefill_plan(q_lens: list[int], kv_lens: list[int], tile: int = 32, target: 
         e = (kv_lens[s] - q_lens[s]) + min(r + 32, q_lens[s])
         ends.append(e)
         work += e
-    if runs and not force and max(ends, default=0) > PREFILL_SPLIT_MIN_KEYS:
+    if runs and not force and max(ends, default=0) > PREFILL_RUNS_MIN_KEYS:
         equal = _prefill_runs(items32, ends, kv_heads)
         if equal is not None:
             return items, *equal

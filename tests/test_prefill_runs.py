@@ -74,6 +74,19 @@ def test_runs_match_reference(q_lens, kv_lens, Hq, Hkv, cache, mode):
     assert (out.float() - want.float()).abs().max().item() < 2 * 2.0 ** -9 * 2.5
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("q_lens,kv_lens,Hq,Hkv", [([28, 28], [1899, 1899], 32, 8), ([139], [1539], 32, 8), ([1], [1089], 4, 1), ([33, 2], [1120, 2048], 16, 4)])
+@pytest.mark.parametrize("cache", [torch.bfloat16, torch.float8_e4m3fn], ids=str)
+def test_runs_of_shorter_contexts_match_reference(q_lens, kv_lens, Hq, Hkv, cache):
+    test_runs_match_reference(q_lens, kv_lens, Hq, Hkv, cache, "plain")
+
+
+@pytest.mark.parametrize("q,kv,runs", [([40], [1088], False), ([40], [1089], True), ([28, 28], [1899, 1899], True), ([300], [1300], True),
+                                       ([1900], [1900], False), ([200] * 4, [1700] * 4, False), ([2000], [6000], False), ([3000], [8000], False)])
+def test_runs_where_they_are_faster(q, kv, runs):
+    assert (ops.prefill_plan(q, kv)[3] < 0) == runs
+
+
 @pytest.mark.parametrize("q,kv", [([64], [15936]), ([256], [4096]), ([33, 64], [9000, 3000]), ([512], [8192]), ([1500], [7600])])
 def test_plan_of_other_layers_is_in_equal_chunks(q, kv):
     """Layers with a window, soft-capping or ALiBi: chunks where the items are too few, none where they fill the chip."""
