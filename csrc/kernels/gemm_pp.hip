@@ -36,7 +36,7 @@ typedef __attribute__((address_space(3))) void pp_lds_t;
 namespace {
 
 constexpr int PP_NT = 512, PP_IMG = 256 * 128, PP_BUF = 2 * PP_IMG;
-enum { PP_BF16 = 0, PP_RES = 1, PP_SILU = 2 };
+enum { PP_BF16 = 0, PP_RES = 1, PP_SILU = 2, PP_PARTS = 3 };
 
 __device__ __forceinline__ int pp_swz(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
 
@@ -306,13 +306,14 @@ template <int EPI, bool BIAS>
 __global__ __launch_bounds__(PP_NT, 1) void moe_pp_kernel(const bf16* __restrict__ X, int64_t ldx,
                                                           const bf16* __restrict__ W, const bf16* __restrict__ bias,
                                                           bf16* __restrict__ out, int64_t ldo, int N, int K, int gm,
-                                                          PpGroups grp) {
+                                                          PpGroups grp, int splits, int rows_all) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = wave >> 2, wi = wave & 3;
   const int fr = lane & 15, fc = lane >> 4;
-  const int tiles_n = (N + 255) >> 8, kt = K >> 6, half = N >> 1;
+  const int tiles_n = (N + 255) >> 8, half = N >> 1;
+  if constexpr (EPI != PP_PARTS) splits = 1;
 
   // ---- this workgroup's tile: lane l holds the row tiles of experts l * per .. + per - 1
   const int per = (grp.E + 63) >> 6;
@@ -327,10 +328,13 @@ __global__ __launch_bounds__(PP_NT, 1) void moe_pp_kernel(const bf16* __restrict
     const int v = __shfl_up(incl, d);
     if (lane >= d) incl += v;
   }
-  const int T = __builtin_amdgcn_readlane(incl, 63) * tiles_n;
-  const int b = blockIdx.x, xcd = b & 7, q8 = T >> 3, r8 = T & 7;
-  if (b >= T) return;   // whole workgroup, before any barrier
-  const int id = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (b >> 3);
+  const int T = __builtin_amdgcn_readlane(incl, 63) * tiles_n, all = T * splits;
+  const int b = blockIdx.x, xcd = b & 7, q8 = all >> 3, r8 = all & 7;
+  if (b >= all) return;   // whole workgroup, before any barrier
+  int id = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (b >> 3);
+  const int part = EPI == PP_PARTS ? id / T : 0;   // (a piece of K of all tiles, then the next)
+  id -= part * T;
+  const int k0 = (K >> 6) * part / splits, kt = (K >> 6) * (part + 1) / splits - k0;   // 64s of K
   const int at = __popcll(__ballot(incl * tiles_n <= id));   // the lane whose experts it belongs to
   int e = at * per, before = at ? __builtin_amdgcn_readlane(incl, at - 1) : 0, mt = 0;
   for (;; ++e) {   // (ends: some expert of that lane has the tile)
@@ -375,7 +379,7 @@ __global__ __launch_bounds__(PP_NT, 1) void moe_pp_kernel(const bf16* __restrict
   auto dma = [&](int t, int buf, int p0, int np) {
     char* base = smem + buf * PP_BUF + img_off;
 #pragma unroll
-    for (int p = p0; p < p0 + np; ++p) pp_dma(rs, base + prow[p] * 128, vo[p], (uint32_t)t * 128);
+    for (int p = p0; p < p0 + np; ++p) pp_dma(rs, base + prow[p] * 128, vo[p], (uint32_t)(k0 + t) * 128);
   };
 
   f32x4 acc[8][4];
@@ -477,6 +481,13 @@ __global__ __launch_bounds__(PP_NT, 1) void moe_pp_kernel(const bf16* __restrict
 #pragma unroll
           for (int r = 0; r < 4; ++r) v[r] = (bf16)(pp_silu(acc[i][j][r]) * acc[i + 1][j][r]);
           *reinterpret_cast<bf16x4*>(out + (int64_t)m * ldo + n) = v;
+        }
+      } else if constexpr (EPI == PP_PARTS) {
+        float* to = reinterpret_cast<float*>(out) + ((int64_t)part * rows_all + m) * ldo;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int n = n0 + g * 128 + i * 16 + 4 * fc;
+          if (n < N) *reinterpret_cast<f32x4*>(to + n) = acc[i][j];
         }
       } else {
 #pragma unroll
@@ -688,12 +699,12 @@ int launch_pp(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, const bf16
 
 template <int EPI, bool BIAS>
 int launch_moe_pp(const bf16* X, int64_t ldx, const bf16* W, const bf16* bias, bf16* out, int64_t ldo, int N, int K,
-                  int row_tiles, const PpGroups& grp, hipStream_t stream) {
+                  int row_tiles, const PpGroups& grp, int splits, int rows, hipStream_t stream) {
   constexpr int LDS = 2 * PP_BUF;
   static const hipError_t attr =   // (once, whichever thread comes first)
       hipFuncSetAttribute((const void*)moe_pp_kernel<EPI, BIAS>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   if (attr != hipSuccess) return (int)attr;
-  moe_pp_kernel<EPI, BIAS><<<row_tiles * ((N + 255) / 256), PP_NT, LDS, stream>>>(X, ldx, W, bias, out, ldo, N, K, pp_gm(), grp);
+  moe_pp_kernel<EPI, BIAS><<<row_tiles * ((N + 255) / 256) * splits, PP_NT, LDS, stream>>>(X, ldx, W, bias, out, ldo, N, K, pp_gm(), grp, splits, rows);
   return (int)hipGetLastError();
 }
 
@@ -748,21 +759,23 @@ OME_API int ome_gemm_pp(const void* X, int64_t ldx, const void* W, int64_t ldw, 
 
 // Grouped GEMM over rows sorted by expert (ome_moe_align): out[p] = X[row(p)] . W[e(p)]^T (+ bias[e(p)]), row(p) =
 // sorted_ids[p] / div, or p where sorted_ids is null.  W [E][N][K]; epi 0: out [rows][N]; epi 2: SiLU of columns
-// [0, N / 2) times columns [N / 2, N), out [rows][N / 2].  x_rows: rows of X (32-bit DMA offsets).  -3: operands that the
-// kernel does not take (nothing is launched).
+// [0, N / 2) times columns [N / 2, N), out [rows][N / 2]; epi 3: K in `splits` pieces, out fp32 [splits][rows][N], which ome_moe_combine_parts adds.
+// x_rows: rows of X (32-bit DMA offsets).  -3: operands that the kernel does not take (nothing is launched).
 OME_API int ome_moe_gemm_pp(const void* X, int64_t ldx, int x_rows, const int* sorted_ids, int div, const void* W,
                             const int* offsets, int E, int N, int K, int rows, void* out, int64_t ldo, const void* bias,
-                            int epi, hipStream_t stream) {
+                            int epi, int splits, hipStream_t stream) {
   if (rows <= 0) return 0;
   if (E <= 0 || N <= 0 || K <= 0 || K % 64 || N % (epi == PP_SILU ? 32 : 4) || (sorted_ids && div <= 0)) return -3;
-  if ((epi != PP_BF16 && epi != PP_SILU) || (epi == PP_SILU && bias)) return -3;
+  if ((epi != PP_BF16 && epi != PP_SILU && epi != PP_PARTS) || (epi != PP_BF16 && bias)) return -3;
+  if (epi == PP_PARTS ? splits < 1 || splits > K / 64 || ldo % 4 || (uintptr_t)out % 16 : splits != 1) return -3;
   if (ldx % 8 || ((uintptr_t)X | (uintptr_t)W) % 16 || ldo % 4 || (uintptr_t)out % 8) return -3;
   if ((int64_t)x_rows * ldx * 2 >= 0x7fffffffLL || (int64_t)N * K * 2 >= 0x7fffffffLL) return -3;
   const int64_t tiles = (rows + 255) / 256 + (E < rows ? E : rows);
-  if (tiles * ((N + 255) / 256) > 0x7fffffffLL) return -3;
+  if (tiles * ((N + 255) / 256) * splits > 0x7fffffffLL) return -3;
   const PpGroups grp{sorted_ids, offsets, sorted_ids ? div : 1, E};
   const bf16 *x = (const bf16*)X, *w = (const bf16*)W, *b = (const bf16*)bias;
-  if (epi == PP_SILU) return launch_moe_pp<PP_SILU, false>(x, ldx, w, b, (bf16*)out, ldo, N, K, (int)tiles, grp, stream);
-  return b ? launch_moe_pp<PP_BF16, true>(x, ldx, w, b, (bf16*)out, ldo, N, K, (int)tiles, grp, stream)
-           : launch_moe_pp<PP_BF16, false>(x, ldx, w, b, (bf16*)out, ldo, N, K, (int)tiles, grp, stream);
+  if (epi == PP_SILU) return launch_moe_pp<PP_SILU, false>(x, ldx, w, b, (bf16*)out, ldo, N, K, (int)tiles, grp, 1, rows, stream);
+  if (epi == PP_PARTS) return launch_moe_pp<PP_PARTS, false>(x, ldx, w, b, (bf16*)out, ldo, N, K, (int)tiles, grp, splits, rows, stream);
+  return b ? launch_moe_pp<PP_BF16, true>(x, ldx, w, b, (bf16*)out, ldo, N, K, (int)tiles, grp, 1, rows, stream)
+           : launch_moe_pp<PP_BF16, false>(x, ldx, w, b, (bf16*)out, ldo, N, K, (int)tiles, grp, 1, rows, stream);
 }

@@ -707,9 +707,12 @@ OME_API int ome_moe_gemm(const void* A, int64_t lda, const int* sorted_ids, int 
 // A thread has eight columns of a token.  The experts' rows come up to eight at a time, added in their order: one after the other, each behind its
 // place and weight, a row took a round trip to memory, and a workgroup took all of a token's
 // columns.  us, 8 rows a token of 7168: 700 tokens 27.8 -> 18.0 (90 MB at 5.0 TB/s), 8 tokens 18.6 -> 4.8; 10 rows of 2048, 48 tokens 7.3 -> 4.8.
-__global__ __launch_bounds__(256) void moe_combine_kernel(const bf16* __restrict__ Y, const float* __restrict__ w,
+// PARTS: the rows as `splits` fp32 pieces `stride` floats apart, which are added first.
+template <bool PARTS>
+__global__ __launch_bounds__(256) void moe_combine_kernel(const void* __restrict__ Yv, const float* __restrict__ w,
                                                           const int* __restrict__ inv, int k, int H,
-                                                          bf16* out, const bf16* add, float scale) {
+                                                          bf16* out, const bf16* add, float scale, int splits, int64_t stride) {
+  const bf16* const Y = (const bf16*)Yv;
   const int64_t t = blockIdx.x;
   const int c = blockIdx.y * 256 + threadIdx.x;
   if (c >= H / 8) return;
@@ -719,6 +722,20 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const bf16* __restrict
   int j = 0;
   const auto take = [&](auto count) {
     constexpr int N = decltype(count)::value;
+    if constexpr (PARTS) {
+      float wj[N], f[N][8];
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        wj[i] = w[t * k + j + i];
+        sum_parts8((const float*)Yv + (int64_t)inv[t * k + j + i] * H + c * 8, stride, splits, f[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) acc[q] += wj[i] * f[i][q];
+      j += N;
+      return;
+    }
     bf16x8 y[N];
     float wj[N];
 #pragma unroll
@@ -751,7 +768,17 @@ OME_API int ome_moe_combine_add(const void* Y, const float* w, const int* inv, i
                                 const void* add, float scale, hipStream_t stream) {
   if (n_tok <= 0) return 0;
   if (H % 8) return -2;
-  moe_combine_kernel<<<dim3(n_tok, (H / 8 + 255) / 256), 256, 0, stream>>>((const bf16*)Y, w, inv, k, H, (bf16*)out, (const bf16*)add, scale);
+  moe_combine_kernel<false><<<dim3(n_tok, (H / 8 + 255) / 256), 256, 0, stream>>>(Y, w, inv, k, H, (bf16*)out, (const bf16*)add, scale, 1, 0);
+  OME_CHECK_LAUNCH();
+  return 0;
+}
+
+// ... of rows that ome_moe_gemm_pp left in `splits` fp32 pieces [splits][rows][H]
+OME_API int ome_moe_combine_parts(const float* Y, const float* w, const int* inv, int n_tok, int k, int H, void* out,
+                                  const void* add, float scale, int splits, int64_t rows, hipStream_t stream) {
+  if (n_tok <= 0) return 0;
+  if (H % 8 || splits < 1) return -2;
+  moe_combine_kernel<true><<<dim3(n_tok, (H / 8 + 255) / 256), 256, 0, stream>>>(Y, w, inv, k, H, (bf16*)out, (const bf16*)add, scale, splits, rows * H);
   OME_CHECK_LAUNCH();
   return 0;
 }

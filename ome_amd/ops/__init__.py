@@ -806,18 +806,31 @@ class _Sorted:
             call("ome_moe_align", ids.data_ptr(), n, E, self.offsets, self.ids, self.ids + 4 * n, stream_ptr())
 
 
+@functools.lru_cache(maxsize=4096)
+def moe_splits(rows: int, E: int, N: int, K: int) -> int:
+    """Pieces of a down projection's K on 256-row tiles: 2 where its tiles are half a round over the CUs or little more than a
+    whole one, and K is long beside the fp32 pieces that are written and read.  Of experts of different sizes each has half a tile
+    more than its share of the rows.  Whole layer of Mixtral (8 experts, 4096 x 14336), us, rounds: one piece -> two: 184 tokens (0.50) 658 -> 561, 300 (0.50) 705 ->
+    594, 600 (0.54) 764 -> 663, 1800 (1.13) 1446 -> 1341, 2200 (1.32) 1644 -> 1550, 2600 (1.52) 1796 -> 1729; not for 800 (0.64) 812 -> 815, 1000 (0.74) 960 ->
+    952, 1200 (0.84) 991 -> 1002, 1500 (0.98) 1104 -> 1119, 3000 (1.71) 1991 -> 2013.  Three or four are a little ahead of two only at 800 and 1000.
+    Nemotron-3-Nano (128 experts, 2688 x 1856) 1000 tokens 556 -> 606."""
+    rounds = max(1.0, rows / E / 256 + 0.5) * E * -(-N // 256) / 256
+    return 2 if K >= 4096 and (rounds <= 0.55 or 1 < rounds <= 1.55) else 1
+
+
 def _moe_pp(x: torch.Tensor, ids: int | None, div: int, w: torch.Tensor, offsets: int, rows: int,
-            bias: torch.Tensor | None, silu: bool) -> torch.Tensor | None:
-    """Grouped GEMM on 256-row tiles (``ome_moe_gemm_pp``; ``silu``: SiLU(gate) * up applied to the accumulators),
+            bias: torch.Tensor | None, silu: bool, splits: int = 1) -> torch.Tensor | None:
+    """Grouped GEMM on 256-row tiles (``ome_moe_gemm_pp``; ``silu``: SiLU(gate) * up applied to the accumulators; ``splits``: K in
+    as many pieces, fp32 [splits, rows, N]),
     or None where the 64 / 128-row tiles run: experts with few rows, shapes the tiles do not take, ``OME_MOE_TILE``."""
     E, N, K = w.shape
     if rows < MOE_PP_ROWS * E or os.environ.get("OME_MOE_TILE") or K % 64 or N % (32 if silu else 4) or (silu and bias is not None) or \
             x.stride(0) % 8 or x.stride(1) != 1 or (x.data_ptr() | w.data_ptr()) % 16 or not w.is_contiguous() or \
             x.shape[0] * x.stride(0) >= 1 << 30 or N * K >= 1 << 30:
         return None
-    out = x.new_empty(rows, N // 2 if silu else N)
+    out = x.new_empty(rows, N // 2 if silu else N) if splits == 1 else x.new_empty(splits, rows, N, dtype=torch.float32)
     call("ome_moe_gemm_pp", x.data_ptr(), x.stride(0), x.shape[0], ids, div, w.data_ptr(), offsets, E, N, K,
-         rows, out.data_ptr(), out.stride(0), ptr(bias), 2 if silu else 0, stream_ptr())
+         rows, out.data_ptr(), out.stride(-2), ptr(bias), 3 if splits > 1 else 2 if silu else 0, splits, stream_ptr())
     return out
 
 
@@ -862,7 +875,7 @@ def fused_moe(x: torch.Tensor, topk_w: torch.Tensor, topk_ids: torch.Tensor, w13
         h = _moe_gemm(x, s, s.ids, k, w13, n, b13)
     if not fused:
         h = act_and_mul(h, act, limit=limit) if gated else _act_inplace(h, act)
-    y = _moe_pp(h, None, 1, w2, s.offsets, n, b2, False)
+    y = _moe_pp(h, None, 1, w2, s.offsets, n, b2, False, moe_splits(n, E, H, I) if b2 is None else 1)
     if y is None:
         y = _moe_gemm(h, s, None, 0, w2, n, b2)
     return _combine(y, topk_w, s.inv, T, k, H, scale, add)
@@ -889,7 +902,12 @@ def _moe_gemm(x: torch.Tensor, s: _Sorted, ids: int | None, div: int, w: torch.T
 
 def _combine(y, topk_w, inv, T, k, H, scale, add):
     if add is not None:
-        assert add.shape == (T, H) and add.is_contiguous() and add.dtype == y.dtype
+        assert add.shape == (T, H) and add.is_contiguous() and add.dtype == (torch.bfloat16 if y.dim() == 3 else y.dtype)
+    if y.dim() == 3:   # pieces of the down projection's K
+        out = add if add is not None else y.new_empty(T, H, dtype=torch.bfloat16)
+        call("ome_moe_combine_parts", y.data_ptr(), topk_w.data_ptr(), inv.data_ptr(), T, k, H, out.data_ptr(), ptr(add),
+             float(scale), y.shape[0], y.shape[1], stream_ptr())
+        return out
     out = add if add is not None else y.new_empty(T, H)
     call("ome_moe_combine_add", y.data_ptr(), topk_w.data_ptr(), inv.data_ptr(), T, k, H, out.data_ptr(), ptr(add),
          float(scale), stream_ptr())

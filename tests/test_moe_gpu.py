@@ -98,6 +98,31 @@ def test_moe_prompt_tile_quarters(monkeypatch, rows):
         test_moe_prompt_tiles(monkeypatch, [rows, 256 + rows, 0, 3], H, I, "silu")
 
 
+@pytest.mark.parametrize("counts", [[1, 0, 255, 257, 0, 512, 3], [40] * 70], ids=lambda c: f"{len(c)}x{max(c)}")
+@pytest.mark.parametrize("H,I", [(256, 128), (192, 192), (128, 1856)])
+@pytest.mark.parametrize("splits", [2, 3])
+def test_moe_down_projection_in_pieces(monkeypatch, counts, H, I, splits):
+    """Pieces of one K step, of unlike length, of many; the shared expert's rows on top."""
+    splits = min(splits, I // 64)
+    monkeypatch.setattr(ops, "moe_splits", lambda *a: splits)
+    for kind in ("silu", "relu2"):
+        test_moe_prompt_tiles(monkeypatch, counts, H, I, kind)
+    torch.manual_seed(I)
+    bf = lambda *s: torch.randn(*s, device=DEV).to(torch.bfloat16)  # noqa: E731
+    x, w13, w2, add = bf(300, H), bf(4, 2 * I, H) * 0.1, bf(4, H, I) * 0.1, bf(300, H)
+    tw, ids = torch.rand(300, 2, device=DEV), torch.rand(300, 4, device=DEV).topk(2).indices.int()
+    got = ops.fused_moe(x, tw, ids, w13, w2, 0, 2.5, add=add.clone()).double()
+    monkeypatch.setattr(ops, "moe_splits", lambda *a: 1)
+    # without pieces each expert's row is rounded to bf16 before they are added, and the output either way
+    plain = ops.fused_moe(x, tw, ids, w13, w2, 0, 2.5, add=add.clone()).double()
+    assert ((got - plain).norm() / plain.norm()).item() < 2.0 ** -8
+
+
+@pytest.mark.parametrize("tokens,splits", [(184, 2), (600, 2), (800, 1), (1500, 1), (1800, 2), (2600, 2), (3000, 1)])
+def test_moe_pieces_where_they_are_faster(tokens, splits):
+    assert ops.moe_splits(2 * tokens, 8, 4096, 14336) == splits
+
+
 @pytest.mark.parametrize("E,k", [(1, 1), (64, 64), (65, 3), (200, 70), (512, 10)])
 def test_moe_route_picks_in_order(E, k):
     """Ties go to the lower expert, zeros of both signs are ties, minus infinity comes last, NaN never (an expert
