@@ -22,13 +22,13 @@
 // the rest, so a chunk is 2000 cycles of issue and some 1400 of LDS latency and dependencies.  Hence the
 // next chunk moves to LDS by DMA, without a register or a store on the way, and where a workgroup has its CU to itself by two waves of their own: a
 // move holds its wave up for some 50 cycles, and the nine of a wave that also computes took a quarter of its time (scan of a delta rule, 192
-// workgroups 91 -> 73 us, 64 61 -> 49; selective scan, 256 54 -> 43, 128 40 -> 32; moves by one or by four such waves 73 and 77 for the first).  With two
+// workgroups 91 -> 73 us, now 70, 64 61 -> 49, now 47; selective scan, 256 54 -> 43, 128 40 -> 32; moves by one or by four such waves 73 and 77 for the first).  With two
 // workgroups a CU each covers the other's moves, and such waves only take slots from them (448 workgroups 36.7 -> 37.8, 512 76 -> 81): none there.  Values and outputs move in pieces of four columns
 // (q S is formed transposed for that); T and P T are products of three bf16 parts each, at half the fp32 product's time.
 // Memory traffic hides behind that.  Two fp16 parts instead of three bf16 ones would take a quarter less time, but the state came out
 // 2.3 times further from 64 bits: an fp16 value below 2^-14 has no lower part.
 // (chunks' matrices + scan, calls that are waited for one by one):
-//   gated delta rule, 32 heads of 128 x 128, prompts of 1001 / 1435 / 1564 rows:   22 + 75 us (before: 24 + 123; row by row: 1098)
+//   gated delta rule, 32 heads of 128 x 128, prompts of 1001 / 1435 / 1564 rows:   20 + 70 us (before: 24 + 123; row by row: 1098)
 //   selective scan, 128 heads of 64 x 128, 8 groups, 1033 / 926 / 1248 / 293 rows:  10 + 85 us (values scaled by dt in three parts: 10 + 93; before: 11 + 116;
 //   row by row: 1745)
 // Largest error of the state against 64 bits: 1.2e-7 (row by row: 2.0e-7) and 1.2e-7 (6.2e-7) of its norm.
@@ -935,6 +935,7 @@ __global__ __launch_bounds__(64 * (NW + MW), 2) void chunk_rule_kernel(RuleArgs 
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) u[rb] = (DELTA ? u[rb] : r[rb]) * vd[rb];
     split3(u[0], u[1], us);
+    if constexpr (DELTA && SEG == 0) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int p = 2; p >= 0; --p)
 #pragma unroll
@@ -956,6 +957,14 @@ __global__ __launch_bounds__(64 * (NW + MW), 2) void chunk_rule_kernel(RuleArgs 
         for (int t = 0; t < 4; ++t) o[rb][t] += Dh * (float)y[rb][t];
     }
     put(b ^ 1);
+    if constexpr (DELTA && SEG == 0) {
+#pragma unroll
+      for (int i = 0; i < 3 * NB; ++i) {   // the outputs' vector instructions beside S's products (a chunk alone on its CU 1.48 -> 1.42 us; segments 0.5%, Mamba-2 1 to 3% slower so)
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 3, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
     if constexpr (MW == 0) {
       __builtin_amdgcn_sched_barrier(0);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the next chunk has landed (before the stores below, which nobody waits for)
