@@ -22,14 +22,14 @@
 // the rest, so a chunk is 2000 cycles of issue and some 1400 of LDS latency and dependencies.  Hence the
 // next chunk moves to LDS by DMA, without a register or a store on the way, and where a workgroup has its CU to itself by two waves of their own: a
 // move holds its wave up for some 50 cycles, and the nine of a wave that also computes took a quarter of its time (scan of a delta rule, 192
-// workgroups 91 -> 73 us, now 70, 64 61 -> 49, now 47; selective scan, 256 54 -> 43, 128 40 -> 32; moves by one or by four such waves 73 and 77 for the first).  With two
+// workgroups 91 -> 73 us, now 70, 64 61 -> 49, now 47; selective scan, 256 54 -> 43, now 42, 128 40 -> 32, now 31; moves by one or by four such waves 73 and 77 for the first).  With two
 // workgroups a CU each covers the other's moves, and such waves only take slots from them (448 workgroups 36.7 -> 37.8, 512 76 -> 81): none there.  Values and outputs move in pieces of four columns
 // (q S is formed transposed for that); T and P T are products of three bf16 parts each, at half the fp32 product's time.
 // Memory traffic hides behind that.  Two fp16 parts instead of three bf16 ones would take a quarter less time, but the state came out
 // 2.3 times further from 64 bits: an fp16 value below 2^-14 has no lower part.
 // (chunks' matrices + scan, calls that are waited for one by one):
 //   gated delta rule, 32 heads of 128 x 128, prompts of 1001 / 1435 / 1564 rows:   20 + 70 us (before: 24 + 123; row by row: 1098)
-//   selective scan, 128 heads of 64 x 128, 8 groups, 1033 / 926 / 1248 / 293 rows:  10 + 85 us (values scaled by dt in three parts: 10 + 93; before: 11 + 116;
+//   selective scan, 128 heads of 64 x 128, 8 groups, 1033 / 926 / 1248 / 293 rows:  9 + 74 us (values scaled by dt in three parts: 10 + 93; before: 11 + 116;
 //   row by row: 1745)
 // Largest error of the state against 64 bits: 1.2e-7 (row by row: 2.0e-7) and 1.2e-7 (6.2e-7) of its norm.
 //
@@ -56,12 +56,12 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // Workspace of one chunk, in bytes: (Mamba-2) of every group q k^T in fp32, which its heads share (they differ in their decays only,
 // which the scan applies: P itself would be 16 times the bytes); of every head (DELTA) the images of T and P T, each in three
-// bf16 parts, as LDS holds them, and its vectors, 32 floats each: DELTA a, b, c, d of the scan, then g_C;  Mamba-2 dt, cum's upper and
-// lower parts, c, d, then g_C.
+// bf16 parts, as LDS holds them, and its vectors, 32 floats each: DELTA a, b, c, d of the scan, then g_C;  Mamba-2 dt, pairs of cum's upper and
+// lower part (of two to the power), c, d, P's diagonal, then g_C.
 constexpr int MAT = RC * RC * 2;      // a part of a 32 x 32 matrix
 constexpr int VECS = 1024;            // the vectors, in whole LDS moves
 template <bool DELTA>
-constexpr int vec_floats() { return (DELTA ? 4 : 5) * RC + 4; }
+constexpr int vec_floats() { return (DELTA ? 4 : 6) * RC + 4; }
 template <bool DELTA>
 __host__ __device__ constexpr int64_t group_bytes() { return DELTA ? 0 : 4 * RC * RC; }
 template <bool DELTA>
@@ -189,17 +189,15 @@ __device__ __forceinline__ void split3(f32x4 x0, f32x4 x1, bf16x8 (&p)[3]) {
   }
 }
 
-// Four, by cutting the lower bits off: half as many instructions again, but a dot product waits for the products around it (20 cycles each way).
+// Two, by cutting the lower bits off: half as many instructions again, but a dot product waits for the products around it (20 cycles each way).
 // For a wave that has little else to do beside its products (Mamba-2's P: 2% of the scan; S and U so: 1 to 2% more).
-__device__ __forceinline__ void cut3(f32x4 x, bf16x4 (&p)[3]) {
+__device__ __forceinline__ void cut3(float a, float b, uint32_t (&p)[3]) {
 #pragma unroll
   for (int t = 0; t < 3; ++t) {
-    uint32_t u[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) u[e] = __float_as_uint(x[e]);
-    p[t] = __builtin_bit_cast(bf16x4, u32x2{__builtin_amdgcn_perm(u[1], u[0], 0x07060302u), __builtin_amdgcn_perm(u[3], u[2], 0x07060302u)});
-#pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] -= __uint_as_float(u[e] & 0xffff0000u);
+    const uint32_t u = __float_as_uint(a), v = __float_as_uint(b);
+    p[t] = __builtin_amdgcn_perm(v, u, 0x07060302u);
+    a -= __uint_as_float(u & 0xffff0000u);
+    b -= __uint_as_float(v & 0xffff0000u);
   }
 }
 
@@ -431,6 +429,7 @@ __global__ __launch_bounds__(256) void ssm_gram_kernel(RuleArgs a) {
   set_turns(a);
   if (!chunk_of(blockIdx.x, a.cu, a.S, r0, n)) return;   // the same in every wave
   char* ws = a.ws + blockIdx.x * ws_bytes<false>(a.H, a.Hk);
+  __shared__ float s_diag[RC];
   if (w == 0) {
     bf16x8 kf[2][NS], qf[2][NS];
 #pragma unroll
@@ -451,7 +450,10 @@ __global__ __launch_bounds__(256) void ssm_gram_kernel(RuleArgs a) {
 #pragma unroll
         for (int s = 0; s < NS; ++s) qk = mma_bf16(qf[rb][s], kf[cb][s], qk);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) gram[(16 * rb + 4 * g + e) * RC + 16 * cb + col] = qk[e];
+        for (int e = 0; e < 4; ++e) {
+          gram[(16 * rb + 4 * g + e) * RC + 16 * cb + col] = qk[e];
+          if (cb == rb && 4 * g + e == col) s_diag[16 * rb + col] = qk[e];
+        }
       }
   }
   const int row = lane & 31, rv = r0 + min(row, n - 1), per = a.H / a.Hk;
@@ -466,16 +468,18 @@ __global__ __launch_bounds__(256) void ssm_gram_kernel(RuleArgs a) {
       if (row >= o) cum += up;
     }
     const double total = __shfl(cum, 31, 32);   // rows past the chunk's end add nothing
+    float* vec = reinterpret_cast<float*>(ws + a.Hk * group_bytes<false>() + h * head_bytes<false>());
     if (i < per) {
-      float* vec = reinterpret_cast<float*>(ws + a.Hk * group_bytes<false>() + h * head_bytes<false>());
-      const float hi = (float)cum;
+      const double two = cum * 1.4426950408889634;
+      const float hi = (float)two;
       vec[row] = ok ? dt : 0.f;
-      vec[RC + row] = hi;
-      vec[2 * RC + row] = (float)(cum - (double)hi);
-      vec[3 * RC + row] = ok ? __expf(hi) : 0.f;
+      *reinterpret_cast<float2*>(vec + RC + 2 * row) = float2{hi, (float)(two - (double)hi)};
+      vec[3 * RC + row] = ok ? __expf((float)cum) : 0.f;
       vec[4 * RC + row] = ok ? dt * __expf((float)(total - cum)) : 0.f;
-      if (row == 0) vec[5 * RC] = __expf((float)total);
+      if (row == 0) vec[6 * RC] = __expf((float)total);
     }
+    if (i0 == 0) __syncthreads();   // (s_diag)
+    if (i < per) vec[5 * RC + row] = ok ? dt * s_diag[row] : 0.f;
   }
 }
 
@@ -496,8 +500,7 @@ __global__ __launch_bounds__(256) void ssm_gram_kernel(RuleArgs a) {
 template <int DK, bool DELTA, int NW, bool VEC, int SEG, int MW>
 __global__ __launch_bounds__(64 * (NW + MW), 2) void chunk_rule_kernel(RuleArgs a) {
   constexpr int NS = DK / 32, NB = DK / 16, NT = 64 * NW, COLS = 16 * NW;
-  constexpr int NML = RC * RC / 4 / NT;                  // 16-byte loads of q k^T per thread (Mamba-2)
-  static_assert(NML * NT * 4 == RC * RC && RC * COLS == 8 * NT, "whole loads");
+  static_assert(RC * COLS == 8 * NT && RC * RC / 4 == NT, "whole loads; a pair below P's diagonal a thread");
   // a chunk in LDS: k and q rows, T and P T (Mamba-2: P) in three parts each, the vectors, the values
   constexpr int ROWS = RC * DK * 2, M_AT = 2 * ROWS, V_AT = M_AT + (DELTA ? 6 : 3) * MAT, X_AT = V_AT + VECS, IMG = X_AT + RC * COLS * 2;
   __shared__ __attribute__((aligned(1024))) char lds[2 * IMG];
@@ -605,8 +608,16 @@ __global__ __launch_bounds__(64 * (NW + MW), 2) void chunk_rule_kernel(RuleArgs 
 
   // What goes through registers comes a chunk ahead of the products: q k^T and its decays (Mamba-2), values by element.  Without a next chunk
   // it is the last one again (no branch, which would part the stages).
-  f32x4 rp[NML], rhj, rlj, rdj;
-  float rhi[NML], rli[NML];
+  // Mamba-2: a thread forms two neighbours of P below its diagonal, which itself joins D.  (Four of all 1024 values, of which half are zero: twice the vector
+  // instructions, some 60 of a chunk's 430; scan of 128 workgroups 32.0 -> 30.6 us, 256 42.8 -> 41.6, 512 76.7 -> 75.2.)  Rows 2 m - 1 and 2 m have m pairs each (row 31: 16), so 32 threads take the rows of m and of 16 - m.
+  int prow = 31, pcol = 2 * (tid % 16);
+  {
+    const int m = tid / 32 + 1, i = tid % 32, n = i < 2 * m ? m : 16 - m, k = i < 2 * m ? i : i - 2 * m;
+    if (m < 8 || i < 16) prow = 2 * n - 1 + (k >= n), pcol = 2 * (k >= n ? k - n : k);
+  }
+  f32x2 rp, rdj;
+  f32x4 rcj;
+  f32x2 rci;
   bf16x8 rx;
   const auto ahead = [&](int c) __attribute__((always_inline)) {   // of chunk c
     if constexpr (!VEC) {
@@ -616,34 +627,22 @@ __global__ __launch_bounds__(64 * (NW + MW), 2) void chunk_rule_kernel(RuleArgs 
       for (int e = 0; e < 8; ++e) rx[e] = x[e];
     }
     if constexpr (!DELTA && SEG != 1) {
-      const uint32_t hj = 4 * (RC + 4 * (tid % (RC / 4)));
-      rhj = *reinterpret_cast<const f32x4*>(hp + hj);
-      rlj = *reinterpret_cast<const f32x4*>(hp + (hj + 4 * RC));
-      rdj = *reinterpret_cast<const f32x4*>(hp + (hj - 4 * RC));
-#pragma unroll
-      for (int i = 0; i < NML; ++i) {
-        const uint32_t e = tid + NT * i, hi = 4 * (RC + e / (RC / 4));
-        rp[i] = *reinterpret_cast<const f32x4*>(gp + 16 * e);
-        rhi[i] = *reinterpret_cast<const float*>(hp + hi);
-        rli[i] = *reinterpret_cast<const float*>(hp + (hi + 4 * RC));
-      }
+      rp = *reinterpret_cast<const f32x2*>(gp + (uint32_t)(4 * (prow * RC + pcol)));
+      rdj = *reinterpret_cast<const f32x2*>(hp + (uint32_t)(4 * pcol));
+      rcj = *reinterpret_cast<const f32x4*>(hp + (uint32_t)(4 * (RC + 2 * pcol)));
+      rci = *reinterpret_cast<const f32x2*>(hp + (uint32_t)(4 * (RC + 2 * prow)));
     }
   };
-  const auto put = [&](int b) __attribute__((always_inline)) {   // P_ij dt_j = q_i.k_j exp(cum_i - cum_j) dt_j, j <= i; cum in two parts (long sums, short differences)
+  const auto pair_at = [](int row, int c) { return mat_img(row, (c & 15) >> 2) + 8 * (c >> 4) + 2 * (c & 3); };
+  const auto put = [&](int b) __attribute__((always_inline)) {   // P_ij dt_j = q_i.k_j exp(cum_i - cum_j) dt_j, j < i; cum in two parts (long sums, short differences)
     if constexpr (!VEC) *reinterpret_cast<bf16x8*>(lds + b * IMG + X_AT + 16 * tid) = rx;
     if constexpr (!DELTA && SEG != 1) {
+      const float x0 = rp[0] * __builtin_amdgcn_exp2f((rci[0] - rcj[0]) + (rci[1] - rcj[1])) * rdj[0];
+      const float x1 = rp[1] * __builtin_amdgcn_exp2f((rci[0] - rcj[2]) + (rci[1] - rcj[3])) * rdj[1];
+      uint32_t p[3];
+      cut3(x0, pcol + 1 < prow ? x1 : 0.f, p);
 #pragma unroll
-      for (int i = 0; i < NML; ++i) {
-        const int e = tid + NT * i, row = e / (RC / 4), jj = 4 * (e % (RC / 4));
-        f32x4 x;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) x[t] = jj + t <= row ? rp[i][t] * __expf((rhi[i] - rhj[t]) + (rli[i] - rlj[t])) * rdj[t] : 0.f;
-        bf16x4 p[3];
-        cut3(x, p);
-        const int at = b * IMG + M_AT + mat_img(row, (jj & 15) >> 2) + 8 * (jj >> 4);
-#pragma unroll
-        for (int m = 0; m < 3; ++m) *reinterpret_cast<bf16x4*>(lds + at + m * MAT) = p[m];
-      }
+      for (int m = 0; m < 3; ++m) *reinterpret_cast<uint32_t*>(lds + b * IMG + M_AT + m * MAT + pair_at(prow, pcol)) = p[m];
     }
   };
 
@@ -805,6 +804,10 @@ __global__ __launch_bounds__(64 * (NW + MW), 2) void chunk_rule_kernel(RuleArgs 
     }
     ahead(0);
     advance(chunks > 1);
+    if constexpr (!DELTA && SEG != 1) {   // the rest of P, of which every thread has as much (a row and a column from the other end): zero
+#pragma unroll
+      for (int m = 0; m < 6; ++m) *reinterpret_cast<uint32_t*>(lds + m / 3 * IMG + M_AT + m % 3 * MAT + pair_at(31 - prow, 30 - pcol)) = 0;
+    }
     put(0);
     if constexpr (MW == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -823,7 +826,7 @@ __global__ __launch_bounds__(64 * (NW + MW), 2) void chunk_rule_kernel(RuleArgs 
     bf16x4 x[2], y[2];
     f32x4 va[2], vb[2], vd[2];
     bf16x8 kf[2][NS], qf[2][NS];
-    const float gc = V[(DELTA ? 4 : 5) * RC];
+    const float gc = V[(DELTA ? 4 : 6) * RC];
 #pragma unroll
     for (int t = 0; t < NS; ++t)
 #pragma unroll
@@ -867,13 +870,14 @@ __global__ __launch_bounds__(64 * (NW + MW), 2) void chunk_rule_kernel(RuleArgs 
     __builtin_amdgcn_sched_barrier(0x0f);
     // ---- q S (transposed); R (DELTA) / U (Mamba-2) ----
     bf16x8 tm[2][3], pm[2][3];
-    float vo[2];
+    float vo[2], vp[2];
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) {
 #pragma unroll
       for (int p = 0; p < 3; ++p)
         if constexpr (DELTA || SEG != 1) tm[rb][p] = mat(p, rb);
       vo[rb] = V[(DELTA ? 2 : 3) * RC + 16 * rb + col];
+      if constexpr (!DELTA && SEG != 1) vp[rb] = V[5 * RC + 16 * rb + col];
       vd[rb] = vec(DELTA ? 3 : 4, rb);
     }
     __builtin_amdgcn_sched_barrier(0x0f);
@@ -935,7 +939,8 @@ __global__ __launch_bounds__(64 * (NW + MW), 2) void chunk_rule_kernel(RuleArgs 
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb) u[rb] = (DELTA ? u[rb] : r[rb]) * vd[rb];
     split3(u[0], u[1], us);
-    if constexpr (DELTA && SEG == 0) __builtin_amdgcn_sched_barrier(0);
+    constexpr bool BESIDE = SEG == 0 && (DELTA || MW == 0);   // the outputs' vector instructions beside S's products
+    if constexpr (BESIDE) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int p = 2; p >= 0; --p)
 #pragma unroll
@@ -954,14 +959,14 @@ __global__ __launch_bounds__(64 * (NW + MW), 2) void chunk_rule_kernel(RuleArgs 
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) o[rb][t] += Dh * (float)y[rb][t];
+        for (int t = 0; t < 4; ++t) o[rb][t] += (Dh + vp[rb]) * (float)y[rb][t];
     }
     put(b ^ 1);
-    if constexpr (DELTA && SEG == 0) {
+    if constexpr (BESIDE) {   // (a delta rule's chunk alone on its CU 1.48 -> 1.42 us, selective scan of 512 workgroups 75 -> 74; segments 0.5%, a selective scan with waves that move 4% slower so)
 #pragma unroll
-      for (int i = 0; i < 3 * NB; ++i) {   // the outputs' vector instructions beside S's products (a chunk alone on its CU 1.48 -> 1.42 us; segments 0.5%, Mamba-2 1 to 3% slower so)
+      for (int i = 0; i < 3 * NB; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x2, 3, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 2, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
     }

@@ -180,6 +180,27 @@ def test_selective_scan_prompts(lens, H, P, N, G, off):
     assert near(ops.ssm_scan(*args, st, *sq, H, P, N, G), st, *want)
 
 
+@pytest.mark.parametrize("rows", [5, 31, 32, 64])
+@pytest.mark.parametrize("N", [64, 128])
+def test_selective_scan_entry_by_entry(rows, N):
+    """Values that are 1 in a column of their own: the output is exp(cum_i - cum_j) dt_j q_i.k_j, each entry by itself, zero above the diagonal."""
+    torch.manual_seed(rows + N)
+    H, P = 2, 64
+    B, C = (torch.randn(rows, N, device=DEV).to(BF) for _ in range(2))
+    dt = torch.randn(rows, H, device=DEV).to(BF)
+    x = torch.eye(rows, P, device=DEV).to(BF).repeat(1, H)
+    A, D, dtb = torch.tensor([-0.02, -1.5], device=DEV), torch.zeros(H, device=DEV), torch.zeros(H, device=DEV)
+    state = torch.zeros(1, H, P, N, device=DEV)
+    out = ops.ssm_scan(x, dt, B, C, A, D, dtb, 0.0, state, i32([0, rows]), i32([0]), i32([1]), H, P, N, 1).view(rows, H, P).transpose(0, 1)
+    step = torch.nn.functional.softplus(dt.double().T)   # [H, rows]
+    cum = (step * A.double()[:, None]).cumsum(1)
+    want = torch.exp(cum[:, :, None] - cum[:, None, :]) * step[:, None, :] * (C.double() @ B.double().T)
+    want = torch.nn.functional.pad(want.tril(), (0, P - rows))
+    size = torch.nn.functional.pad(((C.double().abs() @ B.double().abs().T) * step[:, None, :]).tril(), (0, P - rows))
+    # rounded to bf16 once, of 8 bits: half a step is 2^-8 of a value at the most; fp32 sums of up to 128 products before it
+    assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -20 * size).all())
+
+
 @pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
 @pytest.mark.parametrize("what", ["q", "k", "v", "a", "b"])
 def test_delta_rule_stays_causal(what, bad):
