@@ -228,7 +228,7 @@ __global__ __launch_bounds__(256) void mla_attn_kernel(
 //   O^T [DV x 32] += V^T . P^T          (DV/32 x 2 MFMAs; V^T by hardware-transposed LDS reads, key order of S^T)
 // Nothing else runs on the SIMD meanwhile, so the loop is pipelined by hand.  A product takes 32 cycles of the matrix cores and 4 of issue, so up
 // to six vector instructions beside it cost next to nothing: the softmax of tile n stands between the products of S^T of tile n + 1 (the
-// exponentials of its last 16 keys between those of O^T), and the nine moves of tile n + 3 one by one beside the last products of O^T (four
+// exponentials of its last 16 keys between those of O^T), and of 128 rows the nine moves of tile n + 3 one by one beside the last products of O^T (four
 // images; nine in a row hold a wave up for some 450 cycles).  A branch beside each product, taken or not, costs 40 cycles, so the loop
 // has none there.  Of 128 rows, 256 workgroups of 100 tiles that share their keys, a tile took 2.65 us with moves and softmax ahead of the products and
 // takes 2.42; its products alone take 1.65, the rate at which the card runs out of power (1380 TFLOP/s): the rest is LDS reads at 128 bytes a
@@ -353,15 +353,22 @@ __device__ __forceinline__ void plain_row(const bf16* q, const bf16* cache, cons
   }
 }
 
+// Waves beside the NW that multiply which move the keys to LDS: one on each SIMD that has none.  A move holds its wave up for some 50 cycles, and the 36
+// of a tile by the one wave of 32 rows took as long as its products.  Whole calls, us, moved by the waves that multiply -> by others: 32 rows,
+// 16 heads, 24 x 3000 keys 40.5 -> 35.9, 32 x 8000 83 -> 70, 128 x 3000 145 -> 120; 64 rows, 64 heads, 48 x 3000 63.7 -> 60.4, 100 x 1500 74 -> 69.6;
+// 100 prompt rows of 16 heads over 2000 keys 40.8 -> 38.7.  (128 rows have a wave on every SIMD, each with all of its registers.)
+constexpr int row_movers(int NW) { return 4 - NW; }
+
 template <int DK, int DV, int NW, bool DECODE>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1))) void mla_attn_rows_kernel(
+__global__ __launch_bounds__(64 * (NW + row_movers(NW))) __attribute__((amdgpu_waves_per_eu(1, 1))) void mla_attn_rows_kernel(
     const bf16* __restrict__ q, int64_t q_stride_t, const bf16* __restrict__ cache,
     const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ tok_row,
     const int* __restrict__ kv_lens, int T, int H, int seqs, float scale_log2, int parts, int2* __restrict__ plan,
     bf16* __restrict__ out, int64_t out_stride_t, float* __restrict__ ws_o, float* __restrict__ ws_ml) {
   static_assert(DK == 576 && lds_chunks<DK>() == DK / 8, "LDS DMA image assumes unpadded 72-chunk rows");
-  constexpr int CH = DK / 8, NI = KT * CH / 64, NJ = NI / NW, NV = DV / 32, NS = DK / 16;
-  static_assert(NI % NW == 0, "whole DMA instructions per wave");
+  constexpr int MW = row_movers(NW), ML = MW ? MW : NW;   // ML waves move
+  constexpr int CH = DK / 8, NI = KT * CH / 64, NJ = NI / ML, NV = DV / 32, NS = DK / 16;
+  static_assert(NI % ML == 0 && (MW == 0 || NI / 2 % MW == 0), "whole DMA instructions per wave");
   constexpr int IMG = KT * CH * 16;   // bytes per key-tile image
   constexpr float LAZY = 8.f;
   constexpr int AHEAD = 4;            // LDS operands in flight: 4 x 32 cycles of matrix work cover a read
@@ -460,7 +467,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
     // The queries: a wave's 32 rows are one image, so they come as a tile of keys does, 1 KB a move, and out of LDS into registers.  (Straight into
     // registers a lane holds 16 bytes of its row at a time, 32 rows of two lanes: 128 rows 5.7 us on every CU at once, now 4.2; fewer rows are no slower so.)
     bf16x8 qf[NS];
-    const bool moved = NW == 4 && (((uintptr_t)q | (uintptr_t)(2 * q_stride_t)) & 15) == 0 && (uint64_t)q_stride_t < 1 << 26;   // (9 tokens a wave: 32-bit offsets)
+    const bool moved = MW == 0 && (((uintptr_t)q | (uintptr_t)(2 * q_stride_t)) & 15) == 0 && (uint64_t)q_stride_t < 1 << 26;   // (9 tokens a wave: 32-bit offsets)
     if (moved) {
       const int tw = __builtin_amdgcn_readfirstlane(t);
       const uint32_t at = 2 * ((uint32_t)(t - tw) * (uint32_t)q_stride_t + (uint32_t)head * DK);
@@ -472,7 +479,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
           buffer_to_lds(q + (int64_t)tw * q_stride_t, 0x7fffffffu, (uint32_t)__builtin_amdgcn_ds_bpermute(4 * (8 * a + r8), (int)at) + 16 * (x ^ (a & 1)), 0,
                         lds0 + wave * IMG + 1024 * (9 * a + b));
       }
-    } else {
+    } else if (wave < NW) {
       const bf16* qp = q + (int64_t)t * q_stride_t + (int64_t)head * DK + 8 * hf;
 #pragma unroll
       for (int s = 0; s < NS; ++s) qf[s] = ld8(qp + 16 * s);
@@ -486,10 +493,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
     // instruction reads one page: its descriptor is based at that page.
     // Nine instructions are 8 rows; those of the next 8 differ in the chunk's lowest bit (row_swz).
     static_assert(9 * 64 == 8 * CH && NI == 36, "9 offsets a lane");
+    const int mv = MW ? wave - NW : wave;   // (of a wave that moves)
     uint32_t dofs2[5] = {};   // two in a register (below 2^15)
 #pragma unroll
     for (int j = 0; j < 9; ++j) {
-      const int c = 64 * ((wave + NW * j) % (NI / 2)) + lane, kr = c / CH;
+      const int c = 64 * ((mv + ML * j) % (NI / 2)) + lane, kr = c / CH;
       dofs2[j >> 1] |= (uint32_t)((kr * CH + ((c - kr * CH) ^ row_swz(kr))) * 16) << 16 * (j & 1);
     }
     // The pages of 32 tiles from `pg0` on, one a lane: a scalar load on its way would turn every wait for an LDS operand
@@ -504,16 +512,19 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
     };
     // (The queries have come by then too.  The compiler, which does not know the moves, would otherwise wait for a query ahead of every product of S^T,
     // in the loop too, and so for all but a few of the moves that come after it.)
-    look(begin);
+    if (MW == 0 || wave >= NW) look(begin);
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (moved) {
 #pragma unroll
       for (int s = 0; s < NS; ++s) qf[s] = kfrag(wave * IMG, s);
     }
 #if defined(__HIP_DEVICE_COMPILE__)
+    if (wave < NW) {
 #pragma unroll
-    for (int s = 0; s < NS; ++s) asm volatile("" : "+v"(qf[s]));
+      for (int s = 0; s < NS; ++s) asm volatile("" : "+v"(qf[s]));
+    }
 #endif
-    if constexpr (NW == 4) {
+    if constexpr (MW == 0) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __syncthreads();   // (the images are the keys' from here on)
     }
@@ -529,15 +540,41 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
       asm volatile("" : "+v"(dofs2[0]), "+v"(dofs2[1]), "+v"(dofs2[2]), "+v"(dofs2[3]), "+v"(dofs2[4]));   // (or the loop would hold them unpacked)
     };
     auto landed = [&](bool more) {   // the tile before the one that was moved last (`more`: if one was)
-      if (NW > 1 || more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NJ) : "memory");
+      if (MW == 0 || more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NJ) : "memory");
       else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     };
     auto dma = [&](int j) __attribute__((always_inline)) {
-      const int i = wave + NW * j;
-      const uint32_t two = dofs2[j % 9 >> 1], at = j % 9 & 1 ? two >> 16 : two & 0xffff;
-      buffer_to_lds(j < NJ / 2 || (NW == 4 && i < NI / 2) ? b0 : b1, bytes, NW == 1 && j / 9 % 2 ? at ^ 16 : at, NW == 1 && j / 9 % 2 ? 8 * CH * 16 : 0,
-                    to + 64 * 16 * i);
+      const int i = mv + ML * j;
+      constexpr int OWN = MW ? NI / 2 / ML : 9;   // offsets that a lane has: of a page's moves (MW == 0: two pages have an odd number)
+      const uint32_t two = dofs2[j % OWN >> 1], at = j % OWN & 1 ? two >> 16 : two & 0xffff;
+      buffer_to_lds(i < NI / 2 ? b0 : b1, bytes, at, 0, to + 64 * 16 * i);
     };
+    if constexpr (MW > 0) {
+      if (wave >= NW) {   // three tiles ahead of the one whose values are multiplied; barriers as below
+        const auto put = [&](int tile, int img) __attribute__((always_inline)) {
+          if (tile >= end) return;
+          aim(tile, img);
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) dma(j);
+        };
+        if (begin < end) {
+          put(begin, 0);
+          put(begin + 1, 1);
+          landed(begin + 1 < end);
+          __syncthreads();
+          put(begin + 2, 2);
+          landed(begin + 2 < end);
+          __syncthreads();
+          for (int n = begin; n < end; ++n) {
+            put(n + 3, (n + 3 - begin) & 3);
+            landed(n + 3 < end);
+            __syncthreads();
+          }
+        }
+        __syncthreads();
+        return;
+      }
+    }
 
     f32x16 o[NV];
 
@@ -572,48 +609,34 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
     // The first two tiles together, the third beside the first one's products: the second was asked for beside them as well, and pieces of two
     // and three tiles, which saw its whole latency, took as much longer as the pipeline saved (us, three images -> that -> this: 16 rows of 128
     // heads over 640 keys 30.4 -> 30.5 -> 30.2, six prompts of 59 rows 36.9 -> 37.5 -> 36.4; 32 x 8000 keys of 16 heads 84.8 -> 85.9 -> 84.0).
-    if (begin < end) {
+    if (MW == 0 && begin < end) {
       aim(begin, 0);
 #pragma unroll
       for (int j = 0; j < NJ; ++j) dma(j);
-      if (NW > 1 || begin + 1 < end) {
-        aim(begin + 1, 1);
+      aim(begin + 1, 1);
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) dma(j);
-      }
+      for (int j = 0; j < NJ; ++j) dma(j);
     }
 #pragma unroll
     for (int v = 0; v < NV; ++v)
 #pragma unroll
       for (int i = 0; i < 16; ++i) o[v][i] = 0.f;
     if (begin < end) {
-      landed(begin + 1 < end);
+      if (MW == 0) landed(true);
       __syncthreads();
-      if constexpr (NW == 1) {
-        if (begin + 2 < end) {
-          aim(begin + 2, 2);
-#pragma unroll
-          for (int j = 0; j < NJ; ++j) dma(j);
-        }
-        score(0, sc, [](int) {});
-      } else {
-        static_assert(NW == 1 || NS % NJ == 0, "a move every so many products");
-        score(0, sc, [&](int s) __attribute__((always_inline)) {
-          if (s == 0) aim(begin + 2, 2);
-          if (s % (NS / NJ) == 0) dma(s / (NS / NJ));
-        });
-      }
-      landed(begin + 2 < end);
+      static_assert(MW > 0 || NS % NJ == 0, "a move every so many products");
+      score(0, sc, [&](int s) __attribute__((always_inline)) {
+        if (MW == 0 && s == 0) aim(begin + 2, 2);
+        if (MW == 0 && s % (NS / NJ) == 0) dma(s / (NS / NJ));
+      });
+      if (MW == 0) landed(true);
       __syncthreads();
     }
     const int Lmin = -wave_most(-L);   // the wave's shortest row: tiles below it have no key to mask
     int cur = 0;
     for (int n = begin; n < end; ++n) {
       const int nxt = (cur + 1) & 3;
-      aim(n + 3, (cur + 3) & 3);   // (that image was last read in the previous round, before its barrier)
-      if (NW == 1 && n + 3 < end)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) dma(j);
+      if (MW == 0) aim(n + 3, (cur + 3) & 3);   // (that image was last read in the previous round, before its barrier)
       if ((n + 1) * KT > Lmin) {
         const int key = n * KT + 4 * hf;
 #pragma unroll
@@ -714,7 +737,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
         mma_acc(o[k % NV], vf[k % AHEAD], pb[k / NV]);
         if (k + AHEAD < 2 * NV) vf[k % AHEAD] = vfrag(cur * IMG, (k + AHEAD) % NV, (k + AHEAD) / NV);
         if (k < NV) weights(8 + k / 4 * 2, k % 4);   // the second half's, beside the first half's products
-        if ((NW == 2 && k >= 14) || (NW == 4 && k >= 14 && k % 2 == 0)) dma(NW == 2 ? k - 14 : (k - 14) / 2);
+        if (MW == 0 && k >= 14 && k % 2 == 0) dma((k - 14) / 2);
         __builtin_amdgcn_sched_barrier(0);
       }
       {
@@ -743,7 +766,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
           }
         }
       cur = nxt;
-      landed(n + 3 < end);   // (tile n + 2)
+      if (MW == 0) landed(true);   // (tile n + 2)
       __syncthreads();
     }
     asm volatile(MMA_WAIT "\n\ts_waitcnt vmcnt(0)" ::: "memory");
@@ -809,6 +832,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
   const bool same0 = ((left >> lane) & 1) && tl_row == bt0;
   left &= ~__ballot(same0);
   walk(bt0, same0, lane);
+  if (MW > 0 && wave >= NW) return;
   // Tokens of further block-table rows: an `own_seq` workgroup takes them, unless they are not in order.  (Those go one
   // row at a time: a second pass here would hold its operands over the first one's epilogue, in scratch.)
   if constexpr (!DECODE) {
@@ -1101,7 +1125,7 @@ static void mla_launch(const void* q, int64_t q_stride_t, const void* cache, con
 #define MLA_ROWS(NW)                                                                                                    \
   {                                                                                                                      \
     const auto kernel = plan ? mla_attn_rows_kernel<DK, DV, NW, true> : mla_attn_rows_kernel<DK, DV, NW, false>;          \
-    kernel<<<grid, 64 * NW, 0, stream>>>((const bf16*)q, q_stride_t, (const bf16*)cache, block_tables, bt_stride,         \
+    kernel<<<grid, 64 * (NW + row_movers(NW)), 0, stream>>>((const bf16*)q, q_stride_t, (const bf16*)cache, block_tables, bt_stride,         \
                                          tok_row, kv_lens, T, H, seqs, scale_log2, parts, plan, (bf16*)out,               \
                                          out_stride_t, ws_o, ws_ml);                                                     \
     if (parts > 1)                                                                                                       \
