@@ -1115,7 +1115,10 @@ class MLAWorkspace:
         42 / 15 17 21 32, 24 rows 14 20 36 72 / 16 19 25 41; 32 heads, 12 rows 14 21 32 62 / 16 18 23 30, 16 rows 15 23 37
         72 / 16 19 24 32; 64 heads, 4 rows 12 14 16 23 / 16 16 18 25, 6 rows 15 22 33 65 / 16 18 23 31 of 32 rows, 12 rows 21 30
         44 87 / 19 22 27 36 of 64 rows, 48 rows 22 31 45 95 / 25 29 39 68; 128 heads, 16 rows 29 33 38 52 / 22 27 35 54 of
-        64 rows, 32 rows 32 38 47 75 / 33 38 47 69 of 128 rows; from 64 rows on, ``mla_attn_all_kernel`` in ``mla.hip``."""
+        64 rows, 32 rows 32 38 47 75 / 33 38 47 69 of 128 rows.  Tables that hold short contexts only take tiles of 32 rows, which start sooner, and
+        for fewer rows of 32 heads (before -> now): tables of 11 pages, 24 and 48 rows of 128 heads 26.8 -> 21.4, 29.6 -> 22.8, 128 of 64 26.1 -> 20.4; of 22
+        pages, 48 of 128 37.3 -> 33.3, 128 of 64 36.2 -> 30.1, 24 of 64 20.6 -> 19.0 (26 pages, 100 of 64 33.3 -> 36.7: not there); of 44 pages, 12, 16
+        and 23 of 64 20.8 -> 19.3, 23.2 -> 21.2, 23.3 -> 21.0, 12 of 32 20.1 -> 16.5, of 26 pages 19.0 -> 15.6.  From 64 rows on, ``mla_attn_all_kernel`` in ``mla.hip``."""
         n, wide = T * H, T * -(-H // 16) * 16
         if DK == 576 and H >= 4 and _MLA_ROW_TILES:
             if T >= 4 * seqs:
@@ -1128,8 +1131,10 @@ class MLAWorkspace:
                             us = -(-wgs // cls.TARGET_WGS_ALL) * (start + 0.06 * keys / p) + (p > 1) * (6 + n * p / 1500)
                             best = min(best or (us, rows, p), (us, rows, p))
                     return best[1], False, best[2]
-            elif wide >= (768 if H <= 8 or pages <= 16 and H % 64 else 512 if 16 < H <= 32 else 384) and not (H % 128 == 0 and T >= 64):
-                rows = 32 if n < 704 or 0 < H % 64 <= 32 else 128 if H % 128 == 0 and T >= 24 else 64
+            elif wide >= (768 if H <= 8 or pages <= 16 and H % 64 else 512 if 16 < H <= 32 and not 24 < pages <= 48 else 384) and \
+                    not (H % 128 == 0 and T >= 64):
+                few = n < 704 or pages <= 48 and n < 1536 or pages <= 24 and n <= 8192
+                rows = 32 if few or 0 < H % 64 <= 32 else 128 if H % 128 == 0 and T >= 24 else 64
                 return rows, True, cls.parts(T, H, DK, rows, True)
         return 0, False, cls.parts(T, H, DK, pages=pages)
 

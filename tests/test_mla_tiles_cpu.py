@@ -35,6 +35,15 @@ def test_decode_steps_need_no_context(T, H, want):
         assert 256 * rows <= W.ROWS and (rows or T * H * parts <= W.ROWS)
 
 
+@pytest.mark.parametrize("T,H,pages,want", [(48, 128, 24, 32), (48, 128, 25, 128), (128, 64, 24, 32), (129, 64, 24, 64), (12, 64, 48, 32), (12, 64, 49, 64),
+                                            (24, 64, 48, 64), (12, 32, 24, 0), (12, 32, 25, 32), (12, 32, 48, 32), (11, 32, 48, 0)])
+def test_decode_steps_over_short_tables(T, H, pages, want):
+    """... of which a piece is still one workgroup of the 256."""
+    rows, decode, parts = W.tiles(T, H, 576, T, pages)
+    assert rows == want and decode == (want > 0)
+    assert not rows or (parts == 1 or T * -(-H // rows) <= 256)
+
+
 def test_many_rows_of_128_heads_fill_the_chip_once():
     for T in (64, 96, 128, 200, 256, 600):
         assert W.tiles(T, 128, 576, T, 256) == (0, False, max(1, 256 // T)) and W.tiles(T, 128, 288, T, 256)[0] == 0
