@@ -6,9 +6,9 @@
 // 288 = 256 + 32 for MiniCPM3 (template instances below).  With W_UK folded into the query
 // (q_lat = [q_nope . W_UK | q_pe], 576 wide) and W_UV applied after the attention, MLA is
 // multi-QUERY attention over that latent: scores use all 576 dims, values are the first 512.
-// Three kernels serve decode, prefill and chunked prefill: row tiles (mla_attn_rows_kernel, DK = 576: prompts, and
+// Four kernels serve decode, prefill and chunked prefill: row tiles (mla_attn_rows_kernel, DK = 576: prompts, and
 // decode steps of some 24 rows or 6 with many heads), 128 heads a workgroup (mla_attn_all_kernel: many decode rows of
-// so many heads), and here 16 heads a workgroup (few rows, other widths, sinks, windows): a work item is one query
+// so many heads), and 16 heads a workgroup, of pages (mla_attn_pages_kernel, DK = 576: few rows) and here (other widths; a few rows over short tables): a work item is one query
 // token x 16 heads (every head of a token shares the causal limit) x one split-K partition.
 //
 // Workgroup = 4 waves: all four compute S^T for the same 16 heads x 32 keys (the K tile is
@@ -55,6 +55,7 @@ __device__ __forceinline__ bf16x4 tr_read(const bf16* lds_base, int byte_off) {
 // each keeps four tiles, so short contexts leave the later ones empty (one token of 16 heads, 16 / 32 / 64 partitions of equal size, us:
 // 300 keys 11.6 / 13.0 / 15.8, 3000 23 / 21 / 24, 8000 44 / 31 / 31; every five or six tiles: 3000 23 / 23, 8000 31 / 31).
 __device__ __forceinline__ int live_parts(int tiles, int parts) { return min(parts, max(16, (tiles + 3) / 4)); }
+constexpr int LEAST_PAIRS = 2;   // key tiles of a partition of mla_attn_pages_kernel, whose waves take a page each
 
 }  // namespace
 
@@ -204,6 +205,196 @@ __global__ __launch_bounds__(256) void mla_attn_kernel(
     for (int nb = 0; nb < NB; ++nb)
       *reinterpret_cast<f32x4*>(wp + 16 * nb) = f32x4{o[nb][0] * inv, o[nb][1] * inv, o[nb][2] * inv,
                                                        o[nb][3] * inv};
+    if (wave == 0 && g == 0) {
+      ws_ml[2 * ws_row] = m;
+      ws_ml[2 * ws_row + 1] = lsum;
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------------
+// Few decode rows at DeepSeek's widths: work items and partitions of mla_attn_kernel, but each of the four waves streams pages of its own, every
+// fourth of the partition's, with an online softmax of its own over all DV value dims, and the four meet in LDS at the end.  Bound by the
+// cache's bytes where contexts are long, and by its latency where they are short: a wave has a page (18 KB) on its way to LDS while it multiplies
+// another, 74 KB a CU, and no step waits for another wave.  (Above, 32 keys at a time go through registers, all waves form the same S^T, and
+// two barriers a tile leave the loads of one tile of each workgroup in flight.)  Whole calls, us, that -> this: 16 heads, 8 rows of ~3000 and ~8000 keys
+// 31 -> 27, 58 -> 38, 16 rows 43 -> 31, 85 -> 45, 23 rows of 400, 1000, 3000, 8000 22 -> 17, 32 -> 23, 67 -> 35, 138 -> 59; 32 heads, 12 rows of 1000 and 8000
+// 31 -> 22, 156 -> 61; 64 heads, 4 of 3000 42 -> 29; 128 heads, 2 of 3000 34 -> 25; 8 heads, 40 of 1000 34 -> 24.  At 16 workgroups and fewer over
+// 100 to 400 keys it took 0.2 to 1 us more (4 rows of 16 heads 11.7 -> 12.5, 14.0 -> 14.2; 1 of 128 over 92 pages 18.4 -> 18.9), so tables of at most 96 pages stay there.
+// ------------------------------------------------------------------------------------------
+template <int DK, int DV>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void mla_attn_pages_kernel(
+    const bf16* __restrict__ q, int64_t q_stride_t, const bf16* __restrict__ cache,
+    const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ tok_row,
+    const int* __restrict__ kv_lens, int H, float scale_log2, int parts, bf16* __restrict__ out,
+    int64_t out_stride_t, float* __restrict__ ws_o, float* __restrict__ ws_ml, const float* __restrict__ sinks,
+    int window) {
+  constexpr int CH = DK / 8, NV = DV / 16, NB = NV / 4, MOVES = 16 * CH / 64, IMG = 16 * CH * 16;
+  static_assert(CH % 8 == 0 && MOVES * 64 == 16 * CH && 9 * 64 == 8 * CH, "whole moves, nine of them 8 rows");
+  static_assert(NV * 1024 <= 2 * IMG, "a wave's output fits its images");
+  __shared__ __attribute__((aligned(16))) char sK[4 * 2 * IMG];
+  __shared__ float sM[4][16], sL[4][16];
+  const int t = blockIdx.x, h0 = blockIdx.y * 16, part = blockIdx.z;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int col = lane & 15, g = lane >> 4;
+  const int L = __builtin_amdgcn_readfirstlane(kv_lens[t]);
+  const int lo = window > 0 ? max(L - window, 0) : 0;   // sliding window: keys [lo, L) only
+  const int n_pages = (L + 15) >> 4, pairs = (n_pages + 1) >> 1, pair_lo = lo / KT;   // partitions as in mla_attn_kernel
+  const int live = live_parts(pairs - pair_lo, parts), per_part = max(LEAST_PAIRS, (pairs - pair_lo + live - 1) / live);
+  const int pair_begin = pair_lo + part * per_part, pair_end = min(pairs, pair_begin + per_part);
+  const int p0 = 2 * pair_begin, p1 = min(2 * pair_end, n_pages);
+  const int n = __builtin_amdgcn_readfirstlane(max(0, (p1 - p0 - wave + 3) >> 2));   // this wave's pages: p0 + wave, + 4, ..
+  const int* bt = block_tables + (int64_t)tok_row[t] * bt_stride;
+  const int64_t ws_row = ((int64_t)t * H + h0 + col) * parts + part;
+  const bool hv = h0 + col < H;
+  if (p0 >= p1) {   // whole block: no keys (the merge reads no value of a partition whose sum is 0, and of those beyond 16 not the sum)
+    if (hv && parts == 1) {
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+        *reinterpret_cast<bf16x4*>(out + (int64_t)t * out_stride_t + (int64_t)(h0 + col) * DV + wave * (DV / 4) + 4 * g + 16 * nb) = bf16x4{};
+    } else if (hv && part < 16 && wave == 0 && g == 0) {
+      ws_ml[2 * ws_row] = OME_NEG_INF;
+      ws_ml[2 * ws_row + 1] = 0.f;
+    }
+    return;
+  }
+
+  // The first two pages by scalar loads: their moves wait for neither the queries nor the list
+  const int first = bt[min(p0 + wave, p1 - 1)], second = bt[min(p0 + wave + 4, p1 - 1)];
+  const auto id = [&](int i) { const int p = p0 + wave + 4 * (i + lane); return bt + (p < p1 ? p : p0); };
+  int pages = *id(0), at0 = 0;   // the next 64 of this wave's pages, one a lane
+  // ---- Q^T operand: lane (col, g) holds Q[h0+col][32 s + 8 g + j] ----
+  bf16x8 qf[DK / 32];
+  const bf16* qp = q + (int64_t)t * q_stride_t + (int64_t)(hv ? h0 + col : 0) * DK + 8 * g;
+#pragma unroll
+  for (int s = 0; s < DK / 32; ++s) qf[s] = hv ? ld8(qp + 32 * s) : bf16x8{};
+
+  // A page -> LDS image: move i writes chunks [64 i, 64 i + 64), each lane fetching the source chunk that its row's swizzle puts there
+  uint32_t ofs[9];
+#pragma unroll
+  for (int j = 0; j < 9; ++j) {
+    const int c = 64 * j + lane, r = c / CH;
+    ofs[j] = (r * CH + ((c - r * CH) ^ (r & 7))) * 16;
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)sK + wave * 2 * IMG;
+  const auto look = [&](int i) __attribute__((always_inline)) {
+#if defined(__HIP_DEVICE_COMPILE__)   // (waited for here: the compiler would wait at every use, and for the moves as well)
+    asm volatile("global_load_dword %0, %1, off\n\ts_waitcnt vmcnt(0)" : "=&v"(pages) : "v"(id(i)) : "memory");
+#endif
+    at0 = i;
+  };
+  const auto move_page = [&](int i, int index) __attribute__((always_inline)) {
+    const bf16* page = cache + (int64_t)index * 16 * DK;
+    const uint32_t bytes = min(16, L - 16 * (p0 + wave + 4 * i)) * DK * 2;   // (rows past the context: zeros)
+#pragma unroll
+    for (int j = 0; j < MOVES; ++j) buffer_to_lds(page, bytes, ofs[j % 9] + j / 9 * (8 * CH * 16), 0, lds0 + (i & 1) * IMG + 1024 * j);
+  };
+  const auto move = [&](int i) __attribute__((always_inline)) {
+    if (i >= n) return;
+    if (i - at0 == 64) look(i);
+    move_page(i, __builtin_amdgcn_readlane(pages, i - at0));
+  };
+  f32x4 o[NV];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) o[v] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = OME_NEG_INF, lsum = 0.f;
+  if (n > 0) move_page(0, first);
+  if (n > 1) move_page(1, second);
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+  for (int s = 0; s < DK / 32; ++s) asm volatile("" : "+v"(qf[s]));   // (waited for here, once)
+  asm volatile("" : "+v"(pages));
+#endif
+  const int qrow = col >> 2, pcol = lane & 3, row = 4 * g + qrow;   // tr-read block: rows = keys 4 g + qrow, columns 4 pcol .. + 3
+#pragma unroll 1
+  for (int i = 0; i < n; ++i) {
+    if (i + 1 < n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(MOVES) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const bf16* img = reinterpret_cast<const bf16*>(sK + (wave * 2 + (i & 1)) * IMG);
+    // ---- S^T [16 keys x 16 heads], two chains ----
+    f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < DK / 32; s += 2) {
+      sa = mfma16x32(*reinterpret_cast<const bf16x8*>(&img[swz<DK>(col, 4 * s + g) * 8]), qf[s], sa);
+      sb = mfma16x32(*reinterpret_cast<const bf16x8*>(&img[swz<DK>(col, 4 * s + 4 + g) * 8]), qf[s + 1], sb);
+    }
+    const int k0 = 16 * (p0 + wave + 4 * i) + 4 * g;
+    float mx = OME_NEG_INF;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      sa[e] = (k0 + e < L && k0 + e >= lo) ? (sa[e] + sb[e]) * scale_log2 : OME_NEG_INF;
+      mx = fmaxf(mx, sa[e]);
+    }
+    mx = group4_max(mx);
+    const float m_new = fmaxf(m, mx);
+    const float alpha = m_new == OME_NEG_INF ? 1.f : __builtin_amdgcn_exp2f(m - m_new);
+    s16x4 pb;
+    float ps = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float p = m_new == OME_NEG_INF ? 0.f : __builtin_amdgcn_exp2f(sa[e] - m_new);
+      ps += p;
+      pb[e] = __builtin_bit_cast(short, (bf16)p);
+    }
+    lsum = lsum * alpha + group4_sum(ps);
+    m = m_new;
+    if (__ballot(alpha != 1.f)) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) o[v] *= alpha;
+    }
+    // ---- O^T [DV x 16 heads] += V^T . P^T ----
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+      o[v] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+          __builtin_bit_cast(s16x4, tr_read(img, swz<DK>(row, 2 * v + (pcol >> 1)) * 16 + (pcol & 1) * 8)), pb, o[v], 0, 0, 0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the image is read)
+    move(i + 2);
+  }
+
+  // ---- the waves' sums meet: each writes its own over its images, and takes a quarter of the dims of all ----
+  f32x4* const so = reinterpret_cast<f32x4*>(sK);
+  constexpr int WO = 2 * IMG / 16;   // between waves
+#pragma unroll
+  for (int v = 0; v < NV; ++v)
+    if (n > 0) so[wave * WO + v * 64 + lane] = o[v];
+  if (g == 0) sM[wave][col] = m, sL[wave][col] = lsum;
+  __syncthreads();
+  const int act = min(4, p1 - p0);   // waves that had a page
+  f32x4 sum[NB];
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) sum[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  m = OME_NEG_INF, lsum = 0.f;
+  for (int w = 0; w < act; ++w) m = fmaxf(m, sM[w][col]);
+  for (int w = 0; w < act; ++w) {
+    const float mw = sM[w][col], e = mw == OME_NEG_INF ? 0.f : __builtin_amdgcn_exp2f(mw - m);
+    lsum += e * sL[w][col];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) sum[nb] += e * so[w * WO + (wave * NB + nb) * 64 + lane];
+  }
+
+  // ---- output or partials, as of mla_attn_kernel: dim = 16 nb + 4 g + i of the wave's quarter, head = col ----
+  if (sinks != nullptr && parts == 1 && hv) {
+    const float sk = sinks[h0 + col] * 1.4426950408889634f;
+    const float m_fin = fmaxf(m, sk), a = __builtin_amdgcn_exp2f(m - m_fin);
+    lsum = lsum * a + __builtin_amdgcn_exp2f(sk - m_fin);
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) sum[nb] *= a;
+  }
+  const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+  if (!hv) return;
+  if (parts == 1) {
+    bf16* op = out + (int64_t)t * out_stride_t + (int64_t)(h0 + col) * DV + wave * (DV / 4) + 4 * g;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      bf16x4 v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = (bf16)(sum[nb][i] * inv);
+      *reinterpret_cast<bf16x4*>(op + 16 * nb) = v;
+    }
+  } else {
+    float* wp = ws_o + ws_row * DV + wave * (DV / 4) + 4 * g;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) *reinterpret_cast<f32x4*>(wp + 16 * nb) = sum[nb] * inv;
     if (wave == 0 && g == 0) {
       ws_ml[2 * ws_row] = m;
       ws_ml[2 * ws_row + 1] = lsum;
@@ -547,7 +738,7 @@ __global__ __launch_bounds__(64 * (NW + row_movers(NW))) __attribute__((amdgpu_w
       const int i = mv + ML * j;
       constexpr int OWN = MW ? NI / 2 / ML : 9;   // offsets that a lane has: of a page's moves (MW == 0: two pages have an odd number)
       const uint32_t two = dofs2[j % OWN >> 1], at = j % OWN & 1 ? two >> 16 : two & 0xffff;
-      buffer_to_lds(i < NI / 2 ? b0 : b1, bytes, at, 0, to + 64 * 16 * i);
+      buffer_to_lds(j < NJ / 2 || (NJ % 2 && j == NJ / 2 && i < NI / 2) ? b0 : b1, bytes, at, 0, to + 64 * 16 * i);
     };
     if constexpr (MW > 0) {
       if (wave >= NW) {   // three tiles ahead of the one whose values are multiplied; barriers as below
@@ -1062,12 +1253,12 @@ __global__ __launch_bounds__(128) void mla_reduce_kernel(const float* __restrict
                                                          const float* __restrict__ ws_ml, int H, int parts,
                                                          bf16* __restrict__ out, int64_t out_stride_t,
                                                          const float* __restrict__ sinks, const int* __restrict__ kv_lens,
-                                                         int window, bool equal) {
+                                                         int window, int least) {
   const int t = blockIdx.x, h = blockIdx.y;
   const int64_t row0 = ((int64_t)t * H + h) * parts;
-  if (parts > 16 && !equal) {   // as mla_attn_kernel cut them (with 16 the empty ones cost less than the length's way here)
+  if (parts > 16 && least > 0) {   // as the 16-head kernels cut them, `least` tiles and more (with 16 the empty ones cost less than the length's way here)
     const int L = kv_lens[t], tiles = ((L + 15) / 16 + 1) / 2 - (window > 0 ? max(L - window, 0) / KT : 0);
-    const int live = live_parts(tiles, parts), per = (tiles + live - 1) / live;
+    const int live = live_parts(tiles, parts), per = tiles > 0 ? max(least, (tiles + live - 1) / live) : 0;
     parts = per > 0 ? (tiles + per - 1) / per : 0;
   }
   float M = OME_NEG_INF, den = 0.f;
@@ -1148,12 +1339,24 @@ static void mla_launch(const void* q, int64_t q_stride_t, const void* cache, con
       done = true;
     }
   }
+  if constexpr (DK == 576) {
+    // (few workgroups over short tables: the old kernel starts a microsecond sooner.  It also has a CU hold several workgroups)
+    const int64_t wgs = (int64_t)T * ((H + 15) / 16);
+    if (!done && wgs * parts <= 512 && (wgs > 16 || bt_stride > 96)) {
+      mla_attn_pages_kernel<DK, DV><<<dim3(T, (H + 15) / 16, parts), 256, 0, stream>>>(
+          (const bf16*)q, q_stride_t, (const bf16*)cache, block_tables, bt_stride, tok_row, kv_lens, H, scale_log2,
+          parts, (bf16*)out, out_stride_t, ws_o, ws_ml, sinks, window);
+      if (parts > 1)
+        mla_reduce_kernel<DV><<<dim3(T, H), DV / 4, 0, stream>>>(ws_o, ws_ml, H, parts, (bf16*)out, out_stride_t, sinks, kv_lens, window, LEAST_PAIRS);
+      return;
+    }
+  }
   if (!done)
     mla_attn_kernel<DK, DV><<<dim3(T, (H + 15) / 16, parts), 256, 0, stream>>>(
         (const bf16*)q, q_stride_t, (const bf16*)cache, block_tables, bt_stride, tok_row, kv_lens, H, scale_log2,
         parts, (bf16*)out, out_stride_t, ws_o, ws_ml, sinks, window);
   if (parts > 1)
-    mla_reduce_kernel<DV><<<dim3(T, H), DV / 4, 0, stream>>>(ws_o, ws_ml, H, parts, (bf16*)out, out_stride_t, sinks, kv_lens, window, done);
+    mla_reduce_kernel<DV><<<dim3(T, H), DV / 4, 0, stream>>>(ws_o, ws_ml, H, parts, (bf16*)out, out_stride_t, sinks, kv_lens, window, done ? 0 : 1);
 }
 
 OME_API int ome_mla_attn(const void* q, int64_t q_stride_t, const void* cache, const int* block_tables,

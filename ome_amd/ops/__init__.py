@@ -1075,11 +1075,11 @@ class MLAWorkspace:
     tokens x heads x partitions, bounded by ``ROWS``).
 
     Kernels (``mla.hip``): row tiles (:meth:`tiles`: one workgroup, one to a CU, streams the latent KV once
-    for 32 / 64 / 128 query rows), 128 heads a workgroup for many decode rows, and the 16-head kernel (few rows, other
-    widths, sinks, windows).  Row tiles of prompts are cut into equal partitions up to ~1 workgroup per CU; those of decode
+    for 32 / 64 / 128 query rows), 128 heads a workgroup for many decode rows, and two 16-head kernels (few rows, other
+    widths, sinks, windows; the one with a CU to itself from 17 workgroups or 97 pages on).  Row tiles of prompts are cut into equal partitions up to ~1 workgroup per CU; those of decode
     steps by the kernel itself, by their lengths, into at most 256 pieces (``plan``: each tile's first partial and
     piece count; 256 x 128 rows are ``ROWS``).  The 16-head
-    kernel takes partitions up to ~1024 workgroups, at most 16 unless that leaves CUs without one.  None beyond what the f32 partials' HBM round trip repays."""
+    kernels take partitions up to ~1024 workgroups, or 256, at most 16 unless that leaves CUs without one.  None beyond what the f32 partials' HBM round trip repays."""
 
     TARGET_WGS = 1024
     TARGET_WGS_ALL = 256
@@ -1157,6 +1157,8 @@ class MLAWorkspace:
             # the merge still asks for the length, up to 0.5 us more.  15 workgroups: 17 partitions 1.02 up to 4000 keys, 0.98 at 8000.  With two to
             # a CU 52 at 8000, and 64 for 8 of 32, which 16 take 57)
             most = cls.MAX_PARTS if wgs > 12 or pages <= 128 else min(cls.MAX_PARTS_ALL, cls.TARGET_WGS_ALL // max(wgs, 1))
+            if DK == 576 and 16 < wgs <= 128:   # (a workgroup of mla_attn_pages_kernel to a CU, and a page for each of its waves)
+                most = min(most, cls.TARGET_WGS_ALL // max(wgs, 1), -(-pages // 4) if pages <= 16 else most)
             p = 1 if wgs >= cls.TARGET_WGS else max(1, min(most, cls.TARGET_WGS // max(wgs, 1)))
         return max(1, min(p, cls.ROWS // max(T * H, 1)))
 

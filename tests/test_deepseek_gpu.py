@@ -328,6 +328,32 @@ def test_mla_partitions_by_length(T, H):
         assert ((out - want).flatten(1).norm(dim=1) <= 2.0 ** -8 * want.flatten(1).norm(dim=1)).all(), ctx
 
 
+@pytest.mark.parametrize("T,H", [(20, 16), (11, 24), (40, 8)])
+@pytest.mark.parametrize("longest", [48, 230, 1100, 4500])
+def test_mla_waves_with_pages_of_their_own(T, H, longest):
+    """Contexts at the edges of pages, of a page for each wave and of 64 of a wave's pages, in one partition and in several, over a cache whose rows
+    past the contexts are NaN.  Tolerance as above."""
+    torch.manual_seed(T)
+    every = [n for n in (longest, 0, 1, 15, 16, 17, 32, 33, 48, 49, 64, 65, 128, 129, 240, 513, 1024, 1090, 4096, 4097) if n <= longest]
+    ctx = (every * T)[:T]
+    cache, bt = _setup(ctx)
+    for s, n in enumerate(ctx):
+        if n % 16:
+            cache[bt[s, n // 16].item(), n % 16:] = float("nan")
+    row, kl = torch.arange(T, dtype=torch.int32), torch.tensor(ctx, dtype=torch.int32)
+    q = torch.randn(T, H, 576, device=DEV).to(torch.bfloat16)
+    assert ops.MLAWorkspace.parts(T, H, 576, pages=bt.shape[1]) == {48: 1, 230: 4}.get(longest, 256 // (T * -(-H // 16)))
+    for parts in (None, 1, 3):
+        with pytest.MonkeyPatch.context() as mp:
+            p = parts or ops.MLAWorkspace.parts(T, H, 576, pages=bt.shape[1])
+            mp.setattr(ops.MLAWorkspace, "tiles", lambda *a: (0, False, p))
+            out = ops.mla_attn(q, cache, bt, row.to(DEV), kl.to(DEV), 192 ** -0.5).cpu().double()
+        want = _exact(q, torch.nan_to_num(cache), bt, row, kl, 192 ** -0.5)
+        live = kl > 0
+        assert bool((out[~live] == 0).all())
+        assert ((out - want).flatten(1).norm(dim=1)[live] <= 2.0 ** -8 * want.flatten(1).norm(dim=1)[live]).all()
+
+
 @pytest.mark.parametrize("T,H", [(1, 16), (3, 32), (12, 16)])
 def test_mla_reads_no_partition_that_is_not_written(T, H):
     """A workspace that holds NaN, contexts of fewer partitions than the table's width allows, and the tokens' own lengths.  Tolerance as above."""
