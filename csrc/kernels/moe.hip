@@ -283,10 +283,10 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
       acc = end;
     }
   if (threadIdx.x == 1023) offsets[E] = acc;   // (its run is the last, or empty: the total)
-  if (tiles != nullptr) {   // the rest have no expert
+  if (tiles != nullptr) {   // the rest have no expert, but the number of those that have
     int all = 0;
     for (int w = 0; w < 16; ++w) all += s_tiles[w];
-    for (int i = all + threadIdx.x; i < max_tiles; i += blockDim.x) tiles[i] = int4{-1, 0, 0, 0};
+    for (int i = all + threadIdx.x; i < max_tiles; i += blockDim.x) tiles[i] = int4{-1, 0, 0, all};
   }
   __syncthreads();
   // stable within an expert is not required (the combine uses the inverse map)
@@ -309,7 +309,7 @@ OME_API int ome_moe_align(const int* topk_ids, int n, int E, int* offsets, int* 
 
 // ... and the tiles of `bm` rows of one expert each, of experts below `e_tiles`, (expert, first row, the expert's end, 0), 16-byte aligned: a workgroup of the
 // kernels below reads its own instead of searching the offsets (512 experts: eight rounds of a wave's prefix sum, 2 us a
-// workgroup).  max_tiles >= min(n, E) + n / bm bounds their number; entries past it have expert -1.
+// workgroup).  max_tiles >= min(n, E) + n / bm bounds their number; entries past it have expert -1 and that number in the last place.
 OME_API int ome_moe_align_tiles(const int* topk_ids, int n, int E, int* offsets, int* sorted_ids, int* inv, int* tiles, int bm,
                                 int e_tiles, int max_tiles, hipStream_t stream) {
   if (n <= 0 || bm <= 0 || max_tiles < (n < E ? n : E) + n / bm || (uintptr_t)tiles % 16) return -2;
@@ -560,6 +560,21 @@ __global__ __launch_bounds__(256) void moe_gemm_v2_kernel(const bf16* __restrict
 typedef __attribute__((address_space(3))) void moe_lds_t;
 typedef __attribute__((address_space(1))) void moe_glb_t;
 
+// This workgroup's place in the grid of (blocks of columns, tiles); a tile past the last: none.  Workgroups go to the XCDs in turn.  With `runs` those of an XCD
+// take a run of the tiles, all blocks of each, and so walk through one stretch of the weights.  In the grid's order, where a tile's blocks are a multiple of 8,
+// an XCD has every eighth block of every tile, 64 rows at eight times that distance, which memory serves more slowly.  Whole layers, us, 8 experts of 4096 x
+// 14336, 1, 4, 16, 64 and 128 rows 180 -> 165, 360 -> 328, 468 -> 428, 528 -> 500, 568 -> 552; 512 of 2048 x 512, 48 and 256 rows 326 -> 310, 557 -> 541.  But runs of
+// tiles with many rows are unequal work, and without that multiple there is nothing to gain (128 experts of 2688 x 1856, 400 rows 417 -> 435; 512 experts with 43 rows each
+// 774 -> 783; 8 with 45 664 -> 666).
+__device__ __forceinline__ int2 xcd_place(const int4* __restrict__ tiles, bool runs) {
+  if (!runs) return {(int)blockIdx.x, (int)blockIdx.y};
+  const int4 last = tiles[gridDim.y - 1];
+  const int n = gridDim.x, all = (last.x < 0 ? last.w : (int)gridDim.y) * n, b = blockIdx.y * n + blockIdx.x;
+  if (b >= all) return {0, -1};
+  const int xcd = b & 7, q = all >> 3, r = all & 7, id = xcd * q + min(xcd, r) + (b >> 3), t = id / n;
+  return {id - t * n, t};
+}
+
 // 16-byte piece `chunk` of a 128-byte row in LDS: 16 rows' pieces in all banks
 __device__ __forceinline__ int mswz(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
 
@@ -567,13 +582,15 @@ template <int BM, int BN, int NST, int WM>
 __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16* __restrict__ A, int64_t lda, const int* __restrict__ sorted_ids,
                                                          int gather_div, const bf16* __restrict__ W, const int4* __restrict__ tiles,
                                                          int N, int K, bf16* __restrict__ out, int64_t ldo,
-                                                         const bf16* __restrict__ bias) {
+                                                         const bf16* __restrict__ bias, bool runs) {
   constexpr int AB = BM * 128, STG = AB + BN * 128;             // a stage: 64 k of BM rows and of BN weight rows
   constexpr int WN = 4 / WM, MJ = BM / 16 / WM, NI = BN / 16 / WN;   // waves, 16 x 16 blocks of a wave
   constexpr int AI = BM / 32, WI = BN / 32;                     // moves of 8 rows of a wave
   __shared__ __attribute__((aligned(16))) char smem[NST * STG];
-  const int4 tile = tiles[blockIdx.y];
-  const int e = tile.x, m0 = tile.y, m_end = tile.z, n0 = blockIdx.x * BN, nt = K / 64;
+  const int2 at = xcd_place(tiles, runs);
+  if (at.y < 0) return;
+  const int4 tile = tiles[at.y];
+  const int e = tile.x, m0 = tile.y, m_end = tile.z, n0 = at.x * BN, nt = K / 64;
   if (e < 0) return;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   int srow[AI];
@@ -660,16 +677,16 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16* __restrict_
   }
 }
 
-// tiles: of 64 rows (ome_moe_align_tiles); A, W 16-byte aligned, lda % 8 == 0, K % 64 == 0
+// tiles: of 64 rows (ome_moe_align_tiles); A, W 16-byte aligned, lda % 8 == 0, K % 64 == 0.  runs: xcd_place
 OME_API int ome_moe_gemm_stream(const void* A, int64_t lda, const int* sorted_ids, int gather_div, const void* W, const int* tiles,
-                                int N, int K, int max_tiles, void* out, int64_t ldo, const void* bias, hipStream_t stream) {
+                                int N, int K, int max_tiles, void* out, int64_t ldo, const void* bias, int runs, hipStream_t stream) {
   if (max_tiles <= 0) return 0;
   if (N <= 0 || K <= 0 || K % 64 || lda % 8 || ((uintptr_t)A | (uintptr_t)W | (uintptr_t)tiles) % 16 || (uintptr_t)out % 8) return -2;
   if (max_tiles > 65535) return -3;
   const dim3 grid((N + 63) / 64, max_tiles);
   // up to two workgroups a CU: one stage more out (8 experts, 1 row: 201 -> 182 us; more of them: 398 -> 413 at 8 rows, three fit a CU)
 #define ST(NST) moe_stream_kernel<64, 64, NST, 2><<<grid, 256, 0, stream>>>((const bf16*)A, lda, sorted_ids, gather_div, (const bf16*)W, \
-    (const int4*)tiles, N, K, (bf16*)out, ldo, (const bf16*)bias)
+    (const int4*)tiles, N, K, (bf16*)out, ldo, (const bf16*)bias, runs != 0)
   if ((int64_t)grid.x * max_tiles <= 512) ST(4);
   else ST(3);
 #undef ST

@@ -892,8 +892,9 @@ def _moe_gemm(x: torch.Tensor, s: _Sorted, ids: int | None, div: int, w: torch.T
         # (rows that start on no 16-byte boundary: a copy of them for the streamed tiles.  Whole layers, us, tiles that search -> this: 128 experts with 70
         # rows 670 -> 627, 8 experts with 100 647 -> 558, 512 with 48 470 -> 358)
         x = x.clone(memory_format=torch.contiguous_format) if x.data_ptr() % 16 else x
+        runs = -(-N // 64) % 8 == 0 and rows <= 32 * E   # (measured beside xcd_place in moe.hip)
         call("ome_moe_gemm_stream", x.data_ptr(), x.stride(0), ids, div, w.data_ptr(), s.tiles, N, K, s.max_tiles,
-             out.data_ptr(), out.stride(0), ptr(bias), stream_ptr())
+             out.data_ptr(), out.stride(0), ptr(bias), int(runs), stream_ptr())
     else:
         call("ome_moe_gemm", x.data_ptr(), x.stride(0), ids, div, w.data_ptr(), s.offsets, E, N, K, -(-rows // tm) + E,
              out.data_ptr(), out.stride(0), ptr(bias), tm, stream_ptr())

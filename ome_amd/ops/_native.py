@@ -117,7 +117,7 @@ _SIGNATURES = {
         "ome_mla_attn": [vp, i64, vp, vp, i32, i32, vp, vp, i32, i32, i32, i32, f32, i32, i32, vp, vp, i64, vp, vp, vp],
         "ome_moe_align": [vp, i32, i32, vp, vp, vp, vp],
         "ome_moe_align_tiles": [vp, i32, i32, vp, vp, vp, vp, i32, i32, i32, vp],
-        "ome_moe_gemm_stream": [vp, i64, vp, i32, vp, vp, i32, i32, i32, vp, i64, vp, vp],
+        "ome_moe_gemm_stream": [vp, i64, vp, i32, vp, vp, i32, i32, i32, vp, i64, vp, i32, vp],
         "ome_moe_gemm": [vp, i64, vp, i32, vp, vp, i32, i32, i32, i32, vp, i64, vp, i32, vp],
         "ome_moe_gemm_pp": [vp, i64, i32, vp, i32, vp, vp, i32, i32, i32, i32, vp, i64, vp, i32, i32, vp],
         "ome_moe_gemm_fp8_tile": [vp, i64, vp, vp, i32, vp, vp, vp, i32, i32, i32, i32, vp, i64, vp],

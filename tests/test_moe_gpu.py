@@ -189,6 +189,16 @@ def test_streamed_experts_at_tile_edges(counts, N, K, gather):
     assert torch.allclose(got.double(), want, rtol=2.0 ** -8, atol=2.0 ** -24 * K * 8)
 
 
+@pytest.mark.parametrize("counts", [[1], [1] * 9, [2] * 13, [0, 63, 1, 0] + [0] * 3, [0] * 30 + [31] * 12 + [65], [5] * 40], ids=str)
+@pytest.mark.parametrize("N,K", [(512, 64), (500, 128), (1024, 320), (24576, 64)])
+def test_streamed_experts_in_runs(monkeypatch, counts, N, K):
+    """An XCD's workgroups take a run of the tiles: as many tiles as there may be and fewer, fewer than XCDs, a multiple of 8 workgroups and not."""
+    runs, call = [], ops.call
+    monkeypatch.setattr(ops, "call", lambda fn, *a: (runs.append(a[-2]) if fn == "ome_moe_gemm_stream" else None, call(fn, *a)))
+    test_streamed_experts_at_tile_edges(counts, N, K, True)
+    assert runs == [1]
+
+
 @pytest.mark.parametrize("counts,N,K", [([1, 0, 2, 1], 1024, 512), ([1, 1], 4096, 14336), ([1] * 6, 2688, 1856), ([0, 64, 3], 64, 128)], ids=str)
 @pytest.mark.parametrize("gather", [True, False])
 def test_streamed_experts_out_of_memory(counts, N, K, gather):
