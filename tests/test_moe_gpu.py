@@ -156,6 +156,13 @@ def test_moe_align_offsets(E, n):
     assert torch.equal(srt[inv.long()].cpu(), torch.arange(n, dtype=torch.int32))
 
 
+@pytest.mark.parametrize("E", [1, 512])
+@pytest.mark.parametrize("n", [3072, 3073, 8192, 8193, 32768, 32769])
+def test_moe_align_of_many(E, n):
+    """Assignments that threads keep, to the last of eight at a time and of 32 in all, and one more."""
+    test_moe_align_offsets(E, n)
+
+
 @pytest.mark.parametrize("E,e_tiles", [(1, 1), (64, 64), (300, 299), (1025, 1025)])
 @pytest.mark.parametrize("n,bm", [(1, 64), (65, 64), (5000, 64), (5000, 128)])
 def test_moe_align_tiles(E, e_tiles, n, bm):
