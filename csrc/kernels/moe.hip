@@ -622,6 +622,22 @@ __device__ __forceinline__ int2 xcd_place(const int4* __restrict__ tiles, bool r
   return {id - t * n, t};
 }
 
+// Whether tile t is its expert's only one (of `bm` rows): its weights are read once, so they come with the non-temporal policy, and what is read again (rows,
+// the weights of experts with more tiles) stays in the caches.  Whole layers, us: 512 experts of 2048 x 512, 48, 256 and 1000 rows 310 -> 281 (6.9 TB/s), 541 ->
+// 490, 636 -> 612; 8 of 4096 x 14336, 4, 16 and 128 rows 330 -> 296, 427 -> 386 (7.3 TB/s), 552 -> 509; 128 of 2688 x 1856, 128 and 400 rows 343 -> 315, 415 ->
+// 395; 256 fp8 experts of 7168 x 2048, 16, 128 and 700 rows 577 -> 529, 1303 -> 1210, 1768 -> 1731.  With this policy for experts of more tiles too: 600 rows of
+// 128 experts 485 -> 522, 2200 of 512 770 -> 820.  The policy is a constant of a move, so the loop stands twice: a branch at each move cost
+// few workgroups up to 15%.
+__device__ __forceinline__ bool only_tile(const int4* __restrict__ tiles, int t, const int4& tile, int bm) {
+  return tile.z - tile.y <= bm && (t == 0 || tiles[t - 1].x != tile.x);
+}
+using KeptWeights = std::integral_constant<int, 0>;
+using ReadOnce = std::integral_constant<int, 2>;
+template <int POLICY>
+__device__ __forceinline__ void weights_to_lds(const void* src, char* lds, std::integral_constant<int, POLICY>) {
+  __builtin_amdgcn_global_load_lds((moe_glb_t*)src, (moe_lds_t*)lds, 16, 0, POLICY);
+}
+
 // 16-byte piece `chunk` of a 128-byte row in LDS: 16 rows' pieces in all banks
 __device__ __forceinline__ int mswz(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
 
@@ -638,6 +654,7 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16* __restrict_
   if (at.y < 0) return;
   const int4 tile = tiles[at.y];
   const int e = tile.x, m0 = tile.y, m_end = tile.z, n0 = at.x * BN, nt = K / 64;
+  const bool once = __builtin_amdgcn_readfirstlane(only_tile(tiles, at.y, tile, BM));
   if (e < 0) return;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   int srow[AI];
@@ -660,10 +677,10 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16* __restrict_
     const int r = (wave * AI + j) * 8 + (lane >> 3);
     asrc[j] = A + (int64_t)(gather_div > 0 ? srow[j] / gather_div : srow[j]) * lda + mswz(r, lane & 7) * 8;
   }
-  const auto stage = [&](int buf, int kt) {
+  const auto stage = [&](int buf, int kt, auto policy) {
 #pragma unroll
     for (int j = 0; j < WI; ++j)
-      __builtin_amdgcn_global_load_lds((moe_glb_t*)(wsrc[j] + kt * 64), (moe_lds_t*)(smem + buf * STG + AB + (wave * WI + j) * 1024), 16, 0, 0);
+      weights_to_lds(wsrc[j] + kt * 64, smem + buf * STG + AB + (wave * WI + j) * 1024, policy);
 #pragma unroll
     for (int j = 0; j < AI; ++j)
       __builtin_amdgcn_global_load_lds((moe_glb_t*)(asrc[j] + kt * 64), (moe_lds_t*)(smem + buf * STG + (wave * AI + j) * 1024), 16, 0, 0);
@@ -700,7 +717,8 @@ __global__ __launch_bounds__(256) void moe_stream_kernel(const bf16* __restrict_
       }
     }
   };
-  lds_stages<NST, AI + WI>(nt, stage, landed, multiply);
+  if (once) lds_stages<NST, AI + WI>(nt, [&](int buf, int kt) { stage(buf, kt, ReadOnce{}); }, landed, multiply);
+  else lds_stages<NST, AI + WI>(nt, [&](int buf, int kt) { stage(buf, kt, KeptWeights{}); }, landed, multiply);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the copies of the last block past the end
 #pragma unroll
   for (int j = 0; j < MJ; ++j) {
@@ -893,6 +911,7 @@ __global__ __launch_bounds__(256) void moe_gemm_fp8_kernel(const uint8_t* __rest
   const int4 tile = tiles[blockIdx.y];
   const int e = tile.x, m0 = tile.y, m_end = tile.z;
   if (e < 0) return;
+  const bool once = __builtin_amdgcn_readfirstlane(only_tile(tiles, blockIdx.y, tile, BMF));
   const int n0 = blockIdx.x * BNF;
   const int KB = K / 128, nt = KB;
   const uint8_t* We = W + (int64_t)e * N * K;
@@ -922,7 +941,7 @@ __global__ __launch_bounds__(256) void moe_gemm_fp8_kernel(const uint8_t* __rest
     p = p < m_end ? p : m_end - 1;
     scsrc = sa + (int64_t)(gather_div > 0 ? sorted_ids[p] / gather_div : p) * (K / 128);
   }
-  auto stage = [&](int buf, int kt) {
+  const auto stage_by = [&](int buf, int kt, auto policy) {
     char* la = smem + buf * STG;
     char* lw = la + ABYTES;
     if constexpr (NST == 3)
@@ -933,8 +952,7 @@ __global__ __launch_bounds__(256) void moe_gemm_fp8_kernel(const uint8_t* __rest
                                        0, 0);
 #pragma unroll
     for (int j = 0; j < WI; ++j)
-      __builtin_amdgcn_global_load_lds((moe_glb_t*)(wsrc[j] + kt * 128), (moe_lds_t*)(lw + (wave * WI + j) * 1024), 16,
-                                       0, 0);
+      weights_to_lds(wsrc[j] + kt * 128, lw + (wave * WI + j) * 1024, policy);
   };
   const int wm = wave >> 1, wn = wave & 1;   // wave tile: rows [wm*BMF/2, +BMF/2), cols [wn*BNF/2, +BNF/2)
   constexpr int MJ = BMF / 32, NI = BNF / 32;
@@ -965,67 +983,71 @@ __global__ __launch_bounds__(256) void moe_gemm_fp8_kernel(const uint8_t* __rest
     swn = swe[0];
   }
   constexpr int NL = AI + WI + (NST == 3);   // LDS-DMA instructions per thread per K block
-  if constexpr (NST == 2) {
-    stage(0, 0);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-  } else {
-    // blocks 0 and 1 in flight; the top of step t waits for block t with block t + 1 still out
-    stage(0, 0);
-    stage(1, min(1, nt - 1));
-  }
-  for (int t = 0; t < nt; ++t) {
-    const int cur = NST == 2 ? (t & 1) : t % 3;
-    if constexpr (NST == 3) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL) : "memory");   // block t + 1 (maybe a clamped copy) stays out
-      __builtin_amdgcn_s_barrier();   // every wave's block t landed; every wave done reading block t - 1
-    }
-    float s[MJ];
-    if constexpr (NST == 3) {
-      const char* lsc = smem + cur * STG + ABYTES + WBYTES;
-      const float swv = swe[t];
-#pragma unroll
-      for (int j = 0; j < MJ; ++j) {
-        const int r = wm * (BMF / 2) + j * 16 + fr;
-        s[j] = *reinterpret_cast<const float*>(lsc + (r / (BMF / 4)) * 256 + (r % (BMF / 4)) * 4) * swv;
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < MJ; ++j) s[j] = san[j] * swn;
-    }
+  const auto run = [&](const auto& stage) __attribute__((always_inline)) {
     if constexpr (NST == 2) {
-      if (t + 1 < nt) {
-#pragma unroll
-        for (int j = 0; j < MJ; ++j) san[j] = sar[j][t + 1];
-        swn = swe[t + 1];
-        stage(cur ^ 1, t + 1);
-      }
-    } else {
-      // branch-free: the DMA of block t + 2 (into the buffer block t - 1 left) is issued every
-      // step, clamped to the last block past the end, so the counted wait above stays exact
-      stage((t + 2) % 3, min(t + 2, nt - 1));
-    }
-    const char* la = smem + cur * STG;
-    const char* lw = la + ABYTES;
-    mi32x8 xa[MJ];
-#pragma unroll
-    for (int j = 0; j < MJ; ++j) xa[j] = mfrag32(la, wm * (BMF / 2) + j * 16 + fr, fc);
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const mi32x8 wf = mfrag32(lw, wn * (BNF / 2) + i * 16 + fr, fc);
-#pragma unroll
-      for (int j = 0; j < MJ; ++j) {
-        const f32x4 p = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, xa[j], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0,
-                                                                        127, 0, 127);
-        acc[i][j] += p * s[j];
-      }
-    }
-    if constexpr (NST == 2) {
+      stage(0, 0);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
+    } else {
+      // blocks 0 and 1 in flight; the top of step t waits for block t with block t + 1 still out
+      stage(0, 0);
+      stage(1, min(1, nt - 1));
     }
-  }
-  if constexpr (NST == 3) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // clamped tail DMA retires before exit
+    for (int t = 0; t < nt; ++t) {
+      const int cur = NST == 2 ? (t & 1) : t % 3;
+      if constexpr (NST == 3) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL) : "memory");   // block t + 1 (maybe a clamped copy) stays out
+        __builtin_amdgcn_s_barrier();   // every wave's block t landed; every wave done reading block t - 1
+      }
+      float s[MJ];
+      if constexpr (NST == 3) {
+        const char* lsc = smem + cur * STG + ABYTES + WBYTES;
+        const float swv = swe[t];
+#pragma unroll
+        for (int j = 0; j < MJ; ++j) {
+          const int r = wm * (BMF / 2) + j * 16 + fr;
+          s[j] = *reinterpret_cast<const float*>(lsc + (r / (BMF / 4)) * 256 + (r % (BMF / 4)) * 4) * swv;
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < MJ; ++j) s[j] = san[j] * swn;
+      }
+      if constexpr (NST == 2) {
+        if (t + 1 < nt) {
+#pragma unroll
+          for (int j = 0; j < MJ; ++j) san[j] = sar[j][t + 1];
+          swn = swe[t + 1];
+          stage(cur ^ 1, t + 1);
+        }
+      } else {
+        // branch-free: the DMA of block t + 2 (into the buffer block t - 1 left) is issued every
+        // step, clamped to the last block past the end, so the counted wait above stays exact
+        stage((t + 2) % 3, min(t + 2, nt - 1));
+      }
+      const char* la = smem + cur * STG;
+      const char* lw = la + ABYTES;
+      mi32x8 xa[MJ];
+#pragma unroll
+      for (int j = 0; j < MJ; ++j) xa[j] = mfrag32(la, wm * (BMF / 2) + j * 16 + fr, fc);
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const mi32x8 wf = mfrag32(lw, wn * (BNF / 2) + i * 16 + fr, fc);
+#pragma unroll
+        for (int j = 0; j < MJ; ++j) {
+          const f32x4 p = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, xa[j], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0,
+                                                                          127, 0, 127);
+          acc[i][j] += p * s[j];
+        }
+      }
+      if constexpr (NST == 2) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+      }
+    }
+    if constexpr (NST == 3) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // clamped tail DMA retires before exit
+  };
+  if (once) run([&](int buf, int kt) { stage_by(buf, kt, ReadOnce{}); });
+  else run([&](int buf, int kt) { stage_by(buf, kt, KeptWeights{}); });
   // lane (fr, fc) of block (i, j): row p = m0 + wm*BMF/2 + j*16 + fr, cols n = n0 + wn*BNF/2 + i*16 + 4fc .. +3
 #pragma unroll
   for (int j = 0; j < MJ; ++j) {
