@@ -64,6 +64,10 @@ __device__ __forceinline__ int weight_row(int n0, int r, int N, int D) {
   return p / half * D + p % half + up * half;
 }
 
+// Weights are read once, so they come with the non-temporal policy and leave the rows in the caches: QKV of one row 14.0 -> 13.7 us, 4096 x 4096 9.5 ->
+// 9.4, a whole step of one request 3342 -> 3231 (two runs of one side differ by 2%).
+__device__ __forceinline__ bf16x8 ld8_once(const bf16* p) { return __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p)); }
+
 template <int M, int R, int U, bool ACT = false, int EPI = PLAIN, int F = KV_BF16>   // U: K steps in flight (fewer for more rows: VGPR budget)
 __global__ __launch_bounds__(256) void gemv_kernel(const bf16* __restrict__ X, int64_t ldx, const bf16* __restrict__ W,
                                                    const bf16* __restrict__ bias, bf16* __restrict__ out, int64_t ldo,
@@ -104,7 +108,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(const bf16* __restrict__ X, i
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int r = 0; r < R; ++r) w[u][r] = ld8(wr[r] + k + 512 * u);
+      for (int r = 0; r < R; ++r) w[u][r] = ld8_once(wr[r] + k + 512 * u);
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -119,7 +123,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(const bf16* __restrict__ X, i
   for (; k < K; k += 512) {
     bf16x8 w[R], x[M];
 #pragma unroll
-    for (int r = 0; r < R; ++r) w[r] = ld8(wr[r] + k);
+    for (int r = 0; r < R; ++r) w[r] = ld8_once(wr[r] + k);
 #pragma unroll
     for (int m = 0; m < M; ++m) x[m] = ldx8<ACT>(X + m * ldx + k, K);
 #pragma unroll
