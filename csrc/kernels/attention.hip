@@ -162,9 +162,12 @@ __device__ __forceinline__ bf16x4 v4_bf16(const typename KVRaw<F>::V4& x) {
   if constexpr (F == KV_BF16) return x;
   else return fp8x4_to_bf16<F>(x);
 }
-template <int F>
+template <int F, bool ONCE = false>   // ONCE: with the non-temporal policy
 __device__ __forceinline__ typename KVRaw<F>::K8 k8_load(const typename KVStore<F>::T* p) {
-  return *reinterpret_cast<const typename KVRaw<F>::K8*>(p);
+  using K8 = typename KVRaw<F>::K8;
+  typedef uint32_t words __attribute__((ext_vector_type(sizeof(K8) / 4)));
+  if constexpr (ONCE) return __builtin_bit_cast(K8, __builtin_nontemporal_load(reinterpret_cast<const words*>(p)));
+  else return *reinterpret_cast<const K8*>(p);
 }
 template <int F>
 __device__ __forceinline__ typename KVRaw<F>::V4 v4_load(const typename KVStore<F>::T* p) {
@@ -468,7 +471,7 @@ struct KVTileP {
   typename KVRaw<F>::K8 v[D / 16];
 };
 
-template <int D, int P, int F>
+template <int D, int P, int F, bool ONCE = false>
 __device__ __forceinline__ void kv_tilep_load(KVTileP<D, F>& t, const typename KVStore<F>::T* __restrict__ k_cache,
                                               const typename KVStore<F>::T* __restrict__ v_cache,
                                               const int* __restrict__ bt, int kb, int seq_len, int64_t kpage, int kvh,
@@ -481,11 +484,11 @@ __device__ __forceinline__ void kv_tilep_load(KVTileP<D, F>& t, const typename K
   const typename KVStore<F>::T* vp = v_cache + ((g >> 1) ? pB : pA) * kpage + (int64_t)kvh * D * P + 8 * (g & 1);
 #pragma unroll
   for (int ks = 0; ks < D / 32; ++ks) {
-    t.ka[ks] = k8_load<F>(k0 + 32 * ks + 8 * g);
-    t.kb[ks] = k8_load<F>(k1 + 32 * ks + 8 * g);
+    t.ka[ks] = k8_load<F, ONCE>(k0 + 32 * ks + 8 * g);
+    t.kb[ks] = k8_load<F, ONCE>(k1 + 32 * ks + 8 * g);
   }
 #pragma unroll
-  for (int nb = 0; nb < D / 16; ++nb) t.v[nb] = k8_load<F>(vp + (16 * nb + n) * P);
+  for (int nb = 0; nb < D / 16; ++nb) t.v[nb] = k8_load<F, ONCE>(vp + (16 * nb + n) * P);
 }
 
 template <int D, int F, bool AL = false>
@@ -533,7 +536,7 @@ __device__ __forceinline__ void kv_tilep_compute(const KVTileP<D, F>& t, const b
   }
 }
 
-template <int D, int P, int MODE, int F, bool AL = false>
+template <int D, int P, int MODE, int F, bool AL = false, bool ONCE = false>
 __global__ __launch_bounds__(256) void paged_decode_v2_kernel(
     const bf16* __restrict__ q, int64_t q_stride, const typename KVStore<F>::T* __restrict__ k_cache,
     const typename KVStore<F>::T* __restrict__ v_cache, const int* __restrict__ block_tables, int bt_stride,
@@ -586,7 +589,7 @@ __global__ __launch_bounds__(256) void paged_decode_v2_kernel(
       if (AL && scl.bs_shift && scl.bs_skip && !scl.bs_stage_needed(kb, 32, qb, kvh * G, G)) continue;
       if (AL && kb >= scl.keep && kb + 32 <= lo) continue;   // between the kept keys and the window
       KVTileP<D, F> t;
-      kv_tilep_load<D, P, F>(t, k_cache, v_cache, bt, kb, seq_len, kpage, kvh, n, g);
+      kv_tilep_load<D, P, F, ONCE>(t, k_cache, v_cache, bt, kb, seq_len, kpage, kvh, n, g);
       kv_tilep_compute<D, F, AL>(t, qf, o, m_i, l_i, kb, p_end, lo, scl, g, al, qpos, kvh * G + n);
     }
   } else if (MODE == 0) {
@@ -655,16 +658,23 @@ __global__ __launch_bounds__(256) void paged_decode_v2_kernel(
   }
 }
 
+// Rows of a step from which a bf16 cache, which is read once, comes with the non-temporal policy.  us, 8 heads of 128, 256 rows of ~630 keys 127.7 -> 122.4 (in
+// Llama-3-8B's step 134.4 -> 125.2), of ~300 66.1 -> 62.6, 128 of ~1500 153.4 -> 150.0, 64 of ~300 22.7 -> 21.9; 16 of ~500 14.8 either way (15.0 -> 16.1 in the
+// step).  A lane's 8 bytes of an 8-bit cache ask for a line sixteen times: 256 of ~630 84 -> 94.
+constexpr int DECODE_ONCE_ROWS = 64;
+
 template <int D, int F>
 static void launch_decode_v2(int variant, dim3 grid, size_t smem, hipStream_t stream, const void* q,
                              int64_t q_stride, const void* k_cache, const void* v_cache, const int* block_tables,
                              int bt_stride, const int* seq_lens, void* out, int64_t out_stride, void* part_o,
                              void* part_ml, int Hq, int Hkv, int part_size, int max_parts, Scaler scl,
                              int window, const int* order, float v_scale, const float* sinks) {
+  constexpr bool BF = F == KV_BF16;
   // ALiBi (Bloom / MPT) runs the key-permuted variant only, compiled with the bias term; the
   // other instantiations carry no trace of it
   auto kern = (scl.alibi != nullptr || scl.bs_shift != 0 || scl.keep > 0) ? paged_decode_v2_kernel<D, 16, 2, F, true>
               : variant == 2       ? paged_decode_v2_kernel<D, 16, 1, F>
+              : variant == 4 && BF && grid.z >= DECODE_ONCE_ROWS ? paged_decode_v2_kernel<D, 16, 2, F, false, BF>
               : variant == 4       ? paged_decode_v2_kernel<D, 16, 2, F>
                                    : paged_decode_v2_kernel<D, 16, 0, F>;
   kern<<<grid, 256, smem, stream>>>((const bf16*)q, q_stride, (const typename KVStore<F>::T*)k_cache,

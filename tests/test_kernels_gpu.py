@@ -126,6 +126,20 @@ def test_paged_decode(Hq, Hkv, seq_lens, part_size, variant, monkeypatch):
         _close(ops.paged_decode(q, kc, vc, bt, sl, scale, ws, order=order), expect, atol=2e-2)
 
 
+@pytest.mark.parametrize("rows", [64, 65, 200])
+@pytest.mark.parametrize("D,window", [(64, -1), (128, 100), (128, -1), (256, -1)])
+def test_paged_decode_of_many_rows_is_that_of_few(rows, D, window):
+    """From 64 rows on the cache is read with another policy: the same bits."""
+    torch.manual_seed(rows)
+    lens = [[1, 16, 17, 40, 300, 129][i % 6] for i in range(rows)]
+    npages = sum(-(-n // 16) for n in lens) + 8
+    kc, vc = _cache(npages, 8, D)
+    bt, sl = _block_tables(lens, 16, npages), torch.tensor(lens, dtype=torch.int32, device=DEV)
+    q = torch.randn(rows, 32, D, device=DEV, dtype=torch.bfloat16)
+    run = lambda a, b: ops.paged_decode(q[a:b], kc, vc, bt[a:b], sl[a:b], 0.09, ops.DecodeWorkspace(b - a, 32, D, 512, 256, DEV), window)   # noqa: E731
+    assert torch.equal(run(0, rows), torch.cat([run(a, min(a + 63, rows)) for a in range(0, rows, 63)]))
+
+
 @pytest.mark.parametrize("window", [128, -256, -64])  # sliding; chunked (Llama 4) as window < -1
 @pytest.mark.parametrize("variant", ["1", "2", "3", "4"])
 def test_paged_decode_window(variant, window, monkeypatch):
