@@ -779,11 +779,12 @@ def moe_tile_m(rows: int, E: int, N: int) -> int:
     return 64
 
 
-#: average rows per expert from which the 256-row ping-pong tiles run (:func:`_moe_pp`): where experts begin to need a second
-#: 64-row tile.  Whole layer, 64 / 128-row tiles -> these, us: Mixtral 40 rows 603 -> 642, 45 615 -> 671, 48 702 -> 695, 55 760 -> 696, 75
-#: 756 -> 709, 125 1093 -> 744; Nemotron-3-Nano (widths 2688 / 1856) 42 578 -> 588, 47 602 -> 597, 61 684 -> 628; Qwen3-Next (512
-#: experts) 20 661 -> 659, 39 754 -> 730, 59 860 -> 785.
-MOE_PP_ROWS = 46
+#: average rows per expert from which the 256-row ping-pong tiles run (:func:`_moe_pp`): where experts begin to need a second 64-row
+#: tile, and sooner where SiLU(gate) * up goes with the first product.  Whole layer, 64-row tiles -> these, us: Nemotron-3-Nano (widths 2688 / 1856, no
+#: gate) 33 rows 502 -> 517, 38 518 -> 527, 42 535 -> 534, 61 684 -> 628; Mixtral 32 508 -> 536, 36 542 -> 537, 40 553 -> 539, 44 570 -> 543, 75 756 -> 709;
+#: Qwen3-Next (512 experts) 29 675 -> 689, 35 724 -> 709, 39 744 -> 713, 43 768 -> 722.
+MOE_PP_ROWS = 43
+MOE_PP_ROWS_SILU = 35
 
 
 class _Sorted:
@@ -819,12 +820,12 @@ def moe_splits(rows: int, E: int, N: int, K: int) -> int:
 
 
 def _moe_pp(x: torch.Tensor, ids: int | None, div: int, w: torch.Tensor, offsets: int, rows: int,
-            bias: torch.Tensor | None, silu: bool, splits: int = 1) -> torch.Tensor | None:
+            bias: torch.Tensor | None, silu: bool, splits: int = 1, least: int | None = None) -> torch.Tensor | None:
     """Grouped GEMM on 256-row tiles (``ome_moe_gemm_pp``; ``silu``: SiLU(gate) * up applied to the accumulators; ``splits``: K in
-    as many pieces, fp32 [splits, rows, N]),
+    as many pieces, fp32 [splits, rows, N]; ``least``: rows an expert from which they run),
     or None where the 64 / 128-row tiles run: experts with few rows, shapes the tiles do not take, ``OME_MOE_TILE``."""
     E, N, K = w.shape
-    if rows < MOE_PP_ROWS * E or os.environ.get("OME_MOE_TILE") or K % 64 or N % (32 if silu else 4) or (silu and bias is not None) or \
+    if rows < (MOE_PP_ROWS if least is None else least) * E or os.environ.get("OME_MOE_TILE") or K % 64 or N % (32 if silu else 4) or (silu and bias is not None) or \
             x.stride(0) % 8 or x.stride(1) != 1 or (x.data_ptr() | w.data_ptr()) % 16 or not w.is_contiguous() or \
             x.shape[0] * x.stride(0) >= 1 << 30 or N * K >= 1 << 30:
         return None
@@ -869,13 +870,14 @@ def fused_moe(x: torch.Tensor, topk_w: torch.Tensor, topk_ids: torch.Tensor, w13
     dev = x.device
     s = _Sorted(topk_ids, E, 64)
     fused = gated and act == 0 and b13 is None
-    h = _moe_pp(x, s.ids, k, w13, s.offsets, n, b13, fused)
+    least = min(MOE_PP_ROWS, MOE_PP_ROWS_SILU) if fused else MOE_PP_ROWS
+    h = _moe_pp(x, s.ids, k, w13, s.offsets, n, b13, fused, least=least)
     if h is None:
         fused = False
         h = _moe_gemm(x, s, s.ids, k, w13, n, b13)
     if not fused:
         h = act_and_mul(h, act, limit=limit) if gated else _act_inplace(h, act)
-    y = _moe_pp(h, None, 1, w2, s.offsets, n, b2, False, moe_splits(n, E, H, I) if b2 is None else 1)
+    y = _moe_pp(h, None, 1, w2, s.offsets, n, b2, False, moe_splits(n, E, H, I) if b2 is None else 1, least)
     if y is None:
         y = _moe_gemm(h, s, None, 0, w2, n, b2)
     return _combine(y, topk_w, s.inv, T, k, H, scale, add)
