@@ -212,6 +212,79 @@ __global__ __launch_bounds__(256) void mla_attn_kernel(
   }
 }
 
+// Sums of the lanes up to and with each (a row's lanes shifted, then the rows' last lanes broadcast), without LDS: a step of a __shfl is a round trip
+__device__ __forceinline__ int wave_scan(int x) {
+#define MLA_STEP(CTRL, ROWS) x += __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, true)
+  MLA_STEP(0x111, 0xf);   // row_shr 1, 2, 4, 8
+  MLA_STEP(0x112, 0xf);
+  MLA_STEP(0x114, 0xf);
+  MLA_STEP(0x118, 0xf);
+  MLA_STEP(0x142, 0xa);   // row_bcast 15, 31
+  MLA_STEP(0x143, 0xc);
+#undef MLA_STEP
+  return x;
+}
+__device__ __forceinline__ int wave_total(int x) { return __builtin_amdgcn_readlane(wave_scan(x), 63); }
+__device__ __forceinline__ int wave_most(int x) {   // the largest
+#define MLA_STEP(CTRL, ROWS) x = max(x, __builtin_amdgcn_update_dpp(x, x, CTRL, ROWS, 0xf, false))
+  MLA_STEP(0x111, 0xf);
+  MLA_STEP(0x112, 0xf);
+  MLA_STEP(0x114, 0xf);
+  MLA_STEP(0x118, 0xf);
+  MLA_STEP(0x142, 0xa);
+  MLA_STEP(0x143, 0xc);
+#undef MLA_STEP
+  return __builtin_amdgcn_readlane(x, 63);
+}
+
+// A decode step's units (a token's tiles of heads, HG of them) in at most 256 pieces: workgroup w takes piece w.  The span is the smallest number of key tiles that cuts all units
+// into at most 256 pieces: one a CU (also within each XCD, to which workgroups go in turn), and none longer
+// than it has to be, however ragged the contexts.  Every wave finds it from the lengths: lane l holds
+// tokens 4 l .. 4 l + 3.
+// (unit, and its piece `part` of `my_parts`); false: there is none.
+constexpr int SPAN = 2, UNITS = 256;
+__device__ __forceinline__ bool decode_piece(const int* __restrict__ kv_lens, int T, int H, int HG, int parts, int& unit, int& part, int& my_parts) {
+  const int lane = threadIdx.x & 63;
+  int nt4[4], most = SPAN, all = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int tk = 4 * lane + i;
+    nt4[i] = tk < T ? (kv_lens[tk] + KT - 1) / KT : 0;
+    most = max(most, nt4[i]);
+    all += nt4[i];
+  }
+  auto count = [&](int span, int i) {   // (a quotient of tiles is off by one at most)
+    const int n = nt4[i] + span - 1, about = (int)((float)n * __builtin_amdgcn_rcpf((float)span)), rest = n - about * span;
+    return 4 * lane + i < T ? min(parts, max(1, about + (rest >= span) - (rest < 0))) : 0;
+  };
+  auto pieces = [&](int span) { return wave_total(count(span, 0) + count(span, 1) + count(span, 2) + count(span, 3)) * HG; };
+  most = wave_most(most);
+  all = wave_total(all) * HG;
+  // all / span <= pieces <= all / span + units; one piece a unit is at most 256 (the caller's rule)
+  int lo = max(SPAN, min(most, all / UNITS)), hi = T * HG < UNITS ? max(lo, min(most, all / (UNITS - T * HG) + 1)) : most;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (pieces(mid) <= UNITS) hi = mid;
+    else lo = mid + 1;
+  }
+  // pieces that save fewer key tiles than their partials' way to memory and back costs: none (64 heads, 128 rows of ~100
+  // keys 34 -> 28 us)
+  if (most - lo <= 2 + T * H / 2048) lo = most;
+  const int w = blockIdx.x, c0 = count(lo, 0), c1 = count(lo, 1), c2 = count(lo, 2), c3 = count(lo, 3);
+  const int incl = wave_scan(c0 + c1 + c2 + c3);
+  if (w >= __builtin_amdgcn_readlane(incl, 63) * HG) return false;
+  const int at = __popcll(__ballot(incl * HG <= w));            // the lane whose tokens piece w belongs to
+  int tok = 4 * at, base = at ? __builtin_amdgcn_readlane(incl, at - 1) : 0;
+  my_parts = __builtin_amdgcn_readlane(c0, at);
+  if ((base + my_parts) * HG <= w) base += my_parts, ++tok, my_parts = __builtin_amdgcn_readlane(c1, at);
+  if ((base + my_parts) * HG <= w) base += my_parts, ++tok, my_parts = __builtin_amdgcn_readlane(c2, at);
+  if ((base + my_parts) * HG <= w) base += my_parts, ++tok, my_parts = __builtin_amdgcn_readlane(c3, at);
+  const int hg = (w - base * HG) / my_parts;
+  part = (w - base * HG) - hg * my_parts;
+  unit = tok * HG + hg;
+  return true;
+}
+
 // ------------------------------------------------------------------------------------------
 // Few decode rows at DeepSeek's widths: work items and partitions of mla_attn_kernel, but each of the four waves streams pages of its own, every
 // fourth of the partition's, with an online softmax of its own over all DV value dims, and the four meet in LDS at the end.  Bound by the
@@ -221,12 +294,16 @@ __global__ __launch_bounds__(256) void mla_attn_kernel(
 // 31 -> 27, 58 -> 38, 16 rows 43 -> 31, 85 -> 45, 23 rows of 400, 1000, 3000, 8000 22 -> 17, 32 -> 23, 67 -> 35, 138 -> 59; 32 heads, 12 rows of 1000 and 8000
 // 31 -> 22, 156 -> 61; 64 heads, 4 of 3000 42 -> 29; 128 heads, 2 of 3000 34 -> 25; 8 heads, 40 of 1000 34 -> 24.  At 16 workgroups and fewer over
 // 100 to 400 keys it took 0.2 to 1 us more (4 rows of 16 heads 11.7 -> 12.5, 14.0 -> 14.2; 1 of 128 over 92 pages 18.4 -> 18.9), so tables of at most 96 pages stay there.
+// PLAN: decode steps of up to 16 heads that go to 32-row tiles, in their pieces by length; there half of a tile's rows are none, and one wave's products, 2 us
+// a tile, are behind memory.  Them -> this, us: 128 rows of ~300, ~1000 and ~3000 keys 30 -> 27, 53 -> 44, 120 -> 105, 64 of 1000 33.6 -> 30.8, 32 of 8000 70 -> 60, 24
+// of 3000 36 -> 35; short contexts of few rows not (24 of 400 17.1 -> 18.6, 48 of 150 16.2 -> 16.7): from 3000 pages of tables on.  32 heads as two units 116 -> 171 (100 of
+// 4000), units' tiles dealt out in equal runs 101 -> 107.
 // ------------------------------------------------------------------------------------------
-template <int DK, int DV>
+template <int DK, int DV, bool PLAN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void mla_attn_pages_kernel(
     const bf16* __restrict__ q, int64_t q_stride_t, const bf16* __restrict__ cache,
     const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ tok_row,
-    const int* __restrict__ kv_lens, int H, float scale_log2, int parts, bf16* __restrict__ out,
+    const int* __restrict__ kv_lens, int T, int H, float scale_log2, int parts, int2* __restrict__ plan, bf16* __restrict__ out,
     int64_t out_stride_t, float* __restrict__ ws_o, float* __restrict__ ws_ml, const float* __restrict__ sinks,
     int window) {
   constexpr int CH = DK / 8, NV = DV / 16, NB = NV / 4, MOVES = 16 * CH / 64, IMG = 16 * CH * 16;
@@ -234,25 +311,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   static_assert(NV * 1024 <= 2 * IMG, "a wave's output fits its images");
   __shared__ __attribute__((aligned(16))) char sK[4 * 2 * IMG];
   __shared__ float sM[4][16], sL[4][16];
-  const int t = blockIdx.x, h0 = blockIdx.y * 16, part = blockIdx.z;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int HG = (H + 15) / 16;
+  int unit = blockIdx.x, part = PLAN ? 0 : blockIdx.z;
+  if (PLAN && parts > 1) {
+    if (!decode_piece(kv_lens, T, H, HG, parts, unit, part, parts)) return;   // whole block
+    if (part == 0 && tid == 0) plan[unit] = int2{(int)blockIdx.x, parts};
+  }
+  const int t = PLAN ? unit / HG : blockIdx.x, h0 = (PLAN ? unit - t * HG : (int)blockIdx.y) * 16;
   const int col = lane & 15, g = lane >> 4;
   const int L = __builtin_amdgcn_readfirstlane(kv_lens[t]);
   const int lo = window > 0 ? max(L - window, 0) : 0;   // sliding window: keys [lo, L) only
   const int n_pages = (L + 15) >> 4, pairs = (n_pages + 1) >> 1, pair_lo = lo / KT;   // partitions as in mla_attn_kernel
-  const int live = live_parts(pairs - pair_lo, parts), per_part = max(LEAST_PAIRS, (pairs - pair_lo + live - 1) / live);
+  const int live = PLAN ? parts : live_parts(pairs - pair_lo, parts), per_part = max(PLAN ? 0 : LEAST_PAIRS, (pairs - pair_lo + live - 1) / live);
   const int pair_begin = pair_lo + part * per_part, pair_end = min(pairs, pair_begin + per_part);
   const int p0 = 2 * pair_begin, p1 = min(2 * pair_end, n_pages);
   const int n = __builtin_amdgcn_readfirstlane(max(0, (p1 - p0 - wave + 3) >> 2));   // this wave's pages: p0 + wave, + 4, ..
   const int* bt = block_tables + (int64_t)tok_row[t] * bt_stride;
-  const int64_t ws_row = ((int64_t)t * H + h0 + col) * parts + part;
   const bool hv = h0 + col < H;
+  const int64_t ws_row = PLAN ? (int64_t)blockIdx.x * 16 + col : ((int64_t)t * H + h0 + col) * parts + part;   // (PLAN: pieces' rows one after the other)
+  bf16* const op = out + (int64_t)t * out_stride_t + (int64_t)(h0 + col) * DV + wave * (DV / 4) + 4 * g;
   if (p0 >= p1) {   // whole block: no keys (the merge reads no value of a partition whose sum is 0, and of those beyond 16 not the sum)
     if (hv && parts == 1) {
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
-        *reinterpret_cast<bf16x4*>(out + (int64_t)t * out_stride_t + (int64_t)(h0 + col) * DV + wave * (DV / 4) + 4 * g + 16 * nb) = bf16x4{};
-    } else if (hv && part < 16 && wave == 0 && g == 0) {
+      for (int nb = 0; nb < NB; ++nb) *reinterpret_cast<bf16x4*>(op + 16 * nb) = bf16x4{};
+    } else if (hv && (PLAN || part < 16) && wave == 0 && g == 0) {
       ws_ml[2 * ws_row] = OME_NEG_INF;
       ws_ml[2 * ws_row + 1] = 0.f;
     }
@@ -312,29 +395,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     const bf16* img = reinterpret_cast<const bf16*>(sK + (wave * 2 + (i & 1)) * IMG);
     // ---- S^T [16 keys x 16 heads], two chains ----
-    f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+    f32x4 sc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-    for (int s = 0; s < DK / 32; s += 2) {
-      sa = mfma16x32(*reinterpret_cast<const bf16x8*>(&img[swz<DK>(col, 4 * s + g) * 8]), qf[s], sa);
-      sb = mfma16x32(*reinterpret_cast<const bf16x8*>(&img[swz<DK>(col, 4 * s + 4 + g) * 8]), qf[s + 1], sb);
-    }
+    for (int s = 0; s < DK / 32; ++s) sc[s & 1] = mfma16x32(*reinterpret_cast<const bf16x8*>(&img[swz<DK>(col, 4 * s + g) * 8]), qf[s], sc[s & 1]);
     const int k0 = 16 * (p0 + wave + 4 * i) + 4 * g;
+    f32x4 s = sc[0] + sc[1];
     float mx = OME_NEG_INF;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      sa[e] = (k0 + e < L && k0 + e >= lo) ? (sa[e] + sb[e]) * scale_log2 : OME_NEG_INF;
-      mx = fmaxf(mx, sa[e]);
+      s[e] = (k0 + e < L && k0 + e >= lo) ? s[e] * scale_log2 : OME_NEG_INF;
+      mx = fmaxf(mx, s[e]);
     }
     mx = group4_max(mx);
     const float m_new = fmaxf(m, mx);
     const float alpha = m_new == OME_NEG_INF ? 1.f : __builtin_amdgcn_exp2f(m - m_new);
-    s16x4 pb;
+    // Weights as they are used: their rounding cancels in the quotient.  PLAN: with what rounding took from them in a second product, as the row tiles have it of
+    // weights that stand out (3% of the time; error against 64 bits 0.0017 instead of 0.0018, theirs 0.0017 to 0.0018)
+    s16x4 pb, pr;
     float ps = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float p = m_new == OME_NEG_INF ? 0.f : __builtin_amdgcn_exp2f(sa[e] - m_new);
-      ps += p;
-      pb[e] = __builtin_bit_cast(short, (bf16)p);
+      const float p = m_new == OME_NEG_INF ? 0.f : __builtin_amdgcn_exp2f(s[e] - m_new);
+      const bf16 high = (bf16)p;
+      ps += PLAN ? p : (float)high;
+      pb[e] = __builtin_bit_cast(short, high);
+      pr[e] = __builtin_bit_cast(short, (bf16)(p - (float)high));
     }
     lsum = lsum * alpha + group4_sum(ps);
     m = m_new;
@@ -344,9 +429,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     }
     // ---- O^T [DV x 16 heads] += V^T . P^T ----
 #pragma unroll
-    for (int v = 0; v < NV; ++v)
-      o[v] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
-          __builtin_bit_cast(s16x4, tr_read(img, swz<DK>(row, 2 * v + (pcol >> 1)) * 16 + (pcol & 1) * 8)), pb, o[v], 0, 0, 0);
+    for (int v = 0; v < NV; ++v) {
+      const s16x4 val = __builtin_bit_cast(s16x4, tr_read(img, swz<DK>(row, 2 * v + (pcol >> 1)) * 16 + (pcol & 1) * 8));
+      if constexpr (PLAN) o[v] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(val, pr, o[v], 0, 0, 0);
+      o[v] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(val, pb, o[v], 0, 0, 0);
+    }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the image is read)
     move(i + 2);
   }
@@ -372,8 +459,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     for (int nb = 0; nb < NB; ++nb) sum[nb] += e * so[w * WO + (wave * NB + nb) * 64 + lane];
   }
 
-  // ---- output or partials, as of mla_attn_kernel: dim = 16 nb + 4 g + i of the wave's quarter, head = col ----
-  if (sinks != nullptr && parts == 1 && hv) {
+  // ---- output or partials: dim = 16 nb + 4 g + i of the wave's quarter, head = col ----
+  if (!PLAN && sinks != nullptr && parts == 1 && hv) {
     const float sk = sinks[h0 + col] * 1.4426950408889634f;
     const float m_fin = fmaxf(m, sk), a = __builtin_amdgcn_exp2f(m - m_fin);
     lsum = lsum * a + __builtin_amdgcn_exp2f(sk - m_fin);
@@ -383,7 +470,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
   if (!hv) return;
   if (parts == 1) {
-    bf16* op = out + (int64_t)t * out_stride_t + (int64_t)(h0 + col) * DV + wave * (DV / 4) + 4 * g;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
       bf16x4 v;
@@ -451,31 +537,6 @@ __device__ __forceinline__ void mma_last(f32x16& d, bf16x8 a, bf16x8 b, const f3
 // Chunk x of key row r lies at x ^ row_swz(r): the same chunk of 16 rows, and four chunks of four, in all of the 64 banks (rows are 9 times
 // half of them wide)
 __device__ __forceinline__ int row_swz(int r) { return (r >> 1 & 1) << 2 | (r >> 2 & 1) << 1 | (r >> 3 & 1); }
-
-// Sums of the lanes up to and with each (a row's lanes shifted, then the rows' last lanes broadcast), without LDS: a step of a __shfl is a round trip
-__device__ __forceinline__ int wave_scan(int x) {
-#define MLA_STEP(CTRL, ROWS) x += __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, true)
-  MLA_STEP(0x111, 0xf);   // row_shr 1, 2, 4, 8
-  MLA_STEP(0x112, 0xf);
-  MLA_STEP(0x114, 0xf);
-  MLA_STEP(0x118, 0xf);
-  MLA_STEP(0x142, 0xa);   // row_bcast 15, 31
-  MLA_STEP(0x143, 0xc);
-#undef MLA_STEP
-  return x;
-}
-__device__ __forceinline__ int wave_total(int x) { return __builtin_amdgcn_readlane(wave_scan(x), 63); }
-__device__ __forceinline__ int wave_most(int x) {   // the largest
-#define MLA_STEP(CTRL, ROWS) x = max(x, __builtin_amdgcn_update_dpp(x, x, CTRL, ROWS, 0xf, false))
-  MLA_STEP(0x111, 0xf);
-  MLA_STEP(0x112, 0xf);
-  MLA_STEP(0x114, 0xf);
-  MLA_STEP(0x118, 0xf);
-  MLA_STEP(0x142, 0xa);
-  MLA_STEP(0x143, 0xc);
-#undef MLA_STEP
-  return __builtin_amdgcn_readlane(x, 63);
-}
 
 // First token whose block-table row is e, by a 64-way search of the whole wave; -1: none.  tok_row ascends in the
 // runtime's prompts; of rows in any other order it may miss e, the same way for every caller.
@@ -566,7 +627,7 @@ __global__ __launch_bounds__(64 * (NW + row_movers(NW))) __attribute__((amdgpu_w
   __shared__ __attribute__((aligned(16))) char sK[4 * IMG];
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)sK;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  constexpr int RT = 32 * NW, SPAN = 2, UNITS = 256;
+  constexpr int RT = 32 * NW;
   // DECODE: a tile is RT heads of one token, and contexts are cut by length; else RT rows of [T * H], and the
   // workgroups past the tiles (`own_seq`) take a sequence's first rows where it begins inside a tile
   const int R = T * H, HG = (H + RT - 1) / RT;
@@ -581,48 +642,8 @@ __global__ __launch_bounds__(64 * (NW + row_movers(NW))) __attribute__((amdgpu_w
     }
   }
   if (DECODE && parts > 1) {
-    // Workgroup w of 256 takes piece w.  The span is the smallest number of key tiles that cuts all units
-    // into at most 256 pieces: one a CU (also within each XCD, to which workgroups go in turn), and none longer
-    // than it has to be, however ragged the contexts.  Every wave finds it from the lengths: lane l holds
-    // tokens 4 l .. 4 l + 3.
-    int nt4[4], most = SPAN, all = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int tk = 4 * lane + i;
-      nt4[i] = tk < T ? (kv_lens[tk] + KT - 1) / KT : 0;
-      most = max(most, nt4[i]);
-      all += nt4[i];
-    }
-    auto count = [&](int span, int i) {   // (a quotient of tiles is off by one at most)
-      const int n = nt4[i] + span - 1, about = (int)((float)n * __builtin_amdgcn_rcpf((float)span)), rest = n - about * span;
-      return 4 * lane + i < T ? min(parts, max(1, about + (rest >= span) - (rest < 0))) : 0;
-    };
-    auto pieces = [&](int span) { return wave_total(count(span, 0) + count(span, 1) + count(span, 2) + count(span, 3)) * HG; };
-    most = wave_most(most);
-    all = wave_total(all) * HG;
-    // all / span <= pieces <= all / span + units; one piece a unit is at most 256 (the caller's rule)
-    int lo = max(SPAN, min(most, all / UNITS)), hi = T * HG < UNITS ? max(lo, min(most, all / (UNITS - T * HG) + 1)) : most;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (pieces(mid) <= UNITS) hi = mid;
-      else lo = mid + 1;
-    }
-    // pieces that save fewer key tiles than their partials' way to memory and back costs: none (64 heads, 128 rows of ~100
-    // keys 34 -> 28 us)
-    if (most - lo <= 2 + R / 2048) lo = most;
-    const int w = blockIdx.x, c0 = count(lo, 0), c1 = count(lo, 1), c2 = count(lo, 2), c3 = count(lo, 3);
-    const int incl = wave_scan(c0 + c1 + c2 + c3);
-    if (w >= __builtin_amdgcn_readlane(incl, 63) * HG) return;   // whole block
-    const int at = __popcll(__ballot(incl * HG <= w));            // the lane whose tokens piece w belongs to
-    int tok = 4 * at, base = at ? __builtin_amdgcn_readlane(incl, at - 1) : 0;
-    my_parts = __builtin_amdgcn_readlane(c0, at);
-    if ((base + my_parts) * HG <= w) base += my_parts, ++tok, my_parts = __builtin_amdgcn_readlane(c1, at);
-    if ((base + my_parts) * HG <= w) base += my_parts, ++tok, my_parts = __builtin_amdgcn_readlane(c2, at);
-    if ((base + my_parts) * HG <= w) base += my_parts, ++tok, my_parts = __builtin_amdgcn_readlane(c3, at);
-    const int hg = (w - base * HG) / my_parts;
-    part = (w - base * HG) - hg * my_parts;
-    unit = tok * HG + hg;
-    if (part == 0 && tid == 0) plan[unit] = int2{w, my_parts};
+    if (!decode_piece(kv_lens, T, H, HG, parts, unit, part, my_parts)) return;   // whole block
+    if (part == 0 && tid == 0) plan[unit] = int2{(int)blockIdx.x, my_parts};
   }
   const int row0 = DECODE ? unit / HG * H + unit % HG * RT : unit * RT;
   const int row_end = DECODE ? (unit / HG + 1) * H : R;
@@ -1253,10 +1274,17 @@ __global__ __launch_bounds__(128) void mla_reduce_kernel(const float* __restrict
                                                          const float* __restrict__ ws_ml, int H, int parts,
                                                          bf16* __restrict__ out, int64_t out_stride_t,
                                                          const float* __restrict__ sinks, const int* __restrict__ kv_lens,
-                                                         int window, int least) {
+                                                         int window, int least, const int2* __restrict__ plan) {
   const int t = blockIdx.x, h = blockIdx.y;
-  const int64_t row0 = ((int64_t)t * H + h) * parts;
-  if (parts > 16 && least > 0) {   // as the 16-head kernels cut them, `least` tiles and more (with 16 the empty ones cost less than the length's way here)
+  int64_t row0 = ((int64_t)t * H + h) * parts;
+  int step = 1;
+  if (plan != nullptr) {   // a token's pieces by length, 16 rows each
+    const int2 pl = plan[t];
+    parts = pl.y;
+    if (parts == 1) return;   // written by its one piece
+    row0 = (int64_t)pl.x * 16 + h;
+    step = 16;
+  } else if (parts > 16 && least > 0) {   // as the 16-head kernels cut them, `least` tiles and more (with 16 the empty ones cost less than the length's way here)
     const int L = kv_lens[t], tiles = ((L + 15) / 16 + 1) / 2 - (window > 0 ? max(L - window, 0) / KT : 0);
     const int live = live_parts(tiles, parts), per = tiles > 0 ? max(least, (tiles + live - 1) / live) : 0;
     parts = per > 0 ? (tiles + per - 1) / per : 0;
@@ -1268,7 +1296,7 @@ __global__ __launch_bounds__(128) void mla_reduce_kernel(const float* __restrict
     f32x4 vv[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const int64_t r = row0 + min(p0 + j, parts - 1);
+      const int64_t r = row0 + (int64_t)min(p0 + j, parts - 1) * step;
       mm[j] = ws_ml[2 * r];
       ll[j] = p0 + j < parts ? ws_ml[2 * r + 1] : 0.f;
       vv[j] = *reinterpret_cast<const f32x4*>(ws_o + r * DV + 4 * threadIdx.x);
@@ -1323,7 +1351,14 @@ static void mla_launch(const void* q, int64_t q_stride_t, const void* cache, con
       mla_reduce_rows_kernel<DV, NW><<<dim3(units * NW, DV / 32), 256, 0, stream>>>(ws_o, ws_ml, T, H, parts, plan,       \
                                                                                     (bf16*)out, out_stride_t);            \
   }
-      if (rows == 128) MLA_ROWS(4)
+      if (rows == 32 && plan && H <= 16 && (int64_t)T * bt_stride >= 3000) {
+        mla_attn_pages_kernel<DK, DV, true><<<parts > 1 ? 256 : T, 256, 0, stream>>>(
+            (const bf16*)q, q_stride_t, (const bf16*)cache, block_tables, bt_stride, tok_row, kv_lens, T, H, scale_log2, parts, plan,
+            (bf16*)out, out_stride_t, ws_o, ws_ml, nullptr, -1);
+        if (parts > 1)
+          mla_reduce_kernel<DV><<<dim3(T, H), DV / 4, 0, stream>>>(ws_o, ws_ml, H, parts, (bf16*)out, out_stride_t, nullptr, kv_lens, -1, 0, plan);
+      }
+      else if (rows == 128) MLA_ROWS(4)
       else if (rows == 64) MLA_ROWS(2)
       else MLA_ROWS(1)
 #undef MLA_ROWS
@@ -1343,11 +1378,11 @@ static void mla_launch(const void* q, int64_t q_stride_t, const void* cache, con
     // (few workgroups over short tables: the old kernel starts a microsecond sooner.  It also has a CU hold several workgroups)
     const int64_t wgs = (int64_t)T * ((H + 15) / 16);
     if (!done && wgs * parts <= 512 && (wgs > 16 || bt_stride > 96)) {
-      mla_attn_pages_kernel<DK, DV><<<dim3(T, (H + 15) / 16, parts), 256, 0, stream>>>(
-          (const bf16*)q, q_stride_t, (const bf16*)cache, block_tables, bt_stride, tok_row, kv_lens, H, scale_log2,
-          parts, (bf16*)out, out_stride_t, ws_o, ws_ml, sinks, window);
+      mla_attn_pages_kernel<DK, DV, false><<<dim3(T, (H + 15) / 16, parts), 256, 0, stream>>>(
+          (const bf16*)q, q_stride_t, (const bf16*)cache, block_tables, bt_stride, tok_row, kv_lens, T, H, scale_log2,
+          parts, nullptr, (bf16*)out, out_stride_t, ws_o, ws_ml, sinks, window);
       if (parts > 1)
-        mla_reduce_kernel<DV><<<dim3(T, H), DV / 4, 0, stream>>>(ws_o, ws_ml, H, parts, (bf16*)out, out_stride_t, sinks, kv_lens, window, LEAST_PAIRS);
+        mla_reduce_kernel<DV><<<dim3(T, H), DV / 4, 0, stream>>>(ws_o, ws_ml, H, parts, (bf16*)out, out_stride_t, sinks, kv_lens, window, LEAST_PAIRS, nullptr);
       return;
     }
   }
@@ -1356,7 +1391,7 @@ static void mla_launch(const void* q, int64_t q_stride_t, const void* cache, con
         (const bf16*)q, q_stride_t, (const bf16*)cache, block_tables, bt_stride, tok_row, kv_lens, H, scale_log2,
         parts, (bf16*)out, out_stride_t, ws_o, ws_ml, sinks, window);
   if (parts > 1)
-    mla_reduce_kernel<DV><<<dim3(T, H), DV / 4, 0, stream>>>(ws_o, ws_ml, H, parts, (bf16*)out, out_stride_t, sinks, kv_lens, window, done ? 0 : 1);
+    mla_reduce_kernel<DV><<<dim3(T, H), DV / 4, 0, stream>>>(ws_o, ws_ml, H, parts, (bf16*)out, out_stride_t, sinks, kv_lens, window, done ? 0 : 1, nullptr);
 }
 
 OME_API int ome_mla_attn(const void* q, int64_t q_stride_t, const void* cache, const int* block_tables,

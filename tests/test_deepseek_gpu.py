@@ -354,6 +354,29 @@ def test_mla_waves_with_pages_of_their_own(T, H, longest):
         assert ((out - want).flatten(1).norm(dim=1)[live] <= 2.0 ** -8 * want.flatten(1).norm(dim=1)[live]).all()
 
 
+@pytest.mark.parametrize("H", [4, 9, 16])
+@pytest.mark.parametrize("lens,parts", [([1, 0, 32, 33, 5000], 52), (list(range(1, 257)), 1), ([700, 16, 64, 65, 1] * 13, 8), ([4097, 0] * 12, 22), ([300] * 200, 3)], ids=str)
+def test_mla_pieces_by_length_of_few_heads(monkeypatch, lens, parts, H):
+    """Decode steps of up to 16 heads over wide tables, with pieces of no, one and many pages and none at all, NaN in the workspace and past the contexts, at half the bound
+    above: weights are exact to 2^-17."""
+    torch.manual_seed(H)
+    cache, bt = _setup(lens)
+    for s, n in enumerate(lens):
+        if n % 16:
+            cache[bt[s, n // 16].item(), n % 16:] = float("nan")
+    bt = torch.nn.functional.pad(bt, (0, max(0, 3000 // len(lens) + 1 - bt.shape[1])))
+    row, kl = torch.arange(len(lens), dtype=torch.int32), torch.tensor(lens, dtype=torch.int32)
+    q = torch.randn(len(lens), H, 576, device=DEV).to(torch.bfloat16)
+    ws = ops.MLAWorkspace(DEV)
+    ws.ws_o.fill_(float("nan"))
+    ws.ws_ml.fill_(float("nan"))
+    monkeypatch.setattr(ops.MLAWorkspace, "tiles", lambda *a: (32, True, parts))
+    out = ops.mla_attn(q, cache, bt, row.to(DEV), kl.to(DEV), 192 ** -0.5, ws).cpu().double()
+    want = _exact(q, torch.nan_to_num(cache), bt, row, kl, 192 ** -0.5)
+    assert bool((out[kl == 0] == 0).all())
+    assert ((out - want).flatten(1).norm(dim=1) <= 2.0 ** -9 * want.flatten(1).norm(dim=1)).all()
+
+
 @pytest.mark.parametrize("T,H", [(1, 16), (3, 32), (12, 16)])
 def test_mla_reads_no_partition_that_is_not_written(T, H):
     """A workspace that holds NaN, contexts of fewer partitions than the table's width allows, and the tokens' own lengths.  Tolerance as above."""
