@@ -691,7 +691,7 @@ __global__ __launch_bounds__(64 * (NW + row_movers(NW))) __attribute__((amdgpu_w
           buffer_to_lds(q + (int64_t)tw * q_stride_t, 0x7fffffffu, (uint32_t)__builtin_amdgcn_ds_bpermute(4 * (8 * a + r8), (int)at) + 16 * (x ^ (a & 1)), 0,
                         lds0 + wave * IMG + 1024 * (9 * a + b));
       }
-    } else if (wave < NW) {
+    } else if (MW == 0 || wave < NW) {
       const bf16* qp = q + (int64_t)t * q_stride_t + (int64_t)head * DK + 8 * hf;
 #pragma unroll
       for (int s = 0; s < NS; ++s) qf[s] = ld8(qp + 16 * s);
@@ -731,7 +731,7 @@ __global__ __launch_bounds__(64 * (NW + row_movers(NW))) __attribute__((amdgpu_w
       for (int s = 0; s < NS; ++s) qf[s] = kfrag(wave * IMG, s);
     }
 #if defined(__HIP_DEVICE_COMPILE__)
-    if (wave < NW) {
+    if (MW == 0 || wave < NW) {
 #pragma unroll
       for (int s = 0; s < NS; ++s) asm volatile("" : "+v"(qf[s]));
     }
@@ -740,14 +740,17 @@ __global__ __launch_bounds__(64 * (NW + row_movers(NW))) __attribute__((amdgpu_w
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __syncthreads();   // (the images are the keys' from here on)
     }
-    const bf16 *b0 = cache, *b1 = cache;   // pages of the tile on its way, its image, its descriptors' size
+    int first_page = 0, second_page = 0;   // of the tile on its way (their addresses are formed beside the products, where they cost nothing), its image, its descriptors' size
     uint32_t to = 0, bytes = 0;
     auto aim = [&](int tile, int img) {    // (of a tile past the last nothing is read, zeros are written)
       if (tile < end && tile - pg0 == 32) look(tile);
       const int at = 2 * (tile - pg0);
-      b0 = cache + (int64_t)__builtin_amdgcn_readlane(pages, at & 63) * 16 * DK;
-      b1 = cache + (int64_t)__builtin_amdgcn_readlane(pages, (at + 1) & 63) * 16 * DK;
-      to = lds0 + img * IMG;
+      first_page = __builtin_amdgcn_readlane(pages, at & 63);
+      second_page = __builtin_amdgcn_readlane(pages, (at + 1) & 63);
+#if defined(__HIP_DEVICE_COMPILE__)
+      if constexpr (MW == 0) asm volatile("" : "+s"(first_page), "+s"(second_page));
+#endif
+      to = lds0 + img * IMG + 64 * 16 * mv;
       bytes = tile < end ? 16 * DK * 2 : 0;
       asm volatile("" : "+v"(dofs2[0]), "+v"(dofs2[1]), "+v"(dofs2[2]), "+v"(dofs2[3]), "+v"(dofs2[4]));   // (or the loop would hold them unpacked)
     };
@@ -759,7 +762,8 @@ __global__ __launch_bounds__(64 * (NW + row_movers(NW))) __attribute__((amdgpu_w
       const int i = mv + ML * j;
       constexpr int OWN = MW ? NI / 2 / ML : 9;   // offsets that a lane has: of a page's moves (MW == 0: two pages have an odd number)
       const uint32_t two = dofs2[j % OWN >> 1], at = j % OWN & 1 ? two >> 16 : two & 0xffff;
-      buffer_to_lds(j < NJ / 2 || (NJ % 2 && j == NJ / 2 && i < NI / 2) ? b0 : b1, bytes, at, 0, to + 64 * 16 * i);
+      const int page = j < NJ / 2 || (NJ % 2 && j == NJ / 2 && i < NI / 2) ? first_page : second_page;
+      buffer_to_lds(cache + (int64_t)page * 16 * DK, bytes, at, 0, to + 64 * 16 * ML * j);
     };
     if constexpr (MW > 0) {
       if (wave >= NW) {   // three tiles ahead of the one whose values are multiplied; barriers as below
